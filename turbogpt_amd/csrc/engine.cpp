@@ -4,6 +4,7 @@
 // op sequencing that its persistent kernel does on the device (cuda/trainer.cuh:103-125,
 // cuda/model.cuh:8-99).  All arithmetic is in the tgk_* kernels; this file only sequences them.
 #include "common.h"
+#include "readback.h"
 #include "../../include/tg_model.h"
 #include "../../include/tgk_kernels.h"
 #include <algorithm>
@@ -121,6 +122,9 @@ struct Engine {
     bool batched_wgrad = false; // a block's four weight gradients in one launch (shapes permitting)
     bool list_wgrad = false;    // every weight gradient of a step in one launch (widths that are multiples of 256)
 
+    std::shared_ptr<Readback> readback = Readback::shared();
+    float *batch_means = nullptr; // [context]: the per-position losses of a fixed batch
+
     std::vector<StepRates> schedule;
     uint64_t step = 0;
     uint64_t floor = 0; // oldest weight version that exists: the step at the last tg_set_weights / _set_optimizer_state
@@ -185,9 +189,8 @@ struct Engine {
     template <class T> void upload(T *device, const T *host, size_t n) {
         check_hip(hipMemcpyAsync(device, host, n * sizeof(T), hipMemcpyHostToDevice, stream));
     }
-    template <class T> void download(T *host, const T *device, size_t n) {
-        check_hip(hipMemcpyAsync(host, device, n * sizeof(T), hipMemcpyDeviceToHost, stream));
-    }
+    // results to the caller's memory, behind everything on the engine's stream; returns when they are there
+    void download(const std::vector<ReadbackPiece> &pieces) { readback->fetch(stream, config.base.device, pieces); }
     ~Engine() { // cuda/engine_internal.h:28-37
         (void)hipSetDevice(config.base.device);
         for (Slot &slot : slots)
@@ -435,19 +438,6 @@ struct Engine {
         total_staleness += at - read;
         max_staleness = std::max(max_staleness, int(at - read));
     }
-
-    void read_losses(float *out) { // cuda/runtime.cu:279-290
-        const Config &c = config.base;
-        std::vector<float> losses(static_cast<size_t>(tokens()));
-        download(losses.data(), slots[0].token_losses, losses.size());
-        sync();
-        for (int p = 0; p < c.context; ++p) {
-            double sum = 0;
-            for (int b = 0; b < c.batch; ++b)
-                sum += losses[size_t(b) * c.context + p];
-            out[p] = float(sum / c.batch);
-        }
-    }
 };
 
 namespace {
@@ -602,6 +592,7 @@ TG_API Engine *tg_create(const Config *c) {
         e->allocate(e->variance, P);
         e->allocate(e->norm_partials, NormPartials);
         e->allocate(e->loss_history, size_t(MaxLaunchSteps) * c->context);
+        e->allocate(e->batch_means, size_t(c->context));
         // AdamW owns the embedding, the RMSNorm scales and the head (decayed); Muon the hidden matrices
         // (cuda/optim.cuh:5-15).  Flat order per layer (model.h:20-31): scale 16, qkv 768, attention 256, scale 16,
         // gate 768, up 768, down 768.
@@ -678,6 +669,7 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
         e->allocate(e->variance, P);
         e->allocate(e->norm_partials, NormPartials);
         e->allocate(e->loss_history, size_t(MaxLaunchSteps) * c.context);
+        e->allocate(e->batch_means, size_t(c.context));
         build_segments(e);
         build_transpose_jobs(e);
         for (Slot &slot : e->slots) {
@@ -881,16 +873,8 @@ TG_API int tg_get_weights(Engine *e, float *weights) {
         if (!weights)
             throw std::runtime_error("Missing weights output");
         e->use_device();
-        const size_t n = size_t(e->layout.count);
-        std::vector<uint16_t> high(n), low(n);
         e->sync();
-        e->download(high.data(), e->current().hi, n);
-        e->download(low.data(), e->current().lo, n);
-        e->sync();
-        for (size_t i = 0; i < n; ++i) {
-            const uint32_t bits = (uint32_t(high[i]) << 16) | low[i];
-            std::memcpy(weights + i, &bits, 4);
-        }
+        e->download({{weights, size_t(e->layout.count) * 4, nullptr, e->current().hi, e->current().lo}});
     });
 }
 TG_API int tg_get_optimizer_state(Engine *e, float *momentum, float *variance, uint64_t *step) {
@@ -899,9 +883,8 @@ TG_API int tg_get_optimizer_state(Engine *e, float *momentum, float *variance, u
             throw std::runtime_error("Missing optimizer state output");
         e->use_device();
         e->sync();
-        e->download(momentum, e->momentum, size_t(e->layout.count));
-        e->download(variance, e->variance, size_t(e->layout.count));
-        e->sync();
+        const size_t bytes = size_t(e->layout.count) * 4;
+        e->download({{momentum, bytes, e->momentum}, {variance, bytes, e->variance}});
         *step = e->step;
     });
 }
@@ -995,8 +978,7 @@ TG_API int tg_get_training_losses(Engine *e, float *losses, int count) {
             throw std::runtime_error("Training loss count exceeds the last launch");
         e->use_device();
         e->sync(); // the rows are written on the slots' streams
-        e->download(losses, e->loss_history, size_t(count) * e->config.base.context);
-        e->sync();
+        e->download({{losses, size_t(count) * e->config.base.context * 4, e->loss_history}});
     });
 }
 // cuda/runtime.cu:243-262: the weight version each step of the last tg_train read (a synchronous engine
@@ -1036,11 +1018,14 @@ TG_API int tg_batch(Engine *e, const uint8_t *x, const uint8_t *y, float *logits
         e->forward(slot, e->current(), gradient != nullptr, e->logits_f32);
         if (gradient)
             e->backward(slot, e->current());
+        // per-position means in double (cuda/runtime.cu:279-290)
+        const Config &c = e->config.base;
+        ok(tgk_position_means(slot.stream, slot.token_losses, c.batch, c.context, e->batch_means));
         check_hip(hipStreamSynchronize(slot.stream));
-        e->download(logits, e->logits_f32, M * V);
+        std::vector<ReadbackPiece> pieces = {{logits, M * V * 4, e->logits_f32}, {loss, size_t(c.context) * 4, e->batch_means}};
         if (gradient)
-            e->download(gradient, slot.gradient, size_t(e->layout.count));
-        e->read_losses(loss);
+            pieces.push_back({gradient, size_t(e->layout.count) * 4, slot.gradient});
+        e->download(pieces);
     });
 }
 // cuda/runtime.cu:322-351
@@ -1062,8 +1047,7 @@ TG_API int tg_predict(Engine *e, const uint8_t *context, float *logits) {
         check_hip(hipMemcpyAsync(slot.target, target.data(), M, hipMemcpyHostToDevice, slot.stream));
         e->forward(slot, e->current(), false, e->logits_f32);
         check_hip(hipStreamSynchronize(slot.stream));
-        e->download(logits, e->logits_f32 + size_t(c.context - 1) * V, V);
-        e->sync();
+        e->download({{logits, V * 4, e->logits_f32 + size_t(c.context - 1) * V}});
     });
 }
 // cuda/runtime.cu:352-371

@@ -1,0 +1,141 @@
+// Moves results (weights, gradients, logits, losses) into the caller's pageable memory.
+//
+// What bounds it is PCIe (57 GB/s measured into pinned memory) and, behind it, the host: one core copies and
+// faults in fresh pages at a few GB/s.  So the result is cut into chunks; a kernel writes a chunk straight into pinned
+// memory (joining the weight halves on the way, which a host loop did before), and several host threads, each with
+// two buffers of its own, copy finished chunks into the caller's pages while the next ones cross the bus.
+#include "readback.h"
+#include <algorithm>
+#include <cstring>
+#include <exception>
+#include <thread>
+
+namespace {
+
+constexpr size_t CHUNK = size_t(2) << 20;
+constexpr int LANES = 8;
+
+__global__ __launch_bounds__(256) void readback_copy_kernel(const u32x4 *__restrict__ in, u32x4 *__restrict__ out,
+                                                            size_t n) {
+    for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += size_t(gridDim.x) * 256)
+        __builtin_nontemporal_store(in[i], out + i);
+}
+__global__ __launch_bounds__(256) void readback_join_kernel(const u32x2 *__restrict__ hi, const u32x2 *__restrict__ lo,
+                                                            u32x4 *__restrict__ out, size_t n) {
+    for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += size_t(gridDim.x) * 256) {
+        const u32x2 h = hi[i], l = lo[i];
+        const u32x4 joined = {(h.x << 16) | (l.x & 0xffffu), (h.x & 0xffff0000u) | (l.x >> 16),
+                              (h.y << 16) | (l.y & 0xffffu), (h.y & 0xffff0000u) | (l.y >> 16)};
+        __builtin_nontemporal_store(joined, out + i);
+    }
+}
+
+void enqueue(hipStream_t stream, const ReadbackPiece &piece, size_t offset, size_t bytes, void *out) {
+    const size_t n = bytes / 16;
+    const dim3 grid(unsigned(std::min<size_t>((n + 255) / 256, 512)));
+    if (piece.hi)
+        hipLaunchKernelGGL(readback_join_kernel, grid, dim3(256), 0, stream,
+                           reinterpret_cast<const u32x2 *>(piece.hi + offset / 4),
+                           reinterpret_cast<const u32x2 *>(piece.lo + offset / 4), static_cast<u32x4 *>(out), n);
+    else
+        hipLaunchKernelGGL(readback_copy_kernel, grid, dim3(256), 0, stream,
+                           reinterpret_cast<const u32x4 *>(static_cast<const uint8_t *>(piece.device) + offset),
+                           static_cast<u32x4 *>(out), n);
+    check_hip(hipGetLastError(), "readback launch: ");
+}
+
+} // namespace
+
+std::shared_ptr<Readback> Readback::shared() {
+    static std::mutex guard;
+    static std::weak_ptr<Readback> living;
+    const std::lock_guard<std::mutex> lock(guard);
+    std::shared_ptr<Readback> staging = living.lock();
+    if (!staging)
+        living = staging = std::shared_ptr<Readback>(new Readback);
+    return staging;
+}
+Readback::~Readback() {
+    for (Buffer &buffer : buffers) {
+        if (buffer.written)
+            (void)hipEventDestroy(buffer.written);
+        if (buffer.pinned)
+            (void)hipHostFree(buffer.pinned);
+    }
+}
+void Readback::reserve(size_t count) {
+    while (buffers.size() < count) {
+        buffers.emplace_back();
+        Buffer &buffer = buffers.back();
+        check_hip(hipHostMalloc(&buffer.pinned, CHUNK, hipHostMallocPortable), "pinned staging: ");
+        check_hip(hipHostGetDevicePointer(&buffer.mapped, buffer.pinned, 0), "pinned staging: ");
+        check_hip(hipEventCreateWithFlags(&buffer.written, hipEventDisableTiming));
+    }
+}
+
+void Readback::fetch(hipStream_t stream, int device, const std::vector<ReadbackPiece> &pieces) {
+    struct Chunk {
+        const ReadbackPiece *piece;
+        size_t offset, bytes;
+    };
+    std::vector<Chunk> chunks;
+    for (const ReadbackPiece &piece : pieces) {
+        require(piece.bytes % 16 == 0, "readback: size must be a multiple of 16");
+        for (size_t at = 0; at < piece.bytes; at += CHUNK)
+            chunks.push_back({&piece, at, std::min(CHUNK, piece.bytes - at)});
+    }
+    // lane `l` of `lanes` takes chunks l, l + lanes, ... with two buffers of its own in turn
+    const size_t lanes = std::min<size_t>(LANES, (chunks.size() + 1) / 2);
+    const size_t depth = chunks.size() == 1 ? 1 : 2;
+    const std::lock_guard<std::mutex> lock(busy);
+    reserve(lanes * depth);
+    const auto lane = [&](size_t l) {
+        const auto start = [&](size_t round) {
+            const size_t c = l + round * lanes;
+            if (c >= chunks.size())
+                return;
+            Buffer &buffer = buffers[l * depth + round % depth];
+            enqueue(stream, *chunks[c].piece, chunks[c].offset, chunks[c].bytes, buffer.mapped);
+            check_hip(hipEventRecord(buffer.written, stream));
+        };
+        for (size_t round = 0; round + 1 < depth; ++round)
+            start(round);
+        for (size_t round = 0; l + round * lanes < chunks.size(); ++round) {
+            start(round + depth - 1);
+            const Chunk &c = chunks[l + round * lanes];
+            const Buffer &buffer = buffers[l * depth + round % depth];
+            check_hip(hipEventSynchronize(buffer.written), "readback: ");
+            std::memcpy(static_cast<uint8_t *>(c.piece->host) + c.offset, buffer.pinned, c.bytes);
+        }
+    };
+    if (lanes <= 1) { // a small result: this thread alone
+        if (lanes)
+            lane(0);
+        return;
+    }
+    std::vector<std::exception_ptr> failures(lanes);
+    std::vector<std::thread> threads;
+    const auto guarded_lane = [&](size_t l) {
+        try {
+            check_hip(hipSetDevice(device));
+            lane(l);
+        } catch (...) {
+            failures[l] = std::current_exception();
+        }
+    };
+    try {
+        for (size_t l = 1; l < lanes; ++l)
+            threads.emplace_back(guarded_lane, l);
+    } catch (...) { // no more threads: this one takes the lanes that are left
+        for (size_t l = threads.size() + 1; l < lanes; ++l)
+            guarded_lane(l);
+    }
+    guarded_lane(0);
+    for (std::thread &thread : threads)
+        thread.join();
+    for (const std::exception_ptr &failure : failures)
+        if (failure) {
+            (void)hipStreamSynchronize(stream); // nothing may still write to the staging buffers
+            std::rethrow_exception(failure);
+        }
+}
