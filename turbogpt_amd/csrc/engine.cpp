@@ -17,6 +17,7 @@ namespace {
 
 constexpr int MaxLaunchSteps = 4096; // cuda/types.cuh:10
 constexpr int NormPartials = 1024;
+constexpr int RowTile = 128;    // smallest number of rows the matrix products take
 constexpr int MaxInFlight = 16; // batches in flight, each with its own stream and saved activations
 
 struct LayerBuffers {
@@ -228,14 +229,16 @@ struct Engine {
     }
 
     // cuda/model.cuh:8-59.  evaluate: logits stay logits; otherwise they are replaced by dlogits.
-    // On the slot's stream, with one weight version, from the slot's tokens.
-    void forward(Slot &s, const Version &v, bool with_gradient, float *logits_out) {
+    // On the slot's stream, with one weight version, from the slot's first `batch` sequences.  last_position: one
+    // sequence, and only the logits of its last position are wanted (`logits_out` receives that row): behind the
+    // attention of the last block nothing but the last tile of rows is computed.
+    void forward(Slot &s, const Version &v, bool with_gradient, float *logits_out, int batch, bool last_position = false) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
         const uint8_t *tokens_in = s.input, *targets = s.target;
         float *token_losses = s.token_losses;
         if (width16) {
-            OP(TG_CLASS_OTHER, tgk_w16_forward(stream, c.depth, c.batch, c.context, v.hi, v.lo, tokens_in, targets,
+            OP(TG_CLASS_OTHER, tgk_w16_forward(stream, c.depth, batch, c.context, v.hi, v.lo, tokens_in, targets,
                                                s.workspace, token_losses, logits_out, with_gradient ? 1 : 0));
             return;
         }
@@ -245,18 +248,22 @@ struct Engine {
         std::vector<bf16_t *> &x = s.x;
         std::vector<LayerBuffers> &layers = s.layers;
         bf16_t *nf = s.nf, *logits = s.logits;
-        const int M = tokens(), d = config.d_model, F = config.ffn, V = config.vocab, T = c.context;
+        const int d = config.d_model, F = config.ffn, V = config.vocab, T = c.context;
         const float scale = 1.0f / std::sqrt(float(d / config.heads));
+        int M = batch * T;
         OP(TG_CLASS_OTHER, tgk_embed_fwd(stream, M, T, d, tokens_in, w(layout.embedding), w(layout.positions), x[0]));
         for (int l = 0; l < c.depth; ++l) {
             const TgLayerParameters &p = layout.layers[l];
-            LayerBuffers &b = layers[l];
+            const LayerBuffers &b = layers[l];
             OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[l], w(p.ln1_g), wl(p.ln1_g), w(p.ln1_b), wl(p.ln1_b), b.n1,
                                  config.ln_eps));
             OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, 3 * d, d, b.n1, d, w(p.qkv), d, b.qkv, 3 * d, nullptr, 0, nullptr, 0));
-            OP(TG_CLASS_ATTN_FWD, tgk_attn_fwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d, b.qkv + 2 * d,
+            OP(TG_CLASS_ATTN_FWD, tgk_attn_fwd(stream, batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d, b.qkv + 2 * d,
                             3 * d, b.o, d, b.lse, scale));
-            OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, d, b.o, d, w(p.attn_out), d, b.mid, d, x[l], d, nullptr, 0));
+            const size_t skip = last_position && l == c.depth - 1 ? size_t(M - RowTile) : 0; // rows nobody reads
+            M -= int(skip);
+            const bf16_t *o = b.o + skip * d, *in = x[l] + skip * d;
+            OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, d, o, d, w(p.attn_out), d, b.mid, d, in, d, nullptr, 0));
             OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, b.mid, w(p.ln2_g), wl(p.ln2_g), w(p.ln2_b), wl(p.ln2_b), b.n2,
                                  config.ln_eps));
             OP(TG_CLASS_GEMM_FWD_GELU, tgk_gemm_fwd(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.u, F, nullptr, 0, b.a, F));
@@ -265,8 +272,9 @@ struct Engine {
         OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[c.depth], w(layout.lnf_g), wl(layout.lnf_g), w(layout.lnf_b),
                              wl(layout.lnf_b), nf, config.ln_eps));
         OP(TG_CLASS_HEAD, tgk_gemm_fwd_t(stream, M, V, d, nf, d, wt(layout.head), V, logits, V, nullptr, 0, nullptr, 0));
-        OP(TG_CLASS_OTHER, tgk_cross_entropy(stream, M, V, logits, targets, token_losses, logits_out, 1.0f / float(M),
-                             with_gradient ? 1 : 0));
+        const size_t row = last_position ? size_t(M - 1) : 0; // the first row whose logits are wanted
+        OP(TG_CLASS_OTHER, tgk_cross_entropy(stream, M - int(row), V, logits + row * V, targets, token_losses, logits_out,
+                             1.0f / float(M), with_gradient ? 1 : 0));
     }
 
     // cuda/model.cuh:61-99.  Every element of `gradient` is overwritten: nothing needs zeroing.
@@ -404,7 +412,7 @@ struct Engine {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
         OP(TG_CLASS_OTHER, tgk_sample_batch(stream, data, data_size, c.seed, at, c.batch, c.context, s.input, s.target));
-        forward(s, v, true, nullptr);
+        forward(s, v, true, nullptr, c.batch);
         OP(TG_CLASS_OTHER, tgk_position_means(stream, s.token_losses, c.batch, c.context, history_row));
         backward(s, v);
     }
@@ -1015,7 +1023,7 @@ TG_API int tg_batch(Engine *e, const uint8_t *x, const uint8_t *y, float *logits
         Slot &slot = e->slots[0];
         check_hip(hipMemcpyAsync(slot.input, x, M, hipMemcpyHostToDevice, slot.stream));
         check_hip(hipMemcpyAsync(slot.target, y, M, hipMemcpyHostToDevice, slot.stream));
-        e->forward(slot, e->current(), gradient != nullptr, e->logits_f32);
+        e->forward(slot, e->current(), gradient != nullptr, e->logits_f32, e->config.base.batch);
         if (gradient)
             e->backward(slot, e->current());
         // per-position means in double (cuda/runtime.cu:279-290)
@@ -1038,16 +1046,14 @@ TG_API int tg_predict(Engine *e, const uint8_t *context, float *logits) {
         const size_t M = size_t(e->tokens()), V = size_t(e->config.vocab);
         if (!e->logits_f32)
             e->allocate(e->logits_f32, M * V, false);
-        std::vector<uint8_t> input(M), target(M, 0);
-        for (int b = 0; b < c.batch; ++b)
-            std::copy(context, context + c.context, input.begin() + size_t(b) * c.context);
         e->sync();
+        // Sequences do not see each other: one of them is enough.  (cuda/runtime.cu:322-351 fills the batch with copies.)
+        // The wide model computes the last position's logits alone; the targets only feed losses that nobody reads.
         Slot &slot = e->slots[0];
-        check_hip(hipMemcpyAsync(slot.input, input.data(), M, hipMemcpyHostToDevice, slot.stream));
-        check_hip(hipMemcpyAsync(slot.target, target.data(), M, hipMemcpyHostToDevice, slot.stream));
-        e->forward(slot, e->current(), false, e->logits_f32);
+        check_hip(hipMemcpyAsync(slot.input, context, size_t(c.context), hipMemcpyHostToDevice, slot.stream));
+        e->forward(slot, e->current(), false, e->logits_f32, 1, !e->width16);
         check_hip(hipStreamSynchronize(slot.stream));
-        e->download({{logits, V * 4, e->logits_f32 + size_t(c.context - 1) * V}});
+        e->download({{logits, V * 4, e->logits_f32 + (e->width16 ? size_t(c.context - 1) * V : 0)}});
     });
 }
 // cuda/runtime.cu:352-371
