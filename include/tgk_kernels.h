@@ -39,9 +39,8 @@ TGK_API int tgk_gemm_fwd(hipStream_t stream, int M, int N, int K, const uint16_t
                  uint16_t *gelu_out, int ldg);
 
 /* The same forward projection with the weight given transposed, Wt[K][N] (leading dimension ldwt):
- * whole rows of Wt are copied instead of 64-byte pieces of W, which is faster where tgk_gemm_fwd cannot
- * use its 64-k stages (K not a multiple of 64, or N not a multiple of 192).  Same epilogues and shape
- * rules as tgk_gemm_fwd. */
+ * whole rows of Wt are copied instead of 64-byte pieces of W, which is faster where K is not a multiple of 64 (otherwise
+ * tgk_gemm_fwd is as fast or faster).  Same epilogues and shape rules as tgk_gemm_fwd. */
 TGK_API int tgk_gemm_fwd_t(hipStream_t stream, int M, int N, int K, const uint16_t *X, int ldx,
                            const uint16_t *Wt, int ldwt, uint16_t *Y, int ldy, const uint16_t *residual,
                            int ldr, uint16_t *gelu_out, int ldg);
