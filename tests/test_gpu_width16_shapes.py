@@ -1,0 +1,45 @@
+"""tgk_w16_forward / tgk_w16_backward at the shapes an engine does not make: every context (a wave holds 16, 15, 14 or 12
+tokens), token counts that fill no wave, block or chunk of partial sums, and one more than each; against the CPU checker
+with the tolerances of tests/test_gpu_width16.py, and independent of how many sequences there are, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check, library, stream, sync
+from oracle import width16 as w16
+from test_gpu_width16 import reference_style_weights, relative
+
+pytestmark = pytest.mark.gpu
+
+
+def run(depth, context, batch, flat, x, y):
+    lib = library()
+    bits = torch.from_numpy(flat.view(np.int32))
+    hi, lo = ((bits >> 16).to(torch.int16).cuda(), (bits & 0xffff).to(torch.int16).cuda())
+    tokens, targets = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
+    workspace = torch.full((lib.tgk_w16_workspace(depth, batch, context),), 255, dtype=torch.uint8, device="cuda")
+    losses = torch.empty(batch * context, device="cuda")
+    logits = torch.empty(batch * context, 256, device="cuda")
+    gradient = torch.empty(flat.size, device="cuda")
+    check(lib.tgk_w16_forward(stream(), depth, batch, context, hi.data_ptr(), lo.data_ptr(), tokens.data_ptr(),
+                              targets.data_ptr(), workspace.data_ptr(), losses.data_ptr(), logits.data_ptr(), 1))
+    check(lib.tgk_w16_backward(stream(), depth, batch, context, hi.data_ptr(), lo.data_ptr(), tokens.data_ptr(),
+                               workspace.data_ptr(), gradient.data_ptr()))
+    sync()
+    return logits.cpu().numpy().reshape(batch, context, 256), losses.cpu().numpy(), gradient.cpu().numpy()
+
+
+@pytest.mark.parametrize("depth,context,batch", [(1, 1, 1), (2, 1, 17), (2, 2, 9), (3, 3, 43), (1, 5, 13), (2, 6, 17), (8, 7, 5),
+                                                 (2, 8, 17), (4, 4, 33)])
+def test_against_the_checker(depth, context, batch):
+    flat = reference_style_weights(depth)
+    rng = np.random.default_rng(context * 100 + batch)
+    x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
+    logits, losses, gradient = run(depth, context, batch, flat, x, y)
+    target, expected, expected_losses = w16.Width16(depth, context, batch).batch(flat, x, y)
+    assert relative(logits, target) < .005
+    assert relative(gradient, expected) < .01
+    np.testing.assert_allclose(losses.reshape(batch, context).mean(0), expected_losses, atol=.003, rtol=.001)
+    # a sequence's logits do not depend on its place or its company
+    alone = run(depth, context, 1, flat, x[-1:], y[-1:])[0]
+    np.testing.assert_array_equal(alone[0], logits[-1])

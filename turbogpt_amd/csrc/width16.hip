@@ -3,21 +3,28 @@
 // mantissa-preserving AdamW + Muon.  Follows cuda/model.cuh:8-99 (op order and bf16 rounding points),
 // cuda/ops.cuh:57-144, cuda/attention.cuh:4-106, cuda/optim.cuh:17-119.
 //
-// The reference runs this model as one persistent kernel over 32-token tiles held in shared memory.
-// Here every operator group is a token-parallel kernel: a lane owns one token's 16-wide row in
-// registers and reads the (tiny, wave-uniform) weight matrices through the scalar/constant path;
-// sequences only meet in the two attention kernels, which read the other positions' keys / values /
-// gradients from the saved rows.  Weight gradients are not accumulated by atomics: every matrix,
-// RMSNorm scale and embedding row is one job of a single chunked outer-product kernel whose per-chunk
-// partials a second kernel folds in chunk order (bit-reproducible; takes the place of
-// weight_gradient's read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
+// What bounds it is latency: a step is 1 GFLOP over some ten thousand tokens, and a sequence (at most eight positions)
+// never leaves a wave.  So a wave takes sixteen tokens - whole sequences - through all layers in registers, one launch
+// forward and one backward, with the weights staged in LDS as matrix operands.  Products run on
+// v_mfma_f32_16x16x4_f32, which is bit for bit a chain of fmaf over its four k (measured on random and extreme values;
+// the bf16 forms add in an order of their own): every sum has one order, the k's own, whatever the kernel's shape, so
+// results do not depend on how the work is cut.  Lane 16 g + c works for token c:
+//   "feed" layout: register j holds feature 4 j + g - what step j of a product over features wants from that lane;
+//   "head" layout: register r holds feature 4 g + r - head g of the token, one head a lane, so attention reads other
+//   positions' keys and values with DPP row shifts.
+// A product's results come out in either, by the order of the weight's rows.  Weight gradients are products over tokens,
+// a third launch: a wave per 16 x 16 tile and chunk of tokens turns the saved rows with the identity matrix and adds over
+// the tokens in order; a fourth folds the chunks in order.  No atomics, bit-reproducible (the place of weight_gradient's
+// read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
 #include "common.h"
 #include "../../include/tgk_kernels.h"
+#include <type_traits>
 
 namespace {
 
-constexpr int W = 16, HEADS = 4, HD = 4, F = 48, V = 256, MAX_DEPTH = 8;
-constexpr int CHUNK = 128; // tokens per weight-gradient partial
+constexpr int W = 16, HEADS = 4, F = 48, V = 256, MAX_DEPTH = 8;
+constexpr int WAVES = 4;       // waves of a forward / backward block: they share the staged weights
+constexpr int CHUNK_WAVES = 8; // waves' tokens in one partial sum of a weight gradient (128 tokens)
 
 struct Layer {
     int attention_norm, qkv, attention, mlp_norm, gate, up, down;
@@ -26,185 +33,144 @@ struct Layout { // model.h:12-37
     int embedding, final_norm, head, count;
     Layer layers[MAX_DEPTH];
 };
+constexpr int LAYER_SIZE = W + 3 * W * W + W * W + W + 3 * F * W;
+__host__ __device__ inline Layer layer_layout(int l) {
+    Layer b;
+    b.attention_norm = V * W + l * LAYER_SIZE;
+    b.qkv = b.attention_norm + W;
+    b.attention = b.qkv + 3 * W * W;
+    b.mlp_norm = b.attention + W * W;
+    b.gate = b.mlp_norm + W;
+    b.up = b.gate + F * W;
+    b.down = b.up + F * W;
+    return b;
+}
 Layout make_layout(int depth) {
     Layout p{};
-    int n = 0;
-    auto take = [&](int size) {
-        const int offset = n;
-        n += size;
-        return offset;
-    };
-    p.embedding = take(V * W);
-    for (int l = 0; l < depth; ++l) {
-        Layer &b = p.layers[l];
-        b.attention_norm = take(W);
-        b.qkv = take(3 * W * W);
-        b.attention = take(W * W);
-        b.mlp_norm = take(W);
-        b.gate = take(F * W);
-        b.up = take(F * W);
-        b.down = take(W * F);
-    }
-    p.final_norm = take(W);
-    p.head = take(V * W);
-    p.count = n;
+    for (int l = 0; l < depth; ++l)
+        p.layers[l] = layer_layout(l);
+    p.embedding = 0;
+    p.final_norm = V * W + depth * LAYER_SIZE;
+    p.head = p.final_norm + W;
+    p.count = p.head + V * W;
     return p;
 }
 
-// Saved rows of one layer (what forward keeps for backward: cuda/types.cuh:40-44 plus the gate/up
-// cache of cuda/model.cuh:25-29) and the rows backward leaves for the weight-gradient jobs.
-struct LayerRows {
-    bf16_t *x, *qkv, *middle, *gu;        // forward: block input, post-RoPE q|k|v, post-attention residual, gate|up
-    int *selected;                        // winning key (token row) per (token, head)
-    float *gates, *derivatives;           // GELU(top), GELU'(top)
-    bf16_t *n1, *a, *n2, *act, *dgu, *dqkv; // backward: operands of the five weight gradients
-    bf16_t *dh_down, *dh_attention;        // the residual gradient as the down / attention projections saw it
-    float *gz_attention, *gz_mlp;         // per-token g*z of the two RMSNorm scales
+// Rows kept between the launches, a tile of 64 x 8 bytes a wave and quantity in the lanes' own order.  Forward: block
+// input, normalised rows, post-RoPE query, the winning key and value (head layout), attention output, post-attention
+// residual, gate | up and activation (cuda/types.cuh:40-44, cuda/model.cuh:25-29); backward: the gradients that are
+// operands of the weight gradients.  And words: GELU(top), GELU'(top), distance to the winner, the two inverse norms.
+enum Tile {
+    T_X, T_N1, T_Q, T_KEY, T_VALUE, T_A, T_MIDDLE, T_N2, T_GU, T_ACT = T_GU + 6,
+    T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES
 };
-struct Rows {
-    LayerRows layer[MAX_DEPTH];
-    bf16_t *hidden, *nf, *dlogits, *dh, *dattn;
-    float *dt, *gz_final, *partials;
+enum Word { WORD_GATE, WORD_SLOPE, WORD_DISTANCE, WORD_INV1, WORD_INV2, WORDS };
+struct Workspace {
+    u32x2 *tiles;    // [depth][waves][TILES][64]
+    float *words;    // [depth][waves][WORDS][64]
+    float *gz;       // [2 depth + 1][waves * 16][16]: g * z of every RMSNorm scale; the final norm's last
+    u32x2 *hidden, *nf, *dh; // [waves][64]
+    float *inverse;  // [waves][64] of the final norm
+    u32x2 *dlogits;  // [waves][16][64]
+    float *partials; // [chunks][parameters]
+    int waves, blocks, chunks;
     size_t bytes;
 };
-Rows carve(int depth, int tokens, void *base) {
-    Rows r{};
+int tokens_per_wave(int context) { return 16 / context * context; }
+Workspace carve(int depth, int batch, int context, void *base) {
+    Workspace r{};
     size_t at = 0;
     auto take = [&](size_t bytes) {
         void *p = base ? static_cast<unsigned char *>(base) + at : nullptr;
         at += (bytes + 255) & ~size_t(255);
         return p;
     };
-    const size_t N = size_t(tokens);
-    for (int l = 0; l < depth; ++l) {
-        LayerRows &b = r.layer[l];
-        b.x = static_cast<bf16_t *>(take(N * W * 2));
-        b.qkv = static_cast<bf16_t *>(take(N * 3 * W * 2));
-        b.middle = static_cast<bf16_t *>(take(N * W * 2));
-        b.gu = static_cast<bf16_t *>(take(N * 2 * F * 2));
-        b.selected = static_cast<int *>(take(N * HEADS * 4));
-        b.gates = static_cast<float *>(take(N * HEADS * 4));
-        b.derivatives = static_cast<float *>(take(N * HEADS * 4));
-        b.n1 = static_cast<bf16_t *>(take(N * W * 2));
-        b.a = static_cast<bf16_t *>(take(N * W * 2));
-        b.n2 = static_cast<bf16_t *>(take(N * W * 2));
-        b.act = static_cast<bf16_t *>(take(N * F * 2));
-        b.dgu = static_cast<bf16_t *>(take(N * 2 * F * 2));
-        b.dqkv = static_cast<bf16_t *>(take(N * 3 * W * 2));
-        b.dh_down = static_cast<bf16_t *>(take(N * W * 2));
-        b.dh_attention = static_cast<bf16_t *>(take(N * W * 2));
-        b.gz_attention = static_cast<float *>(take(N * W * 4));
-        b.gz_mlp = static_cast<float *>(take(N * W * 4));
-    }
-    r.hidden = static_cast<bf16_t *>(take(N * W * 2));
-    r.nf = static_cast<bf16_t *>(take(N * W * 2));
-    r.dlogits = static_cast<bf16_t *>(take(N * V * 2));
-    r.dh = static_cast<bf16_t *>(take(N * W * 2));
-    r.dattn = static_cast<bf16_t *>(take(N * W * 2));
-    r.dt = static_cast<float *>(take(N * HEADS * 4));
-    r.gz_final = static_cast<float *>(take(N * W * 4));
-    const size_t chunks = (N + CHUNK - 1) / CHUNK;
-    r.partials = static_cast<float *>(take(chunks * size_t(make_layout(depth).count) * 4));
+    const int per_wave = tokens_per_wave(context);
+    r.blocks = (batch * context + per_wave * WAVES - 1) / (per_wave * WAVES);
+    r.waves = r.blocks * WAVES;
+    r.chunks = (r.waves + CHUNK_WAVES - 1) / CHUNK_WAVES;
+    const size_t n = size_t(r.waves) * 64;
+    r.tiles = static_cast<u32x2 *>(take(n * depth * TILES * sizeof(u32x2)));
+    r.words = static_cast<float *>(take(n * depth * WORDS * sizeof(float)));
+    r.gz = static_cast<float *>(take(n * (2 * depth + 1) * 4 * sizeof(float)));
+    r.hidden = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
+    r.nf = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
+    r.dh = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
+    r.inverse = static_cast<float *>(take(n * sizeof(float)));
+    r.dlogits = static_cast<u32x2 *>(take(n * 16 * sizeof(u32x2)));
+    r.partials = static_cast<float *>(take(size_t(r.chunks) * make_layout(depth).count * sizeof(float)));
     r.bytes = at;
     return r;
 }
 
 // ---- device helpers ---------------------------------------------------------------------------------
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
 TG_DEVICE float master(const bf16_t *hi, const uint16_t *lo, int i) { // cuda/ops.cuh:6-9
     return __uint_as_float((uint32_t(hi[i]) << 16) | lo[i]);
 }
-TG_DEVICE void load_row16(const bf16_t *p, float (&v)[16]) {
-    const u32x4 a = *reinterpret_cast<const u32x4 *>(p), b = *reinterpret_cast<const u32x4 *>(p + 8);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[2 * e] = bf16_lo(a[e]), v[2 * e + 1] = bf16_hi(a[e]);
-        v[8 + 2 * e] = bf16_lo(b[e]), v[8 + 2 * e + 1] = bf16_hi(b[e]);
-    }
+TG_DEVICE u32x2 pack4(const f32x4 &v) {
+    return u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
 }
-// stores RN_bf16 of 16 values and leaves the rounded values in v
-TG_DEVICE void store_row16(bf16_t *p, float (&v)[16]) {
-    u32x4 a, b;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        a[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
-        b[e] = pack_bf16(v[8 + 2 * e], v[8 + 2 * e + 1]);
-    }
-    *reinterpret_cast<u32x4 *>(p) = a;
-    *reinterpret_cast<u32x4 *>(p + 8) = b;
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-        v[e] = round_bf16(v[e]);
+TG_DEVICE f32x4 unpack4(const u32x2 &t) {
+    return f32x4{bf16_lo(t.x), bf16_hi(t.x), bf16_lo(t.y), bf16_hi(t.y)};
 }
-// y[o] = sum_i x[i] W[o][i], W row-major [OUT][IN] bf16 at wave-uniform addresses
-template <int OUT, int IN> TG_DEVICE void matvec(const bf16_t *__restrict__ w, const float (&x)[IN], float (&y)[OUT]) {
-#pragma unroll
-    for (int o = 0; o < OUT; ++o) {
-        float acc = 0.f;
-#pragma unroll
-        for (int i = 0; i < IN; ++i)
-            acc = fmaf(x[i], bf16_to_float(w[o * IN + i]), acc);
-        y[o] = acc;
-    }
+TG_DEVICE f32x4 rounded(const f32x4 &v) {
+    return unpack4(pack4(v));
 }
-// dx[i] = sum_o dy[o] W[o][i]
-template <int OUT, int IN> TG_DEVICE void matvec_t(const bf16_t *__restrict__ w, const float (&dy)[OUT], float (&dx)[IN]) {
+constexpr f32x4 ZERO = {0.f, 0.f, 0.f, 0.f};
+// D[row][col] = fmaf chain over k = 0 .. 15 of A[row][k] B[k][col], on top of acc: lane 16 g + c gives A[c][4 j + g] and
+// B[4 j + g][c] in register j and gets D[4 g + r][c] in register r
+TG_DEVICE f32x4 multiply(const f32x4 &a, const f32x4 &b, f32x4 acc = ZERO) {
 #pragma unroll
-    for (int i = 0; i < IN; ++i)
-        dx[i] = 0.f;
-#pragma unroll
-    for (int o = 0; o < OUT; ++o)
-#pragma unroll
-        for (int i = 0; i < IN; ++i)
-            dx[i] = fmaf(dy[o], bf16_to_float(w[o * IN + i]), dx[i]);
+    for (int j = 0; j < 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+    return acc;
 }
-// cuda/ops.cuh:57-67: y = RN_bf16(v * rsqrt(mean(v^2) + 1e-6) * scale), scale read in full fp32
-TG_DEVICE float inverse_rms(const float (&v)[16]) {
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        sum = fmaf(v[i], v[i], sum);
-    return rsqrtf(sum * (1.f / 16.f) + 1e-6f);
+TG_DEVICE float swap_add_16(float x) {
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
 }
-TG_DEVICE void normalize(const float (&v)[16], const bf16_t *hi, const uint16_t *lo, int scale, float (&y)[16]) {
-    const float inv = inverse_rms(v);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        y[i] = round_bf16(v[i] * inv * master(hi, lo, scale + i));
+TG_DEVICE float swap_add_32(float x) {
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
 }
-// cuda/ops.cuh:68-80: returns RN_bf16(dx) in dx and the per-token g*z terms of the scale gradient
-TG_DEVICE void normalize_backward(const float (&v)[16], const float (&g)[16], const bf16_t *hi, const uint16_t *lo,
-                                  int scale, float (&dx)[16], float *gz) {
-    const float inv = inverse_rms(v);
-    float dot = 0.f, z[16], dz[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        z[i] = v[i] * inv;
-        dz[i] = g[i] * master(hi, lo, scale + i);
-        dot = fmaf(dz[i], z[i], dot);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        dx[i] = round_bf16((dz[i] - z[i] * dot * (1.f / 16.f)) * inv);
-        gz[i] = g[i] * z[i];
-    }
+TG_DEVICE float token_max(float x) { // over the four lanes that hold one token
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
 }
-// cuda/attention.cuh:19-30: first pair of every query and key head, one radian per position, unfused
-TG_DEVICE void rotate(float (&qkv)[48], int position, bool inverse) {
-    float s, c;
-    // float32(cos k), float32(sin k), k = 0..7 (cuda/attention.cuh:7-14)
-    const float cos_table[8] = {1.0f, 0.5403022766113281f, -0.416146844625473f, -0.9899924993515015f,
-                                -0.6536436080932617f, 0.28366219997406006f, 0.9601702690124512f, 0.7539022564888f};
-    const float sin_table[8] = {0.0f, 0.8414709568023682f, 0.9092974066734314f, 0.14112000167369843f,
-                                -0.756802499294281f, -0.9589242935180664f, -0.279415488243103f, 0.6569865942001343f};
-    c = cos_table[position];
-    s = inverse ? -sin_table[position] : sin_table[position];
-#pragma unroll
-    for (int pair = 0; pair < 8; ++pair) {
-        const int at = pair * 4; // query heads 0-3, then key heads 0-3
-        const float x = qkv[at], y = qkv[at + 1];
-        qkv[at] = round_bf16(__fsub_rn(__fmul_rn(x, c), __fmul_rn(y, s)));
-        qkv[at + 1] = round_bf16(__fadd_rn(__fmul_rn(x, s), __fmul_rn(y, c)));
-    }
+// head layout <-> feed layout: the 4 x 4 transposition of (lane group, register)
+TG_DEVICE f32x4 turned(const f32x4 &v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1])};
+}
+// the value of the lane D before / after this one in its row of sixteen (0 beyond the row)
+template <int D> TG_DEVICE uint32_t earlier(uint32_t x) {
+    if constexpr (D == 0)
+        return x;
+    else
+        return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), 0x110 + D, 0xF, 0xF, true));
+}
+template <int D> TG_DEVICE uint32_t later(uint32_t x) {
+    if constexpr (D == 0)
+        return x;
+    else
+        return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), 0x100 + D, 0xF, 0xF, true));
+}
+template <int D, class Body> TG_DEVICE void from(Body &&body) { // D, D - 1, ..., 0
+    body(std::integral_constant<int, D>{});
+    if constexpr (D > 0)
+        from<D - 1>(body);
+}
+template <int D, int END, class Body> TG_DEVICE void up_to(Body &&body) { // D, D + 1, ..., END
+    body(std::integral_constant<int, D>{});
+    if constexpr (D < END)
+        up_to<D + 1, END>(body);
 }
 TG_DEVICE float sigmoid(float x) {
     return 1.f / (1.f + expf(-x));
@@ -213,431 +179,485 @@ TG_DEVICE float sigmoid(float x) {
 struct Model {
     const bf16_t *hi;
     const uint16_t *lo;
-    Layout layout;
-    int tokens, context;
+    int depth, tokens, context, per_wave;
+};
+// a lane's place: token `token` (if `live`) at `position` of its sequence
+struct Lane {
+    int lane, c, g, wave, token, position;
+    bool live;
+};
+TG_DEVICE Lane lane_of(const Model &m) {
+    Lane p;
+    p.lane = threadIdx.x & 63;
+    p.c = p.lane & 15;
+    p.g = p.lane >> 4;
+    p.wave = blockIdx.x * WAVES + (threadIdx.x >> 6);
+    p.token = p.wave * m.per_wave + p.c;
+    p.live = p.c < m.per_wave && p.token < m.tokens;
+    p.position = p.c % m.context;
+    return p;
+}
+
+// The weights in LDS as first operands, a tile of 64 x 8 bytes each (lane 16 g + c: elements (row c, k = 4 j + g), j = 0..3):
+// 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
+// The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
+constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
+__host__ __device__ constexpr int staged_tiles(int depth) { return depth * LAYER_TILES + HEAD_TILES; }
+size_t staged_bytes(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
+TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its own inverse
+// TRANSPOSED: operands of dX = dY W (rows = inputs, k = outputs; the attention projection's rows in head layout)
+// instead of Y = X W^T (rows = outputs; q, k and v in head layout)
+template <bool TRANSPOSED> TG_DEVICE void stage_weights(const Model &m, uint16_t *tiles, float *scales) {
+    const int layer_chunks = LAYER_TILES * 64, total = m.depth * layer_chunks + HEAD_TILES * 64;
+    for (int at = threadIdx.x; at < total; at += 64 * WAVES) { // four elements of one row at a time
+        int tile, row, col, source; // tile of the element's matrix row range, row and column within the tile
+        bool feed = true;
+        if (at < m.depth * layer_chunks) {
+            const int l = at / layer_chunks, k = at - l * layer_chunks;
+            const Layer q = layer_layout(l);
+            if (k < 640) { // q, k, v, attention, gate, up: rows of 16
+                const int r = k >> 2;
+                tile = l * LAYER_TILES + (r >> 4);
+                row = r & 15, col = (k & 3) * 4;
+                source = (r < 64 ? q.qkv + r * W : q.gate + (r - 64) * W) + col;
+                feed = TRANSPOSED ? (r >> 4) != 3 : (r >> 4) > 2;
+            } else { // down: rows of 48
+                const int r = (k - 640) / 12, part = (k - 640) - r * 12;
+                tile = l * LAYER_TILES + 10 + (part >> 2);
+                row = r, col = (part & 3) * 4;
+                source = q.down + r * F + part * 4;
+            }
+        } else {
+            const int k = at - m.depth * layer_chunks, r = k >> 2;
+            tile = m.depth * LAYER_TILES + (r >> 4);
+            row = r & 15, col = (k & 3) * 4;
+            source = V * W + m.depth * LAYER_SIZE + W + r * W + col;
+        }
+        const u32x2 v = *reinterpret_cast<const u32x2 *>(m.hi + source);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int operand_row = TRANSPOSED ? col + e : row, k = TRANSPOSED ? row : col + e;
+            const int c = feed ? feed_row(operand_row) : operand_row;
+            tiles[(tile * 64 + (k & 3) * 16 + c) * 4 + (k >> 2)] = uint16_t((e < 2 ? v.x : v.y) >> ((e & 1) * 16));
+        }
+    }
+    for (int at = threadIdx.x; at < (2 * m.depth + 1) * W; at += 64 * WAVES) { // attention and MLP norm of each layer, final
+        const int n = at >> 4;
+        const Layer q = layer_layout(n >> 1);
+        const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
+        scales[at] = master(m.hi, m.lo, offset + (at & 15));
+    }
+    __syncthreads();
+}
+struct Staged {
+    const u32x2 *tiles;
+    const float *scales;
+    int lane, g;
+    TG_DEVICE f32x4 operator()(int tile) const { return unpack4(tiles[tile * 64 + lane]); }
+    TG_DEVICE f32x4 scale(int norm) const {
+        const float *s = scales + norm * W + g;
+        return f32x4{s[0], s[4], s[8], s[12]};
+    }
 };
 
+// feed-layout rows times feed-layout rows of the same token, an fmaf chain in feature order: the diagonal of a product
+TG_DEVICE float token_dot(const f32x4 &a, const f32x4 &b, const Lane &p) {
+    const f32x4 all = multiply(a, b);
+    float mine = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        mine = 4 * p.g + r == p.c ? all[r] : mine;
+    return swap_add_32(swap_add_16(mine)); // the other three lanes hold zeros
+}
+// cuda/ops.cuh:57-67: y = RN_bf16(v * rsqrt(mean(v^2) + 1e-6) * scale), scale read in full fp32
+TG_DEVICE float inverse_rms(const f32x4 &v, const Lane &p) {
+    const float sum = token_dot(v, v, p);
+    return rsqrtf(sum * (1.f / 16.f) + 1e-6f);
+}
+TG_DEVICE u32x2 normalize(const f32x4 &v, float inv, const f32x4 &scale) {
+    return pack4(f32x4{v[0] * inv * scale[0], v[1] * inv * scale[1], v[2] * inv * scale[2], v[3] * inv * scale[3]});
+}
+// cuda/ops.cuh:68-80: the rounded input gradient; the token's g * z terms of the scale gradient go to gz
+TG_DEVICE f32x4 normalize_backward(const f32x4 &v, float inv, const f32x4 &g, const f32x4 &scale, float *gz, const Lane &p) {
+    f32x4 z, dz, dx;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z[i] = v[i] * inv;
+        dz[i] = g[i] * scale[i];
+        gz[4 * i] = g[i] * z[i];
+    }
+    const float dot = token_dot(dz, z, p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        dx[i] = round_bf16((dz[i] - z[i] * dot * (1.f / 16.f)) * inv);
+    return dx;
+}
+// cuda/attention.cuh:19-30: first pair of every query and key head, one radian per position
+TG_DEVICE void rotation(int position, float &c, float &s) {
+    // float32(cos k), float32(sin k), k = 0..7 (cuda/attention.cuh:7-14)
+    const float cos_table[8] = {1.0f, 0.5403022766113281f, -0.416146844625473f, -0.9899924993515015f,
+                                -0.6536436080932617f, 0.28366219997406006f, 0.9601702690124512f, 0.7539022564888f};
+    const float sin_table[8] = {0.0f, 0.8414709568023682f, 0.9092974066734314f, 0.14112000167369843f,
+                                -0.756802499294281f, -0.9589242935180664f, -0.279415488243103f, 0.6569865942001343f};
+    c = cos_table[0], s = sin_table[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k)
+        if (position == k)
+            c = cos_table[k], s = sin_table[k];
+}
+TG_DEVICE f32x4 rotate(f32x4 v, float c, float s) {
+    const float x = v[0], y = v[1];
+    v[0] = fmaf(x, c, -(y * s));
+    v[1] = fmaf(x, s, y * c);
+    return v;
+}
+TG_DEVICE f32x4 rotate_back(f32x4 v, float c, float s) {
+    const float x = v[0], y = v[1];
+    v[0] = fmaf(x, c, y * s);
+    v[1] = fmaf(y, c, -(x * s));
+    return v;
+}
+
 // ---- forward ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void w16_embed_kernel(Model m, const uint8_t *__restrict__ x, bf16_t *hidden) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const bf16_t *row = m.hi + m.layout.embedding + int(x[t]) * W;
-    *reinterpret_cast<u32x4 *>(hidden + size_t(t) * W) = *reinterpret_cast<const u32x4 *>(row);
-    *reinterpret_cast<u32x4 *>(hidden + size_t(t) * W + 8) = *reinterpret_cast<const u32x4 *>(row + 8);
-}
-
-// save block input, RMSNorm, QKV projection, RoPE (cuda/model.cuh:14-19)
-__global__ __launch_bounds__(64) void w16_qkv_kernel(Model m, int l, const bf16_t *__restrict__ hidden, LayerRows rows) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    float v[16], n[16], qkv[48];
-    load_row16(hidden + size_t(t) * W, v);
-    store_row16(rows.x + size_t(t) * W, v);
-    normalize(v, m.hi, m.lo, p.attention_norm, n);
-    matvec<48, 16>(m.hi + p.qkv, n, qkv);
-#pragma unroll
-    for (int o = 0; o < 48; ++o)
-        qkv[o] = round_bf16(qkv[o]);
-    rotate(qkv, t % m.context, false);
-    bf16_t *out = rows.qkv + size_t(t) * 48;
-#pragma unroll
-    for (int o = 0; o < 48; o += 2)
-        *reinterpret_cast<uint32_t *>(out + o) = pack_bf16(qkv[o], qkv[o + 1]);
-}
-
-// arg-max attention with its GELU gate, output projection and residual (cuda/model.cuh:20-21,
-// cuda/attention.cuh:33-71)
-__global__ __launch_bounds__(64) void w16_attention_kernel(Model m, int l, LayerRows rows) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    const int start = t / m.context * m.context;
-    const bf16_t *mine = rows.qkv + size_t(t) * 48;
-    float a[16];
-#pragma unroll
-    for (int head = 0; head < HEADS; ++head) {
-        float q[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            q[c] = bf16_to_float(mine[head * 4 + c]);
+// cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).
+__global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x,
+                                                               const uint8_t *__restrict__ y, Workspace s,
+                                                               float *__restrict__ token_losses,
+                                                               float *__restrict__ logits_out, int with_gradient) {
+    extern __shared__ __align__(16) unsigned char staged_memory[];
+    uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
+    float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
+    stage_weights<false>(m, staged_tiles_at, scales);
+    const Lane p = lane_of(m);
+    const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
+    float rc, rs;
+    rotation(p.position, rc, rs);
+    f32x4 h = ZERO;
+    if (p.live) {
+        const bf16_t *row = m.hi + int(x[p.token]) * W + p.g;
+        h = f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])};
+    }
+    const int target = p.live ? y[p.token] : 0;
+    for (int l = 0; l < m.depth; ++l) {
+        const int tile = l * LAYER_TILES;
+        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
+        float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
+        // QKV projection, RoPE (cuda/model.cuh:14-19)
+        const float inv1 = inverse_rms(h, p);
+        const u32x2 n1 = normalize(h, inv1, weight.scale(2 * l));
+        const f32x4 n1f = unpack4(n1);
+        const f32x4 query = rounded(rotate(rounded(multiply(weight(tile), n1f)), rc, rs));
+        const u32x2 key = pack4(rotate(rounded(multiply(weight(tile + 1), n1f)), rc, rs));
+        const u32x2 value = pack4(multiply(weight(tile + 2), n1f));
+        // arg-max attention with its GELU gate (cuda/attention.cuh:33-71); keys in order, the first one wins ties
         float top = -INFINITY;
-        int best = start;
-        for (int key = start; key <= t; ++key) {
-            const bf16_t *k = rows.qkv + size_t(key) * 48 + 16 + head * 4;
+        int distance = 0;
+        u32x2 best_key = {0, 0}, best_value = {0, 0};
+        from<7>([&](auto step) {
+            constexpr int D = decltype(step)::value;
+            if (D >= m.context)
+                return;
+            const u32x2 k = {earlier<D>(key.x), earlier<D>(key.y)}, v = {earlier<D>(value.x), earlier<D>(value.y)};
+            const f32x4 kf = unpack4(k);
             float score = 0.f;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                score += q[c] * bf16_to_float(k[c]);
-            if (score > top) { // first index wins ties
-                top = score;
-                best = key;
-            }
-        }
+                score = fmaf(query[c], kf[c], score);
+            const bool wins = D <= p.position && score > top;
+            top = wins ? score : top;
+            distance = wins ? D : distance;
+            best_key.x = wins ? k.x : best_key.x, best_key.y = wins ? k.y : best_key.y;
+            best_value.x = wins ? v.x : best_value.x, best_value.y = wins ? v.y : best_value.y;
+        });
         const float e = 1.f + erff(top * 0.7071067811865475f);
         const float gate = 0.5f * top * e;
-        rows.selected[size_t(t) * HEADS + head] = best;
-        rows.gates[size_t(t) * HEADS + head] = gate;
-        rows.derivatives[size_t(t) * HEADS + head] = 0.5f * e + top * 0.3989422804014327f * expf(-0.5f * top * top);
-        const bf16_t *value = rows.qkv + size_t(best) * 48 + 32 + head * 4;
+        const f32x4 a = turned(rounded(unpack4(best_value) * gate));
+        // output projection and residual: a bf16 add (cuda/model.cuh:20-21, cuda/mma.cuh:95-97)
+        const f32x4 middle = rounded(rounded(multiply(weight(tile + 3), a)) + h);
+        const float inv2 = inverse_rms(middle, p);
+        const u32x2 n2 = normalize(middle, inv2, weight.scale(2 * l + 1));
+        if (with_gradient) {
+            keep[T_X * 64] = pack4(h);
+            keep[T_N1 * 64] = n1;
+            keep[T_Q * 64] = pack4(query);
+            keep[T_KEY * 64] = best_key;
+            keep[T_VALUE * 64] = best_value;
+            keep[T_A * 64] = pack4(a);
+            keep[T_MIDDLE * 64] = pack4(middle);
+            keep[T_N2 * 64] = n2;
+            words[WORD_GATE * 64] = gate;
+            words[WORD_SLOPE * 64] = 0.5f * e + top * 0.3989422804014327f * expf(-0.5f * top * top);
+            words[WORD_DISTANCE * 64] = __int_as_float(distance);
+            words[WORD_INV1 * 64] = inv1;
+            words[WORD_INV2 * 64] = inv2;
+        }
+        // packed gate|up projection, SwiGLU (RN after SiLU and after the product), down projection and residual
+        // (cuda/model.cuh:22-30, cuda/ops.cuh:120-131)
+        const f32x4 n2f = unpack4(n2);
+        f32x4 out = ZERO;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            a[head * 4 + c] = round_bf16(bf16_to_float(value[c]) * gate);
+        for (int t = 0; t < 3; ++t) {
+            const u32x2 gate_row = pack4(multiply(weight(tile + 4 + t), n2f)), up_row = pack4(multiply(weight(tile + 7 + t), n2f));
+            f32x4 act = unpack4(gate_row);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                act[r] = act[r] * sigmoid(act[r]);
+            const u32x2 act_row = pack4(rounded(act) * unpack4(up_row));
+            out = multiply(weight(tile + 10 + t), unpack4(act_row), out);
+            if (with_gradient) {
+                keep[(T_GU + t) * 64] = gate_row;
+                keep[(T_GU + 3 + t) * 64] = up_row;
+                keep[(T_ACT + t) * 64] = act_row;
+            }
+        }
+        h = rounded(rounded(out) + middle);
     }
-    float y[16], x[16];
-    matvec<16, 16>(m.hi + p.attention, a, y);
-    load_row16(rows.x + size_t(t) * W, x);
+    // final RMSNorm, head, softmax cross-entropy (cuda/model.cuh:32-58): register r of tile t is logit 16 t + 4 r + g
+    const float inv = inverse_rms(h, p);
+    const u32x2 nf = normalize(h, inv, weight.scale(2 * m.depth));
+    const f32x4 nff = unpack4(nf);
+    f32x4 logit[16];
+    float high = -INFINITY;
 #pragma unroll
-    for (int o = 0; o < 16; ++o)
-        y[o] = round_bf16(y[o]) + x[o]; // bf16 add of the residual (cuda/mma.cuh:95-97)
-    store_row16(rows.middle + size_t(t) * W, y);
-}
-
-// cuda/ops.cuh:120-131: RN after SiLU and after the product
-TG_DEVICE void swiglu_row(const float (&gu)[96], float (&activated)[48], float (&act)[48]) {
-#pragma unroll
-    for (int j = 0; j < 48; ++j) {
-        activated[j] = round_bf16(gu[j] * sigmoid(gu[j]));
-        act[j] = round_bf16(activated[j] * gu[48 + j]);
+    for (int t = 0; t < 16; ++t) {
+        logit[t] = rounded(multiply(weight(m.depth * LAYER_TILES + t), nff));
+        high = fmaxf(fmaxf(high, fmaxf(logit[t][0], logit[t][1])), fmaxf(logit[t][2], logit[t][3]));
     }
-}
-
-// RMSNorm, packed gate|up projection, SwiGLU, down projection and residual (cuda/model.cuh:22-30)
-__global__ __launch_bounds__(64) void w16_mlp_kernel(Model m, int l, LayerRows rows, bf16_t *hidden) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    float v[16], n[16], gu[96], activated[48], act[48], y[16];
-    load_row16(rows.middle + size_t(t) * W, v);
-    normalize(v, m.hi, m.lo, p.mlp_norm, n);
-    matvec<96, 16>(m.hi + p.gate, n, gu); // gate and up are adjacent (model.h:27-31)
-    bf16_t *cache = rows.gu + size_t(t) * 96;
+    high = token_max(high);
+    if (logits_out && p.live)
 #pragma unroll
-    for (int o = 0; o < 96; o += 2) {
-        *reinterpret_cast<uint32_t *>(cache + o) = pack_bf16(gu[o], gu[o + 1]);
-        gu[o] = round_bf16(gu[o]), gu[o + 1] = round_bf16(gu[o + 1]);
-    }
-    swiglu_row(gu, activated, act);
-    matvec<16, 48>(m.hi + p.down, act, y);
+        for (int t = 0; t < 16; ++t)
 #pragma unroll
-    for (int o = 0; o < 16; ++o)
-        y[o] = round_bf16(y[o]) + v[o];
-    store_row16(hidden + size_t(t) * W, y);
-}
-
-// final RMSNorm, head, softmax cross-entropy; one wave per token, a lane owns four logits
-// (cuda/model.cuh:32-58).  dlogits = RN_bf16((p - onehot) / tokens).
-__global__ __launch_bounds__(256) void w16_head_kernel(Model m, const bf16_t *__restrict__ hidden, bf16_t *nf,
-                                                       const uint8_t *__restrict__ y, float *token_losses,
-                                                       float *logits_out, bf16_t *dlogits, int with_gradient) {
-    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= m.tokens)
-        return;
-    float v[16], n[16];
-    load_row16(hidden + size_t(t) * W, v);
-    normalize(v, m.hi, m.lo, m.layout.final_norm, n);
-    if (lane == 0) {
-        float copy[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            copy[i] = n[i];
-        store_row16(nf + size_t(t) * W, copy);
-    }
-    float logit[4], high = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int o = lane + 64 * k;
-        float w[16], acc = 0.f;
-        load_row16(m.hi + m.layout.head + o * W, w);
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            acc = fmaf(n[i], w[i], acc);
-        logit[k] = round_bf16(acc);
-        high = fmaxf(high, logit[k]);
-    }
-    high = wave_max(high);
-    float sum = 0.f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        sum += expf(logit[k] - high);
-    sum = wave_sum(sum);
-    const int target = y[t];
+            for (int r = 0; r < 4; ++r)
+                logits_out[size_t(p.token) * V + t * 16 + 4 * r + p.g] = logit[t][r];
+    const int mine = target - p.g; // this lane owns the logits 16 t + 4 r of it
     float picked = 0.f;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        picked += (lane + 64 * k == target) ? logit[k] : 0.f;
-    picked = wave_sum(picked);
-    if (lane == 0)
-        token_losses[t] = high + logf(sum) - picked;
+    for (int t = 0; t < 16; ++t)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int o = lane + 64 * k;
-        if (logits_out)
-            logits_out[size_t(t) * V + o] = logit[k];
-        if (with_gradient)
-            dlogits[size_t(t) * V + o] =
-                float_to_bf16((expf(logit[k] - high) / sum - (o == target ? 1.f : 0.f)) / float(m.tokens));
+        for (int r = 0; r < 4; ++r) {
+            picked = 16 * t + 4 * r == mine ? logit[t][r] : picked;
+            logit[t][r] = expf(logit[t][r] - high);
+        }
+    // the sum's tree: every 64th logit in order, then halves of what is left (bits 5 .. 0 of the logit's number)
+    f32x4 quarter[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        quarter[q] = ((logit[q] + logit[q + 4]) + logit[q + 8]) + logit[q + 12];
+    const f32x4 sixteenth = (quarter[0] + quarter[2]) + (quarter[1] + quarter[3]);
+    const float sum = swap_add_16(swap_add_32((sixteenth[0] + sixteenth[2]) + (sixteenth[1] + sixteenth[3])));
+    picked = swap_add_16(swap_add_32(picked));
+    if (p.live && p.g == 0)
+        token_losses[p.token] = high + logf(sum) - picked;
+    if (with_gradient) {
+        s.hidden[size_t(p.wave) * 64 + p.lane] = pack4(h);
+        s.nf[size_t(p.wave) * 64 + p.lane] = nf;
+        s.inverse[size_t(p.wave) * 64 + p.lane] = inv;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            f32x4 d;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                d[r] = p.live ? (logit[t][r] / sum - (16 * t + 4 * r == mine ? 1.f : 0.f)) / float(m.tokens) : 0.f;
+            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = pack4(d);
+        }
     }
 }
 
 // ---- backward --------------------------------------------------------------------------------------
-// head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
-__global__ __launch_bounds__(64) void w16_head_backward_kernel(Model m, const bf16_t *__restrict__ hidden,
-                                                               const bf16_t *__restrict__ dlogits, bf16_t *dh,
-                                                               float *gz_final) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    float dn[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        dn[i] = 0.f;
-    const bf16_t *row = dlogits + size_t(t) * V;
-    for (int o = 0; o < V; o += 2) {
-        const uint32_t pair = *reinterpret_cast<const uint32_t *>(row + o);
-        const float d0 = bf16_lo(pair), d1 = bf16_hi(pair);
-        const bf16_t *w = m.hi + m.layout.head + o * W;
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            dn[i] = fmaf(d1, bf16_to_float(w[W + i]), fmaf(d0, bf16_to_float(w[i]), dn[i]));
-    }
-    float v[16], dx[16], gz[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        dn[i] = round_bf16(dn[i]);
-    load_row16(hidden + size_t(t) * W, v);
-    normalize_backward(v, dn, m.hi, m.lo, m.layout.final_norm, dx, gz);
-    store_row16(dh + size_t(t) * W, dx);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        gz_final[size_t(t) * W + i] = gz[i];
-}
+// cuda/model.cuh:61-99, without the weight gradients
+__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Workspace s) {
+    extern __shared__ __align__(16) unsigned char staged_memory[];
+    uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
+    float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
+    stage_weights<true>(m, staged_tiles_at, scales);
+    const Lane p = lane_of(m);
+    const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
+    const size_t here = size_t(p.wave) * 64 + p.lane;
+    auto gz = [&](int norm) { return s.gz + ((size_t(norm) * s.waves + p.wave) * 16 + p.c) * W + p.g; };
+    float rc, rs;
+    rotation(p.position, rc, rs);
 
-// down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88)
-__global__ __launch_bounds__(64) void w16_mlp_backward_kernel(Model m, int l, LayerRows rows, bf16_t *dh) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    float v[16], n[16], d[16], gu[96], activated[48], act[48], dact[48], dgu[96];
-    load_row16(rows.middle + size_t(t) * W, v);
-    load_row16(dh + size_t(t) * W, d);
-    store_row16(rows.dh_down + size_t(t) * W, d);
-    normalize(v, m.hi, m.lo, p.mlp_norm, n);
-    {
-        float copy[16];
+    // head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
+    f32x4 dn = ZERO;
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-            copy[i] = n[i];
-        store_row16(rows.n2 + size_t(t) * W, copy);
-    }
-    const bf16_t *cache = rows.gu + size_t(t) * 96;
+    for (int t = 0; t < 16; ++t)
+        dn = multiply(weight(m.depth * LAYER_TILES + t), unpack4(s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane]), dn);
+    f32x4 dh = normalize_backward(unpack4(s.hidden[here]), s.inverse[here], rounded(dn), weight.scale(2 * m.depth),
+                                  gz(2 * m.depth), p);
+    for (int l = m.depth - 1; l >= 0; --l) {
+        const int tile = l * LAYER_TILES;
+        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
+        const float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
+        // down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88, cuda/ops.cuh:133-144)
+        keep[T_DH_DOWN * 64] = pack4(dh);
+        f32x4 dgate[3], dup[3];
 #pragma unroll
-    for (int o = 0; o < 96; o += 2) {
-        const uint32_t pair = *reinterpret_cast<const uint32_t *>(cache + o);
-        gu[o] = bf16_lo(pair), gu[o + 1] = bf16_hi(pair);
-    }
-    swiglu_row(gu, activated, act);
-    bf16_t *act_out = rows.act + size_t(t) * F;
+        for (int t = 0; t < 3; ++t) {
+            const f32x4 gate = unpack4(keep[(T_GU + t) * 64]), up = unpack4(keep[(T_GU + 3 + t) * 64]);
+            const f32x4 dy = rounded(multiply(weight(tile + 10 + t), dh)), da = rounded(dy * up);
+            f32x4 silu;
 #pragma unroll
-    for (int j = 0; j < 48; j += 2)
-        *reinterpret_cast<uint32_t *>(act_out + j) = pack_bf16(act[j], act[j + 1]);
-    matvec_t<16, 48>(m.hi + p.down, d, dact);
-    // cuda/ops.cuh:133-144
-#pragma unroll
-    for (int j = 0; j < 48; ++j) {
-        const float dy = round_bf16(dact[j]), g = gu[j], u = gu[48 + j], sig = sigmoid(g);
-        const float da = round_bf16(dy * u);
-        dgu[j] = round_bf16(da * sig * (1.f + g * (1.f - sig)));
-        dgu[48 + j] = round_bf16(dy * activated[j]);
-    }
-    bf16_t *dgu_out = rows.dgu + size_t(t) * 96;
-#pragma unroll
-    for (int o = 0; o < 96; o += 2)
-        *reinterpret_cast<uint32_t *>(dgu_out + o) = pack_bf16(dgu[o], dgu[o + 1]);
-    float dn[16], dx[16], gz[16];
-    matvec_t<96, 16>(m.hi + p.gate, dgu, dn);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        dn[i] = round_bf16(dn[i]);
-    normalize_backward(v, dn, m.hi, m.lo, p.mlp_norm, dx, gz);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        d[i] = d[i] + dx[i]; // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
-        rows.gz_mlp[size_t(t) * W + i] = gz[i];
-    }
-    store_row16(dh + size_t(t) * W, d);
-    store_row16(rows.dh_attention + size_t(t) * W, d);
-}
-
-// replays the attention output from the cached winner and gate, output-projection backward and the
-// per-(token, head) score gradient (cuda/model.cuh:89-91, cuda/attention.cuh:72-85)
-__global__ __launch_bounds__(64) void w16_attention_backward_a_kernel(Model m, int l, LayerRows rows,
-                                                                      const bf16_t *__restrict__ dh, bf16_t *dattn,
-                                                                      float *dt) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    float d[16], a[16], da[16], value[16];
-    load_row16(dh + size_t(t) * W, d);
-#pragma unroll
-    for (int head = 0; head < HEADS; ++head) {
-        const int key = rows.selected[size_t(t) * HEADS + head];
-        const float gate = rows.gates[size_t(t) * HEADS + head];
-        const bf16_t *vrow = rows.qkv + size_t(key) * 48 + 32 + head * 4;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            value[head * 4 + c] = bf16_to_float(vrow[c]);
-            a[head * 4 + c] = value[head * 4 + c] * gate;
-        }
-    }
-    store_row16(rows.a + size_t(t) * W, a);
-    matvec_t<16, 16>(m.hi + p.attention, d, da);
-    store_row16(dattn + size_t(t) * W, da);
-#pragma unroll
-    for (int head = 0; head < HEADS; ++head) {
-        float sum = 0.f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            sum += da[head * 4 + c] * value[head * 4 + c];
-        dt[size_t(t) * HEADS + head] = sum * rows.derivatives[size_t(t) * HEADS + head];
-    }
-}
-
-// query / key / value gradients by gathering over the sequence (no atomics), inverse RoPE, QKV
-// projection and RMSNorm backward (cuda/attention.cuh:86-106, cuda/model.cuh:92-96)
-__global__ __launch_bounds__(64) void w16_attention_backward_b_kernel(Model m, int l, LayerRows rows,
-                                                                      const bf16_t *__restrict__ dattn,
-                                                                      const float *__restrict__ dt, bf16_t *dh) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= m.tokens)
-        return;
-    const Layer &p = m.layout.layers[l];
-    const int start = t / m.context * m.context;
-    float dqkv[48];
-#pragma unroll
-    for (int head = 0; head < HEADS; ++head) {
-        const int key = rows.selected[size_t(t) * HEADS + head];
-        const float mine = dt[size_t(t) * HEADS + head];
-        const bf16_t *krow = rows.qkv + size_t(key) * 48 + 16 + head * 4;
-        float dk[4] = {0.f, 0.f, 0.f, 0.f}, dv[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            dqkv[head * 4 + c] = mine * bf16_to_float(krow[c]);
-        for (int query = start; query < start + m.context; ++query) {
-            if (rows.selected[size_t(query) * HEADS + head] != t)
-                continue;
-            const float their = dt[size_t(query) * HEADS + head], gate = rows.gates[size_t(query) * HEADS + head];
-            const bf16_t *qrow = rows.qkv + size_t(query) * 48 + head * 4;
-            const bf16_t *drow = dattn + size_t(query) * W + head * 4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                dk[c] += their * bf16_to_float(qrow[c]);
-                dv[c] += bf16_to_float(drow[c]) * gate;
+            for (int r = 0; r < 4; ++r) {
+                const float g = gate[r], sig = sigmoid(g);
+                silu[r] = g * sig;
+                dgate[t][r] = da[r] * sig * (1.f + g * (1.f - sig));
             }
+            const u32x2 dgate_row = pack4(dgate[t]), dup_row = pack4(dy * rounded(silu));
+            keep[(T_DGU + t) * 64] = dgate_row;
+            keep[(T_DGU + 3 + t) * 64] = dup_row;
+            dgate[t] = unpack4(dgate_row), dup[t] = unpack4(dup_row);
         }
+        dn = ZERO;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            dqkv[16 + head * 4 + c] = dk[c];
-            dqkv[32 + head * 4 + c] = dv[c];
-        }
+        for (int t = 0; t < 3; ++t)
+            dn = multiply(weight(tile + 4 + t), dgate[t], dn);
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            dn = multiply(weight(tile + 7 + t), dup[t], dn);
+        // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
+        dh = rounded(dh + normalize_backward(unpack4(keep[T_MIDDLE * 64]), words[WORD_INV2 * 64], rounded(dn),
+                                             weight.scale(2 * l + 1), gz(2 * l + 1), p));
+        keep[T_DH_ATTENTION * 64] = pack4(dh);
+
+        // attention: output projection backward, the score gradient of the cached winner, query / key / value gradients
+        // gathered over the sequence, inverse RoPE, QKV projection and RMSNorm backward (cuda/model.cuh:89-96,
+        // cuda/attention.cuh:72-106)
+        const u32x2 query = keep[T_Q * 64];
+        const f32x4 key = unpack4(keep[T_KEY * 64]), value = unpack4(keep[T_VALUE * 64]);
+        const float gate = words[WORD_GATE * 64], slope = words[WORD_SLOPE * 64];
+        const int distance = __float_as_int(words[WORD_DISTANCE * 64]);
+        const u32x2 dattn = pack4(multiply(weight(tile + 3), dh));
+        const f32x4 da = unpack4(dattn);
+        float dt = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            dt = fmaf(da[c], value[c], dt);
+        dt *= slope;
+        f32x4 dk = ZERO, dv = ZERO;
+        up_to<0, 7>([&](auto step) { // queries of this token's sequence that chose it, in order
+            constexpr int D = decltype(step)::value;
+            if (D >= m.context)
+                return;
+            // every lane takes part in the shifts, so none of them may sit behind a condition
+            const uint32_t theirs = later<D>(uint32_t(distance));
+            const float their_dt = __uint_as_float(later<D>(__float_as_uint(dt))), their_gate = __uint_as_float(later<D>(__float_as_uint(gate)));
+            const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
+            const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
+            const bool chose = p.position + D < m.context && theirs == uint32_t(D);
+            const float t = chose ? their_dt : 0.f, g = chose ? their_gate : 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                dk[r] = fmaf(t, qf[r], dk[r]);
+                dv[r] = fmaf(df[r], g, dv[r]);
+            }
+        });
+        const f32x4 dq = turned(rounded(rotate_back(rounded(key * dt), rc, rs)));
+        dk = turned(rounded(rotate_back(rounded(dk), rc, rs)));
+        dv = turned(rounded(dv));
+        keep[T_DQKV * 64] = pack4(dq);
+        keep[(T_DQKV + 1) * 64] = pack4(dk);
+        keep[(T_DQKV + 2) * 64] = pack4(dv);
+        dn = multiply(weight(tile + 2), dv, multiply(weight(tile + 1), dk, multiply(weight(tile), dq)));
+        dh = rounded(dh + normalize_backward(unpack4(keep[T_X * 64]), words[WORD_INV1 * 64], rounded(dn),
+                                             weight.scale(2 * l), gz(2 * l), p));
     }
-#pragma unroll
-    for (int o = 0; o < 48; ++o)
-        dqkv[o] = round_bf16(dqkv[o]);
-    rotate(dqkv, t % m.context, true);
-    bf16_t *out = rows.dqkv + size_t(t) * 48;
-#pragma unroll
-    for (int o = 0; o < 48; o += 2)
-        *reinterpret_cast<uint32_t *>(out + o) = pack_bf16(dqkv[o], dqkv[o + 1]);
-    float v[16], n[16], d[16], dn[16], dx[16], gz[16];
-    load_row16(rows.x + size_t(t) * W, v);
-    normalize(v, m.hi, m.lo, p.attention_norm, n);
-    store_row16(rows.n1 + size_t(t) * W, n);
-    matvec_t<48, 16>(m.hi + p.qkv, dqkv, dn);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        dn[i] = round_bf16(dn[i]);
-    normalize_backward(v, dn, m.hi, m.lo, p.attention_norm, dx, gz);
-    load_row16(dh + size_t(t) * W, d);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        d[i] = d[i] + dx[i];
-        rows.gz_attention[size_t(t) * W + i] = gz[i];
-    }
-    store_row16(dh + size_t(t) * W, d);
+    s.dh[here] = pack4(dh);
 }
 
-// ---- weight gradients: one job per parameter tensor ----------------------------------------------------
-enum JobKind { JOB_OUTER = 0, JOB_COLUMN_SUM = 1, JOB_EMBEDDING = 2 };
-struct Job {
-    const void *dy; // OUTER: bf16 [tokens][ld_dy]; COLUMN_SUM: float [tokens][16]; EMBEDDING: uint8 token ids
-    const bf16_t *x; // OUTER: bf16 [tokens][ld_x]; EMBEDDING: bf16 [tokens][16]
-    int ld_dy, ld_x, out, in, offset, kind;
-};
-constexpr int MAX_JOBS = 3 + MAX_DEPTH * 6;
-struct Jobs {
-    Job job[MAX_JOBS];
-    int count;
-};
-// partial[chunk][offset + o*in + i] = sum over the chunk's tokens, in token order.  A thread owns output row o
-// and a 16-wide slab of inputs: per token it reads one dy value and one 32-byte row piece that every thread of
-// the same slab shares, and keeps 16 sums in registers.  (The widest jobs, head and embedding, are 256 x 16.)
-__global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Jobs jobs, int tokens, int parameters, float *partials) {
-    const Job &job = jobs.job[blockIdx.y];
-    const int first = blockIdx.x * CHUNK, last = min(first + CHUNK, tokens);
-    const int slabs = job.in >> 4, o = threadIdx.x / slabs, slab = threadIdx.x - o * slabs;
-    if (o >= job.out)
+// ---- weight gradients ------------------------------------------------------------------------------
+// A wave sums one 16 x 16 tile of one parameter tensor (or one RMSNorm scale) over the tokens of a chunk, in token order:
+// partial[chunk][parameter].  Jobs: 13 matrix tiles and 2 scales a layer, the head's and the embedding's 16, the final norm.
+constexpr int LAYER_JOBS = 15;
+__host__ __device__ constexpr int gradient_jobs(int depth) { return depth * LAYER_JOBS + 33; }
+__global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const uint8_t *__restrict__ x, Workspace s,
+                                                                  int parameters) {
+    const int job = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (job >= gradient_jobs(m.depth))
         return;
-    float acc[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-        acc[k] = 0.f;
-    if (job.kind == JOB_OUTER) {
-        const bf16_t *dy = static_cast<const bf16_t *>(job.dy) + o;
-        const bf16_t *x = job.x + slab * 16;
-        for (int t = first; t < last; ++t) {
-            const float d = bf16_to_float(dy[size_t(t) * job.ld_dy]);
-            float v[16];
-            load_row16(x + size_t(t) * job.ld_x, v);
-#pragma unroll
-            for (int k = 0; k < 16; ++k)
-                acc[k] = fmaf(d, v[k], acc[k]);
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int first = blockIdx.y * CHUNK_WAVES, last = min(first + CHUNK_WAVES, s.waves);
+    float *out = s.partials + size_t(blockIdx.y) * parameters;
+    // A row operand (rows of the gradient tile) and a column operand, as tiles of tokens x 16 features in feed layout
+    const u32x2 *rows = nullptr, *cols = nullptr;
+    size_t row_stride = 64, col_stride = 64; // from one wave's tile to the next
+    int width = W, norm = -1, vocabulary = -1;
+    if (job < m.depth * LAYER_JOBS) {
+        const int l = job / LAYER_JOBS, k = job - l * LAYER_JOBS;
+        const Layer q = layer_layout(l);
+        const u32x2 *keep = s.tiles + size_t(l) * s.waves * TILES * 64;
+        row_stride = col_stride = TILES * 64;
+        if (k < 3) {
+            rows = keep + (T_DQKV + k) * 64, cols = keep + T_N1 * 64, out += q.qkv + k * 256;
+        } else if (k == 3) {
+            rows = keep + T_DH_ATTENTION * 64, cols = keep + T_A * 64, out += q.attention;
+        } else if (k < 10) {
+            rows = keep + (T_DGU + k - 4) * 64, cols = keep + T_N2 * 64, out += q.gate + (k - 4) * 256; // gate, then up
+        } else if (k < 13) {
+            rows = keep + T_DH_DOWN * 64, cols = keep + (T_ACT + k - 10) * 64, out += q.down + (k - 10) * 16, width = F;
+        } else {
+            norm = 2 * l + k - 13, out += k == 13 ? q.attention_norm : q.mlp_norm;
         }
-    } else if (job.kind == JOB_COLUMN_SUM) {
-        const float *gz = static_cast<const float *>(job.dy);
-        for (int t = first; t < last; ++t)
-#pragma unroll
-            for (int k = 0; k < 16; ++k)
-                acc[k] += gz[size_t(t) * W + k];
     } else {
-        const uint8_t *ids = static_cast<const uint8_t *>(job.dy);
-        for (int t = first; t < last; ++t) {
-            if (ids[t] != o)
-                continue;
-            float v[16];
-            load_row16(job.x + size_t(t) * W, v);
-#pragma unroll
-            for (int k = 0; k < 16; ++k)
-                acc[k] += v[k];
+        const int k = job - m.depth * LAYER_JOBS;
+        if (k < 16) {
+            rows = s.dlogits + k * 64, row_stride = 16 * 64, cols = s.nf, out += V * W + m.depth * LAYER_SIZE + W + k * 256;
+        } else if (k < 32) { // embedding rows: the one-hot matrix of the tokens times the gradient
+            vocabulary = (k - 16) * 16 + c, cols = s.dh, out += (k - 16) * 256;
+        } else {
+            norm = 2 * m.depth, out += V * W + m.depth * LAYER_SIZE;
         }
     }
-    float *out = partials + size_t(blockIdx.x) * parameters + job.offset + o * job.in + slab * 16;
+    f32x4 acc = ZERO;
+    if (norm >= 0) { // a row of ones times the g * z terms
+        const float *gz = s.gz + (size_t(norm) * s.waves + first) * 16 * W + lane;
+        for (int w = first; w < last; ++w, gz += 16 * W) {
+            float v[4];
 #pragma unroll
-    for (int k = 0; k < 16; k += 4)
-        *reinterpret_cast<f32x4 *>(out + k) = f32x4{acc[k], acc[k + 1], acc[k + 2], acc[k + 3]};
+            for (int j = 0; j < 4; ++j)
+                v[j] = gz[j * 64]; // token 4 j + g, feature c
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, v[j], acc, 0, 0, 0);
+        }
+        if (g == 0)
+            out[c] = acc[0];
+        return;
+    }
+    // a feed-layout tile times the identity, on the bf16 instruction (exact: one product a sum), comes out as feature c of
+    // tokens 4 g + r; turned, register j is token 4 j + g: step j of a product over tokens
+    u32x2 identity;
+    identity.x = (g == c ? 0x3f80u : 0u) | (4 + g == c ? 0x3f800000u : 0u);
+    identity.y = (8 + g == c ? 0x3f80u : 0u) | (12 + g == c ? 0x3f800000u : 0u);
+    auto by_token = [&](const u32x2 &tile) {
+        return turned(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, tile), __builtin_bit_cast(s16x4, identity), ZERO, 0, 0, 0));
+    };
+    for (int w = first; w < last; ++w) {
+        const f32x4 col = by_token(cols[size_t(w) * col_stride + lane]);
+        f32x4 row;
+        if (vocabulary >= 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int t = 4 * j + g, token = w * m.per_wave + t; // rows beyond the last token are zero: any id will do
+                row[j] = t < m.per_wave && token < m.tokens && x[token] == vocabulary ? 1.f : 0.f;
+            }
+        } else {
+            row = by_token(rows[size_t(w) * row_stride + lane]);
+        }
+        acc = multiply(row, col, acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        out[(4 * g + r) * width + c] = acc[r];
 }
-__global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
-                                                       float *gradient) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+// gradient = the chunks' sums in chunk order
+__global__ __launch_bounds__(64) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
+                                                      float *__restrict__ gradient) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= parameters)
         return;
     float sum = 0.f;
+#pragma unroll 16
     for (int c = 0; c < chunks; ++c)
         sum += partials[size_t(c) * parameters + i];
     gradient[i] = sum;
@@ -741,7 +761,7 @@ void check_shape(int depth, int batch, int context) {
     require(int64_t(batch) * context <= (1 << 24), "w16: too many tokens");
 }
 Model make_model(int depth, int batch, int context, const uint16_t *hi, const uint16_t *lo) {
-    return Model{hi, lo, make_layout(depth), batch * context, context};
+    return Model{hi, lo, depth, batch * context, context, tokens_per_wave(context)};
 }
 
 } // namespace
@@ -753,7 +773,7 @@ extern "C" int tgk_w16_parameter_count(int depth) {
 extern "C" size_t tgk_w16_workspace(int depth, int batch, int context) {
     if (depth < 1 || depth > MAX_DEPTH || batch < 1 || context < 1 || context > 8)
         return 0;
-    return carve(depth, batch * context, nullptr).bytes;
+    return carve(depth, batch, context, nullptr).bytes;
 }
 
 extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int context, const uint16_t *weight_hi,
@@ -763,17 +783,10 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && y && workspace && token_losses, "w16_forward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
-        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
-        const Rows r = carve(depth, m.tokens, workspace);
-        const dim3 per_token((m.tokens + 63) / 64), wave(64);
-        hipLaunchKernelGGL(w16_embed_kernel, per_token, wave, 0, stream, m, x, r.hidden);
-        for (int l = 0; l < depth; ++l) {
-            hipLaunchKernelGGL(w16_qkv_kernel, per_token, wave, 0, stream, m, l, r.hidden, r.layer[l]);
-            hipLaunchKernelGGL(w16_attention_kernel, per_token, wave, 0, stream, m, l, r.layer[l]);
-            hipLaunchKernelGGL(w16_mlp_kernel, per_token, wave, 0, stream, m, l, r.layer[l], r.hidden);
-        }
-        hipLaunchKernelGGL(w16_head_kernel, dim3((m.tokens + 3) / 4), dim3(256), 0, stream, m, r.hidden, r.nf, y,
-                           token_losses, logits, r.dlogits, with_gradient);
+        const Workspace r = carve(depth, batch, context, workspace);
+        hipLaunchKernelGGL(w16_forward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream,
+                           make_model(depth, batch, context, weight_hi, weight_lo), x, y, r, token_losses, logits,
+                           with_gradient);
         check_hip(hipGetLastError(), "w16_forward launch: ");
     });
 }
@@ -784,40 +797,14 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && workspace && gradient, "w16_backward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
+        const Workspace r = carve(depth, batch, context, workspace);
+        const int parameters = make_layout(depth).count;
         const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
-        const Rows r = carve(depth, m.tokens, workspace);
-        const dim3 per_token((m.tokens + 63) / 64), wave(64);
-        hipLaunchKernelGGL(w16_head_backward_kernel, per_token, wave, 0, stream, m, r.hidden, r.dlogits, r.dh, r.gz_final);
-        for (int l = depth - 1; l >= 0; --l) {
-            hipLaunchKernelGGL(w16_mlp_backward_kernel, per_token, wave, 0, stream, m, l, r.layer[l], r.dh);
-            hipLaunchKernelGGL(w16_attention_backward_a_kernel, per_token, wave, 0, stream, m, l, r.layer[l], r.dh, r.dattn,
-                               r.dt);
-            hipLaunchKernelGGL(w16_attention_backward_b_kernel, per_token, wave, 0, stream, m, l, r.layer[l], r.dattn, r.dt,
-                               r.dh);
-        }
-        Jobs jobs{};
-        auto add = [&](const void *dy, int ld_dy, const bf16_t *xs, int ld_x, int out, int in, int offset, int kind) {
-            jobs.job[jobs.count++] = Job{dy, xs, ld_dy, ld_x, out, in, offset, kind};
-        };
-        const Layout &p = m.layout;
-        add(x, 0, r.dh, W, V, W, p.embedding, JOB_EMBEDDING);
-        for (int l = 0; l < depth; ++l) {
-            const LayerRows &b = r.layer[l];
-            const Layer &q = p.layers[l];
-            add(b.gz_attention, W, nullptr, 0, 1, W, q.attention_norm, JOB_COLUMN_SUM);
-            add(b.dqkv, 3 * W, b.n1, W, 3 * W, W, q.qkv, JOB_OUTER);
-            add(b.dh_attention, W, b.a, W, W, W, q.attention, JOB_OUTER);
-            add(b.gz_mlp, W, nullptr, 0, 1, W, q.mlp_norm, JOB_COLUMN_SUM);
-            add(b.dgu, 2 * F, b.n2, W, 2 * F, W, q.gate, JOB_OUTER); // gate and up are adjacent: one packed job
-            add(b.dh_down, W, b.act, F, W, F, q.down, JOB_OUTER);
-        }
-        add(r.gz_final, W, nullptr, 0, 1, W, p.final_norm, JOB_COLUMN_SUM);
-        add(r.dlogits, V, r.nf, W, V, W, p.head, JOB_OUTER);
-        const int chunks = (m.tokens + CHUNK - 1) / CHUNK;
-        hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3(chunks, jobs.count), dim3(256), 0, stream, jobs, m.tokens,
-                           p.count, r.partials);
-        hipLaunchKernelGGL(w16_fold_kernel, dim3((p.count + 255) / 256), dim3(256), 0, stream, r.partials, chunks,
-                           p.count, gradient);
+        hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
+        hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(depth) + 3) / 4, r.chunks), dim3(256), 0, stream,
+                           m, x, r, parameters);
+        hipLaunchKernelGGL(w16_fold_kernel, dim3((parameters + 63) / 64), dim3(64), 0, stream, r.partials, r.chunks,
+                           parameters, gradient);
         check_hip(hipGetLastError(), "w16_backward launch: ");
     });
 }
