@@ -70,6 +70,12 @@ TG_DEVICE float gelu_grad_f(float x) {
     const float cdf = x < 0.f ? g.tail : 1.0f - g.tail;
     return fmaf(x * g.e, 0.39894228040143268f, cdf);
 }
+TG_DEVICE uint64_t hash_u64(uint64_t x) { // utils.h:13-18
+    x += 0x9e3779b97f4a7c15ULL;
+    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ULL;
+    x = (x ^ (x >> 27)) * 0x94d049bb133111ebULL;
+    return x ^ (x >> 31);
+}
 TG_DEVICE float wave_sum(float x) {
 #pragma unroll
     for (int k = 32; k; k >>= 1)

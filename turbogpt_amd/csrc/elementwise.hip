@@ -3,6 +3,7 @@
 // function of the reference named at its entry point.  All are single pass over their operands
 // with 16-byte accesses; reductions use a fixed order (no atomics), so results are reproducible.
 #include "common.h"
+#include "optimizer.h"
 #include "../../include/tgk_kernels.h"
 
 namespace {
@@ -34,13 +35,6 @@ TG_DEVICE void join8(const u32x4 &h, const u32x4 &l, float (&f)[8]) {
 TG_DEVICE void join8(const uint16_t *hi, const uint16_t *lo, float (&f)[8]) {
     join8(*reinterpret_cast<const u32x4 *>(hi), *reinterpret_cast<const u32x4 *>(lo), f);
 }
-TG_DEVICE uint64_t hash_u64(uint64_t x) { // utils.h:13-18
-    x += 0x9e3779b97f4a7c15ULL;
-    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ULL;
-    x = (x ^ (x >> 27)) * 0x94d049bb133111ebULL;
-    return x ^ (x >> 31);
-}
-
 // ---- embedding ------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void embed_fwd_kernel(const uint8_t *__restrict__ x,
                                                         const bf16_t *__restrict__ table,
@@ -476,7 +470,7 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const float *__restrict__ g,
     const size_t quads = n >> 2;
     for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < quads; i += size_t(gridDim.x) * 256) {
         const f32x4 v = *reinterpret_cast<const f32x4 *>(g + i * 4);
-        sum += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+        sum += quad_squares(v);
     }
     if (blockIdx.x == 0 && threadIdx.x < int(n & 3)) {
         const float v = g[(quads << 2) + threadIdx.x];
@@ -516,9 +510,6 @@ __global__ __launch_bounds__(256) void sumsq_segments_kernel(const float *__rest
         partial[blockIdx.x] = (waves[0] + waves[1]) + (waves[2] + waves[3]);
 }
 
-struct AdamArgs {
-    float lr, beta1, beta2, eps, weight_decay, bc1, sqrt_bc2, clip;
-};
 // cuda/optim.cuh:67-106 on the (hi bf16, lo u16) weight halves (cuda/ops.cuh:6-14).
 // bounds: sorted starts of `segments` parameter ranges, bit 0 of flags[s] = weight decay, bit 1 = skip.
 __global__ __launch_bounds__(256) void adamw_kernel(bf16_t *__restrict__ hi, uint16_t *__restrict__ lo,
@@ -529,22 +520,7 @@ __global__ __launch_bounds__(256) void adamw_kernel(bf16_t *__restrict__ hi, uin
                                                     const uint8_t *__restrict__ flags, int segments,
                                                     AdamArgs a) {
     __shared__ float waves[4];
-    __shared__ float clip_scale;
-    float scale = 1.f;
-    if (a.clip > 0.f) {
-        // every block folds the same partials in the same order (cuda/optim.cuh:67-80)
-        float sum = 0.f;
-        for (int i = threadIdx.x; i < norm_count; i += 256)
-            sum += norm_partials[i];
-        sum = wave_sum(sum);
-        if ((threadIdx.x & 63) == 0)
-            waves[threadIdx.x >> 6] = sum;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            clip_scale = fminf(1.f, a.clip / (sqrtf((waves[0] + waves[1]) + (waves[2] + waves[3])) + 1e-6f));
-        __syncthreads();
-        scale = clip_scale;
-    }
+    const float scale = clip_factor(a.clip, norm_partials, norm_count, waves);
     // Every stream here is touched once per step: non-temporal loads and stores keep 3 GB of optimizer state from
     // evicting what the next step's first kernels read (measured -0.6 % on the step).
     const size_t quads = n >> 2;
@@ -568,13 +544,10 @@ __global__ __launch_bounds__(256) void adamw_kernel(bf16_t *__restrict__ hi, uin
                             (hv.y << 16) | (lv.y & 0xffffu), (hv.y & 0xffff0000u) | (lv.y >> 16)};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const float gk = gv[k] * scale;
-            const float mk = mv[k] + (1.f - a.beta1) * (gk - mv[k]);
-            const float vk = a.beta2 * vv[k] + (1.f - a.beta2) * gk * gk;
+            float mk = mv[k], vk = vv[k];
+            bits[k] = __float_as_uint(adamw_element(a, decay, scale, __uint_as_float(bits[k]), mk, vk, gv[k]));
             mv[k] = mk;
             vv[k] = vk;
-            const float w = __uint_as_float(bits[k]) * (1.f - a.lr * decay);
-            bits[k] = __float_as_uint(w - (a.lr / a.bc1) * mk / (sqrtf(vk) / a.sqrt_bc2 + a.eps));
         }
         __builtin_nontemporal_store(mv, reinterpret_cast<f32x4 *>(m + i));
         __builtin_nontemporal_store(vv, reinterpret_cast<f32x4 *>(v + i));
@@ -602,22 +575,25 @@ __global__ __launch_bounds__(256) void sample_batch_kernel(const uint8_t *__rest
         y[size_t(b) * context + p] = data[e - context + p + 1];
     }
 }
-// cuda/trainer.cuh:79-100: mean over the batch per position, accumulated in double
+// cuda/trainer.cuh:79-100: mean over the batch per position, accumulated in double: a block a position, every thread
+// each 256th sequence (a wave a position took 11 us for the width-16 network's 2560 sequences of 4), a fixed tree on top
 __global__ __launch_bounds__(256) void position_means_kernel(const float *__restrict__ token_loss,
                                                              int batch, int context,
                                                              float *__restrict__ out) {
-    // one wave per position: a lane sums every 64th sequence, then the lanes are folded in a fixed tree
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (p >= context)
-        return;
+    __shared__ double waves[4];
+    const int p = blockIdx.x;
     double sum = 0;
-    for (int b = lane; b < batch; b += 64)
+#pragma unroll 4
+    for (int b = threadIdx.x; b < batch; b += 256)
         sum += token_loss[size_t(b) * context + p];
 #pragma unroll
     for (int k = 32; k; k >>= 1)
         sum += __shfl_xor(sum, k, 64);
-    if (lane == 0)
-        out[p] = float(sum / batch);
+    if ((threadIdx.x & 63) == 0)
+        waves[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        out[p] = float(((waves[0] + waves[1]) + (waves[2] + waves[3])) / batch);
 }
 
 // ---- batched bf16 transposes ------------------------------------------------------------------
@@ -931,9 +907,7 @@ extern "C" int tgk_adamw(hipStream_t stream, size_t n, uint16_t *weight_hi, uint
         aligned(g, "adamw: g");
         require(segment_starts && segment_flags && segments > 0, "adamw: missing segment table");
         require(!(clip > 0.f) || (norm_partials && norm_count > 0), "adamw: clipping needs the norm partials");
-        // bias correction with the current beta1 (cuda/optim.cuh:90-91), evaluated on the host in fp32
-        AdamArgs a{lr, beta1, beta2, eps, weight_decay, 1.f - powf(beta1, float(step + 1)),
-                   sqrtf(1.f - powf(beta2, float(step + 1))), clip};
+        const AdamArgs a = adam_args(lr, beta1, beta2, eps, weight_decay, clip, step);
         hipLaunchKernelGGL(adamw_kernel, dim3(grid_for(n / 4, 256, 8192)), dim3(256), 0, stream, weight_hi,
                            weight_lo, m, v, g, n, norm_partials, norm_count, segment_starts, segment_flags,
                            segments, a);
@@ -957,7 +931,7 @@ extern "C" int tgk_position_means(hipStream_t stream, const float *token_loss, i
                                   float *out) {
     return guarded([&] {
         require(token_loss && out && batch > 0 && context > 0, "position_means: missing operand");
-        hipLaunchKernelGGL(position_means_kernel, dim3((context + 3) / 4), dim3(256), 0, stream, token_loss,
+        hipLaunchKernelGGL(position_means_kernel, dim3(context), dim3(256), 0, stream, token_loss,
                            batch, context, out);
         check_hip(hipGetLastError(), "position_means launch: ");
     });

@@ -5,6 +5,7 @@
 // cuda/model.cuh:8-99).  All arithmetic is in the tgk_* kernels; this file only sequences them.
 #include "common.h"
 #include "readback.h"
+#include "width16.h"
 #include "../../include/tg_model.h"
 #include "../../include/tgk_kernels.h"
 #include <algorithm>
@@ -382,9 +383,9 @@ struct Engine {
     }
 
     // cuda/optim.cuh:66-106 for optimizer step `at` (0-based), on the engine's stream: gradient -> the weights of
-    // version `to` (which already hold the previous version's values)
+    // version `to`, from the previous version's, `now`.
     // `from`: the slot whose backward pass has just written `gradient`, when it left the sums of squares with it
-    void optimize(uint64_t at, const float *gradient, Version &to, const Slot *from = nullptr) {
+    void optimize(uint64_t at, const float *gradient, const Version &now, Version &to, const Slot *from = nullptr) {
         const Config &c = config.base;
         uint16_t *weight_hi = to.hi, *weight_lo = to.lo, *weight_t = to.t;
         float lr = c.learning_rate, beta1 = c.beta1, muon_lr = c.muon_lr, muon_momentum = c.momentum;
@@ -393,17 +394,26 @@ struct Engine {
             muon_lr *= schedule[at].multiplier;
             beta1 = muon_momentum = schedule[at].momentum;
         }
-        const bool fused = from && from->norms && list_wgrad;
+        const bool fused = from && from->norms;
         if (c.clip > 0 && !fused)
             OP(TG_CLASS_OPTIMIZER, tgk_sumsq_partials(stream, gradient, size_t(layout.count), norm_partials, NormPartials));
-        OP(TG_CLASS_OPTIMIZER, tgk_adamw(stream, size_t(layout.count), weight_hi, weight_lo, momentum, variance, gradient,
-                     fused ? from->norms : norm_partials, fused ? from->list_norms + from->range_norms : NormPartials,
-                     segment_starts, segment_flags, segments, lr, beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at));
-        if (width16) { // the hidden matrices, which the AdamW segments skip (cuda/optim.cuh:107-118)
-            OP(TG_CLASS_OPTIMIZER, tgk_w16_muon(stream, c.depth, weight_hi, weight_lo, momentum, gradient, norm_partials,
-                                                NormPartials, c.clip, muon_lr, muon_momentum, c.weight_decay, c.ns_steps));
+        const float *norms = fused ? from->norms : norm_partials;
+        const int norm_count = fused ? from->list_norms + from->range_norms : NormPartials;
+        if (width16) { // AdamW's tensors and the hidden matrices (cuda/optim.cuh:92-118)
+            Scope profile_scope(this, TG_CLASS_OPTIMIZER);
+            w16_update(stream, c.depth, {now.hi, now.lo}, {to.hi, to.lo}, momentum, variance, gradient, norms, norm_count,
+                       adam_args(lr, beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at),
+                       {muon_lr, muon_momentum, c.weight_decay, c.ns_steps});
             return;
         }
+        if (&now != &to) {
+            const size_t bytes = size_t(layout.count) * 2;
+            check_hip(hipMemcpyAsync(to.hi, now.hi, bytes, hipMemcpyDeviceToDevice, stream));
+            check_hip(hipMemcpyAsync(to.lo, now.lo, bytes, hipMemcpyDeviceToDevice, stream));
+        }
+        OP(TG_CLASS_OPTIMIZER, tgk_adamw(stream, size_t(layout.count), weight_hi, weight_lo, momentum, variance, gradient,
+                     norms, norm_count, segment_starts, segment_flags, segments, lr, beta1, c.beta2, c.epsilon, c.weight_decay,
+                     c.clip, at));
         OP(TG_CLASS_OPTIMIZER, tgk_transpose_batch(stream, weight_hi, weight_t, transpose_jobs, transpose_count,
                                                    transpose_tiles));
     }
@@ -411,6 +421,12 @@ struct Engine {
     void batch_gradient(Slot &s, const Version &v, uint64_t at, float *history_row) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
+        if (width16) {
+            Scope profile_scope(this, TG_CLASS_OTHER);
+            w16_gradient(stream, c.depth, c.batch, c.context, {v.hi, v.lo}, {data, data_size, c.seed, at}, s.input, s.workspace,
+                         s.token_losses, history_row, s.gradient, s.norms);
+            return;
+        }
         OP(TG_CLASS_OTHER, tgk_sample_batch(stream, data, data_size, c.seed, at, c.batch, c.context, s.input, s.target));
         forward(s, v, true, nullptr, c.batch);
         OP(TG_CLASS_OTHER, tgk_position_means(stream, s.token_losses, c.batch, c.context, history_row));
@@ -426,7 +442,7 @@ struct Engine {
         const uint64_t K = slots.size(), ring = versions.size();
         if (K == 1) {
             batch_gradient(slots[0], versions[0], at, history_row);
-            optimize(at, slots[0].gradient, versions[0], &slots[0]);
+            optimize(at, slots[0].gradient, versions[0], versions[0], &slots[0]);
             *trace = int(at);
             return;
         }
@@ -437,10 +453,7 @@ struct Engine {
         check_hip(hipEventRecord(s.ready, s.stream));
         Version &from = versions[at % ring], &to = versions[(at + 1) % ring];
         check_hip(hipStreamWaitEvent(stream, s.ready, 0));
-        const size_t bytes = size_t(layout.count) * 2;
-        check_hip(hipMemcpyAsync(to.hi, from.hi, bytes, hipMemcpyDeviceToDevice, stream));
-        check_hip(hipMemcpyAsync(to.lo, from.lo, bytes, hipMemcpyDeviceToDevice, stream));
-        optimize(at, s.gradient, to, &s);
+        optimize(at, s.gradient, from, to, &s);
         check_hip(hipEventRecord(to.done, stream));
         *trace = int(read);
         total_staleness += at - read;
@@ -601,40 +614,13 @@ TG_API Engine *tg_create(const Config *c) {
         e->allocate(e->norm_partials, NormPartials);
         e->allocate(e->loss_history, size_t(MaxLaunchSteps) * c->context);
         e->allocate(e->batch_means, size_t(c->context));
-        // AdamW owns the embedding, the RMSNorm scales and the head (decayed); Muon the hidden matrices
-        // (cuda/optim.cuh:5-15).  Flat order per layer (model.h:20-31): scale 16, qkv 768, attention 256, scale 16,
-        // gate 768, up 768, down 768.
-        std::vector<int64_t> starts;
-        std::vector<uint8_t> flags;
-        int64_t at = 0;
-        const auto add = [&](int64_t size, uint8_t flag) {
-            if (flags.empty() || flags.back() != flag) {
-                starts.push_back(at);
-                flags.push_back(flag);
-            }
-            at += size;
-        };
-        add(256 * 16, 0);
-        for (int l = 0; l < c->depth; ++l) {
-            add(16, 0);
-            add(48 * 16 + 16 * 16, 2);
-            add(16, 0);
-            add(3 * 48 * 16, 2);
-        }
-        add(16, 0);
-        add(256 * 16, 1);
-        if (at != int64_t(P))
-            throw std::runtime_error("internal: width-16 segment table does not cover the parameters");
-        e->segments = int(starts.size());
-        e->allocate(e->segment_starts, starts.size(), false);
-        e->allocate(e->segment_flags, flags.size(), false);
-        e->upload(e->segment_starts, starts.data(), starts.size());
-        e->upload(e->segment_flags, flags.data(), flags.size());
         e->workspace_bytes = tgk_w16_workspace(c->depth, c->batch, c->context);
         for (Slot &slot : e->slots) {
             uint8_t *ws = nullptr;
             e->allocate(ws, e->workspace_bytes, false);
             slot.workspace = ws;
+            slot.list_norms = w16_norm_count(c->depth);
+            e->allocate(slot.norms, size_t(slot.list_norms));
         }
         e->sync();
         return e;
@@ -1070,7 +1056,7 @@ TG_API int tg_optimizer_test(Engine *e, const float *gradient, int steps) {
         e->use_device();
         e->upload(e->slots[0].gradient, gradient, size_t(e->layout.count));
         for (int i = 0; i < steps; ++i)
-            e->optimize(e->step + uint64_t(i), e->slots[0].gradient, e->versions[0]);
+            e->optimize(e->step + uint64_t(i), e->slots[0].gradient, e->versions[0], e->versions[0]);
         e->step += uint64_t(steps);
         e->sync();
     });

@@ -1,0 +1,42 @@
+// What the wide model's and the width-16 network's optimizer kernels share (cuda/optim.cuh:67-106).  Every fused
+// multiply-add is written out, so that the two compile to the same arithmetic.
+#pragma once
+#include "common.h"
+#include <math.h>
+
+struct AdamArgs {
+    float lr, beta1, beta2, eps, weight_decay, bc1, sqrt_bc2, clip;
+};
+// bias correction with the current beta1 (cuda/optim.cuh:90-91), evaluated on the host in fp32
+inline AdamArgs adam_args(float lr, float beta1, float beta2, float eps, float weight_decay, float clip, uint64_t step) {
+    return AdamArgs{lr, beta1, beta2, eps, weight_decay, 1.f - powf(beta1, float(step + 1)),
+                    sqrtf(1.f - powf(beta2, float(step + 1))), clip};
+}
+// one parameter: returns the new weight, updates m and v
+TG_DEVICE float adamw_element(const AdamArgs &a, float decay, float scale, float w, float &m, float &v, float g) {
+    const float gs = g * scale;
+    m = fmaf(1.f - a.beta1, fmaf(g, scale, -m), m);
+    v = fmaf(a.beta2, v, gs * ((1.f - a.beta2) * gs));
+    return fmaf(w, fmaf(-a.lr, decay, 1.f), -((a.lr / a.bc1) * m / (sqrtf(v) / a.sqrt_bc2 + a.eps)));
+}
+// Sum of squares of four elements, in the order every norm pass adds them.
+TG_DEVICE float quad_squares(const f32x4 &v) {
+    return fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[0], v[0], v[1] * v[1])));
+}
+// A block of 256 threads adds one value each, in a fixed tree; every thread gets the sum.  `waves`: shared, 4 floats.
+TG_DEVICE float block_sum_256(float x, float *waves) {
+    x = wave_sum(x);
+    if ((threadIdx.x & 63) == 0)
+        waves[threadIdx.x >> 6] = x;
+    __syncthreads();
+    return (waves[0] + waves[1]) + (waves[2] + waves[3]);
+}
+// Clip factor from the norm partials: every block folds the same partials in the same order (cuda/optim.cuh:67-80).
+TG_DEVICE float clip_factor(float clip, const float *__restrict__ norm_partials, int norm_count, float *waves) {
+    if (!(clip > 0.f))
+        return 1.f;
+    float sum = 0.f;
+    for (int i = threadIdx.x; i < norm_count; i += 256)
+        sum += norm_partials[i];
+    return fminf(1.f, clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
+}

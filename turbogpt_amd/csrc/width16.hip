@@ -17,7 +17,9 @@
 // the tokens in order; a fourth folds the chunks in order.  No atomics, bit-reproducible (the place of weight_gradient's
 // read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
 #include "common.h"
+#include "width16.h"
 #include "../../include/tgk_kernels.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -208,37 +210,39 @@ TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its
 // TRANSPOSED: operands of dX = dY W (rows = inputs, k = outputs; the attention projection's rows in head layout)
 // instead of Y = X W^T (rows = outputs; q, k and v in head layout)
 template <bool TRANSPOSED> TG_DEVICE void stage_weights(const Model &m, uint16_t *tiles, float *scales) {
-    const int layer_chunks = LAYER_TILES * 64, total = m.depth * layer_chunks + HEAD_TILES * 64;
-    for (int at = threadIdx.x; at < total; at += 64 * WAVES) { // four elements of one row at a time
-        int tile, row, col, source; // tile of the element's matrix row range, row and column within the tile
-        bool feed = true;
-        if (at < m.depth * layer_chunks) {
-            const int l = at / layer_chunks, k = at - l * layer_chunks;
-            const Layer q = layer_layout(l);
-            if (k < 640) { // q, k, v, attention, gate, up: rows of 16
-                const int r = k >> 2;
-                tile = l * LAYER_TILES + (r >> 4);
-                row = r & 15, col = (k & 3) * 4;
-                source = (r < 64 ? q.qkv + r * W : q.gate + (r - 64) * W) + col;
-                feed = TRANSPOSED ? (r >> 4) != 3 : (r >> 4) > 2;
-            } else { // down: rows of 48
-                const int r = (k - 640) / 12, part = (k - 640) - r * 12;
-                tile = l * LAYER_TILES + 10 + (part >> 2);
-                row = r, col = (part & 3) * 4;
-                source = q.down + r * F + part * 4;
-            }
-        } else {
-            const int k = at - m.depth * layer_chunks, r = k >> 2;
-            tile = m.depth * LAYER_TILES + (r >> 4);
-            row = r & 15, col = (k & 3) * 4;
-            source = V * W + m.depth * LAYER_SIZE + W + r * W + col;
-        }
-        const u32x2 v = *reinterpret_cast<const u32x2 *>(m.hi + source);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), total = staged_tiles(m.depth);
+    // a lane brings four elements of one row: element e goes to operand row `row` and k = col + e, or the other way round
+    const int row = lane >> 2, col = (lane & 3) * 4;
+    constexpr int AT_ONCE = 8; // loads in flight a wave: the staging waits for memory twice at depth 4, not 17 times
+    for (int base = w; base < total; base += WAVES * AT_ONCE) {
+        u32x2 v[AT_ONCE];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int operand_row = TRANSPOSED ? col + e : row, k = TRANSPOSED ? row : col + e;
-            const int c = feed ? feed_row(operand_row) : operand_row;
-            tiles[(tile * 64 + (k & 3) * 16 + c) * 4 + (k >> 2)] = uint16_t((e < 2 ? v.x : v.y) >> ((e & 1) * 16));
+        for (int i = 0; i < AT_ONCE; ++i) {
+            const int tile = base + i * WAVES, l = tile / LAYER_TILES, k = tile - l * LAYER_TILES;
+            if (tile >= total)
+                continue;
+            const Layer q = layer_layout(l);
+            const bf16_t *source = m.hi;
+            if (tile >= m.depth * LAYER_TILES)
+                source += V * W + m.depth * LAYER_SIZE + W + (tile - m.depth * LAYER_TILES) * 256 + lane * 4;
+            else if (k < 10) // q, k, v, attention; gate, up: rows of 16
+                source += (k < 4 ? q.qkv + k * 256 : q.gate + (k - 4) * 256) + lane * 4;
+            else // down: rows of 48
+                source += q.down + (k - 10) * 16 + row * F + col;
+            v[i] = *reinterpret_cast<const u32x2 *>(source);
+        }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+            const int tile = base + i * WAVES, k = tile % LAYER_TILES;
+            if (tile >= total)
+                continue;
+            const bool feed = tile >= m.depth * LAYER_TILES || (TRANSPOSED ? k != 3 : k > 2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int operand_row = TRANSPOSED ? col + e : row, at = TRANSPOSED ? row : col + e;
+                const int c = feed ? feed_row(operand_row) : operand_row;
+                tiles[(tile * 64 + (at & 3) * 16 + c) * 4 + (at >> 2)] = uint16_t((e < 2 ? v[i].x : v[i].y) >> ((e & 1) * 16));
+            }
         }
     }
     for (int at = threadIdx.x; at < (2 * m.depth + 1) * W; at += 64 * WAVES) { // attention and MLP norm of each layer, final
@@ -320,24 +324,40 @@ TG_DEVICE f32x4 rotate_back(f32x4 v, float c, float s) {
 
 // ---- forward ---------------------------------------------------------------------------------------
 // cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).
+// Tokens and targets come from x and y or, where `data.bytes` is given, straight out of the training bytes (every
+// sequence a window at a hashed place, cuda/dataset.cuh:13-27) and the tokens are left in `sampled` for the backward pass.
 __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x,
-                                                               const uint8_t *__restrict__ y, Workspace s,
+                                                               const uint8_t *__restrict__ y, W16Data data,
+                                                               uint8_t *__restrict__ sampled, Workspace s,
                                                                float *__restrict__ token_losses,
                                                                float *__restrict__ logits_out, int with_gradient) {
     extern __shared__ __align__(16) unsigned char staged_memory[];
     uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
     float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
-    stage_weights<false>(m, staged_tiles_at, scales);
     const Lane p = lane_of(m);
     const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
-    float rc, rs;
-    rotation(p.position, rc, rs);
     f32x4 h = ZERO;
+    int target = 0;
     if (p.live) {
-        const bf16_t *row = m.hi + int(x[p.token]) * W + p.g;
+        int token;
+        if (data.bytes) {
+            const int sequence = p.token / m.context;
+            const int64_t low = m.context > 8 ? m.context : 8;
+            const int64_t end = low + int64_t(hash_u64(data.seed + data.step * uint64_t(m.tokens / m.context) + uint64_t(sequence)) %
+                                              uint64_t(data.size - low));
+            const uint8_t *window = data.bytes + (end - m.context) + p.position;
+            token = window[0], target = window[1];
+            if (p.g == 0)
+                sampled[p.token] = uint8_t(token);
+        } else {
+            token = x[p.token], target = y[p.token];
+        }
+        const bf16_t *row = m.hi + token * W + p.g;
         h = f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])};
     }
-    const int target = p.live ? y[p.token] : 0;
+    stage_weights<false>(m, staged_tiles_at, scales);
+    float rc, rs;
+    rotation(p.position, rc, rs);
     for (int l = 0; l < m.depth; ++l) {
         const int tile = l * LAYER_TILES;
         u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
@@ -470,7 +490,6 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
     extern __shared__ __align__(16) unsigned char staged_memory[];
     uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
     float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
-    stage_weights<true>(m, staged_tiles_at, scales);
     const Lane p = lane_of(m);
     const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
     const size_t here = size_t(p.wave) * 64 + p.lane;
@@ -478,23 +497,51 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
     float rc, rs;
     rotation(p.position, rc, rs);
 
+    // a layer's rows are requested while the layer above is worked on
+    struct Rows {
+        u32x2 x, query, key, value, middle, gate[3], up[3];
+        float gate_of_top, slope, inv1, inv2;
+        int distance;
+    };
+    auto request = [&](int l, Rows &r) {
+        const u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
+        const float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            r.gate[t] = keep[(T_GU + t) * 64], r.up[t] = keep[(T_GU + 3 + t) * 64];
+        r.middle = keep[T_MIDDLE * 64], r.query = keep[T_Q * 64], r.key = keep[T_KEY * 64], r.value = keep[T_VALUE * 64];
+        r.x = keep[T_X * 64];
+        r.gate_of_top = words[WORD_GATE * 64], r.slope = words[WORD_SLOPE * 64], r.inv1 = words[WORD_INV1 * 64];
+        r.inv2 = words[WORD_INV2 * 64], r.distance = __float_as_int(words[WORD_DISTANCE * 64]);
+    };
+
     // head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
+    Rows next;
+    u32x2 dlogits[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        dlogits[t] = s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane];
+    const u32x2 hidden = s.hidden[here];
+    const float inverse = s.inverse[here];
+    request(m.depth - 1, next);
+    stage_weights<true>(m, staged_tiles_at, scales);
     f32x4 dn = ZERO;
 #pragma unroll
     for (int t = 0; t < 16; ++t)
-        dn = multiply(weight(m.depth * LAYER_TILES + t), unpack4(s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane]), dn);
-    f32x4 dh = normalize_backward(unpack4(s.hidden[here]), s.inverse[here], rounded(dn), weight.scale(2 * m.depth),
-                                  gz(2 * m.depth), p);
+        dn = multiply(weight(m.depth * LAYER_TILES + t), unpack4(dlogits[t]), dn);
+    f32x4 dh = normalize_backward(unpack4(hidden), inverse, rounded(dn), weight.scale(2 * m.depth), gz(2 * m.depth), p);
     for (int l = m.depth - 1; l >= 0; --l) {
         const int tile = l * LAYER_TILES;
         u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
-        const float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
+        const Rows rows = next;
+        if (l)
+            request(l - 1, next);
         // down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88, cuda/ops.cuh:133-144)
         keep[T_DH_DOWN * 64] = pack4(dh);
         f32x4 dgate[3], dup[3];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            const f32x4 gate = unpack4(keep[(T_GU + t) * 64]), up = unpack4(keep[(T_GU + 3 + t) * 64]);
+            const f32x4 gate = unpack4(rows.gate[t]), up = unpack4(rows.up[t]);
             const f32x4 dy = rounded(multiply(weight(tile + 10 + t), dh)), da = rounded(dy * up);
             f32x4 silu;
 #pragma unroll
@@ -516,31 +563,30 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
         for (int t = 0; t < 3; ++t)
             dn = multiply(weight(tile + 7 + t), dup[t], dn);
         // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
-        dh = rounded(dh + normalize_backward(unpack4(keep[T_MIDDLE * 64]), words[WORD_INV2 * 64], rounded(dn),
+        dh = rounded(dh + normalize_backward(unpack4(rows.middle), rows.inv2, rounded(dn),
                                              weight.scale(2 * l + 1), gz(2 * l + 1), p));
         keep[T_DH_ATTENTION * 64] = pack4(dh);
 
         // attention: output projection backward, the score gradient of the cached winner, query / key / value gradients
         // gathered over the sequence, inverse RoPE, QKV projection and RMSNorm backward (cuda/model.cuh:89-96,
         // cuda/attention.cuh:72-106)
-        const u32x2 query = keep[T_Q * 64];
-        const f32x4 key = unpack4(keep[T_KEY * 64]), value = unpack4(keep[T_VALUE * 64]);
-        const float gate = words[WORD_GATE * 64], slope = words[WORD_SLOPE * 64];
-        const int distance = __float_as_int(words[WORD_DISTANCE * 64]);
+        const u32x2 query = rows.query;
+        const f32x4 key = unpack4(rows.key), value = unpack4(rows.value);
+        const float gate = rows.gate_of_top;
         const u32x2 dattn = pack4(multiply(weight(tile + 3), dh));
         const f32x4 da = unpack4(dattn);
         float dt = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             dt = fmaf(da[c], value[c], dt);
-        dt *= slope;
+        dt *= rows.slope;
         f32x4 dk = ZERO, dv = ZERO;
         up_to<0, 7>([&](auto step) { // queries of this token's sequence that chose it, in order
             constexpr int D = decltype(step)::value;
             if (D >= m.context)
                 return;
             // every lane takes part in the shifts, so none of them may sit behind a condition
-            const uint32_t theirs = later<D>(uint32_t(distance));
+            const uint32_t theirs = later<D>(uint32_t(rows.distance));
             const float their_dt = __uint_as_float(later<D>(__float_as_uint(dt))), their_gate = __uint_as_float(later<D>(__float_as_uint(gate)));
             const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
             const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
@@ -559,7 +605,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
         keep[(T_DQKV + 1) * 64] = pack4(dk);
         keep[(T_DQKV + 2) * 64] = pack4(dv);
         dn = multiply(weight(tile + 2), dv, multiply(weight(tile + 1), dk, multiply(weight(tile), dq)));
-        dh = rounded(dh + normalize_backward(unpack4(keep[T_X * 64]), words[WORD_INV1 * 64], rounded(dn),
+        dh = rounded(dh + normalize_backward(unpack4(rows.x), rows.inv1, rounded(dn),
                                              weight.scale(2 * l), gz(2 * l), p));
     }
     s.dh[here] = pack4(dh);
@@ -609,17 +655,20 @@ __global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const
         }
     }
     f32x4 acc = ZERO;
+    const int waves = last - first;
     if (norm >= 0) { // a row of ones times the g * z terms
         const float *gz = s.gz + (size_t(norm) * s.waves + first) * 16 * W + lane;
-        for (int w = first; w < last; ++w, gz += 16 * W) {
-            float v[4];
+        float v[CHUNK_WAVES][4];
+#pragma unroll
+        for (int w = 0; w < CHUNK_WAVES; ++w)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                v[j] = gz[j * 64]; // token 4 j + g, feature c
+                v[w][j] = w < waves ? gz[(w * 4 + j) * 64] : 0.f; // token 4 j + g, feature c
+#pragma unroll
+        for (int w = 0; w < CHUNK_WAVES; ++w)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, v[j], acc, 0, 0, 0);
-        }
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, v[w][j], acc, 0, 0, 0);
         if (g == 0)
             out[c] = acc[0];
         return;
@@ -632,127 +681,207 @@ __global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const
     auto by_token = [&](const u32x2 &tile) {
         return turned(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, tile), __builtin_bit_cast(s16x4, identity), ZERO, 0, 0, 0));
     };
-    for (int w = first; w < last; ++w) {
-        const f32x4 col = by_token(cols[size_t(w) * col_stride + lane]);
-        f32x4 row;
-        if (vocabulary >= 0) {
+    // everything the chunk needs is requested before the first product
+    u32x2 col[CHUNK_WAVES], row[CHUNK_WAVES];
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        col[w] = row[w] = u32x2{0, 0};
+        if (w >= waves)
+            continue;
+        col[w] = cols[size_t(first + w) * col_stride + lane];
+        if (vocabulary < 0) {
+            row[w] = rows[size_t(first + w) * row_stride + lane];
+        } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int t = 4 * j + g, token = w * m.per_wave + t; // rows beyond the last token are zero: any id will do
-                row[j] = t < m.per_wave && token < m.tokens && x[token] == vocabulary ? 1.f : 0.f;
+                const int t = 4 * j + g, token = (first + w) * m.per_wave + t; // rows beyond the last token are zero: any id will do
+                row[w].x |= uint32_t(t < m.per_wave && token < m.tokens ? x[token] : 0) << (8 * j);
             }
-        } else {
-            row = by_token(rows[size_t(w) * row_stride + lane]);
         }
-        acc = multiply(row, col, acc);
+    }
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        f32x4 by_row;
+        if (vocabulary < 0)
+            by_row = by_token(row[w]);
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                by_row[j] = int((row[w].x >> (8 * j)) & 255u) == vocabulary ? 1.f : 0.f;
+        acc = multiply(by_row, by_token(col[w]), acc);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         out[(4 * g + r) * width + c] = acc[r];
 }
-// gradient = the chunks' sums in chunk order
-__global__ __launch_bounds__(64) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
-                                                      float *__restrict__ gradient) {
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    if (i >= parameters)
+// gradient = the chunks' sums in chunk order; a block's 1024 elements also leave the sum of their squares in norms[block].
+// Blocks beyond the parameters average the losses: one a position, in double (cuda/trainer.cuh:79-100).
+int fold_blocks(int parameters) { return (parameters + 1023) / 1024; }
+__global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
+                                                       float *__restrict__ gradient, float *__restrict__ norms, int blocks,
+                                                       const float *__restrict__ token_losses, int batch, int context,
+                                                       float *__restrict__ means) {
+    if (int(blockIdx.x) >= blocks) {
+        __shared__ double sums[4];
+        const int position = blockIdx.x - blocks;
+        double sum = 0;
+#pragma unroll 4
+        for (int b = threadIdx.x; b < batch; b += 256)
+            sum += token_losses[size_t(b) * context + position];
+#pragma unroll
+        for (int k = 32; k; k >>= 1)
+            sum += __shfl_xor(sum, k, 64);
+        if ((threadIdx.x & 63) == 0)
+            sums[threadIdx.x >> 6] = sum;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            means[position] = float(((sums[0] + sums[1]) + (sums[2] + sums[3])) / batch);
         return;
-    float sum = 0.f;
+    }
+    __shared__ float waves[4];
+    const int at = (blockIdx.x * 256 + threadIdx.x) * 4;
+    f32x4 sum = ZERO;
+    if (at < parameters) {
+        const float *from = partials + at;
 #pragma unroll 16
-    for (int c = 0; c < chunks; ++c)
-        sum += partials[size_t(c) * parameters + i];
-    gradient[i] = sum;
+        for (int c = 0; c < chunks; ++c)
+            sum += *reinterpret_cast<const f32x4 *>(from + size_t(c) * parameters);
+        *reinterpret_cast<f32x4 *>(gradient + at) = sum;
+    }
+    if (norms) {
+        const float squares = block_sum_256(0.f + quad_squares(sum), waves);
+        if (threadIdx.x == 0)
+            norms[blockIdx.x] = squares;
+    }
 }
 
-// ---- Muon for the hidden matrices: one block per matrix (cuda/optim.cuh:17-62, :107-118) ---------------
-struct MuonArgs {
-    float clip, lr, momentum, weight_decay;
-    int ns_steps, norm_count;
+// ---- optimizer (cuda/optim.cuh:17-119) ------------------------------------------------------------------
+// Blocks 0 .. 5 depth - 1: Muon, a hidden matrix each.  The rest: AdamW, 256 quads of embedding, scales and head each.
+// The Newton-Schulz iterate is a 16 x n matrix in 16 x 16 tiles, one a wave, lane 16 g + c holding rows 4 g .. of column c;
+// the products run on the fp32 matrix instruction (the same fmaf chains as a loop).  X X^T is symmetric to the last bit,
+// so its tile turned is the operand of the two products behind it, every wave computes it for itself, and a step
+// exchanges nothing but X through LDS: one barrier a step where there were four.
+struct Update {
+    W16Weights from, to;
+    float *momentum, *variance;
+    const float *gradient, *norms;
+    int norm_count, depth;
+    AdamArgs adam;
+    MuonArgs muon;
 };
-__global__ __launch_bounds__(256) void w16_muon_kernel(Layout layout, bf16_t *hi, uint16_t *lo, float *momentum,
-                                                       const float *__restrict__ gradient,
-                                                       const float *__restrict__ norm_partials, MuonArgs a) {
-    __shared__ float wide[16 * 48], product[16 * 48], gram[256], work[256], waves[4], shared_scalar;
-    const Layer &p = layout.layers[blockIdx.x / 5];
-    const int type = blockIdx.x % 5;
+TG_DEVICE float difference(float a, float b) { // of two rounded values: a product in b is not fused into it
+#pragma clang fp contract(off)
+    return a - b;
+}
+TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
+    __shared__ float wide[2][16 * F];
+    __shared__ float norm_waves[4];
+    const Layer p = layer_layout(matrix / 5);
+    const int type = matrix % 5;
     const int weight = type == 0 ? p.qkv : type == 1 ? p.attention : type == 2 ? p.gate : type == 3 ? p.up : p.down;
     const int rows = (type == 0 || type == 2 || type == 3) ? 48 : 16, cols = type == 4 ? 48 : 16;
     const int n = rows > cols ? rows : cols, size = rows * cols, tid = threadIdx.x;
-
-    float clip = 1.f;
-    if (a.clip > 0.f) { // the same fold of the same partials as the AdamW kernel (cuda/optim.cuh:67-80)
-        float sum = 0.f;
-        for (int i = tid; i < a.norm_count; i += 256)
-            sum += norm_partials[i];
-        sum = wave_sum(sum);
-        if ((tid & 63) == 0)
-            waves[tid >> 6] = sum;
-        __syncthreads();
-        if (tid == 0)
-            shared_scalar = fminf(1.f, a.clip / (sqrtf((waves[0] + waves[1]) + (waves[2] + waves[3])) + 1e-6f));
-        __syncthreads();
-        clip = shared_scalar;
-        __syncthreads();
-    }
-    float squares = 0.f;
-    for (int i = tid; i < size; i += 256) {
-        const float g = gradient[weight + i] * clip;
-        const float m = momentum[weight + i] + (1.f - a.momentum) * (g - momentum[weight + i]);
-        momentum[weight + i] = m;
-        const float b = round_bf16(g + a.momentum * (m - g));
-        wide[rows > cols ? (i % cols) * rows + i / cols : i] = b; // kept as a 16 x n matrix
-        squares += b * b;
-    }
-    squares = wave_sum(squares);
-    if ((tid & 63) == 0)
-        waves[tid >> 6] = squares;
-    __syncthreads();
-    if (tid == 0)
-        shared_scalar = fmaxf(round_bf16(sqrtf((waves[0] + waves[1]) + (waves[2] + waves[3]))), round_bf16(1e-7f));
-    __syncthreads();
-    const float norm = shared_scalar;
-    for (int i = tid; i < size; i += 256)
-        wide[i] = round_bf16(wide[i] / norm);
-    __syncthreads();
-    for (int step = 0; step < a.ns_steps; ++step) {
-        { // A = X X^T, kept in bf16
-            const int r = tid >> 4, c = tid & 15;
-            float acc = 0.f;
-            for (int k = 0; k < n; ++k)
-                acc = fmaf(wide[r * n + k], wide[c * n + k], acc);
-            gram[tid] = round_bf16(acc);
-        }
-        __syncthreads();
-        { // -4.775 A + 2.0315 A A
-            const int r = tid >> 4, c = tid & 15;
-            float acc = 0.f;
+    // element tid + 256 k of the matrix is this thread's until the iteration and again behind it; its place in the 16 x n form
+    auto place = [&](int i) { return rows > cols ? (i % cols) * rows + i / cols : i; };
+    float g[3], m[3], w[3];
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-                acc = fmaf(gram[r * 16 + k], gram[k * 16 + c], acc);
-            work[tid] = round_bf16(-4.775f * gram[tid] + 2.0315f * acc);
-        }
-        __syncthreads();
-        for (int i = tid; i < size; i += 256) {
-            const int r = i / n, c = i - r * n;
-            float acc = 0.f;
+    for (int k = 0; k < 3; ++k) {
+        const int i = weight + tid + 256 * k;
+        const bool mine = tid + 256 * k < size;
+        g[k] = mine ? u.gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f, w[k] = mine ? master(u.from.hi, u.from.lo, i) : 0.f;
+    }
+    const float clip = clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+    float squares = 0.f, b[3];
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-                acc = fmaf(work[r * 16 + k], wide[k * n + c], acc);
-            product[i] = acc;
+    for (int k = 0; k < 3; ++k)
+        if (tid + 256 * k < size) {
+            const float gs = g[k] * clip;
+            const float next = fmaf(1.f - u.muon.momentum, fmaf(g[k], clip, -m[k]), m[k]);
+            u.momentum[weight + tid + 256 * k] = next;
+            b[k] = round_bf16(fmaf(u.muon.momentum, difference(next, gs), gs));
+            squares = fmaf(b[k], b[k], squares);
         }
-        __syncthreads();
-        for (int i = tid; i < size; i += 256)
-            wide[i] = round_bf16(3.4445f * wide[i] + product[i]);
+    const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        if (tid + 256 * k < size)
+            wide[0][place(tid + 256 * k)] = round_bf16(b[k] / norm);
+    __syncthreads();
+    const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
+    f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
+    if (tile < tiles)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            x[r] = wide[0][(4 * gr + r) * n + 16 * tile + c];
+    for (int step = 0; step < u.muon.ns_steps; ++step) {
+        const float *in = wide[step & 1];
+        float *out = wide[(step & 1) ^ 1];
+        if (tile < tiles) {
+            f32x4 gram = ZERO; // A = X X^T, kept in bf16
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (k < tiles) {
+                    f32x4 row;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        row[j] = in[c * n + 16 * k + 4 * j + gr];
+                    gram = multiply(row, row, gram);
+                }
+            gram = rounded(gram);
+            const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
+            f32x4 work; // -4.775 A + 2.0315 A A
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
+            const f32x4 product = multiply(turned(rounded(work)), turned(x));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                x[r] = round_bf16(fmaf(3.4445f, x[r], product[r]));
+                out[(4 * gr + r) * n + 16 * tile + c] = x[r];
+            }
+        }
         __syncthreads();
     }
-    const float adjusted = a.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols)));
-    for (int i = tid; i < size; i += 256) {
-        const int index = rows > cols ? (i % cols) * rows + i / cols : i;
-        const float w = master(hi, lo, weight + i) * (1.f - a.lr * a.weight_decay);
-        const uint32_t bits = __float_as_uint(w - adjusted * wide[index]);
-        hi[weight + i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
-        lo[weight + i] = uint16_t(bits);
+    const float *result = wide[u.muon.ns_steps & 1];
+    const float adjusted = u.muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-u.muon.lr, u.muon.weight_decay, 1.f);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        if (tid + 256 * k < size) {
+            const int i = weight + tid + 256 * k;
+            const uint32_t bits = __float_as_uint(fmaf(w[k], keep, -(adjusted * result[place(tid + 256 * k)])));
+            u.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
+            u.to.lo[i] = uint16_t(bits);
+        }
+}
+__global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
+    __shared__ float waves[4];
+    if (int(blockIdx.x) < 5 * u.depth)
+        return muon_matrix(u, blockIdx.x, waves);
+    const float scale = clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+    // quads: the embedding's 1024, four for each scale, the head's 1024 (the only ones that decay)
+    const int quad = (blockIdx.x - 5 * u.depth) * 256 + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
+    int at = quad * 4;
+    float decay = 0.f;
+    if (norm >= norms) {
+        const int k = quad - V * W / 4 - 4 * norms;
+        if (k >= V * W / 4)
+            return;
+        at = V * W + u.depth * LAYER_SIZE + W + k * 4;
+        decay = u.adam.weight_decay;
+    } else if (norm >= 0 && quad >= V * W / 4) {
+        const Layer q = layer_layout(norm >> 1);
+        at = (norm == 2 * u.depth ? V * W + u.depth * LAYER_SIZE : (norm & 1) ? q.mlp_norm : q.attention_norm) + (quad & 3) * 4;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        float m = u.momentum[at + k], v = u.variance[at + k];
+        const float next = adamw_element(u.adam, decay, scale, master(u.from.hi, u.from.lo, at + k), m, v, u.gradient[at + k]);
+        u.momentum[at + k] = m, u.variance[at + k] = v;
+        u.to.hi[at + k] = uint16_t(__float_as_uint(next) >> 16);
+        u.to.lo[at + k] = uint16_t(__float_as_uint(next));
     }
 }
+int adam_blocks(int depth) { return (2 * V * W / 4 + 4 * (2 * depth + 1) + 255) / 256; }
 
 void check_shape(int depth, int batch, int context) {
     require(depth >= 1 && depth <= MAX_DEPTH, "w16: depth must be 1..8");
@@ -776,6 +905,25 @@ extern "C" size_t tgk_w16_workspace(int depth, int batch, int context) {
     return carve(depth, batch, context, nullptr).bytes;
 }
 
+namespace {
+void launch_forward(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, const uint8_t *y,
+                    const W16Data &data, uint8_t *sampled, float *token_losses, float *logits, int with_gradient) {
+    hipLaunchKernelGGL(w16_forward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(m.depth), stream, m, x, y, data,
+                       sampled, r, token_losses, logits, with_gradient);
+    check_hip(hipGetLastError(), "w16_forward launch: ");
+}
+void launch_backward(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, float *gradient, float *norms,
+                     const float *token_losses, float *means) {
+    const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
+    hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(m.depth), stream, m, r);
+    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(m.depth) + 3) / 4, r.chunks), dim3(256), 0, stream, m, x,
+                       r, parameters);
+    hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (means ? m.context : 0)), dim3(256), 0, stream, r.partials, r.chunks,
+                       parameters, gradient, norms, blocks, token_losses, m.tokens / m.context, m.context, means);
+    check_hip(hipGetLastError(), "w16_backward launch: ");
+}
+} // namespace
+
 extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int context, const uint16_t *weight_hi,
                                const uint16_t *weight_lo, const uint8_t *x, const uint8_t *y, void *workspace,
                                float *token_losses, float *logits, int with_gradient) {
@@ -783,11 +931,8 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && y && workspace && token_losses, "w16_forward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
-        const Workspace r = carve(depth, batch, context, workspace);
-        hipLaunchKernelGGL(w16_forward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream,
-                           make_model(depth, batch, context, weight_hi, weight_lo), x, y, r, token_losses, logits,
-                           with_gradient);
-        check_hip(hipGetLastError(), "w16_forward launch: ");
+        launch_forward(stream, make_model(depth, batch, context, weight_hi, weight_lo), carve(depth, batch, context, workspace),
+                       x, y, W16Data{}, nullptr, token_losses, logits, with_gradient);
     });
 }
 
@@ -797,16 +942,26 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && workspace && gradient, "w16_backward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
-        const Workspace r = carve(depth, batch, context, workspace);
-        const int parameters = make_layout(depth).count;
-        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
-        hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
-        hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(depth) + 3) / 4, r.chunks), dim3(256), 0, stream,
-                           m, x, r, parameters);
-        hipLaunchKernelGGL(w16_fold_kernel, dim3((parameters + 63) / 64), dim3(64), 0, stream, r.partials, r.chunks,
-                           parameters, gradient);
-        check_hip(hipGetLastError(), "w16_backward launch: ");
+        launch_backward(stream, make_model(depth, batch, context, weight_hi, weight_lo), carve(depth, batch, context, workspace),
+                        x, gradient, nullptr, nullptr, nullptr);
     });
+}
+
+int w16_norm_count(int depth) {
+    return fold_blocks(make_layout(depth).count);
+}
+void w16_gradient(hipStream_t stream, int depth, int batch, int context, const W16Weights &weights, const W16Data &data,
+                  uint8_t *tokens, void *workspace, float *token_losses, float *means, float *gradient, float *norms) {
+    const Model m = make_model(depth, batch, context, weights.hi, weights.lo);
+    const Workspace r = carve(depth, batch, context, workspace);
+    launch_forward(stream, m, r, nullptr, nullptr, data, tokens, token_losses, nullptr, 1);
+    launch_backward(stream, m, r, tokens, gradient, norms, token_losses, means);
+}
+void w16_update(hipStream_t stream, int depth, const W16Weights &from, const W16Weights &to, float *momentum, float *variance,
+                const float *gradient, const float *norms, int norm_count, const AdamArgs &adam, const MuonArgs &muon) {
+    const Update u{from, to, momentum, variance, gradient, norms, norm_count, depth, adam, muon};
+    hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth + adam_blocks(depth)), dim3(256), 0, stream, u);
+    check_hip(hipGetLastError(), "w16_update launch: ");
 }
 
 extern "C" int tgk_w16_muon(hipStream_t stream, int depth, uint16_t *weight_hi, uint16_t *weight_lo, float *momentum,
@@ -817,9 +972,12 @@ extern "C" int tgk_w16_muon(hipStream_t stream, int depth, uint16_t *weight_hi, 
         require(weight_hi && weight_lo && momentum && gradient, "w16_muon: missing operand");
         require(!(clip > 0.f) || (norm_partials && norm_count > 0), "w16_muon: clipping needs the norm partials");
         require(ns_steps >= 1 && ns_steps <= 10, "w16_muon: ns_steps must be 1..10");
-        const MuonArgs a{clip, lr, momentum_rate, weight_decay, ns_steps, norm_count};
-        hipLaunchKernelGGL(w16_muon_kernel, dim3(depth * 5), dim3(256), 0, stream, make_layout(depth), weight_hi,
-                           weight_lo, momentum, gradient, norm_partials, a);
+        AdamArgs adam{};
+        adam.clip = clip;
+        const W16Weights weights{weight_hi, weight_lo};
+        const Update u{weights, weights, momentum, nullptr, gradient, norm_partials, norm_count, depth, adam,
+                       MuonArgs{lr, momentum_rate, weight_decay, ns_steps}};
+        hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth), dim3(256), 0, stream, u); // the matrices' blocks alone
         check_hip(hipGetLastError(), "w16_muon launch: ");
     });
 }
