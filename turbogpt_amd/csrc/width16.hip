@@ -174,8 +174,19 @@ template <int D, int END, class Body> TG_DEVICE void up_to(Body &&body) { // D, 
     if constexpr (D < END)
         up_to<D + 1, END>(body);
 }
+// 1 / b and x / b = divide(x, b, 1 / b), correctly rounded while neither b nor the result leaves the normal range (compared
+// with the division over every mantissa of b and 262 million pairs: no difference): three instructions where the
+// division takes ten, and 140 of them stand in a wave's way at the head alone.
+TG_DEVICE float reciprocal(float b) {
+    const float r = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, r, 1.f), r, r);
+}
+TG_DEVICE float divide(float x, float b, float r) {
+    const float q = x * r;
+    return fmaf(fmaf(-q, b, x), r, q);
+}
 TG_DEVICE float sigmoid(float x) {
-    return 1.f / (1.f + expf(-x));
+    return reciprocal(fminf(1.f + expf(-x), 0x1p126f)); // below -87 it is 1e-38 instead of less
 }
 
 struct Model {
@@ -473,13 +484,16 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
         s.hidden[size_t(p.wave) * 64 + p.lane] = pack4(h);
         s.nf[size_t(p.wave) * 64 + p.lane] = nf;
         s.inverse[size_t(p.wave) * 64 + p.lane] = inv;
+        const float share = reciprocal(sum), tokens = float(m.tokens), per_token = 1.f / tokens;
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             f32x4 d;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                d[r] = p.live ? (logit[t][r] / sum - (16 * t + 4 * r == mine ? 1.f : 0.f)) / float(m.tokens) : 0.f;
-            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = pack4(d);
+                d[r] = divide(divide(logit[t][r], sum, share) - (16 * t + 4 * r == mine ? 1.f : 0.f), tokens, per_token);
+            u32x2 packed = pack4(d);
+            packed.x = p.live ? packed.x : 0, packed.y = p.live ? packed.y : 0;
+            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = packed;
         }
     }
 }
@@ -618,12 +632,15 @@ constexpr int LAYER_JOBS = 15;
 __host__ __device__ constexpr int gradient_jobs(int depth) { return depth * LAYER_JOBS + 33; }
 __global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const uint8_t *__restrict__ x, Workspace s,
                                                                   int parameters) {
-    const int job = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (job >= gradient_jobs(m.depth))
+    // consecutive blocks sit on consecutive XCDs: block 8 i + k takes the i-th job group of XCD k's chunks, so that the jobs
+    // of a chunk, which share their rows, share an L2
+    const int groups = (gradient_jobs(m.depth) + 3) / 4, at = blockIdx.x >> 3;
+    const int chunk = at / groups * 8 + (blockIdx.x & 7), job = at % groups * 4 + (threadIdx.x >> 6);
+    if (chunk >= s.chunks || job >= gradient_jobs(m.depth))
         return;
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-    const int first = blockIdx.y * CHUNK_WAVES, last = min(first + CHUNK_WAVES, s.waves);
-    float *out = s.partials + size_t(blockIdx.y) * parameters;
+    const int first = chunk * CHUNK_WAVES, last = min(first + CHUNK_WAVES, s.waves);
+    float *out = s.partials + size_t(chunk) * parameters;
     // A row operand (rows of the gradient tile) and a column operand, as tiles of tokens x 16 features in feed layout
     const u32x2 *rows = nullptr, *cols = nullptr;
     size_t row_stride = 64, col_stride = 64; // from one wave's tile to the next
@@ -916,7 +933,7 @@ void launch_backward(hipStream_t stream, const Model &m, const Workspace &r, con
                      const float *token_losses, float *means) {
     const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
     hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(m.depth), stream, m, r);
-    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(m.depth) + 3) / 4, r.chunks), dim3(256), 0, stream, m, x,
+    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(m.depth) + 3) / 4 * ((r.chunks + 7) / 8 * 8)), dim3(256), 0, stream, m, x,
                        r, parameters);
     hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (means ? m.context : 0)), dim3(256), 0, stream, r.partials, r.chunks,
                        parameters, gradient, norms, blocks, token_losses, m.tokens / m.context, m.context, means);
