@@ -4,6 +4,7 @@
 // op sequencing that its persistent kernel does on the device (cuda/trainer.cuh:103-125,
 // cuda/model.cuh:8-99).  All arithmetic is in the tgk_* kernels; this file only sequences them.
 #include "common.h"
+#include "gemm_list.h"
 #include "readback.h"
 #include "width16.h"
 #include "../../include/tg_model.h"
@@ -18,6 +19,7 @@ namespace {
 
 constexpr int MaxLaunchSteps = 4096; // cuda/types.cuh:10
 constexpr int NormPartials = 1024;
+constexpr int ListUnit = 128;   // every width is a multiple of it (wgrad_list)
 constexpr int RowTile = 128;    // smallest number of rows the matrix products take
 constexpr int MaxInFlight = 16; // batches in flight, each with its own stream and saved activations
 
@@ -71,9 +73,8 @@ struct Slot {
     float *token_losses = nullptr, *gradient = nullptr;
     std::vector<bf16_t *> x; // x[l] = input of block l; x[depth] = output of the last block
     std::vector<LayerBuffers> layers;
-    bf16_t *nf = nullptr, *logits = nullptr, *dh = nullptr, *t1 = nullptr, *du = nullptr, *dqkv = nullptr;
-    bf16_t *dh_mid = nullptr; // the gradient between a block's two halves, when the block's weight gradients are batched
-    // When all weight gradients of a step go out as one launch behind the backward pass, every block keeps the four
+    bf16_t *nf = nullptr, *logits = nullptr, *t1 = nullptr;
+    // All weight gradients of a step go out as one launch behind the backward pass: every block keeps the four
     // output gradients that launch reads: g_x[l] = gradient of the loss by x[l] (g_x[l + 1] enters block l), g_mid[l]
     // by the block's middle, g_u[l] by the MLP pre-activation, g_qkv[l] by the packed projections.
     std::vector<bf16_t *> g_x, g_mid, g_u, g_qkv;
@@ -121,8 +122,6 @@ struct Engine {
     int64_t data_size = 0;
     float *logits_f32 = nullptr;
     size_t workspace_bytes = 0;
-    bool batched_wgrad = false; // a block's four weight gradients in one launch (shapes permitting)
-    bool list_wgrad = false;    // every weight gradient of a step in one launch (widths that are multiples of 256)
 
     std::shared_ptr<Readback> readback = Readback::shared();
     float *batch_means = nullptr; // [context]: the per-position losses of a fixed batch
@@ -295,7 +294,7 @@ struct Engine {
         const auto wt = [&](int64_t offset) { return v.t + offset; };
         std::vector<bf16_t *> &x = s.x;
         std::vector<LayerBuffers> &layers = s.layers;
-        bf16_t *nf = s.nf, *logits = s.logits, *dh = s.dh, *t1 = s.t1, *du = s.du, *dqkv = s.dqkv;
+        bf16_t *logits = s.logits, *t1 = s.t1;
         const int M = tokens(), d = config.d_model, F = config.ffn, V = config.vocab, T = c.context;
         const float scale = 1.0f / std::sqrt(float(d / config.heads));
         float *g = gradient;
@@ -306,80 +305,35 @@ struct Engine {
             return tgk_layernorm_bwd_rows(stream, M, d, input, dy, w(gamma), wl(gamma), residual, dx, config.ln_eps,
                                           s.ln_partials + size_t(job) * ln_stride, ln_stride);
         };
-        if (list_wgrad) {
-            // No weight gradient in the loop: every block leaves its output gradients in buffers of its own and one
-            // launch at the end computes all 4 * depth + 2 products (the head's included - its operands are dlogits,
-            // still in `logits`, and nf - and the token table's, one-hot^T times the gradient entering the first block).
-            OP(TG_CLASS_HEAD, tgk_gemm_dgrad_t(stream, M, V, d, logits, V, wt(layout.head), V, t1, d, nullptr, 0));
-            OP(TG_CLASS_LAYERNORM_BWD, ln_rows(0, x[c.depth], t1, layout.lnf_g, nullptr, s.g_x[c.depth]));
-            for (int l = c.depth - 1; l >= 0; --l) {
-                const TgLayerParameters &p = layout.layers[l];
-                LayerBuffers &b = layers[l];
-                bf16_t *in = s.g_x[l + 1], *mid = s.g_mid[l], *gu = s.g_u[l], *gqkv = s.g_qkv[l];
-                OP(TG_CLASS_GEMM_DGRAD_GELU, tgk_gemm_dgrad_t(stream, M, d, F, in, d, wt(p.mlp_down), d, gu, F, b.u, F));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, F, d, gu, F, wt(p.mlp_up), F, t1, d, nullptr, 0));
-                OP(TG_CLASS_LAYERNORM_BWD, ln_rows(1 + 2 * l, b.mid, t1, p.ln2_g, in, mid));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, d, d, mid, d, wt(p.attn_out), d, t1, d, nullptr, 0));
-                OP(TG_CLASS_ATTN_BWD, tgk_attn_bwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d,
-                                                   b.qkv + 2 * d, 3 * d, b.o, d, b.lse, t1, d, gqkv, gqkv + d, gqkv + 2 * d,
-                                                   3 * d, scale, workspace, workspace_bytes));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, gqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
-                OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, mid, s.g_x[l]));
-            }
-            OP(TG_CLASS_LAYERNORM_BWD, tgk_layernorm_bwd_fold(stream, M, d, 2 * c.depth + 1, s.ln_partials, ln_stride, s.ln_targets, 0));
-            OP(TG_CLASS_OTHER, tgk_embed_bwd_onehot(stream, c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions, 0));
-            const bool norms = c.clip > 0;
-            OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad_list(stream, M, int(s.wgrad_jobs.size()), s.wgrad_jobs.data(), s.wgrad_table, 0,
-                                                        workspace, workspace_bytes, norms ? s.norms : nullptr));
-            if (norms)
-                OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
-            return;
-        }
-        OP(TG_CLASS_HEAD, tgk_gemm_wgrad(stream, M, V, d, logits, V, nf, d, g + layout.head, d, 0, workspace, workspace_bytes));
+        // No weight gradient in the loop: every block leaves its output gradients in buffers of its own and one
+        // launch at the end computes all 4 * depth + 2 products (the head's included - its operands are dlogits,
+        // still in `logits`, and nf - and the token table's, one-hot^T times the gradient entering the first block).
         OP(TG_CLASS_HEAD, tgk_gemm_dgrad_t(stream, M, V, d, logits, V, wt(layout.head), V, t1, d, nullptr, 0));
-        OP(TG_CLASS_LAYERNORM_BWD, ln_rows(0, x[c.depth], t1, layout.lnf_g, nullptr, dh));
+        OP(TG_CLASS_LAYERNORM_BWD, ln_rows(0, x[c.depth], t1, layout.lnf_g, nullptr, s.g_x[c.depth]));
         for (int l = c.depth - 1; l >= 0; --l) {
             const TgLayerParameters &p = layout.layers[l];
             LayerBuffers &b = layers[l];
-            if (batched_wgrad) {
-                // The four weight gradients wait until all their operands exist (after the attention backward) and
-                // go out as one launch; for that the gradient entering the block (dh) survives the block's first
-                // half: LayerNorm 2 writes its sum with dh into dh_mid.
-                bf16_t *mid = s.dh_mid;
-                OP(TG_CLASS_GEMM_DGRAD_GELU, tgk_gemm_dgrad_t(stream, M, d, F, dh, d, wt(p.mlp_down), d, du, F, b.u, F));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, F, d, du, F, wt(p.mlp_up), F, t1, d, nullptr, 0));
-                OP(TG_CLASS_LAYERNORM_BWD, ln_rows(1 + 2 * l, b.mid, t1, p.ln2_g, dh, mid));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, d, d, mid, d, wt(p.attn_out), d, t1, d, nullptr, 0));
-                OP(TG_CLASS_ATTN_BWD, tgk_attn_bwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d,
-                                                   b.qkv + 2 * d, 3 * d, b.o, d, b.lse, t1, d, dqkv, dqkv + d, dqkv + 2 * d,
-                                                   3 * d, scale, workspace, workspace_bytes));
-                const TgkWgradJob jobs[4] = {{d, F, dh, d, b.a, F, g + p.mlp_down, F},
-                                             {F, d, du, F, b.n2, d, g + p.mlp_up, d},
-                                             {d, d, mid, d, b.o, d, g + p.attn_out, d},
-                                             {3 * d, d, dqkv, 3 * d, b.n1, d, g + p.qkv, d}};
-                OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad_batch(stream, M, 4, jobs, 0, workspace, workspace_bytes));
-                OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, dqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
-                OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, mid, dh));
-                continue;
-            }
-            OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad(stream, M, d, F, dh, d, b.a, F, g + p.mlp_down, F, 0, workspace, workspace_bytes));
-            OP(TG_CLASS_GEMM_DGRAD_GELU, tgk_gemm_dgrad_t(stream, M, d, F, dh, d, wt(p.mlp_down), d, du, F, b.u, F));
-            OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad(stream, M, F, d, du, F, b.n2, d, g + p.mlp_up, d, 0, workspace, workspace_bytes));
-            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, F, d, du, F, wt(p.mlp_up), F, t1, d, nullptr, 0));
-            OP(TG_CLASS_LAYERNORM_BWD, ln_rows(1 + 2 * l, b.mid, t1, p.ln2_g, dh, dh));
-            OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad(stream, M, d, d, dh, d, b.o, d, g + p.attn_out, d, 0, workspace, workspace_bytes));
-            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, d, d, dh, d, wt(p.attn_out), d, t1, d, nullptr, 0));
-            OP(TG_CLASS_ATTN_BWD, tgk_attn_bwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d, b.qkv + 2 * d,
-                            3 * d, b.o, d, b.lse, t1, d, dqkv, dqkv + d, dqkv + 2 * d, 3 * d, scale, workspace,
-                            workspace_bytes));
-            OP(TG_CLASS_GEMM_WGRAD, tgk_gemm_wgrad(stream, M, 3 * d, d, dqkv, 3 * d, b.n1, d, g + p.qkv, d, 0, workspace,
-                              workspace_bytes));
-            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, dqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
-            OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, dh, dh));
+            bf16_t *in = s.g_x[l + 1], *mid = s.g_mid[l], *gu = s.g_u[l], *gqkv = s.g_qkv[l];
+            OP(TG_CLASS_GEMM_DGRAD_GELU, tgk_gemm_dgrad_t(stream, M, d, F, in, d, wt(p.mlp_down), d, gu, F, b.u, F));
+            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, F, d, gu, F, wt(p.mlp_up), F, t1, d, nullptr, 0));
+            OP(TG_CLASS_LAYERNORM_BWD, ln_rows(1 + 2 * l, b.mid, t1, p.ln2_g, in, mid));
+            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, d, d, mid, d, wt(p.attn_out), d, t1, d, nullptr, 0));
+            OP(TG_CLASS_ATTN_BWD, tgk_attn_bwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d,
+                                               b.qkv + 2 * d, 3 * d, b.o, d, b.lse, t1, d, gqkv, gqkv + d, gqkv + 2 * d,
+                                               3 * d, scale, workspace, workspace_bytes));
+            OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, gqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
+            OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, mid, s.g_x[l]));
         }
         OP(TG_CLASS_LAYERNORM_BWD, tgk_layernorm_bwd_fold(stream, M, d, 2 * c.depth + 1, s.ln_partials, ln_stride, s.ln_targets, 0));
-        OP(TG_CLASS_OTHER, tgk_embed_bwd(stream, c.batch, T, d, V, tokens_in, dh, g + layout.embedding, g + layout.positions, 0,
-                                         workspace, workspace_bytes));
+        OP(TG_CLASS_OTHER, tgk_embed_bwd_onehot(stream, c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions, 0));
+        const bool norms = c.clip > 0;
+        {
+            Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
+            wgrad_list(stream, M, int(s.wgrad_jobs.size()), s.wgrad_jobs.data(), ListUnit, s.wgrad_table, workspace,
+                       workspace_bytes, norms ? s.norms : nullptr);
+        }
+        if (norms)
+            OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
     }
 
     // cuda/optim.cuh:66-106 for optimizer step `at` (0-based), on the engine's stream: gradient -> the weights of
@@ -684,18 +638,13 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
             }
             e->allocate(slot.nf, M * d, false);
             e->allocate(slot.logits, M * V, false);
-            e->allocate(slot.dh, M * d, false);
             e->allocate(slot.t1, M * d, false);
-            e->allocate(slot.du, M * F, false);
-            e->allocate(slot.dqkv, M * 3 * d, false);
         }
         const TgkWgradJob block_jobs[4] = {{int(d), int(F), nullptr, int(d), nullptr, int(F), nullptr, int(F)},
                                            {int(F), int(d), nullptr, int(F), nullptr, int(d), nullptr, int(d)},
                                            {int(d), int(d), nullptr, int(d), nullptr, int(d), nullptr, int(d)},
                                            {int(3 * d), int(d), nullptr, int(3 * d), nullptr, int(d), nullptr, int(d)}};
-        size_t batch_need = tgk_gemm_wgrad_batch_workspace(int(M), 4, block_jobs);
-        // One launch for all weight gradients where the shapes allow it (every width a multiple of 256)
-        size_t table_bytes = 0;
+        size_t need = std::max(tgk_attn_bwd_workspace(c.batch, model->heads, c.context), tgk_layernorm_bwd_workspace(int(M), int(d)));
         for (Slot &slot : e->slots) {
             std::vector<TgkWgradJob> &jobs = slot.wgrad_jobs;
             for (int l = 0; l < c.depth; ++l)
@@ -703,82 +652,67 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
                     jobs.push_back(block_jobs[j]);
             jobs.push_back({int(V), int(d), nullptr, int(V), nullptr, int(d), nullptr, int(d)}); // the head
             jobs.push_back({int(V), int(d), nullptr, int(V), nullptr, int(d), nullptr, int(d)}); // the token table
-            table_bytes = tgk_gemm_wgrad_list_table_bytes(int(M), int(jobs.size()), jobs.data());
-        }
-        e->list_wgrad = table_bytes > 0;
-        if (e->list_wgrad) {
-            batch_need = 0;
-            for (Slot &slot : e->slots) {
-                slot.g_x.resize(c.depth + 1), slot.g_mid.resize(c.depth), slot.g_u.resize(c.depth), slot.g_qkv.resize(c.depth);
-                for (int l = 0; l <= c.depth; ++l)
-                    e->allocate(slot.g_x[l], M * d, false);
-                for (int l = 0; l < c.depth; ++l) {
-                    e->allocate(slot.g_mid[l], M * d, false);
-                    e->allocate(slot.g_u[l], M * F, false);
-                    e->allocate(slot.g_qkv[l], M * 3 * d, false);
-                    const TgLayerParameters &p = e->layout.layers[l];
-                    const LayerBuffers &b = slot.layers[l];
-                    float *g = slot.gradient;
-                    TgkWgradJob *jobs = slot.wgrad_jobs.data() + 4 * l;
-                    jobs[0].dY = slot.g_x[l + 1], jobs[0].X = b.a, jobs[0].dW = g + p.mlp_down;
-                    jobs[1].dY = slot.g_u[l], jobs[1].X = b.n2, jobs[1].dW = g + p.mlp_up;
-                    jobs[2].dY = slot.g_mid[l], jobs[2].X = b.o, jobs[2].dW = g + p.attn_out;
-                    jobs[3].dY = slot.g_qkv[l], jobs[3].X = b.n1, jobs[3].dW = g + p.qkv;
-                }
-                TgkWgradJob &head = slot.wgrad_jobs[4 * c.depth], &table_job = slot.wgrad_jobs[4 * c.depth + 1];
-                head.dY = slot.logits, head.X = slot.nf, head.dW = slot.gradient + e->layout.head;
-                e->allocate(slot.onehot, M * V, false);
-                table_job.dY = slot.onehot, table_job.X = slot.g_x[0], table_job.dW = slot.gradient + e->layout.embedding;
-                uint8_t *table = nullptr;
-                e->allocate(table, table_bytes, false);
-                slot.wgrad_table = table;
-                ok(tgk_gemm_wgrad_list_prepare(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), table, table_bytes));
-                // the tensors no matrix product writes, in ranges of at most 8192 elements; with the matrices they
-                // must cover the flat gradient exactly
-                struct Range {
-                    int64_t start, length;
-                };
-                std::vector<Range> ranges;
-                int64_t covered = 2 * int64_t(V) * d; // the head and the token table
-                const auto cover = [&](int64_t start, int64_t length) {
-                    covered += length;
-                    for (int64_t at = 0; at < length; at += 8192)
-                        ranges.push_back({start + at, std::min<int64_t>(8192, length - at)});
-                };
-                cover(e->layout.positions, int64_t(c.context) * d);
-                for (int l = 0; l < c.depth; ++l) {
-                    const TgLayerParameters &p = e->layout.layers[l];
-                    cover(p.ln1_g, d), cover(p.ln1_b, d), cover(p.ln2_g, d), cover(p.ln2_b, d);
-                    covered += 4 * int64_t(d) * d + 2 * int64_t(F) * d;
-                }
-                cover(e->layout.lnf_g, d), cover(e->layout.lnf_b, d);
-                if (covered != e->layout.count)
-                    throw std::runtime_error("engine: gradient norm ranges do not cover the parameters");
-                slot.list_norms = tgk_gemm_wgrad_list_sumsq_count(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data());
-                slot.range_norms = int(ranges.size());
-                if (slot.list_norms <= 0 || slot.list_norms + slot.range_norms > 4096)
-                    throw std::runtime_error("engine: too many gradient norm partials");
-                e->allocate(slot.norms, size_t(slot.list_norms + slot.range_norms), false);
-                uint8_t *device_ranges = nullptr;
-                e->allocate(device_ranges, ranges.size() * sizeof(Range), false);
-                check_hip(hipMemcpy(device_ranges, ranges.data(), ranges.size() * sizeof(Range), hipMemcpyHostToDevice),
-                          "norm ranges: ");
-                slot.norm_ranges = device_ranges;
-                batch_need = std::max(batch_need, tgk_gemm_wgrad_list_workspace(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data()));
+            const size_t table_bytes = wgrad_list_table_bytes(int(M), int(jobs.size()), jobs.data(), ListUnit);
+            if (!table_bytes)
+                throw std::runtime_error("engine: weight gradients do not fit one list");
+            slot.g_x.resize(c.depth + 1), slot.g_mid.resize(c.depth), slot.g_u.resize(c.depth), slot.g_qkv.resize(c.depth);
+            for (int l = 0; l <= c.depth; ++l)
+                e->allocate(slot.g_x[l], M * d, false);
+            for (int l = 0; l < c.depth; ++l) {
+                e->allocate(slot.g_mid[l], M * d, false);
+                e->allocate(slot.g_u[l], M * F, false);
+                e->allocate(slot.g_qkv[l], M * 3 * d, false);
+                const TgLayerParameters &p = e->layout.layers[l];
+                const LayerBuffers &b = slot.layers[l];
+                float *g = slot.gradient;
+                TgkWgradJob *jobs = slot.wgrad_jobs.data() + 4 * l;
+                jobs[0].dY = slot.g_x[l + 1], jobs[0].X = b.a, jobs[0].dW = g + p.mlp_down;
+                jobs[1].dY = slot.g_u[l], jobs[1].X = b.n2, jobs[1].dW = g + p.mlp_up;
+                jobs[2].dY = slot.g_mid[l], jobs[2].X = b.o, jobs[2].dW = g + p.attn_out;
+                jobs[3].dY = slot.g_qkv[l], jobs[3].X = b.n1, jobs[3].dW = g + p.qkv;
             }
+            TgkWgradJob &head = slot.wgrad_jobs[4 * c.depth], &table_job = slot.wgrad_jobs[4 * c.depth + 1];
+            head.dY = slot.logits, head.X = slot.nf, head.dW = slot.gradient + e->layout.head;
+            e->allocate(slot.onehot, M * V, false);
+            table_job.dY = slot.onehot, table_job.X = slot.g_x[0], table_job.dW = slot.gradient + e->layout.embedding;
+            uint8_t *table = nullptr;
+            e->allocate(table, table_bytes, false);
+            slot.wgrad_table = table;
+            wgrad_list_prepare(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit, table, table_bytes);
+            // the tensors no matrix product writes, in ranges of 8192 elements (more where a long context would make
+            // too many of them); with the matrices they must cover the flat gradient exactly
+            struct Range {
+                int64_t start, length;
+            };
+            std::vector<Range> ranges;
+            const int64_t range = std::max<int64_t>(8192, (int64_t(c.context) * int64_t(d) / 1024 + 3) / 4 * 4);
+            int64_t covered = 2 * int64_t(V) * d; // the head and the token table
+            const auto cover = [&](int64_t start, int64_t length) {
+                covered += length;
+                for (int64_t at = 0; at < length; at += range)
+                    ranges.push_back({start + at, std::min<int64_t>(range, length - at)});
+            };
+            cover(e->layout.positions, int64_t(c.context) * d);
+            for (int l = 0; l < c.depth; ++l) {
+                const TgLayerParameters &p = e->layout.layers[l];
+                cover(p.ln1_g, d), cover(p.ln1_b, d), cover(p.ln2_g, d), cover(p.ln2_b, d);
+                covered += 4 * int64_t(d) * d + 2 * int64_t(F) * d;
+            }
+            cover(e->layout.lnf_g, d), cover(e->layout.lnf_b, d);
+            if (covered != e->layout.count)
+                throw std::runtime_error("engine: gradient norm ranges do not cover the parameters");
+            slot.list_norms = wgrad_list_sumsq_count(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit);
+            slot.range_norms = int(ranges.size());
+            if (slot.list_norms <= 0 || slot.list_norms + slot.range_norms > 4096)
+                throw std::runtime_error("engine: too many gradient norm partials");
+            e->allocate(slot.norms, size_t(slot.list_norms + slot.range_norms), false);
+            uint8_t *device_ranges = nullptr;
+            e->allocate(device_ranges, ranges.size() * sizeof(Range), false);
+            check_hip(hipMemcpy(device_ranges, ranges.data(), ranges.size() * sizeof(Range), hipMemcpyHostToDevice),
+                      "norm ranges: ");
+            slot.norm_ranges = device_ranges;
+            need = std::max(need, wgrad_list_workspace(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit));
         }
-        e->batched_wgrad = !e->list_wgrad && batch_need > 0;
-        if (e->batched_wgrad)
-            for (Slot &slot : e->slots)
-                e->allocate(slot.dh_mid, M * d, false);
-        size_t need = std::max(batch_need, tgk_attn_bwd_workspace(c.batch, model->heads, c.context));
-        need = std::max(need, tgk_layernorm_bwd_workspace(int(M), int(d)));
-        need = std::max(need, tgk_embed_bwd_workspace(int(M), int(d)));
-        need = std::max(need, tgk_gemm_wgrad_workspace(int(M), int(V), int(d)));
-        need = std::max(need, tgk_gemm_wgrad_workspace(int(M), int(d), int(F)));
-        need = std::max(need, tgk_gemm_wgrad_workspace(int(M), int(F), int(d)));
-        need = std::max(need, tgk_gemm_wgrad_workspace(int(M), int(d), int(d)));
-        need = std::max(need, tgk_gemm_wgrad_workspace(int(M), int(3 * d), int(d)));
         e->workspace_bytes = need;
         const int norms = 2 * c.depth + 1;
         const size_t ln_stride = tgk_layernorm_bwd_workspace(int(M), int(d));

@@ -25,6 +25,7 @@
 // tiles, k-contiguous operands) gemm64_kernel otherwise, gemm_kernel where 64 does not divide the reduced dimension.
 // Weight gradients: wgrad_list_kernel, wgrad_batch_kernel (several matrices in one launch), gemm64_kernel / gemm_kernel.
 #include "common.h"
+#include "gemm_list.h"
 #include <atomic>
 #include <type_traits>
 #include <vector>
@@ -522,18 +523,18 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const bf16_t *__restrict__
 // ---- 64 k per stage, two stages --------------------------------------------------------------------
 // k-contiguous tile of ROWS rows x 64 k: 128-byte rows (every copy request is a whole cache line), 16-byte
 // chunk c of row r stored at chunk c ^ ((r >> 1) & 7): conflict-free for ds_read_b128 with 64 banks.
-template <int ROWS, int WAVES = 4> struct TileKC64 {
-    static constexpr int LOADS = ROWS * 128 / (WAVES * 1024); // wave-wide copies per thread per stage
+template <int ROWS> struct TileKC64 {
+    static constexpr int LOADS = ROWS * 128 / 4096; // wave-wide copies per thread per stage
     static constexpr int BYTES = ROWS * 128;
     TG_DEVICE static int64_t step(int) { return 64; } // elements from one stage to the next
     TG_DEVICE static int64_t origin(int row0, int k0, int ld) { return int64_t(row0) * ld + k0; }
     TG_DEVICE static int64_t source_offset(int j, int tid, int ld) {
         const int wave = tid >> 6, lane = tid & 63;
-        const int row = (j * WAVES + wave) * 8 + (lane >> 3), phys = lane & 7;
+        const int row = (j * 4 + wave) * 8 + (lane >> 3), phys = lane & 7;
         const int chunk = phys ^ ((row >> 1) & 7);
         return int64_t(row) * ld + chunk * 8;
     }
-    TG_DEVICE static uint32_t lds_offset(int j, int tid) { return uint32_t((j * WAVES + (tid >> 6)) * 1024); }
+    TG_DEVICE static uint32_t lds_offset(int j, int tid) { return uint32_t((j * 4 + (tid >> 6)) * 1024); }
     // fragment for rows row0 + lane%32, 16-k step ks of the stage (0..3): k = ks*16 + 8*(lane/32) .. +7
     TG_DEVICE static bf16x8 frag(const unsigned char *tile, int row0, int ks, int lane) {
         const int row = row0 + (lane & 31), chunk = (ks * 2 + (lane >> 5)) ^ ((row >> 1) & 7);
@@ -546,19 +547,19 @@ template <int ROWS, int WAVES = 4> struct TileKC64 {
     }
 };
 // k-strided tile: 64 k-rows x ROWS columns in the natural [k][row] image, swizzled and read like TileKS
-template <int ROWS, int WAVES = 4> struct TileKS64 {
-    static constexpr int LOADS = ROWS * 128 / (WAVES * 1024);
+template <int ROWS> struct TileKS64 {
+    static constexpr int LOADS = ROWS * 128 / 4096;
     static constexpr int BYTES = ROWS * 128;
     static constexpr int CHUNKS_PER_ROW = ROWS / 8;
     TG_DEVICE static int64_t step(int ld) { return int64_t(64) * ld; }
     TG_DEVICE static int64_t origin(int row0, int k0, int ld) { return int64_t(k0) * ld + row0; }
     TG_DEVICE static int64_t source_offset(int j, int tid, int ld) {
         const int wave = tid >> 6, lane = tid & 63;
-        const int q = (j * WAVES + wave) * 64 + lane, r = q / CHUNKS_PER_ROW, p = q - r * CHUNKS_PER_ROW;
+        const int q = (j * 4 + wave) * 64 + lane, r = q / CHUNKS_PER_ROW, p = q - r * CHUNKS_PER_ROW;
         const int chunk = p ^ TileKS<ROWS>::swizzle(r);
         return int64_t(r) * ld + chunk * 8;
     }
-    TG_DEVICE static uint32_t lds_offset(int j, int tid) { return uint32_t((j * WAVES + (tid >> 6)) * 1024); }
+    TG_DEVICE static uint32_t lds_offset(int j, int tid) { return uint32_t((j * 4 + (tid >> 6)) * 1024); }
     TG_DEVICE static bf16x8 frag(const unsigned char *tile, int row0, int ks, int lane) {
         return TileKS<ROWS>::frag(tile, row0, ks, lane); // k-rows ks*16 .. of the 64
     }
@@ -566,9 +567,9 @@ template <int ROWS, int WAVES = 4> struct TileKS64 {
         return TileKS<ROWS>::frag16(tile, row0, ks * 32, lane); // k-rows ks*32 .. of the 64
     }
 };
-template <int ROWS, bool KC, int WAVES = 4> struct Tile64Of;
-template <int ROWS, int WAVES> struct Tile64Of<ROWS, true, WAVES> { using type = TileKC64<ROWS, WAVES>; };
-template <int ROWS, int WAVES> struct Tile64Of<ROWS, false, WAVES> { using type = TileKS64<ROWS, WAVES>; };
+template <int ROWS, bool KC> struct Tile64Of;
+template <int ROWS> struct Tile64Of<ROWS, true> { using type = TileKC64<ROWS>; };
+template <int ROWS> struct Tile64Of<ROWS, false> { using type = TileKS64<ROWS>; };
 
 // One 64-k stage of a wave's FM x FN blocks of 32 x 32 with v_mfma_f32_16x16x32_bf16: two 32-k steps, every block as
 // 2 x 2 tiles of 16 x 16.  The kernels run against the board's power limit, and on random operands this instruction
@@ -741,120 +742,128 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
     wait_vmcnt<0>();
 }
 
+// The product of one BM x BN tile over k_chunks stages of 64 k, each operand either way round; four waves of
+// BM / 2 x BN / 2 outputs.  S - 1 stages are in flight, and a stage is one wait, one barrier, every fragment read at
+// once (one LDS round trip; read column by column as in multiply_stage, 1024 x 768 with K = 3072 took 17.1 us instead of
+// 13.9), the copies of the stage S - 1 further on, then the matrix instructions, which add in the same order as
+// gemm64_kernel.  Ends behind a barrier: the slots are free.
+template <int BM, int BN, int S, bool AKC, bool BKC> struct TileProduct {
+    using TA = typename Tile64Of<BM, AKC>::type;
+    using TB = typename Tile64Of<BN, BKC>::type;
+    static constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, THREADS = 256;
+    static constexpr int LA = TA::LOADS, LB = TB::LOADS, LOADS = LA + LB, SLOT = TA::BYTES + TB::BYTES;
+    static_assert(S >= 2 && (S - 1) * LOADS <= 63, "the copies in flight fit the wave's counter");
+    TG_DEVICE static void run(const bf16_t *A, int lda, const bf16_t *B, int ldb, int m0, int n0, int k_chunks,
+                              unsigned char *smem, f32x4 (&acc)[FM][FN][2][2]) {
+        const uint32_t smem_base = lds_address(smem);
+        const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+        const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+        const bf16_t *pa[LA], *pb[LB];
+        const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
+#pragma unroll
+        for (int j = 0; j < LA; ++j)
+            pa[j] = A + TA::origin(m0, 0, lda) + TA::source_offset(j, tid, lda);
+#pragma unroll
+        for (int j = 0; j < LB; ++j)
+            pb[j] = B + TB::origin(n0, 0, ldb) + TB::source_offset(j, tid, ldb);
+        int p_slot = 0;
+        auto copy_stage = [&]() {
+            const uint32_t to = smem_base + uint32_t(p_slot) * SLOT;
+#pragma unroll
+            for (int j = 0; j < LA; ++j) {
+                async_copy16(__builtin_amdgcn_readfirstlane(to + TA::lds_offset(j, tid)), pa[j]);
+                pa[j] += a_step;
+            }
+#pragma unroll
+            for (int j = 0; j < LB; ++j) {
+                async_copy16(__builtin_amdgcn_readfirstlane(to + TA::BYTES + TB::lds_offset(j, tid)), pb[j]);
+                pb[j] += b_step;
+            }
+            p_slot = p_slot + 1 == S ? 0 : p_slot + 1;
+        };
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[i][j][t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S - 1; ++s)
+            if (s < k_chunks)
+                copy_stage();
+        int c_slot = 0;
+        for (int c = 0; c < k_chunks; ++c) {
+            // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
+            const int younger = k_chunks - 1 - c;
+            if (S >= 4 && younger >= 2)
+                wait_vmcnt<(S >= 4 ? 2 : 0) * LOADS>();
+            else if (S >= 3 && younger >= 1)
+                wait_vmcnt<(S >= 3 ? 1 : 0) * LOADS>();
+            else
+                wait_vmcnt<0>();
+            __syncthreads(); // everyone's copies are there, and everyone is done with the slot that is refilled next
+            const unsigned char *sa = smem + c_slot * SLOT, *sb = sa + TA::BYTES;
+            bf16x8 af[2][2 * FM], bfr[2][2 * FN];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+                for (int i = 0; i < 2 * FM; ++i)
+                    af[ks][i] = TA::frag16(sa, wm + i * 16, ks, lane);
+#pragma unroll
+                for (int j = 0; j < 2 * FN; ++j)
+                    bfr[ks][j] = TB::frag16(sb, wn + j * 16, ks, lane);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (c + S - 1 < k_chunks)
+                copy_stage();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int j = 0; j < 2 * FN; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2 * FM; ++i) {
+                        f32x4 &t = acc[i >> 1][j >> 1][i & 1][j & 1];
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], t, 0, 0, 0);
+                    }
+            c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
+        }
+        __syncthreads(); // other waves may still read the last stage
+    }
+};
+// Consecutive block ids sit on consecutive XCDs: the place in a row-major list of tiles that gives each XCD a contiguous run.
+TG_DEVICE int xcd_contiguous(int block, int blocks) {
+    const int xcd = block & 7;
+    return xcd * (blocks >> 3) + min(xcd, blocks & 7) + (block >> 3);
+}
+
 // ---- one tile per block: forward and input-gradient products of ordinary and small sizes ----------------------------
 // C = A B^T with A k-contiguous and B either way round.  A product with few outputs is bound by how many compute units
 // have a tile and by the latency of each 64-k stage on them, not by bytes per flop: 1024 x 768 outputs are 32 tiles of
-// 128 x 192 but 192 of 64 x 64.  So the tile is a parameter (choose_block), a block computes one of them, S - 1 stages
-// are in flight, and a stage is one wait, one barrier, every fragment read at once (one LDS round trip; read column by
-// column as in multiply_stage, 1024 x 768 with K = 3072 took 17.1 us instead of 13.9), the copies of the stage S - 1
-// further on, then the matrix instructions, which add in the same order as the other 64-k kernels: results are
-// bit-identical whatever the tile.  Tried and slower: reading stage c + 1's fragments under stage c's products (16.6 us).
+// 128 x 192 but 192 of 64 x 64.  So the tile is a parameter (choose_block) and a block computes one of them; the sums run in
+// the same order whatever the tile: results are bit-identical.  Tried and slower at 1024 x 768, K = 3072: reading stage
+// c + 1's fragments under stage c's products (16.6 us).
 // Measured against the 128-row tiles that took these shapes before, us (M x N, K; weights [N][K]): 2048 x 256, 1024: 12.6 ->
 // 6.2; 1920 x 640, 1920: 25.5 -> 12.9; 1024 x 768, 3072: 40.6 -> 14.9; 1024 x 2304, 768: 13.2 -> 9.0; 8192 x 512, 2048: 28.5 ->
 // 22.3; 16384 x 256, 768: 13.4 -> 10.6; with B k-strided (weights [K][N]) 1024 x 768, 3072: 55.1 -> 15.2; 4096 x 3072, 768: 27.6 -> 22.8;
 // 16384 x 2304, 768: 77.0 -> 67.6.
 template <int BM, int BN, int S, bool BKC, class Epilogue>
-__global__ __launch_bounds__(BM * 4 < 256 ? BM * 4 : 256) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda,
-                                                                             const bf16_t *__restrict__ B, int ldb,
-                                                                             int k_chunks, int tiles_n, Epilogue epilogue) {
-    constexpr int WAVES = BM * 4 < 256 ? BM / 16 : 4;
-    using TA = typename Tile64Of<BM, true, WAVES>::type;
-    using TB = typename Tile64Of<BN, BKC, WAVES>::type;
-    constexpr int WM = BM * 2 / WAVES, WN = BN / 2, FM = WM / 32, FN = WN / 32;
-    constexpr int LA = TA::LOADS, LB = TB::LOADS, LOADS = LA + LB, SLOT = TA::BYTES + TB::BYTES;
-    static_assert(S >= 2 && (S - 1) * LOADS <= 63, "the copies in flight fit the wave's counter");
-    static_assert(WAVES * 2048 <= SLOT, "the epilogue buffers fit one stage");
+__global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B,
+                                                        int ldb, int k_chunks, int tiles_n, Epilogue epilogue) {
+    using P = TileProduct<BM, BN, S, true, BKC>;
+    static_assert(4 * 2048 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
-    const uint32_t smem_base = lds_address(smem);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
-    // consecutive block ids sit on consecutive XCDs: give each XCD a contiguous run of tiles, row-major
-    const int blocks = gridDim.x, xcd = blockIdx.x & 7;
-    const int tile = xcd * (blocks >> 3) + min(xcd, blocks & 7) + (blockIdx.x >> 3);
-    const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
-
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tile = xcd_contiguous(blockIdx.x, gridDim.x), m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+    const int m = m0 + (wave >> 1) * P::WM, n = n0 + (wave & 1) * P::WN;
     // the epilogue's second input first of all: it lands before the operands do
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
     if (epilogue.wants_aux())
-        load_aux_pair<FM, FN>(epilogue, 0, m0 + wm, n0 + wn, lane, aux);
-
-    const bf16_t *pa[LA], *pb[LB];
-    const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
-#pragma unroll
-    for (int j = 0; j < LA; ++j)
-        pa[j] = A + TA::origin(m0, 0, lda) + TA::source_offset(j, tid, lda);
-#pragma unroll
-    for (int j = 0; j < LB; ++j)
-        pb[j] = B + TB::origin(n0, 0, ldb) + TB::source_offset(j, tid, ldb);
-    int p_slot = 0;
-    auto copy_one = [&](int n) { // n-th of the LOADS copies of a stage, into slot p_slot
-        const uint32_t to = smem_base + uint32_t(p_slot) * SLOT;
-        if (n < LA) {
-            async_copy16(__builtin_amdgcn_readfirstlane(to + TA::lds_offset(n, tid)), pa[n]);
-            pa[n] += a_step;
-        } else {
-            async_copy16(__builtin_amdgcn_readfirstlane(to + TA::BYTES + TB::lds_offset(n - LA, tid)), pb[n - LA]);
-            pb[n - LA] += b_step;
-        }
-    };
-    auto copy_stage = [&]() {
-#pragma unroll
-        for (int n = 0; n < LOADS; ++n)
-            copy_one(n);
-        p_slot = p_slot + 1 == S ? 0 : p_slot + 1;
-    };
-    f32x4 acc[FM][FN][2][2];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                acc[i][j][t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < S - 1; ++s)
-        if (s < k_chunks)
-            copy_stage();
-    int c_slot = 0;
-    for (int c = 0; c < k_chunks; ++c) {
-        // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
-        const int younger = k_chunks - 1 - c;
-        if (S >= 4 && younger >= 2)
-            wait_vmcnt<(S >= 4 ? 2 : 0) * LOADS>();
-        else if (S >= 3 && younger >= 1)
-            wait_vmcnt<(S >= 3 ? 1 : 0) * LOADS>();
-        else
-            wait_vmcnt<0>();
-        __syncthreads(); // everyone's copies are there, and everyone is done with the slot that is refilled next
-        // every fragment of the stage is requested before the first matrix instruction: one LDS round trip a stage
-        const unsigned char *sa = smem + c_slot * SLOT, *sb = sa + TA::BYTES;
-        bf16x8 af[2][2 * FM], bfr[2][2 * FN];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-            for (int i = 0; i < 2 * FM; ++i)
-                af[ks][i] = TA::frag16(sa, wm + i * 16, ks, lane);
-#pragma unroll
-            for (int j = 0; j < 2 * FN; ++j)
-                bfr[ks][j] = TB::frag16(sb, wn + j * 16, ks, lane);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (c + S - 1 < k_chunks)
-            copy_stage();
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int j = 0; j < 2 * FN; ++j)
-#pragma unroll
-                for (int i = 0; i < 2 * FM; ++i) {
-                    f32x4 &t = acc[i >> 1][j >> 1][i & 1][j & 1];
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], t, 0, 0, 0);
-                }
-        c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
-    }
-    __syncthreads(); // other waves may still read the last stage
-    staged_store_bf16<FM, FN>(acc, aux, smem + wave * 2048, epilogue, m0 + wm, n0 + wn, lane);
+        load_aux_pair<P::FM, P::FN>(epilogue, 0, m, n, lane, aux);
+    f32x4 acc[P::FM][P::FN][2][2];
+    P::run(A, lda, B, ldb, m0, n0, k_chunks, smem, acc);
+    staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
 }
 
 TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64::frag16's address
@@ -1336,7 +1345,6 @@ struct WgradList {
     int rounds;               // whole tiles per block
     int rem_tiles, rem_splits; // the tiles after rounds * blocks, each cut into rem_splits token ranges
     int k_quads;              // tokens / 128
-    int accumulate;
     float *pieces; // rem_tiles * rem_splits partial tiles of 256 * BN floats, row major
     float *sumsq;  // optional: sums of squares of the gradients written, four per block of the product launch (one per
                    // wave) followed by one per block of the fold launch
@@ -1577,6 +1585,54 @@ __global__ __launch_bounds__(256, 1) void wgrad_list_kernel(const WgradList w) {
     }
 }
 // Sums the pieces of the split tiles, in token order, into the gradient.  Eight blocks per tile.
+// The same list on ordinary tiles, each summed over all tokens by one block: where 256 x 256 tiles would not fill the
+// compute units or do not fit the widths, and for a single gradient.  Block b of g takes tiles b, b + g, ...; nothing is
+// cut along the tokens, so nothing is folded.  What bounds it is a stage's latency on a unit with one tile and the
+// transposing LDS reads on one with several (0.24 and 0.20 us for 64 x 64 outputs, 0.66 and 0.55 for 128 x 128).
+struct WgradTiles {
+    const WgradListJob *jobs; // device memory; NULL: `one`, its tiles row-major, tiles_n a row
+    const int4 *tiles;
+    WgradListJob one;
+    int tiles_n, count, k_chunks, accumulate;
+    float *sumsq; // optional: one sum of squares a block
+};
+template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_tiles_kernel(const WgradTiles w) {
+    using P = TileProduct<BM, BN, S, false, false>;
+    static_assert(4 * 4096 <= P::SLOT, "the epilogue buffers fit one stage");
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ float waves[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float squares = 0.f;
+    for (int base = 0; base + int(blockIdx.x) < w.count; base += gridDim.x) {
+        const int at = base + xcd_contiguous(blockIdx.x, min(int(gridDim.x), w.count - base));
+        const int4 t = w.jobs ? w.tiles[at] : make_int4(0, at / w.tiles_n * BM, at % w.tiles_n * BN, 0);
+        const WgradListJob job = w.jobs ? w.jobs[t.x] : w.one;
+        f32x4 acc[P::FM][P::FN][2][2];
+        P::run(job.dy, job.lddy, job.x, job.ldx, t.y, t.z, w.k_chunks, smem, acc);
+        const EpilogueF32 epilogue{job.dw, job.lddw, 0, w.accumulate};
+        staged_store_f32<P::FM, P::FN>(acc, smem + wave * 4096, epilogue, t.y + (wave >> 1) * P::WM, t.z + (wave & 1) * P::WN,
+                                       lane, 0);
+        if (w.sumsq)
+#pragma unroll
+            for (int i = 0; i < P::FM; ++i)
+#pragma unroll
+                for (int j = 0; j < P::FN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4 v = acc[i][j][q >> 1][q & 1];
+                        squares += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+                    }
+        __syncthreads(); // the next tile's copies go where the stores were staged
+    }
+    if (w.sumsq) {
+        squares = wave_sum(squares);
+        if (lane == 0)
+            waves[wave] = squares;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            w.sumsq[blockIdx.x] = (waves[0] + waves[1]) + (waves[2] + waves[3]);
+    }
+}
 template <int BN>
 __global__ __launch_bounds__(256) void wgrad_list_fold_kernel(const WgradList w, int first_tile, int first_sumsq) {
     constexpr int BM = 256, QUADS = BM * BN / 4 / 8 / 256; // float4 per thread
@@ -1594,8 +1650,6 @@ __global__ __launch_bounds__(256) void wgrad_list_fold_kernel(const WgradList w,
         for (int split = 0; split < w.rem_splits; ++split) // fixed order
             sum += *reinterpret_cast<const f32x4 *>(first + size_t(split) * (BM * BN) + size_t(quad) * 4);
         f32x4 *p = reinterpret_cast<f32x4 *>(job.dw + size_t(t.y + row) * job.lddw + t.z + col);
-        if (w.accumulate)
-            sum += *p;
         __builtin_nontemporal_store(sum, p);
         squares += (sum[0] * sum[0] + sum[1] * sum[1]) + (sum[2] * sum[2] + sum[3] * sum[3]);
     }
@@ -1836,7 +1890,7 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(BM * 4 < 256 ? BM * 4 : 256), lds, stream, A, lda, B, ldb,
+    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256), lds, stream, A, lda, B, ldb,
                        K / 64, N / BN, epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
@@ -1902,6 +1956,21 @@ void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_
     }
 }
 
+template <int BM, int BN, int S> void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int blocks) {
+    auto kernel = wgrad_tiles_kernel<BM, BN, S>;
+    constexpr size_t lds = S * (BM + BN) * 128;
+    static std::atomic<bool> configured[MAX_DEVICES];
+    const int device = current_device();
+    if (!configured[device].load(std::memory_order_acquire)) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
+                  "gemm LDS size: ");
+        configured[device].store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, w);
+    check_hip(hipGetLastError(), "wgrad tiles launch: ");
+}
+
 void check_operand(const void *p, int ld, const char *name) {
     if (!p || (reinterpret_cast<uintptr_t>(p) & 15) || ld % 8)
         throw std::invalid_argument(std::string("gemm operand ") + name +
@@ -1915,6 +1984,23 @@ int wgrad_splits(Tile tile, int tiles, int k_tiles) {
         splits = 1;
     const int max_by_k = k_tiles / 8 > 0 ? k_tiles / 8 : 1; // at least 8 k-tiles (256 tokens) per split
     return splits < max_by_k ? splits : max_by_k;
+}
+
+// One weight gradient on 64 x 64 tiles, every one over all tokens, or split along the tokens into slabs that a second launch
+// folds?  Estimates in us: a stage of 64 tokens on the fullest unit, against two launches, the slabs written and read at
+// 6 TB/s and the products at 0.95 PFLOP/s.  Either side (tokens, N x K; tiles against slabs, measured): 1920, 640 x 1920 15.4 /
+// 22.8; 1024, 2304 x 768 9.4 / 23.9; 4096, 768 x 768 20.5 / 24.6; 4096, 3072 x 768 36.0 / 36.0; 8192, 512 x 512 36.4 / 25.6;
+// 16384, 768 x 768 70.8 / 34.7.
+bool wgrad_on_tiles(int M, int N, int K) {
+    if (M % 64)
+        return false;
+    const Tile tile = choose_tile(N, K);
+    const int splits = wgrad_splits(tile, (N / tile_rows(tile)) * (K / tile_cols(tile)), M / BK);
+    const double elements = double(N) * K;
+    const int units = compute_units(), deepest = int((elements / 4096 + units - 1) / units);
+    const double tiles_us = 3.5 + M / 64 * (deepest == 1 ? 0.24 : 0.20 * deepest);
+    const double slabs_us = (splits > 1 ? 6 + 8e-6 * splits * elements / 6 : 3.5) + 2e-9 * M * elements / 0.95;
+    return tiles_us < slabs_us;
 }
 
 } // namespace
@@ -2052,6 +2138,12 @@ extern "C" int tgk_gemm_wgrad(hipStream_t stream, int M, int N, int K, const uin
         check_operand(X, ldx, "X");
         require(dW && !(reinterpret_cast<uintptr_t>(dW) & 15) && lddw % 4 == 0,
                 "gemm_wgrad: dW must be 16-byte aligned with leading dimension % 4 == 0");
+        if (wgrad_on_tiles(M, N, K)) {
+            WgradTiles w{};
+            w.one = {dY, X, dW, lddy, ldx, lddw, 0};
+            w.tiles_n = K / 64, w.count = (N / 64) * (K / 64), w.k_chunks = M / 64, w.accumulate = accumulate;
+            return launch_wgrad_tiles<64, 64, 3>(stream, w, w.count);
+        }
         const int splits = wgrad_splits(tile, (N / tile_rows(tile)) * (K / tile_cols(tile)), M / BK);
         if (splits == 1) {
             EpilogueF32 e{dW, lddw, 0, accumulate};
@@ -2181,10 +2273,15 @@ extern "C" int tgk_gemm_wgrad_batch(hipStream_t stream, int M, int count, const 
 namespace {
 // Tables and split of a whole-step weight-gradient launch.
 struct WgradListPlan {
+    int edge; // of a tile: 256 (wgrad_list_kernel, fold), or 128 or 64 (wgrad_tiles_kernel)
     int tiles, blocks, rounds, rem_tiles, rem_splits, launch_blocks, fold_blocks;
     size_t jobs_bytes, table_bytes, pieces_bytes;
 };
-bool plan_wgrad_list(int M, int count, const TgkWgradJob *jobs, WgradListPlan &plan, std::string &why) {
+// `unit`: what every width has to be a multiple of.  The tile is the one with the least time by these estimates (us, a
+// stage = 64 tokens of the deepest unit's tiles): 256 x 256: 1.34 a stage in whole rounds, and for the rest 10 + 1.5 a
+// stage, + 15 where it is cut into token ranges and folded; 128 x 128: 0.66 a stage alone on a unit, 0.55 each with
+// company; 64 x 64: 0.24 and 0.20.  Measured: 26 products of d_model 256 over 2048 tokens 46 us on 256, 31 on 128.
+bool plan_wgrad_list(int M, int count, const TgkWgradJob *jobs, int unit, WgradListPlan &plan, std::string &why) {
     if (count < 1 || count > 4096 || !jobs) {
         why = "gemm_wgrad_list: between 1 and 4096 jobs";
         return false;
@@ -2193,61 +2290,76 @@ bool plan_wgrad_list(int M, int count, const TgkWgradJob *jobs, WgradListPlan &p
         why = "gemm_wgrad_list: M (the reduced dimension) must be a multiple of 128";
         return false;
     }
-    int tiles = 0;
+    int64_t elements = 0;
+    bool by_256 = true;
     for (int j = 0; j < count; ++j) {
-        if (jobs[j].N <= 0 || jobs[j].K <= 0 || jobs[j].N % 256 || jobs[j].K % 256) {
-            why = "gemm_wgrad_list: every N and K must be a multiple of 256";
+        if (jobs[j].N <= 0 || jobs[j].K <= 0 || jobs[j].N % unit || jobs[j].K % unit) {
+            why = "gemm_wgrad_list: every N and K must be a multiple of " + std::to_string(unit);
             return false;
         }
-        tiles += (jobs[j].N / 256) * (jobs[j].K / 256);
+        by_256 = by_256 && jobs[j].N % 256 == 0 && jobs[j].K % 256 == 0;
+        elements += int64_t(jobs[j].N) * jobs[j].K;
     }
-    plan.tiles = tiles;
-    plan.blocks = compute_units();
-    plan.rounds = tiles / plan.blocks;
-    plan.rem_tiles = tiles % plan.blocks;
-    const int k_quads = M / 128;
-    plan.rem_splits = plan.rem_tiles ? std::min(plan.blocks / plan.rem_tiles, k_quads) : 1;
+    const int units = compute_units(), stages = M / 64;
+    const auto estimate = [&](int edge, double alone, double each) {
+        const int deepest = int((elements / (edge * edge) + units - 1) / units);
+        return stages * (deepest == 1 ? alone : each * deepest);
+    };
+    const double on_128 = estimate(128, 0.66, 0.55), on_64 = estimate(64, 0.24, 0.20);
+    plan = WgradListPlan{};
+    plan.edge = on_128 <= on_64 ? 128 : 64;
+    if (by_256) {
+        const int tiles = int(elements / 65536), rest = tiles % units;
+        const int splits = rest ? std::min(units / rest, stages / 2) : 1;
+        const double on_256 = tiles / units * stages * 1.34 + (rest ? 10 + (stages + splits - 1) / splits * 1.5 + (splits > 1 ? 15 : 0) : 0);
+        if (on_256 <= std::min(on_128, on_64))
+            plan.edge = 256;
+    }
+    plan.tiles = int(elements / (plan.edge * plan.edge));
+    plan.blocks = units;
     plan.jobs_bytes = (size_t(count) * sizeof(WgradListJob) + 15) / 16 * 16;
-    plan.table_bytes = plan.jobs_bytes + size_t(tiles) * sizeof(int4);
+    plan.table_bytes = plan.jobs_bytes + size_t(plan.tiles) * sizeof(int4);
+    if (plan.edge < 256) { // as many blocks as are resident together, or one a tile
+        plan.launch_blocks = std::min(plan.tiles, units * (plan.edge == 64 ? 3 : 2));
+        return true;
+    }
+    plan.rounds = plan.tiles / plan.blocks;
+    plan.rem_tiles = plan.tiles % plan.blocks;
+    plan.rem_splits = plan.rem_tiles ? std::min(plan.blocks / plan.rem_tiles, M / 128) : 1;
     plan.pieces_bytes = plan.rem_splits > 1 ? size_t(plan.rem_tiles) * plan.rem_splits * 256 * 256 * sizeof(float) : 0;
     plan.launch_blocks = plan.rounds ? plan.blocks : plan.rem_tiles * plan.rem_splits;
     plan.fold_blocks = plan.rem_splits > 1 ? plan.rem_tiles * 8 : 0;
     return true;
 }
+bool planned(int M, int count, const TgkWgradJob *jobs, int unit, WgradListPlan &plan) {
+    try {
+        std::string why;
+        return plan_wgrad_list(M, count, jobs, unit, plan, why);
+    } catch (...) {
+        return false;
+    }
+}
 } // namespace
 
-extern "C" size_t tgk_gemm_wgrad_list_table_bytes(int M, int count, const TgkWgradJob *jobs) {
-    try {
-        WgradListPlan plan;
-        std::string why;
-        return plan_wgrad_list(M, count, jobs, plan, why) ? plan.table_bytes : 0;
-    } catch (...) {
-        return 0;
-    }
+size_t wgrad_list_table_bytes(int M, int count, const TgkWgradJob *jobs, int unit) {
+    WgradListPlan plan;
+    return planned(M, count, jobs, unit, plan) ? plan.table_bytes : 0;
 }
-extern "C" size_t tgk_gemm_wgrad_list_workspace(int M, int count, const TgkWgradJob *jobs) {
-    try {
-        WgradListPlan plan;
-        std::string why;
-        return plan_wgrad_list(M, count, jobs, plan, why) ? plan.pieces_bytes : 0;
-    } catch (...) {
-        return 0;
-    }
+size_t wgrad_list_workspace(int M, int count, const TgkWgradJob *jobs, int unit) {
+    WgradListPlan plan;
+    return planned(M, count, jobs, unit, plan) ? plan.pieces_bytes : 0;
 }
-extern "C" int tgk_gemm_wgrad_list_sumsq_count(int M, int count, const TgkWgradJob *jobs) {
-    try {
-        WgradListPlan plan;
-        std::string why;
-        return plan_wgrad_list(M, count, jobs, plan, why) ? 4 * plan.launch_blocks + plan.fold_blocks : 0;
-    } catch (...) {
+int wgrad_list_sumsq_count(int M, int count, const TgkWgradJob *jobs, int unit) {
+    WgradListPlan plan;
+    if (!planned(M, count, jobs, unit, plan))
         return 0;
-    }
+    return plan.edge < 256 ? plan.launch_blocks : 4 * plan.launch_blocks + plan.fold_blocks;
 }
-extern "C" int tgk_gemm_wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, void *table, size_t table_bytes) {
-    return guarded([&] {
+void wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, int unit, void *table, size_t table_bytes) {
+    {
         WgradListPlan plan;
         std::string why;
-        if (!plan_wgrad_list(M, count, jobs, plan, why))
+        if (!plan_wgrad_list(M, count, jobs, unit, plan, why))
             throw std::invalid_argument(why);
         require(table && table_bytes >= plan.table_bytes && !(reinterpret_cast<uintptr_t>(table) & 15),
                 "gemm_wgrad_list_prepare: table too small (see tgk_gemm_wgrad_list_table_bytes)");
@@ -2263,33 +2375,40 @@ extern "C" int tgk_gemm_wgrad_list_prepare(int M, int count, const TgkWgradJob *
             require(job.dW && !(reinterpret_cast<uintptr_t>(job.dW) & 15) && job.lddw % 4 == 0 && job.lddw >= job.K,
                     "gemm_wgrad_list: dW must be 16-byte aligned with leading dimension % 4 == 0");
             job_table[j] = {job.dY, job.X, job.dW, job.lddy, job.ldx, job.lddw, 0};
-            for (int m = 0; m < job.N; m += 256)
-                for (int n = 0; n < job.K; n += 256)
+            for (int m = 0; m < job.N; m += plan.edge)
+                for (int n = 0; n < job.K; n += plan.edge)
                     tile_table[tile++] = make_int4(j, m, n, 0);
         }
         check_hip(hipMemcpy(table, host.data(), host.size(), hipMemcpyHostToDevice), "wgrad list tables: ");
-    });
+    }
 }
-extern "C" int tgk_gemm_wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, const void *table,
-                                   int accumulate, void *workspace, size_t workspace_bytes, float *sumsq) {
-    return guarded([&] {
+void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
+                size_t workspace_bytes, float *sumsq) {
+    {
         WgradListPlan plan;
         std::string why;
-        if (!plan_wgrad_list(M, count, jobs, plan, why))
+        if (!plan_wgrad_list(M, count, jobs, unit, plan, why))
             throw std::invalid_argument(why);
-        require(accumulate == 0, "gemm_wgrad_list: accumulate is not supported (every gradient is written once)");
         require(table && !(reinterpret_cast<uintptr_t>(table) & 15), "gemm_wgrad_list: no table (see tgk_gemm_wgrad_list_prepare)");
         require(plan.pieces_bytes == 0 ||
                     (workspace && workspace_bytes >= plan.pieces_bytes && !(reinterpret_cast<uintptr_t>(workspace) & 15)),
                 "gemm_wgrad_list: workspace too small (see tgk_gemm_wgrad_list_workspace)");
+        require(!(reinterpret_cast<uintptr_t>(sumsq) & 3), "gemm_wgrad_list: sumsq must be 4-byte aligned");
+        if (plan.edge < 256) {
+            WgradTiles w{};
+            w.jobs = static_cast<const WgradListJob *>(table);
+            w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
+            w.count = plan.tiles, w.k_chunks = M / 64, w.sumsq = sumsq;
+            if (plan.edge == 64)
+                return launch_wgrad_tiles<64, 64, 3>(stream, w, plan.launch_blocks);
+            return launch_wgrad_tiles<128, 128, 2>(stream, w, plan.launch_blocks);
+        }
         WgradList w{};
         w.jobs = static_cast<const WgradListJob *>(table);
         w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
         w.rounds = plan.rounds, w.rem_tiles = plan.rem_tiles, w.rem_splits = plan.rem_splits;
         w.k_quads = M / 128;
-        w.accumulate = accumulate;
         w.pieces = static_cast<float *>(workspace);
-        require(!(reinterpret_cast<uintptr_t>(sumsq) & 3), "gemm_wgrad_list: sumsq must be 4-byte aligned");
         w.sumsq = sumsq;
         auto kernel = wgrad_list_kernel<256>;
         constexpr size_t lds = 4 * (256 + 256) * 64;
@@ -2308,5 +2427,26 @@ extern "C" int tgk_gemm_wgrad_list(hipStream_t stream, int M, int count, const T
                                plan.rounds * plan.blocks, 4 * plan.launch_blocks);
             check_hip(hipGetLastError(), "wgrad list fold launch: ");
         }
+    }
+}
+
+// The public entries take widths that are multiples of 256, the engine multiples of 128.
+extern "C" size_t tgk_gemm_wgrad_list_table_bytes(int M, int count, const TgkWgradJob *jobs) {
+    return wgrad_list_table_bytes(M, count, jobs, 256);
+}
+extern "C" size_t tgk_gemm_wgrad_list_workspace(int M, int count, const TgkWgradJob *jobs) {
+    return wgrad_list_workspace(M, count, jobs, 256);
+}
+extern "C" int tgk_gemm_wgrad_list_sumsq_count(int M, int count, const TgkWgradJob *jobs) {
+    return wgrad_list_sumsq_count(M, count, jobs, 256);
+}
+extern "C" int tgk_gemm_wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, void *table, size_t table_bytes) {
+    return guarded([&] { wgrad_list_prepare(M, count, jobs, 256, table, table_bytes); });
+}
+extern "C" int tgk_gemm_wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, const void *table,
+                                   int accumulate, void *workspace, size_t workspace_bytes, float *sumsq) {
+    return guarded([&] {
+        require(accumulate == 0, "gemm_wgrad_list: accumulate is not supported (every gradient is written once)");
+        wgrad_list(stream, M, count, jobs, 256, table, workspace, workspace_bytes, sumsq);
     });
 }

@@ -1,0 +1,11 @@
+// tgk_gemm_wgrad_list for widths that are multiples of `unit` (the public entries' 256, or 128); see tgk_kernels.h.
+#pragma once
+#include "common.h"
+#include "../../include/tgk_kernels.h"
+
+size_t wgrad_list_table_bytes(int M, int count, const TgkWgradJob *jobs, int unit);
+size_t wgrad_list_workspace(int M, int count, const TgkWgradJob *jobs, int unit);
+int wgrad_list_sumsq_count(int M, int count, const TgkWgradJob *jobs, int unit);
+void wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, int unit, void *table, size_t table_bytes);
+void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
+                size_t workspace_bytes, float *sumsq);
