@@ -15,6 +15,10 @@
 // delta = rowsum(dO o O) for its queries), then dK/dV (one block per 128 keys, loops over query
 // tiles).  No atomics: every output element has one owner and a fixed summation order, so results
 // are bit-reproducible.
+//
+// Where 128-row blocks would leave the chip part idle (few or short sequences), blocks of 32 rows take their place,
+// whose four waves share out the tiles of the reduced side: attn_fwd_split_kernel, and attn_bwd_split_kernel for the
+// whole backward in one launch (split_tiles has the rule).
 #include "common.h"
 #include <atomic>
 #include "../../include/tgk_kernels.h"
@@ -120,18 +124,41 @@ struct ColFragOffsets {
 // Block placement.  The work of a causal tile grows with its index and consecutive block ids go to the
 // eight XCDs in turn, so a (tile, head, batch) grid whose tile extent is a multiple of 8 hands one XCD
 // all the heaviest tiles.  Instead each XCD takes every eighth (batch, head) pair with all of that
-// pair's tiles - which also keeps a pair's keys and values in one L2 - heaviest rank first.
+// pair's tiles - which also keeps a pair's keys and values in one L2 - heaviest rank first.  The last `dealt` pairs
+// are dealt out tile by tile instead, ahead of the others.
 struct CausalBlock {
     int rank, h, b;
     bool live;
 };
-TG_DEVICE CausalBlock causal_block(int H, int pairs) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, per_xcd = (pairs + 7) >> 3;
-    const int pair = (slot % per_xcd) * 8 + xcd;
-    return {slot / per_xcd, pair % H, pair / H, pair < pairs};
-}
-unsigned causal_grid(int tiles, int pairs) {
-    return unsigned(tiles) * unsigned((pairs + 7) / 8) * 8u;
+struct CausalGrid {
+    int H, pairs, ranks, dealt;
+    TG_DEVICE CausalBlock block(unsigned index) const {
+        const int xcd = index & 7, slot = index >> 3, whole = pairs - dealt, per_xcd = (whole + 7) >> 3;
+        const int deals = (dealt * ranks + 7) >> 3; // slots of an XCD that take tiles of the dealt pairs
+        int rank, pair;
+        if (slot < deals) {
+            const int tile = slot * 8 + xcd;
+            rank = tile / dealt;
+            pair = whole + tile % dealt;
+            return {rank, pair % H, pair / H, rank < ranks};
+        }
+        rank = (slot - deals) / per_xcd;
+        pair = (slot - deals) % per_xcd * 8 + xcd;
+        return {rank, pair % H, pair / H, pair < whole};
+    }
+    unsigned blocks() const {
+        return (unsigned(dealt * ranks + 7) / 8 + unsigned((pairs - dealt + 7) / 8) * unsigned(ranks)) * 8;
+    }
+};
+// Where eight does not divide the pairs, whole pairs give some XCDs a pair more than others, or leave some idle.  Dealing
+// the remainder costs every XCD its own copy of those pairs' keys and values, so it is done only where the fullest XCD
+// has more blocks than compute units.  Whole -> dealt, 128-row blocks, forward; backward in us: 1 pair of 8192 106 -> 98;
+// 298 -> 274, 9 pairs of 8192 144 -> 123; 401 -> 329, 13 pairs of 8192 170 -> 160; 479 -> 444; but 15 pairs of 2048 (32
+// blocks an XCD) 28.7 -> 32.5; 76 -> 79.  32-row blocks: 12 pairs of 1024 8.9 -> 8.6; 26.5 -> 20.3, 4 pairs of 4096
+// 33 -> 20; 114 -> 58.
+CausalGrid causal_grid(int B, int H, int T, int rows) {
+    const int pairs = B * H, ranks = T / rows;
+    return {H, pairs, ranks, (pairs + 7) / 8 * ranks > 32 ? pairs % 8 : 0};
 }
 
 template <int N> struct Const {
@@ -167,6 +194,177 @@ TG_DEVICE void store_acc_rows(bf16_t *row, const f32x16 &acc, float scale, int g
     }
 }
 
+// ---- one wave, one 64-row tile: the arithmetic of the three kernels ------------------------------------------
+// forward, S^T: scores of 64 keys against 32 queries (lane % 32)
+TG_DEVICE void scores(const bf16_t *kt, const RowFragOffsets &krows, const bf16x8 (&qf)[4], f32x16 (&s)[2]) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+            s[mt] = mfma(krows.load(kt, mt, ks), qf[ks], ks == 0 ? zero16() : s[mt]);
+}
+// forward: the scores of keys kv0 .. kv0 + 63 to probabilities under the running maximum m; l is this lane's half of
+// the keys only, the halves are joined at the end.  Returns what earlier sums have to be multiplied by.
+TG_DEVICE float online_softmax(f32x16 (&s)[2], int kv0, int wave_q0, int qrow, int g, float c, float &m, float &l) {
+    if (kv0 + 63 > wave_q0) { // diagonal tile: hide keys after the query
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (kv0 + mt * 32 + acc_row(r, g) > qrow)
+                    s[mt][r] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            mx = fmaxf(mx, s[mt][r]);
+    mx = halves_max(mx);
+    const float m_new = fmaxf(m, mx * c);
+    const float alpha = exp2_fast(m - m_new);
+    float sum = 0.f;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float p = exp2_fast(fmaf(s[mt][r], c, -m_new));
+            s[mt][r] = p;
+            sum += p;
+        }
+    l = l * alpha + sum;
+    m = m_new;
+    return alpha;
+}
+// forward: O^T += V^T P of the same 64 keys
+TG_DEVICE void weigh_values(const bf16_t *vt, const ColFragOffsets &vcols, const f32x16 (&s)[2], f32x16 (&o)[2]) {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        const bf16x8 pf = acc_to_frag(s[kk >> 1], kk & 1);
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+            o[dt] = mfma(vcols.load(vt, kk, dt), pf, o[dt]);
+    }
+}
+// dQ of 32 queries from 64 keys, in 32-key halves to keep the registers down
+TG_DEVICE void dq_tile(const bf16_t *kt, const bf16_t *vt, int kv0, int wave_q0, int qrow, int g, float c, float lse,
+                       const RowFragOffsets &krows, const ColFragOffsets &kcols, const bf16x8 (&qf)[4], const bf16x8 (&gf)[4],
+                       const f32x16 &minus_delta, f32x16 (&dq)[2]) {
+    const bool diagonal = kv0 + 63 > wave_q0;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+        if (kv0 + mt * 32 > wave_q0 + 31) // every key of this half follows this wave's queries
+            continue;
+        // dP - delta in one go: the product accumulates onto a register set that holds -delta of this lane's query
+        f32x16 s = zero16(), dp;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            s = mfma(krows.load(kt, mt, ks), qf[ks], s);
+            dp = mfma(krows.load(vt, mt, ks), gf[ks], ks == 0 ? minus_delta : dp);
+        }
+        // the causal mask only in the tiles that straddle the diagonal (wave-uniform branch)
+        auto probabilities = [&](auto masked) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float p = exp2_fast(fmaf(s[r], c, -lse));
+                if (decltype(masked)::value && kv0 + mt * 32 + acc_row(r, g) > qrow)
+                    p = 0.f;
+                dp[r] = p * dp[r];
+            }
+        };
+        if (diagonal)
+            probabilities(Const<1>{});
+        else
+            probabilities(Const<0>{});
+#pragma unroll
+        for (int kk2 = 0; kk2 < 2; ++kk2) {
+            const bf16x8 dsf = acc_to_frag(dp, kk2);
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+                dq[dt] = mfma(kcols.load(kt, mt * 2 + kk2, dt), dsf, dq[dt]);
+        }
+    }
+}
+// dK, dV of 32 keys from 64 queries (from q0), in 32-query halves; `lse2` and `minus` in LDS: the queries' base-2
+// log-sum-exps and negated deltas
+TG_DEVICE void dkdv_tile(const bf16_t *qt_tile, const bf16_t *gt_tile, const float *lse2, const float *minus, int q0, int wave_k0,
+                         int krow, int g, float c, const RowFragOffsets &qrows, const ColFragOffsets &qcols,
+                         const bf16x8 (&kf)[4], const bf16x8 (&vf)[4], f32x16 (&dk)[2], f32x16 (&dv)[2]) {
+    auto half = [&](auto half_tag) {
+        constexpr int qt = decltype(half_tag)::value;
+        const int qh = q0 + qt * 32;
+        if (qh + 31 < wave_k0) // every query of this half precedes this wave's keys (wave uniform)
+            return;
+        // dP - delta in one go: the product accumulates onto -delta of its rows (the dQ kernel leaves the deltas
+        // negated), one subtraction per score less on the vector ALU that bounds this kernel
+        f32x16 s = zero16(), dp;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const f32x4 minus4 = *reinterpret_cast<const f32x4 *>(minus + qt * 32 + 8 * q4 + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                dp[q4 * 4 + e] = minus4[e];
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            s = mfma(qrows.load(qt_tile, qt, ks), kf[ks], s);
+            dp = mfma(qrows.load(gt_tile, qt, ks), vf[ks], dp);
+        }
+        // the causal mask costs three instructions per score: only in the half tiles that straddle the
+        // diagonal (a wave-uniform branch; as a per-element condition it is paid everywhere)
+        auto probabilities = [&](auto masked) {
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const int at = qt * 32 + 8 * q4 + 4 * g;
+                const f32x4 lse4 = *reinterpret_cast<const f32x4 *>(lse2 + at);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = q4 * 4 + e;
+                    float p = exp2_fast(fmaf(s[r], c, -lse4[e]));
+                    if (decltype(masked)::value && krow > q0 + at + e)
+                        p = 0.f;
+                    s[r] = p;
+                    dp[r] = p * dp[r];
+                }
+            }
+        };
+        if (qh < wave_k0 + 31)
+            probabilities(Const<1>{});
+        else
+            probabilities(Const<0>{});
+#pragma unroll
+        for (int kk2 = 0; kk2 < 2; ++kk2) {
+            const bf16x8 pf = acc_to_frag(s, kk2);
+            const bf16x8 dsf = acc_to_frag(dp, kk2);
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) {
+                dv[dt] = mfma(qcols.load(gt_tile, qt * 2 + kk2, dt), pf, dv[dt]);
+                dk[dt] = mfma(qcols.load(qt_tile, qt * 2 + kk2, dt), dsf, dk[dt]);
+            }
+        }
+    };
+    half(Const<0>{});
+    half(Const<1>{});
+}
+// the row's dot product with the fragments of another
+TG_DEVICE float row_product(const bf16x8 (&f)[4], const bf16_t *row, int g) {
+    float sum = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const bf16x8 of = *reinterpret_cast<const bf16x8 *>(row + g * 8 + ks * 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            sum += float(f[ks][e]) * float(of[e]);
+    }
+    return halves_sum(sum);
+}
+// row fragments of 32 rows: row lane % 32, 8 of every 16 columns
+TG_DEVICE void load_row_fragments(bf16x8 (&f)[4], const bf16_t *row, int g) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+        f[ks] = *reinterpret_cast<const bf16x8 *>(row + g * 8 + ks * 16);
+}
+
 // ---------------------------------------------------------------------------------------------
 // forward: block = 128 queries (4 waves x 32), key/value tiles of 64 in three LDS stages filled by
 // asynchronous copies issued two tiles ahead; heavy (late) query tiles first.  The tile loop is
@@ -177,10 +375,9 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
                                                           const bf16_t *__restrict__ K,
                                                           const bf16_t *__restrict__ V, int ld,
                                                           bf16_t *__restrict__ O, int ldo,
-                                                          float *__restrict__ LSE, int T, int H,
-                                                          int pairs, float c) {
+                                                          float *__restrict__ LSE, int T, CausalGrid grid, float c) {
     __shared__ __align__(1024) bf16_t stages[3][2][TILE_ELEMS]; // [stage][K | V]
-    const CausalBlock block = causal_block(H, pairs);
+    const CausalBlock block = grid.block(blockIdx.x);
     if (!block.live)
         return;
     const int q0 = (T / 128 - 1 - block.rank) * 128, h = block.h, b = block.b;
@@ -207,14 +404,9 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
         produce(1, 1);
 
     bf16x8 qf[4];
-    {
-        const bf16_t *qp = Q + (token0 + qrow) * ld + h * HD + g * 8;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-            qf[ks] = *reinterpret_cast<const bf16x8 *>(qp + ks * 16);
-    }
+    load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
     f32x16 o[2] = {zero16(), zero16()};
-    float m = -INFINITY, l = 0.f; // l: this lane's half of the keys only, halves are joined at the end
+    float m = -INFINITY, l = 0.f;
     const RowFragOffsets krows(lane);
     const ColFragOffsets vcols(lane);
 
@@ -233,56 +425,17 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
                 produce((STAGE + 2) % 3, j + 2);
             return;
         }
-        const bf16_t *kt = stages[STAGE][0], *vt = stages[STAGE][1];
-        const int kv0 = j * 64;
-        f32x16 s[2] = {zero16(), zero16()};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
-                s[mt] = mfma(krows.load(kt, mt, ks), qf[ks], s[mt]);
-        if (kv0 + 63 > wave_q0) { // diagonal tile: hide keys after the query
-#pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (kv0 + mt * 32 + acc_row(r, g) > qrow)
-                        s[mt][r] = -INFINITY;
-        }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                mx = fmaxf(mx, s[mt][r]);
-        mx = halves_max(mx);
-        const float m_new = fmaxf(m, mx * c);
-        const float alpha = exp2_fast(m - m_new);
-        float sum = 0.f;
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = exp2_fast(fmaf(s[mt][r], c, -m_new));
-                s[mt][r] = p;
-                sum += p;
-            }
-        l = l * alpha + sum;
-        if (__builtin_amdgcn_ballot_w64(m_new != m)) { // rescale only when some row's maximum moved
+        f32x16 s[2];
+        scores(stages[STAGE][0], krows, qf, s);
+        const float before = m, alpha = online_softmax(s, j * 64, wave_q0, qrow, g, c, m, l);
+        if (__builtin_amdgcn_ballot_w64(m != before)) { // rescale only when some row's maximum moved
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     o[dt][r] *= alpha;
         }
-        m = m_new;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const bf16x8 pf = acc_to_frag(s[kk >> 1], kk & 1);
-#pragma unroll
-            for (int dt = 0; dt < 2; ++dt)
-                o[dt] = mfma(vcols.load(vt, kk, dt), pf, o[dt]);
-        }
+        weigh_values(stages[STAGE][1], vcols, s, o);
         if (j + 2 < tiles)
             produce((STAGE + 2) % 3, j + 2);
     };
@@ -300,7 +453,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
     for (int dt = 0; dt < 2; ++dt)
         store_acc_rows(op + dt * 32, o[dt], inv, g);
     if (g == 0)
-        LSE[(size_t(b) * H + h) * T + qrow] = (m + __log2f(l)) * LN2;
+        LSE[(size_t(b) * grid.H + h) * T + qrow] = (m + __log2f(l)) * LN2;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -313,11 +466,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
     const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
     const bf16_t *__restrict__ dO, int lddo, const float *__restrict__ lse2,
-    const float *__restrict__ delta, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T,
-    int H, int pairs, float scale) {
+    const float *__restrict__ delta, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
     __shared__ __align__(1024) bf16_t stages[3][2][TILE_ELEMS]; // [stage][Q | dO]
     __shared__ __align__(256) float rows[3][2][64];             // [stage][lse2 | -delta]
-    const CausalBlock block = causal_block(H, pairs);
+    const CausalBlock block = grid.block(blockIdx.x);
     if (!block.live)
         return;
     const int k0 = block.rank * 128, h = block.h, b = block.b; // early keys see the most queries
@@ -328,7 +480,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
     const int first = k0 / 64, tiles = T / 64 - first;
     const bf16_t *qbase = Q + (token0 + first * 64) * ld + h * HD;
     const bf16_t *gbase = dO + (token0 + first * 64) * lddo + h * HD;
-    const float *row_source = ((wave & 1) ? delta : lse2) + (size_t(b) * H + h) * T + first * 64 + lane;
+    const float *row_source = ((wave & 1) ? delta : lse2) + (size_t(b) * grid.H + h) * T + first * 64 + lane;
     const uint32_t lds0 = lds_address(&stages[0][0][0]), rows0 = lds_address(&rows[0][wave & 1][0]);
     const uint32_t q_offset[2] = {tile_copy_offset(ld, wave, lane, 0), tile_copy_offset(ld, wave, lane, 1)};
     const uint32_t g_offset[2] = {tile_copy_offset(lddo, wave, lane, 0), tile_copy_offset(lddo, wave, lane, 1)};
@@ -352,15 +504,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
     produce(1, tiles > 1 ? 1 : 0);
 
     bf16x8 kf[4], vf[4];
-    {
-        const bf16_t *kp = K + (token0 + krow) * ld + h * HD + g * 8;
-        const bf16_t *vp = V + (token0 + krow) * ld + h * HD + g * 8;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            kf[ks] = *reinterpret_cast<const bf16x8 *>(kp + ks * 16);
-            vf[ks] = *reinterpret_cast<const bf16x8 *>(vp + ks * 16);
-        }
-    }
+    load_row_fragments(kf, K + (token0 + krow) * ld + h * HD, g);
+    load_row_fragments(vf, V + (token0 + krow) * ld + h * HD, g);
     f32x16 dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
     const RowFragOffsets qrows(lane);
     const ColFragOffsets qcols(lane);
@@ -374,63 +519,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
         // Every step issues five (past the end the last tile once more, into the stage nobody reads any
         // more), so the wait above is always the same.
         const int ahead = j + 2 < tiles ? j + 2 : tiles - 1;
-        const bf16_t *qt_tile = stages[STAGE][0], *gt_tile = stages[STAGE][1];
-        const int q0 = (first + j) * 64;
-        auto half = [&](auto half_tag) {
-            constexpr int qt = decltype(half_tag)::value;
-            const int qh = q0 + qt * 32;
-            if (qh + 31 < wave_k0) // every query of this half precedes this wave's keys (wave uniform)
-                return;
-            // dP - delta in one go: the product accumulates onto -delta of its rows (the dQ kernel leaves the deltas
-            // negated), one subtraction per score less on the vector ALU that bounds this kernel
-            f32x16 s = zero16(), dp;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const f32x4 minus4 = *reinterpret_cast<const f32x4 *>(&rows[STAGE][1][qt * 32 + 8 * q4 + 4 * g]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    dp[q4 * 4 + e] = minus4[e];
-            }
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                s = mfma(qrows.load(qt_tile, qt, ks), kf[ks], s);
-                dp = mfma(qrows.load(gt_tile, qt, ks), vf[ks], dp);
-            }
-            // the causal mask costs three instructions per score: only in the half tiles that straddle the
-            // diagonal (a wave-uniform branch; as a per-element condition it is paid everywhere)
-            auto probabilities = [&](auto masked) {
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    const int at = qt * 32 + 8 * q4 + 4 * g;
-                    const f32x4 lse4 = *reinterpret_cast<const f32x4 *>(&rows[STAGE][0][at]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int r = q4 * 4 + e;
-                        float p = exp2_fast(fmaf(s[r], c, -lse4[e]));
-                        if (decltype(masked)::value && krow > q0 + at + e)
-                            p = 0.f;
-                        s[r] = p;
-                        dp[r] = p * dp[r];
-                    }
-                }
-            };
-            if (qh < wave_k0 + 31)
-                probabilities(Const<1>{});
-            else
-                probabilities(Const<0>{});
-#pragma unroll
-            for (int kk2 = 0; kk2 < 2; ++kk2) {
-                const bf16x8 pf = acc_to_frag(s, kk2);
-                const bf16x8 dsf = acc_to_frag(dp, kk2);
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt) {
-                    dv[dt] = mfma(qcols.load(gt_tile, qt * 2 + kk2, dt), pf, dv[dt]);
-                    dk[dt] = mfma(qcols.load(qt_tile, qt * 2 + kk2, dt), dsf, dk[dt]);
-                }
-            }
-        };
-        half(Const<0>{});
-        half(Const<1>{});
+        dkdv_tile(stages[STAGE][0], stages[STAGE][1], rows[STAGE][0], rows[STAGE][1], (first + j) * 64, wave_k0, krow, g, c,
+                  qrows, qcols, kf, vf, dk, dv);
         produce((STAGE + 2) % 3, ahead);
     };
     for (int j = 0; j < tiles; j += 3) { // tiles is block uniform
@@ -458,9 +548,9 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
     const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
     const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo,
     const float *__restrict__ LSE, float *__restrict__ lse2_out, float *__restrict__ delta_out,
-    bf16_t *__restrict__ dQ, int lddq, int T, int H, int pairs, float scale) {
+    bf16_t *__restrict__ dQ, int lddq, int T, CausalGrid grid, float scale) {
     __shared__ __align__(1024) bf16_t stages[3][2][TILE_ELEMS]; // [stage][K | V]
-    const CausalBlock block = causal_block(H, pairs);
+    const CausalBlock block = grid.block(blockIdx.x);
     if (!block.live)
         return;
     const int q0 = (T / 128 - 1 - block.rank) * 128, h = block.h, b = block.b;
@@ -488,30 +578,12 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
         produce(1, 1);
 
     bf16x8 qf[4], gf[4];
-    {
-        const bf16_t *qp = Q + (token0 + qrow) * ld + h * HD + g * 8;
-        const bf16_t *gp = dO + (token0 + qrow) * lddo + h * HD + g * 8;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            qf[ks] = *reinterpret_cast<const bf16x8 *>(qp + ks * 16);
-            gf[ks] = *reinterpret_cast<const bf16x8 *>(gp + ks * 16);
-        }
-    }
+    load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
+    load_row_fragments(gf, dO + (token0 + qrow) * lddo + h * HD, g);
     // delta = rowsum(dO o O) and the log-sum-exp in base 2, for this block's own queries; also left in
     // memory for the dK/dV kernel, which runs after this one
-    float del = 0.f;
-    {
-        const bf16_t *op = O + (token0 + qrow) * ldo + h * HD + g * 8;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const bf16x8 of = *reinterpret_cast<const bf16x8 *>(op + ks * 16);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                del += float(gf[ks][e]) * float(of[e]);
-        }
-        del = halves_sum(del);
-    }
-    const size_t row_at = (size_t(b) * H + h) * T + qrow;
+    const float del = row_product(gf, O + (token0 + qrow) * ldo + h * HD, g);
+    const size_t row_at = (size_t(b) * grid.H + h) * T + qrow;
     const float lse = LSE[row_at] * LOG2E;
     if (g == 0) {
         delta_out[row_at] = -del; // negated: the dK/dV kernel starts its dP product from it
@@ -539,42 +611,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
                 produce((STAGE + 2) % 3, j + 2);
             return;
         }
-        const bf16_t *kt = stages[STAGE][0], *vt = stages[STAGE][1];
-        const int kv0 = j * 64;
-        const bool diagonal = kv0 + 63 > wave_q0;
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            if (kv0 + mt * 32 > wave_q0 + 31) // every key of this half follows this wave's queries
-                continue;
-            // dP - delta in one go: the product accumulates onto a register set that holds -delta of this lane's query
-            f32x16 s = zero16(), dp;
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                s = mfma(krows.load(kt, mt, ks), qf[ks], s);
-                dp = mfma(krows.load(vt, mt, ks), gf[ks], ks == 0 ? minus_delta : dp);
-            }
-            // the causal mask only in the tiles that straddle the diagonal (wave-uniform branch)
-            auto probabilities = [&](auto masked) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    float p = exp2_fast(fmaf(s[r], c, -lse));
-                    if (decltype(masked)::value && kv0 + mt * 32 + acc_row(r, g) > qrow)
-                        p = 0.f;
-                    dp[r] = p * dp[r];
-                }
-            };
-            if (diagonal)
-                probabilities(Const<1>{});
-            else
-                probabilities(Const<0>{});
-#pragma unroll
-            for (int kk2 = 0; kk2 < 2; ++kk2) {
-                const bf16x8 dsf = acc_to_frag(dp, kk2);
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt)
-                    dq[dt] = mfma(kcols.load(kt, mt * 2 + kk2, dt), dsf, dq[dt]);
-            }
-        }
+        dq_tile(stages[STAGE][0], stages[STAGE][1], j * 64, wave_q0, qrow, g, c, lse, krows, kcols, qf, gf, minus_delta, dq);
         if (j + 2 < tiles)
             produce((STAGE + 2) % 3, j + 2);
     };
@@ -591,6 +628,259 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
         store_acc_rows(qp + dt * 32, dq[dt], scale, g);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Few rows.  A wave of the kernels above walks its row's tiles one after another, T/64 of them at worst, at about
+// 0.8 us each, whatever the number of blocks: with one block of 128 rows per compute unit or less that chain is the
+// kernel's time and most SIMDs are idle or wait.  Here a block is 32 queries (or keys) and its four waves take the
+// tiles of the other side in turn, each into a stage of its own (no barrier in the loop) and with sums of its own,
+// which meet in LDS at the end: a chain a quarter as long on four times the blocks.  The price is that a tile is
+// fetched once per 32 rows instead of once per 128 and that the stages are not double buffered (two blocks of 64 KiB
+// per compute unit fill in for each other); the backward is one launch, because its dK/dV blocks form the deltas of
+// their queries themselves.  Microseconds, 128-row blocks -> these (B, H, T), forward; backward:
+//   1,1,128: 4.6 -> 4.0; 11.6 -> 5.4    8,4,256: 6.5 -> 5.0; 16.7 -> 9.0     5,10,384: 8.3 -> 8.3; 21.8 -> 19.6
+//   1,12,1024: 16.1 -> 8.6; 42.1 -> 20.3    1,4,4096: 53 -> 20; 144 -> 58    1,1,8192: 99 -> 31; 273 -> 79
+// ---------------------------------------------------------------------------------------------
+constexpr int WAVES = 4;
+// this wave's own 64 x 64 tile, rows ld elements apart, in eight copies
+struct WaveTileCopy {
+    uint32_t offset[2];
+    int ld;
+    TG_DEVICE WaveTileCopy(int ld_, int lane) : offset{tile_copy_offset(ld_, 0, lane, 0), tile_copy_offset(ld_, 1, lane, 0)}, ld(ld_) {}
+    TG_DEVICE void operator()(uint32_t lds_tile, const bf16_t *base) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd)
+                async_copy16(__builtin_amdgcn_readfirstlane(lds_tile + (2 * i + odd) * 1024), base + size_t(i) * 16 * ld, offset[odd]);
+    }
+};
+// a wave's 32 x 64 sums to its part of LDS, 16 bytes a lane and store
+TG_DEVICE void leave_sums(float *part, const f32x16 (&acc)[2], int lane) {
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+        *reinterpret_cast<f32x4 *>(part + (n * 64 + lane) * 4) =
+            f32x4{acc[n >> 2][(n & 3) * 4], acc[n >> 2][(n & 3) * 4 + 1], acc[n >> 2][(n & 3) * 4 + 2], acc[n >> 2][(n & 3) * 4 + 3]};
+}
+// columns 16 * wave .. +15 of the block's 32 rows: eight sums a lane, of the `parts` waves that had a tile
+TG_DEVICE void join_sums(float (&sum)[8], const float *part0, size_t stride, int parts, const float *weight, int wave, int lane) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        sum[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+        if (w < parts) {
+            const float *from = part0 + w * stride + (wave * 2 * 64 + lane) * 4;
+            const f32x4 lo = *reinterpret_cast<const f32x4 *>(from), hi = *reinterpret_cast<const f32x4 *>(from + 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sum[e] = fmaf(lo[e], weight[w], sum[e]);
+                sum[e + 4] = fmaf(hi[e], weight[w], sum[e + 4]);
+            }
+        }
+}
+TG_DEVICE void store_joined(bf16_t *row, const float (&sum)[8], float scale, int wave, int g) {
+    const auto x = __builtin_amdgcn_permlane32_swap(pack_bf16(sum[0] * scale, sum[1] * scale),
+                                                    pack_bf16(sum[4] * scale, sum[5] * scale), false, false);
+    const auto y = __builtin_amdgcn_permlane32_swap(pack_bf16(sum[2] * scale, sum[3] * scale),
+                                                    pack_bf16(sum[6] * scale, sum[7] * scale), false, false);
+    *reinterpret_cast<u32x4 *>(row + wave * 16 + 8 * g) = u32x4{x[0], y[0], x[1], y[1]};
+}
+
+__global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
+                                                                const bf16_t *__restrict__ V, int ld, bf16_t *__restrict__ O,
+                                                                int ldo, float *__restrict__ LSE, int T, CausalGrid grid, float c) {
+    __shared__ __align__(1024) bf16_t tile[WAVES][2][TILE_ELEMS]; // [wave][K | V], then the waves' sums
+    __shared__ float2 row_sums[WAVES][32];                        // maximum and sum of a row
+    const CausalBlock block = grid.block(blockIdx.x);
+    if (!block.live)
+        return;
+    const int q0 = (T / 32 - 1 - block.rank) * 32, h = block.h, b = block.b;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 5, qrow = q0 + (lane & 31);
+    const size_t token0 = size_t(b) * T;
+    const int tiles = q0 / 64 + 1;
+    const bf16_t *kbase = K + token0 * ld + h * HD, *vbase = V + token0 * ld + h * HD;
+    const uint32_t slot = lds_address(&tile[wave][0][0]);
+    const WaveTileCopy copy(ld, lane);
+    bf16x8 qf[4];
+    f32x16 o[2] = {zero16(), zero16()};
+    float m = -INFINITY, l = 0.f;
+    if (wave < tiles) {
+        copy(slot, kbase + size_t(wave) * 64 * ld);
+        copy(slot + TILE_ELEMS * 2, vbase + size_t(wave) * 64 * ld);
+        load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
+        const RowFragOffsets krows(lane);
+        const ColFragOffsets vcols(lane);
+        for (int j = wave; j < tiles; j += WAVES) {
+            const bool more = j + WAVES < tiles;
+            f32x16 s[2];
+            wait_vmcnt<8>(); // this tile's keys are there, its values may still be on the way
+            scores(tile[wave][0], krows, qf, s);
+            if (more) {
+                wait_lgkmcnt0(); // the keys have been read
+                copy(slot, kbase + size_t(j + WAVES) * 64 * ld);
+            }
+            const float before = m, alpha = online_softmax(s, j * 64, q0, qrow, g, c, m, l);
+            if (__builtin_amdgcn_ballot_w64(m != before)) {
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        o[dt][r] *= alpha;
+            }
+            if (more)
+                wait_vmcnt<8>();
+            else
+                wait_vmcnt<0>();
+            weigh_values(tile[wave][1], vcols, s, o);
+            if (more) {
+                wait_lgkmcnt0();
+                copy(slot + TILE_ELEMS * 2, vbase + size_t(j + WAVES) * 64 * ld);
+            }
+        }
+        wait_lgkmcnt0(); // the tile has been read
+        l = halves_sum(l);
+        leave_sums(reinterpret_cast<float *>(tile[wave]), o, lane);
+        if (g == 0)
+            row_sums[wave][lane] = make_float2(m, l);
+    }
+    __syncthreads();
+    const int parts = tiles < WAVES ? tiles : WAVES;
+    float weight[WAVES], top = -INFINITY, total = 0.f, sum[8];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+        if (w < parts)
+            top = fmaxf(top, row_sums[w][lane & 31].x);
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        weight[w] = 0.f;
+        if (w < parts) {
+            const float2 row = row_sums[w][lane & 31];
+            weight[w] = exp2_fast(row.x - top);
+            total = fmaf(row.y, weight[w], total);
+        }
+    }
+    join_sums(sum, reinterpret_cast<const float *>(tile[0]), sizeof(tile[0]) / sizeof(float), parts, weight, wave, lane);
+    store_joined(O + (token0 + qrow) * ldo + h * HD, sum, 1.0f / total, wave, g);
+    if (threadIdx.x < 32)
+        LSE[(size_t(b) * grid.H + h) * T + qrow] = (top + __log2f(total)) * LN2;
+}
+
+// dK, dV and dQ in one launch: every other run of eight blocks takes 32 keys, the others 32 queries
+__global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
+    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
+    const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo, const float *__restrict__ LSE,
+    bf16_t *__restrict__ dQ, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
+    __shared__ __align__(1024) bf16_t tile[WAVES][2][TILE_ELEMS]; // [wave][Q | dO] or [K | V], then the waves' sums
+    __shared__ __align__(256) float rows[WAVES][2][64];           // [wave][lse2 | -delta]
+    const CausalBlock block = grid.block((blockIdx.x >> 4) * 8 + (blockIdx.x & 7));
+    if (!block.live)
+        return;
+    const bool keys = !(blockIdx.x & 8);
+    const int h = block.h, b = block.b;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 5;
+    const size_t token0 = size_t(b) * T;
+    const float c = scale * LOG2E;
+    const float *lse_row = LSE + (size_t(b) * grid.H + h) * T;
+    const uint32_t slot = lds_address(&tile[wave][0][0]);
+    float *part = reinterpret_cast<float *>(tile[wave]);
+    const float *part0 = reinterpret_cast<const float *>(tile[0]);
+    constexpr size_t STRIDE = sizeof(tile[0]) / sizeof(float);
+    const float ones[WAVES] = {1.f, 1.f, 1.f, 1.f};
+    float sum[8];
+    const RowFragOffsets along(lane);
+    const ColFragOffsets across(lane);
+    if (keys) {
+        const int k0 = block.rank * 32, krow = k0 + (lane & 31), first = k0 / 64, tiles = T / 64 - first;
+        if (wave < tiles) {
+            const WaveTileCopy copy_q(ld, lane), copy_g(lddo, lane);
+            bf16x8 kf[4], vf[4];
+            f32x16 dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
+            for (int j = wave; j < tiles; j += WAVES) {
+                const int q0 = (first + j) * 64;
+                copy_q(slot, Q + (token0 + q0) * ld + h * HD);
+                copy_g(slot + TILE_ELEMS * 2, dO + (token0 + q0) * lddo + h * HD);
+                if (j == wave) {
+                    load_row_fragments(kf, K + (token0 + krow) * ld + h * HD, g);
+                    load_row_fragments(vf, V + (token0 + krow) * ld + h * HD, g);
+                }
+                bf16x8 of[2][4];
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt)
+                    load_row_fragments(of[mt], O + (token0 + q0 + mt * 32 + (lane & 31)) * ldo + h * HD, g);
+                rows[wave][0][lane] = lse_row[q0 + lane] * LOG2E;
+                wait_vmcnt<0>();
+                // deltas of the tile's queries: the diagonal of dO O^T, on the matrix cores
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) {
+                    f32x16 products = zero16();
+#pragma unroll
+                    for (int ks = 0; ks < 4; ++ks)
+                        products = mfma(along.load(tile[wave][1], mt, ks), of[mt][ks], products);
+                    float diagonal = 0.f;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        diagonal = acc_row(r, g) == (lane & 31) ? products[r] : diagonal;
+                    if (((lane >> 2) & 1) == g)
+                        rows[wave][1][mt * 32 + (lane & 31)] = -diagonal;
+                }
+                dkdv_tile(tile[wave][0], tile[wave][1], rows[wave][0], rows[wave][1], q0, k0, krow, g, c, along, across, kf, vf,
+                          dk, dv);
+                wait_lgkmcnt0(); // the tile has been read
+            }
+            leave_sums(part, dk, lane);
+            leave_sums(part + TILE_ELEMS / 2, dv, lane);
+        }
+        __syncthreads();
+        const int parts = tiles < WAVES ? tiles : WAVES;
+        join_sums(sum, part0, STRIDE, parts, ones, wave, lane);
+        store_joined(dK + (token0 + krow) * lddq + h * HD, sum, scale, wave, g);
+        join_sums(sum, part0 + TILE_ELEMS / 2, STRIDE, parts, ones, wave, lane);
+        store_joined(dV + (token0 + krow) * lddq + h * HD, sum, 1.0f, wave, g);
+    } else {
+        const int q0 = (T / 32 - 1 - block.rank) * 32, qrow = q0 + (lane & 31), tiles = q0 / 64 + 1;
+        if (wave < tiles) {
+            const WaveTileCopy copy(ld, lane);
+            const bf16_t *kbase = K + token0 * ld + h * HD, *vbase = V + token0 * ld + h * HD;
+            copy(slot, kbase + size_t(wave) * 64 * ld);
+            copy(slot + TILE_ELEMS * 2, vbase + size_t(wave) * 64 * ld);
+            bf16x8 qf[4], gf[4];
+            load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
+            load_row_fragments(gf, dO + (token0 + qrow) * lddo + h * HD, g);
+            const float del = row_product(gf, O + (token0 + qrow) * ldo + h * HD, g), lse = lse_row[qrow] * LOG2E;
+            f32x16 dq[2] = {zero16(), zero16()};
+            f32x16 minus_delta;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                minus_delta[r] = -del;
+            for (int j = wave; j < tiles; j += WAVES) {
+                wait_vmcnt<0>();
+                dq_tile(tile[wave][0], tile[wave][1], j * 64, q0, qrow, g, c, lse, along, across, qf, gf, minus_delta, dq);
+                wait_lgkmcnt0();
+                if (j + WAVES < tiles) {
+                    copy(slot, kbase + size_t(j + WAVES) * 64 * ld);
+                    copy(slot + TILE_ELEMS * 2, vbase + size_t(j + WAVES) * 64 * ld);
+                }
+            }
+            leave_sums(part, dq, lane);
+        }
+        __syncthreads();
+        join_sums(sum, part0, STRIDE, tiles < WAVES ? tiles : WAVES, ones, wave, lane);
+        store_joined(dQ + (token0 + qrow) * lddq + h * HD, sum, scale, wave, g);
+    }
+}
+
+// Up to how many 128-row blocks the 32-row ones with shared-out tiles are taken instead.  The longer the context, the
+// longer the chains that they cut, so the line rises with it.  Microseconds, 128-row -> 32-row:
+//   T 128: 128 blocks 5.1 -> 5.0; 12.9 -> 11.0   192: 5.3 -> 7.2; 13.8 -> 15.7
+//   T 256: 128 blocks 6.7 -> 5.7; 17.3 -> 14.2   192: 6.9 -> 8.3; 17.9 -> 19.0
+//   T 512: 192 blocks 10.0 -> 10.0; 25.8 -> 25.6   224: 10.1 -> 10.7; 26.5 -> 28.4
+//   T 1024: 256 blocks 16.7 -> 14.3; 43.3 -> 43.9   320: 17.2 -> 17.5; 46.3 -> 54.5
+//   T 2048: 272 blocks 29.3 -> 20.9; 78 -> 71   384: 29.1 -> 27.2; 81 -> 99    T 4096: 384 blocks 57 -> 43; 150 -> 166
+// The backward does five products where the forward does two and loses by the fetches sooner.
+bool split_tiles(int B, int H, int T, int most_blocks) {
+    return size_t(B) * H * (T / 128) <= size_t(T / 8 + 128 < most_blocks ? T / 8 + 128 : most_blocks);
+}
+constexpr int SPLIT_FORWARD = 384, SPLIT_BACKWARD = 256;
 void check_attention_shape(int B, int H, int T, int hd) {
     require(B > 0 && H > 0 && T > 0, "attention: empty shape");
     require(hd == HD, "attention: head_dim must be 64");
@@ -615,8 +905,10 @@ extern "C" int tgk_attn_fwd(hipStream_t stream, int B, int H, int T, int hd, con
         check_matrix(V, ld, "V");
         check_matrix(O, ldo, "O");
         require(lse && !(reinterpret_cast<uintptr_t>(lse) & 15), "attention: lse must be 16-byte aligned");
-        hipLaunchKernelGGL(attn_fwd_kernel, dim3(causal_grid(T / 128, B * H)), dim3(256), 0, stream, Q, K, V,
-                           ld, O, ldo, lse, T, H, B * H, scale * LOG2E);
+        const bool split = split_tiles(B, H, T, SPLIT_FORWARD);
+        const CausalGrid grid = causal_grid(B, H, T, split ? 32 : 128);
+        hipLaunchKernelGGL(split ? attn_fwd_split_kernel : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
+                           ld, O, ldo, lse, T, grid, scale * LOG2E);
         check_hip(hipGetLastError(), "attention forward launch: ");
     });
 }
@@ -644,12 +936,19 @@ void attn_bwd_check(int B, int H, int T, int hd, const uint16_t *Q, const uint16
 void attn_bwd_launch(hipStream_t stream, int B, int H, int T, const uint16_t *Q, const uint16_t *K,
                      const uint16_t *V, int ld, const uint16_t *O, int ldo, const float *lse, const uint16_t *dO,
                      int lddo, uint16_t *dQ, uint16_t *dK, uint16_t *dV, int lddq, float scale, float *rows) {
+    if (split_tiles(B, H, T, SPLIT_BACKWARD)) {
+        const CausalGrid grid = causal_grid(B, H, T, 32);
+        hipLaunchKernelGGL(attn_bwd_split_kernel, dim3(2 * grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo,
+                           lse, dQ, dK, dV, lddq, T, grid, scale);
+        check_hip(hipGetLastError(), "attention backward launch: ");
+        return;
+    }
     float *delta = rows, *lse2 = delta + size_t(B) * H * T;
-    const dim3 grid(causal_grid(T / 128, B * H));
-    hipLaunchKernelGGL(attn_bwd_dq_kernel, grid, dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo, lse, lse2,
-                       delta, dQ, lddq, T, H, B * H, scale);
-    hipLaunchKernelGGL(attn_bwd_dkdv_kernel, grid, dim3(256), 0, stream, Q, K, V, ld, dO, lddo, lse2, delta, dK, dV,
-                       lddq, T, H, B * H, scale);
+    const CausalGrid grid = causal_grid(B, H, T, 128);
+    hipLaunchKernelGGL(attn_bwd_dq_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo, lse, lse2,
+                       delta, dQ, lddq, T, grid, scale);
+    hipLaunchKernelGGL(attn_bwd_dkdv_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, lse2, delta, dK,
+                       dV, lddq, T, grid, scale);
     check_hip(hipGetLastError(), "attention backward launch: ");
 }
 } // namespace

@@ -108,6 +108,10 @@ TG_DEVICE void async_copy4(uint32_t lds_base, const void *global) {
 template <int N> TG_DEVICE void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// every LDS read and write of this wave has completed
+TG_DEVICE void wait_lgkmcnt0() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
 TG_DEVICE uint32_t lds_address(const void *shared_pointer) {
     return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void *)shared_pointer));
 }
