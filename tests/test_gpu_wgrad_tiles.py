@@ -1,6 +1,7 @@
-"""Weight gradients on 64 x 64 tiles (wgrad_tiles_kernel through tgk_gemm_wgrad, csrc/gemm.hip): fewer 64-token stages than
-the ring holds, odd counts, tile counts that 8 does not divide and more than the compute units, operands and gradient
-that are column slices, accumulation.  fp32 sums of at most 1920 exact bf16 products: 1e-5 in relative L2."""
+"""Weight gradients on 64 x 64 and 128 x 128 tiles (wgrad_tiles_kernel through tgk_gemm_wgrad, csrc/gemm.hip): fewer 64-token
+stages than the ring holds, odd counts, tile counts that 8 does not divide and more than the compute units, token ranges
+that are folded, operands and gradient that are column slices, accumulation.  fp32 sums of at most 16384 exact bf16
+products (2^-24 a partial sum): 1e-5 in relative L2."""
 import pytest
 import torch
 
@@ -13,7 +14,13 @@ pytestmark = pytest.mark.gpu
                                        (128, 128, 192, 8),   # two stages, 6 tiles
                                        (192, 384, 320 + 64, 64),  # three stages, 36 tiles
                                        (320, 640, 640, 0),   # five stages, 100 tiles
-                                       (1920, 640, 1920, 8)])  # 300 tiles: two on some units
+                                       (1920, 640, 1920, 8),  # 300 tiles: two on some units
+                                       (2048, 256, 256, 8),  # token ranges on 64 x 64 tiles, folded
+                                       (4160, 512, 384, 0),  # ranges of different lengths
+                                       (16384, 128, 128, 8),  # many ranges of few tiles
+                                       (8192, 896, 896, 8),  # 128 x 128 tiles, four stages
+                                       (16384, 768, 768, 0),  # the same with two blocks a unit
+                                       (16384, 768, 3072, 0)])  # the persistent kernel
 def test_single_gradient(M, N, K, pad):
     lib = library()
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)

@@ -1586,14 +1586,16 @@ __global__ __launch_bounds__(256, 1) void wgrad_list_kernel(const WgradList w) {
 }
 // Sums the pieces of the split tiles, in token order, into the gradient.  Eight blocks per tile.
 // The same list on ordinary tiles, each summed over all tokens by one block: where 256 x 256 tiles would not fill the
-// compute units or do not fit the widths, and for a single gradient.  Block b of g takes tiles b, b + g, ...; nothing is
-// cut along the tokens, so nothing is folded.  What bounds it is a stage's latency on a unit with one tile and the
-// transposing LDS reads on one with several (0.24 and 0.20 us for 64 x 64 outputs, 0.66 and 0.55 for 128 x 128).
+// compute units or do not fit the widths, and for a single gradient (plan_wgrad).  Block b of g takes tiles b, b + g, ...; a
+// list is not cut along the tokens, so nothing is folded.  What bounds it is a stage's latency on a unit with one tile and the
+// transposing LDS reads on one with several (wgrad_stage_us).
 struct WgradTiles {
     const WgradListJob *jobs; // device memory; NULL: `one`, its tiles row-major, tiles_n a row
     const int4 *tiles;
     WgradListJob one;
     int tiles_n, count, k_chunks, accumulate;
+    int splits = 1;       // `one` only: token ranges a tile is cut into (1 with a list); `count` is tiles x splits
+    size_t split_stride;  // then `one.dw` is the first of `splits` slabs this far apart, for splitk_reduce_kernel
     float *sumsq; // optional: one sum of squares a block
 };
 template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_tiles_kernel(const WgradTiles w) {
@@ -1605,13 +1607,18 @@ template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_ti
     float squares = 0.f;
     for (int base = 0; base + int(blockIdx.x) < w.count; base += gridDim.x) {
         const int at = base + xcd_contiguous(blockIdx.x, min(int(gridDim.x), w.count - base));
-        const int4 t = w.jobs ? w.tiles[at] : make_int4(0, at / w.tiles_n * BM, at % w.tiles_n * BN, 0);
+        // token range by token range, so that an XCD's tiles share their operands' lines
+        const int tiles = w.count / w.splits, split = at / tiles, tile = at - split * tiles;
+        const int first = int(int64_t(split) * w.k_chunks / w.splits);
+        const int chunks = int(int64_t(split + 1) * w.k_chunks / w.splits) - first;
+        const int4 t = w.jobs ? w.tiles[tile] : make_int4(0, tile / w.tiles_n * BM, tile % w.tiles_n * BN, 0);
         const WgradListJob job = w.jobs ? w.jobs[t.x] : w.one;
         f32x4 acc[P::FM][P::FN][2][2];
-        P::run(job.dy, job.lddy, job.x, job.ldx, t.y, t.z, w.k_chunks, smem, acc);
-        const EpilogueF32 epilogue{job.dw, job.lddw, 0, w.accumulate};
+        P::run(job.dy + int64_t(first) * 64 * job.lddy, job.lddy, job.x + int64_t(first) * 64 * job.ldx, job.ldx, t.y, t.z,
+               chunks, smem, acc);
+        const EpilogueF32 epilogue{job.dw, job.lddw, w.split_stride, w.accumulate};
         staged_store_f32<P::FM, P::FN>(acc, smem + wave * 4096, epilogue, t.y + (wave >> 1) * P::WM, t.z + (wave & 1) * P::WN,
-                                       lane, 0);
+                                       lane, split);
         if (w.sumsq)
 #pragma unroll
             for (int i = 0; i < P::FM; ++i)
@@ -1673,17 +1680,26 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     for (size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x; i < total;
          i += size_t(gridDim.x) * blockDim.x) {
         const int r = int(i / cols4), c = int(i % cols4) * 4;
-        float4 sum = make_float4(0, 0, 0, 0);
-        for (int s = 0; s < splits; ++s) {
-            const float4 v = *reinterpret_cast<const float4 *>(slabs + s * slab_stride + size_t(r) * cols + c);
-            sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        const float *at = slabs + size_t(r) * cols + c;
+        int s = 0;
+        for (; s + 4 <= splits; s += 4) { // four loads in flight: a small gradient has few blocks and many slabs
+            f32x4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                v[k] = *reinterpret_cast<const f32x4 *>(at + (s + k) * slab_stride);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                sum += v[k];
         }
+        for (; s < splits; ++s)
+            sum += *reinterpret_cast<const f32x4 *>(at + s * slab_stride);
         float4 *p = reinterpret_cast<float4 *>(out + size_t(r) * ld_out + c);
         if (accumulate) {
             const float4 old = *p;
-            sum.x += old.x, sum.y += old.y, sum.z += old.z, sum.w += old.w;
+            sum += f32x4{old.x, old.y, old.z, old.w};
         }
-        __builtin_nontemporal_store(f32x4{sum.x, sum.y, sum.z, sum.w}, reinterpret_cast<f32x4 *>(p));
+        __builtin_nontemporal_store(sum, reinterpret_cast<f32x4 *>(p));
     }
 }
 
@@ -1971,6 +1987,17 @@ template <int BM, int BN, int S> void launch_wgrad_tiles(hipStream_t stream, con
     check_hip(hipGetLastError(), "wgrad tiles launch: ");
 }
 
+// 128 x 128: alone on its unit a block has room for four stages (8192, 896 x 3584: 0.57 us a stage; 0.66 with two), with
+// another beside it for two.
+void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int edge, int blocks) {
+    if (edge == 64)
+        launch_wgrad_tiles<64, 64, 3>(stream, w, blocks);
+    else if (blocks <= compute_units())
+        launch_wgrad_tiles<128, 128, 4>(stream, w, blocks);
+    else
+        launch_wgrad_tiles<128, 128, 2>(stream, w, blocks);
+}
+
 void check_operand(const void *p, int ld, const char *name) {
     if (!p || (reinterpret_cast<uintptr_t>(p) & 15) || ld % 8)
         throw std::invalid_argument(std::string("gemm operand ") + name +
@@ -1986,21 +2013,46 @@ int wgrad_splits(Tile tile, int tiles, int k_tiles) {
     return splits < max_by_k ? splits : max_by_k;
 }
 
-// One weight gradient on 64 x 64 tiles, every one over all tokens, or split along the tokens into slabs that a second launch
-// folds?  Estimates in us: a stage of 64 tokens on the fullest unit, against two launches, the slabs written and read at
-// 6 TB/s and the products at 0.95 PFLOP/s.  Either side (tokens, N x K; tiles against slabs, measured): 1920, 640 x 1920 15.4 /
-// 22.8; 1024, 2304 x 768 9.4 / 23.9; 4096, 768 x 768 20.5 / 24.6; 4096, 3072 x 768 36.0 / 36.0; 8192, 512 x 512 36.4 / 25.6;
-// 16384, 768 x 768 70.8 / 34.7.
-bool wgrad_on_tiles(int M, int N, int K) {
-    if (M % 64)
-        return false;
+// Time of 64 tokens on a unit that has `deepest` tiles of wgrad_tiles_kernel (us, measured over the shapes named below).
+double wgrad_stage_us(int edge, int deepest) {
+    if (edge == 64)
+        return deepest == 1 ? 0.25 : deepest == 2 ? 0.37 : 0.19 * deepest;
+    return deepest == 1 ? 0.56 : deepest / 2 * 0.76 + deepest % 2 * 0.66;
+}
+// How one weight gradient is cut: tiles of `edge` and token ranges (slabs that a second launch folds), or edge 0: the
+// persistent kernel's tiles.  By estimates in us: launches 3.5 and 2.2, stages as above, slabs written and read at 5.5 TB/s;
+// the persistent kernel at 1.07 PFLOP/s (128 x 192; 0.95 on 128 x 128) when all its blocks have work.  No more slabs than
+// the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: this, 64 x 64 tiles uncut,
+// persistent): 1920, 640 x 640 10.8, 10.8, -; 2048, 256 x 256 7.9, 11.0, 10.3; 4096, 512 x 512 11.5, 19.4, -; 8192, 384 x 384
+// 13.0, 35.8, 25.8; 8192, 896 x 896 25.5, 36.5, 39.8; 16384, 128 x 128 12.4, 69.2, 24.7; 16384, 640 x 640 28.6, 69.8, 42.2;
+// 16384, 2304 x 768 63.4, 98.5, 65.3; 16384, 768 x 3072 - , 210, 82.6.
+struct WgradCut {
+    int edge, splits;
+};
+WgradCut plan_wgrad(int M, int N, int K) {
     const Tile tile = choose_tile(N, K);
-    const int splits = wgrad_splits(tile, (N / tile_rows(tile)) * (K / tile_cols(tile)), M / BK);
+    const int persistent_tiles = (N / tile_rows(tile)) * (K / tile_cols(tile));
+    const int most = wgrad_splits(tile, persistent_tiles, M / BK), units = compute_units();
+    if (M % 64)
+        return {0, most};
     const double elements = double(N) * K;
-    const int units = compute_units(), deepest = int((elements / 4096 + units - 1) / units);
-    const double tiles_us = 3.5 + M / 64 * (deepest == 1 ? 0.24 : 0.20 * deepest);
-    const double slabs_us = (splits > 1 ? 6 + 8e-6 * splits * elements / 6 : 3.5) + 2e-9 * M * elements / 0.95;
-    return tiles_us < slabs_us;
+    const auto slabs = [&](int splits) { return splits > 1 ? 2.2 + 8e-6 * splits * elements / 5.5 : 0.0; };
+    const int blocks = resident_blocks(tile), items = persistent_tiles * most, rounds = (items + blocks - 1) / blocks;
+    const double rate = tile == TILE_128x192 ? 1.07e9 : 0.95e9;
+    WgradCut best{0, most};
+    double least = 3.5 + slabs(most) + 2 * M * elements / rate * (double(rounds) * blocks / items);
+    for (int edge = 64; edge <= 128; edge *= 2) {
+        if (N % edge || K % edge)
+            continue;
+        const int tiles = (N / edge) * (K / edge);
+        for (int splits = 1; splits <= most && (splits == 1 || splits <= M / 128) && (splits == 1 || (splits - 1) * tiles < 2 * units); ++splits) {
+            const int deepest = (tiles * splits + units - 1) / units, stages = (M / 64 + splits - 1) / splits;
+            const double us = 3.5 + slabs(splits) + stages * wgrad_stage_us(edge, deepest);
+            if (us < least)
+                best = {edge, splits}, least = us;
+        }
+    }
+    return best;
 }
 
 } // namespace
@@ -2138,33 +2190,29 @@ extern "C" int tgk_gemm_wgrad(hipStream_t stream, int M, int N, int K, const uin
         check_operand(X, ldx, "X");
         require(dW && !(reinterpret_cast<uintptr_t>(dW) & 15) && lddw % 4 == 0,
                 "gemm_wgrad: dW must be 16-byte aligned with leading dimension % 4 == 0");
-        if (wgrad_on_tiles(M, N, K)) {
-            WgradTiles w{};
-            w.one = {dY, X, dW, lddy, ldx, lddw, 0};
-            w.tiles_n = K / 64, w.count = (N / 64) * (K / 64), w.k_chunks = M / 64, w.accumulate = accumulate;
-            return launch_wgrad_tiles<64, 64, 3>(stream, w, w.count);
-        }
-        const int splits = wgrad_splits(tile, (N / tile_rows(tile)) * (K / tile_cols(tile)), M / BK);
-        if (splits == 1) {
-            EpilogueF32 e{dW, lddw, 0, accumulate};
-            if (takes_64(tile, M))
-                launch_gemm64<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, 1, e);
-            else
-                dispatch_gemm<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, 1, e);
-            return;
-        }
-        const size_t need = size_t(splits) * N * K * sizeof(float);
-        require(workspace && workspace_bytes >= need && !(reinterpret_cast<uintptr_t>(workspace) & 15),
+        const WgradCut cut = plan_wgrad(M, N, K);
+        const size_t need = cut.splits > 1 ? size_t(cut.splits) * N * K * sizeof(float) : 0;
+        require(!need || (workspace && workspace_bytes >= need && !(reinterpret_cast<uintptr_t>(workspace) & 15)),
                 "gemm_wgrad: workspace too small (see tgk_gemm_wgrad_workspace)");
-        EpilogueF32 e{static_cast<float *>(workspace), K, size_t(N) * K, 0};
-        if (takes_64(tile, M))
-            launch_gemm64<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, splits, e);
-        else
-            dispatch_gemm<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, splits, e);
+        const EpilogueF32 e = need ? EpilogueF32{static_cast<float *>(workspace), K, size_t(N) * K, 0}
+                                   : EpilogueF32{dW, lddw, 0, accumulate};
+        if (cut.edge) {
+            WgradTiles w{};
+            w.one = {dY, X, e.out, lddy, ldx, e.ld_out, 0};
+            w.tiles_n = K / cut.edge, w.splits = cut.splits, w.count = (N / cut.edge) * (K / cut.edge) * cut.splits;
+            w.k_chunks = M / 64, w.accumulate = e.accumulate, w.split_stride = e.split_stride;
+            launch_wgrad_tiles(stream, w, cut.edge, w.count);
+        } else if (takes_64(tile, M)) {
+            launch_gemm64<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, cut.splits, e);
+        } else {
+            dispatch_gemm<false, false>(stream, tile, dY, lddy, X, ldx, N, K, M, cut.splits, e);
+        }
+        if (!need)
+            return;
         const size_t quads = size_t(N) * K / 4;
         const int blocks = int((quads + 255) / 256 < 4096 ? (quads + 255) / 256 : 4096);
         hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream,
-                           static_cast<const float *>(workspace), size_t(N) * K, splits, dW, N, K, lddw,
+                           static_cast<const float *>(workspace), size_t(N) * K, cut.splits, dW, N, K, lddw,
                            accumulate);
         check_hip(hipGetLastError(), "split-K reduce launch: ");
     });
@@ -2279,8 +2327,8 @@ struct WgradListPlan {
 };
 // `unit`: what every width has to be a multiple of.  The tile is the one with the least time by these estimates (us, a
 // stage = 64 tokens of the deepest unit's tiles): 256 x 256: 1.34 a stage in whole rounds, and for the rest 10 + 1.5 a
-// stage, + 15 where it is cut into token ranges and folded; 128 x 128: 0.66 a stage alone on a unit, 0.55 each with
-// company; 64 x 64: 0.24 and 0.20.  Measured: 26 products of d_model 256 over 2048 tokens 46 us on 256, 31 on 128.
+// stage, + 15 where it is cut into token ranges and folded; the other two as wgrad_stage_us has it.  Measured: 26 products of d_model 256 over
+// 2048 tokens 46 us on 256, 31 on 128.
 bool plan_wgrad_list(int M, int count, const TgkWgradJob *jobs, int unit, WgradListPlan &plan, std::string &why) {
     if (count < 1 || count > 4096 || !jobs) {
         why = "gemm_wgrad_list: between 1 and 4096 jobs";
@@ -2301,11 +2349,11 @@ bool plan_wgrad_list(int M, int count, const TgkWgradJob *jobs, int unit, WgradL
         elements += int64_t(jobs[j].N) * jobs[j].K;
     }
     const int units = compute_units(), stages = M / 64;
-    const auto estimate = [&](int edge, double alone, double each) {
+    const auto estimate = [&](int edge) {
         const int deepest = int((elements / (edge * edge) + units - 1) / units);
-        return stages * (deepest == 1 ? alone : each * deepest);
+        return 3.5 + stages * wgrad_stage_us(edge, deepest);
     };
-    const double on_128 = estimate(128, 0.66, 0.55), on_64 = estimate(64, 0.24, 0.20);
+    const double on_128 = estimate(128), on_64 = estimate(64);
     plan = WgradListPlan{};
     plan.edge = on_128 <= on_64 ? 128 : 64;
     if (by_256) {
@@ -2399,9 +2447,7 @@ void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, i
             w.jobs = static_cast<const WgradListJob *>(table);
             w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
             w.count = plan.tiles, w.k_chunks = M / 64, w.sumsq = sumsq;
-            if (plan.edge == 64)
-                return launch_wgrad_tiles<64, 64, 3>(stream, w, plan.launch_blocks);
-            return launch_wgrad_tiles<128, 128, 2>(stream, w, plan.launch_blocks);
+            return launch_wgrad_tiles(stream, w, plan.edge, plan.launch_blocks);
         }
         WgradList w{};
         w.jobs = static_cast<const WgradListJob *>(table);
