@@ -64,11 +64,10 @@ StepRates onecycle_point(const OneCycle &s, int step) {
 } // namespace
 
 // Everything one batch in flight owns: its stream, its tokens, its saved activations and its gradient.
-// A synchronous engine has one slot on the engine's stream; inflight = K gives K slots on K streams
+// Slot 0 is on the engine's stream (a synchronous engine has no other); inflight = K gives K slots on K streams
 // (the worker teams of cuda/pipeline.cuh:52-92).
 struct Slot {
     hipStream_t stream = nullptr;
-    hipEvent_t ready = nullptr; // the gradient of the slot's latest step is complete
     uint8_t *input = nullptr, *target = nullptr;
     float *token_losses = nullptr, *gradient = nullptr;
     std::vector<bf16_t *> x; // x[l] = input of block l; x[depth] = output of the last block
@@ -202,8 +201,6 @@ struct Engine {
         for (void *allocation : allocations)
             (void)hipFree(allocation);
         for (Slot &slot : slots) {
-            if (slot.ready)
-                (void)hipEventDestroy(slot.ready);
             if (slot.stream && slot.stream != stream)
                 (void)hipStreamDestroy(slot.stream);
         }
@@ -336,10 +333,11 @@ struct Engine {
             OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
     }
 
-    // cuda/optim.cuh:66-106 for optimizer step `at` (0-based), on the engine's stream: gradient -> the weights of
-    // version `to`, from the previous version's, `now`.
+    // cuda/optim.cuh:66-106 for optimizer step `at` (0-based), on `stream`: gradient -> the weights of version `to`, from
+    // the previous version's, `now`.
     // `from`: the slot whose backward pass has just written `gradient`, when it left the sums of squares with it
-    void optimize(uint64_t at, const float *gradient, const Version &now, Version &to, const Slot *from = nullptr) {
+    void optimize(hipStream_t stream, uint64_t at, const float *gradient, const Version &now, Version &to,
+                  const Slot *from = nullptr) {
         const Config &c = config.base;
         uint16_t *weight_hi = to.hi, *weight_lo = to.lo, *weight_t = to.t;
         float lr = c.learning_rate, beta1 = c.beta1, muon_lr = c.muon_lr, muon_momentum = c.momentum;
@@ -387,28 +385,30 @@ struct Engine {
         backward(s, v);
     }
     // One training step.  Synchronous engine: everything in order on the one stream, weights updated in place
-    // (cuda/trainer.cuh:109-124).  inflight = K (cuda/pipeline.cuh:40-126 as streams and events): batch `at`
-    // runs on slot at % K with the oldest version the ring still guarantees, max(floor, at - K + 1), so it
-    // only waits for optimizer step at - K (which also freed the slot's gradient); the optimizer step waits for
-    // the batch, copies version `at` into ring place at + 1 and updates it there.  The choice is made on the
-    // host, so a run is reproducible; the staleness bound at - K + 1 <= version <= at is the reference's.
+    // (cuda/trainer.cuh:109-124).  inflight = K (cuda/pipeline.cuh:40-126 as streams and events): batch `at` and its
+    // optimizer step run on the stream of slot at % K, behind optimizer step at - K.  That order alone lets the batch
+    // read max(floor, at - K + 1), the oldest version the ring still guarantees, and frees the slot's gradient.  The
+    // optimizer step waits for its predecessor, on another slot's stream; the version that it overwrites, at - K, was
+    // last read by batch at - 1, which that predecessor follows.  Optimizer steps on a stream of their own (K + 1
+    // streams) cost two more events a step and shared one of the process's four hardware queues with a slot at K = 4:
+    // the width-16 network of depth 8, context 8, batch 16 took 54 us a step, now 36 to 40.  The choice is made on the host, so a run is reproducible; the staleness
+    // bound at - K + 1 <= version <= at is the reference's.
     void train_step(uint64_t at, float *history_row, int *trace) {
         const uint64_t K = slots.size(), ring = versions.size();
         if (K == 1) {
             batch_gradient(slots[0], versions[0], at, history_row);
-            optimize(at, slots[0].gradient, versions[0], versions[0], &slots[0]);
+            optimize(stream, at, slots[0].gradient, versions[0], versions[0], &slots[0]);
             *trace = int(at);
             return;
         }
         Slot &s = slots[at % K];
         const uint64_t read = std::max(floor, at + 1 >= K ? at + 1 - K : 0);
-        check_hip(hipStreamWaitEvent(s.stream, versions[read % ring].done, 0));
         batch_gradient(s, versions[read % ring], at, history_row);
-        check_hip(hipEventRecord(s.ready, s.stream));
-        Version &from = versions[at % ring], &to = versions[(at + 1) % ring];
-        check_hip(hipStreamWaitEvent(stream, s.ready, 0));
-        optimize(at, s.gradient, from, to, &s);
-        check_hip(hipEventRecord(to.done, stream));
+        const Version &from = versions[at % ring];
+        Version &to = versions[(at + 1) % ring];
+        check_hip(hipStreamWaitEvent(s.stream, from.done, 0));
+        optimize(s.stream, at, s.gradient, from, to, &s);
+        check_hip(hipEventRecord(to.done, s.stream));
         *trace = int(read);
         total_staleness += at - read;
         max_staleness = std::max(max_staleness, int(at - read));
@@ -445,12 +445,10 @@ void build_slots(Engine *e, int inflight, bool transposed_copies) {
     e->slots.resize(size_t(inflight));
     e->versions.resize(inflight > 1 ? size_t(inflight) + 1 : 1);
     for (Slot &slot : e->slots) {
-        if (inflight > 1) {
-            check_hip(hipStreamCreate(&slot.stream)); // default priority
-            check_hip(hipEventCreateWithFlags(&slot.ready, hipEventDisableTiming));
-        } else {
+        if (&slot == &e->slots[0])
             slot.stream = e->stream;
-        }
+        else
+            check_hip(hipStreamCreate(&slot.stream)); // default priority
         e->allocate(slot.input, M);
         e->allocate(slot.target, M);
         e->allocate(slot.token_losses, M);
@@ -990,7 +988,7 @@ TG_API int tg_optimizer_test(Engine *e, const float *gradient, int steps) {
         e->use_device();
         e->upload(e->slots[0].gradient, gradient, size_t(e->layout.count));
         for (int i = 0; i < steps; ++i)
-            e->optimize(e->step + uint64_t(i), e->slots[0].gradient, e->versions[0], e->versions[0]);
+            e->optimize(e->stream, e->step + uint64_t(i), e->slots[0].gradient, e->versions[0], e->versions[0]);
         e->step += uint64_t(steps);
         e->sync();
     });
