@@ -1,0 +1,27 @@
+"""A fixed batch that is only evaluated runs the up projection without its pre-activation output (EPI_GELU_ONLY,
+csrc/gemm.hip): the same sums and roundings as with it, so the logits and losses are those of the batch with a gradient,
+bit for bit, on each kernel that has the epilogue."""
+import numpy as np
+import pytest
+
+from turbogpt_amd.bridge import ModelConfig, Native
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,ffn,context,batch", [(128, 256, 128, 1),     # 64 x 64 tiles
+                                                 (256, 1024, 256, 8),    # 64 x 128 tiles
+                                                 (640, 2560, 512, 8),    # 128 x 128 tiles
+                                                 (1024, 4096, 1024, 4),  # 256 x 128 tiles
+                                                 (384, 1536, 1024, 16)])  # 128 x 192 tiles
+def test_evaluation_matches_the_batch_with_gradient(d, ffn, context, batch):
+    rng = np.random.default_rng(d + context)
+    tokens = rng.integers(0, 256, (2, batch, context), dtype=np.uint8)
+    with Native(ModelConfig(d_model=d, depth=1, ffn=ffn, context=context, batch=batch)) as engine:
+        weights = (rng.standard_normal(engine.count) * 0.05).astype(np.float32)
+        engine.set_weights(weights)
+        only = engine.batch(tokens[0], tokens[1], backward=False)
+        full = engine.batch(tokens[0], tokens[1], backward=True)
+    assert np.isfinite(full[0]).all()
+    assert np.array_equal(only[0], full[0])
+    assert np.array_equal(only[-1], full[-1])

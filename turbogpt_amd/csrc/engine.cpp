@@ -263,7 +263,10 @@ struct Engine {
             OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, d, o, d, w(p.attn_out), d, b.mid, d, in, d, nullptr, 0));
             OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, b.mid, w(p.ln2_g), wl(p.ln2_g), w(p.ln2_b), wl(p.ln2_b), b.n2,
                                  config.ln_eps));
-            OP(TG_CLASS_GEMM_FWD_GELU, tgk_gemm_fwd(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.u, F, nullptr, 0, b.a, F));
+            if (with_gradient)
+                OP(TG_CLASS_GEMM_FWD_GELU, tgk_gemm_fwd(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.u, F, nullptr, 0, b.a, F));
+            else
+                OP(TG_CLASS_GEMM_FWD_GELU, gemm_fwd_gelu_only(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.a, F));
             OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, F, b.a, F, w(p.mlp_down), F, x[l + 1], d, b.mid, d, nullptr, 0));
         }
         OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[c.depth], w(layout.lnf_g), wl(layout.lnf_g), w(layout.lnf_b),

@@ -33,7 +33,8 @@
 
 namespace {
 
-enum EpilogueMode { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_GELU = 2, EPI_GELU_BWD = 3 };
+// GELU_CACHED: as GELU, the outputs left to the caches; GELU_ONLY: the activation alone
+enum EpilogueMode { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_GELU = 2, EPI_GELU_BWD = 3, EPI_GELU_CACHED = 4, EPI_GELU_ONLY = 5 };
 
 // An accumulator lane holds 4 consecutive n of one m per register quad.  A plain epilogue (fp32
 // outputs) stores from that layout.  A STAGED epilogue has the kernel round each 32x32 tile to bf16 and
@@ -47,7 +48,7 @@ struct EpilogueBf16 {
     int ld_out;
     const bf16_t *aux; // residual (EPI_RESIDUAL) or saved pre-activation (EPI_GELU_BWD)
     int ld_aux;
-    bf16_t *out2; // GELU output (EPI_GELU)
+    bf16_t *out2; // GELU output (EPI_GELU and its two variants)
     int ld_out2;
     int mode;
     TG_DEVICE bool wants_aux() const { return mode == EPI_RESIDUAL || mode == EPI_GELU_BWD; }
@@ -67,11 +68,17 @@ struct EpilogueBf16 {
             for (int e = 0; e < 4; ++e)
                 y[e] = pack_bf16(bf16_lo(y[e]) * gelu_grad_f(bf16_lo(a[e])),
                                  bf16_hi(y[e]) * gelu_grad_f(bf16_hi(a[e])));
-        } else if constexpr (MODE == EPI_GELU) {
+        } else if constexpr (MODE == EPI_GELU || MODE == EPI_GELU_CACHED || MODE == EPI_GELU_ONLY) {
             u32x4 g;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 g[e] = pack_bf16(gelu_f(bf16_lo(y[e])), gelu_f(bf16_hi(y[e])));
+            if constexpr (MODE != EPI_GELU) {
+                *reinterpret_cast<u32x4 *>(out2 + size_t(m) * ld_out2 + n) = g;
+                if constexpr (MODE == EPI_GELU_CACHED)
+                    *reinterpret_cast<u32x4 *>(out + size_t(m) * ld_out + n) = y;
+                return;
+            }
             // Both outputs stream past the L2: the pre-activation is not read again before the backward pass, and the
             // activation (100 MB at the training shape) is far larger than the L2, whose lines the operand panels of
             // this product need (measured on the step: -0.8 % for the first, another -0.8 % for the second; the
@@ -89,6 +96,8 @@ struct EpilogueBf16 {
             finish_as<EPI_GELU_BWD>(m, n, y, a);
         else if (mode == EPI_GELU)
             finish_as<EPI_GELU>(m, n, y, a);
+        else if (mode == EPI_GELU_ONLY)
+            finish_as<EPI_GELU_ONLY>(m, n, y, a);
         else
             finish_as<EPI_PLAIN>(m, n, y, a);
     }
@@ -101,7 +110,8 @@ template <int MODE> struct EpilogueBf16As {
     static constexpr bool BF16 = true;
     // vector-memory instructions per 32 x 32 block of the staged epilogue: two 16-byte stores (four with the GELU
     // output), two 16-byte loads of the second input
-    static constexpr int MEMORY_OPS_PER_BLOCK = MODE == EPI_PLAIN ? 2 : 4;
+    static constexpr int MEMORY_OPS_PER_BLOCK = MODE == EPI_PLAIN || MODE == EPI_GELU_ONLY ? 2 : 4;
+    using Cached = EpilogueBf16As<MODE == EPI_GELU ? int(EPI_GELU_CACHED) : MODE>;
     EpilogueBf16 any;
     TG_DEVICE bool wants_aux() const { return MODE == EPI_RESIDUAL || MODE == EPI_GELU_BWD; }
     TG_DEVICE u32x4 load_aux(int m, int n) const { return any.load_aux(m, n); }
@@ -1886,6 +1896,8 @@ void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const
         return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
     case EPI_GELU:
         return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
+    case EPI_GELU_ONLY:
+        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
     case EPI_GELU_BWD:
         return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_BWD>{e});
     default:
@@ -1895,8 +1907,11 @@ void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const
 
 template <int BM, int BN, int S, bool BKC, class Epilogue>
 void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
-                      const Epilogue &epilogue) {
-    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, Epilogue>;
+                      const Epilogue &given) {
+    // these sizes' GELU outputs are left to the caches, where the next launch finds them (streamed past them the product
+    // itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %)
+    const typename Epilogue::Cached epilogue{given.any};
+    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, typename Epilogue::Cached>;
     constexpr size_t lds = S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
@@ -1965,6 +1980,10 @@ void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_
         return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
     case EPI_GELU:
         return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
+    case EPI_GELU_ONLY:
+        if constexpr (BKC)
+            return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
+        throw std::logic_error("gemm: no such epilogue on a k-strided weight");
     case EPI_GELU_BWD:
         return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_BWD>{e});
     default:
@@ -2057,34 +2076,50 @@ WgradCut plan_wgrad(int M, int N, int K) {
 
 } // namespace
 
+namespace {
+// Y = X W^T with one of the epilogues; Y may be NULL with EPI_GELU_ONLY
+void gemm_fwd(hipStream_t stream, int M, int N, int K, const bf16_t *X, int ldx, const bf16_t *W, int ldw, const EpilogueBf16 &e) {
+    require(M > 0 && N > 0 && K > 0, "gemm_fwd: empty shape");
+    require(K % BK == 0, "gemm_fwd: K must be a multiple of 32");
+    const Tile tile = choose_tile(M, N);
+    require(tile != TILE_NONE, "gemm_fwd: M must be a multiple of 128 and N of 128 or 192");
+    check_operand(X, ldx, "X");
+    check_operand(W, ldw, "W");
+    if (e.mode != EPI_GELU_ONLY)
+        check_operand(e.out, e.ld_out, "Y");
+    if (e.aux)
+        check_operand(e.aux, e.ld_aux, "residual");
+    if (e.out2)
+        check_operand(e.out2, e.ld_out2, "gelu_out");
+    if (takes_256x192(M, N, K, e.mode))
+        launch_gemm256_bf16(stream, X, ldx, W, ldw, M, N, K, e);
+    else if (takes_256x128(M, N, K))
+        launch_gemm256x128_bf16(stream, X, ldx, W, ldw, M, N, K, e);
+    else if (takes_64(tile, K))
+        launch_block_bf16<true>(stream, X, ldx, W, ldw, M, N, K, e);
+    else
+        dispatch_gemm<true, true>(stream, tile, X, ldx, W, ldw, M, N, K, 1, e);
+}
+} // namespace
+
 extern "C" int tgk_gemm_fwd(hipStream_t stream, int M, int N, int K, const uint16_t *X, int ldx,
                             const uint16_t *W, int ldw, uint16_t *Y, int ldy,
                             const uint16_t *residual, int ldr, uint16_t *gelu_out, int ldg) {
     return guarded([&] {
-        require(M > 0 && N > 0 && K > 0, "gemm_fwd: empty shape");
-        require(K % BK == 0, "gemm_fwd: K must be a multiple of 32");
-        const Tile tile = choose_tile(M, N);
-        require(tile != TILE_NONE, "gemm_fwd: M must be a multiple of 128 and N of 128 or 192");
         require(!(residual && gelu_out), "gemm_fwd: residual and GELU epilogues are exclusive");
-        check_operand(X, ldx, "X");
-        check_operand(W, ldw, "W");
-        check_operand(Y, ldy, "Y");
         EpilogueBf16 e{Y, ldy, nullptr, 0, nullptr, 0, EPI_PLAIN};
-        if (residual) {
-            check_operand(residual, ldr, "residual");
+        if (residual)
             e.aux = residual, e.ld_aux = ldr, e.mode = EPI_RESIDUAL;
-        } else if (gelu_out) {
-            check_operand(gelu_out, ldg, "gelu_out");
+        else if (gelu_out)
             e.out2 = gelu_out, e.ld_out2 = ldg, e.mode = EPI_GELU;
-        }
-        if (takes_256x192(M, N, K, e.mode))
-            launch_gemm256_bf16(stream, X, ldx, W, ldw, M, N, K, e);
-        else if (takes_256x128(M, N, K))
-            launch_gemm256x128_bf16(stream, X, ldx, W, ldw, M, N, K, e);
-        else if (takes_64(tile, K))
-            launch_block_bf16<true>(stream, X, ldx, W, ldw, M, N, K, e);
-        else
-            dispatch_gemm<true, true>(stream, tile, X, ldx, W, ldw, M, N, K, 1, e);
+        gemm_fwd(stream, M, N, K, X, ldx, W, ldw, e);
+    });
+}
+int gemm_fwd_gelu_only(hipStream_t stream, int M, int N, int K, const bf16_t *X, int ldx, const bf16_t *W, int ldw,
+                       bf16_t *activation, int lda) {
+    return guarded([&] {
+        check_operand(activation, lda, "gelu_out");
+        gemm_fwd(stream, M, N, K, X, ldx, W, ldw, {nullptr, 0, nullptr, 0, activation, lda, EPI_GELU_ONLY});
     });
 }
 

@@ -9,3 +9,7 @@ int wgrad_list_sumsq_count(int M, int count, const TgkWgradJob *jobs, int unit);
 void wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, int unit, void *table, size_t table_bytes);
 void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
                 size_t workspace_bytes, float *sumsq);
+
+// tgk_gemm_fwd with gelu_out where no backward pass follows: the pre-activation is not written.  0 or -1, as there.
+int gemm_fwd_gelu_only(hipStream_t stream, int M, int N, int K, const bf16_t *X, int ldx, const bf16_t *W, int ldw,
+                       bf16_t *activation, int lda);
