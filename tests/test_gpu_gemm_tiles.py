@@ -13,7 +13,9 @@ BF16 = torch.bfloat16
 SHAPES = [(128, 128, 64),      # 64 x 64: 4 tiles, one stage
           (384, 640, 192),     # 64 x 64: 60 tiles, three stages
           (1920, 640, 128),    # 64 x 64: 300 tiles, two on some units
-          (128, 192, 576),     # 64 x 64: a width 128 does not divide
+          (128, 192, 576),     # 64 x 64, two groups of waves, nine stages: a width 128 does not divide
+          (640, 640, 320),     # the same, five stages
+          (128, 128, 2048),    # the same, 32 stages
           (1024, 2304, 64),    # 64 x 128: 288 tiles, one stage
           (1152, 1920, 320),   # 64 x 128: 270 tiles, five stages
           (1920, 1920, 64),    # 128 x 128, deep ring: one stage

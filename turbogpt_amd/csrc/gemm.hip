@@ -757,16 +757,28 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
 // once (one LDS round trip; read column by column as in multiply_stage, 1024 x 768 with K = 3072 took 17.1 us instead of
 // 13.9), the copies of the stage S - 1 further on, then the matrix instructions, which add in the same order as
 // gemm64_kernel.  Ends behind a barrier: the slots are free.
-template <int BM, int BN, int S, bool AKC, bool BKC> struct TileProduct {
+// GROUPS = 2: two such groups of four waves take the two halves of the stages, each through its own ring (`smem` is the
+// first's), and the second hands its sums to the first, which alone ends with the product.
+template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1> struct TileProduct {
     using TA = typename Tile64Of<BM, AKC>::type;
     using TB = typename Tile64Of<BN, BKC>::type;
     static constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, THREADS = 256;
     static constexpr int LA = TA::LOADS, LB = TB::LOADS, LOADS = LA + LB, SLOT = TA::BYTES + TB::BYTES;
     static_assert(S >= 2 && (S - 1) * LOADS <= 63, "the copies in flight fit the wave's counter");
-    TG_DEVICE static void run(const bf16_t *A, int lda, const bf16_t *B, int ldb, int m0, int n0, int k_chunks,
+    static_assert(GROUPS == 1 || (GROUPS == 2 && BM * BN * 4 <= S * SLOT), "the second group's sums fit its ring");
+    TG_DEVICE static void run(const bf16_t *A, int lda, const bf16_t *B, int ldb, int m0, int n0, int all_chunks,
                               unsigned char *smem, f32x4 (&acc)[FM][FN][2][2]) {
+        const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+        // the first group has the odd stage: the other idles through the last round's barrier
+        const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+        const int rounds = GROUPS == 1 ? all_chunks : (all_chunks + 1) >> 1;
+        const int k_chunks = group == 0 ? rounds : all_chunks - rounds;
+        if (GROUPS > 1) {
+            A += group * rounds * TA::step(lda);
+            B += group * rounds * TB::step(ldb);
+            smem += group * (S * SLOT);
+        }
         const uint32_t smem_base = lds_address(smem);
-        const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
         const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
         const bf16_t *pa[LA], *pb[LB];
         const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
@@ -803,7 +815,11 @@ template <int BM, int BN, int S, bool AKC, bool BKC> struct TileProduct {
             if (s < k_chunks)
                 copy_stage();
         int c_slot = 0;
-        for (int c = 0; c < k_chunks; ++c) {
+        for (int c = 0; c < rounds; ++c) {
+            if (GROUPS > 1 && c >= k_chunks) {
+                __syncthreads();
+                break;
+            }
             // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
             const int younger = k_chunks - 1 - c;
             if (S >= 4 && younger >= 2)
@@ -840,6 +856,26 @@ template <int BM, int BN, int S, bool AKC, bool BKC> struct TileProduct {
             c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
         }
         __syncthreads(); // other waves may still read the last stage
+        if (GROUPS > 1) { // a lane's sums to the same lane of the first group
+            f32x4 *sums = reinterpret_cast<f32x4 *>(smem + (group == 0 ? S * SLOT : 0)) + wave * (64 * FM * FN * 4) + lane;
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (group == 1)
+                            sums[((i * FN + j) * 4 + t) * 64] = acc[i][j][t >> 1][t & 1];
+            __syncthreads();
+            if (group == 0)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            acc[i][j][t >> 1][t & 1] += sums[((i * FN + j) * 4 + t) * 64];
+        }
     }
 };
 // Consecutive block ids sit on consecutive XCDs: the place in a row-major list of tiles that gives each XCD a contiguous run.
@@ -852,28 +888,32 @@ TG_DEVICE int xcd_contiguous(int block, int blocks) {
 // C = A B^T with A k-contiguous and B either way round.  A product with few outputs is bound by how many compute units
 // have a tile and by the latency of each 64-k stage on them, not by bytes per flop: 1024 x 768 outputs are 32 tiles of
 // 128 x 192 but 192 of 64 x 64.  So the tile is a parameter (choose_block) and a block computes one of them; the sums run in
-// the same order whatever the tile: results are bit-identical.  Tried and slower at 1024 x 768, K = 3072: reading stage
+// the same order whatever the tile: results are bit-identical, except where two groups of waves (GROUPS) halve the reduced
+// dimension.  Tried and slower at 1024 x 768, K = 3072: reading stage
 // c + 1's fragments under stage c's products (16.6 us).
 // Measured against the 128-row tiles that took these shapes before, us (M x N, K; weights [N][K]): 2048 x 256, 1024: 12.6 ->
-// 6.2; 1920 x 640, 1920: 25.5 -> 12.9; 1024 x 768, 3072: 40.6 -> 14.9; 1024 x 2304, 768: 13.2 -> 9.0; 8192 x 512, 2048: 28.5 ->
-// 22.3; 16384 x 256, 768: 13.4 -> 10.6; with B k-strided (weights [K][N]) 1024 x 768, 3072: 55.1 -> 15.2; 4096 x 3072, 768: 27.6 -> 22.8;
+// 5.6; 1920 x 640, 1920: 25.5 -> 12.9; 1024 x 768, 3072: 40.6 -> 12.3; 1024 x 2304, 768: 13.2 -> 9.0; 8192 x 512, 2048: 28.5 ->
+// 22.3; 16384 x 256, 768: 13.4 -> 10.6; with B k-strided (weights [K][N]) 1024 x 768, 3072: 55.1 -> 12.6; 4096 x 3072, 768: 27.6 -> 22.8;
 // 16384 x 2304, 768: 77.0 -> 67.6.
-template <int BM, int BN, int S, bool BKC, class Epilogue>
-__global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B,
-                                                        int ldb, int k_chunks, int tiles_n, Epilogue epilogue) {
-    using P = TileProduct<BM, BN, S, true, BKC>;
+template <int BM, int BN, int S, bool BKC, class Epilogue, int GROUPS = 1>
+__global__ __launch_bounds__(256 * GROUPS) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda,
+                                                                 const bf16_t *__restrict__ B, int ldb, int k_chunks,
+                                                                 int tiles_n, Epilogue epilogue) {
+    using P = TileProduct<BM, BN, S, true, BKC, GROUPS>;
     static_assert(4 * 2048 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6 & 3;
+    const bool finishes = GROUPS == 1 || threadIdx.x < 256;
     const int tile = xcd_contiguous(blockIdx.x, gridDim.x), m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
     const int m = m0 + (wave >> 1) * P::WM, n = n0 + (wave & 1) * P::WN;
     // the epilogue's second input first of all: it lands before the operands do
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
-    if (epilogue.wants_aux())
+    if (epilogue.wants_aux() && finishes)
         load_aux_pair<P::FM, P::FN>(epilogue, 0, m, n, lane, aux);
     f32x4 acc[P::FM][P::FN][2][2];
     P::run(A, lda, B, ldb, m0, n0, k_chunks, smem, acc);
-    staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
+    if (finishes)
+        staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
 }
 
 TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64::frag16's address
@@ -1608,12 +1648,14 @@ struct WgradTiles {
     size_t split_stride;  // then `one.dw` is the first of `splits` slabs this far apart, for splitk_reduce_kernel
     float *sumsq; // optional: one sum of squares a block
 };
-template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_tiles_kernel(const WgradTiles w) {
-    using P = TileProduct<BM, BN, S, false, false>;
+template <int BM, int BN, int S, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) void wgrad_tiles_kernel(const WgradTiles w) {
+    using P = TileProduct<BM, BN, S, false, false, GROUPS>;
     static_assert(4 * 4096 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float waves[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6 & 3;
+    const bool finishes = GROUPS == 1 || threadIdx.x < 256;
     float squares = 0.f;
     for (int base = 0; base + int(blockIdx.x) < w.count; base += gridDim.x) {
         const int at = base + xcd_contiguous(blockIdx.x, min(int(gridDim.x), w.count - base));
@@ -1627,9 +1669,10 @@ template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_ti
         P::run(job.dy + int64_t(first) * 64 * job.lddy, job.lddy, job.x + int64_t(first) * 64 * job.ldx, job.ldx, t.y, t.z,
                chunks, smem, acc);
         const EpilogueF32 epilogue{job.dw, job.lddw, w.split_stride, w.accumulate};
-        staged_store_f32<P::FM, P::FN>(acc, smem + wave * 4096, epilogue, t.y + (wave >> 1) * P::WM, t.z + (wave & 1) * P::WN,
-                                       lane, split);
-        if (w.sumsq)
+        if (finishes)
+            staged_store_f32<P::FM, P::FN>(acc, smem + wave * 4096, epilogue, t.y + (wave >> 1) * P::WM,
+                                           t.z + (wave & 1) * P::WN, lane, split);
+        if (w.sumsq && finishes)
 #pragma unroll
             for (int i = 0; i < P::FM; ++i)
 #pragma unroll
@@ -1643,7 +1686,7 @@ template <int BM, int BN, int S> __global__ __launch_bounds__(256) void wgrad_ti
     }
     if (w.sumsq) {
         squares = wave_sum(squares);
-        if (lane == 0)
+        if (lane == 0 && finishes)
             waves[wave] = squares;
         __syncthreads();
         if (threadIdx.x == 0)
@@ -1905,14 +1948,14 @@ void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const
     }
 }
 
-template <int BM, int BN, int S, bool BKC, class Epilogue>
+template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
 void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                       const Epilogue &given) {
     // these sizes' GELU outputs are left to the caches, where the next launch finds them (streamed past them the product
     // itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %)
     const typename Epilogue::Cached epilogue{given.any};
-    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, typename Epilogue::Cached>;
-    constexpr size_t lds = S * (BM + BN) * 128;
+    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, typename Epilogue::Cached, GROUPS>;
+    constexpr size_t lds = GROUPS * S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
     if (!configured[device].load(std::memory_order_acquire)) {
@@ -1921,7 +1964,7 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256), lds, stream, A, lda, B, ldb,
+    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256 * GROUPS), lds, stream, A, lda, B, ldb,
                        K / 64, N / BN, epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
@@ -1952,6 +1995,11 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
                   const Epilogue &e) {
     switch (block) {
     case BLOCK_64x64:
+        // alone on its unit a block of four waves reads fragments, then multiplies; a second group fills the gaps
+        // (us a 64-k stage 0.23 -> 0.16; 1024 x 768, K = 3072 14.7 -> 12.3; 768 5.4 -> 5.1; 2048 x 256, 1024 6.2 -> 5.6; 128 x
+        // 512, 2048 10.0 -> 8.5; no difference up to four stages)
+        if (M / 64 * (N / 64) <= compute_units() && K > 256)
+            return launch_gemm_tile<64, 64, 3, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
         return launch_gemm_tile<64, 64, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
     case BLOCK_64x128:
         return launch_gemm_tile<64, 128, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
@@ -1991,9 +2039,9 @@ void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_
     }
 }
 
-template <int BM, int BN, int S> void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int blocks) {
-    auto kernel = wgrad_tiles_kernel<BM, BN, S>;
-    constexpr size_t lds = S * (BM + BN) * 128;
+template <int BM, int BN, int S, int GROUPS> void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int blocks) {
+    auto kernel = wgrad_tiles_kernel<BM, BN, S, GROUPS>;
+    constexpr size_t lds = GROUPS * S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
     if (!configured[device].load(std::memory_order_acquire)) {
@@ -2002,19 +2050,23 @@ template <int BM, int BN, int S> void launch_wgrad_tiles(hipStream_t stream, con
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, w);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256 * GROUPS), lds, stream, w);
     check_hip(hipGetLastError(), "wgrad tiles launch: ");
 }
 
-// 128 x 128: alone on its unit a block has room for four stages (8192, 896 x 3584: 0.57 us a stage; 0.66 with two), with
-// another beside it for two.
+// Alone on its unit a 64 x 64 block has two groups of waves (1024, 768 x 768 7.4 -> 6.9 us; 16384, 256 x 1024 21.1 -> 19.8) and a
+// 128 x 128 one four stages (8192, 896 x 3584: 0.57 us a stage, 0.66 with two); two groups there gave 4096, 1024 x 1024 20.4 ->
+// 17.6, but 512 x 2048 21.4 -> 25.5.
 void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int edge, int blocks) {
-    if (edge == 64)
-        launch_wgrad_tiles<64, 64, 3>(stream, w, blocks);
-    else if (blocks <= compute_units())
-        launch_wgrad_tiles<128, 128, 4>(stream, w, blocks);
+    const bool alone = blocks <= compute_units();
+    if (edge == 64 && alone)
+        launch_wgrad_tiles<64, 64, 3, 2>(stream, w, blocks);
+    else if (edge == 64)
+        launch_wgrad_tiles<64, 64, 3, 1>(stream, w, blocks);
+    else if (alone)
+        launch_wgrad_tiles<128, 128, 4, 1>(stream, w, blocks);
     else
-        launch_wgrad_tiles<128, 128, 2>(stream, w, blocks);
+        launch_wgrad_tiles<128, 128, 2, 1>(stream, w, blocks);
 }
 
 void check_operand(const void *p, int ld, const char *name) {
@@ -2035,7 +2087,7 @@ int wgrad_splits(Tile tile, int tiles, int k_tiles) {
 // Time of 64 tokens on a unit that has `deepest` tiles of wgrad_tiles_kernel (us, measured over the shapes named below).
 double wgrad_stage_us(int edge, int deepest) {
     if (edge == 64)
-        return deepest == 1 ? 0.25 : deepest == 2 ? 0.37 : 0.19 * deepest;
+        return deepest == 1 ? 0.23 : deepest == 2 ? 0.37 : 0.19 * deepest;
     return deepest == 1 ? 0.56 : deepest / 2 * 0.76 + deepest % 2 * 0.66;
 }
 // How one weight gradient is cut: tiles of `edge` and token ranges (slabs that a second launch folds), or edge 0: the
