@@ -1,5 +1,5 @@
 """Attention on 32-row blocks whose waves share out the tiles, and on either side of the rule that chooses them
-(split_tiles in csrc/attention.hip), with (batch, head) counts that eight does not divide: against fp32 attention.  Bound:
+(forward_splits and backward_way in csrc/attention.hip), with (batch, head) counts that eight does not divide: against fp32 attention.  Bound:
 three bf16 roundings of at most 2^-9 each (probabilities, score gradients or outputs, result), 6e-3 in relative L2; the
 log-sum-exp stays fp32."""
 import pytest
@@ -22,11 +22,17 @@ def reference(qkv, do, B, H, T):
 
 @pytest.mark.parametrize("B,H,T", [(1, 1, 128),    # fewer tiles than waves
                                    (2, 3, 384),    # six tiles: two waves take two
-                                   (16, 9, 128),   # the most blocks that are split at this context
+                                   (16, 9, 128),   # the most blocks that the forward splits at this context
                                    (29, 5, 128),   # one more
+                                   (9, 12, 128),   # the most that the backward splits
+                                   (109, 1, 128),  # one more: its kernels side by side
+                                   (32, 6, 256),   # the most that run side by side at this context
+                                   (11, 7, 640),   # one more
+                                   (4, 13, 1024),  # side by side, pairs dealt
+                                   (5, 13, 1024),  # one after the other
                                    (1, 3, 1280),   # every pair dealt over the XCDs
                                    (1, 9, 1024),   # one of nine dealt
-                                   (3, 11, 1024)])  # forward split, backward not, one pair dealt in both
+                                   (3, 11, 1024)])  # forward split, backward side by side, one pair dealt in both
 def test_matches_fp32(B, H, T):
     lib, d = library(), 64 * H
     gen = torch.Generator(device="cuda").manual_seed(B * 10000 + H * 100 + T)

@@ -18,8 +18,10 @@
 //
 // Where 128-row blocks would leave the chip part idle (few or short sequences), blocks of 32 rows take their place,
 // whose four waves share out the tiles of the reduced side: attn_fwd_split_kernel, and attn_bwd_split_kernel for the
-// whole backward in one launch (split_tiles has the rule).
+// whole backward in one launch; between those sizes and the large ones the two backward kernels run side by side
+// (forward_splits and backward_way have the rules).
 #include "common.h"
+#include <algorithm>
 #include <atomic>
 #include "../../include/tgk_kernels.h"
 
@@ -463,15 +465,13 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
 // of both outputs.  The two 32-query halves of a tile are processed one after the other to keep the
 // live accumulators, and with them the register count, down.
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
-    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
-    const bf16_t *__restrict__ dO, int lddo, const float *__restrict__ lse2,
-    const float *__restrict__ delta, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
-    __shared__ __align__(1024) bf16_t stages[3][2][TILE_ELEMS]; // [stage][Q | dO]
-    __shared__ __align__(256) float rows[3][2][64];             // [stage][lse2 | -delta]
-    const CausalBlock block = grid.block(blockIdx.x);
-    if (!block.live)
-        return;
+typedef bf16_t TileStages[3][2][TILE_ELEMS];
+typedef float RowStages[3][2][64];
+TG_DEVICE void dkdv_block(TileStages &stages /* [stage][Q | dO] */, RowStages &rows /* [stage][lse2 | -delta] */,
+                          const CausalBlock &block, const CausalGrid &grid, const bf16_t *__restrict__ Q,
+                          const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld, const bf16_t *__restrict__ dO,
+                          int lddo, const float *__restrict__ lse2, const float *__restrict__ delta, bf16_t *__restrict__ dK,
+                          bf16_t *__restrict__ dV, int lddq, int T, float scale) {
     const int k0 = block.rank * 128, h = block.h, b = block.b; // early keys see the most queries
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5;
     const int wave_k0 = k0 + wave * 32, krow = wave_k0 + (lane & 31);
@@ -540,19 +540,27 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
     }
 }
 
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(
+    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
+    const bf16_t *__restrict__ dO, int lddo, const float *__restrict__ lse2,
+    const float *__restrict__ delta, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
+    __shared__ __align__(1024) TileStages stages;
+    __shared__ __align__(256) RowStages rows;
+    const CausalBlock block = grid.block(blockIdx.x);
+    if (block.live)
+        dkdv_block(stages, rows, block, grid, Q, K, V, ld, dO, lddo, lse2, delta, dK, dV, lddq, T, scale);
+}
+
 // ---------------------------------------------------------------------------------------------
 // dQ: block = 128 queries (4 waves x 32), loops over 64-key tiles up to the diagonal; K and V tiles
 // arrive by asynchronous copies two tiles ahead; 32-key halves are processed in turn.
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
-    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
-    const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo,
-    const float *__restrict__ LSE, float *__restrict__ lse2_out, float *__restrict__ delta_out,
-    bf16_t *__restrict__ dQ, int lddq, int T, CausalGrid grid, float scale) {
-    __shared__ __align__(1024) bf16_t stages[3][2][TILE_ELEMS]; // [stage][K | V]
-    const CausalBlock block = grid.block(blockIdx.x);
-    if (!block.live)
-        return;
+// `lse2_out` and `delta_out` may be NULL.
+TG_DEVICE void dq_block(TileStages &stages /* [stage][K | V] */, const CausalBlock &block, const CausalGrid &grid,
+                        const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
+                        const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo,
+                        const float *__restrict__ LSE, float *__restrict__ lse2_out, float *__restrict__ delta_out,
+                        bf16_t *__restrict__ dQ, int lddq, int T, float scale) {
     const int q0 = (T / 128 - 1 - block.rank) * 128, h = block.h, b = block.b;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5;
     const int wave_q0 = q0 + wave * 32, qrow = wave_q0 + (lane & 31);
@@ -585,7 +593,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
     const float del = row_product(gf, O + (token0 + qrow) * ldo + h * HD, g);
     const size_t row_at = (size_t(b) * grid.H + h) * T + qrow;
     const float lse = LSE[row_at] * LOG2E;
-    if (g == 0) {
+    if (g == 0 && delta_out) {
         delta_out[row_at] = -del; // negated: the dK/dV kernel starts its dP product from it
         lse2_out[row_at] = lse;
     }
@@ -628,6 +636,58 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
         store_acc_rows(qp + dt * 32, dq[dt], scale, g);
 }
 
+__global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
+    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
+    const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo,
+    const float *__restrict__ LSE, float *__restrict__ lse2_out, float *__restrict__ delta_out,
+    bf16_t *__restrict__ dQ, int lddq, int T, CausalGrid grid, float scale) {
+    __shared__ __align__(1024) TileStages stages;
+    const CausalBlock block = grid.block(blockIdx.x);
+    if (block.live)
+        dq_block(stages, block, grid, Q, K, V, ld, dO, lddo, O, ldo, LSE, lse2_out, delta_out, dQ, lddq, T, scale);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The two side by side, where neither fills the units (backward_way has the rule): every other run of eight blocks takes
+// 128 keys, the others 128 queries, and a launch before them leaves the deltas, which the dQ kernel otherwise hands on.
+// ---------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256, 2) void attn_bwd_both_kernel(
+    const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V, int ld,
+    const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo, const float *__restrict__ LSE,
+    const float *__restrict__ lse2, const float *__restrict__ delta, bf16_t *__restrict__ dQ, bf16_t *__restrict__ dK,
+    bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
+    __shared__ __align__(1024) TileStages stages;
+    __shared__ __align__(256) RowStages rows;
+    const CausalBlock block = grid.block((blockIdx.x >> 4) * 8 + (blockIdx.x & 7));
+    if (!block.live)
+        return;
+    if (blockIdx.x & 8)
+        dq_block(stages, block, grid, Q, K, V, ld, dO, lddo, O, ldo, LSE, nullptr, nullptr, dQ, lddq, T, scale);
+    else
+        dkdv_block(stages, rows, block, grid, Q, K, V, ld, dO, lddo, lse2, delta, dK, dV, lddq, T, scale);
+}
+// -rowsum(dO o O) and the log-sum-exp in base 2 of every row: eight lanes a row, eight consecutive queries a wave
+__global__ __launch_bounds__(256) void attn_delta_kernel(const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O,
+                                                         int ldo, const float *__restrict__ LSE, float *__restrict__ lse2,
+                                                         float *__restrict__ delta, int H, int T) {
+    const int per_head = T / 32, head = blockIdx.x / per_head, t = (blockIdx.x - head * per_head) * 32 + (threadIdx.x >> 3);
+    const int b = head / H, h = head - b * H, part = threadIdx.x & 7;
+    const size_t token = size_t(b) * T + t, row = size_t(head) * T + t;
+    const u32x4 x = *reinterpret_cast<const u32x4 *>(dO + token * lddo + h * HD + part * 8);
+    const u32x4 y = *reinterpret_cast<const u32x4 *>(O + token * ldo + h * HD + part * 8);
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        sum = fmaf(bf16_hi(x[e]), bf16_hi(y[e]), fmaf(bf16_lo(x[e]), bf16_lo(y[e]), sum));
+#pragma unroll
+    for (int k = 1; k < 8; k <<= 1)
+        sum += __shfl_xor(sum, k, 64);
+    if (part == 0) {
+        delta[row] = -sum;
+        lse2[row] = LSE[row] * LOG2E;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Few rows.  A wave of the kernels above walks its row's tiles one after another, T/64 of them at worst, at about
 // 0.8 us each, whatever the number of blocks: with one block of 128 rows per compute unit or less that chain is the
@@ -637,7 +697,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(
 // fetched once per 32 rows instead of once per 128 and that the stages are not double buffered (two blocks of 64 KiB
 // per compute unit fill in for each other); the backward is one launch, because its dK/dV blocks form the deltas of
 // their queries themselves.  Microseconds, 128-row blocks -> these (B, H, T), forward; backward:
-//   1,1,128: 4.6 -> 4.0; 11.6 -> 5.4    8,4,256: 6.5 -> 5.0; 16.7 -> 9.0     5,10,384: 8.3 -> 8.3; 21.8 -> 19.6
+//   1,1,128: 4.6 -> 4.0; 11.6 -> 5.4    8,4,256: 6.5 -> 5.0; 16.7 -> 9.0
 //   1,12,1024: 16.1 -> 8.6; 42.1 -> 20.3    1,4,4096: 53 -> 20; 144 -> 58    1,1,8192: 99 -> 31; 273 -> 79
 // ---------------------------------------------------------------------------------------------
 constexpr int WAVES = 4;
@@ -870,17 +930,30 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
 }
 
 // Up to how many 128-row blocks the 32-row ones with shared-out tiles are taken instead.  The longer the context, the
-// longer the chains that they cut, so the line rises with it.  Microseconds, 128-row -> 32-row:
-//   T 128: 128 blocks 5.1 -> 5.0; 12.9 -> 11.0   192: 5.3 -> 7.2; 13.8 -> 15.7
-//   T 256: 128 blocks 6.7 -> 5.7; 17.3 -> 14.2   192: 6.9 -> 8.3; 17.9 -> 19.0
-//   T 512: 192 blocks 10.0 -> 10.0; 25.8 -> 25.6   224: 10.1 -> 10.7; 26.5 -> 28.4
-//   T 1024: 256 blocks 16.7 -> 14.3; 43.3 -> 43.9   320: 17.2 -> 17.5; 46.3 -> 54.5
-//   T 2048: 272 blocks 29.3 -> 20.9; 78 -> 71   384: 29.1 -> 27.2; 81 -> 99    T 4096: 384 blocks 57 -> 43; 150 -> 166
-// The backward does five products where the forward does two and loses by the fetches sooner.
-bool split_tiles(int B, int H, int T, int most_blocks) {
-    return size_t(B) * H * (T / 128) <= size_t(T / 8 + 128 < most_blocks ? T / 8 + 128 : most_blocks);
+// longer the chains that they cut, so the line rises with it.  Forward, microseconds, 128-row -> 32-row:
+//   T 128: 128 blocks 5.1 -> 5.0   192: 5.3 -> 7.2     T 256: 128 blocks 6.7 -> 5.7   192: 6.9 -> 8.3
+//   T 512: 192 blocks 10.0 -> 10.0   224: 10.1 -> 10.7     T 1024: 256 blocks 16.7 -> 14.3   320: 17.2 -> 17.5
+//   T 2048: 272 blocks 29.3 -> 20.9   384: 29.1 -> 27.2     T 4096: 384 blocks 57 -> 43
+bool forward_splits(int B, int H, int T) {
+    return size_t(B) * H * (T / 128) <= size_t(std::min(T / 8 + 128, 384));
 }
-constexpr int SPLIT_FORWARD = 384, SPLIT_BACKWARD = 256;
+// The backward does five products where the forward does two and loses by the split kernel's fetches sooner.  Next come
+// its two kernels side by side, as long as both sets of blocks are about what the units hold (two each).  Microseconds, split
+// / side by side / one after the other:
+//   T 128: 64 blocks 7.1 / 9.4 / 12.6   128: 10.9 / 9.7 / 13.1   256: 19.0 / 13.5 / 14.4
+//   T 256: 64 blocks 8.9 / 11.7 / 17.1   128: 13.4 / 12.3 / 17.3   256: 22.2 / 15.4 / 18.5   512: 47.9 / 28.3 / 24.6
+//   T 512: 64 blocks 10.7 / 16.3 / 25.0   128: 18.0 / 17.2 / 25.5   256: 30.9 / 20.1 / 26.8   384: 45.1 / 27.6 / 30.0
+//     576: 71.1 / 41.5 / 37.6
+//   T 1024: 96 blocks 19.2 / 26.4 / 41.8   192: 34.9 / 29.1 / 42.5   512: 87.0 / 48.9 / 50.8   768: - / 70.5 / 67.5
+//   T 2048: 128 blocks 37.0 / 45.2 / 74.4   256: 68.0 / 51.1 / 75.7   512: 131 / 78.9 / 87.5   768: - / 112 / 108
+//   T 4096: 256 blocks 114 / 93 / 141   512: 225 / 141 / 163     T 8192: 256 blocks 209 / 178 / 272
+enum Backward { BACKWARD_SPLIT, BACKWARD_BOTH, BACKWARD_IN_TURN };
+Backward backward_way(int B, int H, int T) {
+    const size_t blocks = size_t(B) * H * (T / 128);
+    if (blocks <= size_t(std::min({T / 32 + 104, T / 64 + 128, 216})))
+        return BACKWARD_SPLIT;
+    return blocks <= (T < 1024 ? 384 : 512) ? BACKWARD_BOTH : BACKWARD_IN_TURN;
+}
 void check_attention_shape(int B, int H, int T, int hd) {
     require(B > 0 && H > 0 && T > 0, "attention: empty shape");
     require(hd == HD, "attention: head_dim must be 64");
@@ -905,7 +978,7 @@ extern "C" int tgk_attn_fwd(hipStream_t stream, int B, int H, int T, int hd, con
         check_matrix(V, ld, "V");
         check_matrix(O, ldo, "O");
         require(lse && !(reinterpret_cast<uintptr_t>(lse) & 15), "attention: lse must be 16-byte aligned");
-        const bool split = split_tiles(B, H, T, SPLIT_FORWARD);
+        const bool split = forward_splits(B, H, T);
         const CausalGrid grid = causal_grid(B, H, T, split ? 32 : 128);
         hipLaunchKernelGGL(split ? attn_fwd_split_kernel : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
                            ld, O, ldo, lse, T, grid, scale * LOG2E);
@@ -936,7 +1009,8 @@ void attn_bwd_check(int B, int H, int T, int hd, const uint16_t *Q, const uint16
 void attn_bwd_launch(hipStream_t stream, int B, int H, int T, const uint16_t *Q, const uint16_t *K,
                      const uint16_t *V, int ld, const uint16_t *O, int ldo, const float *lse, const uint16_t *dO,
                      int lddo, uint16_t *dQ, uint16_t *dK, uint16_t *dV, int lddq, float scale, float *rows) {
-    if (split_tiles(B, H, T, SPLIT_BACKWARD)) {
+    const Backward way = backward_way(B, H, T);
+    if (way == BACKWARD_SPLIT) {
         const CausalGrid grid = causal_grid(B, H, T, 32);
         hipLaunchKernelGGL(attn_bwd_split_kernel, dim3(2 * grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo,
                            lse, dQ, dK, dV, lddq, T, grid, scale);
@@ -945,6 +1019,13 @@ void attn_bwd_launch(hipStream_t stream, int B, int H, int T, const uint16_t *Q,
     }
     float *delta = rows, *lse2 = delta + size_t(B) * H * T;
     const CausalGrid grid = causal_grid(B, H, T, 128);
+    if (way == BACKWARD_BOTH) {
+        hipLaunchKernelGGL(attn_delta_kernel, dim3(B * H * (T / 32)), dim3(256), 0, stream, dO, lddo, O, ldo, lse, lse2, delta, H, T);
+        hipLaunchKernelGGL(attn_bwd_both_kernel, dim3(2 * grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo,
+                           lse, lse2, delta, dQ, dK, dV, lddq, T, grid, scale);
+        check_hip(hipGetLastError(), "attention backward launch: ");
+        return;
+    }
     hipLaunchKernelGGL(attn_bwd_dq_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, O, ldo, lse, lse2,
                        delta, dQ, lddq, T, grid, scale);
     hipLaunchKernelGGL(attn_bwd_dkdv_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, dO, lddo, lse2, delta, dK,
