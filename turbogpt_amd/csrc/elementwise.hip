@@ -4,6 +4,7 @@
 // with 16-byte accesses; reductions use a fixed order (no atomics), so results are reproducible.
 #include "common.h"
 #include "optimizer.h"
+#include "step.h"
 #include "../../include/tgk_kernels.h"
 
 namespace {
@@ -36,6 +37,17 @@ TG_DEVICE void join8(const uint16_t *hi, const uint16_t *lo, float (&f)[8]) {
     join8(*reinterpret_cast<const u32x4 *>(hi), *reinterpret_cast<const u32x4 *>(lo), f);
 }
 // ---- embedding ------------------------------------------------------------------------------
+// out[row][c .. c+7] = table[token] + positions[row % T]
+TG_DEVICE void embed_chunk(int token, int row, int c, const bf16_t *__restrict__ table, const bf16_t *__restrict__ positions,
+                           bf16_t *__restrict__ out, int T, int D) {
+    float a[8], b[8];
+    unpack8(*reinterpret_cast<const u32x4 *>(table + size_t(token) * D + c), a);
+    unpack8(*reinterpret_cast<const u32x4 *>(positions + size_t(row % T) * D + c), b);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        a[k] += b[k];
+    *reinterpret_cast<u32x4 *>(out + size_t(row) * D + c) = pack8(a);
+}
 __global__ __launch_bounds__(256) void embed_fwd_kernel(const uint8_t *__restrict__ x,
                                                         const bf16_t *__restrict__ table,
                                                         const bf16_t *__restrict__ positions,
@@ -45,13 +57,7 @@ __global__ __launch_bounds__(256) void embed_fwd_kernel(const uint8_t *__restric
     const size_t total = size_t(rows) * chunks;
     for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
         const int row = int(i / chunks), c = int(i % chunks) * 8;
-        float a[8], b[8];
-        unpack8(*reinterpret_cast<const u32x4 *>(table + size_t(x[row]) * D + c), a);
-        unpack8(*reinterpret_cast<const u32x4 *>(positions + size_t(row % T) * D + c), b);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            a[k] += b[k];
-        *reinterpret_cast<u32x4 *>(out + size_t(row) * D + c) = pack8(a);
+        embed_chunk(x[row], row, c, table, positions, out, T, D);
     }
 }
 
@@ -89,10 +95,10 @@ __global__ __launch_bounds__(256) void embed_bwd_fold_kernel(const float *__rest
     dtable[i] = accumulate ? dtable[i] + sum : sum;
 }
 // onehot[t][v] = (x[t] == v) in bf16; one thread writes 8 columns
-__global__ __launch_bounds__(256) void onehot_kernel(const uint8_t *__restrict__ x, bf16_t *__restrict__ onehot,
-                                                     int rows) {
+// a block's share of each: `block` of `blocks`
+TG_DEVICE void onehot_share(int block, int blocks, const uint8_t *__restrict__ x, bf16_t *__restrict__ onehot, int rows) {
     const size_t total = size_t(rows) * 32;
-    for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
+    for (size_t i = block * size_t(256) + threadIdx.x; i < total; i += size_t(blocks) * 256) {
         const int t = int(i >> 5), c0 = int(i & 31) * 8, hot = int(x[t]) - c0;
         u32x4 v = {0, 0, 0, 0};
         if (hot >= 0 && hot < 8)
@@ -101,16 +107,22 @@ __global__ __launch_bounds__(256) void onehot_kernel(const uint8_t *__restrict__
     }
 }
 // dPositions[p][c] = sum over sequences b of dh[b*T + p][c]
-__global__ __launch_bounds__(256) void embed_bwd_positions_kernel(const bf16_t *__restrict__ dh,
-                                                                  float *__restrict__ dpos, int B, int T,
-                                                                  int D, int accumulate) {
+TG_DEVICE void positions_share(int block, int blocks, const bf16_t *__restrict__ dh, float *__restrict__ dpos, int B, int T, int D,
+                               int accumulate) {
     const size_t total = size_t(T) * D;
-    for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
+    for (size_t i = block * size_t(256) + threadIdx.x; i < total; i += size_t(blocks) * 256) {
         float sum = 0.f;
         for (int b = 0; b < B; ++b)
             sum += bf16_to_float(dh[size_t(b) * total + i]);
         dpos[i] = accumulate ? dpos[i] + sum : sum;
     }
+}
+__global__ __launch_bounds__(256) void onehot_kernel(const uint8_t *__restrict__ x, bf16_t *__restrict__ onehot, int rows) {
+    onehot_share(blockIdx.x, gridDim.x, x, onehot, rows);
+}
+__global__ __launch_bounds__(256) void embed_bwd_positions_kernel(const bf16_t *__restrict__ dh, float *__restrict__ dpos, int B,
+                                                                  int T, int D, int accumulate) {
+    positions_share(blockIdx.x, gridDim.x, dh, dpos, B, T, D, accumulate);
 }
 
 // ---- LayerNorm --------------------------------------------------------------------------------
@@ -385,13 +397,11 @@ __global__ __launch_bounds__(256) void layernorm_bwd_reduce_kernel(const float *
 struct LayerNormFoldTarget {
     float *dgamma, *dbeta;
 };
-__global__ __launch_bounds__(256) void layernorm_bwd_fold_batch_kernel(const float *__restrict__ partial,
-                                                                       size_t job_stride, int blocks, int D,
-                                                                       const LayerNormFoldTarget *__restrict__ targets,
-                                                                       int accumulate) {
-    __shared__ float part[16][17];
-    const float *mine = partial + size_t(blockIdx.y) * job_stride;
-    const int col = threadIdx.x & 15, phase = threadIdx.x >> 4, i = blockIdx.x * 16 + col;
+TG_DEVICE void layernorm_fold_columns(float (&part)[16][17], int group, int job, const float *__restrict__ partial,
+                                      size_t job_stride, int blocks, int D, const LayerNormFoldTarget *__restrict__ targets,
+                                      int accumulate) { // columns 16 * group .. +15
+    const float *mine = partial + size_t(job) * job_stride;
+    const int col = threadIdx.x & 15, phase = threadIdx.x >> 4, i = group * 16 + col;
     const size_t row_stride = size_t(2) * D;
     float s[8];
 #pragma unroll
@@ -412,10 +422,18 @@ __global__ __launch_bounds__(256) void layernorm_bwd_fold_batch_kernel(const flo
 #pragma unroll
         for (int p = 0; p < 16; ++p)
             sum += part[p][col];
-        const LayerNormFoldTarget t = targets[blockIdx.y];
+        const LayerNormFoldTarget t = targets[job];
         float *out = i < D ? t.dgamma + i : t.dbeta + (i - D);
         *out = accumulate ? *out + sum : sum;
     }
+}
+
+__global__ __launch_bounds__(256) void layernorm_bwd_fold_batch_kernel(const float *__restrict__ partial, size_t job_stride,
+                                                                       int blocks, int D,
+                                                                       const LayerNormFoldTarget *__restrict__ targets,
+                                                                       int accumulate) {
+    __shared__ float part[16][17];
+    layernorm_fold_columns(part, blockIdx.x, blockIdx.y, partial, job_stride, blocks, D, targets, accumulate);
 }
 
 // ---- cross-entropy over 256 byte classes ------------------------------------------------------
@@ -575,13 +593,30 @@ __global__ __launch_bounds__(256) void sample_batch_kernel(const uint8_t *__rest
         y[size_t(b) * context + p] = data[e - context + p + 1];
     }
 }
+// The same with the embedding of the tokens drawn: a thread finds its token itself.  One launch instead of two that take 4 us
+// each where the batch is small.
+__global__ __launch_bounds__(256) void sample_embed_kernel(const uint8_t *__restrict__ data, int64_t size, uint64_t seed,
+                                                           uint64_t step, int batch, int context, int D, uint8_t *__restrict__ x,
+                                                           uint8_t *__restrict__ y, const bf16_t *__restrict__ table,
+                                                           const bf16_t *__restrict__ positions, bf16_t *__restrict__ out) {
+    const int chunks = D >> 3;
+    const int64_t low = context > 8 ? context : 8;
+    const size_t total = size_t(batch) * context * chunks;
+    for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
+        const int row = int(i / chunks), c = int(i % chunks) * 8, b = row / context, p = row - b * context;
+        const int64_t e = low + int64_t(hash_u64(seed + step * uint64_t(batch) + uint64_t(b)) % uint64_t(size - low));
+        const int token = data[e - context + p];
+        embed_chunk(token, row, c, table, positions, out, context, D);
+        if (c == 0) {
+            x[row] = uint8_t(token);
+            y[row] = data[e - context + p + 1];
+        }
+    }
+}
 // cuda/trainer.cuh:79-100: mean over the batch per position, accumulated in double: a block a position, every thread
 // each 256th sequence (a wave a position took 11 us for the width-16 network's 2560 sequences of 4), a fixed tree on top
-__global__ __launch_bounds__(256) void position_means_kernel(const float *__restrict__ token_loss,
-                                                             int batch, int context,
-                                                             float *__restrict__ out) {
-    __shared__ double waves[4];
-    const int p = blockIdx.x;
+TG_DEVICE void position_mean(double (&waves)[4], int p, const float *__restrict__ token_loss, int batch, int context,
+                             float *__restrict__ out) {
     double sum = 0;
 #pragma unroll 4
     for (int b = threadIdx.x; b < batch; b += 256)
@@ -594,6 +629,30 @@ __global__ __launch_bounds__(256) void position_means_kernel(const float *__rest
     __syncthreads();
     if (threadIdx.x == 0)
         out[p] = float(((waves[0] + waves[1]) + (waves[2] + waves[3])) / batch);
+}
+__global__ __launch_bounds__(256) void position_means_kernel(const float *__restrict__ token_loss, int batch, int context,
+                                                             float *__restrict__ out) {
+    __shared__ double waves[4];
+    position_mean(waves, blockIdx.x, token_loss, batch, context, out);
+}
+
+// What is left of a backward pass behind its row kernels, none of it waiting for another part: the LayerNorm gradients'
+// folds, the one-hot matrix, the position gradients and (means not NULL) the batch's losses.  Each alone is a launch of 3.5
+// to 4.5 us that leaves most units idle.
+__global__ __launch_bounds__(256) void backward_rest_kernel(const BackwardRest r, int folds, int onehots, int positions) {
+    __shared__ float part[16][17];
+    __shared__ double waves[4];
+    int block = blockIdx.x;
+    if (block < folds) {
+        const int groups = 2 * r.D / 16;
+        return layernorm_fold_columns(part, block % groups, block / groups, r.partials, r.partials_stride, r.partial_rows, r.D,
+                                      static_cast<const LayerNormFoldTarget *>(r.targets), 0);
+    }
+    if ((block -= folds) < onehots)
+        return onehot_share(block, onehots, r.tokens, r.onehot, r.B * r.T);
+    if ((block -= onehots) < positions)
+        return positions_share(block, positions, r.dh, r.dpositions, r.B, r.T, r.D, 0);
+    position_mean(waves, block - positions, r.token_losses, r.B, r.T, r.means);
 }
 
 // ---- batched bf16 transposes ------------------------------------------------------------------
@@ -944,5 +1003,36 @@ extern "C" int tgk_transpose_batch(hipStream_t stream, const uint16_t *in, uint1
         hipLaunchKernelGGL(transpose_batch_kernel, dim3(total_tiles), dim3(256), 0, stream, in, out,
                            static_cast<const TransposeJob *>(jobs), count);
         check_hip(hipGetLastError(), "transpose_batch launch: ");
+    });
+}
+
+int sample_embed(hipStream_t stream, const uint8_t *data, int64_t size, uint64_t seed, uint64_t step, int batch, int context,
+                 int D, uint8_t *x, uint8_t *y, const uint16_t *table, const uint16_t *positions, uint16_t *out) {
+    return guarded([&] {
+        require(data && x && y, "sample_embed: missing operand");
+        require(batch > 0 && context > 0 && D > 0 && D % 8 == 0, "sample_embed: empty batch, or D not a multiple of 8");
+        require(size > (context > 8 ? context : 8), "sample_embed: dataset shorter than one window");
+        aligned(table, "sample_embed: table");
+        aligned(positions, "sample_embed: positions");
+        aligned(out, "sample_embed: out");
+        hipLaunchKernelGGL(sample_embed_kernel, dim3(grid_for(size_t(batch) * context * D / 8, 256)), dim3(256), 0, stream, data,
+                           size, seed, step, batch, context, D, x, y, table, positions, out);
+        check_hip(hipGetLastError(), "sample_embed launch: ");
+    });
+}
+
+int backward_rest(hipStream_t stream, BackwardRest r) {
+    return guarded([&] {
+        require(r.B > 0 && r.T > 0 && r.D > 0 && r.D % 64 == 0 && r.layernorms > 0, "backward_rest: bad shape");
+        require(r.tokens && r.dh && r.dpositions && r.partials && r.targets, "backward_rest: missing operand");
+        require(r.partials_stride * sizeof(float) >= tgk_layernorm_bwd_workspace(r.B * r.T, r.D), "backward_rest: partials overlap");
+        require(!r.means || r.token_losses, "backward_rest: missing losses");
+        aligned(r.onehot, "backward_rest: onehot");
+        r.partial_rows = layernorm_bwd_blocks(r.B * r.T);
+        const int folds = 2 * r.D / 16 * r.layernorms, onehots = grid_for(size_t(r.B) * r.T * 32, 256);
+        const int positions = grid_for(size_t(r.T) * r.D, 256);
+        hipLaunchKernelGGL(backward_rest_kernel, dim3(folds + onehots + positions + (r.means ? r.T : 0)), dim3(256), 0, stream, r,
+                           folds, onehots, positions);
+        check_hip(hipGetLastError(), "backward_rest launch: ");
     });
 }

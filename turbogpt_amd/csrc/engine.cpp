@@ -6,6 +6,7 @@
 #include "common.h"
 #include "gemm_list.h"
 #include "readback.h"
+#include "step.h"
 #include "width16.h"
 #include "../../include/tg_model.h"
 #include "../../include/tgk_kernels.h"
@@ -229,7 +230,9 @@ struct Engine {
     // On the slot's stream, with one weight version, from the slot's first `batch` sequences.  last_position: one
     // sequence, and only the logits of its last position are wanted (`logits_out` receives that row): behind the
     // attention of the last block nothing but the last tile of rows is computed.
-    void forward(Slot &s, const Version &v, bool with_gradient, float *logits_out, int batch, bool last_position = false) {
+    // embedded: the slot's tokens have already been drawn and embedded (sample_embed).
+    void forward(Slot &s, const Version &v, bool with_gradient, float *logits_out, int batch, bool last_position = false,
+                 bool embedded = false) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
         const uint8_t *tokens_in = s.input, *targets = s.target;
@@ -248,7 +251,8 @@ struct Engine {
         const int d = config.d_model, F = config.ffn, V = config.vocab, T = c.context;
         const float scale = 1.0f / std::sqrt(float(d / config.heads));
         int M = batch * T;
-        OP(TG_CLASS_OTHER, tgk_embed_fwd(stream, M, T, d, tokens_in, w(layout.embedding), w(layout.positions), x[0]));
+        if (!embedded)
+            OP(TG_CLASS_OTHER, tgk_embed_fwd(stream, M, T, d, tokens_in, w(layout.embedding), w(layout.positions), x[0]));
         for (int l = 0; l < c.depth; ++l) {
             const TgLayerParameters &p = layout.layers[l];
             const LayerBuffers &b = layers[l];
@@ -277,8 +281,9 @@ struct Engine {
                              1.0f / float(M), with_gradient ? 1 : 0));
     }
 
-    // cuda/model.cuh:61-99.  Every element of `gradient` is overwritten: nothing needs zeroing.
-    void backward(Slot &s, const Version &v) {
+    // cuda/model.cuh:61-99.  Every element of `gradient` is overwritten: nothing needs zeroing.  means: where the batch's
+    // losses per position go.
+    void backward(Slot &s, const Version &v, float *means) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
         const uint8_t *tokens_in = s.input;
@@ -287,6 +292,7 @@ struct Engine {
         if (width16) {
             OP(TG_CLASS_OTHER, tgk_w16_backward(stream, c.depth, c.batch, c.context, v.hi, v.lo, tokens_in, workspace,
                                                 gradient));
+            OP(TG_CLASS_OTHER, tgk_position_means(stream, s.token_losses, c.batch, c.context, means));
             return;
         }
         const auto w = [&](int64_t offset) { return v.hi + offset; };
@@ -324,8 +330,9 @@ struct Engine {
             OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, gqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
             OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, mid, s.g_x[l]));
         }
-        OP(TG_CLASS_LAYERNORM_BWD, tgk_layernorm_bwd_fold(stream, M, d, 2 * c.depth + 1, s.ln_partials, ln_stride, s.ln_targets, 0));
-        OP(TG_CLASS_OTHER, tgk_embed_bwd_onehot(stream, c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions, 0));
+        OP(TG_CLASS_OTHER, backward_rest(stream, {c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions,
+                                                  reinterpret_cast<const float *>(s.ln_partials), ln_stride / sizeof(float),
+                                                  2 * c.depth + 1, 0, s.ln_targets, s.token_losses, means}));
         const bool norms = c.clip > 0;
         {
             Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
@@ -382,10 +389,10 @@ struct Engine {
                          s.token_losses, history_row, s.gradient, s.norms);
             return;
         }
-        OP(TG_CLASS_OTHER, tgk_sample_batch(stream, data, data_size, c.seed, at, c.batch, c.context, s.input, s.target));
-        forward(s, v, true, nullptr, c.batch);
-        OP(TG_CLASS_OTHER, tgk_position_means(stream, s.token_losses, c.batch, c.context, history_row));
-        backward(s, v);
+        OP(TG_CLASS_OTHER, sample_embed(stream, data, data_size, c.seed, at, c.batch, c.context, config.d_model, s.input, s.target,
+                                        v.hi + layout.embedding, v.hi + layout.positions, s.x[0]));
+        forward(s, v, true, nullptr, c.batch, false, true);
+        backward(s, v, history_row);
     }
     // One training step.  Synchronous engine: everything in order on the one stream, weights updated in place
     // (cuda/trainer.cuh:109-124).  inflight = K (cuda/pipeline.cuh:40-126 as streams and events): batch `at` and its
@@ -945,11 +952,12 @@ TG_API int tg_batch(Engine *e, const uint8_t *x, const uint8_t *y, float *logits
         check_hip(hipMemcpyAsync(slot.input, x, M, hipMemcpyHostToDevice, slot.stream));
         check_hip(hipMemcpyAsync(slot.target, y, M, hipMemcpyHostToDevice, slot.stream));
         e->forward(slot, e->current(), gradient != nullptr, e->logits_f32, e->config.base.batch);
-        if (gradient)
-            e->backward(slot, e->current());
-        // per-position means in double (cuda/runtime.cu:279-290)
+        // with per-position means in double (cuda/runtime.cu:279-290)
         const Config &c = e->config.base;
-        ok(tgk_position_means(slot.stream, slot.token_losses, c.batch, c.context, e->batch_means));
+        if (gradient)
+            e->backward(slot, e->current(), e->batch_means);
+        else
+            ok(tgk_position_means(slot.stream, slot.token_losses, c.batch, c.context, e->batch_means));
         check_hip(hipStreamSynchronize(slot.stream));
         std::vector<ReadbackPiece> pieces = {{logits, M * V * 4, e->logits_f32}, {loss, size_t(c.context) * 4, e->batch_means}};
         if (gradient)
