@@ -4,7 +4,7 @@
 // cuda/model.cuh:20 and :86-88); the packed [token][q|k|v] buffer and the [token][head*64+d]
 // output keep the reference's layout (cuda/attention.cuh:38-39,68), so no permutes are needed.
 //
-// All three kernels work on 32x32 MFMA tiles (v_mfma_f32_32x32x16_bf16) and are written in the
+// All kernels work on 32x32 MFMA tiles (v_mfma_f32_32x32x16_bf16) and are written in the
 // "transposed" form: the score tile is produced as S^T[key][query] so that one lane owns one
 // query row - row maxima / sums / rescales are per-lane scalars - and the fp32 accumulator
 // registers of S^T can be fed back, converted to bf16, as the B operand of the next product with
@@ -1053,8 +1053,8 @@ extern "C" int tgk_attn_bwd(hipStream_t stream, int B, int H, int T, int hd, con
 // The two row vectors the kernels exchange (delta and the base-2 log-sum-exp, B*H*T floats each) live in
 // a device array of this library instead of a caller's workspace.  Every GPU the library runs on holds
 // its own copy of the array at its own address; the address is looked up once per device, with that
-// device current, and only that address - never the array's name - is handed to kernels.  The dQ kernel
-// overwrites every row the dK/dV kernel reads, so nothing has to be cleared between calls.
+// device current, and only that address - never the array's name - is handed to kernels.  Every
+// call writes the rows that it reads (dQ or attn_delta_kernel before dK/dV), so nothing has to be cleared between calls.
 namespace {
 constexpr size_t STATIC_BWD_ROWS = size_t(1) << 20; // B*H*T of one call: 8 MiB of device memory per GPU
 static __device__ __align__(256) float scratch[2 * STATIC_BWD_ROWS];

@@ -1634,7 +1634,6 @@ __global__ __launch_bounds__(256, 1) void wgrad_list_kernel(const WgradList w) {
             w.sumsq[blockIdx.x * 4 + wave] = squares;
     }
 }
-// Sums the pieces of the split tiles, in token order, into the gradient.  Eight blocks per tile.
 // The same list on ordinary tiles, each summed over all tokens by one block: where 256 x 256 tiles would not fill the
 // compute units or do not fit the widths, and for a single gradient (plan_wgrad).  Block b of g takes tiles b, b + g, ...; a
 // list is not cut along the tokens, so nothing is folded.  What bounds it is a stage's latency on a unit with one tile and the
@@ -1693,6 +1692,7 @@ __global__ __launch_bounds__(256 * GROUPS) void wgrad_tiles_kernel(const WgradTi
             w.sumsq[blockIdx.x] = (waves[0] + waves[1]) + (waves[2] + waves[3]);
     }
 }
+// Sums the pieces of the split tiles, in token order, into the gradient.  Eight blocks per tile.
 template <int BN>
 __global__ __launch_bounds__(256) void wgrad_list_fold_kernel(const WgradList w, int first_tile, int first_sumsq) {
     constexpr int BM = 256, QUADS = BM * BN / 4 / 8 / 256; // float4 per thread
