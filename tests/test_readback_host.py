@@ -1,0 +1,62 @@
+"""What csrc/readback.hip asks of the HIP runtime and what it does when a call fails, on the host alone: the file is compiled
+without its device code, with a model of the calls that it makes (fake_hip.cpp)."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from turbogpt_amd import build
+
+ROOT = Path(__file__).resolve().parents[1]
+CHUNK = 2 << 20
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("readback")
+    library = folder / "libreadback.so"
+    subprocess.run([build.HIPCC, "-x", "hip", "--offload-host-only", "-fuse-cuid=none", "-O1", "-std=c++17", "-fPIC", "-c",
+                    str(ROOT / "tests/fake_hip.cpp"), "-o", str(folder / "readback.o")], check=True, capture_output=True)
+    subprocess.run(["g++", "-shared", "-pthread", "-o", str(library), str(folder / "readback.o")], check=True, capture_output=True)
+    lib = C.CDLL(str(library))
+    lib.fake_stream.restype = lib.readback_open.restype = C.c_void_p
+    lib.readback_error.restype = C.c_char_p
+    lib.fake_queued.argtypes = lib.readback_close.argtypes = [C.c_void_p]
+    lib.readback_fetch.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int] + [C.c_void_p] * 4
+    return lib
+
+
+class Engine:
+    """What an engine has of it: the staging memory, a device and a stream of that device."""
+
+    def __init__(self, lib, device=0):
+        self.lib, self.device = lib, device
+        self.stream, self.handle = lib.fake_stream(device), lib.readback_open(device)
+
+    def fetch(self, *sizes, seed=0, join=False):
+        """-> whether the call succeeded and whether every byte arrived"""
+        rng = np.random.default_rng(seed)
+        sources = [rng.integers(0, 256, size, dtype=np.uint8) for size in sizes]
+        results = [np.full(size, 0xaa, np.uint8) for size in sizes]
+        count = len(sizes)
+        halves = [(s.view(np.uint32) >> 16).astype(np.uint16) for s in sources], [s.view(np.uint32).astype(np.uint16) for s in sources]
+        address = lambda arrays: (C.c_void_p * count)(*[a.ctypes.data for a in arrays])
+        status = self.lib.readback_fetch(self.handle, self.stream, self.device, count, address(results), (C.c_size_t * count)(*sizes),
+                                         address(halves[0] if join else sources),
+                                         address(halves[1]) if join else (C.c_void_p * count)())
+        return status == 0, all(np.array_equal(a, b) for a, b in zip(results, sources))
+
+    def close(self):
+        self.lib.readback_close(self.handle)
+
+
+@pytest.mark.parametrize("sizes", [(16,), (CHUNK,), (CHUNK + 16,), (65536, 16, 86592), (5 * CHUNK - 32,), (40 * CHUNK + 48, 16)])
+@pytest.mark.parametrize("join", [False, True])
+def test_the_host_reads_what_the_kernels_wrote(host, sizes, join):
+    engine = Engine(host)
+    for seed in range(3):  # the buffers hold an earlier result from the second on
+        assert engine.fetch(*sizes, seed=seed, join=join) == (True, True)
+    engine.close()
+    assert host.fake_pinned() == 0 and host.fake_events() == 0
