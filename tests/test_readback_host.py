@@ -60,3 +60,15 @@ def test_the_host_reads_what_the_kernels_wrote(host, sizes, join):
         assert engine.fetch(*sizes, seed=seed, join=join) == (True, True)
     engine.close()
     assert host.fake_pinned() == 0 and host.fake_events() == 0
+
+
+@pytest.mark.parametrize("call", ["hipHostMalloc", "hipHostGetDevicePointer", "hipEventCreateWithFlags"])
+@pytest.mark.parametrize("at", [1, 2, 4])
+def test_a_buffer_that_could_not_be_made_is_not_used(host, call, at):
+    engine = Engine(host)
+    host.fake_fail(call.encode(), at)
+    assert not engine.fetch(4 * CHUNK)[0]
+    assert host.fake_pinned() == host.fake_events() == at - 1  # what was whole stays, the failed one is given back
+    assert engine.fetch(4 * CHUNK, seed=1) == (True, True)
+    engine.close()
+    assert host.fake_pinned() == 0 and host.fake_events() == 0

@@ -32,6 +32,7 @@ class Readback {
         void *pinned = nullptr, *mapped = nullptr; // the same memory, by host and by device address
         hipEvent_t written = nullptr;
     };
+    static void give_back(const Buffer &buffer);
     void reserve(size_t count);
     std::mutex busy;
     std::vector<Buffer> buffers; // 2 MiB each, as many as the largest result so far could use: at most 16

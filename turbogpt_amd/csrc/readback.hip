@@ -59,22 +59,30 @@ std::shared_ptr<Readback> Readback::shared() {
         living = staging = std::shared_ptr<Readback>(new Readback);
     return staging;
 }
+void Readback::give_back(const Buffer &buffer) {
+    if (buffer.written)
+        (void)hipEventDestroy(buffer.written);
+    if (buffer.pinned)
+        (void)hipHostFree(buffer.pinned);
+}
 Readback::~Readback() {
-    for (Buffer &buffer : buffers) {
-        if (buffer.written)
-            (void)hipEventDestroy(buffer.written);
-        if (buffer.pinned)
-            (void)hipHostFree(buffer.pinned);
-    }
+    for (const Buffer &buffer : buffers)
+        give_back(buffer);
 }
 void Readback::reserve(size_t count) {
-    while (buffers.size() < count) {
-        buffers.emplace_back();
-        Buffer &buffer = buffers.back();
-        check_hip(hipHostMalloc(&buffer.pinned, CHUNK, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent),
-                  "pinned staging: ");
-        check_hip(hipHostGetDevicePointer(&buffer.mapped, buffer.pinned, 0), "pinned staging: ");
-        check_hip(hipEventCreateWithFlags(&buffer.written, hipEventDisableTiming | hipEventReleaseToSystem), "readback event: ");
+    buffers.reserve(count);
+    while (buffers.size() < count) { // a buffer joins the others whole or not at all
+        Buffer buffer;
+        try {
+            check_hip(hipHostMalloc(&buffer.pinned, CHUNK, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent),
+                      "pinned staging: ");
+            check_hip(hipHostGetDevicePointer(&buffer.mapped, buffer.pinned, 0), "pinned staging: ");
+            check_hip(hipEventCreateWithFlags(&buffer.written, hipEventDisableTiming | hipEventReleaseToSystem), "readback event: ");
+        } catch (...) {
+            give_back(buffer);
+            throw;
+        }
+        buffers.push_back(buffer);
     }
 }
 
