@@ -10,6 +10,7 @@
 #include <deque>
 #include <functional>
 #include <map>
+#include <utility>
 
 namespace {
 
@@ -43,6 +44,7 @@ std::map<std::string, int> failing; // call -> fails at this call from now (1 = 
 int events = 0;
 thread_local int current_device = 0;
 thread_local hipStream_t launch_stream;
+thread_local hipError_t last_error = hipSuccess;
 
 bool fails(const char *call) {
     auto at = failing.find(call);
@@ -77,7 +79,7 @@ thread_local std::string tg_last_error;
 
 extern "C" {
 
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return std::exchange(last_error, hipSuccess); }
 const char *hipGetErrorString(hipError_t error) { return error == hipErrorInvalidHandle ? "invalid handle" : "injected failure"; }
 hipError_t hipSetDevice(int device) {
     current_device = device;
@@ -154,7 +156,7 @@ hipError_t hipStreamSynchronize(hipStream_t stream) {
 hipError_t hipLaunchKernel(const void *function, dim3, dim3, void **args, size_t, hipStream_t stream) {
     const Lock lock(guard);
     if (fails("hipLaunchKernel"))
-        return hipErrorLaunchFailure;
+        return last_error = hipErrorLaunchFailure;
     const bool join = kernels.at(function).find("join") != std::string::npos;
     std::vector<uint64_t> values; // they live on the launching thread's stack
     for (int i = 0; i < (join ? 4 : 3); ++i)

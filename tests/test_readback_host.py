@@ -72,3 +72,18 @@ def test_a_buffer_that_could_not_be_made_is_not_used(host, call, at):
     assert engine.fetch(4 * CHUNK, seed=1) == (True, True)
     engine.close()
     assert host.fake_pinned() == 0 and host.fake_events() == 0
+
+
+@pytest.mark.parametrize("size", [16, CHUNK + 16, 2 * CHUNK, 3 * CHUNK, 20 * CHUNK])
+@pytest.mark.parametrize("call,at", [("hipEventRecord", 1), ("hipEventRecord", 2), ("hipEventSynchronize", 1), ("hipLaunchKernel", 2)])
+def test_a_failed_result_leaves_no_kernel_writing_to_the_shared_buffers(host, size, call, at):
+    if at == 2 and size <= CHUNK:
+        return  # the call is made once
+    first, second = Engine(host), Engine(host)
+    host.fake_fail(call.encode(), at)
+    assert not first.fetch(size, seed=2)[0]
+    assert b"injected" in host.readback_error()
+    assert host.fake_queued(first.stream) == 0
+    assert second.fetch(size, seed=3) == (True, True)
+    first.close()
+    second.close()

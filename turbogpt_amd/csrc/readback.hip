@@ -121,11 +121,8 @@ void Readback::fetch(hipStream_t stream, int device, const std::vector<ReadbackP
             std::memcpy(static_cast<uint8_t *>(c.piece->host) + c.offset, buffer.pinned, c.bytes);
         }
     };
-    if (lanes <= 1) { // a small result: this thread alone
-        if (lanes)
-            lane(0);
+    if (!lanes)
         return;
-    }
     std::vector<std::exception_ptr> failures(lanes);
     std::vector<std::thread> threads;
     const auto guarded_lane = [&](size_t l) {
@@ -143,7 +140,7 @@ void Readback::fetch(hipStream_t stream, int device, const std::vector<ReadbackP
         for (size_t l = threads.size() + 1; l < lanes; ++l)
             guarded_lane(l);
     }
-    guarded_lane(0);
+    guarded_lane(0); // this thread; a small result has no other
     for (std::thread &thread : threads)
         thread.join();
     for (const std::exception_ptr &failure : failures)
