@@ -189,7 +189,7 @@ int fake_events() { return events; }
 
 void *readback_open(int device) {
     current_device = device;
-    return new std::shared_ptr<Readback>(Readback::shared());
+    return new std::shared_ptr<Readback>(Readback::shared(device));
 }
 void readback_close(void *handle) { delete static_cast<std::shared_ptr<Readback> *>(handle); }
 // plain copies of `count` pieces, or joins where lo[i] is given; 0, or -1 with the message in readback_error()
@@ -200,7 +200,7 @@ int readback_fetch(void *handle, void *stream, int device, int count, void **hos
         for (int i = 0; i < count; ++i)
             pieces.push_back({host[i], bytes[i], lo[i] ? nullptr : source[i], static_cast<uint16_t *>(lo[i] ? source[i] : nullptr),
                               static_cast<uint16_t *>(lo[i])});
-        (*static_cast<std::shared_ptr<Readback> *>(handle))->fetch(static_cast<hipStream_t>(stream), device, pieces);
+        (*static_cast<std::shared_ptr<Readback> *>(handle))->fetch(static_cast<hipStream_t>(stream), pieces);
     });
 }
 const char *readback_error() { return tg_last_error.c_str(); }

@@ -87,3 +87,18 @@ def test_a_failed_result_leaves_no_kernel_writing_to_the_shared_buffers(host, si
     assert second.fetch(size, seed=3) == (True, True)
     first.close()
     second.close()
+
+
+@pytest.mark.parametrize("size", [16, 3 * CHUNK, 40 * CHUNK])
+def test_engines_on_two_devices(host, size):
+    engines = [Engine(host, 0), Engine(host, 1), Engine(host, 0)]
+    for seed in range(2):
+        for engine in engines:
+            assert engine.fetch(size, seed=seed) == (True, True), host.readback_error()
+    held = host.fake_pinned()
+    engines.pop(0).close()  # the other engine of device 0 goes on with the staging memory of the first
+    assert host.fake_pinned() == held
+    for engine in engines:
+        assert engine.fetch(size, seed=5) == (True, True), host.readback_error()
+        engine.close()
+    assert host.fake_pinned() == host.fake_events() == 0

@@ -123,7 +123,7 @@ struct Engine {
     float *logits_f32 = nullptr;
     size_t workspace_bytes = 0;
 
-    std::shared_ptr<Readback> readback = Readback::shared();
+    std::shared_ptr<Readback> readback; // of the engine's device
     float *batch_means = nullptr; // [context]: the per-position losses of a fixed batch
 
     std::vector<StepRates> schedule;
@@ -191,7 +191,7 @@ struct Engine {
         check_hip(hipMemcpyAsync(device, host, n * sizeof(T), hipMemcpyHostToDevice, stream));
     }
     // results to the caller's memory, behind everything on the engine's stream; returns when they are there
-    void download(const std::vector<ReadbackPiece> &pieces) { readback->fetch(stream, config.base.device, pieces); }
+    void download(const std::vector<ReadbackPiece> &pieces) { readback->fetch(stream, pieces); }
     ~Engine() { // cuda/engine_internal.h:28-37
         (void)hipSetDevice(config.base.device);
         for (Slot &slot : slots)
@@ -449,9 +449,10 @@ void validate(const TgModelConfig &m) {
         throw std::runtime_error("ln_eps must be positive");
 }
 
-// Streams, events and the buffers every model kind needs per slot and per weight version.
+// Streams, events, staging memory and the buffers every model kind needs per slot and per weight version.
 void build_slots(Engine *e, int inflight, bool transposed_copies) {
     const size_t P = size_t(e->layout.count), M = size_t(e->tokens());
+    e->readback = Readback::shared(e->config.base.device);
     e->slots.resize(size_t(inflight));
     e->versions.resize(inflight > 1 ? size_t(inflight) + 1 : 1);
     for (Slot &slot : e->slots) {

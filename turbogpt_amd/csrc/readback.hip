@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstring>
 #include <exception>
+#include <map>
 #include <thread>
 
 namespace {
@@ -50,13 +51,14 @@ void enqueue(hipStream_t stream, const ReadbackPiece &piece, size_t offset, size
 
 } // namespace
 
-std::shared_ptr<Readback> Readback::shared() {
+std::shared_ptr<Readback> Readback::shared(int device) {
     static std::mutex guard;
-    static std::weak_ptr<Readback> living;
+    static std::map<int, std::weak_ptr<Readback>> living;
     const std::lock_guard<std::mutex> lock(guard);
-    std::shared_ptr<Readback> staging = living.lock();
+    std::weak_ptr<Readback> &place = living[device];
+    std::shared_ptr<Readback> staging = place.lock();
     if (!staging)
-        living = staging = std::shared_ptr<Readback>(new Readback);
+        place = staging = std::shared_ptr<Readback>(new Readback(device));
     return staging;
 }
 void Readback::give_back(const Buffer &buffer) {
@@ -86,7 +88,7 @@ void Readback::reserve(size_t count) {
     }
 }
 
-void Readback::fetch(hipStream_t stream, int device, const std::vector<ReadbackPiece> &pieces) {
+void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces) {
     struct Chunk {
         const ReadbackPiece *piece;
         size_t offset, bytes;
@@ -101,6 +103,7 @@ void Readback::fetch(hipStream_t stream, int device, const std::vector<ReadbackP
     const size_t lanes = std::min<size_t>(LANES, (chunks.size() + 1) / 2);
     const size_t depth = chunks.size() == 1 ? 1 : 2;
     const std::lock_guard<std::mutex> lock(busy);
+    check_hip(hipSetDevice(device)); // its events are made here
     reserve(lanes * depth);
     const auto lane = [&](size_t l) {
         const auto start = [&](size_t round) {
