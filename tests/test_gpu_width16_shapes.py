@@ -43,3 +43,27 @@ def test_against_the_checker(depth, context, batch):
     # a sequence's logits do not depend on its place or its company
     alone = run(depth, context, 1, flat, x[-1:], y[-1:])[0]
     np.testing.assert_array_equal(alone[0], logits[-1])
+
+
+def test_gates_far_below_zero():
+    """SiLU and its derivative vanish there, whatever the gate's size: -80 to -1.6e38, past the points where the sigmoid
+    leaves the normal range (-87.3) and becomes 0 (-88.7)."""
+    depth, context, batch = 2, 4, 12
+    flat = reference_style_weights(depth)
+    entries = w16.layout(depth)[0]
+    view = lambda name: flat[entries[name][0]:entries[name][0] + int(np.prod(entries[name][1]))].reshape(entries[name][1])
+    view("embedding")[:, 0] = 4  # it carries the residual stream: 3.9 in every normalised row
+    below = np.array([80, 87.5, 88, 89, 89.5, 100, 1e4, 1e20, 1e30, 1.6e38], np.float32)
+    for l in range(depth):
+        view(f"{l}.gate")[:4 * len(below):4] = 0
+        view(f"{l}.gate")[:4 * len(below):4, 0] = -below / 4
+    rng = np.random.default_rng(5)
+    x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
+    logits, _, gradient = run(depth, context, batch, flat, x, y)
+    with np.errstate(over="ignore"):
+        target, expected, _ = w16.Width16(depth, context, batch).batch(flat, x, y)
+    assert np.isfinite(target).all() and np.isfinite(expected).all()
+    assert relative(logits, target) < .005
+    for name, (offset, shape) in entries.items():
+        part = slice(offset, offset + int(np.prod(shape)))
+        assert relative(gradient[part], expected[part]) < .02, name

@@ -175,8 +175,10 @@ template <int D, int END, class Body> TG_DEVICE void up_to(Body &&body) { // D, 
         up_to<D + 1, END>(body);
 }
 // 1 / b and x / b = divide(x, b, 1 / b), correctly rounded while neither b nor the result leaves the normal range (compared
-// with the division over every mantissa of b and 262 million pairs: no difference): three instructions where the
-// division takes ten, and 140 of them stand in a wave's way at the head alone.
+// with the division over every mantissa of b and 262 million pairs: no difference): a Newton step on the hardware's
+// approximate reciprocal, and for the quotient a correction by its residual, both with fused multiply-adds (Markstein, IBM
+// Journal of Research and Development 34, 1990).  Three instructions where the division takes ten, and 140 of them stand in
+// a wave's way at the head alone.
 TG_DEVICE float reciprocal(float b) {
     const float r = __builtin_amdgcn_rcpf(b);
     return fmaf(fmaf(-b, r, 1.f), r, r);
@@ -185,8 +187,10 @@ TG_DEVICE float divide(float x, float b, float r) {
     const float q = x * r;
     return fmaf(fmaf(-q, b, x), r, q);
 }
+// 1 / (1 + e^-x) taken 2^24 times too large, where the reciprocal stays in the normal range down to e^-x = 2^128; beyond that
+// 2^-126 stands for it, which the last product rounds to 0.
 TG_DEVICE float sigmoid(float x) {
-    return reciprocal(fminf(1.f + expf(-x), 0x1p126f)); // below -87 it is 1e-38 instead of less
+    return reciprocal(fminf(fmaf(expf(-x), 0x1p-24f, 0x1p-24f), 0x1p126f)) * 0x1p-24f;
 }
 
 struct Model {
