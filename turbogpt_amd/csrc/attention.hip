@@ -207,6 +207,9 @@ TG_DEVICE void scores(const bf16_t *kt, const RowFragOffsets &krows, const bf16x
 }
 // forward: the scores of keys kv0 .. kv0 + 63 to probabilities under the running maximum m; l is this lane's half of
 // the keys only, the halves are joined at the end.  Returns what earlier sums have to be multiplied by.
+// ANY_TILE: the first tile seen need not be the row's first, so its scores may all be -inf (products that overflow) where
+// the row has others: they get probability 0 and the maximum stays -inf.
+template <bool ANY_TILE>
 TG_DEVICE float online_softmax(f32x16 (&s)[2], int kv0, int wave_q0, int qrow, int g, float c, float &m, float &l) {
     if (kv0 + 63 > wave_q0) { // diagonal tile: hide keys after the query
 #pragma unroll
@@ -224,13 +227,14 @@ TG_DEVICE float online_softmax(f32x16 (&s)[2], int kv0, int wave_q0, int qrow, i
             mx = fmaxf(mx, s[mt][r]);
     mx = halves_max(mx);
     const float m_new = fmaxf(m, mx * c);
-    const float alpha = exp2_fast(m - m_new);
+    const float shift = ANY_TILE && m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = exp2_fast(m - shift);
     float sum = 0.f;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float p = exp2_fast(fmaf(s[mt][r], c, -m_new));
+            const float p = exp2_fast(fmaf(s[mt][r], c, -shift));
             s[mt][r] = p;
             sum += p;
         }
@@ -429,7 +433,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_kernel(const bf16_t *__restri
         }
         f32x16 s[2];
         scores(stages[STAGE][0], krows, qf, s);
-        const float before = m, alpha = online_softmax(s, j * 64, wave_q0, qrow, g, c, m, l);
+        const float before = m, alpha = online_softmax<false>(s, j * 64, wave_q0, qrow, g, c, m, l);
         if (__builtin_amdgcn_ballot_w64(m != before)) { // rescale only when some row's maximum moved
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt)
@@ -779,7 +783,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(const bf16_t *__
                 wait_lgkmcnt0(); // the keys have been read
                 copy(slot, kbase + size_t(j + WAVES) * 64 * ld);
             }
-            const float before = m, alpha = online_softmax(s, j * 64, q0, qrow, g, c, m, l);
+            const float before = m, alpha = online_softmax<true>(s, j * 64, q0, qrow, g, c, m, l);
             if (__builtin_amdgcn_ballot_w64(m != before)) {
 #pragma unroll
                 for (int dt = 0; dt < 2; ++dt)
