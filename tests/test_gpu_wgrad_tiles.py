@@ -2,10 +2,13 @@
 stages than the ring holds, odd counts, tile counts that 8 does not divide and more than the compute units, token ranges
 that are folded, operands and gradient that are column slices, accumulation.  fp32 sums of at most 16384 exact bf16
 products (2^-24 a partial sum): 1e-5 in relative L2."""
+import ctypes as C
+
 import pytest
 import torch
 
 from gpu_util import check, library, stream, sync
+from turbogpt_amd.bridge import WgradJob
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +40,50 @@ def test_single_gradient(M, N, K, pad):
         got = dw[:, :K].double() / (1 + accumulate)
         assert float((got - want).norm() / want.norm()) < 1e-5
         assert bool(dw[:, K:].isnan().all())  # nothing written beside the gradient
+
+
+def fold_bound(tokens):
+    """Relative rms error of fp32 sums over `tokens` products: the matrix instruction adds eight at a time, 24 such steps make a
+    partial sum (three stages of 64) and the partial sums are added in turn.  A rounding is uniform within half an ulp, 0.416 *
+    2^-24 of the value in the mean square; n steps of a random walk add up to sqrt(n / 2) of it.  15 % on top."""
+    return 1.15 * 0.416 * 2 ** -24 * (24 / 2 + -(-tokens // 192) / 2) ** 0.5
+
+
+def distance(dw, dy, x):
+    want = dy.double().t().contiguous() @ x.double()
+    return float((dw.double() - want).norm() / want.norm())
+
+
+def operands(M, N, K, gen):
+    return (torch.randn(M, N, device="cuda", generator=gen).bfloat16(), torch.randn(M, K, device="cuda", generator=gen).bfloat16(),
+            torch.full((N, K), float("nan"), device="cuda"))
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 3072, 768), (1024, 128, 2048), (1920, 640, 1920), (4096, 1024, 1024), (8192, 896, 896),
+                                   (16384, 256, 1024)])
+def test_single_gradient_against_64_bits(M, N, K):
+    lib = library()
+    dy, x, dw = operands(M, N, K, torch.Generator(device="cuda").manual_seed(M + N + K))
+    need = lib.tgk_gemm_wgrad_workspace(M, N, K)
+    workspace = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    check(lib.tgk_gemm_wgrad(stream(), M, N, K, dy.data_ptr(), N, x.data_ptr(), K, dw.data_ptr(), K, 0, workspace.data_ptr(), need))
+    sync()
+    assert distance(dw, dy, x) < fold_bound(M)
+
+
+@pytest.mark.parametrize("M,d,ffn,depth", [(1024, 256, 1024, 4), (2048, 512, 2048, 4)])
+def test_list_against_64_bits(M, d, ffn, depth):
+    lib = library()
+    gen = torch.Generator(device="cuda").manual_seed(M + d)
+    shapes = [(d, ffn), (ffn, d), (d, d), (3 * d, d)] * depth + [(256, d)] * 2
+    matrices = [operands(M, N, K, gen) for N, K in shapes]
+    jobs = (WgradJob * len(shapes))(*[WgradJob(N, K, dy.data_ptr(), N, x.data_ptr(), K, dw.data_ptr(), K)
+                                      for (N, K), (dy, x, dw) in zip(shapes, matrices)])
+    at = C.addressof(jobs)
+    table_bytes, need = (f(M, len(shapes), at) for f in (lib.tgk_gemm_wgrad_list_table_bytes, lib.tgk_gemm_wgrad_list_workspace))
+    table, workspace = (torch.empty(max(n, 16), dtype=torch.uint8, device="cuda") for n in (table_bytes, need))
+    check(lib.tgk_gemm_wgrad_list_prepare(M, len(shapes), at, table.data_ptr(), table_bytes))
+    check(lib.tgk_gemm_wgrad_list(stream(), M, len(shapes), at, table.data_ptr(), 0, workspace.data_ptr(), need, None))
+    sync()
+    for dy, x, dw in matrices:
+        assert distance(dw, dy, x) < fold_bound(M)

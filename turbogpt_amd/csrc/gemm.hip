@@ -759,7 +759,8 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
 // gemm64_kernel.  Ends behind a barrier: the slots are free.
 // GROUPS = 2: two such groups of four waves take the two halves of the stages, each through its own ring (`smem` is the
 // first's), and the second hands its sums to the first, which alone ends with the product.
-template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1> struct TileProduct {
+// FOLD > 0: the sums of every FOLD stages are added up by themselves and then join a second set of sums.
+template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 0> struct TileProduct {
     using TA = typename Tile64Of<BM, AKC>::type;
     using TB = typename Tile64Of<BN, BKC>::type;
     static constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, THREADS = 256;
@@ -803,23 +804,23 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1> struct Tile
             }
             p_slot = p_slot + 1 == S ? 0 : p_slot + 1;
         };
+        f32x4 sums_of_folds[FM][FN][2][2];
+        auto each = [&](auto &&body) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+            for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
+                for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    acc[i][j][t >> 1][t & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int t = 0; t < 4; ++t)
+                        body(acc[i][j][t >> 1][t & 1], sums_of_folds[i][j][t >> 1][t & 1]);
+        };
+        each([](f32x4 &sum, f32x4 &total) { sum = total = f32x4{0.f, 0.f, 0.f, 0.f}; });
 #pragma unroll
         for (int s = 0; s < S - 1; ++s)
             if (s < k_chunks)
                 copy_stage();
         int c_slot = 0;
-        for (int c = 0; c < rounds; ++c) {
-            if (GROUPS > 1 && c >= k_chunks) {
-                __syncthreads();
-                break;
-            }
+        auto multiply = [&](int c, auto anew) { // anew: the stage's sums replace those before it
             // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
             const int younger = k_chunks - 1 - c;
             if (S >= 4 && younger >= 2)
@@ -851,10 +852,26 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1> struct Tile
 #pragma unroll
                     for (int i = 0; i < 2 * FM; ++i) {
                         f32x4 &t = acc[i >> 1][j >> 1][i & 1][j & 1];
-                        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], t, 0, 0, 0);
+                        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], anew && ks == 0 ? zero : t, 0, 0, 0);
                     }
             c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
+        };
+        if constexpr (FOLD > 0) {
+            for (int c = 0; c < k_chunks;) {
+                const int end = min(c + FOLD, k_chunks);
+                multiply(c, std::true_type{});
+                while (++c < end)
+                    multiply(c, std::false_type{});
+                each([](f32x4 &sum, f32x4 &total) { total += sum; });
+            }
+            each([](f32x4 &sum, f32x4 &total) { sum = total; });
+        } else {
+            for (int c = 0; c < k_chunks; ++c)
+                multiply(c, std::false_type{});
         }
+        if (GROUPS > 1 && k_chunks < rounds)
+            __syncthreads(); // the other group's last stage
         __syncthreads(); // other waves may still read the last stage
         if (GROUPS > 1) { // a lane's sums to the same lane of the first group
             f32x4 *sums = reinterpret_cast<f32x4 *>(smem + (group == 0 ? S * SLOT : 0)) + wave * (64 * FM * FN * 4) + lane;
@@ -1647,9 +1664,17 @@ struct WgradTiles {
     size_t split_stride;  // then `one.dw` is the first of `splits` slabs this far apart, for splitk_reduce_kernel
     float *sumsq; // optional: one sum of squares a block
 };
+// One chain of fp32 sums over all tokens is further from 64 bits than slabs of some tokens added up, so the sums of every
+// three stages join a second set.  Relative error in 1e-7 (tokens, N x K: one chain, this, slabs): 512, 3072 x 768 1.25, 0.79,
+// 0.90; 1920, 640 x 1920 2.62, 0.96, 1.03; 4096, 1024 x 1024 2.72, 1.02, 1.37; 16384, 256 x 1024 2.77, 1.13, 1.64; the 18
+// products of d_model 256 over 2048 2.73, 0.98, 1.21; with two stages 0.72 to 1.13, with four 0.90 to 1.17.  It costs 3 to 4 % on 128 x
+// 128 tiles (8192, 896 x 896 25.3 -> 26.1 us, that list 24.4 -> 25.3), nothing on 64 x 64.  The first stage of three starts from a zero
+// operand instead of cleared registers (with those 27.5 and 27.0 us).  Without the bound of two waves a SIMD the compiler takes
+// 304 registers and one block fits a unit where two did: 16384, 2304 x 768 120 us instead of 66.
+constexpr int WGRAD_FOLD = 3;
 template <int BM, int BN, int S, int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS) void wgrad_tiles_kernel(const WgradTiles w) {
-    using P = TileProduct<BM, BN, S, false, false, GROUPS>;
+__global__ __launch_bounds__(256 * GROUPS, 2) void wgrad_tiles_kernel(const WgradTiles w) {
+    using P = TileProduct<BM, BN, S, false, false, GROUPS, WGRAD_FOLD>;
     static_assert(4 * 4096 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float waves[4];
@@ -2087,16 +2112,16 @@ int wgrad_splits(Tile tile, int tiles, int k_tiles) {
 // Time of 64 tokens on a unit that has `deepest` tiles of wgrad_tiles_kernel (us, measured over the shapes named below).
 double wgrad_stage_us(int edge, int deepest) {
     if (edge == 64)
-        return deepest == 1 ? 0.23 : deepest == 2 ? 0.37 : 0.19 * deepest;
-    return deepest == 1 ? 0.56 : deepest / 2 * 0.76 + deepest % 2 * 0.66;
+        return deepest == 1 ? 0.24 : deepest == 2 ? 0.38 : 0.20 * deepest;
+    return deepest == 1 ? 0.63 : deepest / 2 * 0.82 + deepest % 2 * 0.72;
 }
 // How one weight gradient is cut: tiles of `edge` and token ranges (slabs that a second launch folds), or edge 0: the
 // persistent kernel's tiles.  By estimates in us: launches 3.5 and 2.2, stages as above, slabs written and read at 5.5 TB/s;
 // the persistent kernel at 1.07 PFLOP/s (128 x 192; 0.95 on 128 x 128) when all its blocks have work.  No more slabs than
-// the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: this, 64 x 64 tiles uncut,
-// persistent): 1920, 640 x 640 10.8, 10.8, -; 2048, 256 x 256 7.9, 11.0, 10.3; 4096, 512 x 512 11.5, 19.4, -; 8192, 384 x 384
-// 13.0, 35.8, 25.8; 8192, 896 x 896 25.5, 36.5, 39.8; 16384, 128 x 128 12.4, 69.2, 24.7; 16384, 640 x 640 28.6, 69.8, 42.2;
-// 16384, 2304 x 768 63.4, 98.5, 65.3; 16384, 768 x 3072 - , 210, 82.6.
+// the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: this, persistent): 1920, 640 x 640
+// 10.6, 14.8; 2048, 256 x 256 7.3, 10.7; 4096, 512 x 512 10.8, 19.0; 8192, 384 x 384 11.6, 25.6; 8192, 896 x 896 26.1, 40.3;
+// 16384, 128 x 128 11.4, 24.7; 16384, 640 x 640 26.1, 42.0; 16384, 2304 x 768 66.1, 63.7; 16384, 768 x 3072 86.8, 83.9.  Uncut
+// on 64 x 64 tiles 8192, 384 x 384 took 35.8 and 16384, 128 x 128 69.2.
 struct WgradCut {
     int edge, splits;
 };
