@@ -76,10 +76,16 @@ struct Slot {
     bf16_t *nf = nullptr, *logits = nullptr, *t1 = nullptr;
     // All weight gradients of a step go out as one launch behind the backward pass: every block keeps the four
     // output gradients that launch reads: g_x[l] = gradient of the loss by x[l] (g_x[l + 1] enters block l), g_mid[l]
-    // by the block's middle, g_u[l] by the MLP pre-activation, g_qkv[l] by the packed projections.
+    // by the block's middle, g_u[l] by the MLP pre-activation, g_qkv[l] by the packed projections.  Where the device
+    // has no room for that, all blocks share one set of the four (g_x: one buffer) and every block's weight gradients
+    // are a launch of their own, behind its attention.
     std::vector<bf16_t *> g_x, g_mid, g_u, g_qkv;
-    std::vector<TgkWgradJob> wgrad_jobs;
-    void *wgrad_table = nullptr;
+    std::vector<TgkWgradJob> wgrad_jobs; // four a block, the head, the token table
+    struct WgradLaunch {
+        int first, count; // of wgrad_jobs
+        void *table;
+    };
+    std::vector<WgradLaunch> wgrads; // one; or one a block, the head's and the token table's
     bf16_t *onehot = nullptr; // [tokens][256]: the token table's gradient is one more product of that launch
     // ... and the kernels that write the gradient leave the sums of its squares here (cuda/trainer.cuh:35-46): the
     // launch above for the matrices, one more small launch for the ranges in `norm_ranges` (every other tensor)
@@ -178,6 +184,13 @@ struct Engine {
         allocated_bytes += n * sizeof(T);
         if (zero)
             check_hip(hipMemsetAsync(raw, 0, n * sizeof(T), stream));
+    }
+    // gives back every allocation behind the first `count`
+    void release_after(size_t count, size_t bytes) {
+        (void)hipStreamSynchronize(stream);
+        for (; allocations.size() > count; allocations.pop_back())
+            (void)hipFree(allocations.back());
+        allocated_bytes = bytes;
     }
     void use_device() const { check_hip(hipSetDevice(config.base.device)); }
     void sync() const { // every stream: the engine is quiescent afterwards
@@ -314,7 +327,17 @@ struct Engine {
         // No weight gradient in the loop: every block leaves its output gradients in buffers of its own and one
         // launch at the end computes all 4 * depth + 2 products (the head's included - its operands are dlogits,
         // still in `logits`, and nf - and the token table's, one-hot^T times the gradient entering the first block).
+        // Or, where those buffers did not fit, a launch behind the head's input gradient, one in every block, before
+        // the block's last kernel overwrites the gradient that entered it, and one at the end.
+        const bool together = s.wgrads.size() == 1, norms = together && c.clip > 0;
+        const auto weight_gradients = [&](const Slot::WgradLaunch &part) {
+            Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
+            wgrad_list(stream, M, part.count, s.wgrad_jobs.data() + part.first, ListUnit, part.table, workspace, workspace_bytes,
+                       norms ? s.norms : nullptr);
+        };
         OP(TG_CLASS_HEAD, tgk_gemm_dgrad_t(stream, M, V, d, logits, V, wt(layout.head), V, t1, d, nullptr, 0));
+        if (!together)
+            weight_gradients(s.wgrads[c.depth]);
         OP(TG_CLASS_LAYERNORM_BWD, ln_rows(0, x[c.depth], t1, layout.lnf_g, nullptr, s.g_x[c.depth]));
         for (int l = c.depth - 1; l >= 0; --l) {
             const TgLayerParameters &p = layout.layers[l];
@@ -327,18 +350,15 @@ struct Engine {
             OP(TG_CLASS_ATTN_BWD, tgk_attn_bwd(stream, c.batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d,
                                                b.qkv + 2 * d, 3 * d, b.o, d, b.lse, t1, d, gqkv, gqkv + d, gqkv + 2 * d,
                                                3 * d, scale, workspace, workspace_bytes));
+            if (!together)
+                weight_gradients(s.wgrads[l]);
             OP(TG_CLASS_GEMM_DGRAD, tgk_gemm_dgrad_t(stream, M, 3 * d, d, gqkv, 3 * d, wt(p.qkv), 3 * d, t1, d, nullptr, 0));
             OP(TG_CLASS_LAYERNORM_BWD, ln_rows(2 + 2 * l, x[l], t1, p.ln1_g, mid, s.g_x[l]));
         }
         OP(TG_CLASS_OTHER, backward_rest(stream, {c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions,
                                                   reinterpret_cast<const float *>(s.ln_partials), ln_stride / sizeof(float),
                                                   2 * c.depth + 1, 0, s.ln_targets, s.token_losses, means}));
-        const bool norms = c.clip > 0;
-        {
-            Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
-            wgrad_list(stream, M, int(s.wgrad_jobs.size()), s.wgrad_jobs.data(), ListUnit, s.wgrad_table, workspace,
-                       workspace_bytes, norms ? s.norms : nullptr);
-        }
+        weight_gradients(s.wgrads.back());
         if (norms)
             OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
     }
@@ -534,6 +554,122 @@ void build_segments(Engine *e) {
     e->sync(); // the host vectors go out of scope
 }
 
+// What the backward pass of the wide model works in.  keep: the output gradients of every block, for one launch of all
+// weight gradients; otherwise one set that the blocks share.
+void build_backward(Engine *e, bool keep) {
+    const Config &c = e->config.base;
+    const size_t M = size_t(e->tokens()), d = size_t(e->config.d_model), F = size_t(e->config.ffn), V = size_t(e->config.vocab);
+    size_t need = std::max(tgk_attn_bwd_workspace(c.batch, e->config.heads, c.context), tgk_layernorm_bwd_workspace(int(M), int(d)));
+    for (Slot &slot : e->slots) {
+        slot.g_x.assign(c.depth + 1, nullptr);
+        slot.g_mid.assign(c.depth, nullptr), slot.g_u.assign(c.depth, nullptr), slot.g_qkv.assign(c.depth, nullptr);
+        slot.norms = nullptr;
+        const auto allocate = [&](std::vector<bf16_t *> &buffers, size_t n) {
+            for (bf16_t *&buffer : buffers)
+                if (keep || &buffer == &buffers[0])
+                    e->allocate(buffer, n, false);
+                else
+                    buffer = buffers[0];
+        };
+        allocate(slot.g_x, M * d);
+        allocate(slot.g_mid, M * d);
+        allocate(slot.g_u, M * F);
+        allocate(slot.g_qkv, M * 3 * d);
+        if (keep)
+            e->allocate(slot.onehot, M * V, false);
+        else
+            slot.onehot = slot.logits; // the head's launch has read them
+        float *g = slot.gradient;
+        std::vector<TgkWgradJob> &jobs = slot.wgrad_jobs;
+        jobs.clear();
+        for (int l = 0; l < c.depth; ++l) {
+            const TgLayerParameters &p = e->layout.layers[l];
+            const LayerBuffers &b = slot.layers[l];
+            const int D = int(d), U = int(F);
+            jobs.push_back({D, U, slot.g_x[l + 1], D, b.a, U, g + p.mlp_down, U});
+            jobs.push_back({U, D, slot.g_u[l], U, b.n2, D, g + p.mlp_up, D});
+            jobs.push_back({D, D, slot.g_mid[l], D, b.o, D, g + p.attn_out, D});
+            jobs.push_back({3 * D, D, slot.g_qkv[l], 3 * D, b.n1, D, g + p.qkv, D});
+        }
+        jobs.push_back({int(V), int(d), slot.logits, int(V), slot.nf, int(d), g + e->layout.head, int(d)});
+        jobs.push_back({int(V), int(d), slot.onehot, int(V), slot.g_x[0], int(d), g + e->layout.embedding, int(d)});
+        slot.wgrads.clear();
+        if (keep) {
+            slot.wgrads.push_back({0, int(jobs.size()), nullptr});
+        } else {
+            for (int l = 0; l < c.depth; ++l)
+                slot.wgrads.push_back({4 * l, 4, nullptr});
+            slot.wgrads.push_back({4 * c.depth, 1, nullptr});
+            slot.wgrads.push_back({4 * c.depth + 1, 1, nullptr});
+        }
+        for (Slot::WgradLaunch &part : slot.wgrads) {
+            const TgkWgradJob *list = jobs.data() + part.first;
+            const size_t table_bytes = wgrad_list_table_bytes(int(M), part.count, list, ListUnit);
+            if (!table_bytes)
+                throw std::runtime_error("engine: weight gradients do not fit one list");
+            uint8_t *table = nullptr;
+            e->allocate(table, table_bytes, false);
+            part.table = table;
+            wgrad_list_prepare(int(M), part.count, list, ListUnit, table, table_bytes);
+            need = std::max(need, wgrad_list_workspace(int(M), part.count, list, ListUnit));
+        }
+        if (!keep)
+            continue; // the optimizer step takes the norm of the whole gradient itself
+        // the tensors no matrix product writes, in ranges of 8192 elements (more where a long context would make
+        // too many of them); with the matrices they must cover the flat gradient exactly
+        struct Range {
+            int64_t start, length;
+        };
+        std::vector<Range> ranges;
+        const int64_t range = std::max<int64_t>(8192, (int64_t(c.context) * int64_t(d) / 1024 + 3) / 4 * 4);
+        int64_t covered = 2 * int64_t(V) * d; // the head and the token table
+        const auto cover = [&](int64_t start, int64_t length) {
+            covered += length;
+            for (int64_t at = 0; at < length; at += range)
+                ranges.push_back({start + at, std::min<int64_t>(range, length - at)});
+        };
+        cover(e->layout.positions, int64_t(c.context) * d);
+        for (int l = 0; l < c.depth; ++l) {
+            const TgLayerParameters &p = e->layout.layers[l];
+            cover(p.ln1_g, d), cover(p.ln1_b, d), cover(p.ln2_g, d), cover(p.ln2_b, d);
+            covered += 4 * int64_t(d) * d + 2 * int64_t(F) * d;
+        }
+        cover(e->layout.lnf_g, d), cover(e->layout.lnf_b, d);
+        if (covered != e->layout.count)
+            throw std::runtime_error("engine: gradient norm ranges do not cover the parameters");
+        slot.list_norms = wgrad_list_sumsq_count(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit);
+        slot.range_norms = int(ranges.size());
+        if (slot.list_norms <= 0 || slot.list_norms + slot.range_norms > 4096)
+            throw std::runtime_error("engine: too many gradient norm partials");
+        e->allocate(slot.norms, size_t(slot.list_norms + slot.range_norms), false);
+        uint8_t *device_ranges = nullptr;
+        e->allocate(device_ranges, ranges.size() * sizeof(Range), false);
+        check_hip(hipMemcpy(device_ranges, ranges.data(), ranges.size() * sizeof(Range), hipMemcpyHostToDevice),
+                  "norm ranges: ");
+        slot.norm_ranges = device_ranges;
+    }
+    e->workspace_bytes = need;
+    const int norms = 2 * c.depth + 1;
+    const size_t ln_stride = tgk_layernorm_bwd_workspace(int(M), int(d));
+    for (Slot &slot : e->slots) {
+        uint8_t *ws = nullptr;
+        e->allocate(ws, need, false);
+        slot.workspace = ws;
+        e->allocate(slot.ln_partials, size_t(norms) * ln_stride, false);
+        std::vector<float *> targets(size_t(2 * norms));
+        targets[0] = slot.gradient + e->layout.lnf_g, targets[1] = slot.gradient + e->layout.lnf_b;
+        for (int l = 0; l < c.depth; ++l) {
+            const TgLayerParameters &p = e->layout.layers[l];
+            targets[size_t(2 * (1 + 2 * l))] = slot.gradient + p.ln2_g, targets[size_t(2 * (1 + 2 * l) + 1)] = slot.gradient + p.ln2_b;
+            targets[size_t(2 * (2 + 2 * l))] = slot.gradient + p.ln1_g, targets[size_t(2 * (2 + 2 * l) + 1)] = slot.gradient + p.ln1_b;
+        }
+        uint8_t *table = nullptr;
+        e->allocate(table, targets.size() * sizeof(float *), false);
+        check_hip(hipMemcpy(table, targets.data(), targets.size() * sizeof(float *), hipMemcpyHostToDevice));
+        slot.ln_targets = table;
+    }
+}
+
 } // namespace
 
 // cuda/runtime.cu:62-155: the reference's own width-16 network (config.h:4)
@@ -649,98 +785,21 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
             e->allocate(slot.logits, M * V, false);
             e->allocate(slot.t1, M * d, false);
         }
-        const TgkWgradJob block_jobs[4] = {{int(d), int(F), nullptr, int(d), nullptr, int(F), nullptr, int(F)},
-                                           {int(F), int(d), nullptr, int(F), nullptr, int(d), nullptr, int(d)},
-                                           {int(d), int(d), nullptr, int(d), nullptr, int(d), nullptr, int(d)},
-                                           {int(3 * d), int(d), nullptr, int(3 * d), nullptr, int(d), nullptr, int(d)}};
-        size_t need = std::max(tgk_attn_bwd_workspace(c.batch, model->heads, c.context), tgk_layernorm_bwd_workspace(int(M), int(d)));
-        for (Slot &slot : e->slots) {
-            std::vector<TgkWgradJob> &jobs = slot.wgrad_jobs;
-            for (int l = 0; l < c.depth; ++l)
-                for (int j = 0; j < 4; ++j)
-                    jobs.push_back(block_jobs[j]);
-            jobs.push_back({int(V), int(d), nullptr, int(V), nullptr, int(d), nullptr, int(d)}); // the head
-            jobs.push_back({int(V), int(d), nullptr, int(V), nullptr, int(d), nullptr, int(d)}); // the token table
-            const size_t table_bytes = wgrad_list_table_bytes(int(M), int(jobs.size()), jobs.data(), ListUnit);
-            if (!table_bytes)
-                throw std::runtime_error("engine: weight gradients do not fit one list");
-            slot.g_x.resize(c.depth + 1), slot.g_mid.resize(c.depth), slot.g_u.resize(c.depth), slot.g_qkv.resize(c.depth);
-            for (int l = 0; l <= c.depth; ++l)
-                e->allocate(slot.g_x[l], M * d, false);
-            for (int l = 0; l < c.depth; ++l) {
-                e->allocate(slot.g_mid[l], M * d, false);
-                e->allocate(slot.g_u[l], M * F, false);
-                e->allocate(slot.g_qkv[l], M * 3 * d, false);
-                const TgLayerParameters &p = e->layout.layers[l];
-                const LayerBuffers &b = slot.layers[l];
-                float *g = slot.gradient;
-                TgkWgradJob *jobs = slot.wgrad_jobs.data() + 4 * l;
-                jobs[0].dY = slot.g_x[l + 1], jobs[0].X = b.a, jobs[0].dW = g + p.mlp_down;
-                jobs[1].dY = slot.g_u[l], jobs[1].X = b.n2, jobs[1].dW = g + p.mlp_up;
-                jobs[2].dY = slot.g_mid[l], jobs[2].X = b.o, jobs[2].dW = g + p.attn_out;
-                jobs[3].dY = slot.g_qkv[l], jobs[3].X = b.n1, jobs[3].dW = g + p.qkv;
-            }
-            TgkWgradJob &head = slot.wgrad_jobs[4 * c.depth], &table_job = slot.wgrad_jobs[4 * c.depth + 1];
-            head.dY = slot.logits, head.X = slot.nf, head.dW = slot.gradient + e->layout.head;
-            e->allocate(slot.onehot, M * V, false);
-            table_job.dY = slot.onehot, table_job.X = slot.g_x[0], table_job.dW = slot.gradient + e->layout.embedding;
-            uint8_t *table = nullptr;
-            e->allocate(table, table_bytes, false);
-            slot.wgrad_table = table;
-            wgrad_list_prepare(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit, table, table_bytes);
-            // the tensors no matrix product writes, in ranges of 8192 elements (more where a long context would make
-            // too many of them); with the matrices they must cover the flat gradient exactly
-            struct Range {
-                int64_t start, length;
-            };
-            std::vector<Range> ranges;
-            const int64_t range = std::max<int64_t>(8192, (int64_t(c.context) * int64_t(d) / 1024 + 3) / 4 * 4);
-            int64_t covered = 2 * int64_t(V) * d; // the head and the token table
-            const auto cover = [&](int64_t start, int64_t length) {
-                covered += length;
-                for (int64_t at = 0; at < length; at += range)
-                    ranges.push_back({start + at, std::min<int64_t>(range, length - at)});
-            };
-            cover(e->layout.positions, int64_t(c.context) * d);
-            for (int l = 0; l < c.depth; ++l) {
-                const TgLayerParameters &p = e->layout.layers[l];
-                cover(p.ln1_g, d), cover(p.ln1_b, d), cover(p.ln2_g, d), cover(p.ln2_b, d);
-                covered += 4 * int64_t(d) * d + 2 * int64_t(F) * d;
-            }
-            cover(e->layout.lnf_g, d), cover(e->layout.lnf_b, d);
-            if (covered != e->layout.count)
-                throw std::runtime_error("engine: gradient norm ranges do not cover the parameters");
-            slot.list_norms = wgrad_list_sumsq_count(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit);
-            slot.range_norms = int(ranges.size());
-            if (slot.list_norms <= 0 || slot.list_norms + slot.range_norms > 4096)
-                throw std::runtime_error("engine: too many gradient norm partials");
-            e->allocate(slot.norms, size_t(slot.list_norms + slot.range_norms), false);
-            uint8_t *device_ranges = nullptr;
-            e->allocate(device_ranges, ranges.size() * sizeof(Range), false);
-            check_hip(hipMemcpy(device_ranges, ranges.data(), ranges.size() * sizeof(Range), hipMemcpyHostToDevice),
-                      "norm ranges: ");
-            slot.norm_ranges = device_ranges;
-            need = std::max(need, wgrad_list_workspace(int(M), int(slot.wgrad_jobs.size()), slot.wgrad_jobs.data(), ListUnit));
+        // Every block's output gradients are kept where that leaves room for tg_batch's logits and 256 MiB of data.  It
+        // takes 18 * tokens * d_model bytes a block more than one set for all of them (ffn = 4 d_model), a third of an engine.
+        const size_t allocations = e->allocations.size(), bytes = e->allocated_bytes;
+        bool kept = false;
+        try {
+            build_backward(e, true);
+            size_t free = 0, total = 0;
+            check_hip(hipMemGetInfo(&free, &total));
+            kept = free >= M * V * sizeof(float) + (size_t(256) << 20);
+        } catch (const std::exception &) {
+            (void)hipGetLastError(); // the refused allocation is no later launch's error
         }
-        e->workspace_bytes = need;
-        const int norms = 2 * c.depth + 1;
-        const size_t ln_stride = tgk_layernorm_bwd_workspace(int(M), int(d));
-        for (Slot &slot : e->slots) {
-            uint8_t *ws = nullptr;
-            e->allocate(ws, need, false);
-            slot.workspace = ws;
-            e->allocate(slot.ln_partials, size_t(norms) * ln_stride, false);
-            std::vector<float *> targets(size_t(2 * norms));
-            targets[0] = slot.gradient + e->layout.lnf_g, targets[1] = slot.gradient + e->layout.lnf_b;
-            for (int l = 0; l < c.depth; ++l) {
-                const TgLayerParameters &p = e->layout.layers[l];
-                targets[size_t(2 * (1 + 2 * l))] = slot.gradient + p.ln2_g, targets[size_t(2 * (1 + 2 * l) + 1)] = slot.gradient + p.ln2_b;
-                targets[size_t(2 * (2 + 2 * l))] = slot.gradient + p.ln1_g, targets[size_t(2 * (2 + 2 * l) + 1)] = slot.gradient + p.ln1_b;
-            }
-            uint8_t *table = nullptr;
-            e->allocate(table, targets.size() * sizeof(float *), false);
-            check_hip(hipMemcpy(table, targets.data(), targets.size() * sizeof(float *), hipMemcpyHostToDevice));
-            slot.ln_targets = table;
+        if (!kept) {
+            e->release_after(allocations, bytes);
+            build_backward(e, false);
         }
         e->sync();
         return e;
