@@ -67,3 +67,47 @@ def test_gates_far_below_zero():
     for name, (offset, shape) in entries.items():
         part = slice(offset, offset + int(np.prod(shape)))
         assert relative(gradient[part], expected[part]) < .02, name
+
+
+def part(flat, depth, name):
+    offset, shape = w16.layout(depth)[0][name]
+    return flat[offset:offset + int(np.prod(shape))].reshape(shape)
+
+
+def test_a_token_that_is_not_finite_leaves_other_ids_their_gradient():
+    """The last token of the first sequence has an infinite embedding and a gradient of NaN: its id's row has that, and the
+    rows of the ids of other sequences are what they are beside a sequence without it."""
+    depth, context, batch = 2, 4, 33
+    flat = reference_style_weights(depth)
+    part(flat, depth, "embedding")[250] = np.inf
+    rng = np.random.default_rng(6)
+    x, y = (rng.integers(0, 200, (batch, context), dtype=np.uint8) for _ in range(2))
+    x[0] = 200 + np.arange(context)
+    ordinary = part(run(depth, context, batch, flat, x, y)[2], depth, "embedding")
+    x[0, -1] = 250
+    embedding = part(run(depth, context, batch, flat, x, y)[2], depth, "embedding")
+    assert np.isfinite(ordinary).all() and not np.isfinite(embedding[250]).any()
+    np.testing.assert_array_equal(embedding[:200], ordinary[:200])
+    np.testing.assert_array_equal(embedding[204:250], 0)
+
+
+def test_an_infinite_feature_leaves_the_other_rows_their_gradient():
+    """One feature of the last layer's up projection has an infinite output gradient (its own output is 0, so nothing else of
+    that layer's is): the other rows of the weight gradient have the bits that they have without."""
+    depth, context, batch = 2, 4, 33
+    flat = reference_style_weights(depth)
+    part(flat, depth, "embedding")[:, 0] = 4
+    part(flat, depth, "1.up")[5] = 0
+    part(flat, depth, "1.down")[:, 5] = 3e38
+    part(flat, depth, "1.gate")[5] = 0
+    rng = np.random.default_rng(7)
+    x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
+    ordinary = run(depth, context, batch, flat, x, y)[2]
+    part(flat, depth, "1.gate")[5, 0] = 1e8
+    logits, _, gradient = run(depth, context, batch, flat, x, y)
+    assert np.isfinite(logits).all() and np.isfinite(ordinary).all()
+    assert not np.isfinite(part(gradient, depth, "1.up")[5]).all()
+    others = np.arange(48) != 5
+    np.testing.assert_array_equal(part(gradient, depth, "1.up")[others], part(ordinary, depth, "1.up")[others])
+    for name in ("1.gate", "1.down", "final_norm", "head"):
+        np.testing.assert_array_equal(part(gradient, depth, name), part(ordinary, depth, name), name)

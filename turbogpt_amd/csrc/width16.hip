@@ -731,6 +731,43 @@ __global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const
                 by_row[j] = int((row[w].x >> (8 * j)) & 255u) == vocabulary ? 1.f : 0.f;
         acc = multiply(by_row, by_token(col[w]), acc);
     }
+    // The products with the identity and the one-hot matrix are exact for finite rows alone: 0 times an infinity is NaN,
+    // in features and ids that have no part in it.  A wave whose sums are not finite takes them again with the rows
+    // turned by moving them; no other wave pays for it.
+    const auto finite = [](float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; };
+    if (__builtin_amdgcn_ballot_w64(!(finite(acc[0]) && finite(acc[1]) && finite(acc[2]) && finite(acc[3])))) {
+        const auto moved = [&](const u32x2 &tile, int token) { // feature c of `token`, out of lane 16 (c % 4) + token
+            const int from = 16 * (c & 3) + token;
+            const uint32_t low = uint32_t(__shfl(int(tile.x), from, 64)), high = uint32_t(__shfl(int(tile.y), from, 64));
+            const uint32_t pair = c & 8 ? high : low;
+            return __uint_as_float(c & 4 ? pair & 0xffff0000u : pair << 16);
+        };
+        acc = ZERO;
+#pragma unroll 1
+        for (int w = 0; w < waves; ++w) {
+            u32x2 this_col = col[0], this_row = row[0];
+#pragma unroll
+            for (int k = 1; k < CHUNK_WAVES; ++k)
+                this_col = k == w ? col[k] : this_col, this_row = k == w ? row[k] : this_row;
+            if (vocabulary < 0) {
+                f32x4 a, b;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    a[j] = moved(this_row, 4 * j + g), b[j] = moved(this_col, 4 * j + g);
+                acc = multiply(a, b, acc);
+                continue;
+            }
+            for (int t = 0; t < m.per_wave; ++t) {
+                const float value = moved(this_col, t);
+                const int id = int(uint32_t(__shfl(int(this_row.x), 16 * (t & 3), 64)) >> (8 * (t >> 2)) & 255u);
+                const int mine = id - (vocabulary - c + 4 * g); // the register of this lane that is the id's, if it is one of four
+                if ((first + w) * m.per_wave + t < m.tokens)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[r] = mine == r ? acc[r] + value : acc[r];
+            }
+        }
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         out[(4 * g + r) * width + c] = acc[r];
