@@ -111,3 +111,16 @@ def test_an_infinite_feature_leaves_the_other_rows_their_gradient():
     np.testing.assert_array_equal(part(gradient, depth, "1.up")[others], part(ordinary, depth, "1.up")[others])
     for name in ("1.gate", "1.down", "final_norm", "head"):
         np.testing.assert_array_equal(part(gradient, depth, name), part(ordinary, depth, name), name)
+
+
+def test_a_query_that_is_not_finite_leaves_the_keys_it_did_not_choose():
+    """The positions before a token whose embedding is infinite: it chose none of them, so their gradients are finite, and the
+    ids that stand there alone have rows without a NaN."""
+    depth, context, batch = 2, 4, 33
+    flat = reference_style_weights(depth)
+    part(flat, depth, "embedding")[250] = np.inf
+    rng = np.random.default_rng(8)
+    x, y = (rng.integers(0, 200, (batch, context), dtype=np.uint8) for _ in range(2))
+    x[0] = [201, 202, 203, 250]
+    embedding = part(run(depth, context, batch, flat, x, y)[2], depth, "embedding")
+    assert np.isfinite(embedding[:250]).all() and (embedding[201:204] != 0).any(axis=1).all()

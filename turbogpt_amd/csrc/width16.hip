@@ -608,12 +608,13 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
             const float their_dt = __uint_as_float(later<D>(__float_as_uint(dt))), their_gate = __uint_as_float(later<D>(__float_as_uint(gate)));
             const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
             const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
-            const bool chose = p.position + D < m.context && theirs == uint32_t(D);
-            const float t = chose ? their_dt : 0.f, g = chose ? their_gate : 0.f;
+            // skipped, not multiplied by 0: what did not choose this token may be infinite
+            if (p.position + D < m.context && theirs == uint32_t(D)) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                dk[r] = fmaf(t, qf[r], dk[r]);
-                dv[r] = fmaf(df[r], g, dv[r]);
+                for (int r = 0; r < 4; ++r) {
+                    dk[r] = fmaf(their_dt, qf[r], dk[r]);
+                    dv[r] = fmaf(df[r], their_gate, dv[r]);
+                }
             }
         });
         const f32x4 dq = turned(rounded(rotate_back(rounded(key * dt), rc, rs)));
