@@ -197,3 +197,22 @@ def test_pipeline_state_survives_resume(orc):
     # schedule: bounded staleness, and a deterministic result
     assert trace.tolist() == [4, 4, 4, 5, 6, 7]
     assert np.isfinite(resumed).all() and np.abs(resumed - expected).max() < 0.05
+
+
+def test_losses_of_launches_that_follow_one_another():
+    """Launches that nobody waits between, shorter than the batches in flight and past the end of the loss history: the last
+    one's losses are those of its own steps."""
+    initial = reference_style_weights(4, scale=0.05)
+    data = np.random.default_rng(9).integers(0, 256, 4096, dtype=np.uint8)
+
+    def losses(*launches):
+        with bridge.Native(bridge.Config(inflight=4, context=8, depth=4, batch=16)) as engine:
+            engine.set_weights(initial)
+            engine.set_data(data)
+            for steps in launches:
+                engine.train(steps)
+            return engine.training_losses(launches[-1])
+
+    np.testing.assert_array_equal(losses(*[1] * 6), losses(6)[-1:])
+    np.testing.assert_array_equal(losses(3, 2), losses(5)[-2:])
+    np.testing.assert_array_equal(losses(4096, 40), losses(4000, 136)[-40:])

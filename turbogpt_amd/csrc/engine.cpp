@@ -23,6 +23,9 @@ constexpr int NormPartials = 1024;
 constexpr int ListUnit = 128;   // every width is a multiple of it (wgrad_list)
 constexpr int RowTile = 128;    // smallest number of rows the matrix products take
 constexpr int MaxInFlight = 16; // batches in flight, each with its own stream and saved activations
+// Rows of the loss history, a ring over the steps: two steps that share a row are at least MaxInFlight apart, so the later
+// one is behind the earlier one also where they are in different launches and on different streams.
+constexpr int HistoryRows = MaxLaunchSteps + MaxInFlight;
 
 struct LayerBuffers {
     bf16_t *n1, *qkv, *o, *mid, *n2, *u, *a;
@@ -136,6 +139,7 @@ struct Engine {
     uint64_t step = 0;
     uint64_t floor = 0; // oldest weight version that exists: the step at the last tg_set_weights / _set_optimizer_state
     int last_train_steps = 0;
+    uint64_t last_train_first = 0;
     std::vector<int> version_trace; // weight version each step of the last tg_train read
     uint64_t total_staleness = 0;
     int max_staleness = 0;
@@ -174,6 +178,7 @@ struct Engine {
         }
     };
 
+    float *history_row(uint64_t at) const { return loss_history + size_t(at % HistoryRows) * config.base.context; }
     int tokens() const { return config.base.batch * config.base.context; }
 
     template <class T> void allocate(T *&ptr, size_t n, bool zero = true) { // cuda/engine_internal.h:17-27
@@ -400,19 +405,19 @@ struct Engine {
                                                    transpose_tiles));
     }
     // batch `at`: sample, forward, loss row, backward, on one slot with one weight version
-    void batch_gradient(Slot &s, const Version &v, uint64_t at, float *history_row) {
+    void batch_gradient(Slot &s, const Version &v, uint64_t at) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
         if (width16) {
             Scope profile_scope(this, TG_CLASS_OTHER);
             w16_gradient(stream, c.depth, c.batch, c.context, {v.hi, v.lo}, {data, data_size, c.seed, at}, s.input, s.workspace,
-                         s.token_losses, history_row, s.gradient, s.norms);
+                         s.token_losses, history_row(at), s.gradient, s.norms);
             return;
         }
         OP(TG_CLASS_OTHER, sample_embed(stream, data, data_size, c.seed, at, c.batch, c.context, config.d_model, s.input, s.target,
                                         v.hi + layout.embedding, v.hi + layout.positions, s.x[0]));
         forward(s, v, true, nullptr, c.batch, false, true);
-        backward(s, v, history_row);
+        backward(s, v, history_row(at));
     }
     // One training step.  Synchronous engine: everything in order on the one stream, weights updated in place
     // (cuda/trainer.cuh:109-124).  inflight = K (cuda/pipeline.cuh:40-126 as streams and events): batch `at` and its
@@ -420,20 +425,21 @@ struct Engine {
     // read max(floor, at - K + 1), the oldest version the ring still guarantees, and frees the slot's gradient.  The
     // optimizer step waits for its predecessor, on another slot's stream; the version that it overwrites, at - K, was
     // last read by batch at - 1, which that predecessor follows.  Optimizer steps on a stream of their own (K + 1
-    // streams) cost two more events a step and shared one of the process's four hardware queues with a slot at K = 4:
-    // the width-16 network of depth 8, context 8, batch 16 took 54 us a step, now 36 to 40.  The choice is made on the host, so a run is reproducible; the staleness
-    // bound at - K + 1 <= version <= at is the reference's.
-    void train_step(uint64_t at, float *history_row, int *trace) {
+    // streams) cost two more events a step and shared one of the process's four hardware queues with a slot at K = 4: long
+    // runs of the width-16 network of depth 8, context 8, batch 16 took 54 us a step, now 36 to 40 (16 steps and the weights
+    // to the host 0.73 ms).  The choice is made on the host, so a run is reproducible; the staleness bound at - K + 1 <=
+    // version <= at is the reference's.
+    void train_step(uint64_t at, int *trace) {
         const uint64_t K = slots.size(), ring = versions.size();
         if (K == 1) {
-            batch_gradient(slots[0], versions[0], at, history_row);
+            batch_gradient(slots[0], versions[0], at);
             optimize(stream, at, slots[0].gradient, versions[0], versions[0], &slots[0]);
             *trace = int(at);
             return;
         }
         Slot &s = slots[at % K];
         const uint64_t read = std::max(floor, at + 1 >= K ? at + 1 - K : 0);
-        batch_gradient(s, versions[read % ring], at, history_row);
+        batch_gradient(s, versions[read % ring], at);
         const Version &from = versions[at % ring];
         Version &to = versions[(at + 1) % ring];
         check_hip(hipStreamWaitEvent(s.stream, from.done, 0));
@@ -711,7 +717,7 @@ TG_API Engine *tg_create(const Config *c) {
         e->allocate(e->momentum, P);
         e->allocate(e->variance, P);
         e->allocate(e->norm_partials, NormPartials);
-        e->allocate(e->loss_history, size_t(MaxLaunchSteps) * c->context);
+        e->allocate(e->loss_history, size_t(HistoryRows) * c->context);
         e->allocate(e->batch_means, size_t(c->context));
         e->workspace_bytes = tgk_w16_workspace(c->depth, c->batch, c->context);
         for (Slot &slot : e->slots) {
@@ -761,7 +767,7 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
         e->allocate(e->momentum, P);
         e->allocate(e->variance, P);
         e->allocate(e->norm_partials, NormPartials);
-        e->allocate(e->loss_history, size_t(MaxLaunchSteps) * c.context);
+        e->allocate(e->loss_history, size_t(HistoryRows) * c.context);
         e->allocate(e->batch_means, size_t(c.context));
         build_segments(e);
         build_transpose_jobs(e);
@@ -959,9 +965,8 @@ TG_API int tg_train(Engine *e, int steps) {
         e->use_device();
         e->version_trace.assign(size_t(steps), 0);
         for (int i = 0; i < steps; ++i)
-            e->train_step(e->step + uint64_t(i), e->loss_history + size_t(i) * e->config.base.context,
-                          &e->version_trace[size_t(i)]);
-        e->last_train_steps = steps;
+            e->train_step(e->step + uint64_t(i), &e->version_trace[size_t(i)]);
+        e->last_train_steps = steps, e->last_train_first = e->step;
         e->step += uint64_t(steps);
     });
 }
@@ -974,7 +979,10 @@ TG_API int tg_get_training_losses(Engine *e, float *losses, int count) {
             throw std::runtime_error("Training loss count exceeds the last launch");
         e->use_device();
         e->sync(); // the rows are written on the slots' streams
-        e->download({{losses, size_t(count) * e->config.base.context * 4, e->loss_history}});
+        const uint64_t first = e->last_train_first;
+        const size_t row = size_t(e->config.base.context) * 4, together = std::min<size_t>(count, HistoryRows - first % HistoryRows);
+        e->download({{losses, together * row, e->history_row(first)},
+                     {losses + together * row / 4, (size_t(count) - together) * row, e->loss_history}});
     });
 }
 // cuda/runtime.cu:243-262: the weight version each step of the last tg_train read (a synchronous engine
@@ -1082,13 +1090,13 @@ TG_API int tg_profile_step(Engine *e, float *class_ms, int *class_launches, int 
         e->version_trace.assign(1, 0);
         e->profiling = true;
         try {
-            e->train_step(e->step, e->loss_history, e->version_trace.data());
+            e->train_step(e->step, e->version_trace.data());
         } catch (...) {
             e->profiling = false;
             throw;
         }
         e->profiling = false;
-        e->last_train_steps = 1;
+        e->last_train_steps = 1, e->last_train_first = e->step;
         e->step += 1;
         e->sync();
         std::fill(class_ms, class_ms + classes, 0.f);
