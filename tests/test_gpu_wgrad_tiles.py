@@ -23,7 +23,9 @@ pytestmark = pytest.mark.gpu
                                        (16384, 128, 128, 8),  # many ranges of few tiles
                                        (8192, 896, 896, 8),  # 128 x 128 tiles, four stages
                                        (16384, 768, 768, 0),  # the same with two blocks a unit
-                                       (16384, 768, 3072, 0)])  # the persistent kernel
+                                       (16384, 768, 3072, 0),  # the persistent kernel
+                                       (4096, 512, 4096, 0),  # the same: few rows of tiles, a wide X
+                                       (16384, 2304, 768, 8)])
 def test_single_gradient(M, N, K, pad):
     lib = library()
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
@@ -40,6 +42,33 @@ def test_single_gradient(M, N, K, pad):
         got = dw[:, :K].double() / (1 + accumulate)
         assert float((got - want).norm() / want.norm()) < 1e-5
         assert bool(dw[:, K:].isnan().all())  # nothing written beside the gradient
+
+
+@pytest.mark.parametrize("M,N,K", [(16384, 2304, 2304), (12288, 1920, 2304)])
+def test_wide_gradient_is_no_slower_than_a_batch_of_one(M, N, K):
+    """Where every XCD would read nearly all of X, tiles lose to the persistent kernel (242 against 173 us and 154 against 124).
+    tgk_gemm_wgrad_batch runs the same product persistently, so it tells the two apart: the shortest of twenty, 15 % for the
+    kernels' own difference."""
+    lib = library()
+    dy, x, dw = operands(M, N, K, torch.Generator(device="cuda").manual_seed(M))
+    job = (WgradJob * 1)(WgradJob(N, K, dy.data_ptr(), N, x.data_ptr(), K, dw.data_ptr(), K))
+    at = C.addressof(job)
+    need = max(lib.tgk_gemm_wgrad_workspace(M, N, K), lib.tgk_gemm_wgrad_batch_workspace(M, 1, at))
+    workspace = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    calls = [lambda: lib.tgk_gemm_wgrad(stream(), M, N, K, dy.data_ptr(), N, x.data_ptr(), K, dw.data_ptr(), K, 0,
+                                        workspace.data_ptr(), need),
+             lambda: lib.tgk_gemm_wgrad_batch(stream(), M, 1, at, 0, workspace.data_ptr(), need)]
+    shortest = [float("inf")] * 2
+    for _ in range(20):
+        for i, call in enumerate(calls):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            check(call())
+            end.record()
+            sync()
+            shortest[i] = min(shortest[i], begin.elapsed_time(end))
+    print(f"{M} tokens, {N} x {K}: alone {shortest[0] * 1e3:.1f} us, batch of one {shortest[1] * 1e3:.1f} us", flush=True)
+    assert shortest[0] < 1.15 * shortest[1]
 
 
 def fold_bound(tokens):

@@ -2116,12 +2116,18 @@ double wgrad_stage_us(int edge, int deepest) {
     return deepest == 1 ? 0.63 : deepest / 2 * 0.82 + deepest % 2 * 0.72;
 }
 // How one weight gradient is cut: tiles of `edge` and token ranges (slabs that a second launch folds), or edge 0: the
-// persistent kernel's tiles.  By estimates in us: launches 3.5 and 2.2, stages as above, slabs written and read at 5.5 TB/s;
-// the persistent kernel at 1.07 PFLOP/s (128 x 192; 0.95 on 128 x 128) when all its blocks have work.  No more slabs than
-// the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: this, persistent): 1920, 640 x 640
+// persistent kernel's tiles.  By estimates in us: launches 3.5 and 2.2, slabs written and read at 5.5 TB/s.  A tile's stages as
+// above, a quarter longer beyond two on a unit, or what the eight XCDs read at 5.5 TB/s, if that is longer: an XCD has a run of the
+// tiles, row by row, and with wide matrices every XCD reads nearly all of X (4096, 512 x 4096 on 64 x 64 tiles: 272 MB, 50.5 us; 30.9
+// persistent).  The persistent kernel has two blocks a unit, 1.05 us for their 64 tokens on 128 x 192 (0.92 on 128 x 128),
+// a third more where four does not divide its tiles, which its placement on the XCDs needs.  No more slabs than
+// the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: tiles, persistent): 1920, 640 x 640
 // 10.6, 14.8; 2048, 256 x 256 7.3, 10.7; 4096, 512 x 512 10.8, 19.0; 8192, 384 x 384 11.6, 25.6; 8192, 896 x 896 26.1, 40.3;
-// 16384, 128 x 128 11.4, 24.7; 16384, 640 x 640 26.1, 42.0; 16384, 2304 x 768 66.1, 63.7; 16384, 768 x 3072 86.8, 83.9.  Uncut
-// on 64 x 64 tiles 8192, 384 x 384 took 35.8 and 16384, 128 x 128 69.2.
+// 16384, 128 x 128 11.4, 24.7; 16384, 640 x 640 26.1, 42.0.  Uncut on 64 x 64 tiles 8192, 384 x 384 took 35.8 and
+// 16384, 128 x 128 69.2.  With the persistent kernel at a rate and without the XCDs' reading, the
+// rule took tiles that lose: 16384, 2304 x 2304 242 against 173, 2304 x 768 74 against 70, 4096, 640 x 2560 38.6 against 27.0.
+// Of 2448 shapes from 512 to 32768 tokens and widths from 128 to 4096, 198 were more than 1.5 % behind the persistent
+// kernel, up to 63 %; now 29 are by more than 2 %, at most 11 %, and the mean over all of them is 1.32 times as fast.
 struct WgradCut {
     int edge, splits;
 };
@@ -2133,17 +2139,22 @@ WgradCut plan_wgrad(int M, int N, int K) {
         return {0, most};
     const double elements = double(N) * K;
     const auto slabs = [&](int splits) { return splits > 1 ? 2.2 + 8e-6 * splits * elements / 5.5 : 0.0; };
-    const int blocks = resident_blocks(tile), items = persistent_tiles * most, rounds = (items + blocks - 1) / blocks;
-    const double rate = tile == TILE_128x192 ? 1.07e9 : 0.95e9;
+    const int blocks = resident_blocks(tile), rounds = (persistent_tiles * most + blocks - 1) / blocks;
+    const double pair_us = (tile == TILE_128x192 ? 1.05 : 0.92) * (persistent_tiles % 4 ? 1.3 : 1.0);
     WgradCut best{0, most};
-    double least = 3.5 + slabs(most) + 2 * M * elements / rate * (double(rounds) * blocks / items);
+    double least = 3.5 + slabs(most) + rounds * (M / 64.0 / most) * pair_us;
     for (int edge = 64; edge <= 128; edge *= 2) {
         if (N % edge || K % edge)
             continue;
         const int tiles = (N / edge) * (K / edge);
         for (int splits = 1; splits <= most && (splits == 1 || splits <= M / 128) && (splits == 1 || (splits - 1) * tiles < 2 * units); ++splits) {
             const int deepest = (tiles * splits + units - 1) / units, stages = (M / 64 + splits - 1) / splits;
-            const double us = 3.5 + slabs(splits) + stages * wgrad_stage_us(edge, deepest);
+            // one XCD's run of tiles: whole ranges and what of one is left, as rows and columns of tiles
+            const int run = (tiles * splits + 7) / 8, in_range = std::min(run, tiles), across = K / edge;
+            const double read = 8.0 * std::max(1.0, double(run) / tiles) * M / splits * 2 * edge *
+                                ((in_range + across - 1) / across + std::min(in_range, across));
+            const double body = std::max(stages * wgrad_stage_us(edge, deepest) * (deepest > 2 ? 1.25 : 1.0), read / 5.5e6);
+            const double us = 3.5 + slabs(splits) + body;
             if (us < least)
                 best = {edge, splits}, least = us;
         }
