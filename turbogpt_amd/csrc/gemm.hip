@@ -26,6 +26,7 @@
 // Weight gradients: wgrad_list_kernel, wgrad_batch_kernel (several matrices in one launch), gemm64_kernel / gemm_kernel.
 #include "common.h"
 #include "gemm_list.h"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <vector>
@@ -900,6 +901,27 @@ TG_DEVICE int xcd_contiguous(int block, int blocks) {
     const int xcd = block & 7;
     return xcd * (blocks >> 3) + min(xcd, blocks & 7) + (block >> 3);
 }
+// A matrix in tiles, listed row by row or column by column, whichever lets an XCD's run of `run` tiles read fewer rows of
+// the two operands: with 16 rows of 32 tiles a run of 64 is two rows of tiles and every column, or four columns and every
+// row.  1024 x 4096 on 64 x 128 tiles, K = 3072 / 2560 / 1536: row by row 53.7 / 44.9 / 26.8 us, column by column
+// 30.8 / 28.2 / 17.4; weight gradient, 4096 tokens, 512 x 4096: 50.5, 27.6.
+struct TileGrid {
+    int rows, cols, by_columns;
+    TG_DEVICE void place(int tile, int &row, int &col) const {
+        const int across = by_columns ? rows : cols, line = tile / across, at = tile - line * across;
+        row = by_columns ? at : line;
+        col = by_columns ? line : at;
+    }
+};
+// rows of both operands that a run reads
+int run_reads(const TileGrid &grid, int bm, int bn, int run) {
+    const int across = grid.by_columns ? grid.rows : grid.cols, lines = (run + across - 1) / across, along = std::min(run, across);
+    return grid.by_columns ? along * bm + lines * bn : lines * bm + along * bn;
+}
+TileGrid tile_grid(int rows, int cols, int bm, int bn, int run) {
+    const TileGrid by_rows{rows, cols, 0}, by_columns{rows, cols, 1};
+    return run_reads(by_columns, bm, bn, run) < run_reads(by_rows, bm, bn, run) ? by_columns : by_rows;
+}
 
 // ---- one tile per block: forward and input-gradient products of ordinary and small sizes ----------------------------
 // C = A B^T with A k-contiguous and B either way round.  A product with few outputs is bound by how many compute units
@@ -915,13 +937,15 @@ TG_DEVICE int xcd_contiguous(int block, int blocks) {
 template <int BM, int BN, int S, bool BKC, class Epilogue, int GROUPS = 1>
 __global__ __launch_bounds__(256 * GROUPS) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda,
                                                                  const bf16_t *__restrict__ B, int ldb, int k_chunks,
-                                                                 int tiles_n, Epilogue epilogue) {
+                                                                 TileGrid grid, Epilogue epilogue) {
     using P = TileProduct<BM, BN, S, true, BKC, GROUPS>;
     static_assert(4 * 2048 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6 & 3;
     const bool finishes = GROUPS == 1 || threadIdx.x < 256;
-    const int tile = xcd_contiguous(blockIdx.x, gridDim.x), m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+    int m0, n0;
+    grid.place(xcd_contiguous(blockIdx.x, gridDim.x), m0, n0);
+    m0 *= BM, n0 *= BN;
     const int m = m0 + (wave >> 1) * P::WM, n = n0 + (wave & 1) * P::WN;
     // the epilogue's second input first of all: it lands before the operands do
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
@@ -1656,10 +1680,11 @@ __global__ __launch_bounds__(256, 1) void wgrad_list_kernel(const WgradList w) {
 // list is not cut along the tokens, so nothing is folded.  What bounds it is a stage's latency on a unit with one tile and the
 // transposing LDS reads on one with several (wgrad_stage_us).
 struct WgradTiles {
-    const WgradListJob *jobs; // device memory; NULL: `one`, its tiles row-major, tiles_n a row
+    const WgradListJob *jobs; // device memory; NULL: `one`, its tiles as `grid` has them
     const int4 *tiles;
     WgradListJob one;
-    int tiles_n, count, k_chunks, accumulate;
+    TileGrid grid;
+    int count, k_chunks, accumulate;
     int splits = 1;       // `one` only: token ranges a tile is cut into (1 with a list); `count` is tiles x splits
     size_t split_stride;  // then `one.dw` is the first of `splits` slabs this far apart, for splitk_reduce_kernel
     float *sumsq; // optional: one sum of squares a block
@@ -1687,7 +1712,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void wgrad_tiles_kernel(const Wgra
         const int tiles = w.count / w.splits, split = at / tiles, tile = at - split * tiles;
         const int first = int(int64_t(split) * w.k_chunks / w.splits);
         const int chunks = int(int64_t(split + 1) * w.k_chunks / w.splits) - first;
-        const int4 t = w.jobs ? w.tiles[tile] : make_int4(0, tile / w.tiles_n * BM, tile % w.tiles_n * BN, 0);
+        int4 t{};
+        if (w.jobs) {
+            t = w.tiles[tile];
+        } else {
+            w.grid.place(tile, t.y, t.z);
+            t.y *= BM, t.z *= BN;
+        }
         const WgradListJob job = w.jobs ? w.jobs[t.x] : w.one;
         f32x4 acc[P::FM][P::FN][2][2];
         P::run(job.dy + int64_t(first) * 64 * job.lddy, job.lddy, job.x + int64_t(first) * 64 * job.ldx, job.ldx, t.y, t.z,
@@ -1990,7 +2021,7 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
         configured[device].store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256 * GROUPS), lds, stream, A, lda, B, ldb,
-                       K / 64, N / BN, epilogue);
+                       K / 64, tile_grid(M / BM, N / BN, BM, BN, ((M / BM) * (N / BN) + 7) / 8), epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
 // Which tile a product whose reduced dimension 64 divides is cut into.  The cost of a 64-k stage on the fullest compute
@@ -2117,20 +2148,22 @@ double wgrad_stage_us(int edge, int deepest) {
 }
 // How one weight gradient is cut: tiles of `edge` and token ranges (slabs that a second launch folds), or edge 0: the
 // persistent kernel's tiles.  By estimates in us: launches 3.5 and 2.2, slabs written and read at 5.5 TB/s.  A tile's stages as
-// above, a quarter longer beyond two on a unit, or what the eight XCDs read at 5.5 TB/s, if that is longer: an XCD has a run of the
-// tiles, row by row, and with wide matrices every XCD reads nearly all of X (4096, 512 x 4096 on 64 x 64 tiles: 272 MB, 50.5 us; 30.9
-// persistent).  The persistent kernel has two blocks a unit, 1.05 us for their 64 tokens on 128 x 192 (0.92 on 128 x 128),
+// above, a quarter longer beyond two on a unit, or what the eight XCDs read at 5.5 TB/s, if that is longer.  The persistent
+// kernel has two blocks a unit, 1.05 us for their 64 tokens on 128 x 192 (0.92 on 128 x 128),
 // a third more where four does not divide its tiles, which its placement on the XCDs needs.  No more slabs than
 // the persistent kernel would use, so the workspace is the same.  Measured (tokens, N x K: tiles, persistent): 1920, 640 x 640
 // 10.6, 14.8; 2048, 256 x 256 7.3, 10.7; 4096, 512 x 512 10.8, 19.0; 8192, 384 x 384 11.6, 25.6; 8192, 896 x 896 26.1, 40.3;
 // 16384, 128 x 128 11.4, 24.7; 16384, 640 x 640 26.1, 42.0.  Uncut on 64 x 64 tiles 8192, 384 x 384 took 35.8 and
-// 16384, 128 x 128 69.2.  With the persistent kernel at a rate and without the XCDs' reading, the
-// rule took tiles that lose: 16384, 2304 x 2304 242 against 173, 2304 x 768 74 against 70, 4096, 640 x 2560 38.6 against 27.0.
-// Of 2448 shapes from 512 to 32768 tokens and widths from 128 to 4096, 198 were more than 1.5 % behind the persistent
-// kernel, up to 63 %; now 29 are by more than 2 %, at most 11 %, and the mean over all of them is 1.32 times as fast.
+// 16384, 128 x 128 69.2.  16384, 2304 x 2304 242, 173; 2304 x 768 74, 70.  Of 2448 shapes from 512 to 32768 tokens and widths
+// from 128 to 4096, 17 are more than 2 % behind the persistent kernel, at most 12 %; the mean over all of them is 1.32
+// times as fast.
 struct WgradCut {
     int edge, splits;
 };
+TileGrid wgrad_grid(int N, int K, int edge, int splits) {
+    const int rows = N / edge, cols = K / edge, tiles = rows * cols;
+    return tile_grid(rows, cols, edge, edge, std::min((tiles * splits + 7) / 8, tiles));
+}
 WgradCut plan_wgrad(int M, int N, int K) {
     const Tile tile = choose_tile(N, K);
     const int persistent_tiles = (N / tile_rows(tile)) * (K / tile_cols(tile));
@@ -2149,10 +2182,10 @@ WgradCut plan_wgrad(int M, int N, int K) {
         const int tiles = (N / edge) * (K / edge);
         for (int splits = 1; splits <= most && (splits == 1 || splits <= M / 128) && (splits == 1 || (splits - 1) * tiles < 2 * units); ++splits) {
             const int deepest = (tiles * splits + units - 1) / units, stages = (M / 64 + splits - 1) / splits;
-            // one XCD's run of tiles: whole ranges and what of one is left, as rows and columns of tiles
-            const int run = (tiles * splits + 7) / 8, in_range = std::min(run, tiles), across = K / edge;
-            const double read = 8.0 * std::max(1.0, double(run) / tiles) * M / splits * 2 * edge *
-                                ((in_range + across - 1) / across + std::min(in_range, across));
+            // one XCD's run of tiles: whole ranges, or a part of one
+            const int run = (tiles * splits + 7) / 8;
+            const double read = 8.0 * std::max(1.0, double(run) / tiles) * M / splits * 2 *
+                                run_reads(wgrad_grid(N, K, edge, splits), edge, edge, std::min(run, tiles));
             const double body = std::max(stages * wgrad_stage_us(edge, deepest) * (deepest > 2 ? 1.25 : 1.0), read / 5.5e6);
             const double us = 3.5 + slabs(splits) + body;
             if (us < least)
@@ -2322,7 +2355,8 @@ extern "C" int tgk_gemm_wgrad(hipStream_t stream, int M, int N, int K, const uin
         if (cut.edge) {
             WgradTiles w{};
             w.one = {dY, X, e.out, lddy, ldx, e.ld_out, 0};
-            w.tiles_n = K / cut.edge, w.splits = cut.splits, w.count = (N / cut.edge) * (K / cut.edge) * cut.splits;
+            w.grid = wgrad_grid(N, K, cut.edge, cut.splits);
+            w.splits = cut.splits, w.count = w.grid.rows * w.grid.cols * cut.splits;
             w.k_chunks = M / 64, w.accumulate = e.accumulate, w.split_stride = e.split_stride;
             launch_wgrad_tiles(stream, w, cut.edge, w.count);
         } else if (takes_64(tile, M)) {
