@@ -2005,12 +2005,9 @@ void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const
 }
 
 template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
-void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
-                      const Epilogue &given) {
-    // these sizes' GELU outputs are left to the caches, where the next launch finds them (streamed past them the product
-    // itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %)
-    const typename Epilogue::Cached epilogue{given.any};
-    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, typename Epilogue::Cached, GROUPS>;
+void launch_gemm_tile_as(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
+                            const Epilogue &epilogue) {
+    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, Epilogue, GROUPS>;
     constexpr size_t lds = GROUPS * S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
@@ -2023,6 +2020,17 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
     hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256 * GROUPS), lds, stream, A, lda, B, ldb,
                        K / 64, tile_grid(M / BM, N / BN, BM, BN, ((M / BM) * (N / BN) + 7) / 8), epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
+}
+// GELU outputs that the eight L2s hold are left to them, where the next launch finds them (streamed past them the product
+// itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %); larger ones are streamed: the two of
+// 16384 x 4096, K = 1920 / 896 / 640 took 352 / 200 / 165 us through the caches, 285 / 160 / 128 past them.
+template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
+void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
+                      const Epilogue &e) {
+    if (size_t(M) * N * 2 * sizeof(bf16_t) > size_t(8) * (4 << 20))
+        launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, e);
+    else
+        launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
 }
 // Which tile a product whose reduced dimension 64 divides is cut into.  The cost of a 64-k stage on the fullest compute
 // unit, in 10 ns, as measured with one, two and more tiles on it (they overlap: 16 KB of operands take 0.23 us alone and 0.19
