@@ -22,6 +22,7 @@ SHAPES = [(128, 128, 64),      # 64 x 64: 4 tiles, one stage
           (1920, 1920, 448),   # 128 x 128, deep ring: seven stages
           (16384, 384, 192),   # 128 x 128, two stages in flight
           (16384, 640, 64),    # the same, GELU outputs that the caches do not hold
+          (16384, 2944, 64),   # 128 x 128, the persistent kernel: more than ten tiles a unit
           (8192, 2688, 64)]    # 128 x 192
 
 
