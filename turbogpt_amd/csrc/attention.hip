@@ -158,9 +158,11 @@ struct CausalGrid {
 // 298 -> 274, 9 pairs of 8192 144 -> 123; 401 -> 329, 13 pairs of 8192 170 -> 160; 479 -> 444; but 15 pairs of 2048 (32
 // blocks an XCD) 28.7 -> 32.5; 76 -> 79.  32-row blocks: 12 pairs of 1024 8.9 -> 8.6; 26.5 -> 20.3, 4 pairs of 4096
 // 33 -> 20; 114 -> 58.
-CausalGrid causal_grid(int B, int H, int T, int rows) {
+// The forward's 128-row blocks are short enough for the copies to outweigh that below 64 blocks a pair: whole -> dealt us, 4096
+// positions 13 pairs 58.3 -> 62.2, 30 pairs 83.3 -> 89.5, 1920 and 2048 30 pairs 30.1 -> 31.3 and 32.2 -> 33.3; 8192 20 pairs 219 -> 200.
+CausalGrid causal_grid(int B, int H, int T, int rows, int least_ranks = 1) {
     const int pairs = B * H, ranks = T / rows;
-    return {H, pairs, ranks, (pairs + 7) / 8 * ranks > 32 ? pairs % 8 : 0};
+    return {H, pairs, ranks, (pairs + 7) / 8 * ranks > 32 && ranks >= least_ranks ? pairs % 8 : 0};
 }
 
 template <int N> struct Const {
@@ -983,7 +985,7 @@ extern "C" int tgk_attn_fwd(hipStream_t stream, int B, int H, int T, int hd, con
         check_matrix(O, ldo, "O");
         require(lse && !(reinterpret_cast<uintptr_t>(lse) & 15), "attention: lse must be 16-byte aligned");
         const bool split = forward_splits(B, H, T);
-        const CausalGrid grid = causal_grid(B, H, T, split ? 32 : 128);
+        const CausalGrid grid = split ? causal_grid(B, H, T, 32) : causal_grid(B, H, T, 128, 64);
         hipLaunchKernelGGL(split ? attn_fwd_split_kernel : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
                            ld, O, ldo, lse, T, grid, scale * LOG2E);
         check_hip(hipGetLastError(), "attention forward launch: ");
