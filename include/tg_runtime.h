@@ -84,7 +84,11 @@ TG_API int tg_set_onecycle(Engine *engine, const OneCycle *schedule); /* once, b
  * mean loss [context] (cuda/runtime.cu:291-320). */
 TG_API int tg_batch(Engine *engine, const uint8_t *x, const uint8_t *y, float *logits, float *gradients,
                     float *per_position);
-TG_API int tg_predict(Engine *engine, const uint8_t *context, float *logits); /* last position, [vocab] */
+/* The logits [vocab] of one sequence's last position.  The width-16 network's are tg_batch's bit for bit.  The wide model
+ * computes one sequence, whose size may choose other kernels than a whole batch's: their sums run in another order, so the
+ * two differ as correct results of the same precision do (1 % at 12 layers of 768), and are the same bits only where the
+ * kernels are. */
+TG_API int tg_predict(Engine *engine, const uint8_t *context, float *logits);
 TG_API int tg_optimizer_test(Engine *engine, const float *gradients, int steps); /* 1..64 */
 TG_API int tg_synchronize(Engine *engine);
 
