@@ -389,7 +389,7 @@ struct Engine {
         if (width16) { // AdamW's tensors and the hidden matrices (cuda/optim.cuh:92-118)
             Scope profile_scope(this, TG_CLASS_OPTIMIZER);
             w16_update(stream, c.depth, {now.hi, now.lo}, {to.hi, to.lo}, momentum, variance, gradient, norms, norm_count,
-                       adam_args(lr, beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at),
+                       fused ? w16_norm_parts() : 1, adam_args(lr, beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at),
                        {muon_lr, muon_momentum, c.weight_decay, c.ns_steps});
             return;
         }
@@ -725,7 +725,7 @@ TG_API Engine *tg_create(const Config *c) {
             e->allocate(ws, e->workspace_bytes, false);
             slot.workspace = ws;
             slot.list_norms = w16_norm_count(c->depth);
-            e->allocate(slot.norms, size_t(slot.list_norms));
+            e->allocate(slot.norms, size_t(slot.list_norms * w16_norm_parts()));
         }
         e->sync();
         return e;

@@ -4,8 +4,8 @@
 // cuda/ops.cuh:57-144, cuda/attention.cuh:4-106, cuda/optim.cuh:17-119.
 //
 // What bounds it is latency: a step is 1 GFLOP over some ten thousand tokens, and a sequence (at most eight positions)
-// never leaves a wave.  So a wave takes sixteen tokens - whole sequences - through all layers in registers, one launch
-// forward and one backward, with the weights staged in LDS as matrix operands.  Products run on
+// never leaves a wave.  So a wave takes sixteen tokens - whole sequences - through all layers in registers, forward and
+// backward, with the weights staged in LDS as matrix operands.  Products run on
 // v_mfma_f32_16x16x4_f32, which is bit for bit a chain of fmaf over its four k (measured on random and extreme values;
 // the bf16 forms add in an order of their own): every sum has one order, the k's own, whatever the kernel's shape, so
 // results do not depend on how the work is cut.  Lane 16 g + c works for token c:
@@ -13,19 +13,23 @@
 //   "head" layout: register r holds feature 4 g + r - head g of the token, one head a lane, so attention reads other
 //   positions' keys and values with DPP row shifts.
 // A product's results come out in either, by the order of the weight's rows.  Weight gradients are products over tokens,
-// a third launch: a wave per 16 x 16 tile and chunk of tokens turns the saved rows with the identity matrix and adds over
-// the tokens in order; a fourth folds the chunks in order.  No atomics, bit-reproducible (the place of weight_gradient's
-// read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
+// another launch: a block for the rows that one layer kept of a chunk of tokens, which the transposing load reads across,
+// so that a chain of fmaf runs over the tokens in order; one more folds the chunks in order.  No atomics, bit-reproducible
+// (the place of weight_gradient's read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
 #include "common.h"
 #include "width16.h"
 #include "../../include/tgk_kernels.h"
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
+
+// No product and sum is fused that is not written as fmaf: the kernels that share a function below have the same bits.
+#pragma clang fp contract(off)
 
 namespace {
 
 constexpr int W = 16, HEADS = 4, F = 48, V = 256, MAX_DEPTH = 8;
-constexpr int WAVES = 4;       // waves of a forward / backward block: they share the staged weights
+constexpr int WAVES = 4;       // waves of a block: they share the staged weights
 constexpr int CHUNK_WAVES = 8; // waves' tokens in one partial sum of a weight gradient (128 tokens)
 
 struct Layer {
@@ -58,14 +62,16 @@ Layout make_layout(int depth) {
     return p;
 }
 
-// Rows kept between the launches, a tile of 64 x 8 bytes a wave and quantity in the lanes' own order.  Forward: block
-// input, normalised rows, post-RoPE query, the winning key and value (head layout), attention output, post-attention
-// residual, gate | up and activation (cuda/types.cuh:40-44, cuda/model.cuh:25-29); backward: the gradients that are
-// operands of the weight gradients.  And words: GELU(top), GELU'(top), distance to the winner, the two inverse norms.
+// Rows kept between the launches, a tile of 64 x 8 bytes a wave and quantity in the lanes' own order.  For the backward
+// pass: block input, post-RoPE query, the winning key and value (head layout), post-attention residual, gate | up
+// (cuda/types.cuh:40-44, cuda/model.cuh:25-29).  For the weight gradients, side by side: normalised rows, attention output,
+// activation, and the gradients that are their other operands.  And words: GELU(top), GELU'(top), distance to the
+// winner, the two inverse norms.
 enum Tile {
-    T_X, T_N1, T_Q, T_KEY, T_VALUE, T_A, T_MIDDLE, T_N2, T_GU, T_ACT = T_GU + 6,
-    T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES
+    T_X, T_Q, T_KEY, T_VALUE, T_MIDDLE, T_GU, T_OPERANDS = T_GU + 6,
+    T_N1 = T_OPERANDS, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES
 };
+constexpr int OPERANDS = TILES - T_OPERANDS;
 enum Word { WORD_GATE, WORD_SLOPE, WORD_DISTANCE, WORD_INV1, WORD_INV2, WORDS };
 struct Workspace {
     u32x2 *tiles;    // [depth][waves][TILES][64]
@@ -107,6 +113,8 @@ Workspace carve(int depth, int batch, int context, void *base) {
 
 // ---- device helpers ---------------------------------------------------------------------------------
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 TG_DEVICE float master(const bf16_t *hi, const uint16_t *lo, int i) { // cuda/ops.cuh:6-9
     return __uint_as_float((uint32_t(hi[i]) << 16) | lo[i]);
@@ -218,61 +226,134 @@ TG_DEVICE Lane lane_of(const Model &m) {
 // The weights in LDS as first operands, a tile of 64 x 8 bytes each (lane 16 g + c: elements (row c, k = 4 j + g), j = 0..3):
 // 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
 // The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
+// Operands of dX = dY W (rows = inputs, k = outputs) are read from the same tiles with the transposing load, in feed
+// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Last
+// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own.
 constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
-__host__ __device__ constexpr int staged_tiles(int depth) { return depth * LAYER_TILES + HEAD_TILES; }
-size_t staged_bytes(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
+__host__ __device__ constexpr int staged_tiles(int depth) { return depth * (LAYER_TILES + 1) + HEAD_TILES; }
+__host__ __device__ constexpr size_t embedding_at(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
+__host__ __device__ constexpr size_t staged_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
 TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its own inverse
-// TRANSPOSED: operands of dX = dY W (rows = inputs, k = outputs; the attention projection's rows in head layout)
-// instead of Y = X W^T (rows = outputs; q, k and v in head layout)
-template <bool TRANSPOSED> TG_DEVICE void stage_weights(const Model &m, uint16_t *tiles, float *scales) {
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), total = staged_tiles(m.depth);
-    // a lane brings four elements of one row: element e goes to operand row `row` and k = col + e, or the other way round
-    const int row = lane >> 2, col = (lane & 3) * 4;
-    constexpr int AT_ONCE = 8; // loads in flight a wave: the staging waits for memory twice at depth 4, not 17 times
-    for (int base = w; base < total; base += WAVES * AT_ONCE) {
-        u32x2 v[AT_ONCE];
-#pragma unroll
-        for (int i = 0; i < AT_ONCE; ++i) {
-            const int tile = base + i * WAVES, l = tile / LAYER_TILES, k = tile - l * LAYER_TILES;
-            if (tile >= total)
-                continue;
-            const Layer q = layer_layout(l);
-            const bf16_t *source = m.hi;
-            if (tile >= m.depth * LAYER_TILES)
-                source += V * W + m.depth * LAYER_SIZE + W + (tile - m.depth * LAYER_TILES) * 256 + lane * 4;
-            else if (k < 10) // q, k, v, attention; gate, up: rows of 16
-                source += (k < 4 ? q.qkv + k * 256 : q.gate + (k - 4) * 256) + lane * 4;
-            else // down: rows of 48
-                source += q.down + (k - 10) * 16 + row * F + col;
-            v[i] = *reinterpret_cast<const u32x2 *>(source);
-        }
-#pragma unroll
-        for (int i = 0; i < AT_ONCE; ++i) {
-            const int tile = base + i * WAVES, k = tile % LAYER_TILES;
-            if (tile >= total)
-                continue;
-            const bool feed = tile >= m.depth * LAYER_TILES || (TRANSPOSED ? k != 3 : k > 2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int operand_row = TRANSPOSED ? col + e : row, at = TRANSPOSED ? row : col + e;
-                const int c = feed ? feed_row(operand_row) : operand_row;
-                tiles[(tile * 64 + (at & 3) * 16 + c) * 4 + (at >> 2)] = uint16_t((e < 2 ? v[i].x : v[i].y) >> ((e & 1) * 16));
-            }
-        }
-    }
-    for (int at = threadIdx.x; at < (2 * m.depth + 1) * W; at += 64 * WAVES) { // attention and MLP norm of each layer, final
-        const int n = at >> 4;
-        const Layer q = layer_layout(n >> 1);
-        const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
-        scales[at] = master(m.hi, m.lo, offset + (at & 15));
-    }
-    __syncthreads();
+// Byte offset, in a tile of items (g, c), of the item that lane 16 q + 4 j + m addresses for a transposing load: (m, 4 q + j)
+// or (m, 4 j + q).  Lane 16 q + i then gets element i % 4 of items (i / 4, 4 q + 0..3) or (i / 4, 4 * 0..3 + q).
+TG_DEVICE int across_offset(int lane, bool natural) {
+    const int q = lane >> 4, j = (lane >> 2) & 3, m = lane & 3;
+    return (16 * m + (natural ? 4 * j + q : 4 * q + j)) * 8;
 }
+TG_DEVICE u32x2 read_across(const unsigned char *at) {
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)at));
+}
+// Wave w stages tiles w, w + 4 and w + 8 of every layer, the thirteenth of layers w and w + 4, and four of the head's: all
+// loads go out before the first is waited for, and every address is a layer's away from the one before.
+struct Staging {
+    static constexpr int PER_LAYER = 3, TAIL = MAX_DEPTH * PER_LAYER, LAST = MAX_DEPTH / WAVES, HEADS = HEAD_TILES / WAVES, SCALES = 2;
+    const Model &m;
+    unsigned char *tiles;
+    u32x2 v[TAIL + LAST + HEADS];
+    float scale[SCALES];
+    int lane, wave;
+    TG_DEVICE Staging(const Model &m_, unsigned char *memory)
+        : m(m_), tiles(memory), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
+    TG_DEVICE float *scales() const { return reinterpret_cast<float *>(tiles + staged_tiles(m.depth) * 512); }
+    // a lane brings four elements of one row: k = 4 (lane % 4) .. + 3
+    TG_DEVICE int row_offset(int width) const { return (lane >> 2) * width + (lane & 3) * 4; }
+    TG_DEVICE static int tile_offset(int k) { // of tile k in its layer's weights
+        const Layer q = layer_layout(0);
+        return k < 4 ? q.qkv + k * 256 : k < 10 ? q.gate + (k - 4) * 256 : q.down + (k - 10) * 16;
+    }
+    TG_DEVICE void request() {
+        const bf16_t *of_layer[PER_LAYER], *last = m.hi + tile_offset(12) + wave * LAYER_SIZE + row_offset(F);
+#pragma unroll
+        for (int i = 0; i < PER_LAYER; ++i) // rows of `down` are 48 long
+            of_layer[i] = m.hi + tile_offset(wave + i * WAVES) + (wave + i * WAVES < 10 ? row_offset(W) : row_offset(F));
+#pragma unroll
+        for (int l = 0; l < MAX_DEPTH; ++l)
+            if (l < m.depth)
+#pragma unroll
+                for (int i = 0; i < PER_LAYER; ++i)
+                    v[l * PER_LAYER + i] = *reinterpret_cast<const u32x2 *>(of_layer[i] + l * LAYER_SIZE);
+#pragma unroll
+        for (int i = 0; i < LAST; ++i)
+            if (wave + i * WAVES < m.depth)
+                v[TAIL + i] = *reinterpret_cast<const u32x2 *>(last + i * WAVES * LAYER_SIZE);
+        const bf16_t *head = m.hi + V * W + m.depth * LAYER_SIZE + W + wave * 256 + row_offset(W);
+#pragma unroll
+        for (int i = 0; i < HEADS; ++i)
+            v[TAIL + LAST + i] = *reinterpret_cast<const u32x2 *>(head + i * WAVES * 256);
+#pragma unroll
+        for (int i = 0; i < SCALES; ++i) {
+            const int at = threadIdx.x + i * 64 * WAVES, n = at >> 4; // attention and MLP norm of each layer, final
+            const Layer q = layer_layout(n >> 1);
+            const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
+            if (n <= 2 * m.depth)
+                scale[i] = master(m.hi, m.lo, offset + (at & 15));
+        }
+    }
+    TG_DEVICE void request_embedding() const { // 8 KiB
+#pragma unroll
+        for (int i = 0; i < V * W * 2 / 1024 / WAVES; ++i) {
+            const int piece = i * WAVES + wave;
+            async_copy16(lds_address(tiles) + uint32_t(embedding_at(m.depth)) + uint32_t(piece * 1024), m.hi, uint32_t(piece * 1024 + lane * 16));
+        }
+    }
+    TG_DEVICE static uint16_t element(const u32x2 &v, int e) { return uint16_t((e < 2 ? v.x : v.y) >> ((e & 1) * 16)); }
+    // element e of a lane's four is k = 4 j + e: item (e, row), element j.  `to`: the lane's place in the tile
+    TG_DEVICE static void put(unsigned char *to, const u32x2 &v) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint16_t *>(to + e * 128) = element(v, e);
+    }
+    TG_DEVICE void finish(bool backward) {
+        const int row = lane >> 2, j = lane & 3;
+        unsigned char *natural = tiles + row * 8 + j * 2, *feed = tiles + feed_row(row) * 8 + j * 2, *of_layer[PER_LAYER];
+#pragma unroll
+        for (int i = 0; i < PER_LAYER; ++i)
+            of_layer[i] = (wave + i * WAVES > 2 ? feed : natural) + (wave + i * WAVES) * 512;
+        // the attention projection (wave 3's first) again: rows = inputs 4 j + e, k = output `row`: item (row % 4, input), element row / 4
+        unsigned char *turned = tiles + (m.depth * LAYER_TILES + HEAD_TILES) * 512 + ((row & 3) * 16 + 4 * j) * 8 + (row >> 2) * 2;
+#pragma unroll
+        for (int l = 0; l < MAX_DEPTH; ++l)
+            if (l < m.depth) {
+#pragma unroll
+                for (int i = 0; i < PER_LAYER; ++i)
+                    put(of_layer[i] + l * LAYER_TILES * 512, v[l * PER_LAYER + i]);
+                if (backward && wave == 3)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        *reinterpret_cast<uint16_t *>(turned + l * 512 + e * 8) = element(v[l * PER_LAYER], e);
+            }
+#pragma unroll
+        for (int i = 0; i < LAST; ++i)
+            if (wave + i * WAVES < m.depth)
+                put(feed + ((wave + i * WAVES) * LAYER_TILES + 12) * 512, v[TAIL + i]);
+#pragma unroll
+        for (int i = 0; i < HEADS; ++i)
+            put(feed + (m.depth * LAYER_TILES + wave + i * WAVES) * 512, v[TAIL + LAST + i]);
+#pragma unroll
+        for (int i = 0; i < SCALES; ++i) {
+            const int at = threadIdx.x + i * 64 * WAVES;
+            if (at < (2 * m.depth + 1) * W)
+                scales()[at] = scale[i];
+        }
+        wait_vmcnt<0>(); // the embedding
+        __syncthreads();
+    }
+};
+static_assert(Staging::SCALES * 64 * WAVES >= (2 * MAX_DEPTH + 1) * W && LAYER_TILES == Staging::PER_LAYER * WAVES + 1,
+              "every scale has a thread, every tile a wave");
 struct Staged {
-    const u32x2 *tiles;
+    const unsigned char *tiles;
     const float *scales;
-    int lane, g;
-    TG_DEVICE f32x4 operator()(int tile) const { return unpack4(tiles[tile * 64 + lane]); }
+    int lane, g, head, turned_attention; // tiles: the head's first, the first attention projection for the backward pass
+    int feed, natural; // across_offset
+    TG_DEVICE Staged(const Model &m, const unsigned char *memory, const Lane &p)
+        : tiles(memory), scales(reinterpret_cast<const float *>(memory + staged_tiles(m.depth) * 512)), lane(p.lane), g(p.g),
+          head(m.depth * LAYER_TILES), turned_attention(head + HEAD_TILES), feed(across_offset(p.lane, false)),
+          natural(across_offset(p.lane, true)) {}
+    TG_DEVICE f32x4 operator()(int tile) const { return unpack4(*reinterpret_cast<const u32x2 *>(tiles + tile * 512 + lane * 8)); }
+    // the transposed operand, of a tile in feed order or (q, k, v) in the matrix's own
+    TG_DEVICE f32x4 turned_feed(int tile) const { return unpack4(read_across(tiles + tile * 512 + feed)); }
+    TG_DEVICE f32x4 turned_natural(int tile) const { return unpack4(read_across(tiles + tile * 512 + natural)); }
     TG_DEVICE f32x4 scale(int norm) const {
         const float *s = scales + norm * W + g;
         return f32x4{s[0], s[4], s[8], s[12]};
@@ -338,41 +419,20 @@ TG_DEVICE f32x4 rotate_back(f32x4 v, float c, float s) {
 }
 
 // ---- forward ---------------------------------------------------------------------------------------
-// cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).
-// Tokens and targets come from x and y or, where `data.bytes` is given, straight out of the training bytes (every
-// sequence a window at a hashed place, cuda/dataset.cuh:13-27) and the tokens are left in `sampled` for the backward pass.
-__global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x,
-                                                               const uint8_t *__restrict__ y, W16Data data,
-                                                               uint8_t *__restrict__ sampled, Workspace s,
-                                                               float *__restrict__ token_losses,
-                                                               float *__restrict__ logits_out, int with_gradient) {
-    extern __shared__ __align__(16) unsigned char staged_memory[];
-    uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
-    float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
-    const Lane p = lane_of(m);
-    const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
-    f32x4 h = ZERO;
-    int target = 0;
-    if (p.live) {
-        int token;
-        if (data.bytes) {
-            const int sequence = p.token / m.context;
-            const int64_t low = m.context > 8 ? m.context : 8;
-            const int64_t end = low + int64_t(hash_u64(data.seed + data.step * uint64_t(m.tokens / m.context) + uint64_t(sequence)) %
-                                              uint64_t(data.size - low));
-            const uint8_t *window = data.bytes + (end - m.context) + p.position;
-            token = window[0], target = window[1];
-            if (p.g == 0)
-                sampled[p.token] = uint8_t(token);
-        } else {
-            token = x[p.token], target = y[p.token];
-        }
-        const bf16_t *row = m.hi + token * W + p.g;
-        h = f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])};
-    }
-    stage_weights<false>(m, staged_tiles_at, scales);
-    float rc, rs;
-    rotation(p.position, rc, rs);
+// What the head leaves for the backward pass; the logits' gradients in tiles of sixteen.
+struct Head {
+    u32x2 dlogits[16], hidden;
+    float inverse;
+};
+TG_DEVICE f32x4 embedding_row(const Model &m, const unsigned char *memory, const Lane &p, int token) {
+    const bf16_t *row = reinterpret_cast<const bf16_t *>(memory + embedding_at(m.depth)) + token * W + p.g;
+    return p.live ? f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])} : ZERO;
+}
+// cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).  GRADIENT: rows are kept in `s` and the head's in `head`.
+template <bool GRADIENT, int CONTEXT>
+TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight, const Workspace &s, f32x4 h, int target, float rc,
+                            float rs, float *__restrict__ token_losses, float *__restrict__ logits_out, Head &head) {
+    const int context = CONTEXT ? CONTEXT : m.context;
     for (int l = 0; l < m.depth; ++l) {
         const int tile = l * LAYER_TILES;
         u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
@@ -388,9 +448,9 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
         float top = -INFINITY;
         int distance = 0;
         u32x2 best_key = {0, 0}, best_value = {0, 0};
-        from<7>([&](auto step) {
+        from<CONTEXT ? CONTEXT - 1 : 7>([&](auto step) {
             constexpr int D = decltype(step)::value;
-            if (D >= m.context)
+            if (D >= context)
                 return;
             const u32x2 k = {earlier<D>(key.x), earlier<D>(key.y)}, v = {earlier<D>(value.x), earlier<D>(value.y)};
             const f32x4 kf = unpack4(k);
@@ -411,7 +471,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
         const f32x4 middle = rounded(rounded(multiply(weight(tile + 3), a)) + h);
         const float inv2 = inverse_rms(middle, p);
         const u32x2 n2 = normalize(middle, inv2, weight.scale(2 * l + 1));
-        if (with_gradient) {
+        if constexpr (GRADIENT) {
             keep[T_X * 64] = pack4(h);
             keep[T_N1 * 64] = n1;
             keep[T_Q * 64] = pack4(query);
@@ -421,7 +481,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
             keep[T_MIDDLE * 64] = pack4(middle);
             keep[T_N2 * 64] = n2;
             words[WORD_GATE * 64] = gate;
-            words[WORD_SLOPE * 64] = 0.5f * e + top * 0.3989422804014327f * expf(-0.5f * top * top);
+            words[WORD_SLOPE * 64] = fmaf(top * 0.3989422804014327f, expf(-0.5f * top * top), 0.5f * e);
             words[WORD_DISTANCE * 64] = __int_as_float(distance);
             words[WORD_INV1 * 64] = inv1;
             words[WORD_INV2 * 64] = inv2;
@@ -439,7 +499,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
                 act[r] = act[r] * sigmoid(act[r]);
             const u32x2 act_row = pack4(rounded(act) * unpack4(up_row));
             out = multiply(weight(tile + 10 + t), unpack4(act_row), out);
-            if (with_gradient) {
+            if constexpr (GRADIENT) {
                 keep[(T_GU + t) * 64] = gate_row;
                 keep[(T_GU + 3 + t) * 64] = up_row;
                 keep[(T_ACT + t) * 64] = act_row;
@@ -455,7 +515,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
     float high = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        logit[t] = rounded(multiply(weight(m.depth * LAYER_TILES + t), nff));
+        logit[t] = rounded(multiply(weight(weight.head + t), nff));
         high = fmaxf(fmaxf(high, fmaxf(logit[t][0], logit[t][1])), fmaxf(logit[t][2], logit[t][3]));
     }
     high = token_max(high);
@@ -465,15 +525,25 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 logits_out[size_t(p.token) * V + t * 16 + 4 * r + p.g] = logit[t][r];
-    const int mine = target - p.g; // this lane owns the logits 16 t + 4 r of it
-    float picked = 0.f;
+    // the target's logit: tile target / 16, register target / 4 % 4 of the lane g = target % 4, by halves
+    float of_four[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        const float even = target & 4 ? logit[t][1] : logit[t][0], odd = target & 4 ? logit[t][3] : logit[t][2];
+        of_four[t] = target & 8 ? odd : even;
+    }
+#pragma unroll
+    for (int bit = 0; bit < 4; ++bit)
+#pragma unroll
+        for (int t = 0; t < 8 >> bit; ++t)
+            of_four[t] = target & (16 << bit) ? of_four[2 * t + 1] : of_four[2 * t];
+    const bool holder = p.g == (target & 3);
+    float picked = holder ? of_four[0] : 0.f;
 #pragma unroll
     for (int t = 0; t < 16; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            picked = 16 * t + 4 * r == mine ? logit[t][r] : picked;
+        for (int r = 0; r < 4; ++r)
             logit[t][r] = expf(logit[t][r] - high);
-        }
     // the sum's tree: every 64th logit in order, then halves of what is left (bits 5 .. 0 of the logit's number)
     f32x4 quarter[4];
 #pragma unroll
@@ -484,36 +554,31 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
     picked = swap_add_16(swap_add_32(picked));
     if (p.live && p.g == 0)
         token_losses[p.token] = high + logf(sum) - picked;
-    if (with_gradient) {
-        s.hidden[size_t(p.wave) * 64 + p.lane] = pack4(h);
+    if constexpr (GRADIENT) {
+        head.hidden = pack4(h), head.inverse = inv;
         s.nf[size_t(p.wave) * 64 + p.lane] = nf;
-        s.inverse[size_t(p.wave) * 64 + p.lane] = inv;
         const float share = reciprocal(sum), tokens = float(m.tokens), per_token = 1.f / tokens;
+        const int mine = holder ? target >> 2 : -1; // 4 t + r
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             f32x4 d;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                d[r] = divide(divide(logit[t][r], sum, share) - (16 * t + 4 * r == mine ? 1.f : 0.f), tokens, per_token);
-            u32x2 packed = pack4(d);
-            packed.x = p.live ? packed.x : 0, packed.y = p.live ? packed.y : 0;
-            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = packed;
+                d[r] = divide(divide(logit[t][r], sum, share) - (4 * t + r == mine ? 1.f : 0.f), tokens, per_token);
+            const u32x2 packed = pack4(d);
+            head.dlogits[t].x = p.live ? packed.x : 0, head.dlogits[t].y = p.live ? packed.y : 0;
+            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = head.dlogits[t];
         }
     }
 }
 
 // ---- backward --------------------------------------------------------------------------------------
 // cuda/model.cuh:61-99, without the weight gradients
-__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Workspace s) {
-    extern __shared__ __align__(16) unsigned char staged_memory[];
-    uint16_t *staged_tiles_at = reinterpret_cast<uint16_t *>(staged_memory);
-    float *scales = reinterpret_cast<float *>(staged_memory + staged_tiles(m.depth) * 512);
-    const Lane p = lane_of(m);
-    const Staged weight{reinterpret_cast<const u32x2 *>(staged_memory), scales, p.lane, p.g};
-    const size_t here = size_t(p.wave) * 64 + p.lane;
+template <int CONTEXT>
+TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight, const Workspace &s, float rc, float rs,
+                             const Head &head) {
+    const int context = CONTEXT ? CONTEXT : m.context;
     auto gz = [&](int norm) { return s.gz + ((size_t(norm) * s.waves + p.wave) * 16 + p.c) * W + p.g; };
-    float rc, rs;
-    rotation(p.position, rc, rs);
 
     // a layer's rows are requested while the layer above is worked on
     struct Rows {
@@ -535,19 +600,12 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
 
     // head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
     Rows next;
-    u32x2 dlogits[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-        dlogits[t] = s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane];
-    const u32x2 hidden = s.hidden[here];
-    const float inverse = s.inverse[here];
     request(m.depth - 1, next);
-    stage_weights<true>(m, staged_tiles_at, scales);
     f32x4 dn = ZERO;
 #pragma unroll
     for (int t = 0; t < 16; ++t)
-        dn = multiply(weight(m.depth * LAYER_TILES + t), unpack4(dlogits[t]), dn);
-    f32x4 dh = normalize_backward(unpack4(hidden), inverse, rounded(dn), weight.scale(2 * m.depth), gz(2 * m.depth), p);
+        dn = multiply(weight.turned_feed(weight.head + t), unpack4(head.dlogits[t]), dn);
+    f32x4 dh = normalize_backward(unpack4(head.hidden), head.inverse, rounded(dn), weight.scale(2 * m.depth), gz(2 * m.depth), p);
     for (int l = m.depth - 1; l >= 0; --l) {
         const int tile = l * LAYER_TILES;
         u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
@@ -560,13 +618,13 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const f32x4 gate = unpack4(rows.gate[t]), up = unpack4(rows.up[t]);
-            const f32x4 dy = rounded(multiply(weight(tile + 10 + t), dh)), da = rounded(dy * up);
+            const f32x4 dy = rounded(multiply(weight.turned_feed(tile + 10 + t), dh)), da = rounded(dy * up);
             f32x4 silu;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float g = gate[r], sig = sigmoid(g);
                 silu[r] = g * sig;
-                dgate[t][r] = da[r] * sig * (1.f + g * (1.f - sig));
+                dgate[t][r] = da[r] * sig * fmaf(g, 1.f - sig, 1.f);
             }
             const u32x2 dgate_row = pack4(dgate[t]), dup_row = pack4(dy * rounded(silu));
             keep[(T_DGU + t) * 64] = dgate_row;
@@ -576,13 +634,12 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
         dn = ZERO;
 #pragma unroll
         for (int t = 0; t < 3; ++t)
-            dn = multiply(weight(tile + 4 + t), dgate[t], dn);
+            dn = multiply(weight.turned_feed(tile + 4 + t), dgate[t], dn);
 #pragma unroll
         for (int t = 0; t < 3; ++t)
-            dn = multiply(weight(tile + 7 + t), dup[t], dn);
+            dn = multiply(weight.turned_feed(tile + 7 + t), dup[t], dn);
         // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
-        dh = rounded(dh + normalize_backward(unpack4(rows.middle), rows.inv2, rounded(dn),
-                                             weight.scale(2 * l + 1), gz(2 * l + 1), p));
+        dh = rounded(dh + normalize_backward(unpack4(rows.middle), rows.inv2, rounded(dn), weight.scale(2 * l + 1), gz(2 * l + 1), p));
         keep[T_DH_ATTENTION * 64] = pack4(dh);
 
         // attention: output projection backward, the score gradient of the cached winner, query / key / value gradients
@@ -591,7 +648,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
         const u32x2 query = rows.query;
         const f32x4 key = unpack4(rows.key), value = unpack4(rows.value);
         const float gate = rows.gate_of_top;
-        const u32x2 dattn = pack4(multiply(weight(tile + 3), dh));
+        const u32x2 dattn = pack4(multiply(weight(weight.turned_attention + l), dh));
         const f32x4 da = unpack4(dattn);
         float dt = 0.f;
 #pragma unroll
@@ -599,9 +656,9 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
             dt = fmaf(da[c], value[c], dt);
         dt *= rows.slope;
         f32x4 dk = ZERO, dv = ZERO;
-        up_to<0, 7>([&](auto step) { // queries of this token's sequence that chose it, in order
+        up_to<0, CONTEXT ? CONTEXT - 1 : 7>([&](auto step) { // queries of this token's sequence that chose it, in order
             constexpr int D = decltype(step)::value;
-            if (D >= m.context)
+            if (D >= context)
                 return;
             // every lane takes part in the shifts, so none of them may sit behind a condition
             const uint32_t theirs = later<D>(uint32_t(rows.distance));
@@ -609,7 +666,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
             const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
             const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
             // skipped, not multiplied by 0: what did not choose this token may be infinite
-            if (p.position + D < m.context && theirs == uint32_t(D)) {
+            if (p.position + D < context && theirs == uint32_t(D)) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     dk[r] = fmaf(their_dt, qf[r], dk[r]);
@@ -623,159 +680,309 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
         keep[T_DQKV * 64] = pack4(dq);
         keep[(T_DQKV + 1) * 64] = pack4(dk);
         keep[(T_DQKV + 2) * 64] = pack4(dv);
-        dn = multiply(weight(tile + 2), dv, multiply(weight(tile + 1), dk, multiply(weight(tile), dq)));
-        dh = rounded(dh + normalize_backward(unpack4(rows.x), rows.inv1, rounded(dn),
-                                             weight.scale(2 * l), gz(2 * l), p));
+        dn = multiply(weight.turned_natural(tile + 2), dv,
+                      multiply(weight.turned_natural(tile + 1), dk, multiply(weight.turned_natural(tile), dq)));
+        dh = rounded(dh + normalize_backward(unpack4(rows.x), rows.inv1, rounded(dn), weight.scale(2 * l), gz(2 * l), p));
     }
-    s.dh[here] = pack4(dh);
+    s.dh[size_t(p.wave) * 64 + p.lane] = pack4(dh);
+}
+
+// ---- kernels -----------------------------------------------------------------------------------------
+template <bool GRADIENT>
+__global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
+                                                               Workspace s, float *__restrict__ token_losses,
+                                                               float *__restrict__ logits_out) {
+    extern __shared__ __align__(16) unsigned char memory[];
+    const Lane p = lane_of(m);
+    const Staged weight(m, memory, p);
+    Staging staging(m, memory);
+    const int token = p.live ? x[p.token] : 0, target = p.live ? y[p.token] : 0;
+    staging.request();
+    staging.request_embedding();
+    staging.finish(false);
+    const f32x4 h = embedding_row(m, memory, p, token);
+    float rc, rs;
+    rotation(p.position, rc, rs);
+    Head head;
+    forward_pass<GRADIENT, 0>(m, p, weight, s, h, target, rc, rs, token_losses, logits_out, head);
+    if constexpr (GRADIENT) {
+        const size_t here = size_t(p.wave) * 64 + p.lane;
+        s.hidden[here] = head.hidden, s.inverse[here] = head.inverse;
+    }
+}
+__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Workspace s) {
+    extern __shared__ __align__(16) unsigned char memory[];
+    const Lane p = lane_of(m);
+    const Staged weight(m, memory, p);
+    Staging staging(m, memory);
+    staging.request();
+    Head head;
+    const size_t here = size_t(p.wave) * 64 + p.lane;
+    head.hidden = s.hidden[here], head.inverse = s.inverse[here];
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        head.dlogits[t] = s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane];
+    staging.finish(true);
+    float rc, rs;
+    rotation(p.position, rc, rs);
+    backward_pass<0>(m, p, weight, s, rc, rs, head);
+}
+// A training step's both passes: a wave's backward pass reads only what its own forward pass kept, so the two are one launch
+// and the weights are staged once.  Depth 4, 2560 sequences of 4: 53.0 us as two launches that staged eight tiles at a time,
+// 38.8 so; depth 8, 16 of 8: 79.3 and 62.6.  Two waves a SIMD, which batches of more than 256 blocks need (10000 of 8 at depth 8
+// 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training bytes, every sequence a window at a
+// hashed place (cuda/dataset.cuh:13-27); the tokens are left in `sampled` for the embedding's gradient.
+template <int CONTEXT>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(Model m, W16Data data, uint64_t inverse, uint8_t *__restrict__ sampled,
+                                                               Workspace s, float *__restrict__ token_losses) {
+    extern __shared__ __align__(16) unsigned char memory[];
+    const Lane p = lane_of(m);
+    const Staged weight(m, memory, p);
+    Staging staging(m, memory);
+    int token = 0, target = 0;
+    if (p.live) {
+        const int sequence = p.token / CONTEXT;
+        // the hash modulo the places: `inverse` is 2^64 / places rounded down, so the quotient is at most one too small
+        const uint64_t hash = hash_u64(data.seed + data.step * uint64_t(m.tokens / CONTEXT) + uint64_t(sequence));
+        const uint64_t low = 8, places = uint64_t(data.size) - low;
+        uint64_t place = hash - __umul64hi(hash, inverse) * places;
+        place -= place >= places ? places : 0;
+        const int64_t end = int64_t(low + place);
+        const uint8_t *window = data.bytes + (end - CONTEXT) + p.position;
+        token = window[0], target = window[1];
+    }
+    staging.request();
+    staging.request_embedding();
+    staging.finish(true);
+    if (p.live && p.g == 0)
+        sampled[p.token] = uint8_t(token);
+    const f32x4 h = embedding_row(m, memory, p, token);
+    float rc, rs;
+    rotation(p.position, rc, rs);
+    Head head;
+    forward_pass<true, CONTEXT>(m, p, weight, s, h, target, rc, rs, token_losses, nullptr, head);
+    backward_pass<CONTEXT>(m, p, weight, s, rc, rs, head);
 }
 
 // ---- weight gradients ------------------------------------------------------------------------------
-// A wave sums one 16 x 16 tile of one parameter tensor (or one RMSNorm scale) over the tokens of a chunk, in token order:
-// partial[chunk][parameter].  Jobs: 13 matrix tiles and 2 scales a layer, the head's and the embedding's 16, the final norm.
-constexpr int LAYER_JOBS = 15;
-__host__ __device__ constexpr int gradient_jobs(int depth) { return depth * LAYER_JOBS + 33; }
-__global__ __launch_bounds__(256) void w16_weight_gradient_kernel(Model m, const uint8_t *__restrict__ x, Workspace s,
-                                                                  int parameters) {
-    // consecutive blocks sit on consecutive XCDs: block 8 i + k takes the i-th job group of XCD k's chunks, so that the jobs
-    // of a chunk, which share their rows, share an L2
-    const int groups = (gradient_jobs(m.depth) + 3) / 4, at = blockIdx.x >> 3;
-    const int chunk = at / groups * 8 + (blockIdx.x & 7), job = at % groups * 4 + (threadIdx.x >> 6);
-    if (chunk >= s.chunks || job >= gradient_jobs(m.depth))
-        return;
-    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-    const int first = chunk * CHUNK_WAVES, last = min(first + CHUNK_WAVES, s.waves);
-    float *out = s.partials + size_t(chunk) * parameters;
-    // A row operand (rows of the gradient tile) and a column operand, as tiles of tokens x 16 features in feed layout
-    const u32x2 *rows = nullptr, *cols = nullptr;
-    size_t row_stride = 64, col_stride = 64; // from one wave's tile to the next
-    int width = W, norm = -1, vocabulary = -1;
-    if (job < m.depth * LAYER_JOBS) {
-        const int l = job / LAYER_JOBS, k = job - l * LAYER_JOBS;
-        const Layer q = layer_layout(l);
-        const u32x2 *keep = s.tiles + size_t(l) * s.waves * TILES * 64;
-        row_stride = col_stride = TILES * 64;
-        if (k < 3) {
-            rows = keep + (T_DQKV + k) * 64, cols = keep + T_N1 * 64, out += q.qkv + k * 256;
-        } else if (k == 3) {
-            rows = keep + T_DH_ATTENTION * 64, cols = keep + T_A * 64, out += q.attention;
-        } else if (k < 10) {
-            rows = keep + (T_DGU + k - 4) * 64, cols = keep + T_N2 * 64, out += q.gate + (k - 4) * 256; // gate, then up
-        } else if (k < 13) {
-            rows = keep + T_DH_DOWN * 64, cols = keep + (T_ACT + k - 10) * 64, out += q.down + (k - 10) * 16, width = F;
-        } else {
-            norm = 2 * l + k - 13, out += k == 13 ? q.attention_norm : q.mlp_norm;
-        }
-    } else {
-        const int k = job - m.depth * LAYER_JOBS;
-        if (k < 16) {
-            rows = s.dlogits + k * 64, row_stride = 16 * 64, cols = s.nf, out += V * W + m.depth * LAYER_SIZE + W + k * 256;
-        } else if (k < 32) { // embedding rows: the one-hot matrix of the tokens times the gradient
-            vocabulary = (k - 16) * 16 + c, cols = s.dh, out += (k - 16) * 256;
-        } else {
-            norm = 2 * m.depth, out += V * W + m.depth * LAYER_SIZE;
-        }
-    }
-    f32x4 acc = ZERO;
-    const int waves = last - first;
-    if (norm >= 0) { // a row of ones times the g * z terms
-        const float *gz = s.gz + (size_t(norm) * s.waves + first) * 16 * W + lane;
-        float v[CHUNK_WAVES][4];
-#pragma unroll
-        for (int w = 0; w < CHUNK_WAVES; ++w)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[w][j] = w < waves ? gz[(w * 4 + j) * 64] : 0.f; // token 4 j + g, feature c
-#pragma unroll
-        for (int w = 0; w < CHUNK_WAVES; ++w)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, v[w][j], acc, 0, 0, 0);
-        if (g == 0)
-            out[c] = acc[0];
-        return;
-    }
-    // a feed-layout tile times the identity, on the bf16 instruction (exact: one product a sum), comes out as feature c of
-    // tokens 4 g + r; turned, register j is token 4 j + g: step j of a product over tokens
-    u32x2 identity;
-    identity.x = (g == c ? 0x3f80u : 0u) | (4 + g == c ? 0x3f800000u : 0u);
-    identity.y = (8 + g == c ? 0x3f80u : 0u) | (12 + g == c ? 0x3f800000u : 0u);
-    auto by_token = [&](const u32x2 &tile) {
-        return turned(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, tile), __builtin_bit_cast(s16x4, identity), ZERO, 0, 0, 0));
-    };
-    // everything the chunk needs is requested before the first product
-    u32x2 col[CHUNK_WAVES], row[CHUNK_WAVES];
-#pragma unroll
-    for (int w = 0; w < CHUNK_WAVES; ++w) {
-        col[w] = row[w] = u32x2{0, 0};
-        if (w >= waves)
-            continue;
-        col[w] = cols[size_t(first + w) * col_stride + lane];
-        if (vocabulary < 0) {
-            row[w] = rows[size_t(first + w) * row_stride + lane];
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = 4 * j + g, token = (first + w) * m.per_wave + t; // rows beyond the last token are zero: any id will do
-                row[w].x |= uint32_t(t < m.per_wave && token < m.tokens ? x[token] : 0) << (8 * j);
-            }
-        }
-    }
-#pragma unroll
-    for (int w = 0; w < CHUNK_WAVES; ++w) {
-        f32x4 by_row;
-        if (vocabulary < 0)
-            by_row = by_token(row[w]);
-        else
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                by_row[j] = int((row[w].x >> (8 * j)) & 255u) == vocabulary ? 1.f : 0.f;
-        acc = multiply(by_row, by_token(col[w]), acc);
-    }
-    // The products with the identity and the one-hot matrix are exact for finite rows alone: 0 times an infinity is NaN,
-    // in features and ids that have no part in it.  A wave whose sums are not finite takes them again with the rows
-    // turned by moving them; no other wave pays for it.
-    const auto finite = [](float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; };
-    if (__builtin_amdgcn_ballot_w64(!(finite(acc[0]) && finite(acc[1]) && finite(acc[2]) && finite(acc[3])))) {
-        const auto moved = [&](const u32x2 &tile, int token) { // feature c of `token`, out of lane 16 (c % 4) + token
-            const int from = 16 * (c & 3) + token;
-            const uint32_t low = uint32_t(__shfl(int(tile.x), from, 64)), high = uint32_t(__shfl(int(tile.y), from, 64));
-            const uint32_t pair = c & 8 ? high : low;
-            return __uint_as_float(c & 4 ? pair & 0xffff0000u : pair << 16);
-        };
-        acc = ZERO;
-#pragma unroll 1
-        for (int w = 0; w < waves; ++w) {
-            u32x2 this_col = col[0], this_row = row[0];
-#pragma unroll
-            for (int k = 1; k < CHUNK_WAVES; ++k)
-                this_col = k == w ? col[k] : this_col, this_row = k == w ? row[k] : this_row;
-            if (vocabulary < 0) {
-                f32x4 a, b;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    a[j] = moved(this_row, 4 * j + g), b[j] = moved(this_col, 4 * j + g);
-                acc = multiply(a, b, acc);
-                continue;
-            }
-            for (int t = 0; t < m.per_wave; ++t) {
-                const float value = moved(this_col, t);
-                const int id = int(uint32_t(__shfl(int(this_row.x), 16 * (t & 3), 64)) >> (8 * (t >> 2)) & 255u);
-                const int mine = id - (vocabulary - c + 4 * g); // the register of this lane that is the id's, if it is one of four
-                if ((first + w) * m.per_wave + t < m.tokens)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        acc[r] = mine == r ? acc[r] + value : acc[r];
-            }
-        }
-    }
+// A block sums what one layer (or the head, or the embedding) has of a chunk's tokens, in token order: partial[chunk].  Its
+// rows come to LDS as the waves kept them; the transposing load then gives lane 16 q + i feature 4 (i % 4) + i / 4 of tokens
+// 4 j + q, an operand of the fp32 instruction whose steps run over the tokens.  That moves data and computes nothing: an
+// infinity stays in its own feature.  A wave has three or four tiles of the gradient at a time, whose chains of dependent
+// instructions fill the matrix pipe, which bounds the kernel together with what the rows take on their way (half of them
+// are worked on while the others come): 93 tiles of 32 instructions a chunk at depth 4.  2560 sequences of 4 there: 15.3 us
+// with a wave for each tile that loaded its rows and turned them with the identity matrix, 13.1 so; 16 of 8 at depth 8 7.7 and 7.9.
+constexpr int HEAD_ROWS = 17; // the head's tiles of a wave in LDS: dlogits, and the normalised rows
+constexpr size_t GRADIENT_LDS = size_t(CHUNK_WAVES) * OPERANDS * 512;
+static_assert(HEAD_ROWS <= OPERANDS, "the head's rows fit a layer's");
+// a lane's rows 4 r + g and column 4 (c % 4) + c / 4 of a gradient tile
+TG_DEVICE void store_tile(float *out, const f32x4 &sum, int width, int lane) {
+    const int g = lane >> 4, column = feed_row(lane & 15);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        out[(4 * g + r) * width + c] = acc[r];
+        out[(4 * r + g) * width + column] = sum[r];
 }
-// gradient = the chunks' sums in chunk order; a block's 1024 elements also leave the sum of their squares in norms[block].
+// the g * z terms of a norm's scale: token 4 j + g of every wave, feature c
+struct ScaleTerms {
+    float v[CHUNK_WAVES][4];
+    TG_DEVICE void request(const Workspace &s, int norm, int first, int waves, int lane) {
+        const float *gz = s.gz + (size_t(norm) * s.waves + first) * 16 * W + lane;
+#pragma unroll
+        for (int w = 0; w < CHUNK_WAVES; ++w)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[w][j] = w < waves ? gz[(w * 4 + j) * 64] : 0.f;
+    }
+};
+// TILES chains of products over the tokens of half a chunk's waves, and with SCALE one of a row of ones times the terms.
+// `rows` and `columns`: this lane's place in the first wave's tiles; a wave's are `stride` (columns: `column_stride`) bytes.
+template <int TILES, bool SCALE>
+TG_DEVICE void add_half(f32x4 (&sum)[4], const unsigned char *const (&rows)[TILES], const unsigned char *const (&columns)[TILES], int stride,
+                        int column_stride, const ScaleTerms &terms, int half) {
+#pragma unroll
+    for (int k = 0; k < CHUNK_WAVES / 2; ++k) {
+        const int w = half * (CHUNK_WAVES / 2) + k;
+        f32x4 a[TILES], b[TILES];
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+            a[n] = unpack4(read_across(rows[n] + w * stride)), b[n] = unpack4(read_across(columns[n] + w * column_stride));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int n = 0; n < TILES; ++n)
+                sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][j], b[n][j], sum[n], 0, 0, 0);
+            if constexpr (SCALE)
+                sum[TILES] = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], sum[TILES], 0, 0, 0);
+        }
+    }
+}
+__global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m, const uint8_t *__restrict__ x, Workspace s,
+                                                                       int parameters) {
+    extern __shared__ __align__(16) unsigned char memory[];
+    // consecutive blocks sit on consecutive XCDs: block 8 i + k takes the i-th unit of XCD k's chunks
+    const int units = m.depth + 2, chunk = (blockIdx.x >> 3) / units * 8 + (blockIdx.x & 7), unit = (blockIdx.x >> 3) % units;
+    if (chunk >= s.chunks)
+        return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+    const int first = chunk * CHUNK_WAVES, waves = min(CHUNK_WAVES, s.waves - first);
+    float *out = s.partials + size_t(chunk) * parameters;
+    const uint32_t lds = lds_address(memory);
+    // TILES tiles of every wave, `apart` bytes from one wave to the next in memory, one behind another in LDS; 16 bytes a lane.
+    // The last chunk's missing waves are zeros.
+    const auto copy = [&](auto tiles, const u32x2 *source, int apart, int to) {
+        constexpr int PIECES = decltype(tiles)::value * 32;
+        static_assert(CHUNK_WAVES * PIECES % (WAVES * 64) == 0, "every wave has as many copies");
+#pragma unroll
+        for (int i = 0; i < CHUNK_WAVES * PIECES / (WAVES * 64); ++i) {
+            const int base = (i * WAVES + wave) * 64, piece = base + lane, w = piece / PIECES;
+            if (w < waves)
+                async_copy16(lds + uint32_t(to + base * 16), source, uint32_t(w * apart + (piece - w * PIECES) * 16));
+            else
+                *reinterpret_cast<u32x4 *>(memory + to + piece * 16) = u32x4{0, 0, 0, 0};
+        }
+    };
+    const auto half_there = [&]() { // all but a wave's last eight copies; a chunk that is not full has fewer
+        if (waves == CHUNK_WAVES)
+            wait_vmcnt<8>();
+        else
+            wait_vmcnt<0>();
+        wait_lgkmcnt0();
+        __syncthreads();
+    };
+    const unsigned char *mine = memory + across_offset(lane, true);
+    const auto tile = [&](int n) { return mine + n * 512; };
+    f32x4 sum[4] = {ZERO, ZERO, ZERO, ZERO};
+    ScaleTerms terms;
+    if (unit < m.depth) {
+        const Layer q = layer_layout(unit);
+        // waves 1 and 2 have a norm's scale besides gate and up
+        if (wave == 1 || wave == 2)
+            terms.request(s, 2 * unit + wave - 1, first, waves, lane);
+        copy(std::integral_constant<int, OPERANDS>{}, s.tiles + ((size_t(unit) * s.waves + first) * TILES + T_OPERANDS) * 64, TILES * 512, 0);
+        constexpr int N1 = T_N1 - T_OPERANDS, A = T_A - T_OPERANDS, N2 = T_N2 - T_OPERANDS, ACT = T_ACT - T_OPERANDS,
+                      DQKV = T_DQKV - T_OPERANDS, DH_ATTENTION = T_DH_ATTENTION - T_OPERANDS, DGU = T_DGU - T_OPERANDS,
+                      DH_DOWN = T_DH_DOWN - T_OPERANDS, STRIDE = OPERANDS * 512;
+        const auto layer = [&](int half) {
+            if (wave == 0)
+                add_half<4, false>(sum, {tile(DQKV), tile(DQKV + 1), tile(DQKV + 2), tile(DH_ATTENTION)}, {tile(N1), tile(N1), tile(N1), tile(A)},
+                                   STRIDE, STRIDE, terms, half);
+            else if (wave == 3)
+                add_half<3, false>(sum, {tile(DH_DOWN), tile(DH_DOWN), tile(DH_DOWN)}, {tile(ACT), tile(ACT + 1), tile(ACT + 2)}, STRIDE, STRIDE,
+                                   terms, half);
+            else
+                add_half<3, true>(sum, {tile(DGU + 3 * wave - 3), tile(DGU + 3 * wave - 2), tile(DGU + 3 * wave - 1)}, {tile(N2), tile(N2), tile(N2)},
+                                  STRIDE, STRIDE, terms, half);
+        };
+        half_there(); // brought by nine of a wave's seventeen copies
+        layer(0);
+        wait_vmcnt<0>();
+        __syncthreads();
+        layer(1);
+        if (wave == 0) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) // the attention projection lies behind q, k, v
+                store_tile(out + q.qkv + t * 256, sum[t], W, lane);
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            store_tile(wave == 3 ? out + q.down + t * 16 : out + q.gate + ((wave - 1) * 3 + t) * 256, sum[t], wave == 3 ? F : W, lane);
+        if (wave < 3 && g == 0)
+            out[(wave == 1 ? q.attention_norm : q.mlp_norm) + c] = sum[3][0];
+        return;
+    }
+    if (unit == m.depth) { // the head: a wave four tiles of logits
+        constexpr int NF = CHUNK_WAVES * 16;
+        copy(std::integral_constant<int, 1>{}, s.nf + size_t(first) * 64, 512, NF * 512);
+        copy(std::integral_constant<int, 16>{}, s.dlogits + size_t(first) * 16 * 64, 16 * 512, 0);
+        const auto head = [&](int half) {
+            add_half<4, false>(sum, {tile(wave * 4), tile(wave * 4 + 1), tile(wave * 4 + 2), tile(wave * 4 + 3)},
+                               {tile(NF), tile(NF), tile(NF), tile(NF)}, 16 * 512, 512, terms, half);
+        };
+        half_there(); // eight of the sixteen
+        head(0);
+        wait_vmcnt<0>();
+        __syncthreads();
+        head(1);
+        const int at = V * W + m.depth * LAYER_SIZE + W;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            store_tile(out + at + (wave * 4 + t) * 256, sum[t], W, lane);
+        if (wave == 0) {
+            terms.request(s, 2 * m.depth, first, waves, lane);
+            f32x4 scale = ZERO;
+#pragma unroll
+            for (int w = 0; w < CHUNK_WAVES; ++w)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    scale = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], scale, 0, 0, 0);
+            if (g == 0)
+                out[at - W + c] = scale[0];
+        }
+        return;
+    }
+    // The embedding's rows: the one-hot matrix of the tokens times the gradient.  0 times an infinity is NaN, in ids that have
+    // no part in it, so where a row is not finite the rows are added one by one.
+    copy(std::integral_constant<int, 1>{}, s.dh + size_t(first) * 64, 512, 0);
+    uint32_t ids[CHUNK_WAVES];
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        ids[w] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = 4 * j + g, token = (first + w) * m.per_wave + t; // rows beyond the last token are zero: any id will do
+            ids[w] |= uint32_t(w < waves && t < m.per_wave && token < m.tokens ? x[token] : 0) << (8 * j);
+        }
+    }
+    wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    __syncthreads();
+    const int vocabulary = wave * 64; // of the four tiles' first id
+    bool extreme = false;
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        const u32x2 row = read_across(tile(w));
+        const auto either = [](uint32_t two) { return (two & 0x7f80u) == 0x7f80u || (two & 0x7f800000u) == 0x7f800000u; };
+        extreme = extreme || either(row.x) || either(row.y);
+        const f32x4 b = unpack4(row);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(int((ids[w] >> (8 * j)) & 255u) == vocabulary + t * 16 + c ? 1.f : 0.f, b[j],
+                                                              sum[t], 0, 0, 0);
+    }
+    if (__builtin_amdgcn_ballot_w64(extreme)) {
+        sum[0] = sum[1] = sum[2] = sum[3] = ZERO;
+#pragma unroll 1
+        for (int w = 0; w < waves; ++w)
+#pragma unroll 1
+            for (int t = 0; t < m.per_wave; ++t) {
+                const int token = (first + w) * m.per_wave + t;
+                if (token >= m.tokens)
+                    break;
+                // column 4 (c % 4) + c / 4 is element c % 4 of item (c / 4, t)
+                const float value = bf16_to_float(reinterpret_cast<const bf16_t *>(memory)[(w * 64 + 16 * (c >> 2) + t) * 4 + (c & 3)]);
+                const int id = int(x[token]) - vocabulary - 4 * g;
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        sum[n][r] = id == 16 * n + r ? sum[n][r] + value : sum[n][r];
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) // the ids are in their own order
+            out[(vocabulary + t * 16 + 4 * g + r) * W + feed_row(c)] = sum[t][r];
+}
+// gradient = the chunks' sums in chunk order, an element a thread, whose loads are in flight together: 80 chunks of 21648
+// parameters took 5.9 us with four elements a thread on a quarter of the blocks and sixteen loads at a time, 5.2 so.
+// Where `norms` is given, four blocks leave the parts of one sum of squares, of 1024 elements (FOLD_QUARTERS).
 // Blocks beyond the parameters average the losses: one a position, in double (cuda/trainer.cuh:79-100).
-int fold_blocks(int parameters) { return (parameters + 1023) / 1024; }
+constexpr int FOLD_QUARTERS = 4;
+int fold_blocks(int parameters) { return (parameters + 1023) / 1024 * FOLD_QUARTERS; }
 __global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
                                                        float *__restrict__ gradient, float *__restrict__ norms, int blocks,
                                                        const float *__restrict__ token_losses, int batch, int context,
@@ -797,18 +1004,31 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__
             means[position] = float(((sums[0] + sums[1]) + (sums[2] + sums[3])) / batch);
         return;
     }
-    __shared__ float waves[4];
-    const int at = (blockIdx.x * 256 + threadIdx.x) * 4;
-    f32x4 sum = ZERO;
+    __shared__ __align__(16) float row[256];
+    constexpr int AT_ONCE = 40;
+    const int at = blockIdx.x * 256 + threadIdx.x;
+    float sum = 0.f;
     if (at < parameters) {
         const float *from = partials + at;
-#pragma unroll 16
-        for (int c = 0; c < chunks; ++c)
-            sum += *reinterpret_cast<const f32x4 *>(from + size_t(c) * parameters);
-        *reinterpret_cast<f32x4 *>(gradient + at) = sum;
+        for (int c = 0; c < chunks; c += AT_ONCE) {
+            float v[AT_ONCE];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (c + i < chunks)
+                    v[i] = from[size_t(c + i) * parameters];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (c + i < chunks)
+                    sum += v[i];
+        }
+        gradient[at] = sum;
     }
-    if (norms) {
-        const float squares = block_sum_256(0.f + quad_squares(sum), waves);
+    if (!norms)
+        return;
+    row[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const float squares = wave_sum(0.f + quad_squares(reinterpret_cast<const f32x4 *>(row)[threadIdx.x]));
         if (threadIdx.x == 0)
             norms[blockIdx.x] = squares;
     }
@@ -824,13 +1044,20 @@ struct Update {
     W16Weights from, to;
     float *momentum, *variance;
     const float *gradient, *norms;
-    int norm_count, depth;
+    int norm_count, norm_parts, depth; // norms: norm_count sums of norm_parts partial sums each, 1 or FOLD_QUARTERS
     AdamArgs adam;
     MuonArgs muon;
 };
-TG_DEVICE float difference(float a, float b) { // of two rounded values: a product in b is not fused into it
-#pragma clang fp contract(off)
-    return a - b;
+// clip_factor of the norms, with the sums of a fold's quarters formed first
+TG_DEVICE float clip_factor(const Update &u, float *waves) {
+    if (u.norm_parts == 1 || !(u.adam.clip > 0.f))
+        return ::clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+    float sum = 0.f;
+    for (int i = threadIdx.x; i < u.norm_count; i += 256) {
+        const f32x4 part = *reinterpret_cast<const f32x4 *>(u.norms + i * FOLD_QUARTERS);
+        sum += (part[0] + part[1]) + (part[2] + part[3]);
+    }
+    return fminf(1.f, u.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
 }
 TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
     __shared__ float wide[2][16 * F];
@@ -849,7 +1076,7 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
         const bool mine = tid + 256 * k < size;
         g[k] = mine ? u.gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f, w[k] = mine ? master(u.from.hi, u.from.lo, i) : 0.f;
     }
-    const float clip = clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+    const float clip = clip_factor(u, waves);
     float squares = 0.f, b[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -857,7 +1084,7 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
             const float gs = g[k] * clip;
             const float next = fmaf(1.f - u.muon.momentum, fmaf(g[k], clip, -m[k]), m[k]);
             u.momentum[weight + tid + 256 * k] = next;
-            b[k] = round_bf16(fmaf(u.muon.momentum, difference(next, gs), gs));
+            b[k] = round_bf16(fmaf(u.muon.momentum, next - gs, gs));
             squares = fmaf(b[k], b[k], squares);
         }
     const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
@@ -916,7 +1143,7 @@ __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
     __shared__ float waves[4];
     if (int(blockIdx.x) < 5 * u.depth)
         return muon_matrix(u, blockIdx.x, waves);
-    const float scale = clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+    const float scale = clip_factor(u, waves);
     // quads: the embedding's 1024, four for each scale, the head's 1024 (the only ones that decay)
     const int quad = (blockIdx.x - 5 * u.depth) * 256 + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
     int at = quad * 4;
@@ -965,21 +1192,27 @@ extern "C" size_t tgk_w16_workspace(int depth, int batch, int context) {
 }
 
 namespace {
-void launch_forward(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, const uint8_t *y,
-                    const W16Data &data, uint8_t *sampled, float *token_losses, float *logits, int with_gradient) {
-    hipLaunchKernelGGL(w16_forward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(m.depth), stream, m, x, y, data,
-                       sampled, r, token_losses, logits, with_gradient);
-    check_hip(hipGetLastError(), "w16_forward launch: ");
+// the kernels' LDS beyond 64 KiB is a per-device attribute
+template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&configured)[64], size_t bytes) {
+    int device = 0;
+    check_hip(hipGetDevice(&device));
+    require(device >= 0 && device < 64, "w16: device index out of range");
+    if (configured[device].load(std::memory_order_acquire))
+        return;
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)),
+              "w16 LDS size: ");
+    configured[device].store(true, std::memory_order_release);
 }
-void launch_backward(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, float *gradient, float *norms,
-                     const float *token_losses, float *means) {
+void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, float *gradient, float *norms,
+                             const float *token_losses, float *means) {
     const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
-    hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(m.depth), stream, m, r);
-    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((gradient_jobs(m.depth) + 3) / 4 * ((r.chunks + 7) / 8 * 8)), dim3(256), 0, stream, m, x,
-                       r, parameters);
+    static std::atomic<bool> configured[64];
+    allow_lds(w16_weight_gradient_kernel, configured, GRADIENT_LDS);
+    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((m.depth + 2) * ((r.chunks + 7) / 8 * 8)), dim3(64 * WAVES), GRADIENT_LDS, stream, m,
+                       x, r, parameters);
     hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (means ? m.context : 0)), dim3(256), 0, stream, r.partials, r.chunks,
                        parameters, gradient, norms, blocks, token_losses, m.tokens / m.context, m.context, means);
-    check_hip(hipGetLastError(), "w16_backward launch: ");
+    check_hip(hipGetLastError(), "w16 weight gradient launch: ");
 }
 } // namespace
 
@@ -990,8 +1223,13 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && y && workspace && token_losses, "w16_forward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
-        launch_forward(stream, make_model(depth, batch, context, weight_hi, weight_lo), carve(depth, batch, context, workspace),
-                       x, y, W16Data{}, nullptr, token_losses, logits, with_gradient);
+        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
+        const Workspace r = carve(depth, batch, context, workspace);
+        static std::atomic<bool> configured[2][64];
+        const auto kernel = with_gradient ? w16_forward_kernel<true> : w16_forward_kernel<false>;
+        allow_lds(kernel, configured[with_gradient != 0], staged_bytes(MAX_DEPTH));
+        hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, x, y, r, token_losses, logits);
+        check_hip(hipGetLastError(), "w16_forward launch: ");
     });
 }
 
@@ -1001,24 +1239,39 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && workspace && gradient, "w16_backward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
-        launch_backward(stream, make_model(depth, batch, context, weight_hi, weight_lo), carve(depth, batch, context, workspace),
-                        x, gradient, nullptr, nullptr, nullptr);
+        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
+        const Workspace r = carve(depth, batch, context, workspace);
+        static std::atomic<bool> configured[64];
+        allow_lds(w16_backward_kernel, configured, staged_bytes(MAX_DEPTH));
+        hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
+        check_hip(hipGetLastError(), "w16_backward launch: ");
+        launch_weight_gradients(stream, m, r, x, gradient, nullptr, nullptr, nullptr);
     });
 }
 
 int w16_norm_count(int depth) {
-    return fold_blocks(make_layout(depth).count);
+    return fold_blocks(make_layout(depth).count) / FOLD_QUARTERS;
+}
+int w16_norm_parts() {
+    return FOLD_QUARTERS;
 }
 void w16_gradient(hipStream_t stream, int depth, int batch, int context, const W16Weights &weights, const W16Data &data,
                   uint8_t *tokens, void *workspace, float *token_losses, float *means, float *gradient, float *norms) {
+    require(context == 4 || context == 8, "w16: a training step has a context of 4 or 8");
     const Model m = make_model(depth, batch, context, weights.hi, weights.lo);
     const Workspace r = carve(depth, batch, context, workspace);
-    launch_forward(stream, m, r, nullptr, nullptr, data, tokens, token_losses, nullptr, 1);
-    launch_backward(stream, m, r, tokens, gradient, norms, token_losses, means);
+    static std::atomic<bool> configured[2][64];
+    const auto kernel = context == 4 ? w16_step_kernel<4> : w16_step_kernel<8>;
+    allow_lds(kernel, configured[context == 8], staged_bytes(MAX_DEPTH));
+    const uint64_t places = uint64_t(data.size) - 8, inverse = places > 1 ? uint64_t((static_cast<unsigned __int128>(1) << 64) / places) : ~uint64_t(0);
+    hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, data, inverse, tokens, r, token_losses);
+    check_hip(hipGetLastError(), "w16_step launch: ");
+    launch_weight_gradients(stream, m, r, tokens, gradient, norms, token_losses, means);
 }
 void w16_update(hipStream_t stream, int depth, const W16Weights &from, const W16Weights &to, float *momentum, float *variance,
-                const float *gradient, const float *norms, int norm_count, const AdamArgs &adam, const MuonArgs &muon) {
-    const Update u{from, to, momentum, variance, gradient, norms, norm_count, depth, adam, muon};
+                const float *gradient, const float *norms, int norm_count, int norm_parts, const AdamArgs &adam,
+                const MuonArgs &muon) {
+    const Update u{from, to, momentum, variance, gradient, norms, norm_count, norm_parts, depth, adam, muon};
     hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth + adam_blocks(depth)), dim3(256), 0, stream, u);
     check_hip(hipGetLastError(), "w16_update launch: ");
 }
@@ -1034,7 +1287,7 @@ extern "C" int tgk_w16_muon(hipStream_t stream, int depth, uint16_t *weight_hi, 
         AdamArgs adam{};
         adam.clip = clip;
         const W16Weights weights{weight_hi, weight_lo};
-        const Update u{weights, weights, momentum, nullptr, gradient, norm_partials, norm_count, depth, adam,
+        const Update u{weights, weights, momentum, nullptr, gradient, norm_partials, norm_count, 1, depth, adam,
                        MuonArgs{lr, momentum_rate, weight_decay, ns_steps}};
         hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth), dim3(256), 0, stream, u); // the matrices' blocks alone
         check_hip(hipGetLastError(), "w16_muon launch: ");
