@@ -69,7 +69,7 @@ StepRates onecycle_point(const OneCycle &s, int step) {
 
 // Everything one batch in flight owns: its stream, its tokens, its saved activations and its gradient.
 // Slot 0 is on the engine's stream (a synchronous engine has no other); inflight = K gives K slots on K streams
-// (the worker teams of cuda/pipeline.cuh:52-92).
+// (the worker teams of cuda/pipeline.cuh:52-92), of the width-16 network on the engine's.
 struct Slot {
     hipStream_t stream = nullptr;
     uint8_t *input = nullptr, *target = nullptr;
@@ -368,6 +368,26 @@ struct Engine {
             OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
     }
 
+    // learning rates and momenta of optimizer step `at` (0-based)
+    struct Rates {
+        float lr, beta1, muon_lr, muon_momentum;
+    };
+    Rates rates(uint64_t at) const {
+        const Config &c = config.base;
+        if (schedule.empty())
+            return {c.learning_rate, c.beta1, c.muon_lr, c.momentum};
+        // cuda/optim.cuh:81-88: one point drives both learning rates and both momenta
+        const StepRates &point = schedule[at];
+        return {c.learning_rate * point.multiplier, point.momentum, c.muon_lr * point.multiplier, point.momentum};
+    }
+    W16Step w16_step(uint64_t at, const float *gradient, const float *norms, const Version &now, const Version &to) const {
+        const Config &c = config.base;
+        const Rates r = rates(at);
+        return {{now.hi, now.lo}, {to.hi, to.lo}, gradient, norms,
+                adam_args(r.lr, r.beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at),
+                {r.muon_lr, r.muon_momentum, c.weight_decay, c.ns_steps}};
+    }
+
     // cuda/optim.cuh:66-106 for optimizer step `at` (0-based), on `stream`: gradient -> the weights of version `to`, from
     // the previous version's, `now`.
     // `from`: the slot whose backward pass has just written `gradient`, when it left the sums of squares with it
@@ -375,31 +395,24 @@ struct Engine {
                   const Slot *from = nullptr) {
         const Config &c = config.base;
         uint16_t *weight_hi = to.hi, *weight_lo = to.lo, *weight_t = to.t;
-        float lr = c.learning_rate, beta1 = c.beta1, muon_lr = c.muon_lr, muon_momentum = c.momentum;
-        if (!schedule.empty()) { // cuda/optim.cuh:81-88: one point drives both learning rates and both momenta
-            lr *= schedule[at].multiplier;
-            muon_lr *= schedule[at].multiplier;
-            beta1 = muon_momentum = schedule[at].momentum;
-        }
         const bool fused = from && from->norms;
         if (c.clip > 0 && !fused)
             OP(TG_CLASS_OPTIMIZER, tgk_sumsq_partials(stream, gradient, size_t(layout.count), norm_partials, NormPartials));
         const float *norms = fused ? from->norms : norm_partials;
         const int norm_count = fused ? from->list_norms + from->range_norms : NormPartials;
         if (width16) { // AdamW's tensors and the hidden matrices (cuda/optim.cuh:92-118)
-            Scope profile_scope(this, TG_CLASS_OPTIMIZER);
-            w16_update(stream, c.depth, {now.hi, now.lo}, {to.hi, to.lo}, momentum, variance, gradient, norms, norm_count,
-                       fused ? w16_norm_parts() : 1, adam_args(lr, beta1, c.beta2, c.epsilon, c.weight_decay, c.clip, at),
-                       {muon_lr, muon_momentum, c.weight_decay, c.ns_steps});
+            const W16Step step = w16_step(at, gradient, norms, now, to);
+            w16_updates(stream, c.depth, momentum, variance, norm_count, 1, 1, &step);
             return;
         }
+        const Rates r = rates(at);
         if (&now != &to) {
             const size_t bytes = size_t(layout.count) * 2;
             check_hip(hipMemcpyAsync(to.hi, now.hi, bytes, hipMemcpyDeviceToDevice, stream));
             check_hip(hipMemcpyAsync(to.lo, now.lo, bytes, hipMemcpyDeviceToDevice, stream));
         }
         OP(TG_CLASS_OPTIMIZER, tgk_adamw(stream, size_t(layout.count), weight_hi, weight_lo, momentum, variance, gradient,
-                     norms, norm_count, segment_starts, segment_flags, segments, lr, beta1, c.beta2, c.epsilon, c.weight_decay,
+                     norms, norm_count, segment_starts, segment_flags, segments, r.lr, r.beta1, c.beta2, c.epsilon, c.weight_decay,
                      c.clip, at));
         OP(TG_CLASS_OPTIMIZER, tgk_transpose_batch(stream, weight_hi, weight_t, transpose_jobs, transpose_count,
                                                    transpose_tiles));
@@ -408,27 +421,50 @@ struct Engine {
     void batch_gradient(Slot &s, const Version &v, uint64_t at) {
         const Config &c = config.base;
         hipStream_t stream = s.stream;
-        if (width16) {
-            Scope profile_scope(this, TG_CLASS_OTHER);
-            w16_gradient(stream, c.depth, c.batch, c.context, {v.hi, v.lo}, {data, data_size, c.seed, at}, s.input, s.workspace,
-                         s.token_losses, history_row(at), s.gradient, s.norms);
-            return;
-        }
         OP(TG_CLASS_OTHER, sample_embed(stream, data, data_size, c.seed, at, c.batch, c.context, config.d_model, s.input, s.target,
                                         v.hi + layout.embedding, v.hi + layout.positions, s.x[0]));
         forward(s, v, true, nullptr, c.batch, false, true);
         backward(s, v, history_row(at));
     }
-    // One training step.  Synchronous engine: everything in order on the one stream, weights updated in place
+    // Training steps of the width-16 network from `at` on, as many as share their launches: at most as many as are in flight.
+    // Batch s reads the weights of version max(floor, s - K + 1), which are there for all of them before the first of their
+    // optimizer steps, and those follow one another.  The order is that of the wide model's streams below; what it saves is
+    // launches, events and the host's time for them, which bounded small batches.  Microseconds a step on K streams and
+    // so: depth 8, context 8, 16 sequences, K = 4: 46 to 54 and 26; depth 4, context 4, 16 sequences, K = 8: 32 to 36 and 12;
+    // depth 8, context 8, 1280 sequences, K = 4: 76 and 68.
+    int train_width16(uint64_t at, int most, int *trace) {
+        const Config &c = config.base;
+        const uint64_t K = slots.size(), ring = versions.size();
+        const int count = int(std::min<uint64_t>(K, uint64_t(most)));
+        W16Batch batches[MaxInFlight];
+        W16Step steps[MaxInFlight];
+        for (int i = 0; i < count; ++i) {
+            const uint64_t step = at + uint64_t(i), read = K == 1 ? step : std::max(floor, step + 1 >= K ? step + 1 - K : 0);
+            const Slot &s = slots[step % K];
+            const Version &v = versions[read % ring];
+            batches[i] = {{v.hi, v.lo}, step, s.input, s.workspace, s.token_losses, history_row(step), s.gradient, s.norms};
+            steps[i] = w16_step(step, s.gradient, s.norms, versions[step % ring], versions[(step + 1) % ring]);
+            trace[i] = int(read);
+            total_staleness += step - read;
+            max_staleness = std::max(max_staleness, int(step - read));
+        }
+        {
+            Scope profile_scope(this, TG_CLASS_OTHER);
+            w16_gradients(stream, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, batches);
+        }
+        Scope profile_scope(this, TG_CLASS_OPTIMIZER);
+        w16_updates(stream, c.depth, momentum, variance, slots[0].list_norms, w16_norm_parts(), count, steps);
+        return count;
+    }
+    // One training step of the wide model.  Synchronous engine: everything in order on the one stream, weights updated in place
     // (cuda/trainer.cuh:109-124).  inflight = K (cuda/pipeline.cuh:40-126 as streams and events): batch `at` and its
     // optimizer step run on the stream of slot at % K, behind optimizer step at - K.  That order alone lets the batch
     // read max(floor, at - K + 1), the oldest version the ring still guarantees, and frees the slot's gradient.  The
     // optimizer step waits for its predecessor, on another slot's stream; the version that it overwrites, at - K, was
     // last read by batch at - 1, which that predecessor follows.  Optimizer steps on a stream of their own (K + 1
-    // streams) cost two more events a step and shared one of the process's four hardware queues with a slot at K = 4: long
-    // runs of the width-16 network of depth 8, context 8, batch 16 took 54 us a step, now 36 to 40 (16 steps and the weights
-    // to the host 0.73 ms).  The choice is made on the host, so a run is reproducible; the staleness bound at - K + 1 <=
-    // version <= at is the reference's.
+    // streams) cost two more events a step and shared one of the process's four hardware queues with a slot at K = 4.  The
+    // choice is made on the host, so a run is reproducible; the staleness bound at - K + 1 <= version <= at is the
+    // reference's.
     void train_step(uint64_t at, int *trace) {
         const uint64_t K = slots.size(), ring = versions.size();
         if (K == 1) {
@@ -448,6 +484,13 @@ struct Engine {
         *trace = int(read);
         total_staleness += at - read;
         max_staleness = std::max(max_staleness, int(at - read));
+    }
+    // the next steps, at most `most`; returns how many
+    int train_some(uint64_t at, int most, int *trace) {
+        if (width16)
+            return train_width16(at, most, trace);
+        train_step(at, trace);
+        return 1;
     }
 };
 
@@ -482,7 +525,7 @@ void build_slots(Engine *e, int inflight, bool transposed_copies) {
     e->slots.resize(size_t(inflight));
     e->versions.resize(inflight > 1 ? size_t(inflight) + 1 : 1);
     for (Slot &slot : e->slots) {
-        if (&slot == &e->slots[0])
+        if (&slot == &e->slots[0] || e->width16) // the width-16 network's batches share their launches
             slot.stream = e->stream;
         else
             check_hip(hipStreamCreate(&slot.stream)); // default priority
@@ -496,7 +539,7 @@ void build_slots(Engine *e, int inflight, bool transposed_copies) {
         e->allocate(version.lo, P);
         if (transposed_copies)
             e->allocate(version.t, P);
-        if (inflight > 1)
+        if (inflight > 1 && !e->width16)
             check_hip(hipEventCreateWithFlags(&version.done, hipEventDisableTiming));
     }
 }
@@ -964,8 +1007,8 @@ TG_API int tg_train(Engine *e, int steps) {
             throw std::runtime_error("Training would exceed the OneCycle schedule");
         e->use_device();
         e->version_trace.assign(size_t(steps), 0);
-        for (int i = 0; i < steps; ++i)
-            e->train_step(e->step + uint64_t(i), &e->version_trace[size_t(i)]);
+        for (int i = 0; i < steps;)
+            i += e->train_some(e->step + uint64_t(i), steps - i, &e->version_trace[size_t(i)]);
         e->last_train_steps = steps, e->last_train_first = e->step;
         e->step += uint64_t(steps);
     });
@@ -1090,7 +1133,7 @@ TG_API int tg_profile_step(Engine *e, float *class_ms, int *class_launches, int 
         e->version_trace.assign(1, 0);
         e->profiling = true;
         try {
-            e->train_step(e->step, e->version_trace.data());
+            e->train_some(e->step, 1, e->version_trace.data());
         } catch (...) {
             e->profiling = false;
             throw;

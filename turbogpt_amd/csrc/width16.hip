@@ -84,6 +84,12 @@ struct Workspace {
     int waves, blocks, chunks;
     size_t bytes;
 };
+// another batch's, whose memory lies `apart` bytes further on
+TG_DEVICE Workspace moved(Workspace s, int64_t apart) {
+    const auto move = [&](auto *&p) { p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<char *>(p) + apart); };
+    move(s.tiles), move(s.words), move(s.gz), move(s.hidden), move(s.nf), move(s.dh), move(s.inverse), move(s.dlogits), move(s.partials);
+    return s;
+}
 int tokens_per_wave(int context) { return 16 / context * context; }
 Workspace carve(int depth, int batch, int context, void *base) {
     Workspace r{};
@@ -418,6 +424,14 @@ TG_DEVICE f32x4 rotate_back(f32x4 v, float c, float s) {
     return v;
 }
 
+// Batches that share a launch: grid row y is member y's.  The members' workspaces are alike.
+struct Group {
+    W16Batch member[W16_BATCHES];
+    TG_DEVICE Workspace workspace(const Workspace &first, int y) const {
+        return moved(first, static_cast<const char *>(member[y].workspace) - static_cast<const char *>(member[0].workspace));
+    }
+};
+
 // ---- forward ---------------------------------------------------------------------------------------
 // What the head leaves for the backward pass; the logits' gradients in tiles of sixteen.
 struct Head {
@@ -731,11 +745,14 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
 // and the weights are staged once.  Depth 4, 2560 sequences of 4: 53.0 us as two launches that staged eight tiles at a time,
 // 38.8 so; depth 8, 16 of 8: 79.3 and 62.6.  Two waves a SIMD, which batches of more than 256 blocks need (10000 of 8 at depth 8
 // 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training bytes, every sequence a window at a
-// hashed place (cuda/dataset.cuh:13-27); the tokens are left in `sampled` for the embedding's gradient.
+// hashed place (cuda/dataset.cuh:13-27); the tokens are left for the embedding's gradient.
 template <int CONTEXT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(Model m, W16Data data, uint64_t inverse, uint8_t *__restrict__ sampled,
-                                                               Workspace s, float *__restrict__ token_losses) {
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(Model m, W16Data data, uint64_t inverse, Workspace first,
+                                                                                                      Group group) {
     extern __shared__ __align__(16) unsigned char memory[];
+    const W16Batch &batch = group.member[blockIdx.y];
+    const Workspace s = group.workspace(first, blockIdx.y);
+    m.hi = batch.weights.hi, m.lo = batch.weights.lo;
     const Lane p = lane_of(m);
     const Staged weight(m, memory, p);
     Staging staging(m, memory);
@@ -743,7 +760,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     if (p.live) {
         const int sequence = p.token / CONTEXT;
         // the hash modulo the places: `inverse` is 2^64 / places rounded down, so the quotient is at most one too small
-        const uint64_t hash = hash_u64(data.seed + data.step * uint64_t(m.tokens / CONTEXT) + uint64_t(sequence));
+        const uint64_t hash = hash_u64(data.seed + batch.step * uint64_t(m.tokens / CONTEXT) + uint64_t(sequence));
         const uint64_t low = 8, places = uint64_t(data.size) - low;
         uint64_t place = hash - __umul64hi(hash, inverse) * places;
         place -= place >= places ? places : 0;
@@ -755,12 +772,12 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     staging.request_embedding();
     staging.finish(true);
     if (p.live && p.g == 0)
-        sampled[p.token] = uint8_t(token);
+        batch.tokens[p.token] = uint8_t(token);
     const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
     rotation(p.position, rc, rs);
     Head head;
-    forward_pass<true, CONTEXT>(m, p, weight, s, h, target, rc, rs, token_losses, nullptr, head);
+    forward_pass<true, CONTEXT>(m, p, weight, s, h, target, rc, rs, batch.token_losses, nullptr, head);
     backward_pass<CONTEXT>(m, p, weight, s, rc, rs, head);
 }
 
@@ -816,9 +833,10 @@ TG_DEVICE void add_half(f32x4 (&sum)[4], const unsigned char *const (&rows)[TILE
         }
     }
 }
-__global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m, const uint8_t *__restrict__ x, Workspace s,
-                                                                       int parameters) {
+__global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m, Workspace whole, Group group, int parameters) {
     extern __shared__ __align__(16) unsigned char memory[];
+    const Workspace s = group.workspace(whole, blockIdx.y);
+    const uint8_t *x = group.member[blockIdx.y].tokens;
     // consecutive blocks sit on consecutive XCDs: block 8 i + k takes the i-th unit of XCD k's chunks
     const int units = m.depth + 2, chunk = (blockIdx.x >> 3) / units * 8 + (blockIdx.x & 7), unit = (blockIdx.x >> 3) % units;
     if (chunk >= s.chunks)
@@ -979,21 +997,22 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
 }
 // gradient = the chunks' sums in chunk order, an element a thread, whose loads are in flight together: 80 chunks of 21648
 // parameters took 5.9 us with four elements a thread on a quarter of the blocks and sixteen loads at a time, 5.2 so.
-// Where `norms` is given, four blocks leave the parts of one sum of squares, of 1024 elements (FOLD_QUARTERS).
+// Where norms are wanted, four blocks leave the parts of one sum of squares, of 1024 elements (FOLD_QUARTERS).
 // Blocks beyond the parameters average the losses: one a position, in double (cuda/trainer.cuh:79-100).
 constexpr int FOLD_QUARTERS = 4;
 int fold_blocks(int parameters) { return (parameters + 1023) / 1024 * FOLD_QUARTERS; }
-__global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__ partials, int chunks, int parameters,
-                                                       float *__restrict__ gradient, float *__restrict__ norms, int blocks,
-                                                       const float *__restrict__ token_losses, int batch, int context,
-                                                       float *__restrict__ means) {
+__global__ __launch_bounds__(256) void w16_fold_kernel(Workspace whole, Group group, int parameters, int blocks, int batch,
+                                                       int context) {
+    const W16Batch &member = group.member[blockIdx.y];
+    const float *partials = group.workspace(whole, blockIdx.y).partials;
+    const int chunks = whole.chunks;
     if (int(blockIdx.x) >= blocks) {
         __shared__ double sums[4];
         const int position = blockIdx.x - blocks;
         double sum = 0;
 #pragma unroll 4
         for (int b = threadIdx.x; b < batch; b += 256)
-            sum += token_losses[size_t(b) * context + position];
+            sum += member.token_losses[size_t(b) * context + position];
 #pragma unroll
         for (int k = 32; k; k >>= 1)
             sum += __shfl_xor(sum, k, 64);
@@ -1001,7 +1020,7 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__
             sums[threadIdx.x >> 6] = sum;
         __syncthreads();
         if (threadIdx.x == 0)
-            means[position] = float(((sums[0] + sums[1]) + (sums[2] + sums[3])) / batch);
+            member.means[position] = float(((sums[0] + sums[1]) + (sums[2] + sums[3])) / batch);
         return;
     }
     __shared__ __align__(16) float row[256];
@@ -1021,16 +1040,16 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__
                 if (c + i < chunks)
                     sum += v[i];
         }
-        gradient[at] = sum;
+        member.gradient[at] = sum;
     }
-    if (!norms)
+    if (!member.norms)
         return;
     row[threadIdx.x] = sum;
     __syncthreads();
     if (threadIdx.x < 64) {
         const float squares = wave_sum(0.f + quad_squares(reinterpret_cast<const f32x4 *>(row)[threadIdx.x]));
         if (threadIdx.x == 0)
-            norms[blockIdx.x] = squares;
+            member.norms[blockIdx.x] = squares;
     }
 }
 
@@ -1040,26 +1059,27 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(const float *__restrict__
 // the products run on the fp32 matrix instruction (the same fmaf chains as a loop).  X X^T is symmetric to the last bit,
 // so its tile turned is the operand of the two products behind it, every wave computes it for itself, and a step
 // exchanges nothing but X through LDS: one barrier a step where there were four.
+// One launch makes as many steps, one after another, as there are gradients at hand: an element's (Muon: a matrix's) weights
+// and state stay in the registers between them.
 struct Update {
-    W16Weights from, to;
     float *momentum, *variance;
-    const float *gradient, *norms;
     int norm_count, norm_parts, depth; // norms: norm_count sums of norm_parts partial sums each, 1 or FOLD_QUARTERS
-    AdamArgs adam;
-    MuonArgs muon;
+    int count;
+    W16Step step[W16_BATCHES];
 };
 // clip_factor of the norms, with the sums of a fold's quarters formed first
-TG_DEVICE float clip_factor(const Update &u, float *waves) {
-    if (u.norm_parts == 1 || !(u.adam.clip > 0.f))
-        return ::clip_factor(u.adam.clip, u.norms, u.norm_count, waves);
+TG_DEVICE float clip_factor(const Update &u, int n, float *waves) {
+    const W16Step &step = u.step[n];
+    if (u.norm_parts == 1 || !(step.adam.clip > 0.f))
+        return ::clip_factor(step.adam.clip, step.norms, u.norm_count, waves);
     float sum = 0.f;
     for (int i = threadIdx.x; i < u.norm_count; i += 256) {
-        const f32x4 part = *reinterpret_cast<const f32x4 *>(u.norms + i * FOLD_QUARTERS);
+        const f32x4 part = *reinterpret_cast<const f32x4 *>(step.norms + i * FOLD_QUARTERS);
         sum += (part[0] + part[1]) + (part[2] + part[3]);
     }
-    return fminf(1.f, u.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
+    return fminf(1.f, step.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
 }
-TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
+TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
     __shared__ float wide[2][16 * F];
     __shared__ float norm_waves[4];
     const Layer p = layer_layout(matrix / 5);
@@ -1069,103 +1089,135 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *waves) {
     const int n = rows > cols ? rows : cols, size = rows * cols, tid = threadIdx.x;
     // element tid + 256 k of the matrix is this thread's until the iteration and again behind it; its place in the 16 x n form
     auto place = [&](int i) { return rows > cols ? (i % cols) * rows + i / cols : i; };
-    float g[3], m[3], w[3];
+    float next_g[3], m[3], w[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const int i = weight + tid + 256 * k;
         const bool mine = tid + 256 * k < size;
-        g[k] = mine ? u.gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f, w[k] = mine ? master(u.from.hi, u.from.lo, i) : 0.f;
+        next_g[k] = mine ? u.step[0].gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f;
+        w[k] = mine ? master(u.step[0].from.hi, u.step[0].from.lo, i) : 0.f;
     }
-    const float clip = clip_factor(u, waves);
-    float squares = 0.f, b[3];
+    const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
+    for (int at = 0; at < u.count; ++at) {
+        const W16Step &u_step = u.step[at];
+        const MuonArgs &muon = u_step.muon;
+        const float g[3] = {next_g[0], next_g[1], next_g[2]};
+        if (at + 1 < u.count)
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        if (tid + 256 * k < size) {
-            const float gs = g[k] * clip;
-            const float next = fmaf(1.f - u.muon.momentum, fmaf(g[k], clip, -m[k]), m[k]);
-            u.momentum[weight + tid + 256 * k] = next;
-            b[k] = round_bf16(fmaf(u.muon.momentum, next - gs, gs));
-            squares = fmaf(b[k], b[k], squares);
+            for (int k = 0; k < 3; ++k)
+                next_g[k] = tid + 256 * k < size ? u.step[at + 1].gradient[weight + tid + 256 * k] : 0.f;
+        const float clip = clip_factor(u, at, waves[at & 1]);
+        float squares = 0.f, b[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (tid + 256 * k < size) {
+                const float gs = g[k] * clip;
+                m[k] = fmaf(1.f - muon.momentum, fmaf(g[k], clip, -m[k]), m[k]);
+                b[k] = round_bf16(fmaf(muon.momentum, m[k] - gs, gs));
+                squares = fmaf(b[k], b[k], squares);
+            }
+        const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (tid + 256 * k < size)
+                wide[0][place(tid + 256 * k)] = round_bf16(b[k] / norm);
+        __syncthreads();
+        f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
+        if (tile < tiles)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                x[r] = wide[0][(4 * gr + r) * n + 16 * tile + c];
+        for (int step = 0; step < muon.ns_steps; ++step) {
+            const float *in = wide[step & 1];
+            float *out = wide[(step & 1) ^ 1];
+            if (tile < tiles) {
+                f32x4 gram = ZERO; // A = X X^T, kept in bf16
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    if (k < tiles) {
+                        f32x4 row;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            row[j] = in[c * n + 16 * k + 4 * j + gr];
+                        gram = multiply(row, row, gram);
+                    }
+                gram = rounded(gram);
+                const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
+                f32x4 work; // -4.775 A + 2.0315 A A
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
+                const f32x4 product = multiply(turned(rounded(work)), turned(x));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x[r] = round_bf16(fmaf(3.4445f, x[r], product[r]));
+                    out[(4 * gr + r) * n + 16 * tile + c] = x[r];
+                }
+            }
+            __syncthreads();
         }
-    const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
+        const float *result = wide[muon.ns_steps & 1];
+        const float adjusted = muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-muon.lr, muon.weight_decay, 1.f);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (tid + 256 * k < size) {
+                const int i = weight + tid + 256 * k;
+                w[k] = fmaf(w[k], keep, -(adjusted * result[place(tid + 256 * k)]));
+                const uint32_t bits = __float_as_uint(w[k]);
+                u_step.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
+                u_step.to.lo[i] = uint16_t(bits);
+            }
+        __syncthreads(); // the next step's matrix goes where this one's result is read
+    }
 #pragma unroll
     for (int k = 0; k < 3; ++k)
         if (tid + 256 * k < size)
-            wide[0][place(tid + 256 * k)] = round_bf16(b[k] / norm);
-    __syncthreads();
-    const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
-    f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
-    if (tile < tiles)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            x[r] = wide[0][(4 * gr + r) * n + 16 * tile + c];
-    for (int step = 0; step < u.muon.ns_steps; ++step) {
-        const float *in = wide[step & 1];
-        float *out = wide[(step & 1) ^ 1];
-        if (tile < tiles) {
-            f32x4 gram = ZERO; // A = X X^T, kept in bf16
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                if (k < tiles) {
-                    f32x4 row;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        row[j] = in[c * n + 16 * k + 4 * j + gr];
-                    gram = multiply(row, row, gram);
-                }
-            gram = rounded(gram);
-            const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
-            f32x4 work; // -4.775 A + 2.0315 A A
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
-            const f32x4 product = multiply(turned(rounded(work)), turned(x));
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                x[r] = round_bf16(fmaf(3.4445f, x[r], product[r]));
-                out[(4 * gr + r) * n + 16 * tile + c] = x[r];
-            }
-        }
-        __syncthreads();
-    }
-    const float *result = wide[u.muon.ns_steps & 1];
-    const float adjusted = u.muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-u.muon.lr, u.muon.weight_decay, 1.f);
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        if (tid + 256 * k < size) {
-            const int i = weight + tid + 256 * k;
-            const uint32_t bits = __float_as_uint(fmaf(w[k], keep, -(adjusted * result[place(tid + 256 * k)])));
-            u.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
-            u.to.lo[i] = uint16_t(bits);
-        }
+            u.momentum[weight + tid + 256 * k] = m[k];
 }
 __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
-    __shared__ float waves[4];
+    __shared__ float waves[2][4];
     if (int(blockIdx.x) < 5 * u.depth)
         return muon_matrix(u, blockIdx.x, waves);
-    const float scale = clip_factor(u, waves);
     // quads: the embedding's 1024, four for each scale, the head's 1024 (the only ones that decay)
     const int quad = (blockIdx.x - 5 * u.depth) * 256 + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
     int at = quad * 4;
-    float decay = 0.f;
+    bool decays = false, live = true;
     if (norm >= norms) {
         const int k = quad - V * W / 4 - 4 * norms;
-        if (k >= V * W / 4)
-            return;
-        at = V * W + u.depth * LAYER_SIZE + W + k * 4;
-        decay = u.adam.weight_decay;
+        live = k < V * W / 4;
+        at = live ? V * W + u.depth * LAYER_SIZE + W + k * 4 : 0;
+        decays = true;
     } else if (norm >= 0 && quad >= V * W / 4) {
         const Layer q = layer_layout(norm >> 1);
         at = (norm == 2 * u.depth ? V * W + u.depth * LAYER_SIZE : (norm & 1) ? q.mlp_norm : q.attention_norm) + (quad & 3) * 4;
     }
+    f32x4 m = *reinterpret_cast<const f32x4 *>(u.momentum + at), v = *reinterpret_cast<const f32x4 *>(u.variance + at), w;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        float m = u.momentum[at + k], v = u.variance[at + k];
-        const float next = adamw_element(u.adam, decay, scale, master(u.from.hi, u.from.lo, at + k), m, v, u.gradient[at + k]);
-        u.momentum[at + k] = m, u.variance[at + k] = v;
-        u.to.hi[at + k] = uint16_t(__float_as_uint(next) >> 16);
-        u.to.lo[at + k] = uint16_t(__float_as_uint(next));
+    for (int k = 0; k < 4; ++k)
+        w[k] = master(u.step[0].from.hi, u.step[0].from.lo, at + k);
+    f32x4 next_g = *reinterpret_cast<const f32x4 *>(u.step[0].gradient + at);
+    for (int n = 0; n < u.count; ++n) {
+        const W16Step &step = u.step[n];
+        const f32x4 g = next_g;
+        if (n + 1 < u.count)
+            next_g = *reinterpret_cast<const f32x4 *>(u.step[n + 1].gradient + at);
+        const float scale = clip_factor(u, n, waves[n & 1]);
+        if (!live)
+            continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float mk = m[k], vk = v[k];
+            w[k] = adamw_element(step.adam, decays ? step.adam.weight_decay : 0.f, scale, w[k], mk, vk, g[k]);
+            m[k] = mk, v[k] = vk;
+        }
+        const auto half = [&](int k, int shift) { return (__float_as_uint(w[k]) >> shift) & 0xffffu; };
+        *reinterpret_cast<u32x2 *>(step.to.hi + at) = u32x2{half(0, 16) | half(1, 16) << 16, half(2, 16) | half(3, 16) << 16};
+        *reinterpret_cast<u32x2 *>(step.to.lo + at) = u32x2{half(0, 0) | half(1, 0) << 16, half(2, 0) | half(3, 0) << 16};
     }
+    if (!live)
+        return;
+    *reinterpret_cast<f32x4 *>(u.momentum + at) = m;
+    *reinterpret_cast<f32x4 *>(u.variance + at) = v;
 }
 int adam_blocks(int depth) { return (2 * V * W / 4 + 4 * (2 * depth + 1) + 255) / 256; }
 
@@ -1203,15 +1255,14 @@ template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&config
               "w16 LDS size: ");
     configured[device].store(true, std::memory_order_release);
 }
-void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const uint8_t *x, float *gradient, float *norms,
-                             const float *token_losses, float *means) {
+void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const Group &group, int count, bool losses) {
     const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
     static std::atomic<bool> configured[64];
     allow_lds(w16_weight_gradient_kernel, configured, GRADIENT_LDS);
-    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((m.depth + 2) * ((r.chunks + 7) / 8 * 8)), dim3(64 * WAVES), GRADIENT_LDS, stream, m,
-                       x, r, parameters);
-    hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (means ? m.context : 0)), dim3(256), 0, stream, r.partials, r.chunks,
-                       parameters, gradient, norms, blocks, token_losses, m.tokens / m.context, m.context, means);
+    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((m.depth + 2) * ((r.chunks + 7) / 8 * 8), count), dim3(64 * WAVES), GRADIENT_LDS,
+                       stream, m, r, group, parameters);
+    hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (losses ? m.context : 0), count), dim3(256), 0, stream, r, group, parameters, blocks,
+                       m.tokens / m.context, m.context);
     check_hip(hipGetLastError(), "w16 weight gradient launch: ");
 }
 } // namespace
@@ -1245,7 +1296,9 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         allow_lds(w16_backward_kernel, configured, staged_bytes(MAX_DEPTH));
         hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
         check_hip(hipGetLastError(), "w16_backward launch: ");
-        launch_weight_gradients(stream, m, r, x, gradient, nullptr, nullptr, nullptr);
+        Group group{};
+        group.member[0].tokens = const_cast<uint8_t *>(x), group.member[0].workspace = workspace, group.member[0].gradient = gradient;
+        launch_weight_gradients(stream, m, r, group, 1, false);
     });
 }
 
@@ -1255,23 +1308,26 @@ int w16_norm_count(int depth) {
 int w16_norm_parts() {
     return FOLD_QUARTERS;
 }
-void w16_gradient(hipStream_t stream, int depth, int batch, int context, const W16Weights &weights, const W16Data &data,
-                  uint8_t *tokens, void *workspace, float *token_losses, float *means, float *gradient, float *norms) {
+void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, const W16Batch *batches) {
     require(context == 4 || context == 8, "w16: a training step has a context of 4 or 8");
-    const Model m = make_model(depth, batch, context, weights.hi, weights.lo);
-    const Workspace r = carve(depth, batch, context, workspace);
+    require(count >= 1 && count <= W16_BATCHES, "w16: too many batches for one launch");
+    const Model m = make_model(depth, batch, context, nullptr, nullptr);
+    const Workspace r = carve(depth, batch, context, batches[0].workspace);
+    Group group{};
+    std::copy(batches, batches + count, group.member);
     static std::atomic<bool> configured[2][64];
     const auto kernel = context == 4 ? w16_step_kernel<4> : w16_step_kernel<8>;
     allow_lds(kernel, configured[context == 8], staged_bytes(MAX_DEPTH));
     const uint64_t places = uint64_t(data.size) - 8, inverse = places > 1 ? uint64_t((static_cast<unsigned __int128>(1) << 64) / places) : ~uint64_t(0);
-    hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, data, inverse, tokens, r, token_losses);
+    hipLaunchKernelGGL(kernel, dim3(r.blocks, count), dim3(64 * WAVES), staged_bytes(depth), stream, m, data, inverse, r, group);
     check_hip(hipGetLastError(), "w16_step launch: ");
-    launch_weight_gradients(stream, m, r, tokens, gradient, norms, token_losses, means);
+    launch_weight_gradients(stream, m, r, group, count, true);
 }
-void w16_update(hipStream_t stream, int depth, const W16Weights &from, const W16Weights &to, float *momentum, float *variance,
-                const float *gradient, const float *norms, int norm_count, int norm_parts, const AdamArgs &adam,
-                const MuonArgs &muon) {
-    const Update u{from, to, momentum, variance, gradient, norms, norm_count, norm_parts, depth, adam, muon};
+void w16_updates(hipStream_t stream, int depth, float *momentum, float *variance, int norm_count, int norm_parts, int count,
+                 const W16Step *steps) {
+    require(count >= 1 && count <= W16_BATCHES, "w16: too many steps for one launch");
+    Update u{momentum, variance, norm_count, norm_parts, depth, count, {}};
+    std::copy(steps, steps + count, u.step);
     hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth + adam_blocks(depth)), dim3(256), 0, stream, u);
     check_hip(hipGetLastError(), "w16_update launch: ");
 }
@@ -1287,8 +1343,8 @@ extern "C" int tgk_w16_muon(hipStream_t stream, int depth, uint16_t *weight_hi, 
         AdamArgs adam{};
         adam.clip = clip;
         const W16Weights weights{weight_hi, weight_lo};
-        const Update u{weights, weights, momentum, nullptr, gradient, norm_partials, norm_count, 1, depth, adam,
-                       MuonArgs{lr, momentum_rate, weight_decay, ns_steps}};
+        Update u{momentum, nullptr, norm_count, 1, depth, 1, {}};
+        u.step[0] = {weights, weights, gradient, norm_partials, adam, MuonArgs{lr, momentum_rate, weight_decay, ns_steps}};
         hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth), dim3(256), 0, stream, u); // the matrices' blocks alone
         check_hip(hipGetLastError(), "w16_muon launch: ");
     });
