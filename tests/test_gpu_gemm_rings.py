@@ -1,0 +1,47 @@
+"""Products whose stages (64 of the reduced dimension) fill the ring of a lone tile not at all, once and several times, weights
+either way round; and rows too far apart for the tile kernels' 32-bit offsets.  Bound: one bf16 rounding,
+2^-9 of the value, and 0.5e-3 for the fp32 sums."""
+import pytest
+import torch
+
+from gpu_util import check, library, stream, sync
+
+pytestmark = pytest.mark.gpu
+
+BF16 = torch.bfloat16
+
+
+def product(x, w, transposed):
+    (M, K), N, lib = x.shape, w.shape[0], library()
+    weight = w.t().contiguous() if transposed else w
+    y = torch.full((M, N), float("nan"), device="cuda", dtype=BF16)
+    fn = lib.tgk_gemm_fwd_t if transposed else lib.tgk_gemm_fwd
+    check(fn(stream(), M, N, K, x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(), N, None, 0, None, 0))
+    sync()
+    return y
+
+
+def relative(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# lone 64 x 64 tiles have four slots, lone 64 x 128 ones too from K = 1024 on (1024 x 2048: 256 of them), others three
+@pytest.mark.parametrize("M,N,stages", [(256, 128, s) for s in (2, 4, 6, 7, 8, 10, 11, 15)] + [(1024, 2048, s) for s in (15, 16, 17, 19)])
+def test_turns_of_the_ring(M, N, stages):
+    K = 64 * stages
+    gen = torch.Generator(device="cuda").manual_seed(stages)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(BF16)
+    w = (torch.randn(N, K, device="cuda", generator=gen) * K ** -0.5).to(BF16)
+    y = product(x, w, False)
+    assert relative(y, x.double() @ w.double().t()) < 2.5e-3
+    assert torch.equal(y, product(x, w, True))
+
+
+def test_far_rows():
+    M, N, K, ld = 128, 128, 128, (1 << 23) + 64
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    memory = torch.zeros((M - 1) * ld + K, device="cuda", dtype=BF16)
+    x = memory.as_strided((M, K), (ld, 1))
+    x.copy_(torch.randn(M, K, device="cuda", generator=gen))
+    w = (torch.randn(N, K, device="cuda", generator=gen) * K ** -0.5).to(BF16)
+    assert relative(product(x, w, False), x.double() @ w.double().t()) < 2.5e-3

@@ -101,6 +101,12 @@ TG_DEVICE void async_copy16(uint32_t lds_base, const void *uniform_base, uint32_
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base)
                  : "memory");
 }
+// a pointer that is the same in every lane, in scalar registers
+template <class T> TG_DEVICE T *uniform(T *p) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(p);
+    const uint32_t low = __builtin_amdgcn_readfirstlane(uint32_t(bits)), high = __builtin_amdgcn_readfirstlane(uint32_t(bits >> 32));
+    return reinterpret_cast<T *>(uint64_t(high) << 32 | low);
+}
 // the 4-byte form: lane l lands at lds_base + 4*l
 TG_DEVICE void async_copy4(uint32_t lds_base, const void *global) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(global) : "memory");
