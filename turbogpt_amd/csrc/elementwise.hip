@@ -241,15 +241,15 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const bf16_t *__rest
 }
 
 // dx (+ residual), and per-block partial sums of dgamma / dbeta into partial[block][2][D].
-template <int NC, int GROUP>
-__global__ __launch_bounds__(256) void layernorm_bwd_kernel(const bf16_t *__restrict__ x,
+template <int NC, int GROUP, int THREADS>
+__global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__restrict__ x,
                                                             const bf16_t *__restrict__ dy,
                                                             const uint16_t *__restrict__ gamma_hi,
                                                             const uint16_t *__restrict__ gamma_lo,
                                                             const bf16_t *residual, bf16_t *dx,
                                                             float *__restrict__ partial, int rows, int D,
                                                             float eps) {
-    constexpr int PER_BLOCK = 256 / GROUP;
+    constexpr int PER_BLOCK = THREADS / GROUP;
     extern __shared__ float lds[]; // [PER_BLOCK row slots][2][D]
     const int lane = threadIdx.x & (GROUP - 1), slot = threadIdx.x / GROUP, chunks = D >> 3;
     const float inv_d = 1.0f / D;
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const bf16_t *__rest
             }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * D; i += 256) {
+    for (int i = threadIdx.x; i < 2 * D; i += THREADS) {
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < PER_BLOCK; ++r) // fixed order
@@ -854,16 +854,23 @@ void launch_layernorm_bwd_rows(hipStream_t stream, int rows, int D, const uint16
     // one row per wave here: two rows per wave cost registers (148 for D = 768) and LDS that lower the
     // occupancy, and measured slower
     const int per_lane = (D / 8 + 63) / 64;
-    const size_t lds = size_t(4) * 2 * D * sizeof(float);
-#define TG_LN_BWD(NC, GROUP)                                                                                      \
-    hipLaunchKernelGGL((layernorm_bwd_kernel<NC, GROUP>), dim3(blocks), dim3(256), lds, stream, x, dy, gamma_hi,  \
-                       gamma_lo, residual, dx, partial, rows, D, eps)
-    if (per_lane == 1)
-        TG_LN_BWD(1, 64);
+    // Where a block has eight rows, eight waves take one each: with four a wave's second row waits for its first (us in a
+    // training step: 1920 x 640 7.8 -> 6.6, 2048 x 256 4.5 -> 3.9).  Wider rows and more of them keep the four (LDS, registers).
+    const bool once = rows <= blocks * 8 && per_lane <= 2;
+    const size_t lds = size_t(once ? 8 : 4) * 2 * D * sizeof(float);
+#define TG_LN_BWD(NC, THREADS)                                                                                    \
+    hipLaunchKernelGGL((layernorm_bwd_kernel<NC, 64, THREADS>), dim3(blocks), dim3(THREADS), lds, stream, x, dy,  \
+                       gamma_hi, gamma_lo, residual, dx, partial, rows, D, eps)
+    if (per_lane == 1 && once)
+        TG_LN_BWD(1, 512);
+    else if (per_lane == 1)
+        TG_LN_BWD(1, 256);
+    else if (per_lane == 2 && once)
+        TG_LN_BWD(2, 512);
     else if (per_lane == 2)
-        TG_LN_BWD(2, 64);
+        TG_LN_BWD(2, 256);
     else
-        TG_LN_BWD(4, 64);
+        TG_LN_BWD(4, 256);
 #undef TG_LN_BWD
     check_hip(hipGetLastError(), "layernorm_bwd launch: ");
 }
