@@ -45,3 +45,35 @@ def test_far_rows():
     x.copy_(torch.randn(M, K, device="cuda", generator=gen))
     w = (torch.randn(N, K, device="cuda", generator=gen) * K ** -0.5).to(BF16)
     assert relative(product(x, w, False), x.double() @ w.double().t()) < 2.5e-3
+
+
+# Lone tiles of 128 x 96 (192 to 256 of them), whose waves lie one above the other: every epilogue and strides of their own,
+# bit for bit what the k-strided weight's tiles of another shape give.
+@pytest.mark.parametrize("stages", (1, 3, 4, 5, 12))
+@pytest.mark.parametrize("M,N", [(1024, 2304), (1024, 3072), (4096, 768), (8192, 384)])
+@pytest.mark.parametrize("mode", ("plain", "residual", "gelu"))
+def test_waves_one_above_the_other(M, N, stages, mode):
+    K, ldy = 64 * stages, N + 64
+    gen = torch.Generator(device="cuda").manual_seed(stages)
+    x = torch.randn(M, K + 8, device="cuda", generator=gen).to(BF16)[:, :K]
+    w = (torch.randn(N, K + 16, device="cuda", generator=gen) * K ** -0.5).to(BF16)[:, :K]
+    wt = w.t().contiguous()
+    residual = torch.randn(M, N + 8, device="cuda", generator=gen).to(BF16)[:, :N]
+    want = x.double() @ w.double().t()
+    if mode == "residual":
+        want = want.to(BF16).double() + residual.double()
+    outputs = []
+    for fn, weight in ((library().tgk_gemm_fwd, w), (library().tgk_gemm_fwd_t, wt)):
+        y = torch.full((M, ldy), float("nan"), device="cuda", dtype=BF16)
+        g = torch.full((M, ldy), float("nan"), device="cuda", dtype=BF16)
+        r = (residual.data_ptr(), residual.stride(0)) if mode == "residual" else (None, 0)
+        second = (g.data_ptr(), ldy) if mode == "gelu" else (None, 0)
+        check(fn(stream(), M, N, K, x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(), ldy, *r, *second))
+        sync()
+        assert y[:, N:].isnan().all() and g[:, N:].isnan().all()
+        outputs.append((y[:, :N], g[:, :N]))
+    (y, g), (yt, gt) = outputs
+    assert relative(y, want) < 4e-3  # two bf16 roundings where there is a residual
+    assert torch.equal(y, yt)
+    if mode == "gelu":
+        assert torch.equal(g, gt) and not g.isnan().any()

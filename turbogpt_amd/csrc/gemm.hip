@@ -754,7 +754,7 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
 }
 
 // The product of one BM x BN tile over k_chunks stages of 64 k, each operand either way round; four waves of
-// BM / 2 x BN / 2 outputs.  S - 1 stages are in flight, and a stage is one wait, one barrier, every fragment read at
+// a quarter of the outputs each.  S - 1 stages are in flight, and a stage is one wait, one barrier, every fragment read at
 // once (one LDS round trip; read column by column as in multiply_stage, 1024 x 768 with K = 3072 took 17.1 us instead of
 // 13.9), the copies of the stage S - 1 further on, then the matrix instructions, which add in the same order as
 // gemm64_kernel.  Ends behind a barrier: the slots are free.
@@ -764,7 +764,11 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
 template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 0> struct TileProduct {
     using TA = typename Tile64Of<BM, AKC>::type;
     using TB = typename Tile64Of<BN, BKC>::type;
-    static constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, THREADS = 256;
+    // four waves two by two, or one above the other where half the columns are no blocks of 32
+    static constexpr int ACROSS = BN % 64 == 0 ? 2 : 1, WM = BM / (4 / ACROSS), WN = BN / ACROSS, FM = WM / 32, FN = WN / 32, THREADS = 256;
+    static_assert(FM * 32 == WM && FN * 32 == WN);
+    TG_DEVICE static int wave_row(int wave) { return wave / ACROSS * WM; }
+    TG_DEVICE static int wave_col(int wave) { return wave % ACROSS * WN; }
     static constexpr int LA = TA::LOADS, LB = TB::LOADS, LOADS = LA + LB, SLOT = TA::BYTES + TB::BYTES;
     static_assert(S >= 2 && (S - 1) * LOADS <= 63, "the copies in flight fit the wave's counter");
     static_assert(GROUPS == 1 || (GROUPS == 2 && BM * BN * 4 <= S * SLOT), "the second group's sums fit its ring");
@@ -781,7 +785,7 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
             smem += group * (S * SLOT);
         }
         const uint32_t ring = lds_address(smem) + uint32_t(__builtin_amdgcn_readfirstlane(wave)) * 1024;
-        const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+        const int wm = wave_row(wave), wn = wave_col(wave);
         const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
         // a copy's address is the block's own, advanced stage by stage, plus 32 bits that a lane keeps (near): scalar instructions,
         // all but the copies themselves.  Weight gradients, whose lists take any leading dimension, keep a pointer a copy.
@@ -966,7 +970,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t *__restrict
     int m0, n0;
     grid.place(xcd_contiguous(blockIdx.x, gridDim.x), m0, n0);
     m0 *= BM, n0 *= BN;
-    const int m = m0 + (wave >> 1) * P::WM, n = n0 + (wave & 1) * P::WN;
+    const int m = m0 + P::wave_row(wave), n = n0 + P::wave_col(wave);
     // the epilogue's second input first of all: it lands before the operands do
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
     if (epilogue.wants_aux())
@@ -2058,17 +2062,23 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
 // each in company): small tiles where there would be idle units, larger ones as soon as the units are full.  Shapes on
 // either side, us: 1920 x 640, K = 640 (300 / 150 / 75 tiles) 6.1 / 6.4 / 8.5; 1024 x 2304, 768 (576 / 288 / 144) 10.4 / 9.0 / 9.9;
 // 16384 x 640, 640 22.8 / 21.5 / 21.4; 16384 x 384, 384 11.0 / 10.7 / 9.3 and 10.4 on 128 x 192; 16384 x 2560, 640 99.9 / 87.4 / 74.5.
-enum Block { BLOCK_64x64, BLOCK_64x128, BLOCK_128x128, BLOCK_128x192 };
-Block choose_block(int M, int N) {
+// 128 x 96 (k-contiguous weights only) fills the units once where 64 x 128 needs a second, mostly idle turn: 64 x 128 -> 128 x 96,
+// 1024 x 2304, 768 9.5 -> 8.9; 1024 x 3072, 768 9.7 -> 8.9, with GELU 11.6 -> 11.0; 4096 x 768, 1024 11.4 -> 10.6, 3072 28.4 -> 25.3 and
+// 36.8 -> 26.8 with operands from memory; 2048 x 1152, 384 6.1 -> 6.0; on a second turn it loses to 128 x 128 (1920 x 1920, 640 15.1,
+// 10.0).
+enum Block { BLOCK_64x64, BLOCK_64x128, BLOCK_128x96, BLOCK_128x128, BLOCK_128x192 };
+Block choose_block(int M, int N, bool k_contiguous) {
     static constexpr struct {
         int rows, cols, alone, both, each;
-    } kinds[] = {{64, 64, 21, 32, 19}, {64, 128, 34, 57, 31}, {128, 128, 60, 92, 50}, {128, 192, 95, 150, 72}};
+    } kinds[] = {{64, 64, 21, 32, 19}, {64, 128, 34, 57, 31}, {128, 96, 44, 88, 44}, {128, 128, 60, 92, 50}, {128, 192, 95, 150, 72}};
     const int units = compute_units();
     int best = BLOCK_64x64, least = 0;
-    for (int kind = 0; kind < 4; ++kind) {
+    for (int kind = 0; kind < 5; ++kind) {
         if (M % kinds[kind].rows || N % kinds[kind].cols)
             continue;
         const int tiles = (M / kinds[kind].rows) * (N / kinds[kind].cols), deepest = (tiles + units - 1) / units;
+        if (kind == BLOCK_128x96 && (deepest > 1 || !k_contiguous))
+            continue;
         const int cost = deepest == 1 ? kinds[kind].alone : deepest == 2 ? kinds[kind].both : deepest * kinds[kind].each;
         if (!least || cost <= least) // equal: the larger tile moves fewer bytes
             best = kind, least = cost;
@@ -2091,6 +2101,10 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
         if (M / 64 * (N / 128) <= compute_units() && K >= 1024)
             return launch_gemm_tile<64, 128, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         return launch_gemm_tile<64, 128, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+    case BLOCK_128x96:
+        if constexpr (BKC)
+            return launch_gemm_tile<128, 96, 4, true>(stream, A, lda, B, ldb, M, N, K, e);
+        throw std::logic_error("gemm: no such tile on a k-strided weight");
     case BLOCK_128x128:
         // alone on its unit a block needs the deeper ring (1920 x 1920, K = 640: 9.6 us against 11.1), with a second
         // one beside it the room (16384 x 2560, 640: 74.5 against 84.5)
@@ -2116,7 +2130,7 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
 template <bool BKC>
 void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                        const EpilogueBf16 &e) {
-    const Block block = choose_block(M, N);
+    const Block block = choose_block(M, N, BKC);
     switch (e.mode) {
     case EPI_RESIDUAL:
         return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
