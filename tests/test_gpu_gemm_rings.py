@@ -25,8 +25,8 @@ def relative(a, b):
     return float((a.double() - b).norm() / b.norm())
 
 
-# lone 64 x 64 tiles have four slots, lone 64 x 128 ones too from K = 1024 on (1024 x 2048: 256 of them), others three
-@pytest.mark.parametrize("M,N,stages", [(256, 128, s) for s in (2, 4, 6, 7, 8, 10, 11, 15)] + [(1024, 2048, s) for s in (15, 16, 17, 19)])
+# lone 64 x 64 tiles: a ring of four, from 7 stages on two groups of waves with three each, from 16 on with four
+@pytest.mark.parametrize("M,N,stages", [(256, 128, s) for s in (2, 4, 6, 7, 8, 10, 11, 15, 16, 17, 23)] + [(1024, 2048, s) for s in (15, 16, 17, 19)])
 def test_turns_of_the_ring(M, N, stages):
     K = 64 * stages
     gen = torch.Generator(device="cuda").manual_seed(stages)

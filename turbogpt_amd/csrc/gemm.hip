@@ -758,7 +758,7 @@ __global__ __launch_bounds__(256, 2) void gemm64_kernel(const bf16_t *__restrict
 // once (one LDS round trip; read column by column as in multiply_stage, 1024 x 768 with K = 3072 took 17.1 us instead of
 // 13.9), the copies of the stage S - 1 further on, then the matrix instructions, which add in the same order as
 // gemm64_kernel.  Ends behind a barrier: the slots are free.
-// GROUPS = 2 (weight gradients): two such groups of four waves take the two halves of the stages, each through its own ring (`smem` is the
+// GROUPS = 2: two such groups of four waves take the two halves of the stages, each through its own ring (`smem` is the
 // first's), and the second hands its sums to the first, which alone ends with the product.
 // FOLD > 0: the sums of every FOLD stages are added up by themselves and then join a second set of sums.
 template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 0> struct TileProduct {
@@ -949,7 +949,8 @@ TileGrid tile_grid(int rows, int cols, int bm, int bn, int run) {
 // C = A B^T with A k-contiguous and B either way round.  A product with few outputs is bound by how many compute units
 // have a tile and by the latency of each 64-k stage on them, not by bytes per flop: 1024 x 768 outputs are 32 tiles of
 // 128 x 192 but 192 of 64 x 64.  So the tile is a parameter (choose_block) and a block computes one of them; the sums run in
-// the same order whatever the tile: results are bit-identical.  A stage's copies take scalar addresses, so that a wave's vector
+// the same order whatever the tile: results are bit-identical, except where two groups of waves (GROUPS) halve the reduced
+// dimension.  A stage's copies take scalar addresses, so that a wave's vector
 // instructions are reads and products: in a step of d_model 640 over 1920 rows 1920 x 1920, K = 640 with GELU 12.5 -> 11.7 us,
 // with GELU' 13.3 -> 12.4.  What is left is the LDS: it takes 64 bytes a cycle from the copies and gives 128 to the reads, one
 // after the other, and a stage of 64 x 64, 64 x 128, 128 x 128 takes the 0.21, 0.31, 0.49 us of that.  Tried and not faster: reading
@@ -960,24 +961,27 @@ TileGrid tile_grid(int rows, int cols, int bm, int bn, int run) {
 // 5.6; 1920 x 640, 1920: 25.5 -> 12.9; 1024 x 768, 3072: 40.6 -> 12.3; 1024 x 2304, 768: 13.2 -> 9.0; 8192 x 512, 2048: 28.5 ->
 // 22.3; 16384 x 256, 768: 13.4 -> 10.6; with B k-strided (weights [K][N]) 1024 x 768, 3072: 55.1 -> 12.6; 4096 x 3072, 768: 27.6 -> 22.8;
 // 16384 x 2304, 768: 77.0 -> 67.6.
-template <int BM, int BN, int S, bool BKC, class Epilogue>
-__global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B, int ldb,
-                                                        int k_chunks, TileGrid grid, Epilogue epilogue) {
-    using P = TileProduct<BM, BN, S, true, BKC>;
+template <int BM, int BN, int S, bool BKC, class Epilogue, int GROUPS = 1>
+__global__ __launch_bounds__(256 * GROUPS) void gemm_tile_kernel(const bf16_t *__restrict__ A, int lda,
+                                                                 const bf16_t *__restrict__ B, int ldb, int k_chunks,
+                                                                 TileGrid grid, Epilogue epilogue) {
+    using P = TileProduct<BM, BN, S, true, BKC, GROUPS>;
     static_assert(4 * 2048 <= P::SLOT, "the epilogue buffers fit one stage");
     extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6 & 3;
+    const bool finishes = GROUPS == 1 || threadIdx.x < 256;
     int m0, n0;
     grid.place(xcd_contiguous(blockIdx.x, gridDim.x), m0, n0);
     m0 *= BM, n0 *= BN;
     const int m = m0 + P::wave_row(wave), n = n0 + P::wave_col(wave);
     // the epilogue's second input first of all: it lands before the operands do
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
-    if (epilogue.wants_aux())
+    if (epilogue.wants_aux() && finishes)
         load_aux_pair<P::FM, P::FN>(epilogue, 0, m, n, lane, aux);
     f32x4 acc[P::FM][P::FN][2][2];
     P::run(A, lda, B, ldb, m0, n0, k_chunks, smem, acc);
-    staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
+    if (finishes)
+        staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
 }
 
 TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64::frag16's address
@@ -2029,11 +2033,11 @@ void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const
     }
 }
 
-template <int BM, int BN, int S, bool BKC, class Epilogue>
+template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
 void launch_gemm_tile_as(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                             const Epilogue &epilogue) {
-    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, Epilogue>;
-    constexpr size_t lds = S * (BM + BN) * 128;
+    auto kernel = gemm_tile_kernel<BM, BN, S, BKC, Epilogue, GROUPS>;
+    constexpr size_t lds = GROUPS * S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
     if (!configured[device].load(std::memory_order_acquire)) {
@@ -2042,20 +2046,20 @@ void launch_gemm_tile_as(hipStream_t stream, const bf16_t *A, int lda, const bf1
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256), lds, stream, A, lda, B, ldb,
+    hipLaunchKernelGGL(kernel, dim3((M / BM) * (N / BN)), dim3(256 * GROUPS), lds, stream, A, lda, B, ldb,
                        K / 64, tile_grid(M / BM, N / BN, BM, BN, ((M / BM) * (N / BN) + 7) / 8), epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
 // GELU outputs that the eight L2s hold are left to them, where the next launch finds them (streamed past them the product
 // itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %); larger ones are streamed: the two of
 // 16384 x 4096, K = 1920 / 896 / 640 took 352 / 200 / 165 us through the caches, 285 / 160 / 128 past them.
-template <int BM, int BN, int S, bool BKC, class Epilogue>
+template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
 void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                       const Epilogue &e) {
     if (size_t(M) * N * 2 * sizeof(bf16_t) > size_t(8) * (4 << 20))
-        launch_gemm_tile_as<BM, BN, S, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+        launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, e);
     else
-        launch_gemm_tile_as<BM, BN, S, BKC>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
+        launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
 }
 // Which tile a product whose reduced dimension 64 divides is cut into.  The cost of a 64-k stage on the fullest compute
 // unit, in 10 ns, as measured with one, two and more tiles on it (they overlap: 16 KB of operands take 0.21 us alone and 0.19
@@ -2090,16 +2094,22 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
                   const Epilogue &e) {
     switch (block) {
     case BLOCK_64x64:
-        // alone on its unit a block needs the deeper ring (us with three and four stages: 1024 x 768, K = 3072 16.2, 13.1; 768
-        // 5.3, 4.6; 2048 x 256, 1024 7.2, 6.3; with others beside it three: 1920 x 640, 640 6.4, 6.7).  In a step of d_model 768
-        // over 1024 rows 11.0 -> 10.6 us on average against two groups of waves with a ring each, which took its place before.
-        if (M / 64 * (N / 64) <= compute_units())
+        // alone on its unit a block of four waves reads fragments, then multiplies; a second group fills the gaps, from the
+        // reduction on that gives it a few stages, and a longer one is worth a deeper ring when its operands come from memory.
+        // us, one group with four stages in the ring / two with three each / two with four, weights [N][K]; [K][N]:
+        //   128 x 128, K = 3072 12.8 / 10.6 / 10.5; 13.4 / 10.5 / 10.4   1024 x 768: 3072 13.4 / 11.8 / 11.8; 14.1 / 12.2 / 12.2
+        //   1024 6.7 / 6.2 / 6.3; 6.9 / 6.5 / 6.4   576 5.0 / 4.9 / 5.1; 5.2 / 5.1 / 5.3   320 3.9 / 4.1 / 4.1   192 3.4 / 3.4 / 3.4; 3.4 / 3.6 / 3.6
+        //   in a text pass of d_model 768 1024 x 768, 3072 15.7 / 16.2 / 16.0; in a step of d_model 256 2048 x 256, 1024 6.6 / 7.2 / 6.9
+        // In company one group with three (1920 x 640, 640 6.4; four 6.7).
+        if (M / 64 * (N / 64) <= compute_units()) {
+            if (K >= 1024)
+                return launch_gemm_tile<64, 64, 4, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
+            if (K >= 448)
+                return launch_gemm_tile<64, 64, 3, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
             return launch_gemm_tile<64, 64, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+        }
         return launch_gemm_tile<64, 64, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
     case BLOCK_64x128:
-        // here too, if the reduction is long (three, four: 2048 x 1024, K = 4096 26.2, 23.6; 1024 x 768, 768 6.3, 6.3)
-        if (M / 64 * (N / 128) <= compute_units() && K >= 1024)
-            return launch_gemm_tile<64, 128, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         return launch_gemm_tile<64, 128, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
     case BLOCK_128x96:
         if constexpr (BKC)
