@@ -241,17 +241,20 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const bf16_t *__rest
 }
 
 // dx (+ residual), and per-block partial sums of dgamma / dbeta into partial[block][2][D].
-template <int NC, int GROUP, int THREADS>
-__global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__restrict__ x,
+// A block has four slots, each of which adds its rows in turn: block b takes rows 4 b .. 4 b + 3, then those 4 * gridDim.x
+// further on.  TURNS = 2, for at most two rows a slot: a second set of waves takes the second rows at the same time and
+// leaves their factors, and the block's fold adds them on top of the first, so the sums are those of one set, bit for bit.
+template <int NC, int GROUP, int TURNS>
+__global__ __launch_bounds__(256 * TURNS) void layernorm_bwd_kernel(const bf16_t *__restrict__ x,
                                                             const bf16_t *__restrict__ dy,
                                                             const uint16_t *__restrict__ gamma_hi,
                                                             const uint16_t *__restrict__ gamma_lo,
                                                             const bf16_t *residual, bf16_t *dx,
                                                             float *__restrict__ partial, int rows, int D,
                                                             float eps) {
-    constexpr int PER_BLOCK = THREADS / GROUP;
-    extern __shared__ float lds[]; // [PER_BLOCK row slots][2][D]
-    const int lane = threadIdx.x & (GROUP - 1), slot = threadIdx.x / GROUP, chunks = D >> 3;
+    constexpr int SLOTS = 256 / GROUP;
+    extern __shared__ float lds[]; // [TURNS][SLOTS][2][D]
+    const int lane = threadIdx.x & (GROUP - 1), slot = threadIdx.x / GROUP % SLOTS, turn = threadIdx.x >> 8, chunks = D >> 3;
     const float inv_d = 1.0f / D;
     float dg[NC][8], db[NC][8], gm[NC][8];
 #pragma unroll
@@ -263,7 +266,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__
         if (c < chunks)
             join8(gamma_hi + c * 8, gamma_lo + c * 8, gm[j]);
     }
-    for (int row0 = blockIdx.x * PER_BLOCK; row0 < rows; row0 += gridDim.x * PER_BLOCK) {
+    for (int row0 = (blockIdx.x + turn * gridDim.x) * SLOTS; row0 < rows; row0 += gridDim.x * SLOTS * TURNS) {
         const int row = row0 + slot;
         const bool live = row < rows;
         // the row's residual gradient is only needed at the end, but requested with x and dy: behind the
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__
                     v[j][k] = z;
                     s1 += dz;
                     s2 += dz * z;
-                    dg[j][k] += g[j][k] * z;
+                    dg[j][k] = TURNS == 2 && turn ? z : fmaf(g[j][k], z, dg[j][k]);
                     db[j][k] += g[j][k];
                 }
         s1 = group_sum<GROUP>(s1) * inv_d;
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__
             }
         }
     }
-    float *mine = lds + slot * 2 * D;
+    float *mine = lds + (turn * SLOTS + slot) * 2 * D;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         const int c = lane + j * GROUP;
@@ -349,12 +352,16 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_kernel(const bf16_t *__
             }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 2 * D; i += THREADS) {
-        float sum = 0.f;
+    float *out = partial + size_t(blockIdx.x) * 2 * D;
+    for (int i = threadIdx.x; i < D; i += 256 * TURNS) {
+        float gamma = 0.f, beta = 0.f;
 #pragma unroll
-        for (int r = 0; r < PER_BLOCK; ++r) // fixed order
-            sum += lds[r * 2 * D + i];
-        partial[size_t(blockIdx.x) * 2 * D + i] = sum;
+        for (int r = 0; r < SLOTS; ++r) { // fixed order
+            const float *first = lds + r * 2 * D + i, *second = first + SLOTS * 2 * D;
+            gamma += TURNS == 2 ? fmaf(second[D], second[0], first[0]) : first[0];
+            beta += TURNS == 2 ? first[D] + second[D] : first[D];
+        }
+        out[i] = gamma, out[D + i] = beta;
     }
 }
 // dgamma[c] (+)= sum_b partial[b][0][c], dbeta likewise.  16 columns x 16 row phases per block; every
@@ -854,23 +861,25 @@ void launch_layernorm_bwd_rows(hipStream_t stream, int rows, int D, const uint16
     // one row per wave here: two rows per wave cost registers (148 for D = 768) and LDS that lower the
     // occupancy, and measured slower
     const int per_lane = (D / 8 + 63) / 64;
-    // Where a block has eight rows, eight waves take one each: with four a wave's second row waits for its first (us in a
-    // training step: 1920 x 640 7.8 -> 6.6, 2048 x 256 4.5 -> 3.9).  Wider rows and more of them keep the four (LDS, registers).
-    const bool once = rows <= blocks * 8 && per_lane <= 2;
+    // With four waves a block, a wave's second row waits for its first.  While every block has a unit of its own (256 of them,
+    // 2048 rows) eight waves take its eight rows at once; with more blocks the units have waves enough.  us, four waves / eight:
+    // 1920 x 640 6.1 / 5.4, 2048 x 1024 6.8 / 6.4, 2048 x 512 4.6 / 4.5, narrower ones alike; 4096 x 640 7.3 / 7.5, 6144 x 512 6.3 / 6.9,
+    // 6144 x 1024 12.1 / 16.1.  Wider rows keep the four (registers).
+    const bool once = blocks <= 256 && per_lane <= 2;
     const size_t lds = size_t(once ? 8 : 4) * 2 * D * sizeof(float);
-#define TG_LN_BWD(NC, THREADS)                                                                                    \
-    hipLaunchKernelGGL((layernorm_bwd_kernel<NC, 64, THREADS>), dim3(blocks), dim3(THREADS), lds, stream, x, dy,  \
-                       gamma_hi, gamma_lo, residual, dx, partial, rows, D, eps)
+#define TG_LN_BWD(NC, TURNS)                                                                                      \
+    hipLaunchKernelGGL((layernorm_bwd_kernel<NC, 64, TURNS>), dim3(blocks), dim3(256 * TURNS), lds, stream, x,    \
+                       dy, gamma_hi, gamma_lo, residual, dx, partial, rows, D, eps)
     if (per_lane == 1 && once)
-        TG_LN_BWD(1, 512);
+        TG_LN_BWD(1, 2);
     else if (per_lane == 1)
-        TG_LN_BWD(1, 256);
+        TG_LN_BWD(1, 1);
     else if (per_lane == 2 && once)
-        TG_LN_BWD(2, 512);
+        TG_LN_BWD(2, 2);
     else if (per_lane == 2)
-        TG_LN_BWD(2, 256);
+        TG_LN_BWD(2, 1);
     else
-        TG_LN_BWD(4, 256);
+        TG_LN_BWD(4, 1);
 #undef TG_LN_BWD
     check_hip(hipGetLastError(), "layernorm_bwd launch: ");
 }
