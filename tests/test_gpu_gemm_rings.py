@@ -25,7 +25,7 @@ def relative(a, b):
     return float((a.double() - b).norm() / b.norm())
 
 
-# lone 64 x 64 tiles: a ring of four, from 7 stages on two groups of waves with three each, from 16 on with four
+# lone 64 x 64 tiles: a ring of four, from 5 stages on two groups of waves with three each, from 16 on with four
 @pytest.mark.parametrize("M,N,stages", [(256, 128, s) for s in (2, 4, 6, 7, 8, 10, 11, 15, 16, 17, 23)] + [(1024, 2048, s) for s in (15, 16, 17, 19)])
 def test_turns_of_the_ring(M, N, stages):
     K = 64 * stages
@@ -35,6 +35,19 @@ def test_turns_of_the_ring(M, N, stages):
     y = product(x, w, False)
     assert relative(y, x.double() @ w.double().t()) < 2.5e-3
     assert torch.equal(y, product(x, w, True))
+
+
+@pytest.mark.parametrize("transposed", (False, True))
+@pytest.mark.parametrize("stages", (5, 6, 7, 16))
+def test_order_of_two_groups(stages, transposed):
+    """From five stages on a lone 64 x 64 tile is two sums, of its first half of the stages (the odd one with it) and of the rest.
+    A 1 in the first half outlives 2^30 and -2^30 in two stages of the second; in one chain it would be lost (an ulp is 64)."""
+    M, N, K, half = 256, 128, 64 * stages, 64 * ((stages + 1) // 2)
+    x, w = (torch.zeros(n, K, device="cuda", dtype=BF16) for n in (M, N))
+    x[:, 3] = w[:, 3] = 1
+    x[:, half + 8], w[:, half + 8] = 2.0 ** 15, 2.0 ** 15
+    x[:, half + 72], w[:, half + 72] = 2.0 ** 15, -(2.0 ** 15)
+    assert (product(x, w, transposed) == 1).all()
 
 
 def test_far_rows():

@@ -2094,8 +2094,9 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
                   const Epilogue &e) {
     switch (block) {
     case BLOCK_64x64:
-        // alone on its unit a block of four waves reads fragments, then multiplies; a second group fills the gaps, from the
-        // reduction on that gives it a few stages, and a longer one is worth a deeper ring when its operands come from memory.
+        // alone on its unit a block of four waves reads fragments, then multiplies; a second group fills the gaps, and a longer
+        // reduction is worth a deeper ring when its operands come from memory.  From K = 320 on (one group is as fast or faster
+        // up to there), since the two groups' sums have an order of their own, in which these products have always been added.
         // us, one group with four stages in the ring / two with three each / two with four, weights [N][K]; [K][N]:
         //   128 x 128, K = 3072 12.8 / 10.6 / 10.5; 13.4 / 10.5 / 10.4   1024 x 768: 3072 13.4 / 11.8 / 11.8; 14.1 / 12.2 / 12.2
         //   1024 6.7 / 6.2 / 6.3; 6.9 / 6.5 / 6.4   576 5.0 / 4.9 / 5.1; 5.2 / 5.1 / 5.3   320 3.9 / 4.1 / 4.1   192 3.4 / 3.4 / 3.4; 3.4 / 3.6 / 3.6
@@ -2104,7 +2105,7 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
         if (M / 64 * (N / 64) <= compute_units()) {
             if (K >= 1024)
                 return launch_gemm_tile<64, 64, 4, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
-            if (K >= 448)
+            if (K > 256)
                 return launch_gemm_tile<64, 64, 3, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
             return launch_gemm_tile<64, 64, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         }
