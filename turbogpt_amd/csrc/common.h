@@ -93,12 +93,18 @@ TG_DEVICE float wave_max(float x) {
 // LDS byte address lds_base + 16*l, lds_base wave-uniform.  The compiler does not track these copies;
 // completion is awaited explicitly with wait_vmcnt<N>() ("at most N of this wave's vector-memory
 // operations still outstanding") before the barrier that publishes the data to the other waves.
+// The hardware needs one wait state between the write of m0 and the copy, and the compiler puts none into assembly text.
 TG_DEVICE void async_copy16(uint32_t lds_base, const void *global) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(global) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(global) : "memory");
 }
-// the same copy from a wave-uniform base plus a 32-bit byte offset per lane: one address register instead of two
+// The same copy from a wave-uniform base plus a 32-bit byte offset per lane: one address register instead of two.  A base
+// that a vector instruction has just written would need five wait states: the scalar copy of it needs none, and stands where
+// m0's has to be.
 TG_DEVICE void async_copy16(uint32_t lds_base, const void *uniform_base, uint32_t lane_offset) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base)
+    uint64_t base;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+                 : "=&s"(base)
+                 : "s"(lds_base), "v"(lane_offset), "s"(uniform_base)
                  : "memory");
 }
 // a pointer that is the same in every lane, in scalar registers
@@ -109,7 +115,7 @@ template <class T> TG_DEVICE T *uniform(T *p) {
 }
 // the 4-byte form: lane l lands at lds_base + 4*l
 TG_DEVICE void async_copy4(uint32_t lds_base, const void *global) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(global) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(global) : "memory");
 }
 template <int N> TG_DEVICE void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
