@@ -8,6 +8,7 @@ Every replayed step is also checked against the CPU checker, as tests/pipeline.p
 the independent PyTorch model: logits 0.005, gradient 0.02 as a whole and per parameter tensor, and the
 checker's own optimizer fed with the engine's gradients ends within 0.01 of the total update."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -216,3 +217,48 @@ def test_losses_of_launches_that_follow_one_another():
     np.testing.assert_array_equal(losses(*[1] * 6), losses(6)[-1:])
     np.testing.assert_array_equal(losses(3, 2), losses(5)[-2:])
     np.testing.assert_array_equal(losses(4096, 40), losses(4000, 136)[-40:])
+
+
+@pytest.mark.parametrize("inflight,depth,context,batch", [(2, 4, 4, 16), (4, 8, 8, 16), (8, 4, 4, 16), (4, 8, 8, 1280)])
+def test_calls_of_any_length_train_alike(inflight, depth, context, batch):
+    """Steps that share their launches and steps on streams of their own, behind one another in every order, and before and
+    behind new weights: the weights are those of one call."""
+    initial = reference_style_weights(depth, scale=0.05)
+    data = np.random.default_rng(9).integers(0, 256, 4096, dtype=np.uint8)
+    long, total = 4 * inflight, 16 * inflight + 16
+
+    with bridge.Native(bridge.Config(inflight=inflight, context=context, depth=depth, batch=batch)) as engine:
+        engine.set_data(data)
+
+        def trained(*calls):
+            assert sum(calls) == total
+            engine.set_weights(initial)
+            for steps in calls:
+                engine.train(steps)
+            return engine.weights()
+
+        whole = trained(total)
+        ones = [1] * (inflight + 1)
+        mixed = [long, *ones, long, 2, *ones, inflight, 3, *ones, long]
+        rest = total - sum(mixed)
+        for calls in ([1] * total, [*mixed, *[1] * rest], [*[1] * rest, *mixed[::-1]], [2] * (total // 2), [3, total - 3], [total - 1, 1]):
+            np.testing.assert_array_equal(trained(*calls), whole)
+
+
+def test_short_calls_overlap():
+    """Calls of one step leave their batch in flight for the next call: on streams of their own four batches take some 60 us a step,
+    one behind another some 100."""
+    initial = reference_style_weights(8, scale=0.05)
+    data = np.random.default_rng(9).integers(0, 256, 4096, dtype=np.uint8)
+    best = {}
+    for inflight in (1, 4):
+        with bridge.Native(bridge.Config(inflight=inflight, context=8, depth=8, batch=1280)) as engine:
+            engine.set_weights(initial)
+            engine.set_data(data)
+            for _ in range(6):
+                start = time.perf_counter()
+                for _ in range(64):
+                    engine.train(1)
+                engine.synchronize()
+                best[inflight] = min(best.get(inflight, 1e9), time.perf_counter() - start)
+    assert best[4] < 0.8 * best[1], best

@@ -69,7 +69,7 @@ StepRates onecycle_point(const OneCycle &s, int step) {
 
 // Everything one batch in flight owns: its stream, its tokens, its saved activations and its gradient.
 // Slot 0 is on the engine's stream (a synchronous engine has no other); inflight = K gives K slots on K streams
-// (the worker teams of cuda/pipeline.cuh:52-92), of the width-16 network on the engine's.
+// (the worker teams of cuda/pipeline.cuh:52-92).
 struct Slot {
     hipStream_t stream = nullptr;
     uint8_t *input = nullptr, *target = nullptr;
@@ -138,6 +138,8 @@ struct Engine {
     std::vector<StepRates> schedule;
     uint64_t step = 0;
     uint64_t floor = 0; // oldest weight version that exists: the step at the last tg_set_weights / _set_optimizer_state
+    // the version that the last shared launch left (train_width16), or `floor`: the steps up to it are on the engine's stream
+    uint64_t shared_end = 0;
     int last_train_steps = 0;
     uint64_t last_train_first = 0;
     std::vector<int> version_trace; // weight version each step of the last tg_train read
@@ -426,16 +428,30 @@ struct Engine {
         forward(s, v, true, nullptr, c.batch, false, true);
         backward(s, v, history_row(at));
     }
-    // Training steps of the width-16 network from `at` on, as many as share their launches: at most as many as are in flight.
-    // Batch s reads the weights of version max(floor, s - K + 1), which are there for all of them before the first of their
-    // optimizer steps, and those follow one another.  The order is that of the wide model's streams below; what it saves is
-    // launches, events and the host's time for them, which bounded small batches.  Microseconds a step on K streams and
-    // so: depth 8, context 8, 16 sequences, K = 4: 46 to 54 and 26; depth 4, context 4, 16 sequences, K = 8: 32 to 36 and 12;
-    // depth 8, context 8, 1280 sequences, K = 4: 76 and 68.
-    int train_width16(uint64_t at, int most, int *trace) {
+    // Whether the batches of a call of `steps` steps share their launches.  On K streams a step costs the host 32 us of
+    // launches and events at least, however small its batch, but steps of one call overlap with those of the next.  A shared launch
+    // takes as long as one batch, 48 us at depth 4 and 77 at depth 8, and 8 us of optimizer a step: worth it from two and from 3.25
+    // steps a launch on, while a batch fills few units.  us a step on streams and shared (depth and context equal):
+    //   depth 8, 16 sequences: K = 2 46, 46; 4 37, 27; 16 35, 13; calls of one step at K = 4 38, 81; of five 36, 42
+    //   depth 4, 16 sequences: K = 2 35, 32; 8 34, 13; calls of two 32, 32   640 (40 blocks): K = 4 32, 23
+    //   80 blocks: depth 8, K = 4 46, 44; 8 47, 38; depth 4 35, 30; 36, 24   160 blocks: depth 8, K = 4 60, 69; 8 61, 61; depth 4 36, 41; 38, 38
+    //   depth 8, 10000 sequences, K = 4 379, 395
+    bool shares_launches(int steps) const {
+        const Config &c = config.base;
+        const int K = int(slots.size()), launches = (steps + K - 1) / K;
+        return K == 1 || (w16_blocks(c.batch, c.context) <= 96 && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
+    }
+    // Training steps of the width-16 network from `at` on; returns how many.  Batch s reads the weights of version
+    // max(floor, s - K + 1), whichever way it is launched.
+    // `shared`: up to K batches go out as one launch of each kernel on the engine's stream, and their optimizer steps as one
+    // more.  The versions that they read are there before the first of those, as batch s reads nothing newer than `at`.
+    // Otherwise one batch and its optimizer step, on its slot's stream, as the wide model's below.  Its slot is free, and
+    // the version that it reads is there, behind step at - K: that ran on this stream, or shared a launch, whose last one left
+    // version shared_end.
+    int train_width16(uint64_t at, int most, bool shared, int *trace) {
         const Config &c = config.base;
         const uint64_t K = slots.size(), ring = versions.size();
-        const int count = int(std::min<uint64_t>(K, uint64_t(most)));
+        const int count = shared ? int(std::min<uint64_t>(K, uint64_t(most))) : 1;
         W16Batch batches[MaxInFlight];
         W16Step steps[MaxInFlight];
         for (int i = 0; i < count; ++i) {
@@ -448,12 +464,26 @@ struct Engine {
             total_staleness += step - read;
             max_staleness = std::max(max_staleness, int(step - read));
         }
+        const hipStream_t on = shared ? stream : slots[at % K].stream;
+        const auto wait_for = [&](uint64_t version) { check_hip(hipStreamWaitEvent(on, versions[version % ring].done, 0)); };
+        if (shared && K > 1 && at != shared_end) // the steps before ran on their slots' streams
+            wait_for(at);
+        if (!shared && at < shared_end + K)
+            wait_for(shared_end);
         {
             Scope profile_scope(this, TG_CLASS_OTHER);
-            w16_gradients(stream, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, batches);
+            w16_gradients(on, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, batches);
         }
-        Scope profile_scope(this, TG_CLASS_OPTIMIZER);
-        w16_updates(stream, c.depth, momentum, variance, slots[0].list_norms, w16_norm_parts(), count, steps);
+        if (!shared && at != shared_end)
+            wait_for(at);
+        {
+            Scope profile_scope(this, TG_CLASS_OPTIMIZER);
+            w16_updates(on, c.depth, momentum, variance, slots[0].list_norms, w16_norm_parts(), count, steps);
+        }
+        if (K > 1)
+            check_hip(hipEventRecord(versions[(at + uint64_t(count)) % ring].done, on));
+        if (shared)
+            shared_end = at + uint64_t(count);
         return count;
     }
     // One training step of the wide model.  Synchronous engine: everything in order on the one stream, weights updated in place
@@ -485,12 +515,14 @@ struct Engine {
         total_staleness += at - read;
         max_staleness = std::max(max_staleness, int(at - read));
     }
-    // the next steps, at most `most`; returns how many
-    int train_some(uint64_t at, int most, int *trace) {
-        if (width16)
-            return train_width16(at, most, trace);
-        train_step(at, trace);
-        return 1;
+    void train(uint64_t at, int steps, int *trace) {
+        const bool shared = width16 && shares_launches(steps);
+        for (int i = 0; i < steps;) {
+            if (width16)
+                i += train_width16(at + uint64_t(i), steps - i, shared, trace + i);
+            else
+                train_step(at + uint64_t(i), trace + i), ++i;
+        }
     }
 };
 
@@ -525,7 +557,7 @@ void build_slots(Engine *e, int inflight, bool transposed_copies) {
     e->slots.resize(size_t(inflight));
     e->versions.resize(inflight > 1 ? size_t(inflight) + 1 : 1);
     for (Slot &slot : e->slots) {
-        if (&slot == &e->slots[0] || e->width16) // the width-16 network's batches share their launches
+        if (&slot == &e->slots[0])
             slot.stream = e->stream;
         else
             check_hip(hipStreamCreate(&slot.stream)); // default priority
@@ -539,7 +571,7 @@ void build_slots(Engine *e, int inflight, bool transposed_copies) {
         e->allocate(version.lo, P);
         if (transposed_copies)
             e->allocate(version.t, P);
-        if (inflight > 1 && !e->width16)
+        if (inflight > 1)
             check_hip(hipEventCreateWithFlags(&version.done, hipEventDisableTiming));
     }
 }
@@ -901,7 +933,7 @@ TG_API int tg_set_weights(Engine *e, const float *weights) {
         }
         e->sync(); // nothing may still read the version that is overwritten
         e->step = 0;
-        e->floor = 0;
+        e->floor = 0, e->shared_end = 0;
         e->total_staleness = 0, e->max_staleness = 0;
         Version &v = e->current();
         e->upload(v.hi, high.data(), n);
@@ -952,7 +984,7 @@ TG_API int tg_set_optimizer_state(Engine *e, const float *momentum, const float 
         e->upload(e->momentum, momentum, size_t(e->layout.count));
         e->upload(e->variance, variance, size_t(e->layout.count));
         e->step = step;
-        e->floor = step;
+        e->floor = step, e->shared_end = step;
         e->sync();
     });
 }
@@ -1007,8 +1039,7 @@ TG_API int tg_train(Engine *e, int steps) {
             throw std::runtime_error("Training would exceed the OneCycle schedule");
         e->use_device();
         e->version_trace.assign(size_t(steps), 0);
-        for (int i = 0; i < steps;)
-            i += e->train_some(e->step + uint64_t(i), steps - i, &e->version_trace[size_t(i)]);
+        e->train(e->step, steps, e->version_trace.data());
         e->last_train_steps = steps, e->last_train_first = e->step;
         e->step += uint64_t(steps);
     });
@@ -1133,7 +1164,7 @@ TG_API int tg_profile_step(Engine *e, float *class_ms, int *class_launches, int 
         e->version_trace.assign(1, 0);
         e->profiling = true;
         try {
-            e->train_some(e->step, 1, e->version_trace.data());
+            e->train(e->step, 1, e->version_trace.data());
         } catch (...) {
             e->profiling = false;
             throw;

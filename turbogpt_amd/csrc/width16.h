@@ -1,5 +1,5 @@
 // Whole training-step halves of the width-16 network, for the engine: the same kernels as tgk_w16_*, with the batch
-// sampled, the losses averaged and the gradient squared on the way.  Batches in flight share their launches: a few
+// sampled, the losses averaged and the gradient squared on the way.  Batches in flight may share their launches: a few
 // sequences fill a few compute units, and a launch costs the host more than it costs them.
 #pragma once
 #include "optimizer.h"
@@ -23,6 +23,7 @@ struct W16Batch {
     void *workspace;
     float *token_losses, *means, *gradient, *norms;
 };
+int w16_blocks(int batch, int context); // of a batch's forward and backward pass
 int w16_norm_count(int depth);
 int w16_norm_parts();
 // Samples the batches, forward, backward.  A context of 4 or 8.

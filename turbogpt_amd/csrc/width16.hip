@@ -91,6 +91,10 @@ TG_DEVICE Workspace moved(Workspace s, int64_t apart) {
     return s;
 }
 int tokens_per_wave(int context) { return 16 / context * context; }
+int blocks_of(int batch, int context) {
+    const int per_block = tokens_per_wave(context) * WAVES;
+    return (batch * context + per_block - 1) / per_block;
+}
 Workspace carve(int depth, int batch, int context, void *base) {
     Workspace r{};
     size_t at = 0;
@@ -99,8 +103,7 @@ Workspace carve(int depth, int batch, int context, void *base) {
         at += (bytes + 255) & ~size_t(255);
         return p;
     };
-    const int per_wave = tokens_per_wave(context);
-    r.blocks = (batch * context + per_wave * WAVES - 1) / (per_wave * WAVES);
+    r.blocks = blocks_of(batch, context);
     r.waves = r.blocks * WAVES;
     r.chunks = (r.waves + CHUNK_WAVES - 1) / CHUNK_WAVES;
     const size_t n = size_t(r.waves) * 64;
@@ -1302,6 +1305,9 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
     });
 }
 
+int w16_blocks(int batch, int context) {
+    return blocks_of(batch, context);
+}
 int w16_norm_count(int depth) {
     return fold_blocks(make_layout(depth).count) / FOLD_QUARTERS;
 }
