@@ -242,7 +242,8 @@ TGK_API int tgk_position_means(hipStream_t stream, const float *token_loss, int 
  * arg-max attention with a GELU gate, SwiGLU(48), 4 heads of 4, vocabulary 256.  These four calls stand in
  * for forward / backward / optimize of the persistent kernel (cuda/model.cuh:8-99, cuda/optim.cuh:17-119)
  * when an engine is created from the plain Config.  depth 1..8, context 1..8 (the RoPE table of
- * cuda/attention.cuh:7-14 has eight entries); weights in the flat order of model.h:12-37. ---- */
+ * cuda/attention.cuh:7-14 has eight entries); weights in the flat order of model.h:12-37, their high halves 8-byte
+ * aligned. ---- */
 TGK_API int tgk_w16_parameter_count(int depth);
 /* bytes of device workspace (256-byte aligned) that forward fills and backward consumes */
 TGK_API size_t tgk_w16_workspace(int depth, int batch, int context);

@@ -12,10 +12,11 @@ from test_gpu_width16 import reference_style_weights, relative
 pytestmark = pytest.mark.gpu
 
 
-def run(depth, context, batch, flat, x, y):
+def run(depth, context, batch, flat, x, y, shift=0):
+    """`shift`: elements between a 16-byte boundary and the weights."""
     lib = library()
-    bits = torch.from_numpy(flat.view(np.int32))
-    hi, lo = ((bits >> 16).to(torch.int16).cuda(), (bits & 0xffff).to(torch.int16).cuda())
+    bits = torch.from_numpy(np.concatenate([np.zeros(shift, np.float32), flat]).view(np.int32))
+    hi, lo = (half.to(torch.int16).cuda()[shift:] for half in (bits >> 16, bits & 0xffff))
     tokens, targets = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
     workspace = torch.full((lib.tgk_w16_workspace(depth, batch, context),), 255, dtype=torch.uint8, device="cuda")
     losses = torch.empty(batch * context, device="cuda")
@@ -124,3 +125,12 @@ def test_a_query_that_is_not_finite_leaves_the_keys_it_did_not_choose():
     x[0] = [201, 202, 203, 250]
     embedding = part(run(depth, context, batch, flat, x, y)[2], depth, "embedding")
     assert np.isfinite(embedding[:250]).all() and (embedding[201:204] != 0).any(axis=1).all()
+
+
+@pytest.mark.parametrize("depth,context,batch", [(1, 1, 1), (4, 8, 40), (8, 4, 33)])
+def test_weights_on_any_8_byte_boundary(depth, context, batch):
+    flat = reference_style_weights(depth)
+    rng = np.random.default_rng(batch)
+    x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
+    for got, want in zip(run(depth, context, batch, flat, x, y, 4), run(depth, context, batch, flat, x, y)):
+        np.testing.assert_array_equal(got, want)

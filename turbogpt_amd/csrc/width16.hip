@@ -298,7 +298,16 @@ struct Staging {
                 scale[i] = master(m.hi, m.lo, offset + (at & 15));
         }
     }
-    TG_DEVICE void request_embedding() const { // 8 KiB
+    // 8 KiB, 16 bytes a lane; `aligned` is false where the weights are not
+    TG_DEVICE void request_embedding(bool aligned = true) const {
+        if (!aligned) {
+            const u32x2 *from = reinterpret_cast<const u32x2 *>(m.hi);
+            u32x2 *to = reinterpret_cast<u32x2 *>(tiles + embedding_at(m.depth));
+#pragma unroll
+            for (int i = 0; i < V * W / 4 / (64 * WAVES); ++i)
+                to[threadIdx.x + i * 64 * WAVES] = from[threadIdx.x + i * 64 * WAVES];
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < V * W * 2 / 1024 / WAVES; ++i) {
             const int piece = i * WAVES + wave;
@@ -715,7 +724,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const 
     Staging staging(m, memory);
     const int token = p.live ? x[p.token] : 0, target = p.live ? y[p.token] : 0;
     staging.request();
-    staging.request_embedding();
+    staging.request_embedding(!(reinterpret_cast<uintptr_t>(m.hi) & 15));
     staging.finish(false);
     const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
