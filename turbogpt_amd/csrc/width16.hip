@@ -801,6 +801,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 // instructions fill the matrix pipe, which bounds the kernel together with what the rows take on their way (half of them
 // are worked on while the others come): 93 tiles of 32 instructions a chunk at depth 4.  2560 sequences of 4 there: 15.3 us
 // with a wave for each tile that loaded its rows and turned them with the identity matrix, 13.1 so; 16 of 8 at depth 8 7.7 and 7.9.
+// Half a chunk, as the last one or the only one may be, is all that is worked on: 16 sequences of 4 at depth 4 6.4 us with the
+// missing half as zeros, 4.6 so.
 constexpr int HEAD_ROWS = 17; // the head's tiles of a wave in LDS: dlogits, and the normalised rows
 constexpr size_t GRADIENT_LDS = size_t(CHUNK_WAVES) * OPERANDS * 512;
 static_assert(HEAD_ROWS <= OPERANDS, "the head's rows fit a layer's");
@@ -855,10 +857,11 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
         return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
     const int first = chunk * CHUNK_WAVES, waves = min(CHUNK_WAVES, s.waves - first);
+    const bool second_half = waves > CHUNK_WAVES / 2;
     float *out = s.partials + size_t(chunk) * parameters;
     const uint32_t lds = lds_address(memory);
     // TILES tiles of every wave, `apart` bytes from one wave to the next in memory, one behind another in LDS; 16 bytes a lane.
-    // The last chunk's missing waves are zeros.
+    // The last chunk's missing waves are zeros, of the second half only where it has any.
     const auto copy = [&](auto tiles, const u32x2 *source, int apart, int to) {
         constexpr int PIECES = decltype(tiles)::value * 32;
         static_assert(CHUNK_WAVES * PIECES % (WAVES * 64) == 0, "every wave has as many copies");
@@ -867,7 +870,7 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
             const int base = (i * WAVES + wave) * 64, piece = base + lane, w = piece / PIECES;
             if (w < waves)
                 async_copy16(lds + uint32_t(to + base * 16), source, uint32_t(w * apart + (piece - w * PIECES) * 16));
-            else
+            else if (w < CHUNK_WAVES / 2 || second_half)
                 *reinterpret_cast<u32x4 *>(memory + to + piece * 16) = u32x4{0, 0, 0, 0};
         }
     };
@@ -905,9 +908,11 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
         };
         half_there(); // brought by nine of a wave's seventeen copies
         layer(0);
-        wait_vmcnt<0>();
-        __syncthreads();
-        layer(1);
+        if (second_half) {
+            wait_vmcnt<0>();
+            __syncthreads();
+            layer(1);
+        }
         if (wave == 0) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) // the attention projection lies behind q, k, v
@@ -931,9 +936,11 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
         };
         half_there(); // eight of the sixteen
         head(0);
-        wait_vmcnt<0>();
-        __syncthreads();
-        head(1);
+        if (second_half) {
+            wait_vmcnt<0>();
+            __syncthreads();
+            head(1);
+        }
         const int at = V * W + m.depth * LAYER_SIZE + W;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
@@ -971,6 +978,8 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
     bool extreme = false;
 #pragma unroll
     for (int w = 0; w < CHUNK_WAVES; ++w) {
+        if (w == CHUNK_WAVES / 2 && !second_half)
+            break;
         const u32x2 row = read_across(tile(w));
         const auto either = [](uint32_t two) { return (two & 0x7f80u) == 0x7f80u || (two & 0x7f800000u) == 0x7f800000u; };
         extreme = extreme || either(row.x) || either(row.y);
@@ -1008,7 +1017,8 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
             out[(vocabulary + t * 16 + 4 * g + r) * W + feed_row(c)] = sum[t][r];
 }
 // gradient = the chunks' sums in chunk order, an element a thread, whose loads are in flight together: 80 chunks of 21648
-// parameters took 5.9 us with four elements a thread on a quarter of the blocks and sixteen loads at a time, 5.2 so.
+// parameters took 5.9 us with four elements a thread on a quarter of the blocks and sixteen loads at a time, 5.2 so.  Four
+// chunks and fewer ask forty times for nothing: 1 chunk 2.5 us, with four at a time 1.2.
 // Where norms are wanted, four blocks leave the parts of one sum of squares, of 1024 elements (FOLD_QUARTERS).
 // Blocks beyond the parameters average the losses: one a position, in double (cuda/trainer.cuh:79-100).
 constexpr int FOLD_QUARTERS = 4;
@@ -1036,22 +1046,28 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(Workspace whole, Group gr
         return;
     }
     __shared__ __align__(16) float row[256];
-    constexpr int AT_ONCE = 40;
     const int at = blockIdx.x * 256 + threadIdx.x;
     float sum = 0.f;
     if (at < parameters) {
         const float *from = partials + at;
-        for (int c = 0; c < chunks; c += AT_ONCE) {
-            float v[AT_ONCE];
+        const auto add = [&](auto at_once) {
+            constexpr int AT_ONCE = decltype(at_once)::value;
+            for (int c = 0; c < chunks; c += AT_ONCE) {
+                float v[AT_ONCE];
 #pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-                if (c + i < chunks)
-                    v[i] = from[size_t(c + i) * parameters];
+                for (int i = 0; i < AT_ONCE; ++i)
+                    if (c + i < chunks)
+                        v[i] = from[size_t(c + i) * parameters];
 #pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-                if (c + i < chunks)
-                    sum += v[i];
-        }
+                for (int i = 0; i < AT_ONCE; ++i)
+                    if (c + i < chunks)
+                        sum += v[i];
+            }
+        };
+        if (chunks <= 4)
+            add(std::integral_constant<int, 4>{});
+        else
+            add(std::integral_constant<int, 40>{});
         member.gradient[at] = sum;
     }
     if (!member.norms)
