@@ -807,8 +807,9 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
             async_copy16(to, p);
             p += step;
         };
-        auto copy_to = [&](int slot) {
-            const uint32_t to = ring + uint32_t(slot) * SLOT;
+        int p_slot = 0;
+        auto copy_stage = [&]() {
+            const uint32_t to = ring + uint32_t(p_slot) * SLOT;
 #pragma unroll
             for (int j = 0; j < LA; ++j)
                 copy(to + uint32_t(j) * 4096, A, at_a[j], pa[j], a_step);
@@ -816,10 +817,6 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
             for (int j = 0; j < LB; ++j)
                 copy(to + TA::BYTES + uint32_t(j) * 4096, B, at_b[j], pb[j], b_step);
             A += a_step, B += b_step;
-        };
-        int p_slot = 0;
-        auto copy_stage = [&]() {
-            copy_to(p_slot);
             p_slot = p_slot + 1 == S ? 0 : p_slot + 1;
         };
         f32x4 sums_of_folds[FM][FN][2][2];
@@ -838,9 +835,17 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
             if (s < k_chunks)
                 copy_stage();
         int c_slot = 0;
-        auto multiply_slot = [&](int slot, auto anew, auto &&copies) { // anew: the stage's sums replace those before it
+        auto multiply = [&](int c, auto anew) { // anew: the stage's sums replace those before it
+            // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
+            const int younger = k_chunks - 1 - c;
+            if (S >= 4 && younger >= 2)
+                wait_vmcnt<(S >= 4 ? 2 : 0) * LOADS>();
+            else if (S >= 3 && younger >= 1)
+                wait_vmcnt<(S >= 3 ? 1 : 0) * LOADS>();
+            else
+                wait_vmcnt<0>();
             __syncthreads(); // everyone's copies are there, and everyone is done with the slot that is refilled next
-            const unsigned char *sa = smem + slot * SLOT, *sb = sa + TA::BYTES;
+            const unsigned char *sa = smem + c_slot * SLOT, *sb = sa + TA::BYTES;
             bf16x8 af[2][2 * FM], bfr[2][2 * FN];
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
@@ -852,7 +857,8 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
                     bfr[ks][j] = TB::frag16(sb, wn + j * 16, ks, lane);
             }
             __builtin_amdgcn_sched_barrier(0);
-            copies();
+            if (c + S - 1 < k_chunks)
+                copy_stage();
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
@@ -864,20 +870,6 @@ template <int BM, int BN, int S, bool AKC, bool BKC, int GROUPS = 1, int FOLD = 
                         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
                         t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], anew && ks == 0 ? zero : t, 0, 0, 0);
                     }
-        };
-        auto multiply = [&](int c, auto anew) {
-            // stage c has landed when at most the younger ones are in flight: S - 2 of them, fewer at the end
-            const int younger = k_chunks - 1 - c;
-            if (S >= 4 && younger >= 2)
-                wait_vmcnt<(S >= 4 ? 2 : 0) * LOADS>();
-            else if (S >= 3 && younger >= 1)
-                wait_vmcnt<(S >= 3 ? 1 : 0) * LOADS>();
-            else
-                wait_vmcnt<0>();
-            multiply_slot(c_slot, anew, [&] {
-                if (c + S - 1 < k_chunks)
-                    copy_stage();
-            });
             c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
         };
         if constexpr (FOLD > 0) {
@@ -950,10 +942,11 @@ TileGrid tile_grid(int rows, int cols, int bm, int bn, int run) {
 // have a tile and by the latency of each 64-k stage on them, not by bytes per flop: 1024 x 768 outputs are 32 tiles of
 // 128 x 192 but 192 of 64 x 64.  So the tile is a parameter (choose_block) and a block computes one of them; the sums run in
 // the same order whatever the tile: results are bit-identical, except where two groups of waves (GROUPS) halve the reduced
-// dimension.  A stage's copies take scalar addresses, so that a wave's vector
+// dimension (lone 64 x 64 tiles from K = 320 on, launch_block).  A stage's copies take scalar addresses, so that a wave's vector
 // instructions are reads and products: in a step of d_model 640 over 1920 rows 1920 x 1920, K = 640 with GELU 12.5 -> 11.7 us,
-// with GELU' 13.3 -> 12.4.  What is left is the LDS: it takes 64 bytes a cycle from the copies and gives 128 to the reads, one
-// after the other, and a stage of 64 x 64, 64 x 128, 128 x 128 takes the 0.21, 0.31, 0.49 us of that.  Tried and not faster: reading
+// with GELU' 13.3 -> 12.4.  A stage of one group of waves alone takes 0.21, 0.31, 0.49 us on 64 x 64, 64 x 128, 128 x 128: about what
+// its copies and reads take one after the other, at the 64 and 128 bytes a cycle of the LDS.  That is the group's own chain of
+// wait, reads, copies and products and not a limit of the LDS: two groups on the same unit take 0.17 us a 64 x 64 stage.  Tried and not faster: reading
 // stage c + 1's fragments under stage c's products, with up to six slots; two groups of waves on one ring, each with half of
 // a stage's k; fragments straight from memory to registers, the waves taking stages in turn (0.50 us a stage of 64 x 64: sixteen
 // rows a request); a ring's turn as straight code (faster alone, slower in a step, whose kernels find no code in the caches).
@@ -1936,7 +1929,8 @@ void dispatch_gemm(hipStream_t stream, Tile tile, const bf16_t *A, int lda, cons
 
 // A reduced dimension that is a multiple of 64 takes the two-stage 64-k kernel.
 bool takes_64(Tile tile, int reduced) { return tile != TILE_NONE && reduced % 64 == 0; }
-// The tile kernels address a block's rows (at most 192) with 32 bits; farther rows are left to gemm_kernel.
+// The tile kernels address a block's rows (at most 128 of an operand) with a 32-bit byte offset; rows more than 16 MiB apart are
+// left to gemm_kernel.
 bool near(int lda, int ldb) { return std::max(lda, ldb) <= (1 << 23); }
 
 template <int BN, bool AKC, bool BKC, class Epilogue>
@@ -2117,11 +2111,9 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
             return launch_gemm_tile<128, 96, 4, true>(stream, A, lda, B, ldb, M, N, K, e);
         throw std::logic_error("gemm: no such tile on a k-strided weight");
     case BLOCK_128x128:
-        // alone on its unit a block needs the deeper ring (1920 x 1920, K = 640: 9.6 us against 11.1), with a second
-        // one beside it the room (16384 x 2560, 640: 74.5 against 84.5)
-        if ((M / 128) * (N / 128) <= compute_units())
-            return launch_gemm_tile<128, 128, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
-        // with k-contiguous operands and many tiles a unit, the persistent kernel: its placement lets an XCD read less, its
+        // never alone on its unit, where twice as many 64 x 128 cost less: a short ring leaves room for a second block (16384 x
+        // 2560, K = 640: 74.5 us, with four stages 84.5).
+        // With k-contiguous operands and many tiles a unit, the persistent kernel: its placement lets an XCD read less, its
         // copies run on across tiles.  Tiles -> persistent, us: 16 a unit, 16384 x 4096, 384: 68 -> 58, with a residual 103 -> 88; 896
         // 169 -> 151; but 10 a unit, 16384 x 2560: 1.5 % slower on average, 2.5 % with GELU
         if constexpr (BKC)
