@@ -16,10 +16,10 @@ SHAPES = [(128, 128, 64),      # 64 x 64: 4 tiles, one stage
           (128, 192, 576),     # 64 x 64, two groups of waves, nine stages: a width 128 does not divide
           (640, 640, 320),     # the same, five stages
           (128, 128, 2048),    # the same, 32 stages
-          (1024, 2304, 64),    # 64 x 128: 288 tiles, one stage
-          (1152, 1920, 320),   # 64 x 128: 270 tiles, five stages
-          (1920, 1920, 64),    # 128 x 128, deep ring: one stage
-          (1920, 1920, 448),   # 128 x 128, deep ring: seven stages
+          (1024, 2304, 64),    # weights [N][K] on 192 tiles of 128 x 96, [K][N] on 288 of 64 x 128: one stage
+          (1152, 1920, 320),   # the same, 180 and 270 tiles, five stages
+          (1920, 1920, 64),    # 64 x 128: 450 tiles, one stage
+          (1920, 1920, 448),   # 64 x 128: 450 tiles, seven stages
           (16384, 384, 192),   # 128 x 128, two stages in flight
           (16384, 640, 64),    # the same, GELU outputs that the caches do not hold
           (16384, 2944, 64),   # 128 x 128, the persistent kernel: more than ten tiles a unit
