@@ -140,6 +140,7 @@ struct Engine {
     uint64_t floor = 0; // oldest weight version that exists: the step at the last tg_set_weights / _set_optimizer_state
     // the version that the last shared launch left (train_width16), or `floor`: the steps up to it are on the engine's stream
     uint64_t shared_end = 0;
+    bool shared_recorded = false; // whether that version's event has been recorded behind it
     int last_train_steps = 0;
     uint64_t last_train_first = 0;
     std::vector<int> version_trace; // weight version each step of the last tg_train read
@@ -468,8 +469,12 @@ struct Engine {
         const auto wait_for = [&](uint64_t version) { check_hip(hipStreamWaitEvent(on, versions[version % ring].done, 0)); };
         if (shared && K > 1 && at != shared_end) // the steps before ran on their slots' streams
             wait_for(at);
-        if (!shared && at < shared_end + K)
+        if (!shared && at < shared_end + K) {
+            if (!shared_recorded) // an event costs every shared launch 2 us, and only the first step off the stream needs one
+                check_hip(hipEventRecord(versions[shared_end % ring].done, stream));
+            shared_recorded = true;
             wait_for(shared_end);
+        }
         {
             Scope profile_scope(this, TG_CLASS_OTHER);
             w16_gradients(on, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, batches);
@@ -480,10 +485,10 @@ struct Engine {
             Scope profile_scope(this, TG_CLASS_OPTIMIZER);
             w16_updates(on, c.depth, momentum, variance, slots[0].list_norms, w16_norm_parts(), count, steps);
         }
-        if (K > 1)
-            check_hip(hipEventRecord(versions[(at + uint64_t(count)) % ring].done, on));
         if (shared)
-            shared_end = at + uint64_t(count);
+            shared_end = at + uint64_t(count), shared_recorded = false;
+        else
+            check_hip(hipEventRecord(versions[(at + 1) % ring].done, on));
         return count;
     }
     // One training step of the wide model.  Synchronous engine: everything in order on the one stream, weights updated in place
@@ -933,7 +938,7 @@ TG_API int tg_set_weights(Engine *e, const float *weights) {
         }
         e->sync(); // nothing may still read the version that is overwritten
         e->step = 0;
-        e->floor = 0, e->shared_end = 0;
+        e->floor = 0, e->shared_end = 0, e->shared_recorded = false;
         e->total_staleness = 0, e->max_staleness = 0;
         Version &v = e->current();
         e->upload(v.hi, high.data(), n);
@@ -984,7 +989,7 @@ TG_API int tg_set_optimizer_state(Engine *e, const float *momentum, const float 
         e->upload(e->momentum, momentum, size_t(e->layout.count));
         e->upload(e->variance, variance, size_t(e->layout.count));
         e->step = step;
-        e->floor = step, e->shared_end = step;
+        e->floor = step, e->shared_end = step, e->shared_recorded = false;
         e->sync();
     });
 }
