@@ -88,8 +88,9 @@ def test_far_rows(entry, M, N, ld, far):
 
 # Lone tiles of 128 x 96 (192 to 256 of them), whose waves lie one above the other: every epilogue and strides of their own,
 # bit for bit what the k-strided weight's tiles of another shape give.
-@pytest.mark.parametrize("stages", (1, 3, 4, 5, 12))
-@pytest.mark.parametrize("M,N", [(1024, 2304), (1024, 3072), (4096, 768), (8192, 384)])
+# A width that 128 does not divide takes them from 17 stages on.
+@pytest.mark.parametrize("M,N,stages", [(M, N, stages) for M, N in ((1024, 2304), (1024, 3072), (4096, 768), (8192, 384))
+                                        for stages in (1, 3, 4, 5, 12)] + [(640, 4032, 16), (640, 4032, 17)])
 @pytest.mark.parametrize("mode", ("plain", "residual", "gelu", "gelu slope"))
 def test_waves_one_above_the_other(M, N, stages, mode):
     K, ldy = 64 * stages, N + 64

@@ -2063,9 +2063,11 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
 // 128 x 96 (k-contiguous weights only) fills the units once where 64 x 128 needs a second, mostly idle turn: 64 x 128 -> 128 x 96,
 // 1024 x 2304, 768 9.5 -> 8.9; 1024 x 3072, 768 9.7 -> 8.9, with GELU 11.6 -> 11.0; 4096 x 768, 1024 11.4 -> 10.6, 3072 28.4 -> 25.3 and
 // 36.8 -> 26.8 with operands from memory; 2048 x 1152, 384 6.1 -> 6.0; on a second turn it loses to 128 x 128 (1920 x 1920, 640 15.1,
-// 10.0).
+// 10.0).  Where 128 does not divide N it stands against three and more tiles of 64 x 64 a unit, whose start and end, GELU above all,
+// take less: it is 5 to 10 % slower up to K = 512 (640 x 4032, 256 with GELU 6.5, 7.0), as fast from 640 to 1024 (4224 x 576, 1024 -2 to
+// +5 %) and 10 to 20 % faster from 1536 on.
 enum Block { BLOCK_64x64, BLOCK_64x128, BLOCK_128x96, BLOCK_128x128, BLOCK_128x192 };
-Block choose_block(int M, int N, bool k_contiguous) {
+Block choose_block(int M, int N, int K, bool k_contiguous) {
     static constexpr struct {
         int rows, cols, alone, both, each;
     } kinds[] = {{64, 64, 21, 32, 19}, {64, 128, 34, 57, 31}, {128, 96, 44, 88, 44}, {128, 128, 60, 92, 50}, {128, 192, 95, 150, 72}};
@@ -2075,7 +2077,7 @@ Block choose_block(int M, int N, bool k_contiguous) {
         if (M % kinds[kind].rows || N % kinds[kind].cols)
             continue;
         const int tiles = (M / kinds[kind].rows) * (N / kinds[kind].cols), deepest = (tiles + units - 1) / units;
-        if (kind == BLOCK_128x96 && (deepest > 1 || !k_contiguous))
+        if (kind == BLOCK_128x96 && (deepest > 1 || !k_contiguous || (N % 128 && K <= 1024)))
             continue;
         const int cost = deepest == 1 ? kinds[kind].alone : deepest == 2 ? kinds[kind].both : deepest * kinds[kind].each;
         if (!least || cost <= least) // equal: the larger tile moves fewer bytes
@@ -2133,7 +2135,7 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
 template <bool BKC>
 void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                        const EpilogueBf16 &e) {
-    const Block block = choose_block(M, N, BKC);
+    const Block block = choose_block(M, N, K, BKC);
     switch (e.mode) {
     case EPI_RESIDUAL:
         return launch_block<BKC>(stream, block, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
