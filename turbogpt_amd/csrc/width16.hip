@@ -756,11 +756,11 @@ __global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Works
 // A training step's both passes: a wave's backward pass reads only what its own forward pass kept, so the two are one launch
 // and the weights are staged once.  Depth 4, 2560 sequences of 4: 53.0 us as two launches that staged eight tiles at a time,
 // 38.8 so; depth 8, 16 of 8: 79.3 and 62.6.  Two waves a SIMD, which batches of more than 256 blocks need (10000 of 8 at depth 8
-// 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training bytes, every sequence a window at a
-// hashed place (cuda/dataset.cuh:13-27); the tokens are left for the embedding's gradient.
+// 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training
+// bytes, every sequence a window at a hashed place (cuda/dataset.cuh:13-27); the tokens are left for the embedding's gradient.
 template <int CONTEXT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(Model m, W16Data data, uint64_t inverse, Workspace first,
-                                                                                                      Group group) {
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(
+    Model m, W16Data data, uint64_t inverse, Workspace first, Group group) {
     extern __shared__ __align__(16) unsigned char memory[];
     const W16Batch &batch = group.member[blockIdx.y];
     const Workspace s = group.workspace(first, blockIdx.y);
