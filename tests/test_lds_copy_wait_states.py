@@ -8,6 +8,8 @@ from pathlib import Path
 
 import pytest
 
+from turbogpt_amd import build
+
 LIBRARY = Path(__file__).resolve().parent.parent / "turbogpt_amd" / "libturbogpt.so"
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 LINE = re.compile(r"^\t(\S+)\s*(.*?)\s*// ([0-9A-F]{12}):(?:.*<(.+?)(?:\+0x([0-9a-f]+))?>)?")
@@ -85,6 +87,8 @@ def kernels(listing):
 
 @pytest.fixture(scope="module")
 def built(tmp_path_factory):
+    if not LIBRARY.exists():
+        build.build()
     folder = tmp_path_factory.mktemp("listing")
     copy = shutil.copy(LIBRARY, folder / "library.so")  # the code objects are extracted beside it
     subprocess.run([OBJDUMP, "--offloading", copy], check=True, capture_output=True, cwd=folder)
