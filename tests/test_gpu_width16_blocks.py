@@ -1,0 +1,31 @@
+"""The width-16 network where the cut of the work changes: four or eight waves a block (more than 1024 waves), one wave or eight for
+an element's sum over the blocks (more than sixteen), each on both sides of the line, with last blocks that hold one sequence."""
+import numpy as np
+import pytest
+
+from oracle import width16 as w16
+from test_gpu_width16 import reference_style_weights, relative
+from test_gpu_width16_shapes import run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("depth,context,batch", [(2, 4, 256), (2, 4, 257), (1, 5, 204), (1, 8, 2048), (1, 8, 2049), (1, 5, 3073), (2, 1, 16385)])
+def test_blocks(depth, context, batch):
+    """Against the checker within the reference's own bounds; and the same sequences, the last one first, which moves all of them
+    to another wave: every tensor differs by the order of its sums alone, 1e-4 for at most 512 additions of 2^-24 each, three times
+    over."""
+    flat = reference_style_weights(depth)
+    rng = np.random.default_rng(depth * 100 + context)
+    x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
+    logits, losses, gradient = run(depth, context, batch, flat, x, y)
+    target, expected, expected_losses = w16.Width16(depth, context, batch).batch(flat, x, y)
+    assert relative(logits, target) < .005
+    np.testing.assert_allclose(losses.reshape(batch, context).mean(0), expected_losses, atol=.003, rtol=.001)
+    moved_logits, _, moved = run(depth, context, batch, flat, np.roll(x, 1, 0), np.roll(y, 1, 0))
+    np.testing.assert_array_equal(moved_logits, np.roll(logits, 1, 0))
+    assert relative(gradient, expected) < .01
+    for name, (offset, shape) in w16.layout(depth)[0].items():
+        part = slice(offset, offset + int(np.prod(shape)))
+        assert relative(gradient[part], expected[part]) < .02, name
+        assert relative(gradient[part], moved[part]) < 1e-4, name
