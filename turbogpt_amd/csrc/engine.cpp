@@ -201,10 +201,13 @@ struct Engine {
         allocated_bytes = bytes;
     }
     void use_device() const { check_hip(hipSetDevice(config.base.device)); }
-    void sync() const { // every stream: the engine is quiescent afterwards
+    void sync_slots() const { // every slot's stream but the engine's own
         for (const Slot &slot : slots)
             if (slot.stream && slot.stream != stream)
                 check_hip(hipStreamSynchronize(slot.stream));
+    }
+    void sync() const { // every stream: the engine is quiescent afterwards
+        sync_slots();
         check_hip(hipStreamSynchronize(stream));
     }
     Version &current() { return versions[step % versions.size()]; }
@@ -1095,7 +1098,7 @@ TG_API int tg_batch(Engine *e, const uint8_t *x, const uint8_t *y, float *logits
         const size_t M = size_t(e->tokens()), V = size_t(e->config.vocab);
         if (!e->logits_f32)
             e->allocate(e->logits_f32, M * V, false);
-        e->sync(); // fixed batches run on slot 0 with the newest weights, after everything in flight
+        e->sync_slots(); // fixed batches run on slot 0, the engine's stream, with the newest weights, after everything in flight
         Slot &slot = e->slots[0];
         check_hip(hipMemcpyAsync(slot.input, x, M, hipMemcpyHostToDevice, slot.stream));
         check_hip(hipMemcpyAsync(slot.target, y, M, hipMemcpyHostToDevice, slot.stream));
@@ -1106,7 +1109,6 @@ TG_API int tg_batch(Engine *e, const uint8_t *x, const uint8_t *y, float *logits
             e->backward(slot, e->current(), e->batch_means);
         else
             ok(tgk_position_means(slot.stream, slot.token_losses, c.batch, c.context, e->batch_means));
-        check_hip(hipStreamSynchronize(slot.stream));
         std::vector<ReadbackPiece> pieces = {{logits, M * V * 4, e->logits_f32}, {loss, size_t(c.context) * 4, e->batch_means}};
         if (gradient)
             pieces.push_back({gradient, size_t(e->layout.count) * 4, slot.gradient});
@@ -1123,13 +1125,12 @@ TG_API int tg_predict(Engine *e, const uint8_t *context, float *logits) {
         const size_t M = size_t(e->tokens()), V = size_t(e->config.vocab);
         if (!e->logits_f32)
             e->allocate(e->logits_f32, M * V, false);
-        e->sync();
+        e->sync_slots();
         // Sequences do not see each other: one of them is enough.  (cuda/runtime.cu:322-351 fills the batch with copies.)
         // The wide model computes the last position's logits alone; the targets only feed losses that nobody reads.
         Slot &slot = e->slots[0];
         check_hip(hipMemcpyAsync(slot.input, context, size_t(c.context), hipMemcpyHostToDevice, slot.stream));
         e->forward(slot, e->current(), false, e->logits_f32, 1, !e->width16);
-        check_hip(hipStreamSynchronize(slot.stream));
         e->download({{logits, V * 4, e->logits_f32 + (e->width16 ? size_t(c.context - 1) * V : 0)}});
     });
 }

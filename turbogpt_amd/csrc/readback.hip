@@ -3,7 +3,10 @@
 // What bounds it is PCIe (57 GB/s measured into pinned memory) and, behind it, the host: one core copies and
 // faults in fresh pages at a few GB/s.  So the result is cut into chunks; a kernel writes a chunk straight into pinned
 // memory (joining the weight halves on the way, which a host loop did before), and several host threads, each with
-// two buffers of its own, copy finished chunks into the caller's pages while the next ones cross the bus.
+// two buffers of its own, copy finished chunks into the caller's pages while the next ones cross the bus.  What is left
+// behind the last chunk is one thread's copy of it (90 us for 2 MiB), so the last 2 MiB are cut in halves down to 512 KiB; not
+// smaller, as every chunk costs the bus 6 us for its event.  The threads start while what is on the stream still runs: a batch's
+// 16 MB of gradient and logits at d256 875 us behind a wait for the device and in chunks of 2 MiB, 829 so.
 //
 // The host reads what a kernel wrote once the event behind the kernel has passed, and nothing else stands between the two.
 // So both halves of that order are asked for by name, whatever the environment's default is: coherent memory, and events
@@ -17,7 +20,7 @@
 
 namespace {
 
-constexpr size_t CHUNK = size_t(2) << 20;
+constexpr size_t CHUNK = size_t(2) << 20, SMALLEST_CHUNK = size_t(512) << 10;
 constexpr int LANES = 8;
 
 __global__ __launch_bounds__(256) void readback_copy_kernel(const u32x4 *__restrict__ in, u32x4 *__restrict__ out,
@@ -94,11 +97,18 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
         size_t offset, bytes;
     };
     std::vector<Chunk> chunks;
+    size_t left = 0;
     for (const ReadbackPiece &piece : pieces) {
         require(piece.bytes % 16 == 0, "readback: size must be a multiple of 16");
-        for (size_t at = 0; at < piece.bytes; at += CHUNK)
-            chunks.push_back({&piece, at, std::min(CHUNK, piece.bytes - at)});
+        left += piece.bytes;
     }
+    for (const ReadbackPiece &piece : pieces)
+        for (size_t at = 0; at < piece.bytes;) {
+            const size_t half = left / 2 & ~size_t(0xffff); // whole 64 KiB
+            const size_t bytes = std::min(std::clamp(half, SMALLEST_CHUNK, CHUNK), piece.bytes - at);
+            chunks.push_back({&piece, at, bytes});
+            at += bytes, left -= bytes;
+        }
     // lane `l` of `lanes` takes chunks l, l + lanes, ... with two buffers of its own in turn
     const size_t lanes = std::min<size_t>(LANES, (chunks.size() + 1) / 2);
     const size_t depth = chunks.size() == 1 ? 1 : 2;
