@@ -310,7 +310,8 @@ template <int ROWS> struct TileKS {
     TG_DEVICE static int swizzle(int r) {
         // row stride of 256 B multiples: 4 consecutive k-rows start in the same bank; 384 B: every other one.  The
         // 16-row fragments read k-rows r and r + 8 in one pass, 32 bytes of each: bit 3 of r moves them 32 bytes apart.
-        return (ROWS % 128 == 0 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2)) | (((r >> 3) & 1) << 1);
+        // 64 B: they start in four different places by themselves.
+        return (ROWS % 128 == 0 ? ((r & 3) << 2) : ROWS % 64 == 0 ? (((r >> 1) & 1) << 2) : 0) | (((r >> 3) & 1) << 1);
     }
     TG_DEVICE static int64_t source_offset(int j, int tid, int ld) {
         const int wave = tid >> 6, lane = tid & 63;
@@ -977,29 +978,32 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_tile_kernel(const bf16_t *_
         staged_store_bf16<P::FM, P::FN>(acc, aux, smem + wave * 2048, epilogue, m, n, lane);
 }
 
-// ---- few tiles: waves that share out the reduced dimension ----------------------------------------------------------------
+// ---- few tiles: every wave with a ring of its own ----------------------------------------------------------------------
 // A product of at most 128 tiles of 64 x 64 leaves half of the units without one, and a lone tile's time is its chain of stages.
-// Here tiles are 32 x 64 or 32 x 32 and each of a block's four waves takes a quarter of the stages for the whole tile, through a ring
-// of its own: nothing but its own copies is waited for, no barrier stands in the loop, and a stage's slot is refilled as soon as its
-// fragments are in registers.  The waves' sums meet in LDS: those of the two quarters of a half, then the halves, which are the
-// two groups' above.  What is left is that chain, a
-// quarter as long: the arrival of a stage's operands, eight to sixteen fragment reads, the products (launch_block has the times).
-template <int BM, int BN, int S, bool BKC, class Epilogue>
-__global__ __launch_bounds__(256) void gemm_waves_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B, int ldb,
-                                                               int k_chunks, TileGrid grid, Epilogue epilogue) {
-    using TA = TileKC64<BM>;
-    using TB = typename Tile64Of<BN, BKC>::type;
-    constexpr int WAVES = 4, CA = BM / 8, CB = BN / 8, COPIES = CA + CB, SLOT = (BM + BN) * 128, FM = BM / 32, FN = BN / 32, BLOCKS = FM * FN;
-    static_assert(BKC || BN % 64 == 0, "a k-strided tile's swizzle wants eight chunks a row");
-    static_assert(S * COPIES <= 63 && BM * BN * 4 <= S * SLOT && BLOCKS <= WAVES);
+// Here tiles are smaller, and each of a block's waves takes WM x WN outputs over half of the reduced dimension, with a ring of its
+// own: nothing but its own copies is waited for, no barrier stands in the loop, and a stage's slot is refilled as soon as its
+// fragments are in registers.  The halves are those of the two groups of a lone 64 x 64 tile and meet in LDS, so the results are the
+// same bit for bit.  What bounds it is still that chain: the arrival of a stage's operands, three to four fragment reads, the
+// products (launch_block has the times).  Four quarters a tile of 32 x 32 are 10 % faster at K = 3072, and another order of sums.
+template <int BM, int BN, int WM, int WN, int S, bool BKC, class Epilogue>
+__global__ __launch_bounds__(128 * (BM / WM) * (BN / WN)) void gemm_waves_kernel(const bf16_t *__restrict__ A, int lda,
+                                                                                 const bf16_t *__restrict__ B, int ldb, int k_chunks,
+                                                                                 TileGrid grid, Epilogue epilogue) {
+    using TA = TileKC64<WM>;
+    using TB = typename Tile64Of<WN, BKC>::type;
+    constexpr int ACROSS = BN / WN, SUBS = BM / WM * ACROSS, WAVES = 2 * SUBS, CA = WM / 8, CB = WN / 8, COPIES = CA + CB;
+    constexpr int SLOT = (WM + WN) * 128, FM = WM / 16, FN = WN / 16, BLOCKS = BM / 32 * (BN / 32), COLS16 = BN / 16;
+    constexpr int HALF = BM / 16 * COLS16 * 64, SUMS = 2 * HALF * 16;
+    static_assert(S == 4 && S * COPIES <= 63 && BLOCKS <= WAVES && SUMS + WAVES * 2048 <= WAVES * S * SLOT);
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = wave / SUBS, sub = wave % SUBS, row16 = sub / ACROSS * FM, col16 = sub % ACROSS * FN; // in tiles of 16 x 16
     int m0, n0;
     grid.place(xcd_contiguous(blockIdx.x, gridDim.x), m0, n0);
     m0 *= BM, n0 *= BN;
-    // wave b finishes block b; its second input first of all
+    // wave b finishes block b of 32 x 32; its second input first of all
     const bool finishes = wave < BLOCKS;
-    const int m = m0 + wave / FN * 32, n = n0 + wave % FN * 32;
+    const int block_m = wave / (BN / 32), block_n = wave % (BN / 32), m = m0 + block_m * 32, n = n0 + block_n * 32;
     u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
     if (epilogue.wants_aux() && finishes)
         load_aux_pair<1, 1>(epilogue, 0, m, n, lane, aux);
@@ -1013,10 +1017,9 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(const bf16_t *__restric
     for (int j = 0; j < CB; ++j)
         at_b[j] = uint32_t(TB::source_offset(j >> 2, (j & 3) * 64 + lane, ldb)) * 2;
     const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
-    // the halves, the first one's odd stage with it, and likewise the quarters
-    const int half = (k_chunks + 1) >> 1, mine_of = wave < 2 ? half : k_chunks - half, quarter = (mine_of + 1) >> 1;
-    const int stages = wave & 1 ? mine_of - quarter : quarter, first = (wave < 2 ? 0 : half) + (wave & 1 ? quarter : 0);
-    A = uniform(A + TA::origin(m0, 0, lda) + first * a_step), B = uniform(B + TB::origin(n0, 0, ldb) + first * b_step);
+    const int half = (k_chunks + 1) >> 1, first = group * half, stages = group ? k_chunks - half : half;
+    A = uniform(A + TA::origin(m0 + row16 * 16, 0, lda) + first * a_step);
+    B = uniform(B + TB::origin(n0 + col16 * 16, 0, ldb) + first * b_step);
     auto copy_stage = [&](int slot) {
         const uint32_t to = ring + uint32_t(slot) * SLOT;
 #pragma unroll
@@ -1027,11 +1030,11 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(const bf16_t *__restric
             async_copy16(to + TA::BYTES + uint32_t(j) * 1024, B, at_b[j]);
         A += a_step, B += b_step;
     };
-    f32x4 acc[2 * FM][2 * FN];
+    f32x4 acc[FM][FN];
 #pragma unroll
-    for (int i = 0; i < 2 * FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < 2 * FN; ++j)
+        for (int j = 0; j < FN; ++j)
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < S; ++s)
@@ -1040,23 +1043,23 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(const bf16_t *__restric
     int slot = 0;
     for (int c = 0; c < stages; ++c) {
         const int younger = min(stages - 1 - c, S - 1);
-        if (S >= 4 && younger >= 3)
-            wait_vmcnt<(S >= 4 ? 3 : 0) * COPIES>();
-        else if (S >= 3 && younger >= 2)
-            wait_vmcnt<(S >= 3 ? 2 : 0) * COPIES>();
-        else if (S >= 2 && younger >= 1)
+        if (younger >= 3)
+            wait_vmcnt<3 * COPIES>();
+        else if (younger == 2)
+            wait_vmcnt<2 * COPIES>();
+        else if (younger == 1)
             wait_vmcnt<COPIES>();
         else
             wait_vmcnt<0>();
         const unsigned char *sa = mine + slot * SLOT, *sb = sa + TA::BYTES;
-        bf16x8 af[2][2 * FM], bfr[2][2 * FN];
+        bf16x8 af[2][FM], bfr[2][FN];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-            for (int i = 0; i < 2 * FM; ++i)
+            for (int i = 0; i < FM; ++i)
                 af[ks][i] = TA::frag16(sa, i * 16, ks, lane);
 #pragma unroll
-            for (int j = 0; j < 2 * FN; ++j)
+            for (int j = 0; j < FN; ++j)
                 bfr[ks][j] = TB::frag16(sb, j * 16, ks, lane);
         }
         wait_lgkmcnt0(); // the slot has been read
@@ -1067,31 +1070,29 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(const bf16_t *__restric
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int j = 0; j < 2 * FN; ++j)
+            for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int i = 0; i < 2 * FM; ++i)
+                for (int i = 0; i < FM; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
         slot = slot + 1 == S ? 0 : slot + 1;
     }
-    __syncthreads(); // the rings are free: [block][wave][tile of 16 x 16][lane]
-    f32x4 *sums = reinterpret_cast<f32x4 *>(smem);
+    __syncthreads(); // the rings are free: [half][tile of 16 x 16][lane], then the epilogue's buffers
+    f32x4 *sums = reinterpret_cast<f32x4 *>(smem) + lane;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                sums[(((i * FN + j) * WAVES + wave) * 4 + t) * 64 + lane] = acc[2 * i + (t >> 1)][2 * j + (t & 1)];
+            sums[group * HALF + ((row16 + i) * COLS16 + col16 + j) * 64] = acc[i][j];
     __syncthreads();
     if (!finishes)
         return;
     f32x4 total[1][1][2][2];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        const f32x4 *from = sums + (wave * WAVES * 4 + t) * 64 + lane;
-        total[0][0][t >> 1][t & 1] = (from[0] + from[4 * 64]) + (from[8 * 64] + from[12 * 64]);
+        const f32x4 *from = sums + ((2 * block_m + (t >> 1)) * COLS16 + 2 * block_n + (t & 1)) * 64;
+        total[0][0][t >> 1][t & 1] = from[0] + from[HALF];
     }
-    staged_store_bf16<1, 1>(total, aux, smem + wave * (WAVES * 4096), epilogue, m, n, lane);
+    staged_store_bf16<1, 1>(total, aux, smem + SUMS + wave * 2048, epilogue, m, n, lane);
 }
 
 TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64::frag16's address
@@ -2172,11 +2173,12 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
     else
         launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
 }
-template <int BM, int BN, int S, bool BKC, class Epilogue>
+template <int BM, int BN, int WM, int WN, int S, bool BKC, class Epilogue>
 void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K, const Epilogue &e) {
     using Cached = typename Epilogue::Cached; // few outputs: the L2s hold them
-    auto kernel = gemm_waves_kernel<BM, BN, S, BKC, Cached>;
-    constexpr size_t lds = 4 * S * (BM + BN) * 128;
+    auto kernel = gemm_waves_kernel<BM, BN, WM, WN, S, BKC, Cached>;
+    constexpr int waves = 2 * (BM / WM) * (BN / WN);
+    constexpr size_t lds = waves * S * (WM + WN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
     if (!configured[device].load(std::memory_order_acquire)) {
@@ -2185,7 +2187,7 @@ void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_
         configured[device].store(true, std::memory_order_release);
     }
     const int rows = M / BM, cols = N / BN;
-    hipLaunchKernelGGL(kernel, dim3(rows * cols), dim3(256), lds, stream, A, lda, B, ldb, K / 64,
+    hipLaunchKernelGGL(kernel, dim3(rows * cols), dim3(64 * waves), lds, stream, A, lda, B, ldb, K / 64,
                        tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Cached{e.any});
     check_hip(hipGetLastError(), "gemm launch: ");
 }
@@ -2224,16 +2226,17 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
                   const Epilogue &e) {
     switch (block) {
     case BLOCK_64x64:
-        // At most half of the units: smaller tiles whose waves share out the reduced dimension, four ways whichever tile it is, so
-        // that the weights' layout does not show in the bits.  us, two groups here / 32 x 64 / 32 x 32, from the caches; from memory
-        // (K = 256: the launch is all there is, 4.0 / 3.9 / 4.0):
-        //   512 x 512, K = 768 4.5 / 4.4 / 3.9; 5.2 / 4.8 / 4.1   3072 10.2 / 7.6 / 6.4; 11.5 / 9.4 / 7.5   128 x 768, 1024 5.2 / 4.7 / 4.0
-        //   2048 x 256, 1024 5.4 / 4.9 / 6.7; 5.7 / 5.3 / 7.2   3072 10.3 / 8.1 / 11.2   [K][N] 10.9 / 8.1; 768 x 768, 1024 5.4 / 8.2
-        if (M / 64 * (N / 64) <= compute_units() / 2) {
+        // At most half of the units, and two halves to share out (K > 256: the launch is most of it below, 4.0 against 3.9): 32 x 32
+        // tiles up to a quarter of the units, 32 x 64 above.  us, two groups here / this, operands from the caches; from memory:
+        //   512 x 512, K = 768 4.6 / 4.1; 5.2 / 4.3   1024 5.3 / 4.2; 5.6 / 4.5   3072 10.1 / 7.0; 11.5 / 8.1   [K][N] 10.9 / 8.8; 13.1 / 12.5
+        //   2048 x 256, 768 4.6 / 4.5; 5.0 / 4.9   1024 5.3 / 5.0; 5.6 / 5.4   3072 10.3 / 8.8; 15.3 / 13.1
+        // 32 x 64 with weights [K][N] reads half lines of them: 768 x 512, 1024 5.6 / 5.0; 6.0 / 6.1   2304 8.9 / 7.9; 9.7 / 10.5
+        if (K > 256) {
+            if (M / 64 * (N / 64) <= compute_units() / 4)
+                return launch_gemm_waves<32, 32, 16, 32, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
             if constexpr (BKC)
-                if (M / 64 * (N / 64) <= compute_units() / 4)
-                    return launch_gemm_waves<32, 32, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
-            return launch_gemm_waves<32, 64, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+                if (M / 64 * (N / 64) <= compute_units() / 2)
+                    return launch_gemm_waves<32, 64, 32, 32, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         }
         // alone on its unit a block of four waves reads fragments, then multiplies; a second group fills the gaps, and a longer
         // reduction is worth a deeper ring when its operands come from memory.  From K = 320 on (one group is as fast or faster
