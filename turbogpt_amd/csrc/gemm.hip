@@ -310,7 +310,7 @@ template <int ROWS> struct TileKS {
     TG_DEVICE static int swizzle(int r) {
         // row stride of 256 B multiples: 4 consecutive k-rows start in the same bank; 384 B: every other one.  The
         // 16-row fragments read k-rows r and r + 8 in one pass, 32 bytes of each: bit 3 of r moves them 32 bytes apart.
-        // 64 B: they start in four different places by themselves.
+        // 64 B and 192 B: four different places already.
         return (ROWS % 128 == 0 ? ((r & 3) << 2) : ROWS % 64 == 0 ? (((r >> 1) & 1) << 2) : 0) | (((r >> 3) & 1) << 1);
     }
     TG_DEVICE static int64_t source_offset(int j, int tid, int ld) {
@@ -1093,6 +1093,118 @@ __global__ __launch_bounds__(128 * (BM / WM) * (BN / WN)) void gemm_waves_kernel
         total[0][0][t >> 1][t & 1] = from[0] + from[HALF];
     }
     staged_store_bf16<1, 1>(total, aux, smem + SUMS + wave * 2048, epilogue, m, n, lane);
+}
+
+// ---- tiles whose waves hold an odd number of 16 x 16 products one way ---------------------------------------------------
+// 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48): between 64 x 64 and what choose_block has next.
+// 257 to 384 tiles of 64 x 64 put two on some units and leave others one; these are at most one a unit.  A stage is TileProduct's,
+// with one barrier and every fragment read at once, and costs 0.28 us, two 64 x 64 in company 0.33: copies, reads and products one
+// after the other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 against
+// 16.6 us from the caches, 19.3 and 17.5 against 17.4 from memory), 96 x 32 or 96 x 16 a wave slower (22.8, 19.3).  The sums' order is
+// that of every tile.  Rows of 16-byte pieces: a lane finishes pieces l, l + 64 and l + 128 of its wave's 192.
+template <int BM, int BN, int S, bool BKC, class Epilogue>
+__global__ __launch_bounds__(256) void gemm_uneven_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B, int ldb,
+                                                          int k_chunks, TileGrid grid, Epilogue epilogue) {
+    using TA = TileKC64<BM>;
+    using TB = typename Tile64Of<BN, BKC>::type;
+    constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16, LA = TA::LOADS, LB = TB::LOADS, LOADS = LA + LB;
+    constexpr int SLOT = TA::BYTES + TB::BYTES, ROW_PIECES = WN / 8, PIECES = WM * ROW_PIECES / 64;
+    static_assert(S == 4 && BM * BN * 2 <= SLOT && PIECES * 64 == WM * ROW_PIECES);
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / 2 * WM, wn = wave % 2 * WN;
+    int m0, n0;
+    grid.place(xcd_contiguous(blockIdx.x, gridDim.x), m0, n0);
+    m0 *= BM, n0 *= BN;
+    // the epilogue's second input first of all
+    u32x4 aux[PIECES];
+    int m[PIECES], n[PIECES];
+#pragma unroll
+    for (int t = 0; t < PIECES; ++t) {
+        const int piece = t * 64 + lane, row = piece / ROW_PIECES;
+        m[t] = m0 + wm + row, n[t] = n0 + wn + (piece - row * ROW_PIECES) * 8;
+        aux[t] = epilogue.wants_aux() ? epilogue.load_aux(m[t], n[t]) : u32x4{0, 0, 0, 0};
+    }
+    const uint32_t ring = lds_address(smem) + uint32_t(wave) * 1024;
+    uint32_t at_a[LA], at_b[LB]; // as in TileProduct
+#pragma unroll
+    for (int j = 0; j < LA; ++j)
+        at_a[j] = uint32_t(TA::source_offset(j, tid, lda)) * 2;
+#pragma unroll
+    for (int j = 0; j < LB; ++j)
+        at_b[j] = uint32_t(TB::source_offset(j, tid, ldb)) * 2;
+    const int64_t a_step = TA::step(lda), b_step = TB::step(ldb);
+    A = uniform(A + TA::origin(m0, 0, lda)), B = uniform(B + TB::origin(n0, 0, ldb));
+    int p_slot = 0;
+    auto copy_stage = [&]() {
+        const uint32_t to = ring + uint32_t(p_slot) * SLOT;
+#pragma unroll
+        for (int j = 0; j < LA; ++j)
+            async_copy16(to + uint32_t(j) * 4096, A, at_a[j]);
+#pragma unroll
+        for (int j = 0; j < LB; ++j)
+            async_copy16(to + TA::BYTES + uint32_t(j) * 4096, B, at_b[j]);
+        A += a_step, B += b_step;
+        p_slot = p_slot + 1 == S ? 0 : p_slot + 1;
+    };
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s)
+        if (s < k_chunks)
+            copy_stage();
+    int c_slot = 0;
+    for (int c = 0; c < k_chunks; ++c) {
+        const int younger = k_chunks - 1 - c;
+        if (younger >= 2)
+            wait_vmcnt<2 * LOADS>();
+        else if (younger == 1)
+            wait_vmcnt<LOADS>();
+        else
+            wait_vmcnt<0>();
+        __syncthreads(); // everyone's copies are there, and everyone is done with the slot that is refilled next
+        const unsigned char *sa = smem + c_slot * SLOT, *sb = sa + TA::BYTES;
+        bf16x8 af[2][FM], bfr[2][FN];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                af[ks][i] = TA::frag16(sa, wm + i * 16, ks, lane);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                bfr[ks][j] = TB::frag16(sb, wn + j * 16, ks, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + S - 1 < k_chunks)
+            copy_stage();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
+        c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
+    }
+    // the last stage's slot may still be read; the one behind it held the stage S - 1 before, which every wave has left
+    unsigned char *mine = smem + c_slot * SLOT + wave * (WM * WN * 2);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            u32x2 packed;
+            packed.x = pack_bf16(acc[i][j][0], acc[i][j][1]);
+            packed.y = pack_bf16(acc[i][j][2], acc[i][j][3]);
+            *reinterpret_cast<u32x2 *>(mine + (i * 16 + (lane & 15)) * (WN * 2) + j * 32 + (lane >> 4) * 8) = packed;
+        }
+#pragma unroll
+    for (int t = 0; t < PIECES; ++t)
+        epilogue.finish(m[t], n[t], *reinterpret_cast<const u32x4 *>(mine + (t * 64 + lane) * 16), aux[t]);
 }
 
 TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64::frag16's address
@@ -2173,6 +2285,24 @@ void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t
     else
         launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
 }
+template <int BM, int BN, bool BKC, class Epilogue>
+void launch_gemm_uneven(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K, const Epilogue &e) {
+    using Cached = typename Epilogue::Cached; // few outputs: the L2s hold them
+    constexpr int S = 4;
+    auto kernel = gemm_uneven_kernel<BM, BN, S, BKC, Cached>;
+    constexpr size_t lds = S * (BM + BN) * 128;
+    static std::atomic<bool> configured[MAX_DEVICES];
+    const int device = current_device();
+    if (!configured[device].load(std::memory_order_acquire)) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
+                  "gemm LDS size: ");
+        configured[device].store(true, std::memory_order_release);
+    }
+    const int rows = M / BM, cols = N / BN;
+    hipLaunchKernelGGL(kernel, dim3(rows * cols), dim3(256), lds, stream, A, lda, B, ldb, K / 64,
+                       tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Cached{e.any});
+    check_hip(hipGetLastError(), "gemm launch: ");
+}
 template <int BM, int BN, int WM, int WN, int S, bool BKC, class Epilogue>
 void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K, const Epilogue &e) {
     using Cached = typename Epilogue::Cached; // few outputs: the L2s hold them
@@ -2252,6 +2382,17 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
             if (K > 256)
                 return launch_gemm_tile<64, 64, 3, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
             return launch_gemm_tile<64, 64, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+        }
+        // More tiles than units, where tiles half as large again leave no unit with two (gemm_uneven_kernel).  us, 64 x 64 / this,
+        // operands from the caches; from memory; weights [K][N] from the caches; from memory:
+        //   1920 x 640, K = 640 5.9 / 5.8; 6.6 / 6.1   1280 8.5 / 8.7; 10.0 / 8.9; 8.8 / 9.1; 9.9 / 9.2   1920 12.1 / 11.5; 13.4 / 12.5; 12.4 / 12.1; 13.4 / 12.5
+        //   2048 x 768, 640 5.8 / 5.7; 6.6 / 6.1   1280 8.6 / 8.3; 10.0 / 8.6; 8.9 / 9.1; 11.0 / 9.7   3072 18.7 / 15.9; 22.4 / 17.5; 18.6 / 17.5; 18.6 / 17.7
+        // and 384 4.8 / 4.8, 256 4.3 / 4.3.
+        if (K >= (BKC ? 512 : 1536)) {
+            if (M % 96 == 0 && M / 96 * (N / 64) <= compute_units())
+                return launch_gemm_uneven<96, 64, BKC>(stream, A, lda, B, ldb, M, N, K, e);
+            if (N % 96 == 0 && M / 64 * (N / 96) <= compute_units())
+                return launch_gemm_uneven<64, 96, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         }
         return launch_gemm_tile<64, 64, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
     case BLOCK_64x128:
