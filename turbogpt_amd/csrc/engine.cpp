@@ -279,15 +279,19 @@ struct Engine {
             OP(TG_CLASS_OTHER, tgk_embed_fwd(stream, M, T, d, tokens_in, w(layout.embedding), w(layout.positions), x[0]));
         for (int l = 0; l < c.depth; ++l) {
             const TgLayerParameters &p = layout.layers[l];
-            const LayerBuffers &b = layers[l];
-            OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[l], w(p.ln1_g), wl(p.ln1_g), w(p.ln1_b), wl(p.ln1_b), b.n1,
+            // without a backward pass every layer writes where the first one did: the Infinity Cache then holds the weights from one
+            // pass to the next
+            const LayerBuffers &b = layers[with_gradient ? l : 0];
+            const bf16_t *from = x[with_gradient ? l : l & 1];
+            bf16_t *to = x[with_gradient ? l + 1 : (l + 1) & 1];
+            OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, from, w(p.ln1_g), wl(p.ln1_g), w(p.ln1_b), wl(p.ln1_b), b.n1,
                                  config.ln_eps));
             OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, 3 * d, d, b.n1, d, w(p.qkv), d, b.qkv, 3 * d, nullptr, 0, nullptr, 0));
             OP(TG_CLASS_ATTN_FWD, tgk_attn_fwd(stream, batch, config.heads, T, d / config.heads, b.qkv, b.qkv + d, b.qkv + 2 * d,
                             3 * d, b.o, d, b.lse, scale));
             const size_t skip = last_position && l == c.depth - 1 ? size_t(M - RowTile) : 0; // rows nobody reads
             M -= int(skip);
-            const bf16_t *o = b.o + skip * d, *in = x[l] + skip * d;
+            const bf16_t *o = b.o + skip * d, *in = from + skip * d;
             OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, d, o, d, w(p.attn_out), d, b.mid, d, in, d, nullptr, 0));
             OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, b.mid, w(p.ln2_g), wl(p.ln2_g), w(p.ln2_b), wl(p.ln2_b), b.n2,
                                  config.ln_eps));
@@ -295,9 +299,9 @@ struct Engine {
                 OP(TG_CLASS_GEMM_FWD_GELU, tgk_gemm_fwd(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.u, F, nullptr, 0, b.a, F));
             else
                 OP(TG_CLASS_GEMM_FWD_GELU, gemm_fwd_gelu_only(stream, M, F, d, b.n2, d, w(p.mlp_up), d, b.a, F));
-            OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, F, b.a, F, w(p.mlp_down), F, x[l + 1], d, b.mid, d, nullptr, 0));
+            OP(TG_CLASS_GEMM_FWD, tgk_gemm_fwd(stream, M, d, F, b.a, F, w(p.mlp_down), F, to, d, b.mid, d, nullptr, 0));
         }
-        OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[c.depth], w(layout.lnf_g), wl(layout.lnf_g), w(layout.lnf_b),
+        OP(TG_CLASS_LAYERNORM_FWD, tgk_layernorm_fwd(stream, M, d, x[with_gradient ? c.depth : c.depth & 1], w(layout.lnf_g), wl(layout.lnf_g), w(layout.lnf_b),
                              wl(layout.lnf_b), nf, config.ln_eps));
         OP(TG_CLASS_HEAD, tgk_gemm_fwd_t(stream, M, V, d, nf, d, wt(layout.head), V, logits, V, nullptr, 0, nullptr, 0));
         const size_t row = last_position ? size_t(M - 1) : 0; // the first row whose logits are wanted
