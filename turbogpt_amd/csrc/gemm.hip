@@ -1098,9 +1098,10 @@ __global__ __launch_bounds__(128 * (BM / WM) * (BN / WN)) void gemm_waves_kernel
 // ---- tiles whose waves hold an odd number of 16 x 16 products one way ---------------------------------------------------
 // 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48): between 64 x 64 and what choose_block has next.
 // 257 to 384 tiles of 64 x 64 put two on some units and leave others one; these are at most one a unit.  A stage is TileProduct's,
-// with one barrier and every fragment read at once, and costs 0.28 us, two 64 x 64 in company 0.33: copies, reads and products one
-// after the other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 against
-// 16.6 us from the caches, 19.3 and 17.5 against 17.4 from memory), 96 x 32 or 96 x 16 a wave slower (22.8, 19.3).  The sums' order is
+// with one barrier and every fragment read at once, and costs 0.27 us, two 64 x 64 in company 0.38: copies, reads and products one
+// after the other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 us from
+// the caches against 15.6, 19.3 and 17.5 from memory against 16.7), nor are two stages a barrier (17.9; 18.5); 96 x 32 or 96 x 16 a
+// wave are slower (22.8, 19.3).  The sums' order is
 // that of every tile.  Rows of 16-byte pieces: a lane finishes pieces l, l + 64 and l + 128 of its wave's 192.
 template <int BM, int BN, int S, bool BKC, class Epilogue>
 __global__ __launch_bounds__(256) void gemm_uneven_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B, int ldb,
@@ -2383,12 +2384,13 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
                 return launch_gemm_tile<64, 64, 3, BKC, 2>(stream, A, lda, B, ldb, M, N, K, e);
             return launch_gemm_tile<64, 64, 4, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         }
-        // More tiles than units, where tiles half as large again leave no unit with two (gemm_uneven_kernel).  us, 64 x 64 / this,
-        // operands from the caches; from memory; weights [K][N] from the caches; from memory:
-        //   1920 x 640, K = 640 5.9 / 5.8; 6.6 / 6.1   1280 8.5 / 8.7; 10.0 / 8.9; 8.8 / 9.1; 9.9 / 9.2   1920 12.1 / 11.5; 13.4 / 12.5; 12.4 / 12.1; 13.4 / 12.5
-        //   2048 x 768, 640 5.8 / 5.7; 6.6 / 6.1   1280 8.6 / 8.3; 10.0 / 8.6; 8.9 / 9.1; 11.0 / 9.7   3072 18.7 / 15.9; 22.4 / 17.5; 18.6 / 17.5; 18.6 / 17.7
-        // and 384 4.8 / 4.8, 256 4.3 / 4.3.
-        if (K >= (BKC ? 512 : 1536)) {
+        // More tiles than units, where tiles half as large again leave no unit with two (gemm_uneven_kernel); up to K = 256 the launch
+        // is most of either.  us, 64 x 64 / this, operands from the caches; from memory; weights [K][N] from the caches; from memory:
+        //   1920 x 640, K = 256 4.3 / 4.3; 4.5 / 4.4; 4.3 / 4.3; 4.5 / 4.5   384 4.8 / 4.7; 5.2 / 4.9; 4.8 / 4.8; 5.3 / 5.1
+        //   640 5.8 / 5.7; 6.5 / 6.0; 5.9 / 5.9; 6.5 / 6.1   1920 11.9 / 10.8; 13.3 / 12.6; 12.0 / 11.5; 13.5 / 12.3
+        //   2048 x 768, 1280 8.6 / 8.1; 11.4 / 9.2; 9.0 / 8.8; 11.4 / 9.6   3072 18.7 / 15.7; 24.1 / 17.9; 18.6 / 16.7; 25.0 / 19.1
+        //   1408 x 768 (264 tiles), 640 5.6 / 5.4; 6.0 / 5.7; 5.8 / 5.7; 6.1 / 6.0   1920 11.1 / 10.6; 12.4 / 11.5; 11.9 / 11.4; 12.1 / 11.5
+        if (K > 256) {
             if (M % 96 == 0 && M / 96 * (N / 64) <= compute_units())
                 return launch_gemm_uneven<96, 64, BKC>(stream, A, lda, B, ldb, M, N, K, e);
             if (N % 96 == 0 && M / 64 * (N / 96) <= compute_units())
