@@ -1095,9 +1095,9 @@ __global__ __launch_bounds__(128 * (BM / WM) * (BN / WN)) void gemm_waves_kernel
     staged_store_bf16<1, 1>(total, aux, smem + SUMS + wave * 2048, epilogue, m, n, lane);
 }
 
-// ---- tiles whose waves hold an odd number of 16 x 16 products one way ---------------------------------------------------
-// 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48): between 64 x 64 and what choose_block has next.
-// 257 to 384 tiles of 64 x 64 put two on some units and leave others one; these are at most one a unit.  A stage is TileProduct's,
+// ---- tiles between 64 x 64 and 128 x 96, one a unit ---------------------------------------------------
+// 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48), and 128 x 64 (64 x 32).
+// 257 to 384 tiles of 64 x 64 put two on some units and leave others one; these are at most one a unit (launch_block).  A stage is TileProduct's,
 // with one barrier and every fragment read at once, and costs 0.27 us, two 64 x 64 in company 0.38: copies, reads and products one
 // after the other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 us from
 // the caches against 15.6, 19.3 and 17.5 from memory against 16.7), nor are two stages a barrier (17.9; 18.5); 96 x 32 or 96 x 16 a
@@ -2396,6 +2396,13 @@ void launch_block(hipStream_t stream, Block block, const bf16_t *A, int lda, con
             if (N % 96 == 0 && M / 64 * (N / 96) <= compute_units())
                 return launch_gemm_uneven<64, 96, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         }
+        // Two on nearly every unit: one of 128 x 64 instead reads a quarter less, which counts once the operands come from beyond the
+        // L2s.  us, 64 x 64 / 128 x 64, from the caches; from memory; [K][N] likewise:
+        //   2048 x 1024, K = 1024 8.1 / 8.8; 9.3 / 9.3; 8.2 / 8.9; 10.0 / 9.6   1920 14.5 / 14.0; 16.5 / 14.9; 15.3 / 14.2; 16.6 / 14.7
+        //   3072 20.7 / 20.0; 24.5 / 21.6; 22.4 / 20.2; 24.6 / 21.2   4096 x 512, 1920 13.8 / 14.0; 16.7 / 15.3; 14.2 / 14.1; 16.7 / 15.1
+        //   7168 x 256 (448 tiles), 1920 13.6 / 13.8; 17.5 / 15.8; 13.2 / 14.0; 17.0 / 15.4   640 x 2560 (400), 1920 12.4 / 13.5; 16.1 / 14.7
+        if (K >= 1536 && M % 128 == 0 && M / 128 * (N / 64) <= compute_units() && M / 64 * (N / 64) * 4 > compute_units() * 7)
+            return launch_gemm_uneven<128, 64, BKC>(stream, A, lda, B, ldb, M, N, K, e);
         return launch_gemm_tile<64, 64, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
     case BLOCK_64x128:
         return launch_gemm_tile<64, 128, 3, BKC>(stream, A, lda, B, ldb, M, N, K, e);
