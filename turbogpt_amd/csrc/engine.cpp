@@ -91,7 +91,8 @@ struct Slot {
     std::vector<WgradLaunch> wgrads; // one; or one a block, the head's and the token table's
     bf16_t *onehot = nullptr; // [tokens][256]: the token table's gradient is one more product of that launch
     // ... and the kernels that write the gradient leave the sums of its squares here (cuda/trainer.cuh:35-46): the
-    // launch above for the matrices, one more small launch for the ranges in `norm_ranges` (every other tensor)
+    // launch above for the matrices, and with it, of the gradients that are there already, for the ranges in `norm_ranges` (every
+    // other tensor)
     float *norms = nullptr;
     int list_norms = 0, range_norms = 0;
     void *norm_ranges = nullptr;
@@ -348,7 +349,9 @@ struct Engine {
         const auto weight_gradients = [&](const Slot::WgradLaunch &part) {
             Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
             wgrad_list(stream, M, part.count, s.wgrad_jobs.data() + part.first, ListUnit, part.table, workspace, workspace_bytes,
-                       norms ? s.norms : nullptr);
+                       norms ? s.norms : nullptr,
+                       norms ? SumsqSegments{g, static_cast<const SumsqSegment *>(s.norm_ranges), s.range_norms, s.norms + s.list_norms}
+                             : SumsqSegments{});
         };
         OP(TG_CLASS_HEAD, tgk_gemm_dgrad_t(stream, M, V, d, logits, V, wt(layout.head), V, t1, d, nullptr, 0));
         if (!together)
@@ -374,8 +377,6 @@ struct Engine {
                                                   reinterpret_cast<const float *>(s.ln_partials), ln_stride / sizeof(float),
                                                   2 * c.depth + 1, 0, s.ln_targets, s.token_losses, means}));
         weight_gradients(s.wgrads.back());
-        if (norms)
-            OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, s.norm_ranges, s.range_norms, s.norms + s.list_norms));
     }
 
     // learning rates and momenta of optimizer step `at` (0-based)

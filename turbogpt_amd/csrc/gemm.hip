@@ -1939,6 +1939,8 @@ struct WgradTiles {
     int splits = 1;       // `one` only: token ranges a tile is cut into (1 with a list); `count` is tiles x splits
     size_t split_stride;  // then `one.dw` is the first of `splits` slabs this far apart, for splitk_reduce_kernel
     float *sumsq; // optional: one sum of squares a block
+    int blocks = 0;       // of the launch, with a list; those behind them take `ranges`
+    SumsqSegments ranges;
 };
 // One chain of fp32 sums over all tokens is further from 64 bits than slabs of some tokens added up, so the sums of every
 // three stages join a second set.  Relative error in 1e-7 (tokens, N x K: one chain, this, slabs): 512, 3072 x 768 1.25, 0.79,
@@ -1956,9 +1958,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void wgrad_tiles_kernel(const Wgra
     __shared__ float waves[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6 & 3;
     const bool finishes = GROUPS == 1 || threadIdx.x < 256;
+    // they have nothing to do with these products, but were a launch of 4.6 us behind them (a step of d_model 256 over 2048 tokens
+    // 387.9 -> 386.2 us)
+    if (int(blockIdx.x) >= w.blocks)
+        return sumsq_segment(w.ranges, blockIdx.x - w.blocks, waves);
     float squares = 0.f;
-    for (int base = 0; base + int(blockIdx.x) < w.count; base += gridDim.x) {
-        const int at = base + xcd_contiguous(blockIdx.x, min(int(gridDim.x), w.count - base));
+    for (int base = 0; base + int(blockIdx.x) < w.count; base += w.blocks) {
+        const int at = base + xcd_contiguous(blockIdx.x, min(w.blocks, w.count - base));
         // token range by token range, so that an XCD's tiles share their operands' lines
         const int tiles = w.count / w.splits, split = at / tiles, tile = at - split * tiles;
         const int first = int(int64_t(split) * w.k_chunks / w.splits);
@@ -2461,7 +2467,9 @@ template <int BM, int BN, int S, int GROUPS> void launch_wgrad_tiles(hipStream_t
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256 * GROUPS), lds, stream, w);
+    WgradTiles with = w;
+    with.blocks = blocks;
+    hipLaunchKernelGGL(kernel, dim3(blocks + w.ranges.count), dim3(256 * GROUPS), lds, stream, with);
     check_hip(hipGetLastError(), "wgrad tiles launch: ");
 }
 
@@ -2943,7 +2951,7 @@ void wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, int unit, voi
     }
 }
 void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
-                size_t workspace_bytes, float *sumsq) {
+                size_t workspace_bytes, float *sumsq, const SumsqSegments &ranges) {
     {
         WgradListPlan plan;
         std::string why;
@@ -2958,9 +2966,11 @@ void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, i
             WgradTiles w{};
             w.jobs = static_cast<const WgradListJob *>(table);
             w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
-            w.count = plan.tiles, w.k_chunks = M / 64, w.sumsq = sumsq;
+            w.count = plan.tiles, w.k_chunks = M / 64, w.sumsq = sumsq, w.ranges = ranges;
             return launch_wgrad_tiles(stream, w, plan.edge, plan.launch_blocks);
         }
+        if (ranges.count && tgk_sumsq_segments(stream, ranges.g, ranges.segments, ranges.count, ranges.partials))
+            throw std::runtime_error(tg_last_error);
         WgradList w{};
         w.jobs = static_cast<const WgradListJob *>(table);
         w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);

@@ -31,6 +31,33 @@ TG_DEVICE float block_sum_256(float x, float *waves) {
     __syncthreads();
     return (waves[0] + waves[1]) + (waves[2] + waves[3]);
 }
+// Sums of squares of a list of ranges of g, one block of 256 threads per range.  Starts and lengths multiples of 4.
+struct SumsqSegment {
+    int64_t start, length;
+};
+struct SumsqSegments {
+    const float *g;
+    const SumsqSegment *segments;
+    int count;
+    float *partials;
+};
+TG_DEVICE void sumsq_segment(const SumsqSegments &s, int at, float *waves) { // `waves`: shared, 4 floats; the block's first 256 threads
+    const SumsqSegment segment = s.segments[at];
+    const f32x4 *p = reinterpret_cast<const f32x4 *>(s.g + segment.start);
+    const int quads = threadIdx.x < 256 ? int(segment.length >> 2) : 0;
+    float sum = 0.f;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < quads; i += 256) {
+        const f32x4 v = p[i];
+        sum += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+    }
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < 256)
+        waves[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s.partials[at] = (waves[0] + waves[1]) + (waves[2] + waves[3]);
+}
 // Clip factor from the norm partials: every block folds the same partials in the same order (cuda/optim.cuh:67-80).
 TG_DEVICE float clip_factor(float clip, const float *__restrict__ norm_partials, int norm_count, float *waves) {
     if (!(clip > 0.f))
