@@ -703,8 +703,12 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16_t *__restric
 // fetched once per 32 rows instead of once per 128 and that the stages are not double buffered (two blocks of 64 KiB
 // per compute unit fill in for each other); the backward is one launch, because its dK/dV blocks form the deltas of
 // their queries themselves.  Microseconds, 128-row blocks -> these (B, H, T), forward; backward:
-//   1,1,128: 4.6 -> 4.0; 11.6 -> 5.4    8,4,256: 6.5 -> 5.0; 16.7 -> 9.0
-//   1,12,1024: 16.1 -> 8.6; 42.1 -> 20.3    1,4,4096: 53 -> 20; 144 -> 58    1,1,8192: 99 -> 31; 273 -> 79
+//   1,1,128: 4.6 -> 4.0; 11.6 -> 4.9    8,4,256: 6.5 -> 4.7; 16.7 -> 7.5
+//   1,12,1024: 16.1 -> 8.1; 42.1 -> 17.2    1,4,4096: 53 -> 20; 144 -> 51    1,1,8192: 99 -> 29; 273 -> 68
+// What bounds the short ones is the copy path: of the backward's 8.2 us at 8,4,256 (back to back in a graph, where an empty launch
+// takes 1.6) loads and joins alone were 6.1.  The fragments of the block's own 32 rows were a quarter line a lane and load, in
+// each of four waves, and so was O for the deltas.  The own rows now come to LDS once, O as whole lines, and a lane multiplies what
+// it holds of a row: 8,4,256 8.2 -> 6.6, 1,16,1024 26.0 -> 21.1, 1,2,8192 103 -> 94; forward 4.4 -> 4.2, 8.2 -> 7.8, 37.4 -> 34.7.
 // ---------------------------------------------------------------------------------------------
 constexpr int WAVES = 4;
 // this wave's own 64 x 64 tile, rows ld elements apart, in eight copies
@@ -720,6 +724,49 @@ struct WaveTileCopy {
                 async_copy16(__builtin_amdgcn_readfirstlane(lds_tile + (2 * i + odd) * 1024), base + size_t(i) * 16 * ld, offset[odd]);
     }
 };
+// The block's own 32 rows, the first half of a tile's image, eight to a wave.  Read from there they are four fragments a wave for
+// one copy; as fragments from memory each of the four waves asks for 32 lines of which it takes a quarter at a time.
+TG_DEVICE void copy_own_rows(bf16_t *half_tile, const bf16_t *base, int ld, int wave, int lane) {
+    async_copy16(__builtin_amdgcn_readfirstlane(lds_address(half_tile) + wave * 1024), base, tile_copy_offset(ld, wave, lane, 0));
+}
+TG_DEVICE void own_fragments(bf16x8 (&f)[4], const bf16_t *half_tile, const RowFragOffsets &along) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+        f[ks] = along.load(half_tile, 0, ks);
+}
+// Rows' dot products, a row to eight lanes.  First this lane's part: of what it copied to `copied` with the same 16 bytes of another
+// matrix.  Lane 4 b + i holds row i of both factors of block b of the 4 x 4 x 4 instruction, so its part stands on the diagonal: two
+// such instructions and three selections where unpacking and multiplying takes 25 vector instructions.
+TG_DEVICE float chunk_product(const unsigned char *copied, const u32x4 &other, int lane) {
+    const u32x4 mine = *reinterpret_cast<const u32x4 *>(copied);
+    const auto four = [](uint32_t x, uint32_t y) { return __builtin_bit_cast(s16x4, u32x2{x, y}); };
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    sum = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(four(mine[0], mine[1]), four(other[0], other[1]), sum, 0, 0, 0);
+    sum = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(four(mine[2], mine[3]), four(other[2], other[3]), sum, 0, 0, 0);
+    const float even = lane & 2 ? sum[2] : sum[0], odd = lane & 2 ? sum[3] : sum[1];
+    return lane & 1 ? odd : even;
+}
+// the value of another of the eight lanes: the neighbour, the one two further on, the one opposite
+constexpr int NEIGHBOUR = 0xB1, TWO_ON = 0x4E, OPPOSITE = 0x141;
+template <int WHICH> TG_DEVICE float from_lane(float x) {
+    return __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), WHICH, 0xF, 0xF, true)));
+}
+TG_DEVICE float eight_lanes_sum(float x) {
+    x += from_lane<OPPOSITE>(x);
+    x += from_lane<TWO_ON>(x);
+    return x + from_lane<NEIGHBOUR>(x);
+}
+// part[i] summed over the eight lanes, in the lane with lane % 8 = i: each step keeps the half that the lane is in
+TG_DEVICE float eight_sums(const float (&part)[8], int lane) {
+    float four[4], two[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        four[i] = (lane & 4 ? part[i + 4] : part[i]) + from_lane<OPPOSITE>(lane & 4 ? part[i] : part[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        two[i] = (lane & 2 ? four[i + 2] : four[i]) + from_lane<TWO_ON>(lane & 2 ? four[i] : four[i + 2]);
+    return (lane & 1 ? two[1] : two[0]) + from_lane<NEIGHBOUR>(lane & 1 ? two[0] : two[1]);
+}
 // a wave's 32 x 64 sums to its part of LDS, 16 bytes a lane and store
 TG_DEVICE void leave_sums(float *part, const f32x16 (&acc)[2], int lane) {
 #pragma unroll
@@ -752,6 +799,8 @@ TG_DEVICE void store_joined(bf16_t *row, const float (&sum)[8], float scale, int
     *reinterpret_cast<u32x4 *>(row + wave * 16 + 8 * g) = u32x4{x[0], y[0], x[1], y[1]};
 }
 
+// SHARED: the queries come by way of LDS.  At 128 positions only one or two waves want them, which have them sooner from memory.
+template <bool SHARED>
 __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
                                                                 const bf16_t *__restrict__ V, int ld, bf16_t *__restrict__ O,
                                                                 int ldo, float *__restrict__ LSE, int T, CausalGrid grid, float c) {
@@ -770,11 +819,27 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(const bf16_t *__
     bf16x8 qf[4];
     f32x16 o[2] = {zero16(), zero16()};
     float m = -INFINITY, l = 0.f;
-    if (wave < tiles) {
+    const RowFragOffsets krows(lane);
+    const auto first_tile = [&] {
         copy(slot, kbase + size_t(wave) * 64 * ld);
         copy(slot + TILE_ELEMS * 2, vbase + size_t(wave) * 64 * ld);
+    };
+    if constexpr (SHARED) {
+        __shared__ __align__(1024) bf16_t own[TILE_ELEMS / 2];
+        copy_own_rows(own, Q + (token0 + q0) * ld + h * HD, ld, wave, lane);
+        if (wave < tiles) {
+            first_tile();
+            wait_vmcnt<8>(); // the queries and the first tile's keys are there, its values may still be on the way
+        } else {
+            wait_vmcnt<0>();
+        }
+        __syncthreads();
+        own_fragments(qf, own, krows);
+    } else if (wave < tiles) {
+        first_tile();
         load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
-        const RowFragOffsets krows(lane);
+    }
+    if (wave < tiles) {
         const ColFragOffsets vcols(lane);
         for (int j = wave; j < tiles; j += WAVES) {
             const bool more = j + WAVES < tiles;
@@ -837,6 +902,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
     const bf16_t *__restrict__ dO, int lddo, const bf16_t *__restrict__ O, int ldo, const float *__restrict__ LSE,
     bf16_t *__restrict__ dQ, bf16_t *__restrict__ dK, bf16_t *__restrict__ dV, int lddq, int T, CausalGrid grid, float scale) {
     __shared__ __align__(1024) bf16_t tile[WAVES][2][TILE_ELEMS]; // [wave][Q | dO] or [K | V], then the waves' sums
+    __shared__ __align__(1024) bf16_t own[2][TILE_ELEMS / 2];     // K | V or Q | dO
     __shared__ __align__(256) float rows[WAVES][2][64];           // [wave][lse2 | -delta]
     const CausalBlock block = grid.block((blockIdx.x >> 4) * 8 + (blockIdx.x & 7));
     if (!block.live)
@@ -857,38 +923,44 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
     const ColFragOffsets across(lane);
     if (keys) {
         const int k0 = block.rank * 32, krow = k0 + (lane & 31), first = k0 / 64, tiles = T / 64 - first;
+        copy_own_rows(own[0], K + (token0 + k0) * ld + h * HD, ld, wave, lane);
+        copy_own_rows(own[1], V + (token0 + k0) * ld + h * HD, ld, wave, lane);
+        const WaveTileCopy copy_q(ld, lane), copy_g(lddo, lane);
+        const uint32_t o_offset[2] = {tile_copy_offset(ldo, 0, lane, 0), tile_copy_offset(ldo, 1, lane, 0)};
+        u32x4 of[8];
+        float lse = 0.f;
+        // a tile's copies to LDS, and its O as the copies of dO lie
+        const auto request = [&](int q0) {
+            copy_q(slot, Q + (token0 + q0) * ld + h * HD);
+            copy_g(slot + TILE_ELEMS * 2, dO + (token0 + q0) * lddo + h * HD);
+            const char *o = reinterpret_cast<const char *>(O + (token0 + q0) * ldo + h * HD);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                of[i] = *reinterpret_cast<const u32x4 *>(o + size_t(i >> 1) * 32 * ldo + o_offset[i & 1]);
+            lse = lse_row[q0 + lane];
+        };
+        if (wave < tiles)
+            request((first + wave) * 64);
+        wait_vmcnt<0>();
+        __syncthreads();
         if (wave < tiles) {
-            const WaveTileCopy copy_q(ld, lane), copy_g(lddo, lane);
             bf16x8 kf[4], vf[4];
+            own_fragments(kf, own[0], along);
+            own_fragments(vf, own[1], along);
             f32x16 dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
             for (int j = wave; j < tiles; j += WAVES) {
                 const int q0 = (first + j) * 64;
-                copy_q(slot, Q + (token0 + q0) * ld + h * HD);
-                copy_g(slot + TILE_ELEMS * 2, dO + (token0 + q0) * lddo + h * HD);
-                if (j == wave) {
-                    load_row_fragments(kf, K + (token0 + krow) * ld + h * HD, g);
-                    load_row_fragments(vf, V + (token0 + krow) * ld + h * HD, g);
+                if (j != wave) {
+                    request(q0);
+                    wait_vmcnt<0>();
                 }
-                bf16x8 of[2][4];
+                rows[wave][0][lane] = lse * LOG2E;
+                // deltas of the tile's queries: this lane gets that of row 8 * (lane % 8) + lane / 8
+                float part[8];
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-                    load_row_fragments(of[mt], O + (token0 + q0 + mt * 32 + (lane & 31)) * ldo + h * HD, g);
-                rows[wave][0][lane] = lse_row[q0 + lane] * LOG2E;
-                wait_vmcnt<0>();
-                // deltas of the tile's queries: the diagonal of dO O^T, on the matrix cores
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt) {
-                    f32x16 products = zero16();
-#pragma unroll
-                    for (int ks = 0; ks < 4; ++ks)
-                        products = mfma(along.load(tile[wave][1], mt, ks), of[mt][ks], products);
-                    float diagonal = 0.f;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        diagonal = acc_row(r, g) == (lane & 31) ? products[r] : diagonal;
-                    if (((lane >> 2) & 1) == g)
-                        rows[wave][1][mt * 32 + (lane & 31)] = -diagonal;
-                }
+                for (int i = 0; i < 8; ++i)
+                    part[i] = chunk_product(reinterpret_cast<const unsigned char *>(tile[wave][1]) + i * 1024 + lane * 16, of[i], lane);
+                rows[wave][1][(lane & 7) * 8 + (lane >> 3)] = -eight_sums(part, lane);
                 dkdv_tile(tile[wave][0], tile[wave][1], rows[wave][0], rows[wave][1], q0, k0, krow, g, c, along, across, kf, vf,
                           dk, dv);
                 wait_lgkmcnt0(); // the tile has been read
@@ -904,20 +976,32 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
         store_joined(dV + (token0 + krow) * lddq + h * HD, sum, 1.0f, wave, g);
     } else {
         const int q0 = (T / 32 - 1 - block.rank) * 32, qrow = q0 + (lane & 31), tiles = q0 / 64 + 1;
+        const WaveTileCopy copy(ld, lane);
+        const bf16_t *kbase = K + token0 * ld + h * HD, *vbase = V + token0 * ld + h * HD;
+        copy_own_rows(own[0], Q + (token0 + q0) * ld + h * HD, ld, wave, lane);
+        copy_own_rows(own[1], dO + (token0 + q0) * lddo + h * HD, lddo, wave, lane);
+        const u32x4 of = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(O + (token0 + q0) * ldo + h * HD) +
+                                                          tile_copy_offset(ldo, wave, lane, 0));
         if (wave < tiles) {
-            const WaveTileCopy copy(ld, lane);
-            const bf16_t *kbase = K + token0 * ld + h * HD, *vbase = V + token0 * ld + h * HD;
             copy(slot, kbase + size_t(wave) * 64 * ld);
             copy(slot + TILE_ELEMS * 2, vbase + size_t(wave) * 64 * ld);
+        }
+        const float lse = lse_row[qrow] * LOG2E;
+        wait_vmcnt<0>();
+        const float product = eight_lanes_sum(chunk_product(reinterpret_cast<const unsigned char *>(own[1]) + wave * 1024 + lane * 16, of, lane));
+        if (!(lane & 7))
+            rows[0][1][wave * 8 + (lane >> 3)] = -product;
+        __syncthreads();
+        if (wave < tiles) {
             bf16x8 qf[4], gf[4];
-            load_row_fragments(qf, Q + (token0 + qrow) * ld + h * HD, g);
-            load_row_fragments(gf, dO + (token0 + qrow) * lddo + h * HD, g);
-            const float del = row_product(gf, O + (token0 + qrow) * ldo + h * HD, g), lse = lse_row[qrow] * LOG2E;
+            own_fragments(qf, own[0], along);
+            own_fragments(gf, own[1], along);
+            const float minus = rows[0][1][lane & 31];
             f32x16 dq[2] = {zero16(), zero16()};
             f32x16 minus_delta;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                minus_delta[r] = -del;
+                minus_delta[r] = minus;
             for (int j = wave; j < tiles; j += WAVES) {
                 wait_vmcnt<0>();
                 dq_tile(tile[wave][0], tile[wave][1], j * 64, q0, qrow, g, c, lse, along, across, qf, gf, minus_delta, dq);
@@ -936,27 +1020,28 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
 }
 
 // Up to how many 128-row blocks the 32-row ones with shared-out tiles are taken instead.  The longer the context, the
-// longer the chains that they cut, so the line rises with it.  Forward, microseconds, 128-row -> 32-row:
-//   T 128: 128 blocks 5.1 -> 5.0   192: 5.3 -> 7.2     T 256: 128 blocks 6.7 -> 5.7   192: 6.9 -> 8.3
-//   T 512: 192 blocks 10.0 -> 10.0   224: 10.1 -> 10.7     T 1024: 256 blocks 16.7 -> 14.3   320: 17.2 -> 17.5
-//   T 2048: 272 blocks 29.3 -> 20.9   384: 29.1 -> 27.2     T 4096: 384 blocks 57 -> 43
+// longer the chains that they cut, so the line rises with it.  Forward, microseconds, 128-row / 32-row:
+//   T 128: 120 blocks 4.7 / 4.6   144: 5.0 / 6.6     T 256: 128 blocks 6.6 / 5.3   144: 6.8 / 7.3
+//   T 384: 144 blocks 8.2 / 7.6   162: 8.6 / 8.7     T 512: 192 blocks 10.6 / 9.6   256: 11.0 / 11.0
+//   T 768: 252 blocks 14.4 / 12.6     T 1024: 288 blocks 18.1 / 16.2     T 1152: 324 blocks 20.0 / 18.6     T 1536: 384 blocks 26.1 / 24.2
 bool forward_splits(int B, int H, int T) {
-    return size_t(B) * H * (T / 128) <= size_t(std::min(T / 8 + 128, 384));
+    return size_t(B) * H * (T / 128) <= size_t(std::clamp(T / 4 + 64, 128, 384));
 }
 // The backward does five products where the forward does two and loses by the split kernel's fetches sooner.  Next come
-// its two kernels side by side, as long as both sets of blocks are about what the units hold (two each).  Microseconds, split
-// / side by side / one after the other:
-//   T 128: 64 blocks 7.1 / 9.4 / 12.6   128: 10.9 / 9.7 / 13.1   256: 19.0 / 13.5 / 14.4
-//   T 256: 64 blocks 8.9 / 11.7 / 17.1   128: 13.4 / 12.3 / 17.3   256: 22.2 / 15.4 / 18.5   512: 47.9 / 28.3 / 24.6
-//   T 512: 64 blocks 10.7 / 16.3 / 25.0   128: 18.0 / 17.2 / 25.5   256: 30.9 / 20.1 / 26.8   384: 45.1 / 27.6 / 30.0
-//     576: 71.1 / 41.5 / 37.6
-//   T 1024: 96 blocks 19.2 / 26.4 / 41.8   192: 34.9 / 29.1 / 42.5   512: 87.0 / 48.9 / 50.8   768: - / 70.5 / 67.5
-//   T 2048: 128 blocks 37.0 / 45.2 / 74.4   256: 68.0 / 51.1 / 75.7   512: 131 / 78.9 / 87.5   768: - / 112 / 108
-//   T 4096: 256 blocks 114 / 93 / 141   512: 225 / 141 / 163     T 8192: 256 blocks 209 / 178 / 272
+// its two kernels side by side, as long as both sets of blocks are about what the units hold (two each).  Microseconds, split /
+// side by side:
+//   T 128: 128 blocks 10.5 / 10.9   144: 13.3 / 13.0     T 256: 128 blocks 11.9 / 13.3   144: 14.1 / 14.4   154: 15.2 / 14.7
+//   T 384: 144 blocks 16.1 / 16.2   162: 17.4 / 16.8     T 512: 128 blocks 14.9 / 18.2   160: 18.7 / 19.0   192: 20.6 / 19.9
+//   T 768: 144 blocks 20.8 / 23.6   192: 24.8 / 25.0     T 1024: 184 blocks 29.8 / 29.9     T 1280: 200 blocks 33.8 / 35.9
+//   T 1536: 216 blocks 41.2 / 41.1     T 2048: 192 blocks 44.5 / 51.4   208: 53.2 / 52.2     T 4096: 192 blocks 82 / 95   224: 98 / 95
+//   T 8192: 128 blocks 99 / 161   192: 148 / 176   256: 185 / 180
+// and side by side / one after the other:
+//   T 128: 256 blocks 13.5 / 14.4     T 256: 256 blocks 15.4 / 18.5   512: 28.3 / 24.6     T 512: 384 blocks 27.6 / 30.0   576: 41.5 / 37.6
+//   T 1024: 512 blocks 48.9 / 50.8   768: 70.5 / 67.5     T 2048: 512 blocks 78.9 / 87.5   768: 112 / 108     T 4096: 512 blocks 141 / 163
 enum Backward { BACKWARD_SPLIT, BACKWARD_BOTH, BACKWARD_IN_TURN };
 Backward backward_way(int B, int H, int T) {
     const size_t blocks = size_t(B) * H * (T / 128);
-    if (blocks <= size_t(std::min({T / 32 + 104, T / 64 + 128, 216})))
+    if (blocks <= size_t(std::min(T / 16 + 120, 200)))
         return BACKWARD_SPLIT;
     return blocks <= (T < 1024 ? 384 : 512) ? BACKWARD_BOTH : BACKWARD_IN_TURN;
 }
@@ -986,7 +1071,7 @@ extern "C" int tgk_attn_fwd(hipStream_t stream, int B, int H, int T, int hd, con
         require(lse && !(reinterpret_cast<uintptr_t>(lse) & 15), "attention: lse must be 16-byte aligned");
         const bool split = forward_splits(B, H, T);
         const CausalGrid grid = split ? causal_grid(B, H, T, 32) : causal_grid(B, H, T, 128, 64);
-        hipLaunchKernelGGL(split ? attn_fwd_split_kernel : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
+        hipLaunchKernelGGL(split ? (T > 128 ? attn_fwd_split_kernel<true> : attn_fwd_split_kernel<false>) : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
                            ld, O, ldo, lse, T, grid, scale * LOG2E);
         check_hip(hipGetLastError(), "attention forward launch: ");
     });
