@@ -1,5 +1,5 @@
-"""The width-16 network where the cut of the work changes: four or eight waves a block (more than 1024 waves), one wave or eight for
-an element's sum over the blocks (more than sixteen), each on both sides of the line, with last blocks that hold one sequence."""
+"""The width-16 network on batches whose last blocks hold one sequence or few, on sequences that do not fill a wave's sixteen
+tokens, and on few and many blocks."""
 import numpy as np
 import pytest
 

@@ -437,19 +437,18 @@ struct Engine {
         forward(s, v, true, nullptr, c.batch, false, true);
         backward(s, v, history_row(at));
     }
-    // Whether the batches of a call of `steps` steps share their launches.  On K streams a step costs the host 25 us of
+    // Whether the batches of a call of `steps` steps share their launches.  On K streams a step costs the host 32 us of
     // launches and events at least, however small its batch, but steps of one call overlap with those of the next.  A shared launch
-    // takes as long as one batch, 28 us at depth 4 and 43 at depth 8, and 5 us of optimizer a step: worth it from two and from
-    // 2.75 steps a launch on (K = 2: from two), while a batch fills few units.  us a step on streams and shared (depth and
-    // context equal):
-    //   depth 8, 16 sequences: K = 2 29, 27; 4 29, 16; 8 28, 10; at K = 4 calls of one step 26, 50; of two 25, 27; of three 26, 20
-    //   depth 4, 16 sequences: K = 2 28, 18; 8 28, 8; at K = 4 calls of one step 23, 33; of two 29, 18   160 blocks: K = 2 29, 29; 4 26, 22; 8 26, 20
-    //   depth 8, 80 blocks: K = 4 30, 30; 8 29, 24   160 blocks: K = 2 42, 52; 4 35, 40
+    // takes as long as one batch, 48 us at depth 4 and 77 at depth 8, and 8 us of optimizer a step: worth it from two and from 3.25
+    // steps a launch on, while a batch fills few units.  us a step on streams and shared (depth and context equal):
+    //   depth 8, 16 sequences: K = 2 46, 46; 4 37, 27; 16 35, 13; calls of one step at K = 4 38, 81; of five 36, 42
+    //   depth 4, 16 sequences: K = 2 35, 32; 8 34, 13; calls of two 32, 32   640 (40 blocks): K = 4 32, 23
+    //   80 blocks: depth 8, K = 4 46, 44; 8 47, 38; depth 4 35, 30; 36, 24   160 blocks: depth 8, K = 4 60, 69; 8 61, 61; depth 4 36, 41; 38, 38
+    //   depth 8, 10000 sequences, K = 4 379, 395
     bool shares_launches(int steps) const {
         const Config &c = config.base;
         const int K = int(slots.size()), launches = (steps + K - 1) / K;
-        const bool shallow = c.depth == 4;
-        return K == 1 || (w16_blocks(c.batch, c.context) <= (shallow ? 192 : 96) && steps * 4 >= launches * (shallow || K == 2 ? 8 : 11));
+        return K == 1 || (w16_blocks(c.batch, c.context) <= 96 && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
     }
     // Training steps of the width-16 network from `at` on; returns how many.  Batch s reads the weights of version
     // max(floor, s - K + 1), whichever way it is launched.
@@ -468,7 +467,7 @@ struct Engine {
             const uint64_t step = at + uint64_t(i), read = K == 1 ? step : std::max(floor, step + 1 >= K ? step + 1 - K : 0);
             const Slot &s = slots[step % K];
             const Version &v = versions[read % ring];
-            batches[i] = {{v.hi, v.lo}, step, s.workspace, s.token_losses, history_row(step), s.gradient, s.norms};
+            batches[i] = {{v.hi, v.lo}, step, s.input, s.workspace, s.token_losses, history_row(step), s.gradient, s.norms};
             steps[i] = w16_step(step, s.gradient, s.norms, versions[step % ring], versions[(step + 1) % ring]);
             trace[i] = int(read);
             total_staleness += step - read;

@@ -14,11 +14,12 @@ struct W16Data {
     int64_t size;
     uint64_t seed;
 };
-// One batch: the weights that it reads, the step that it is drawn for, and what it leaves: its losses and their
+// One batch: the weights that it reads, the step that it is drawn for, and what it leaves: its tokens, losses and their
 // per-position means, the gradient, and w16_norm_count(depth) sums of the gradient's squares in w16_norm_parts() parts each.
 struct W16Batch {
     W16Weights weights;
     uint64_t step;
+    uint8_t *tokens;
     void *workspace;
     float *token_losses, *means, *gradient, *norms;
 };

@@ -5,17 +5,17 @@
 //
 // What bounds it is latency: a step is 1 GFLOP over some ten thousand tokens, and a sequence (at most eight positions)
 // never leaves a wave.  So a wave takes sixteen tokens - whole sequences - through all layers in registers, forward and
-// backward, with the weights in LDS as they are in memory.  Every factor of a product is a bf16 value, so products run on the
-// bf16 matrix instructions, sixteen or thirty-two features at a time: 16 x 16 x 16 outputs are one instruction where the fp32 form
-// takes four that wait for one another, and operands need no conversion.  Their sums are closer to 64 bits than a chain of fmaf in
-// the features' order (normal factors, 16 / 48 / 256 terms: relative error 1.9e-8 / 3.7e-8 / 8.6e-8 against 2.2e-8 / 4.4e-8 /
-// 1.07e-7), and an output depends on its own row and column alone, so results do not depend on how the tokens are cut.
-// Lane 16 g + c holds features 4 g .. 4 g + 3 of token c: what such an instruction gives is what the next one takes, and head
-// g of the token, one head a lane, so attention reads other positions' keys and values with DPP row shifts.
-// Weight gradients are products over tokens: the waves of a block leave a layer's rows in LDS, the transposing load reads them
-// across, and each wave sums some of the layer's tiles over the block's tokens; another launch adds the blocks' sums in order.
-// No atomics, bit-reproducible (the place of weight_gradient's read-modify-write and of reduce_gradients,
-// cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
+// backward, with the weights staged in LDS as matrix operands.  Products run on
+// v_mfma_f32_16x16x4_f32, which is bit for bit a chain of fmaf over its four k (measured on random and extreme values;
+// the bf16 forms add in an order of their own): every sum has one order, the k's own, whatever the kernel's shape, so
+// results do not depend on how the work is cut.  Lane 16 g + c works for token c:
+//   "feed" layout: register j holds feature 4 j + g - what step j of a product over features wants from that lane;
+//   "head" layout: register r holds feature 4 g + r - head g of the token, one head a lane, so attention reads other
+//   positions' keys and values with DPP row shifts.
+// A product's results come out in either, by the order of the weight's rows.  Weight gradients are products over tokens,
+// another launch: a block for the rows that one layer kept of a chunk of tokens, which the transposing load reads across,
+// so that a chain of fmaf runs over the tokens in order; one more folds the chunks in order.  No atomics, bit-reproducible
+// (the place of weight_gradient's read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
 #include "common.h"
 #include "width16.h"
 #include "../../include/tgk_kernels.h"
@@ -29,7 +29,8 @@
 namespace {
 
 constexpr int W = 16, HEADS = 4, F = 48, V = 256, MAX_DEPTH = 8;
-constexpr int MAX_WAVES = 8; // waves of a block: they share the staged weights
+constexpr int WAVES = 4;       // waves of a block: they share the staged weights
+constexpr int CHUNK_WAVES = 8; // waves' tokens in one partial sum of a weight gradient (128 tokens)
 
 struct Layer {
     int attention_norm, qkv, attention, mlp_norm, gate, up, down;
@@ -61,32 +62,37 @@ Layout make_layout(int depth) {
     return p;
 }
 
-// What a layer's forward pass keeps for its backward pass, 16 bytes a lane and slot: block input | post-attention residual,
-// post-RoPE query | winning key, winning value | the two inverse norms, GELU(top) | GELU'(top) | distance to the winner, gate | up
-// thrice, the gates' sigmoids thrice (cuda/types.cuh:40-44, cuda/model.cuh:25-29).  What else the backward pass wants it
-// computes again: normalised rows, attention output and activation are a product of two of these each.
-enum Slot { S_RESIDUAL, S_QUERY_KEY, S_VALUE_NORMS, S_GATE, S_GATE_UP, S_SIGMOID = S_GATE_UP + 3, SLOTS = S_SIGMOID + 3 };
+// Rows kept between the launches, a tile of 64 x 8 bytes a wave and quantity in the lanes' own order.  For the backward
+// pass: block input, post-RoPE query, the winning key and value (head layout), post-attention residual, gate | up
+// (cuda/types.cuh:40-44, cuda/model.cuh:25-29).  For the weight gradients, side by side: normalised rows, attention output,
+// activation, and the gradients that are their other operands.  And words: GELU(top), GELU'(top), distance to the
+// winner, the two inverse norms.
+enum Tile {
+    T_X, T_Q, T_KEY, T_VALUE, T_MIDDLE, T_GU, T_OPERANDS = T_GU + 6,
+    T_N1 = T_OPERANDS, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES
+};
+constexpr int OPERANDS = TILES - T_OPERANDS;
+enum Word { WORD_GATE, WORD_SLOPE, WORD_DISTANCE, WORD_INV1, WORD_INV2, WORDS };
 struct Workspace {
-    u32x4 *rows;               // [depth][waves][SLOTS][64]
-    u32x2 *hidden, *nf;        // [waves][64], of the head
-    float *inverse;            // [waves][64], of the final norm
-    u32x2 *dlogits;            // [waves][16][64]
-    float *partials;           // [blocks][parameters]
-    int waves, blocks, waves_per_block;
+    u32x2 *tiles;    // [depth][waves][TILES][64]
+    float *words;    // [depth][waves][WORDS][64]
+    float *gz;       // [2 depth + 1][waves * 16][16]: g * z of every RMSNorm scale; the final norm's last
+    u32x2 *hidden, *nf, *dh; // [waves][64]
+    float *inverse;  // [waves][64] of the final norm
+    u32x2 *dlogits;  // [waves][16][64]
+    float *partials; // [chunks][parameters]
+    int waves, blocks, chunks;
     size_t bytes;
 };
 // another batch's, whose memory lies `apart` bytes further on
 TG_DEVICE Workspace moved(Workspace s, int64_t apart) {
     const auto move = [&](auto *&p) { p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<char *>(p) + apart); };
-    move(s.rows), move(s.hidden), move(s.nf), move(s.inverse), move(s.dlogits), move(s.partials);
+    move(s.tiles), move(s.words), move(s.gz), move(s.hidden), move(s.nf), move(s.dh), move(s.inverse), move(s.dlogits), move(s.partials);
     return s;
 }
 int tokens_per_wave(int context) { return 16 / context * context; }
-// Four waves, one to a SIMD; eight where that fills more than the 256 units, whose LDS has room for one block each at depth 8: a
-// step of 2304 sequences of 8 there 98 us with four, 75 with eight; of 10000 270 and 224; 4608 of 4 at depth 4 52 and 49.
-int waves_per_block(int batch, int context) { return batch * context > tokens_per_wave(context) * 4 * 256 ? 8 : 4; }
 int blocks_of(int batch, int context) {
-    const int per_block = tokens_per_wave(context) * waves_per_block(batch, context);
+    const int per_block = tokens_per_wave(context) * WAVES;
     return (batch * context + per_block - 1) / per_block;
 }
 Workspace carve(int depth, int batch, int context, void *base) {
@@ -97,16 +103,19 @@ Workspace carve(int depth, int batch, int context, void *base) {
         at += (bytes + 255) & ~size_t(255);
         return p;
     };
-    r.waves_per_block = waves_per_block(batch, context);
     r.blocks = blocks_of(batch, context);
-    r.waves = r.blocks * r.waves_per_block;
+    r.waves = r.blocks * WAVES;
+    r.chunks = (r.waves + CHUNK_WAVES - 1) / CHUNK_WAVES;
     const size_t n = size_t(r.waves) * 64;
-    r.rows = static_cast<u32x4 *>(take(n * depth * SLOTS * sizeof(u32x4)));
+    r.tiles = static_cast<u32x2 *>(take(n * depth * TILES * sizeof(u32x2)));
+    r.words = static_cast<float *>(take(n * depth * WORDS * sizeof(float)));
+    r.gz = static_cast<float *>(take(n * (2 * depth + 1) * 4 * sizeof(float)));
     r.hidden = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
     r.nf = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
+    r.dh = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
     r.inverse = static_cast<float *>(take(n * sizeof(float)));
     r.dlogits = static_cast<u32x2 *>(take(n * 16 * sizeof(u32x2)));
-    r.partials = static_cast<float *>(take(size_t(r.blocks) * make_layout(depth).count * sizeof(float)));
+    r.partials = static_cast<float *>(take(size_t(r.chunks) * make_layout(depth).count * sizeof(float)));
     r.bytes = at;
     return r;
 }
@@ -129,6 +138,14 @@ TG_DEVICE f32x4 rounded(const f32x4 &v) {
     return unpack4(pack4(v));
 }
 constexpr f32x4 ZERO = {0.f, 0.f, 0.f, 0.f};
+// D[row][col] = fmaf chain over k = 0 .. 15 of A[row][k] B[k][col], on top of acc: lane 16 g + c gives A[c][4 j + g] and
+// B[4 j + g][c] in register j and gets D[4 g + r][c] in register r
+TG_DEVICE f32x4 multiply(const f32x4 &a, const f32x4 &b, f32x4 acc = ZERO) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+    return acc;
+}
 TG_DEVICE float swap_add_16(float x) {
     const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
@@ -137,28 +154,19 @@ TG_DEVICE float swap_add_32(float x) {
     const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
 }
-TG_DEVICE float token_sum(const f32x4 &x) { // over a token's sixteen features
-    return swap_add_32(swap_add_16((x[0] + x[1]) + (x[2] + x[3])));
-}
 TG_DEVICE float token_max(float x) { // over the four lanes that hold one token
     const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     x = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
     const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
 }
-// D[row][col] = sum over k of A[row][k] B[k][col] on top of acc, factors in bf16: lane 16 g + c gives A[c][4 g + j] and
-// B[4 g + j][c] in element j and gets D[4 g + r][c] in register r; with two pairs of factors, k = 0 .. 15 of both.  A sum of three is
-// two of the second form, with zeros: the first form right behind the second, adding to its result, gave wrong sums, and the
-// compiler puts nothing between them.
-TG_DEVICE f32x4 product(u32x2 a, u32x2 b, f32x4 acc = ZERO) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), acc, 0, 0, 0);
-}
-TG_DEVICE f32x4 product(u32x2 a0, u32x2 b0, u32x2 a1, u32x2 b1, f32x4 acc = ZERO) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, u32x4{a0.x, a0.y, a1.x, a1.y}),
-                                                   __builtin_bit_cast(bf16x8, u32x4{b0.x, b0.y, b1.x, b1.y}), acc, 0, 0, 0);
-}
-TG_DEVICE f32x4 product(u32x2 a0, u32x2 b0, u32x2 a1, u32x2 b1, u32x2 a2, u32x2 b2) {
-    return product(a2, b2, u32x2{0, 0}, u32x2{0, 0}, product(a0, b0, a1, b1));
+// head layout <-> feed layout: the 4 x 4 transposition of (lane group, register)
+TG_DEVICE f32x4 turned(const f32x4 &v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return f32x4{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1])};
 }
 // the value of the lane D before / after this one in its row of sixteen (0 beyond the row)
 template <int D> TG_DEVICE uint32_t earlier(uint32_t x) {
@@ -196,18 +204,10 @@ TG_DEVICE float divide(float x, float b, float r) {
     const float q = x * r;
     return fmaf(fmaf(-q, b, x), r, q);
 }
-// e^x with the error of the library's (against 64 bits over (-87, 0) and (0, 88): 2.6e-8 of the value, at most 8.3e-8): 2^n times
-// 2^f of the hardware, f within half of 0 and with what the rounding of x / ln 2 lost.  The bounds put in place of the library's
-// two selections let infinities and NaN through the second term: ten instructions where it takes thirteen.
-TG_DEVICE float exponential(float x) {
-    constexpr float PER_LN2 = 1.44269504088896341f, REST = 1.92596299e-8f; // 1 / ln 2 in two parts
-    const float t = __builtin_amdgcn_fmed3f(x * PER_LN2, -200.f, 200.f), n = rintf(t);
-    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + fmaf(x, REST, fmaf(x, PER_LN2, -t))), int(n));
-}
 // 1 / (1 + e^-x) taken 2^24 times too large, where the reciprocal stays in the normal range down to e^-x = 2^128; beyond that
 // 2^-126 stands for it, which the last product rounds to 0.
 TG_DEVICE float sigmoid(float x) {
-    return reciprocal(fminf(fmaf(exponential(-x), 0x1p-24f, 0x1p-24f), 0x1p126f)) * 0x1p-24f;
+    return reciprocal(fminf(fmaf(expf(-x), 0x1p-24f, 0x1p-24f), 0x1p126f)) * 0x1p-24f;
 }
 
 struct Model {
@@ -220,7 +220,7 @@ struct Lane {
     int lane, c, g, wave, token, position;
     bool live;
 };
-template <int WAVES> TG_DEVICE Lane lane_of(const Model &m) {
+TG_DEVICE Lane lane_of(const Model &m) {
     Lane p;
     p.lane = threadIdx.x & 63;
     p.c = p.lane & 15;
@@ -232,86 +232,183 @@ template <int WAVES> TG_DEVICE Lane lane_of(const Model &m) {
     return p;
 }
 
-// A block's LDS: the weights' upper halves as they are in memory, from the embedding to the head, so that staging them is a
-// copy and a token's row no further trip to memory behind the token's own; every RMSNorm scale in fp32; and for weight gradients
-// each wave's rows, TILES tiles of 64 x 8 bytes in the lanes' order, its sums of the scales' gradients, and its tokens.
-// Of a matrix of rows of 32 bytes a lane reads 8, operand of dX W^T; the transposing load gives it the operand of dY W.
-constexpr int LAYER_BYTES = LAYER_SIZE * 2, QKV_AT = W * 2, ATTENTION_AT = QKV_AT + 3 * W * W * 2, GATE_AT = ATTENTION_AT + W * W * 2 + W * 2,
-              UP_AT = GATE_AT + F * W * 2, DOWN_AT = UP_AT + F * W * 2, TILE = W * W * 2;
-// of a layer; the head's dlogits and normalised rows, and the embedding's gradient, take their places
-enum Tile { T_N1, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES };
-constexpr int T_DLOGITS = 0, T_NF = 16, T_DH = 0;
-static_assert(TILES == 17, "the head's tiles fit a layer's");
-__host__ __device__ constexpr int layer_at(int l) { return V * W * 2 + l * LAYER_BYTES; }
-__host__ __device__ constexpr int head_at(int depth) { return layer_at(depth) + W * 2; }
-__host__ __device__ constexpr int scales_at(int depth) { return head_at(depth) + V * W * 2; }
-__host__ __device__ constexpr int rows_at(int depth) { return scales_at(depth) + (2 * depth + 1) * W * 4; }
-__host__ __device__ constexpr int sums_at(int depth, int waves) { return rows_at(depth) + waves * TILES * 512; }
-__host__ __device__ constexpr int ids_at(int depth, int waves) { return sums_at(depth, waves) + (2 * depth + 1) * waves * W * 4; }
-__host__ __device__ constexpr int lds_bytes(int depth, int waves, bool gradients) {
-    return gradients ? ids_at(depth, waves) + waves * 16 : rows_at(depth);
-}
-static_assert(layer_at(1) % 16 == 0 && head_at(1) % 16 == 0 && lds_bytes(MAX_DEPTH, MAX_WAVES, true) <= 160 * 1024, "LDS of a unit");
-
-// `aligned` is false where the weights do not lie on 16 bytes
-template <int WAVES> TG_DEVICE void stage(const Model &m, unsigned char *memory, bool aligned = true) {
-    constexpr int THREADS = 64 * WAVES;
-    const int bytes = scales_at(m.depth), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (aligned) {
-        const uint32_t lds = lds_address(memory) + uint32_t(wave * 1024);
-        for (int at = 0; at < bytes; at += THREADS * 16) {
-            const int mine = at + int(threadIdx.x) * 16;
-            if (mine < bytes)
-                async_copy16(lds + uint32_t(at), m.hi, uint32_t(mine));
-        }
-    } else {
-#pragma unroll 4
-        for (int at = int(threadIdx.x) * 8; at < bytes; at += THREADS * 8)
-            *reinterpret_cast<u32x2 *>(memory + at) = *reinterpret_cast<const u32x2 *>(reinterpret_cast<const char *>(m.hi) + at);
-    }
-    float *scales = reinterpret_cast<float *>(memory + scales_at(m.depth));
-    for (int at = threadIdx.x; at < (2 * m.depth + 1) * W; at += THREADS) {
-        const int n = at >> 4; // attention and MLP norm of each layer, final
-        const Layer q = layer_layout(n >> 1);
-        const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
-        scales[at] = master(m.hi, m.lo, offset + (at & 15));
-    }
-    wait_vmcnt<0>();
-    __syncthreads();
+// The weights in LDS as first operands, a tile of 64 x 8 bytes each (lane 16 g + c: elements (row c, k = 4 j + g), j = 0..3):
+// 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
+// The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
+// Operands of dX = dY W (rows = inputs, k = outputs) are read from the same tiles with the transposing load, in feed
+// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Last
+// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own.
+constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
+__host__ __device__ constexpr int staged_tiles(int depth) { return depth * (LAYER_TILES + 1) + HEAD_TILES; }
+__host__ __device__ constexpr size_t embedding_at(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
+__host__ __device__ constexpr size_t staged_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
+TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its own inverse
+// Byte offset, in a tile of items (g, c), of the item that lane 16 q + 4 j + m addresses for a transposing load: (m, 4 q + j)
+// or (m, 4 j + q).  Lane 16 q + i then gets element i % 4 of items (i / 4, 4 q + 0..3) or (i / 4, 4 * 0..3 + q).
+TG_DEVICE int across_offset(int lane, bool natural) {
+    const int q = lane >> 4, j = (lane >> 2) & 3, m = lane & 3;
+    return (16 * m + (natural ? 4 * j + q : 4 * q + j)) * 8;
 }
 TG_DEVICE u32x2 read_across(const unsigned char *at) {
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)at));
 }
-// Lane 16 q + 4 j + m addresses eight bytes for a transposing load, and lane 16 q + i gets element i % 4 of what lanes
-// 16 q + 4 * 0..3 + i / 4 address: with row 4 q + j, columns 4 m .. there, rows 4 q .. 4 q + 3 of column i.
-struct Staged {
-    const unsigned char *memory, *mine, *mine_down, *across, *across_down; // `down` has rows of 96 bytes
-    const float *scales;
-    int head;
-    TG_DEVICE Staged(const Model &m, const unsigned char *memory_, const Lane &p) : memory(memory_) {
-        const int row = 4 * p.g + ((p.lane >> 2) & 3), column = p.lane & 3;
-        mine = memory + p.c * 32 + p.g * 8, mine_down = memory + DOWN_AT + p.c * 96 + p.g * 8;
-        across = memory + row * 32 + column * 8, across_down = memory + DOWN_AT + row * 96 + column * 8;
-        scales = reinterpret_cast<const float *>(memory + scales_at(m.depth)) + 4 * p.g;
-        head = head_at(m.depth);
+// Wave w stages tiles w, w + 4 and w + 8 of every layer, the thirteenth of layers w and w + 4, and four of the head's: all
+// loads go out before the first is waited for, and every address is a layer's away from the one before.
+struct Staging {
+    static constexpr int PER_LAYER = 3, TAIL = MAX_DEPTH * PER_LAYER, LAST = MAX_DEPTH / WAVES, HEADS = HEAD_TILES / WAVES, SCALES = 2;
+    const Model &m;
+    unsigned char *tiles;
+    u32x2 v[TAIL + LAST + HEADS];
+    float scale[SCALES];
+    int lane, wave;
+    TG_DEVICE Staging(const Model &m_, unsigned char *memory)
+        : m(m_), tiles(memory), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
+    TG_DEVICE float *scales() const { return reinterpret_cast<float *>(tiles + staged_tiles(m.depth) * 512); }
+    // a lane brings four elements of one row: k = 4 (lane % 4) .. + 3
+    TG_DEVICE int row_offset(int width) const { return (lane >> 2) * width + (lane & 3) * 4; }
+    TG_DEVICE static int tile_offset(int k) { // of tile k in its layer's weights
+        const Layer q = layer_layout(0);
+        return k < 4 ? q.qkv + k * 256 : k < 10 ? q.gate + (k - 4) * 256 : q.down + (k - 10) * 16;
     }
-    // operands of X W^T and of dY W: sixteen rows of a matrix; sixteen columns of `down`
-    TG_DEVICE u32x2 operator()(int at) const { return *reinterpret_cast<const u32x2 *>(mine + at); }
-    TG_DEVICE u32x2 down(int layer, int t) const { return *reinterpret_cast<const u32x2 *>(mine_down + layer + t * 32); }
-    TG_DEVICE u32x2 turned(int at) const { return read_across(across + at); }
-    TG_DEVICE u32x2 turned_down(int layer, int t) const { return read_across(across_down + layer + t * 32); }
-    TG_DEVICE f32x4 scale(int norm) const { return *reinterpret_cast<const f32x4 *>(scales + norm * W); }
+    TG_DEVICE void request() {
+        const bf16_t *of_layer[PER_LAYER], *last = m.hi + tile_offset(12) + wave * LAYER_SIZE + row_offset(F);
+#pragma unroll
+        for (int i = 0; i < PER_LAYER; ++i) // rows of `down` are 48 long
+            of_layer[i] = m.hi + tile_offset(wave + i * WAVES) + (wave + i * WAVES < 10 ? row_offset(W) : row_offset(F));
+#pragma unroll
+        for (int l = 0; l < MAX_DEPTH; ++l)
+            if (l < m.depth)
+#pragma unroll
+                for (int i = 0; i < PER_LAYER; ++i)
+                    v[l * PER_LAYER + i] = *reinterpret_cast<const u32x2 *>(of_layer[i] + l * LAYER_SIZE);
+#pragma unroll
+        for (int i = 0; i < LAST; ++i)
+            if (wave + i * WAVES < m.depth)
+                v[TAIL + i] = *reinterpret_cast<const u32x2 *>(last + i * WAVES * LAYER_SIZE);
+        const bf16_t *head = m.hi + V * W + m.depth * LAYER_SIZE + W + wave * 256 + row_offset(W);
+#pragma unroll
+        for (int i = 0; i < HEADS; ++i)
+            v[TAIL + LAST + i] = *reinterpret_cast<const u32x2 *>(head + i * WAVES * 256);
+#pragma unroll
+        for (int i = 0; i < SCALES; ++i) {
+            const int at = threadIdx.x + i * 64 * WAVES, n = at >> 4; // attention and MLP norm of each layer, final
+            const Layer q = layer_layout(n >> 1);
+            const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
+            if (n <= 2 * m.depth)
+                scale[i] = master(m.hi, m.lo, offset + (at & 15));
+        }
+    }
+    // 8 KiB, 16 bytes a lane; `aligned` is false where the weights are not
+    TG_DEVICE void request_embedding(bool aligned = true) const {
+        if (!aligned) {
+            const u32x2 *from = reinterpret_cast<const u32x2 *>(m.hi);
+            u32x2 *to = reinterpret_cast<u32x2 *>(tiles + embedding_at(m.depth));
+#pragma unroll
+            for (int i = 0; i < V * W / 4 / (64 * WAVES); ++i)
+                to[threadIdx.x + i * 64 * WAVES] = from[threadIdx.x + i * 64 * WAVES];
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < V * W * 2 / 1024 / WAVES; ++i) {
+            const int piece = i * WAVES + wave;
+            async_copy16(lds_address(tiles) + uint32_t(embedding_at(m.depth)) + uint32_t(piece * 1024), m.hi, uint32_t(piece * 1024 + lane * 16));
+        }
+    }
+    TG_DEVICE static uint16_t element(const u32x2 &v, int e) { return uint16_t((e < 2 ? v.x : v.y) >> ((e & 1) * 16)); }
+    // element e of a lane's four is k = 4 j + e: item (e, row), element j.  `to`: the lane's place in the tile
+    TG_DEVICE static void put(unsigned char *to, const u32x2 &v) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint16_t *>(to + e * 128) = element(v, e);
+    }
+    TG_DEVICE void finish(bool backward) {
+        const int row = lane >> 2, j = lane & 3;
+        unsigned char *natural = tiles + row * 8 + j * 2, *feed = tiles + feed_row(row) * 8 + j * 2, *of_layer[PER_LAYER];
+#pragma unroll
+        for (int i = 0; i < PER_LAYER; ++i)
+            of_layer[i] = (wave + i * WAVES > 2 ? feed : natural) + (wave + i * WAVES) * 512;
+        // the attention projection (wave 3's first) again: rows = inputs 4 j + e, k = output `row`: item (row % 4, input), element row / 4
+        unsigned char *turned = tiles + (m.depth * LAYER_TILES + HEAD_TILES) * 512 + ((row & 3) * 16 + 4 * j) * 8 + (row >> 2) * 2;
+#pragma unroll
+        for (int l = 0; l < MAX_DEPTH; ++l)
+            if (l < m.depth) {
+#pragma unroll
+                for (int i = 0; i < PER_LAYER; ++i)
+                    put(of_layer[i] + l * LAYER_TILES * 512, v[l * PER_LAYER + i]);
+                if (backward && wave == 3)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        *reinterpret_cast<uint16_t *>(turned + l * 512 + e * 8) = element(v[l * PER_LAYER], e);
+            }
+#pragma unroll
+        for (int i = 0; i < LAST; ++i)
+            if (wave + i * WAVES < m.depth)
+                put(feed + ((wave + i * WAVES) * LAYER_TILES + 12) * 512, v[TAIL + i]);
+#pragma unroll
+        for (int i = 0; i < HEADS; ++i)
+            put(feed + (m.depth * LAYER_TILES + wave + i * WAVES) * 512, v[TAIL + LAST + i]);
+#pragma unroll
+        for (int i = 0; i < SCALES; ++i) {
+            const int at = threadIdx.x + i * 64 * WAVES;
+            if (at < (2 * m.depth + 1) * W)
+                scales()[at] = scale[i];
+        }
+        wait_vmcnt<0>(); // the embedding
+        __syncthreads();
+    }
+};
+static_assert(Staging::SCALES * 64 * WAVES >= (2 * MAX_DEPTH + 1) * W && LAYER_TILES == Staging::PER_LAYER * WAVES + 1,
+              "every scale has a thread, every tile a wave");
+struct Staged {
+    const unsigned char *tiles;
+    const float *scales;
+    int lane, g, head, turned_attention; // tiles: the head's first, the first attention projection for the backward pass
+    int feed, natural; // across_offset
+    TG_DEVICE Staged(const Model &m, const unsigned char *memory, const Lane &p)
+        : tiles(memory), scales(reinterpret_cast<const float *>(memory + staged_tiles(m.depth) * 512)), lane(p.lane), g(p.g),
+          head(m.depth * LAYER_TILES), turned_attention(head + HEAD_TILES), feed(across_offset(p.lane, false)),
+          natural(across_offset(p.lane, true)) {}
+    TG_DEVICE f32x4 operator()(int tile) const { return unpack4(*reinterpret_cast<const u32x2 *>(tiles + tile * 512 + lane * 8)); }
+    // the transposed operand, of a tile in feed order or (q, k, v) in the matrix's own
+    TG_DEVICE f32x4 turned_feed(int tile) const { return unpack4(read_across(tiles + tile * 512 + feed)); }
+    TG_DEVICE f32x4 turned_natural(int tile) const { return unpack4(read_across(tiles + tile * 512 + natural)); }
+    TG_DEVICE f32x4 scale(int norm) const {
+        const float *s = scales + norm * W + g;
+        return f32x4{s[0], s[4], s[8], s[12]};
+    }
 };
 
-// cuda/ops.cuh:57-67: y = RN_bf16(v * rsqrt(mean(v^2) + 1e-6) * scale), scale read in full fp32
-TG_DEVICE float inverse_rms(const f32x4 &v) {
-    return __builtin_amdgcn_rsqf(token_sum(v * v) * (1.f / 16.f) + 1e-6f); // never denormal
+// feed-layout rows times feed-layout rows of the same token, an fmaf chain in feature order: the diagonal of a product
+TG_DEVICE float token_dot(const f32x4 &a, const f32x4 &b, const Lane &p) {
+    const f32x4 all = multiply(a, b);
+    float mine = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        mine = 4 * p.g + r == p.c ? all[r] : mine;
+    return swap_add_32(swap_add_16(mine)); // the other three lanes hold zeros
 }
-// cuda/ops.cuh:68-80: the rounded input gradient of a row of inverse norm `inv` with z = v * inv
-TG_DEVICE f32x4 normalize_backward(const f32x4 &z, float inv, const f32x4 &g, const f32x4 &scale) {
-    const f32x4 dz = g * scale;
-    const float dot = token_sum(dz * z);
-    return rounded((dz - z * dot * (1.f / 16.f)) * inv);
+// cuda/ops.cuh:57-67: y = RN_bf16(v * rsqrt(mean(v^2) + 1e-6) * scale), scale read in full fp32
+TG_DEVICE float inverse_rms(const f32x4 &v, const Lane &p) {
+    const float sum = token_dot(v, v, p);
+    return rsqrtf(sum * (1.f / 16.f) + 1e-6f);
+}
+TG_DEVICE u32x2 normalize(const f32x4 &v, float inv, const f32x4 &scale) {
+    return pack4(f32x4{v[0] * inv * scale[0], v[1] * inv * scale[1], v[2] * inv * scale[2], v[3] * inv * scale[3]});
+}
+// cuda/ops.cuh:68-80: the rounded input gradient; the token's g * z terms of the scale gradient go to gz
+TG_DEVICE f32x4 normalize_backward(const f32x4 &v, float inv, const f32x4 &g, const f32x4 &scale, float *gz, const Lane &p) {
+    f32x4 z, dz, dx;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z[i] = v[i] * inv;
+        dz[i] = g[i] * scale[i];
+        gz[4 * i] = g[i] * z[i];
+    }
+    const float dot = token_dot(dz, z, p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        dx[i] = round_bf16((dz[i] - z[i] * dot * (1.f / 16.f)) * inv);
+    return dx;
 }
 // cuda/attention.cuh:19-30: first pair of every query and key head, one radian per position
 TG_DEVICE void rotation(int position, float &c, float &s) {
@@ -348,25 +445,14 @@ struct Group {
 };
 
 // ---- forward ---------------------------------------------------------------------------------------
-// What the head leaves for the backward pass; the logits' gradients in tiles of sixteen, but for the target's: lane g = target / 4
-// % 4 has that (`at` in its own four of tile `tile`), the others none.
+// What the head leaves for the backward pass; the logits' gradients in tiles of sixteen.
 struct Head {
-    u32x2 dlogits[16], hidden, nf;
+    u32x2 dlogits[16], hidden;
     float inverse;
-    bool holder;
-    int tile, at;
-    bf16_t of_target;
-    // into a tile's four elements of this lane, behind the others
-    template <class Place> TG_DEVICE void put(Place &&place) const {
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-            *reinterpret_cast<u32x2 *>(place(t)) = dlogits[t];
-        if (holder)
-            reinterpret_cast<bf16_t *>(place(tile))[at] = of_target;
-    }
 };
-TG_DEVICE f32x4 embedding_row(const unsigned char *memory, const Lane &p, int token) {
-    return p.live ? unpack4(*reinterpret_cast<const u32x2 *>(memory + token * W * 2 + p.g * 8)) : ZERO;
+TG_DEVICE f32x4 embedding_row(const Model &m, const unsigned char *memory, const Lane &p, int token) {
+    const bf16_t *row = reinterpret_cast<const bf16_t *>(memory + embedding_at(m.depth)) + token * W + p.g;
+    return p.live ? f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])} : ZERO;
 }
 // cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).  GRADIENT: rows are kept in `s` and the head's in `head`.
 template <bool GRADIENT, int CONTEXT>
@@ -374,14 +460,16 @@ TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight,
                             float rs, float *__restrict__ token_losses, float *__restrict__ logits_out, Head &head) {
     const int context = CONTEXT ? CONTEXT : m.context;
     for (int l = 0; l < m.depth; ++l) {
-        const int at = layer_at(l);
-        u32x4 *keep = s.rows + (size_t(l) * s.waves + p.wave) * SLOTS * 64 + p.lane;
+        const int tile = l * LAYER_TILES;
+        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
+        float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
         // QKV projection, RoPE (cuda/model.cuh:14-19)
-        const float inv1 = inverse_rms(h);
-        const u32x2 n1 = pack4(h * inv1 * weight.scale(2 * l));
-        const f32x4 query = rounded(rotate(rounded(product(weight(at + QKV_AT), n1)), rc, rs));
-        const u32x2 key = pack4(rotate(rounded(product(weight(at + QKV_AT + TILE), n1)), rc, rs));
-        const u32x2 value = pack4(product(weight(at + QKV_AT + 2 * TILE), n1));
+        const float inv1 = inverse_rms(h, p);
+        const u32x2 n1 = normalize(h, inv1, weight.scale(2 * l));
+        const f32x4 n1f = unpack4(n1);
+        const f32x4 query = rounded(rotate(rounded(multiply(weight(tile), n1f)), rc, rs));
+        const u32x2 key = pack4(rotate(rounded(multiply(weight(tile + 1), n1f)), rc, rs));
+        const u32x2 value = pack4(multiply(weight(tile + 2), n1f));
         // arg-max attention with its GELU gate (cuda/attention.cuh:33-71); keys in order, the first one wins ties
         float top = -INFINITY;
         int distance = 0;
@@ -404,47 +492,56 @@ TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight,
         });
         const float e = 1.f + erff(top * 0.7071067811865475f);
         const float gate = 0.5f * top * e;
-        const u32x2 a = pack4(unpack4(best_value) * gate);
+        const f32x4 a = turned(rounded(unpack4(best_value) * gate));
         // output projection and residual: a bf16 add (cuda/model.cuh:20-21, cuda/mma.cuh:95-97)
-        const f32x4 middle = rounded(rounded(product(weight(at + ATTENTION_AT), a)) + h);
-        const float inv2 = inverse_rms(middle);
-        const u32x2 n2 = pack4(middle * inv2 * weight.scale(2 * l + 1));
+        const f32x4 middle = rounded(rounded(multiply(weight(tile + 3), a)) + h);
+        const float inv2 = inverse_rms(middle, p);
+        const u32x2 n2 = normalize(middle, inv2, weight.scale(2 * l + 1));
         if constexpr (GRADIENT) {
-            const u32x2 x = pack4(h), mid = pack4(middle), q = pack4(query);
-            keep[S_RESIDUAL * 64] = u32x4{x.x, x.y, mid.x, mid.y};
-            keep[S_QUERY_KEY * 64] = u32x4{q.x, q.y, best_key.x, best_key.y};
-            keep[S_VALUE_NORMS * 64] = u32x4{best_value.x, best_value.y, __float_as_uint(inv1), __float_as_uint(inv2)};
-            const float slope = fmaf(top * 0.3989422804014327f, exponential(-0.5f * top * top), 0.5f * e);
-            keep[S_GATE * 64] = u32x4{__float_as_uint(gate), __float_as_uint(slope), uint32_t(distance), 0};
+            keep[T_X * 64] = pack4(h);
+            keep[T_N1 * 64] = n1;
+            keep[T_Q * 64] = pack4(query);
+            keep[T_KEY * 64] = best_key;
+            keep[T_VALUE * 64] = best_value;
+            keep[T_A * 64] = pack4(a);
+            keep[T_MIDDLE * 64] = pack4(middle);
+            keep[T_N2 * 64] = n2;
+            words[WORD_GATE * 64] = gate;
+            words[WORD_SLOPE * 64] = fmaf(top * 0.3989422804014327f, expf(-0.5f * top * top), 0.5f * e);
+            words[WORD_DISTANCE * 64] = __int_as_float(distance);
+            words[WORD_INV1 * 64] = inv1;
+            words[WORD_INV2 * 64] = inv2;
         }
         // packed gate|up projection, SwiGLU (RN after SiLU and after the product), down projection and residual
         // (cuda/model.cuh:22-30, cuda/ops.cuh:120-131)
-        u32x2 act[3];
+        const f32x4 n2f = unpack4(n2);
+        f32x4 out = ZERO;
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            const u32x2 gate_row = pack4(product(weight(at + GATE_AT + t * TILE), n2)), up_row = pack4(product(weight(at + UP_AT + t * TILE), n2));
-            const f32x4 x = unpack4(gate_row);
-            f32x4 sig;
+            const u32x2 gate_row = pack4(multiply(weight(tile + 4 + t), n2f)), up_row = pack4(multiply(weight(tile + 7 + t), n2f));
+            f32x4 act = unpack4(gate_row);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                sig[r] = sigmoid(x[r]);
-            act[t] = pack4(rounded(x * sig) * unpack4(up_row));
+                act[r] = act[r] * sigmoid(act[r]);
+            const u32x2 act_row = pack4(rounded(act) * unpack4(up_row));
+            out = multiply(weight(tile + 10 + t), unpack4(act_row), out);
             if constexpr (GRADIENT) {
-                keep[(S_GATE_UP + t) * 64] = u32x4{gate_row.x, gate_row.y, up_row.x, up_row.y};
-                keep[(S_SIGMOID + t) * 64] = __builtin_bit_cast(u32x4, sig);
+                keep[(T_GU + t) * 64] = gate_row;
+                keep[(T_GU + 3 + t) * 64] = up_row;
+                keep[(T_ACT + t) * 64] = act_row;
             }
         }
-        const f32x4 out = product(weight.down(at, 0), act[0], weight.down(at, 1), act[1], weight.down(at, 2), act[2]);
         h = rounded(rounded(out) + middle);
     }
-    // final RMSNorm, head, softmax cross-entropy (cuda/model.cuh:32-58): register r of tile t is logit 16 t + 4 g + r
-    const float inv = inverse_rms(h);
-    const u32x2 nf = pack4(h * inv * weight.scale(2 * m.depth));
+    // final RMSNorm, head, softmax cross-entropy (cuda/model.cuh:32-58): register r of tile t is logit 16 t + 4 r + g
+    const float inv = inverse_rms(h, p);
+    const u32x2 nf = normalize(h, inv, weight.scale(2 * m.depth));
+    const f32x4 nff = unpack4(nf);
     f32x4 logit[16];
     float high = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        logit[t] = rounded(product(weight(weight.head + t * TILE), nf));
+        logit[t] = rounded(multiply(weight(weight.head + t), nff));
         high = fmaxf(fmaxf(high, fmaxf(logit[t][0], logit[t][1])), fmaxf(logit[t][2], logit[t][3]));
     }
     high = token_max(high);
@@ -453,285 +550,144 @@ TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight,
         for (int t = 0; t < 16; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                logits_out[size_t(p.token) * V + t * 16 + 4 * p.g + r] = logit[t][r];
-    // the target's logit: tile target / 16, register target % 4 of the lane g = target / 4 % 4, by halves
+                logits_out[size_t(p.token) * V + t * 16 + 4 * r + p.g] = logit[t][r];
+    // the target's logit: tile target / 16, register target / 4 % 4 of the lane g = target % 4, by halves
     float of_four[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        const float even = target & 2 ? logit[t][2] : logit[t][0], odd = target & 2 ? logit[t][3] : logit[t][1];
-        of_four[t] = target & 1 ? odd : even;
+        const float even = target & 4 ? logit[t][1] : logit[t][0], odd = target & 4 ? logit[t][3] : logit[t][2];
+        of_four[t] = target & 8 ? odd : even;
     }
 #pragma unroll
     for (int bit = 0; bit < 4; ++bit)
 #pragma unroll
         for (int t = 0; t < 8 >> bit; ++t)
             of_four[t] = target & (16 << bit) ? of_four[2 * t + 1] : of_four[2 * t];
-    const bool holder = p.g == ((target >> 2) & 3);
+    const bool holder = p.g == (target & 3);
     float picked = holder ? of_four[0] : 0.f;
 #pragma unroll
     for (int t = 0; t < 16; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            logit[t][r] = exponential(logit[t][r] - high);
-    // the sum's tree: every 64th logit in order, then halves of what is left
+            logit[t][r] = expf(logit[t][r] - high);
+    // the sum's tree: every 64th logit in order, then halves of what is left (bits 5 .. 0 of the logit's number)
     f32x4 quarter[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
         quarter[q] = ((logit[q] + logit[q + 4]) + logit[q + 8]) + logit[q + 12];
-    const float sum = token_sum((quarter[0] + quarter[2]) + (quarter[1] + quarter[3]));
+    const f32x4 sixteenth = (quarter[0] + quarter[2]) + (quarter[1] + quarter[3]);
+    const float sum = swap_add_16(swap_add_32((sixteenth[0] + sixteenth[2]) + (sixteenth[1] + sixteenth[3])));
     picked = swap_add_16(swap_add_32(picked));
     if (p.live && p.g == 0)
         token_losses[p.token] = high + logf(sum) - picked;
     if constexpr (GRADIENT) {
-        head.hidden = pack4(h), head.nf = nf, head.inverse = inv;
-        // the quotient by sum * tokens in two parts: one rounding where two divisions have two
-        const float tokens = float(m.tokens), whole = sum * tokens, share = reciprocal(whole);
-        const float rest = share * fmaf(-fmaf(sum, tokens, -whole), share, fmaf(-whole, share, 1.f));
+        head.hidden = pack4(h), head.inverse = inv;
+        s.nf[size_t(p.wave) * 64 + p.lane] = nf;
+        const float share = reciprocal(sum), tokens = float(m.tokens), per_token = 1.f / tokens;
+        const int mine = holder ? target >> 2 : -1; // 4 t + r
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             f32x4 d;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                d[r] = fmaf(logit[t][r], share, logit[t][r] * rest);
+                d[r] = divide(divide(logit[t][r], sum, share) - (4 * t + r == mine ? 1.f : 0.f), tokens, per_token);
             const u32x2 packed = pack4(d);
             head.dlogits[t].x = p.live ? packed.x : 0, head.dlogits[t].y = p.live ? packed.y : 0;
+            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = head.dlogits[t];
         }
-        const float probability = divide(exponential(picked - high), sum, reciprocal(sum));
-        head.of_target = float_to_bf16(divide(probability - 1.f, tokens, 1.f / tokens));
-        head.holder = holder && p.live, head.tile = target >> 4, head.at = target & 3;
     }
 }
 
-// ---- weight gradients ------------------------------------------------------------------------------
-// A block sums what its waves kept in LDS over their tokens, in token order, tile by tile: partial[block].  The transposing load
-// gives lane 16 q + i feature i of tokens 4 q .. 4 q + 3 of a wave, an operand of the instruction whose steps run over the
-// tokens, two waves' tokens each.  That moves data and computes nothing: an infinity stays in its own feature.
-template <int WAVES> struct Gradients {
-    unsigned char *mine;         // this lane's place in this wave's tiles
-    const unsigned char *across; // and in the first wave's, for the transposing load
-    float *sums, *out;           // the waves' sums of the scales' gradients; partial[block]
-    int c, g, wave;
-    TG_DEVICE Gradients(const Model &m, unsigned char *memory, const Workspace &s, const Lane &p, int parameters)
-        : c(p.c), g(p.g), wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
-        mine = memory + rows_at(m.depth) + wave * TILES * 512 + p.lane * 8;
-        across = memory + rows_at(m.depth) + (16 * (p.lane & 3) + 4 * p.g + ((p.lane >> 2) & 3)) * 8;
-        sums = reinterpret_cast<float *>(memory + sums_at(m.depth, WAVES));
-        out = s.partials + size_t(blockIdx.x) * parameters;
-    }
-    TG_DEVICE void put(int tile, u32x2 row) const { *reinterpret_cast<u32x2 *>(mine + tile * 512) = row; }
-    // sixteen rows of dW = dY^T X of `width` columns, sixteen of them
-    TG_DEVICE void tile(int x, int dy, int at, int width) const {
-        const auto row = [&](int n, int w) { return read_across(across + (w * TILES + n) * 512); };
-        f32x4 sum = ZERO;
-#pragma unroll
-        for (int w = 0; w < WAVES; w += 2)
-            sum = product(row(x, w), row(dy, w), row(x, w + 1), row(dy, w + 1), sum);
-        *reinterpret_cast<f32x4 *>(out + at + c * width + 4 * g) = sum;
-    }
-    TG_DEVICE void layer(int l) const {
-        const Layer q = layer_layout(l);
-        // thirteen tiles
-        constexpr int HALVES = WAVES / 4;
-        const int part = wave / HALVES, half = HALVES == 1 ? -1 : wave % HALVES; // a half: the first two tiles or the rest
-        const auto mine_too = [&](int n) { return half < 0 || half == (n >= 2); };
-        if (part == 0) {
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-                if (mine_too(t))
-                    tile(T_N1, T_DQKV + t, q.qkv + t * W * W, W);
-            if (mine_too(3))
-                tile(T_A, T_DH_ATTENTION, q.attention, W);
-        } else if (part == 3) {
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-                if (mine_too(t))
-                    tile(T_ACT + t, T_DH_DOWN, q.down + t * W, F);
-        } else {
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-                if (mine_too(t))
-                    tile(T_N2, T_DGU + 3 * (part - 1) + t, (part == 1 ? q.gate : q.up) + t * W * W, W);
-        }
-    }
-    TG_DEVICE void head(int depth) const {
-#pragma unroll
-        for (int t = 0; t < 16 / WAVES; ++t)
-            tile(T_NF, T_DLOGITS + wave * (16 / WAVES) + t, V * W + depth * LAYER_SIZE + W + (wave * (16 / WAVES) + t) * W * W, W);
-    }
-    // the terms g * z of a norm's scale, over this wave's tokens
-    TG_DEVICE void scale(int norm, f32x4 terms) const {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const auto turn = [&](auto by) {
-                terms[r] += __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(terms[r])), 0x120 + decltype(by)::value, 0xF, 0xF, true)));
-            };
-            turn(std::integral_constant<int, 8>{}), turn(std::integral_constant<int, 4>{}), turn(std::integral_constant<int, 2>{}), turn(std::integral_constant<int, 1>{});
-        }
-        if (c == 0)
-            *reinterpret_cast<f32x4 *>(sums + (norm * WAVES + wave) * W + 4 * g) = terms;
-    }
-    TG_DEVICE void scales(int depth) const {
-        for (int at = threadIdx.x; at < (2 * depth + 1) * W; at += 64 * WAVES) {
-            const int norm = at >> 4;
-            float sum = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w)
-                sum += sums[(norm * WAVES + w) * W + (at & 15)];
-            const Layer q = layer_layout(norm >> 1);
-            out[(norm == 2 * depth ? V * W + depth * LAYER_SIZE : (norm & 1) ? q.mlp_norm : q.attention_norm) + (at & 15)] = sum;
-        }
-    }
-    // The embedding's rows: the one-hot matrix of the tokens times the gradient.  0 times an infinity is NaN, in ids that have
-    // no part in it, so where a row is not finite the rows are added one by one.
-    TG_DEVICE void embedding(const unsigned char *ids) const {
-        constexpr int N = V / 16 / WAVES; // tiles of sixteen ids
-        const int first = wave * N * 16 + c;
-        f32x4 sum[N];
-        bool extreme = false;
-#pragma unroll
-        for (int n = 0; n < N; ++n)
-            sum[n] = ZERO;
-#pragma unroll
-        for (int w = 0; w < WAVES; w += 2) {
-            u32x2 rows[2];
-            uint32_t four[2];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                rows[k] = read_across(across + ((w + k) * TILES + T_DH) * 512);
-                four[k] = *reinterpret_cast<const uint32_t *>(ids + (w + k) * 16 + 4 * g);
-                const auto either = [](uint32_t two) { return (two & 0x7f80u) == 0x7f80u || (two & 0x7f800000u) == 0x7f800000u; };
-                extreme = extreme || either(rows[k].x) || either(rows[k].y);
-            }
-#pragma unroll
-            for (int n = 0; n < N; ++n) {
-                u32x2 hot[2];
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const auto one = [&](int j) { return int((four[k] >> (8 * j)) & 255u) == first + n * 16; };
-                    hot[k].x = (one(0) ? 0x3f80u : 0u) | (one(1) ? 0x3f800000u : 0u);
-                    hot[k].y = (one(2) ? 0x3f80u : 0u) | (one(3) ? 0x3f800000u : 0u);
-                }
-                sum[n] = product(rows[0], hot[0], rows[1], hot[1], sum[n]);
-            }
-        }
-        if (__builtin_amdgcn_ballot_w64(extreme)) {
-#pragma unroll
-            for (int n = 0; n < N; ++n)
-                sum[n] = ZERO;
-#pragma unroll 1
-            for (int t = 0; t < WAVES * 16; ++t) {
-                const int w = t >> 4, id = ids[t];
-                const f32x4 row = unpack4(*reinterpret_cast<const u32x2 *>(mine + ((w - wave) * TILES + T_DH) * 512 + ((t & 15) - c) * 8));
-#pragma unroll
-                for (int n = 0; n < N; ++n)
-                    if (id == first + n * 16)
-                        sum[n] = sum[n] + row;
-            }
-        }
-#pragma unroll
-        for (int n = 0; n < N; ++n)
-            *reinterpret_cast<f32x4 *>(out + (first + n * 16) * W + 4 * g) = sum[n];
-    }
-};
-
 // ---- backward --------------------------------------------------------------------------------------
-// cuda/model.cuh:61-99
-template <int CONTEXT, int WAVES>
+// cuda/model.cuh:61-99, without the weight gradients
+template <int CONTEXT>
 TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight, const Workspace &s, float rc, float rs,
-                             const Head &head, unsigned char *memory, int token, int parameters) {
+                             const Head &head) {
     const int context = CONTEXT ? CONTEXT : m.context;
-    const Gradients<WAVES> gradients(m, memory, s, p, parameters);
-    unsigned char *ids = memory + ids_at(m.depth, WAVES);
+    auto gz = [&](int norm) { return s.gz + ((size_t(norm) * s.waves + p.wave) * 16 + p.c) * W + p.g; };
 
     // a layer's rows are requested while the layer above is worked on
     struct Rows {
-        u32x4 slot[SLOTS];
+        u32x2 x, query, key, value, middle, gate[3], up[3];
+        float gate_of_top, slope, inv1, inv2;
+        int distance;
     };
     auto request = [&](int l, Rows &r) {
-        const u32x4 *keep = s.rows + (size_t(l) * s.waves + p.wave) * SLOTS * 64 + p.lane;
+        const u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
+        const float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
 #pragma unroll
-        for (int i = 0; i < SLOTS; ++i)
-            r.slot[i] = keep[i * 64];
+        for (int t = 0; t < 3; ++t)
+            r.gate[t] = keep[(T_GU + t) * 64], r.up[t] = keep[(T_GU + 3 + t) * 64];
+        r.middle = keep[T_MIDDLE * 64], r.query = keep[T_Q * 64], r.key = keep[T_KEY * 64], r.value = keep[T_VALUE * 64];
+        r.x = keep[T_X * 64];
+        r.gate_of_top = words[WORD_GATE * 64], r.slope = words[WORD_SLOPE * 64], r.inv1 = words[WORD_INV1 * 64];
+        r.inv2 = words[WORD_INV2 * 64], r.distance = __float_as_int(words[WORD_DISTANCE * 64]);
     };
 
     // head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
     Rows next;
     request(m.depth - 1, next);
-    if (p.g == 0)
-        ids[gradients.wave * 16 + p.c] = uint8_t(token);
     f32x4 dn = ZERO;
-    head.put([&](int t) { return gradients.mine + (T_DLOGITS + t) * 512; });
-    gradients.put(T_NF, head.nf);
-    const auto dlogits = [&](int t) { return *reinterpret_cast<const u32x2 *>(gradients.mine + (T_DLOGITS + t) * 512); };
 #pragma unroll
-    for (int t = 0; t < 16; t += 2)
-        dn = product(weight.turned(weight.head + t * TILE), dlogits(t), weight.turned(weight.head + (t + 1) * TILE), dlogits(t + 1), dn);
-    const f32x4 z = unpack4(head.hidden) * head.inverse;
-    dn = rounded(dn);
-    gradients.scale(2 * m.depth, dn * z);
-    f32x4 dh = normalize_backward(z, head.inverse, dn, weight.scale(2 * m.depth));
-    __syncthreads();
-    gradients.head(m.depth);
+    for (int t = 0; t < 16; ++t)
+        dn = multiply(weight.turned_feed(weight.head + t), unpack4(head.dlogits[t]), dn);
+    f32x4 dh = normalize_backward(unpack4(head.hidden), head.inverse, rounded(dn), weight.scale(2 * m.depth), gz(2 * m.depth), p);
     for (int l = m.depth - 1; l >= 0; --l) {
-        const int at = layer_at(l);
+        const int tile = l * LAYER_TILES;
+        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
         const Rows rows = next;
         if (l)
             request(l - 1, next);
         // down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88, cuda/ops.cuh:133-144)
-        u32x2 packed = pack4(dh), act[3], dgate[3], dup[3];
+        keep[T_DH_DOWN * 64] = pack4(dh);
+        f32x4 dgate[3], dup[3];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            const u32x4 gu = rows.slot[S_GATE_UP + t];
-            const f32x4 gate = unpack4(u32x2{gu.x, gu.y}), up = unpack4(u32x2{gu.z, gu.w}), sig = __builtin_bit_cast(f32x4, rows.slot[S_SIGMOID + t]);
-            const f32x4 dy = rounded(product(weight.turned_down(at, t), packed)), da = rounded(dy * up), silu = rounded(gate * sig);
-            f32x4 d;
+            const f32x4 gate = unpack4(rows.gate[t]), up = unpack4(rows.up[t]);
+            const f32x4 dy = rounded(multiply(weight.turned_feed(tile + 10 + t), dh)), da = rounded(dy * up);
+            f32x4 silu;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                d[r] = da[r] * sig[r] * fmaf(gate[r], 1.f - sig[r], 1.f);
-            dgate[t] = pack4(d), dup[t] = pack4(dy * silu), act[t] = pack4(silu * up);
+            for (int r = 0; r < 4; ++r) {
+                const float g = gate[r], sig = sigmoid(g);
+                silu[r] = g * sig;
+                dgate[t][r] = da[r] * sig * fmaf(g, 1.f - sig, 1.f);
+            }
+            const u32x2 dgate_row = pack4(dgate[t]), dup_row = pack4(dy * rounded(silu));
+            keep[(T_DGU + t) * 64] = dgate_row;
+            keep[(T_DGU + 3 + t) * 64] = dup_row;
+            dgate[t] = unpack4(dgate_row), dup[t] = unpack4(dup_row);
         }
-        __syncthreads(); // the tiles above this layer's have been read
-        gradients.put(T_DH_DOWN, packed);
+        dn = ZERO;
 #pragma unroll
         for (int t = 0; t < 3; ++t)
-            gradients.put(T_ACT + t, act[t]), gradients.put(T_DGU + t, dgate[t]), gradients.put(T_DGU + 3 + t, dup[t]);
-        const auto gate_at = [&](int t) { return weight.turned(at + GATE_AT + t * TILE); }; // up's tiles lie behind
-        dn = product(gate_at(4), dup[1], gate_at(5), dup[2],
-                     product(gate_at(2), dgate[2], gate_at(3), dup[0], product(gate_at(0), dgate[0], gate_at(1), dgate[1])));
-        dn = rounded(dn);
-        const u32x4 residual = rows.slot[S_RESIDUAL], value_norms = rows.slot[S_VALUE_NORMS];
-        const float inv1 = __uint_as_float(value_norms.z), inv2 = __uint_as_float(value_norms.w);
-        const f32x4 z2 = unpack4(u32x2{residual.z, residual.w}) * inv2, scale2 = weight.scale(2 * l + 1);
-        gradients.put(T_N2, pack4(z2 * scale2));
-        gradients.scale(2 * l + 1, dn * z2);
+            dn = multiply(weight.turned_feed(tile + 4 + t), dgate[t], dn);
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            dn = multiply(weight.turned_feed(tile + 7 + t), dup[t], dn);
         // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
-        dh = rounded(dh + normalize_backward(z2, inv2, dn, scale2));
-        packed = pack4(dh);
-        gradients.put(T_DH_ATTENTION, packed);
+        dh = rounded(dh + normalize_backward(unpack4(rows.middle), rows.inv2, rounded(dn), weight.scale(2 * l + 1), gz(2 * l + 1), p));
+        keep[T_DH_ATTENTION * 64] = pack4(dh);
 
         // attention: output projection backward, the score gradient of the cached winner, query / key / value gradients
         // gathered over the sequence, inverse RoPE, QKV projection and RMSNorm backward (cuda/model.cuh:89-96,
         // cuda/attention.cuh:72-106)
-        const u32x4 query_key = rows.slot[S_QUERY_KEY];
-        const u32x2 query = {query_key.x, query_key.y};
-        const f32x4 key = unpack4(u32x2{query_key.z, query_key.w}), value = unpack4(u32x2{value_norms.x, value_norms.y});
-        const float gate = __uint_as_float(rows.slot[S_GATE].x), slope = __uint_as_float(rows.slot[S_GATE].y);
-        const uint32_t distance = rows.slot[S_GATE].z;
-        gradients.put(T_A, pack4(value * gate));
-        const u32x2 dattn = pack4(product(weight.turned(at + ATTENTION_AT), packed));
+        const u32x2 query = rows.query;
+        const f32x4 key = unpack4(rows.key), value = unpack4(rows.value);
+        const float gate = rows.gate_of_top;
+        const u32x2 dattn = pack4(multiply(weight(weight.turned_attention + l), dh));
         const f32x4 da = unpack4(dattn);
         float dt = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             dt = fmaf(da[c], value[c], dt);
-        dt *= slope;
+        dt *= rows.slope;
         f32x4 dk = ZERO, dv = ZERO;
         up_to<0, CONTEXT ? CONTEXT - 1 : 7>([&](auto step) { // queries of this token's sequence that chose it, in order
             constexpr int D = decltype(step)::value;
             if (D >= context)
                 return;
             // every lane takes part in the shifts, so none of them may sit behind a condition
-            const uint32_t theirs = later<D>(distance);
+            const uint32_t theirs = later<D>(uint32_t(rows.distance));
             const float their_dt = __uint_as_float(later<D>(__float_as_uint(dt))), their_gate = __uint_as_float(later<D>(__float_as_uint(gate)));
             const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
             const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
@@ -744,77 +700,74 @@ TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight
                 }
             }
         });
-        const u32x2 dq_row = pack4(rotate_back(rounded(key * dt), rc, rs)), dk_row = pack4(rotate_back(rounded(dk), rc, rs)), dv_row = pack4(dv);
-        gradients.put(T_DQKV, dq_row), gradients.put(T_DQKV + 1, dk_row), gradients.put(T_DQKV + 2, dv_row);
-        dn = product(weight.turned(at + QKV_AT), dq_row, weight.turned(at + QKV_AT + TILE), dk_row, weight.turned(at + QKV_AT + 2 * TILE), dv_row);
-        dn = rounded(dn);
-        const f32x4 z1 = unpack4(u32x2{residual.x, residual.y}) * inv1, scale1 = weight.scale(2 * l);
-        gradients.put(T_N1, pack4(z1 * scale1));
-        gradients.scale(2 * l, dn * z1);
-        dh = rounded(dh + normalize_backward(z1, inv1, dn, scale1));
-        __syncthreads();
-        gradients.layer(l);
+        const f32x4 dq = turned(rounded(rotate_back(rounded(key * dt), rc, rs)));
+        dk = turned(rounded(rotate_back(rounded(dk), rc, rs)));
+        dv = turned(rounded(dv));
+        keep[T_DQKV * 64] = pack4(dq);
+        keep[(T_DQKV + 1) * 64] = pack4(dk);
+        keep[(T_DQKV + 2) * 64] = pack4(dv);
+        dn = multiply(weight.turned_natural(tile + 2), dv,
+                      multiply(weight.turned_natural(tile + 1), dk, multiply(weight.turned_natural(tile), dq)));
+        dh = rounded(dh + normalize_backward(unpack4(rows.x), rows.inv1, rounded(dn), weight.scale(2 * l), gz(2 * l), p));
     }
-    __syncthreads();
-    gradients.put(T_DH, pack4(dh));
-    __syncthreads();
-    gradients.embedding(ids);
-    gradients.scales(m.depth);
+    s.dh[size_t(p.wave) * 64 + p.lane] = pack4(dh);
 }
 
 // ---- kernels -----------------------------------------------------------------------------------------
-template <bool GRADIENT, int WAVES>
+template <bool GRADIENT>
 __global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
                                                                Workspace s, float *__restrict__ token_losses,
                                                                float *__restrict__ logits_out) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of<WAVES>(m);
+    const Lane p = lane_of(m);
     const Staged weight(m, memory, p);
+    Staging staging(m, memory);
     const int token = p.live ? x[p.token] : 0, target = p.live ? y[p.token] : 0;
-    stage<WAVES>(m, memory, !(reinterpret_cast<uintptr_t>(m.hi) & 15));
-    const f32x4 h = embedding_row(memory, p, token);
+    staging.request();
+    staging.request_embedding(!(reinterpret_cast<uintptr_t>(m.hi) & 15));
+    staging.finish(false);
+    const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
     rotation(p.position, rc, rs);
     Head head;
     forward_pass<GRADIENT, 0>(m, p, weight, s, h, target, rc, rs, token_losses, logits_out, head);
     if constexpr (GRADIENT) {
         const size_t here = size_t(p.wave) * 64 + p.lane;
-        s.hidden[here] = head.hidden, s.nf[here] = head.nf, s.inverse[here] = head.inverse;
-        head.put([&](int t) { return s.dlogits + (size_t(p.wave) * 16 + t) * 64 + p.lane; });
+        s.hidden[here] = head.hidden, s.inverse[here] = head.inverse;
     }
 }
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, const uint8_t *__restrict__ x, Workspace s, int parameters) {
+__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Workspace s) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of<WAVES>(m);
+    const Lane p = lane_of(m);
     const Staged weight(m, memory, p);
-    const int token = p.live ? x[p.token] : 0;
+    Staging staging(m, memory);
+    staging.request();
     Head head;
     const size_t here = size_t(p.wave) * 64 + p.lane;
-    head.hidden = s.hidden[here], head.nf = s.nf[here], head.inverse = s.inverse[here];
+    head.hidden = s.hidden[here], head.inverse = s.inverse[here];
 #pragma unroll
     for (int t = 0; t < 16; ++t)
         head.dlogits[t] = s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane];
-    head.holder = false; // the target's is among them
-    stage<WAVES>(m, memory, !(reinterpret_cast<uintptr_t>(m.hi) & 15));
+    staging.finish(true);
     float rc, rs;
     rotation(p.position, rc, rs);
-    backward_pass<0, WAVES>(m, p, weight, s, rc, rs, head, memory, token, parameters);
+    backward_pass<0>(m, p, weight, s, rc, rs, head);
 }
 // A training step's both passes: a wave's backward pass reads only what its own forward pass kept, so the two are one launch
-// and the weights are staged once.  What bounds it is a wave's chain of some 1100 dependent vector instructions a layer and 1200 at
-// the head.  Depth 4, 2560 sequences of 4: 38.7 us on fp32 matrix instructions, weights converted on the way, without the weight
-// gradients, which took 13.1 us more from rows kept in memory; 24.6 so.  Depth 8, 16 of 8: 64.9 + 11.1 and 39.0.  Tokens and
-// targets come straight out of the training bytes, every sequence a window at a hashed place (cuda/dataset.cuh:13-27).
-template <int CONTEXT, int WAVES>
+// and the weights are staged once.  Depth 4, 2560 sequences of 4: 53.0 us as two launches that staged eight tiles at a time,
+// 38.8 so; depth 8, 16 of 8: 79.3 and 62.6.  Two waves a SIMD, which batches of more than 256 blocks need (10000 of 8 at depth 8
+// 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training
+// bytes, every sequence a window at a hashed place (cuda/dataset.cuh:13-27); the tokens are left for the embedding's gradient.
+template <int CONTEXT>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(
-    Model m, W16Data data, uint64_t inverse, Workspace first, Group group, int parameters) {
+    Model m, W16Data data, uint64_t inverse, Workspace first, Group group) {
     extern __shared__ __align__(16) unsigned char memory[];
     const W16Batch &batch = group.member[blockIdx.y];
     const Workspace s = group.workspace(first, blockIdx.y);
     m.hi = batch.weights.hi, m.lo = batch.weights.lo;
-    const Lane p = lane_of<WAVES>(m);
+    const Lane p = lane_of(m);
     const Staged weight(m, memory, p);
+    Staging staging(m, memory);
     int token = 0, target = 0;
     if (p.live) {
         const int sequence = p.token / CONTEXT;
@@ -827,128 +780,336 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         const uint8_t *window = data.bytes + (end - CONTEXT) + p.position;
         token = window[0], target = window[1];
     }
-    stage<WAVES>(m, memory);
-    const f32x4 h = embedding_row(memory, p, token);
+    staging.request();
+    staging.request_embedding();
+    staging.finish(true);
+    if (p.live && p.g == 0)
+        batch.tokens[p.token] = uint8_t(token);
+    const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
     rotation(p.position, rc, rs);
     Head head;
     forward_pass<true, CONTEXT>(m, p, weight, s, h, target, rc, rs, batch.token_losses, nullptr, head);
-    backward_pass<CONTEXT, WAVES>(m, p, weight, s, rc, rs, head, memory, token, parameters);
+    backward_pass<CONTEXT>(m, p, weight, s, rc, rs, head);
 }
 
-// ---- the blocks' sums --------------------------------------------------------------------------------
-// gradient = the blocks' sums in block order, in up to GROUPS parts: a wave takes 64 elements, GROUPS waves share out the blocks,
-// and a part's loads are in flight together.  160 blocks of 21648 parameters: 8.2 us with one wave for 64 elements, 5.2 so; of 2
-// blocks (35088 parameters, four batches) eight waves make 7.5 and one 4.8: up to sixteen blocks take one.
-// Where norms are wanted, every wave's elements leave a part of a sum of squares of 1024 (FOLD_PARTS).
+// ---- weight gradients ------------------------------------------------------------------------------
+// A block sums what one layer (or the head, or the embedding) has of a chunk's tokens, in token order: partial[chunk].  Its
+// rows come to LDS as the waves kept them; the transposing load then gives lane 16 q + i feature 4 (i % 4) + i / 4 of tokens
+// 4 j + q, an operand of the fp32 instruction whose steps run over the tokens.  That moves data and computes nothing: an
+// infinity stays in its own feature.  A wave has three or four tiles of the gradient at a time, whose chains of dependent
+// instructions fill the matrix pipe, which bounds the kernel together with what the rows take on their way (half of them
+// are worked on while the others come): 93 tiles of 32 instructions a chunk at depth 4.  2560 sequences of 4 there: 15.3 us
+// with a wave for each tile that loaded its rows and turned them with the identity matrix, 13.1 so; 16 of 8 at depth 8 7.7 and 7.9.
+// Half a chunk, as the last one or the only one may be, is all that is worked on: 16 sequences of 4 at depth 4 6.4 us with the
+// missing half as zeros, 4.6 so.
+constexpr int HEAD_ROWS = 17; // the head's tiles of a wave in LDS: dlogits, and the normalised rows
+constexpr size_t GRADIENT_LDS = size_t(CHUNK_WAVES) * OPERANDS * 512;
+static_assert(HEAD_ROWS <= OPERANDS, "the head's rows fit a layer's");
+// a lane's rows 4 r + g and column 4 (c % 4) + c / 4 of a gradient tile
+TG_DEVICE void store_tile(float *out, const f32x4 &sum, int width, int lane) {
+    const int g = lane >> 4, column = feed_row(lane & 15);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        out[(4 * r + g) * width + column] = sum[r];
+}
+// the g * z terms of a norm's scale: token 4 j + g of every wave, feature c
+struct ScaleTerms {
+    float v[CHUNK_WAVES][4];
+    TG_DEVICE void request(const Workspace &s, int norm, int first, int waves, int lane) {
+        const float *gz = s.gz + (size_t(norm) * s.waves + first) * 16 * W + lane;
+#pragma unroll
+        for (int w = 0; w < CHUNK_WAVES; ++w)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[w][j] = w < waves ? gz[(w * 4 + j) * 64] : 0.f;
+    }
+};
+// TILES chains of products over the tokens of half a chunk's waves, and with SCALE one of a row of ones times the terms.
+// `rows` and `columns`: this lane's place in the first wave's tiles; a wave's are `stride` (columns: `column_stride`) bytes.
+template <int TILES, bool SCALE>
+TG_DEVICE void add_half(f32x4 (&sum)[4], const unsigned char *const (&rows)[TILES], const unsigned char *const (&columns)[TILES], int stride,
+                        int column_stride, const ScaleTerms &terms, int half) {
+#pragma unroll
+    for (int k = 0; k < CHUNK_WAVES / 2; ++k) {
+        const int w = half * (CHUNK_WAVES / 2) + k;
+        f32x4 a[TILES], b[TILES];
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+            a[n] = unpack4(read_across(rows[n] + w * stride)), b[n] = unpack4(read_across(columns[n] + w * column_stride));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int n = 0; n < TILES; ++n)
+                sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][j], b[n][j], sum[n], 0, 0, 0);
+            if constexpr (SCALE)
+                sum[TILES] = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], sum[TILES], 0, 0, 0);
+        }
+    }
+}
+__global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m, Workspace whole, Group group, int parameters) {
+    extern __shared__ __align__(16) unsigned char memory[];
+    const Workspace s = group.workspace(whole, blockIdx.y);
+    const uint8_t *x = group.member[blockIdx.y].tokens;
+    // consecutive blocks sit on consecutive XCDs: block 8 i + k takes the i-th unit of XCD k's chunks
+    const int units = m.depth + 2, chunk = (blockIdx.x >> 3) / units * 8 + (blockIdx.x & 7), unit = (blockIdx.x >> 3) % units;
+    if (chunk >= s.chunks)
+        return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+    const int first = chunk * CHUNK_WAVES, waves = min(CHUNK_WAVES, s.waves - first);
+    const bool second_half = waves > CHUNK_WAVES / 2;
+    float *out = s.partials + size_t(chunk) * parameters;
+    const uint32_t lds = lds_address(memory);
+    // TILES tiles of every wave, `apart` bytes from one wave to the next in memory, one behind another in LDS; 16 bytes a lane.
+    // The last chunk's missing waves are zeros, of the second half only where it has any.
+    const auto copy = [&](auto tiles, const u32x2 *source, int apart, int to) {
+        constexpr int PIECES = decltype(tiles)::value * 32;
+        static_assert(CHUNK_WAVES * PIECES % (WAVES * 64) == 0, "every wave has as many copies");
+#pragma unroll
+        for (int i = 0; i < CHUNK_WAVES * PIECES / (WAVES * 64); ++i) {
+            const int base = (i * WAVES + wave) * 64, piece = base + lane, w = piece / PIECES;
+            if (w < waves)
+                async_copy16(lds + uint32_t(to + base * 16), source, uint32_t(w * apart + (piece - w * PIECES) * 16));
+            else if (w < CHUNK_WAVES / 2 || second_half)
+                *reinterpret_cast<u32x4 *>(memory + to + piece * 16) = u32x4{0, 0, 0, 0};
+        }
+    };
+    const auto half_there = [&]() { // all but a wave's last eight copies; a chunk that is not full has fewer
+        if (waves == CHUNK_WAVES)
+            wait_vmcnt<8>();
+        else
+            wait_vmcnt<0>();
+        wait_lgkmcnt0();
+        __syncthreads();
+    };
+    const unsigned char *mine = memory + across_offset(lane, true);
+    const auto tile = [&](int n) { return mine + n * 512; };
+    f32x4 sum[4] = {ZERO, ZERO, ZERO, ZERO};
+    ScaleTerms terms;
+    if (unit < m.depth) {
+        const Layer q = layer_layout(unit);
+        // waves 1 and 2 have a norm's scale besides gate and up
+        if (wave == 1 || wave == 2)
+            terms.request(s, 2 * unit + wave - 1, first, waves, lane);
+        copy(std::integral_constant<int, OPERANDS>{}, s.tiles + ((size_t(unit) * s.waves + first) * TILES + T_OPERANDS) * 64, TILES * 512, 0);
+        constexpr int N1 = T_N1 - T_OPERANDS, A = T_A - T_OPERANDS, N2 = T_N2 - T_OPERANDS, ACT = T_ACT - T_OPERANDS,
+                      DQKV = T_DQKV - T_OPERANDS, DH_ATTENTION = T_DH_ATTENTION - T_OPERANDS, DGU = T_DGU - T_OPERANDS,
+                      DH_DOWN = T_DH_DOWN - T_OPERANDS, STRIDE = OPERANDS * 512;
+        const auto layer = [&](int half) {
+            if (wave == 0)
+                add_half<4, false>(sum, {tile(DQKV), tile(DQKV + 1), tile(DQKV + 2), tile(DH_ATTENTION)}, {tile(N1), tile(N1), tile(N1), tile(A)},
+                                   STRIDE, STRIDE, terms, half);
+            else if (wave == 3)
+                add_half<3, false>(sum, {tile(DH_DOWN), tile(DH_DOWN), tile(DH_DOWN)}, {tile(ACT), tile(ACT + 1), tile(ACT + 2)}, STRIDE, STRIDE,
+                                   terms, half);
+            else
+                add_half<3, true>(sum, {tile(DGU + 3 * wave - 3), tile(DGU + 3 * wave - 2), tile(DGU + 3 * wave - 1)}, {tile(N2), tile(N2), tile(N2)},
+                                  STRIDE, STRIDE, terms, half);
+        };
+        half_there(); // brought by nine of a wave's seventeen copies
+        layer(0);
+        if (second_half) {
+            wait_vmcnt<0>();
+            __syncthreads();
+            layer(1);
+        }
+        if (wave == 0) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) // the attention projection lies behind q, k, v
+                store_tile(out + q.qkv + t * 256, sum[t], W, lane);
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            store_tile(wave == 3 ? out + q.down + t * 16 : out + q.gate + ((wave - 1) * 3 + t) * 256, sum[t], wave == 3 ? F : W, lane);
+        if (wave < 3 && g == 0)
+            out[(wave == 1 ? q.attention_norm : q.mlp_norm) + c] = sum[3][0];
+        return;
+    }
+    if (unit == m.depth) { // the head: a wave four tiles of logits
+        constexpr int NF = CHUNK_WAVES * 16;
+        copy(std::integral_constant<int, 1>{}, s.nf + size_t(first) * 64, 512, NF * 512);
+        copy(std::integral_constant<int, 16>{}, s.dlogits + size_t(first) * 16 * 64, 16 * 512, 0);
+        const auto head = [&](int half) {
+            add_half<4, false>(sum, {tile(wave * 4), tile(wave * 4 + 1), tile(wave * 4 + 2), tile(wave * 4 + 3)},
+                               {tile(NF), tile(NF), tile(NF), tile(NF)}, 16 * 512, 512, terms, half);
+        };
+        half_there(); // eight of the sixteen
+        head(0);
+        if (second_half) {
+            wait_vmcnt<0>();
+            __syncthreads();
+            head(1);
+        }
+        const int at = V * W + m.depth * LAYER_SIZE + W;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            store_tile(out + at + (wave * 4 + t) * 256, sum[t], W, lane);
+        if (wave == 0) {
+            terms.request(s, 2 * m.depth, first, waves, lane);
+            f32x4 scale = ZERO;
+#pragma unroll
+            for (int w = 0; w < CHUNK_WAVES; ++w)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    scale = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], scale, 0, 0, 0);
+            if (g == 0)
+                out[at - W + c] = scale[0];
+        }
+        return;
+    }
+    // The embedding's rows: the one-hot matrix of the tokens times the gradient.  0 times an infinity is NaN, in ids that have
+    // no part in it, so where a row is not finite the rows are added one by one.
+    copy(std::integral_constant<int, 1>{}, s.dh + size_t(first) * 64, 512, 0);
+    uint32_t ids[CHUNK_WAVES];
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        ids[w] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = 4 * j + g, token = (first + w) * m.per_wave + t; // rows beyond the last token are zero: any id will do
+            ids[w] |= uint32_t(w < waves && t < m.per_wave && token < m.tokens ? x[token] : 0) << (8 * j);
+        }
+    }
+    wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    __syncthreads();
+    const int vocabulary = wave * 64; // of the four tiles' first id
+    bool extreme = false;
+#pragma unroll
+    for (int w = 0; w < CHUNK_WAVES; ++w) {
+        if (w == CHUNK_WAVES / 2 && !second_half)
+            break;
+        const u32x2 row = read_across(tile(w));
+        const auto either = [](uint32_t two) { return (two & 0x7f80u) == 0x7f80u || (two & 0x7f800000u) == 0x7f800000u; };
+        extreme = extreme || either(row.x) || either(row.y);
+        const f32x4 b = unpack4(row);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(int((ids[w] >> (8 * j)) & 255u) == vocabulary + t * 16 + c ? 1.f : 0.f, b[j],
+                                                              sum[t], 0, 0, 0);
+    }
+    if (__builtin_amdgcn_ballot_w64(extreme)) {
+        sum[0] = sum[1] = sum[2] = sum[3] = ZERO;
+#pragma unroll 1
+        for (int w = 0; w < waves; ++w)
+#pragma unroll 1
+            for (int t = 0; t < m.per_wave; ++t) {
+                const int token = (first + w) * m.per_wave + t;
+                if (token >= m.tokens)
+                    break;
+                // column 4 (c % 4) + c / 4 is element c % 4 of item (c / 4, t)
+                const float value = bf16_to_float(reinterpret_cast<const bf16_t *>(memory)[(w * 64 + 16 * (c >> 2) + t) * 4 + (c & 3)]);
+                const int id = int(x[token]) - vocabulary - 4 * g;
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        sum[n][r] = id == 16 * n + r ? sum[n][r] + value : sum[n][r];
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) // the ids are in their own order
+            out[(vocabulary + t * 16 + 4 * g + r) * W + feed_row(c)] = sum[t][r];
+}
+// gradient = the chunks' sums in chunk order, an element a thread, whose loads are in flight together: 80 chunks of 21648
+// parameters took 5.9 us with four elements a thread on a quarter of the blocks and sixteen loads at a time, 5.2 so.  Four
+// chunks and fewer ask forty times for nothing: 1 chunk 2.5 us, with four at a time 1.2.
+// Where norms are wanted, four blocks leave the parts of one sum of squares, of 1024 elements (FOLD_QUARTERS).
 // Blocks beyond the parameters average the losses: one a position, in double (cuda/trainer.cuh:79-100).
-constexpr int FOLD_PARTS = 1024 / 64;
-int fold_parts(int parameters) { return (parameters + 1023) / 1024 * FOLD_PARTS; }
-template <int GROUPS>
-__global__ __launch_bounds__(GROUPS == 1 ? 256 : 64 * GROUPS) void w16_fold_kernel(Workspace whole, Group group, int parameters, int blocks,
-                                                                                 int batch, int context) {
-    constexpr int WAVES = GROUPS == 1 ? 4 : GROUPS;
+constexpr int FOLD_QUARTERS = 4;
+int fold_blocks(int parameters) { return (parameters + 1023) / 1024 * FOLD_QUARTERS; }
+__global__ __launch_bounds__(256) void w16_fold_kernel(Workspace whole, Group group, int parameters, int blocks, int batch,
+                                                       int context) {
     const W16Batch &member = group.member[blockIdx.y];
-    const int count = whole.blocks, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float *partials = group.workspace(whole, blockIdx.y).partials;
+    const int chunks = whole.chunks;
     if (int(blockIdx.x) >= blocks) {
-        __shared__ double sums[WAVES];
+        __shared__ double sums[4];
         const int position = blockIdx.x - blocks;
         double sum = 0;
 #pragma unroll 4
-        for (int b = threadIdx.x; b < batch; b += 64 * WAVES)
+        for (int b = threadIdx.x; b < batch; b += 256)
             sum += member.token_losses[size_t(b) * context + position];
 #pragma unroll
         for (int k = 32; k; k >>= 1)
             sum += __shfl_xor(sum, k, 64);
-        if (lane == 0)
-            sums[wave] = sum;
+        if ((threadIdx.x & 63) == 0)
+            sums[threadIdx.x >> 6] = sum;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            sum = sums[0];
-            for (int w = 1; w < WAVES; ++w)
-                sum += sums[w];
-            member.means[position] = float(sum / batch);
-        }
+        if (threadIdx.x == 0)
+            member.means[position] = float(((sums[0] + sums[1]) + (sums[2] + sums[3])) / batch);
         return;
     }
-    const int part = GROUPS == 1 ? blockIdx.x * WAVES + wave : blockIdx.x, at = part * 64 + lane;
-    const int share = (count + GROUPS - 1) / GROUPS, first = GROUPS == 1 ? 0 : wave * share, mine = min(share, count - first);
+    __shared__ __align__(16) float row[256];
+    const int at = blockIdx.x * 256 + threadIdx.x;
     float sum = 0.f;
     if (at < parameters) {
-        const float *from = group.workspace(whole, blockIdx.y).partials + size_t(first) * parameters + at;
-        constexpr int AT_ONCE = GROUPS == 1 ? 8 : 20;
-        for (int c = 0; c < mine; c += AT_ONCE) {
-            float v[AT_ONCE];
+        const float *from = partials + at;
+        const auto add = [&](auto at_once) {
+            constexpr int AT_ONCE = decltype(at_once)::value;
+            for (int c = 0; c < chunks; c += AT_ONCE) {
+                float v[AT_ONCE];
 #pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-                if (c + i < mine)
-                    v[i] = from[size_t(c + i) * parameters];
+                for (int i = 0; i < AT_ONCE; ++i)
+                    if (c + i < chunks)
+                        v[i] = from[size_t(c + i) * parameters];
 #pragma unroll
-            for (int i = 0; i < AT_ONCE; ++i)
-                if (c + i < mine)
-                    sum += v[i];
-        }
-    }
-    if constexpr (GROUPS > 1) {
-        __shared__ float rows[GROUPS][64];
-        rows[wave][lane] = sum;
-        __syncthreads();
-        if (wave)
-            return;
-        sum = rows[0][lane];
-#pragma unroll
-        for (int w = 1; w < GROUPS; ++w)
-            sum += rows[w][lane];
-    }
-    if (at < parameters)
+                for (int i = 0; i < AT_ONCE; ++i)
+                    if (c + i < chunks)
+                        sum += v[i];
+            }
+        };
+        if (chunks <= 4)
+            add(std::integral_constant<int, 4>{});
+        else
+            add(std::integral_constant<int, 40>{});
         member.gradient[at] = sum;
+    }
     if (!member.norms)
         return;
-    const float squares = wave_sum(sum * sum);
-    if (lane == 0)
-        member.norms[part] = squares;
+    row[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const float squares = wave_sum(0.f + quad_squares(reinterpret_cast<const f32x4 *>(row)[threadIdx.x]));
+        if (threadIdx.x == 0)
+            member.norms[blockIdx.x] = squares;
+    }
 }
 
 // ---- optimizer (cuda/optim.cuh:17-119) ------------------------------------------------------------------
 // Blocks 0 .. 5 depth - 1: Muon, a hidden matrix each.  The rest: AdamW, 256 quads of embedding, scales and head each.
-// The Newton-Schulz iterate is a 16 x n matrix of bf16 values in 16 x 16 tiles, one a wave, lane 16 g + c holding rows 4 g .. of
-// column c.  X X^T is symmetric to the last bit, so what a lane holds of it is the operand of the two products behind it, every
-// wave computes it for itself, and a step exchanges nothing but X through LDS: one barrier a step.  What bounds it is that chain:
-// 8.6 us a launch on fp32 matrix instructions, 5.5 more for every further step; on the bf16 ones, with the clip factors of all
-// steps formed at the start, 6.8 and 3.0.
+// The Newton-Schulz iterate is a 16 x n matrix in 16 x 16 tiles, one a wave, lane 16 g + c holding rows 4 g .. of column c;
+// the products run on the fp32 matrix instruction (the same fmaf chains as a loop).  X X^T is symmetric to the last bit,
+// so its tile turned is the operand of the two products behind it, every wave computes it for itself, and a step
+// exchanges nothing but X through LDS: one barrier a step where there were four.
 // One launch makes as many steps, one after another, as there are gradients at hand: an element's (Muon: a matrix's) weights
 // and state stay in the registers between them.
 struct Update {
     float *momentum, *variance;
-    int norm_count, norm_parts, depth; // norms: norm_count sums of norm_parts partial sums each, 1 or FOLD_PARTS
+    int norm_count, norm_parts, depth; // norms: norm_count sums of norm_parts partial sums each, 1 or FOLD_QUARTERS
     int count;
     W16Step step[W16_BATCHES];
 };
-// The steps' clip factors, a step a wave: clip_factor of the norms.  A barrier stands between this and their first use.
-TG_DEVICE void clip_factors(const Update &u, float *factors) {
-    const int lane = threadIdx.x & 63;
-    for (int n = threadIdx.x >> 6; n < u.count; n += 4) {
-        const W16Step &step = u.step[n];
-        float factor = 1.f;
-        if (step.adam.clip > 0.f) {
-            float sum = 0.f;
-            if (u.norm_parts == 1)
-                for (int i = lane; i < u.norm_count; i += 64)
-                    sum += step.norms[i];
-            else
-                for (int i = lane; i < u.norm_count * FOLD_PARTS / 4; i += 64) {
-                    const f32x4 part = reinterpret_cast<const f32x4 *>(step.norms)[i];
-                    sum += (part[0] + part[1]) + (part[2] + part[3]);
-                }
-            factor = fminf(1.f, step.adam.clip / (sqrtf(wave_sum(sum)) + 1e-6f));
-        }
-        if (lane == 0)
-            factors[n] = factor;
+// clip_factor of the norms, with the sums of a fold's quarters formed first
+TG_DEVICE float clip_factor(const Update &u, int n, float *waves) {
+    const W16Step &step = u.step[n];
+    if (u.norm_parts == 1 || !(step.adam.clip > 0.f))
+        return ::clip_factor(step.adam.clip, step.norms, u.norm_count, waves);
+    float sum = 0.f;
+    for (int i = threadIdx.x; i < u.norm_count; i += 256) {
+        const f32x4 part = *reinterpret_cast<const f32x4 *>(step.norms + i * FOLD_QUARTERS);
+        sum += (part[0] + part[1]) + (part[2] + part[3]);
     }
+    return fminf(1.f, step.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
 }
-TG_DEVICE void muon_matrix(const Update &u, int matrix, float *factors) {
-    __shared__ __align__(8) bf16_t wide[2][16 * F];
-    __shared__ float norm_waves[2][4];
+TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
+    __shared__ float wide[2][16 * F];
+    __shared__ float norm_waves[4];
     const Layer p = layer_layout(matrix / 5);
     const int type = matrix % 5;
     const int weight = type == 0 ? p.qkv : type == 1 ? p.attention : type == 2 ? p.gate : type == 3 ? p.up : p.down;
@@ -964,8 +1125,6 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *factors) {
         next_g[k] = mine ? u.step[0].gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f;
         w[k] = mine ? master(u.step[0].from.hi, u.step[0].from.lo, i) : 0.f;
     }
-    clip_factors(u, factors);
-    __syncthreads();
     const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
     for (int at = 0; at < u.count; ++at) {
         const W16Step &u_step = u.step[at];
@@ -975,7 +1134,7 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *factors) {
 #pragma unroll
             for (int k = 0; k < 3; ++k)
                 next_g[k] = tid + 256 * k < size ? u.step[at + 1].gradient[weight + tid + 256 * k] : 0.f;
-        const float clip = factors[at];
+        const float clip = clip_factor(u, at, waves[at & 1]);
         float squares = 0.f, b[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k)
@@ -985,55 +1144,53 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *factors) {
                 b[k] = round_bf16(fmaf(muon.momentum, m[k] - gs, gs));
                 squares = fmaf(b[k], b[k], squares);
             }
-        const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves[at & 1]))), round_bf16(1e-7f));
+        const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (tid + 256 * k < size)
-                wide[0][place(tid + 256 * k)] = float_to_bf16(b[k] / norm);
+                wide[0][place(tid + 256 * k)] = round_bf16(b[k] / norm);
         __syncthreads();
         f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
         if (tile < tiles)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                x[r] = bf16_to_float(wide[0][(4 * gr + r) * n + 16 * tile + c]);
+                x[r] = wide[0][(4 * gr + r) * n + 16 * tile + c];
         for (int step = 0; step < muon.ns_steps; ++step) {
-            const bf16_t *in = wide[step & 1] + c * n + 4 * gr;
-            bf16_t *out = wide[(step & 1) ^ 1] + 4 * gr * n + 16 * tile + c;
+            const float *in = wide[step & 1];
+            float *out = wide[(step & 1) ^ 1];
             if (tile < tiles) {
-                const auto row = [&](int k) { return *reinterpret_cast<const u32x2 *>(in + 16 * k); };
-                const u32x2 first = row(0);
-                f32x4 gram; // A = X X^T, kept in bf16
-                if (tiles == 1)
-                    gram = product(first, first);
-                else {
-                    const u32x2 second = row(1), third = row(2);
-                    gram = product(first, first, second, second, third, third);
-                }
-                const u32x2 gram_row = pack4(gram);
-                gram = unpack4(gram_row);
-                const f32x4 square = product(gram_row, gram_row);
+                f32x4 gram = ZERO; // A = X X^T, kept in bf16
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    if (k < tiles) {
+                        f32x4 row;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            row[j] = in[c * n + 16 * k + 4 * j + gr];
+                        gram = multiply(row, row, gram);
+                    }
+                gram = rounded(gram);
+                const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
                 f32x4 work; // -4.775 A + 2.0315 A A
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
-                const f32x4 change = product(pack4(work), pack4(x));
+                const f32x4 product = multiply(turned(rounded(work)), turned(x));
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    x[r] = fmaf(3.4445f, x[r], change[r]);
-                const u32x2 packed = pack4(x);
-                x = unpack4(packed);
-                out[0] = bf16_t(packed.x), out[n] = bf16_t(packed.x >> 16);
-                out[2 * n] = bf16_t(packed.y), out[3 * n] = bf16_t(packed.y >> 16);
+                for (int r = 0; r < 4; ++r) {
+                    x[r] = round_bf16(fmaf(3.4445f, x[r], product[r]));
+                    out[(4 * gr + r) * n + 16 * tile + c] = x[r];
+                }
             }
             __syncthreads();
         }
-        const bf16_t *result = wide[muon.ns_steps & 1];
+        const float *result = wide[muon.ns_steps & 1];
         const float adjusted = muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-muon.lr, muon.weight_decay, 1.f);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (tid + 256 * k < size) {
                 const int i = weight + tid + 256 * k;
-                w[k] = fmaf(w[k], keep, -(adjusted * bf16_to_float(result[place(tid + 256 * k)])));
+                w[k] = fmaf(w[k], keep, -(adjusted * result[place(tid + 256 * k)]));
                 const uint32_t bits = __float_as_uint(w[k]);
                 u_step.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
                 u_step.to.lo[i] = uint16_t(bits);
@@ -1046,9 +1203,9 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float *factors) {
             u.momentum[weight + tid + 256 * k] = m[k];
 }
 __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
-    __shared__ float factors[W16_BATCHES];
+    __shared__ float waves[2][4];
     if (int(blockIdx.x) < 5 * u.depth)
-        return muon_matrix(u, blockIdx.x, factors);
+        return muon_matrix(u, blockIdx.x, waves);
     // quads: the embedding's 1024, four for each scale, the head's 1024 (the only ones that decay)
     const int quad = (blockIdx.x - 5 * u.depth) * 256 + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
     int at = quad * 4;
@@ -1067,25 +1224,26 @@ __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
     for (int k = 0; k < 4; ++k)
         w[k] = master(u.step[0].from.hi, u.step[0].from.lo, at + k);
     f32x4 next_g = *reinterpret_cast<const f32x4 *>(u.step[0].gradient + at);
-    clip_factors(u, factors);
-    __syncthreads();
-    if (!live)
-        return;
     for (int n = 0; n < u.count; ++n) {
         const W16Step &step = u.step[n];
         const f32x4 g = next_g;
         if (n + 1 < u.count)
             next_g = *reinterpret_cast<const f32x4 *>(u.step[n + 1].gradient + at);
+        const float scale = clip_factor(u, n, waves[n & 1]);
+        if (!live)
+            continue;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             float mk = m[k], vk = v[k];
-            w[k] = adamw_element(step.adam, decays ? step.adam.weight_decay : 0.f, factors[n], w[k], mk, vk, g[k]);
+            w[k] = adamw_element(step.adam, decays ? step.adam.weight_decay : 0.f, scale, w[k], mk, vk, g[k]);
             m[k] = mk, v[k] = vk;
         }
         const auto half = [&](int k, int shift) { return (__float_as_uint(w[k]) >> shift) & 0xffffu; };
         *reinterpret_cast<u32x2 *>(step.to.hi + at) = u32x2{half(0, 16) | half(1, 16) << 16, half(2, 16) | half(3, 16) << 16};
         *reinterpret_cast<u32x2 *>(step.to.lo + at) = u32x2{half(0, 0) | half(1, 0) << 16, half(2, 0) | half(3, 0) << 16};
     }
+    if (!live)
+        return;
     *reinterpret_cast<f32x4 *>(u.momentum + at) = m;
     *reinterpret_cast<f32x4 *>(u.variance + at) = v;
 }
@@ -1125,13 +1283,15 @@ template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&config
               "w16 LDS size: ");
     configured[device].store(true, std::memory_order_release);
 }
-void launch_fold(hipStream_t stream, const Model &m, const Workspace &r, const Group &group, int count, bool losses) {
-    const int parameters = make_layout(m.depth).count;
-    const bool many = r.blocks > 16;
-    const int blocks = many ? fold_parts(parameters) : fold_parts(parameters) / 4;
-    hipLaunchKernelGGL(many ? w16_fold_kernel<8> : w16_fold_kernel<1>, dim3(blocks + (losses ? m.context : 0), count), dim3(many ? 512 : 256), 0,
-                       stream, r, group, parameters, blocks, m.tokens / m.context, m.context);
-    check_hip(hipGetLastError(), "w16 fold launch: ");
+void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const Group &group, int count, bool losses) {
+    const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
+    static std::atomic<bool> configured[64];
+    allow_lds(w16_weight_gradient_kernel, configured, GRADIENT_LDS);
+    hipLaunchKernelGGL(w16_weight_gradient_kernel, dim3((m.depth + 2) * ((r.chunks + 7) / 8 * 8), count), dim3(64 * WAVES), GRADIENT_LDS,
+                       stream, m, r, group, parameters);
+    hipLaunchKernelGGL(w16_fold_kernel, dim3(blocks + (losses ? m.context : 0), count), dim3(256), 0, stream, r, group, parameters, blocks,
+                       m.tokens / m.context, m.context);
+    check_hip(hipGetLastError(), "w16 weight gradient launch: ");
 }
 } // namespace
 
@@ -1144,13 +1304,10 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
         const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        static std::atomic<bool> configured[4][64];
-        const bool wide = r.waves_per_block == 8;
-        const auto kernel = with_gradient ? (wide ? w16_forward_kernel<true, 8> : w16_forward_kernel<true, 4>)
-                                          : (wide ? w16_forward_kernel<false, 8> : w16_forward_kernel<false, 4>);
-        allow_lds(kernel, configured[2 * (with_gradient != 0) + wide], lds_bytes(MAX_DEPTH, r.waves_per_block, false));
-        hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * r.waves_per_block), lds_bytes(depth, r.waves_per_block, false), stream, m, x, y, r,
-                           token_losses, logits);
+        static std::atomic<bool> configured[2][64];
+        const auto kernel = with_gradient ? w16_forward_kernel<true> : w16_forward_kernel<false>;
+        allow_lds(kernel, configured[with_gradient != 0], staged_bytes(MAX_DEPTH));
+        hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, x, y, r, token_losses, logits);
         check_hip(hipGetLastError(), "w16_forward launch: ");
     });
 }
@@ -1163,16 +1320,13 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
         const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        static std::atomic<bool> configured[2][64];
-        const bool wide = r.waves_per_block == 8;
-        const auto kernel = wide ? w16_backward_kernel<8> : w16_backward_kernel<4>;
-        allow_lds(kernel, configured[wide], lds_bytes(MAX_DEPTH, r.waves_per_block, true));
-        hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * r.waves_per_block), lds_bytes(depth, r.waves_per_block, true), stream, m, x, r,
-                           make_layout(depth).count);
+        static std::atomic<bool> configured[64];
+        allow_lds(w16_backward_kernel, configured, staged_bytes(MAX_DEPTH));
+        hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
         check_hip(hipGetLastError(), "w16_backward launch: ");
         Group group{};
-        group.member[0].workspace = workspace, group.member[0].gradient = gradient;
-        launch_fold(stream, m, r, group, 1, false);
+        group.member[0].tokens = const_cast<uint8_t *>(x), group.member[0].workspace = workspace, group.member[0].gradient = gradient;
+        launch_weight_gradients(stream, m, r, group, 1, false);
     });
 }
 
@@ -1180,10 +1334,10 @@ int w16_blocks(int batch, int context) {
     return blocks_of(batch, context);
 }
 int w16_norm_count(int depth) {
-    return fold_parts(make_layout(depth).count) / FOLD_PARTS;
+    return fold_blocks(make_layout(depth).count) / FOLD_QUARTERS;
 }
 int w16_norm_parts() {
-    return FOLD_PARTS;
+    return FOLD_QUARTERS;
 }
 void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, const W16Batch *batches) {
     require(context == 4 || context == 8, "w16: a training step has a context of 4 or 8");
@@ -1192,15 +1346,13 @@ void w16_gradients(hipStream_t stream, int depth, int batch, int context, const 
     const Workspace r = carve(depth, batch, context, batches[0].workspace);
     Group group{};
     std::copy(batches, batches + count, group.member);
-    static std::atomic<bool> configured[4][64];
-    const bool wide = r.waves_per_block == 8;
-    const auto kernel = context == 4 ? (wide ? w16_step_kernel<4, 8> : w16_step_kernel<4, 4>) : (wide ? w16_step_kernel<8, 8> : w16_step_kernel<8, 4>);
-    allow_lds(kernel, configured[2 * (context == 8) + wide], lds_bytes(MAX_DEPTH, r.waves_per_block, true));
+    static std::atomic<bool> configured[2][64];
+    const auto kernel = context == 4 ? w16_step_kernel<4> : w16_step_kernel<8>;
+    allow_lds(kernel, configured[context == 8], staged_bytes(MAX_DEPTH));
     const uint64_t places = uint64_t(data.size) - 8, inverse = places > 1 ? uint64_t((static_cast<unsigned __int128>(1) << 64) / places) : ~uint64_t(0);
-    hipLaunchKernelGGL(kernel, dim3(r.blocks, count), dim3(64 * r.waves_per_block), lds_bytes(depth, r.waves_per_block, true), stream, m, data,
-                       inverse, r, group, make_layout(depth).count);
+    hipLaunchKernelGGL(kernel, dim3(r.blocks, count), dim3(64 * WAVES), staged_bytes(depth), stream, m, data, inverse, r, group);
     check_hip(hipGetLastError(), "w16_step launch: ");
-    launch_fold(stream, m, r, group, count, true);
+    launch_weight_gradients(stream, m, r, group, count, true);
 }
 void w16_updates(hipStream_t stream, int depth, float *momentum, float *variance, int norm_count, int norm_parts, int count,
                  const W16Step *steps) {
