@@ -22,10 +22,10 @@ def reference(qkv, do, B, H, T):
 
 @pytest.mark.parametrize("B,H,T", [(1, 1, 128),    # fewer tiles than waves
                                    (2, 3, 384),    # six tiles: two waves take two
-                                   (16, 9, 128),   # the most blocks that the forward splits at this context
-                                   (29, 5, 128),   # one more
-                                   (9, 12, 128),   # the most that the backward splits
-                                   (109, 1, 128),  # one more: its kernels side by side
+                                   (16, 9, 128),   # 144 blocks of 128 rows: past both lines at this context
+                                   (29, 5, 128),   # one more, a batch that eight does not divide
+                                   (9, 12, 128),   # 108 blocks: both passes split
+                                   (109, 1, 128),  # one more
                                    (32, 6, 256),   # the most that run side by side at this context
                                    (11, 7, 640),   # one more
                                    (4, 13, 1024),  # side by side, pairs dealt
