@@ -1,11 +1,13 @@
 // csrc/readback.hip with the HIP runtime calls that it makes, on the host: compiled for the host alone and not linked with the
 // runtime, so that its error paths and what it asks of the runtime can be tested without a GPU.
 //
-// Modelled is what the runtime documents and no more.  Work queued on a stream runs when somebody waits for it.  An event
+// Modelled is what the runtime documents and no more.  Work queued on a stream runs when somebody waits for it, or, on a stream
+// that a test holds, when the test lets it go.  An event
 // belongs to the device that is current when it is created and is recorded on that device's streams only.  What a kernel
 // writes to pinned memory is there for the host once the kernel has run if the memory was asked for as coherent, otherwise
 // behind an event that releases to the system or a stream synchronization.
 #include "../turbogpt_amd/csrc/readback.hip"
+#include <condition_variable>
 #include <cstring>
 #include <deque>
 #include <functional>
@@ -22,6 +24,7 @@ struct Pinned {
 struct Stream {
     int device;
     std::deque<std::function<void()>> queue;
+    bool held = false; // a kernel in front of the queue still runs
     bool step() {
         if (queue.empty())
             return false;
@@ -37,6 +40,8 @@ struct Event {
     bool pending;
 };
 std::recursive_mutex guard;
+std::condition_variable_any released;
+int waiting = 0; // threads that wait for a held stream
 typedef std::lock_guard<std::recursive_mutex> Lock;
 std::map<void *, Pinned *> pinned; // by the host's address
 std::map<const void *, std::string> kernels;
@@ -138,10 +143,13 @@ hipError_t hipEventRecord(hipEvent_t handle, hipStream_t stream) {
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t handle) {
-    const Lock lock(guard);
+    std::unique_lock<std::recursive_mutex> lock(guard);
     Event *event = reinterpret_cast<Event *>(handle);
     if (fails("hipEventSynchronize"))
         return hipErrorUnknown;
+    ++waiting;
+    released.wait(lock, [&] { return !event->pending || !event->stream->held; });
+    --waiting;
     while (event->pending)
         event->stream->step();
     return hipSuccess;
@@ -181,7 +189,16 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
 }
 
 // ---- for the tests -------------------------------------------------------------------------------------
-void *fake_stream(int device) { return new Stream{device, {}}; }
+void *fake_stream(int device) { return new Stream{device}; }
+void fake_hold(void *stream, int held) {
+    const Lock lock(guard);
+    static_cast<Stream *>(stream)->held = held;
+    released.notify_all();
+}
+int fake_waiting() {
+    const Lock lock(guard);
+    return waiting;
+}
 int fake_queued(void *stream) { return int(static_cast<Stream *>(stream)->queue.size()); }
 void fake_fail(const char *call, int in) { failing[call] = in; }
 int fake_pinned() { return int(pinned.size()); }

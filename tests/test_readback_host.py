@@ -2,6 +2,8 @@
 without its device code, with a model of the calls that it makes (fake_hip.cpp)."""
 import ctypes as C
 import subprocess
+import threading
+import time
 from pathlib import Path
 
 import numpy as np
@@ -23,6 +25,7 @@ def host(tmp_path_factory):
     lib = C.CDLL(str(library))
     lib.fake_stream.restype = lib.readback_open.restype = C.c_void_p
     lib.readback_error.restype = C.c_char_p
+    lib.fake_hold.argtypes = [C.c_void_p, C.c_int]
     lib.fake_queued.argtypes = lib.readback_close.argtypes = [C.c_void_p]
     lib.readback_fetch.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int] + [C.c_void_p] * 4
     return lib
@@ -101,4 +104,33 @@ def test_engines_on_two_devices(host, size):
     for engine in engines:
         assert engine.fetch(size, seed=5) == (True, True), host.readback_error()
         engine.close()
+    assert host.fake_pinned() == host.fake_events() == 0
+
+
+@pytest.mark.parametrize("behind,size", [(16, 16), (20 * CHUNK, 16), (20 * CHUNK, 20 * CHUNK)])
+def test_a_result_does_not_wait_for_another_engines_kernels(host, behind, size):
+    """While one engine's kernels still run, one thread waits for them, however large the result behind them; another engine of the
+    device gets its own result meanwhile, and both have buffers of their own."""
+    slow, other, results = Engine(host), Engine(host), {}
+    host.fake_hold(slow.stream, 1)
+    threads = [threading.Thread(target=lambda: results.update(slow=slow.fetch(behind, seed=1))),
+               threading.Thread(target=lambda: results.update(other=other.fetch(size, seed=2)))]
+    threads[0].start()
+    end = time.monotonic() + 10
+    while not host.fake_waiting() and time.monotonic() < end:
+        time.sleep(0.01)
+    threads[1].start()
+    threads[1].join(5)
+    meanwhile, waiting = dict(results), host.fake_waiting()
+    host.fake_hold(slow.stream, 0)
+    for thread in threads:
+        thread.join()
+    assert meanwhile == {"other": (True, True)} and waiting == 1
+    assert results["slow"] == (True, True)
+    held = host.fake_pinned()
+    for seed in range(2):  # one after the other they need no more
+        assert slow.fetch(behind, seed=seed) == (True, True) and other.fetch(size, seed=seed) == (True, True)
+    assert host.fake_pinned() == held
+    slow.close()
+    other.close()
     assert host.fake_pinned() == host.fake_events() == 0

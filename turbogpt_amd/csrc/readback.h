@@ -18,13 +18,14 @@ class Readback {
   public:
     // The staging memory of a device is shared by its engines in this process and given back with the last of them: pinning
     // it takes longer than most results do (1.2 ms for the 16 MB of a d256 model's gradient and logits, against 1.1 ms for the
-    // whole call).  Calls on several threads take turns; they share one bus.  Devices do not share it: an event is recorded
-    // on streams of the device that it was made on.
+    // whole call).  Devices do not share it: an event is recorded on streams of the device that it was made on.
     static std::shared_ptr<Readback> shared(int device);
     ~Readback();
     Readback(const Readback &) = delete;
     Readback &operator=(const Readback &) = delete;
     // Copies the pieces out behind everything already on `stream`, one of the device's; returns when they are in host memory.
+    // Calls on several threads run side by side, each with buffers of its own: what is on one engine's stream may take long, and
+    // another engine's result does not wait for it.
     void fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces);
 
   private:
@@ -33,9 +34,11 @@ class Readback {
         void *pinned = nullptr, *mapped = nullptr; // the same memory, by host and by device address
         hipEvent_t written = nullptr;
     };
-    static void give_back(const Buffer &buffer);
-    void reserve(size_t count);
+    struct Held; // what a call has taken
+    static void release(const Buffer &buffer);
+    Buffer make() const;
     const int device;
-    std::mutex busy;
-    std::vector<Buffer> buffers; // 2 MiB each, as many as the largest result so far could use: at most 16
+    std::mutex guard;         // of the two below, never held during a wait or a copy
+    std::vector<Buffer> idle; // 2 MiB each
+    size_t made = 0;          // as many as the calls at one time have needed so far, at most 16 each
 };

@@ -5,8 +5,10 @@
 // memory (joining the weight halves on the way, which a host loop did before), and several host threads, each with
 // two buffers of its own, copy finished chunks into the caller's pages while the next ones cross the bus.  What is left
 // behind the last chunk is one thread's copy of it (90 us for 2 MiB), so the last 2 MiB are cut in halves down to 512 KiB; not
-// smaller, as every chunk costs the bus 6 us for its event.  The threads start while what is on the stream still runs: a batch's
-// 16 MB of gradient and logits at d256 875 us behind a wait for the device and in chunks of 2 MiB, 829 so.
+// smaller, as every chunk costs the bus 6 us for its event.  The first chunks go out behind what is on the stream, while that still
+// runs; the caller's thread alone waits for it, and the others start with the first chunk that is there (the next ones take 37 us
+// each to arrive, longer than a thread takes to start): a batch's 16 MB of gradient and logits at d256 812 us with
+// every thread at its own chunks from the start, 751 so.
 //
 // The host reads what a kernel wrote once the event behind the kernel has passed, and nothing else stands between the two.
 // So both halves of that order are asked for by name, whatever the environment's default is: coherent memory, and events
@@ -64,32 +66,59 @@ std::shared_ptr<Readback> Readback::shared(int device) {
         place = staging = std::shared_ptr<Readback>(new Readback(device));
     return staging;
 }
-void Readback::give_back(const Buffer &buffer) {
+void Readback::release(const Buffer &buffer) {
     if (buffer.written)
         (void)hipEventDestroy(buffer.written);
     if (buffer.pinned)
         (void)hipHostFree(buffer.pinned);
 }
 Readback::~Readback() {
-    for (const Buffer &buffer : buffers)
-        give_back(buffer);
+    for (const Buffer &buffer : idle)
+        release(buffer);
 }
-void Readback::reserve(size_t count) {
-    buffers.reserve(count);
-    while (buffers.size() < count) { // a buffer joins the others whole or not at all
-        Buffer buffer;
+Readback::Buffer Readback::make() const { // whole or not at all
+    Buffer buffer;
+    try {
+        check_hip(hipHostMalloc(&buffer.pinned, CHUNK, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent),
+                  "pinned staging: ");
+        check_hip(hipHostGetDevicePointer(&buffer.mapped, buffer.pinned, 0), "pinned staging: ");
+        check_hip(hipEventCreateWithFlags(&buffer.written, hipEventDisableTiming | hipEventReleaseToSystem), "readback event: ");
+    } catch (...) {
+        release(buffer);
+        throw;
+    }
+    return buffer;
+}
+struct Readback::Held {
+    Readback &pool;
+    std::vector<Buffer> buffers;
+    Held(Readback &pool_, size_t count) : pool(pool_) {
+        buffers.reserve(count);
+        size_t missing;
+        {
+            const std::lock_guard<std::mutex> lock(pool.guard);
+            const size_t found = std::min(count, pool.idle.size());
+            missing = count - found;
+            pool.idle.reserve(pool.made + missing); // giving back does not fail
+            pool.made += missing;
+            buffers.insert(buffers.end(), pool.idle.end() - found, pool.idle.end());
+            pool.idle.resize(pool.idle.size() - found);
+        }
         try {
-            check_hip(hipHostMalloc(&buffer.pinned, CHUNK, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent),
-                      "pinned staging: ");
-            check_hip(hipHostGetDevicePointer(&buffer.mapped, buffer.pinned, 0), "pinned staging: ");
-            check_hip(hipEventCreateWithFlags(&buffer.written, hipEventDisableTiming | hipEventReleaseToSystem), "readback event: ");
+            for (; missing; --missing)
+                buffers.push_back(pool.make());
         } catch (...) {
-            give_back(buffer);
+            give_back(missing);
             throw;
         }
-        buffers.push_back(buffer);
     }
-}
+    ~Held() { give_back(0); }
+    void give_back(size_t never_made) {
+        const std::lock_guard<std::mutex> lock(pool.guard);
+        pool.made -= never_made;
+        pool.idle.insert(pool.idle.end(), buffers.begin(), buffers.end());
+    }
+};
 
 void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces) {
     struct Chunk {
@@ -112,30 +141,27 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
     // lane `l` of `lanes` takes chunks l, l + lanes, ... with two buffers of its own in turn
     const size_t lanes = std::min<size_t>(LANES, (chunks.size() + 1) / 2);
     const size_t depth = chunks.size() == 1 ? 1 : 2;
-    const std::lock_guard<std::mutex> lock(busy);
-    check_hip(hipSetDevice(device)); // its events are made here
-    reserve(lanes * depth);
-    const auto lane = [&](size_t l) {
-        const auto start = [&](size_t round) {
-            const size_t c = l + round * lanes;
-            if (c >= chunks.size())
-                return;
-            Buffer &buffer = buffers[l * depth + round % depth];
-            enqueue(stream, *chunks[c].piece, chunks[c].offset, chunks[c].bytes, buffer.mapped);
-            check_hip(hipEventRecord(buffer.written, stream));
-        };
-        for (size_t round = 0; round + 1 < depth; ++round)
-            start(round);
-        for (size_t round = 0; l + round * lanes < chunks.size(); ++round) {
-            start(round + depth - 1);
-            const Chunk &c = chunks[l + round * lanes];
-            const Buffer &buffer = buffers[l * depth + round % depth];
-            check_hip(hipEventSynchronize(buffer.written), "readback: ");
-            std::memcpy(static_cast<uint8_t *>(c.piece->host) + c.offset, buffer.pinned, c.bytes);
-        }
-    };
     if (!lanes)
         return;
+    check_hip(hipSetDevice(device)); // its events are made here
+    const Held held(*this, lanes * depth);
+    const auto buffer = [&](size_t l, size_t round) -> const Buffer & { return held.buffers[l * depth + round % depth]; };
+    const auto start = [&](size_t l, size_t round) {
+        const size_t c = l + round * lanes;
+        if (c >= chunks.size())
+            return;
+        enqueue(stream, *chunks[c].piece, chunks[c].offset, chunks[c].bytes, buffer(l, round).mapped);
+        check_hip(hipEventRecord(buffer(l, round).written, stream));
+    };
+    const auto wait = [&](size_t l, size_t round) { check_hip(hipEventSynchronize(buffer(l, round).written), "readback: "); };
+    const auto lane = [&](size_t l) {
+        for (size_t round = 0; l + round * lanes < chunks.size(); ++round) {
+            const Chunk &c = chunks[l + round * lanes];
+            wait(l, round);
+            std::memcpy(static_cast<uint8_t *>(c.piece->host) + c.offset, buffer(l, round).pinned, c.bytes);
+            start(l, round + depth);
+        }
+    };
     std::vector<std::exception_ptr> failures(lanes);
     std::vector<std::thread> threads;
     const auto guarded_lane = [&](size_t l) {
@@ -146,6 +172,15 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
             failures[l] = std::current_exception();
         }
     };
+    try {
+        for (size_t round = 0; round < depth; ++round)
+            for (size_t l = 0; l < lanes; ++l)
+                start(l, round);
+        wait(0, 0);
+    } catch (...) {
+        (void)hipStreamSynchronize(stream); // nothing may still write to the staging buffers
+        throw;
+    }
     try {
         for (size_t l = 1; l < lanes; ++l)
             threads.emplace_back(guarded_lane, l);
@@ -158,7 +193,7 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
         thread.join();
     for (const std::exception_ptr &failure : failures)
         if (failure) {
-            (void)hipStreamSynchronize(stream); // nothing may still write to the staging buffers
+            (void)hipStreamSynchronize(stream); // as above
             std::rethrow_exception(failure);
         }
 }
