@@ -157,7 +157,8 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
     const auto lane = [&](size_t l) {
         for (size_t round = 0; l + round * lanes < chunks.size(); ++round) {
             const Chunk &c = chunks[l + round * lanes];
-            wait(l, round);
+            if (l || round) // the first chunk has been waited for
+                wait(l, round);
             std::memcpy(static_cast<uint8_t *>(c.piece->host) + c.offset, buffer(l, round).pinned, c.bytes);
             start(l, round + depth);
         }
