@@ -967,11 +967,9 @@ extern "C" int tgk_sumsq_partials(hipStream_t stream, const float *g, size_t n, 
 
 extern "C" int tgk_sumsq_segments(hipStream_t stream, const float *g, const void *segments, int count, float *partials) {
     return guarded([&] {
-        aligned(g, "sumsq_segments: g");
-        require(segments && !(reinterpret_cast<uintptr_t>(segments) & 7) && partials && count > 0 && count <= 4096,
-                "sumsq_segments: 1..4096 ranges in a device array, and their partials");
-        hipLaunchKernelGGL(sumsq_segments_kernel, dim3(count), dim3(256), 0, stream,
-                           SumsqSegments{g, static_cast<const SumsqSegment *>(segments), count, partials});
+        const SumsqSegments s{g, static_cast<const SumsqSegment *>(segments), count, partials};
+        check_sumsq_segments(s);
+        hipLaunchKernelGGL(sumsq_segments_kernel, dim3(count), dim3(256), 0, stream, s);
         check_hip(hipGetLastError(), "sumsq_segments launch: ");
     });
 }

@@ -2962,6 +2962,8 @@ void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, i
                     (workspace && workspace_bytes >= plan.pieces_bytes && !(reinterpret_cast<uintptr_t>(workspace) & 15)),
                 "gemm_wgrad_list: workspace too small (see tgk_gemm_wgrad_list_workspace)");
         require(!(reinterpret_cast<uintptr_t>(sumsq) & 3), "gemm_wgrad_list: sumsq must be 4-byte aligned");
+        if (ranges.count)
+            check_sumsq_segments(ranges);
         if (plan.edge < 256) {
             WgradTiles w{};
             w.jobs = static_cast<const WgradListJob *>(table);

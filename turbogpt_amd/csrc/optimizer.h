@@ -41,6 +41,11 @@ struct SumsqSegments {
     int count;
     float *partials;
 };
+inline void check_sumsq_segments(const SumsqSegments &s) {
+    require(s.g && !(reinterpret_cast<uintptr_t>(s.g) & 15), "sumsq_segments: g must be non-null and 16-byte aligned");
+    require(s.segments && !(reinterpret_cast<uintptr_t>(s.segments) & 7) && s.partials && s.count > 0 && s.count <= 4096,
+            "sumsq_segments: 1..4096 ranges in a device array, and their partials");
+}
 TG_DEVICE void sumsq_segment(const SumsqSegments &s, int at, float *waves) { // `waves`: shared, 4 floats; the block's first 256 threads
     const SumsqSegment segment = s.segments[at];
     const f32x4 *p = reinterpret_cast<const f32x4 *>(s.g + segment.start);
