@@ -105,7 +105,7 @@ enum {
     TG_CLASS_LAYERNORM_BWD = 6,
     TG_CLASS_HEAD = 7,       /* vocabulary projection: forward, dgrad, wgrad */
     TG_CLASS_OTHER = 8,      /* sampling, embedding, cross-entropy, loss means */
-    TG_CLASS_OPTIMIZER = 9,  /* gradient norm + AdamW */
+    TG_CLASS_OPTIMIZER = 9,  /* gradient norm, where the weight gradients' launch does not leave it, + AdamW */
     TG_CLASS_GEMM_FWD_GELU = 10,   /* MLP-up forward: two outputs, pre-activation and GELU */
     TG_CLASS_GEMM_DGRAD_GELU = 11, /* MLP-down input gradient times GELU' of the saved pre-activation */
     TG_CLASSES = 12

@@ -91,8 +91,8 @@ struct Slot {
     std::vector<WgradLaunch> wgrads; // one; or one a block, the head's and the token table's
     bf16_t *onehot = nullptr; // [tokens][256]: the token table's gradient is one more product of that launch
     // ... and the kernels that write the gradient leave the sums of its squares here (cuda/trainer.cuh:35-46): the
-    // launch above for the matrices, and with it, of the gradients that are there already, for the ranges in `norm_ranges` (every
-    // other tensor)
+    // launch above for the matrices and, of the gradients that are there already, for the ranges in `norm_ranges` (every other
+    // tensor), which are a launch of their own where the tiles are large
     float *norms = nullptr;
     int list_norms = 0, range_norms = 0;
     void *norm_ranges = nullptr;
@@ -346,12 +346,13 @@ struct Engine {
         // Or, where those buffers did not fit, a launch behind the head's input gradient, one in every block, before
         // the block's last kernel overwrites the gradient that entered it, and one at the end.
         const bool together = s.wgrads.size() == 1, norms = together && c.clip > 0;
+        const SumsqSegments ranges = norms ? SumsqSegments{g, static_cast<const SumsqSegment *>(s.norm_ranges), s.range_norms,
+                                                           s.norms + s.list_norms}
+                                           : SumsqSegments{};
         const auto weight_gradients = [&](const Slot::WgradLaunch &part) {
             Scope profile_scope(this, TG_CLASS_GEMM_WGRAD);
-            wgrad_list(stream, M, part.count, s.wgrad_jobs.data() + part.first, ListUnit, part.table, workspace, workspace_bytes,
-                       norms ? s.norms : nullptr,
-                       norms ? SumsqSegments{g, static_cast<const SumsqSegment *>(s.norm_ranges), s.range_norms, s.norms + s.list_norms}
-                             : SumsqSegments{});
+            return wgrad_list(stream, M, part.count, s.wgrad_jobs.data() + part.first, ListUnit, part.table, workspace,
+                              workspace_bytes, norms ? s.norms : nullptr, ranges);
         };
         OP(TG_CLASS_HEAD, tgk_gemm_dgrad_t(stream, M, V, d, logits, V, wt(layout.head), V, t1, d, nullptr, 0));
         if (!together)
@@ -376,7 +377,9 @@ struct Engine {
         OP(TG_CLASS_OTHER, backward_rest(stream, {c.batch, T, d, tokens_in, s.g_x[0], s.onehot, g + layout.positions,
                                                   reinterpret_cast<const float *>(s.ln_partials), ln_stride / sizeof(float),
                                                   2 * c.depth + 1, 0, s.ln_targets, s.token_losses, means}));
-        weight_gradients(s.wgrads.back());
+        const bool summed = weight_gradients(s.wgrads.back());
+        if (norms && !summed)
+            OP(TG_CLASS_OPTIMIZER, tgk_sumsq_segments(stream, g, ranges.segments, ranges.count, ranges.partials));
     }
 
     // learning rates and momenta of optimizer step `at` (0-based)

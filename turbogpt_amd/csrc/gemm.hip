@@ -2950,7 +2950,7 @@ void wgrad_list_prepare(int M, int count, const TgkWgradJob *jobs, int unit, voi
         check_hip(hipMemcpy(table, host.data(), host.size(), hipMemcpyHostToDevice), "wgrad list tables: ");
     }
 }
-void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
+bool wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, int unit, const void *table, void *workspace,
                 size_t workspace_bytes, float *sumsq, const SumsqSegments &ranges) {
     {
         WgradListPlan plan;
@@ -2969,10 +2969,9 @@ void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, i
             w.jobs = static_cast<const WgradListJob *>(table);
             w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
             w.count = plan.tiles, w.k_chunks = M / 64, w.sumsq = sumsq, w.ranges = ranges;
-            return launch_wgrad_tiles(stream, w, plan.edge, plan.launch_blocks);
+            launch_wgrad_tiles(stream, w, plan.edge, plan.launch_blocks);
+            return true;
         }
-        if (ranges.count && tgk_sumsq_segments(stream, ranges.g, ranges.segments, ranges.count, ranges.partials))
-            throw std::runtime_error(tg_last_error);
         WgradList w{};
         w.jobs = static_cast<const WgradListJob *>(table);
         w.tiles = reinterpret_cast<const int4 *>(static_cast<const unsigned char *>(table) + plan.jobs_bytes);
@@ -2997,6 +2996,7 @@ void wgrad_list(hipStream_t stream, int M, int count, const TgkWgradJob *jobs, i
                                plan.rounds * plan.blocks, 4 * plan.launch_blocks);
             check_hip(hipGetLastError(), "wgrad list fold launch: ");
         }
+        return false;
     }
 }
 
