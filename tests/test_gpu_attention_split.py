@@ -32,7 +32,11 @@ def reference(qkv, do, B, H, T):
                                    (5, 13, 1024),  # one after the other
                                    (1, 3, 1280),   # every pair dealt over the XCDs
                                    (1, 9, 1024),   # one of nine dealt
-                                   (3, 11, 1024)])  # forward split, backward side by side, one pair dealt in both
+                                   (3, 11, 1024),   # forward split, backward side by side, one pair dealt in both
+                                   (1, 20, 1280),   # 200 blocks of 128 rows: the most that the backward splits at any context
+                                   (3, 7, 1280),    # 210: side by side
+                                   (2, 12, 2048),   # 384: the most that the forward splits at any context
+                                   (1, 25, 2048)])  # 400: 128-row blocks
 def test_matches_fp32(B, H, T):
     lib, d = library(), 64 * H
     gen = torch.Generator(device="cuda").manual_seed(B * 10000 + H * 100 + T)

@@ -25,8 +25,8 @@ def relative(a, b):
     return float((a.double() - b).norm() / b.norm())
 
 
-# lone 64 x 64 tiles, 8 and 192 of them: a ring of four, from 5 stages on two groups of waves with three each, from 16 on with
-# four; and 512 of them, two a unit, on one group with three
+# 192 lone 64 x 64 tiles: a ring of four, from 5 stages on two groups of waves with three each, from 16 on with four; 8 of them, from
+# 5 stages on as 32 x 32 tiles whose waves have a ring of four each; and 512, two a unit, on one group with three
 @pytest.mark.parametrize("M,N,stages", [(256, 128, s) for s in (2, 4, 6, 7, 8, 10, 11, 15, 16, 17, 23)] +
                          [(1024, 768, s) for s in (4, 5, 7, 15, 16, 17)] + [(1024, 2048, s) for s in (15, 16, 17, 19)])
 def test_turns_of_the_ring(M, N, stages):
@@ -42,7 +42,7 @@ def test_turns_of_the_ring(M, N, stages):
 @pytest.mark.parametrize("transposed", (False, True))
 @pytest.mark.parametrize("stages", (5, 6, 7, 16))
 def test_order_of_two_groups(stages, transposed):
-    """From five stages on a lone 64 x 64 tile is two sums, of its first half of the stages (the odd one with it) and of the rest.
+    """From five stages on a lone 64 x 64 tile, also one cut smaller, is two sums, of its first half of the stages (the odd one with it) and of the rest.
     A 1 in the first half outlives 2^30 and -2^30 in two stages of the second; in one chain it would be lost (an ulp is 64)."""
     M, N, K, half = 256, 128, 64 * stages, 64 * ((stages + 1) // 2)
     x, w = (torch.zeros(n, K, device="cuda", dtype=BF16) for n in (M, N))

@@ -13,9 +13,9 @@ BF16 = torch.bfloat16
 SHAPES = [(128, 128, 64),      # 64 x 64: 4 tiles, one stage
           (384, 640, 192),     # 64 x 64: 60 tiles, three stages
           (1920, 640, 128),    # 64 x 64: 300 tiles, two on some units
-          (128, 192, 576),     # 64 x 64, two groups of waves, nine stages: a width 128 does not divide
-          (640, 640, 320),     # the same, five stages
-          (128, 128, 2048),    # the same, 32 stages
+          (128, 192, 576),     # 6 of 64 x 64 as 32 x 32, nine stages: a width 128 does not divide
+          (640, 640, 320),     # 100 of 64 x 64, [N][K] as 32 x 64, [K][N] on two groups of waves: five stages
+          (128, 128, 2048),    # 4 of 64 x 64 as 32 x 32, 32 stages
           (1024, 2304, 64),    # weights [N][K] on 192 tiles of 128 x 96, [K][N] on 288 of 64 x 128: one stage
           (1152, 1920, 320),   # the same, 180 and 270 tiles, five stages
           (1920, 1920, 64),    # 64 x 128: 450 tiles, one stage

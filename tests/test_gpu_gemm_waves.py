@@ -15,13 +15,13 @@ pytestmark = tiles.pytestmark
                                    (512, 512, 512),    # 64 tiles, four stages a wave: the ring of four
                                    (512, 512, 576),    # one half has a fifth
                                    (384, 192, 960), (512, 512, 1088), (128, 128, 4096),
-                                   (128, 2112, 448), (640, 448, 320),  # 66 and 70 tiles of 64 x 64: on 32 x 64, odd columns
-                                   (384, 704, 832),    # 66 tiles, thirteen stages
+                                   (128, 2048, 448), (128, 2112, 448),  # 64 tiles of 64 x 64, and 66: on 32 x 64, odd columns
+                                   (512, 512, 832), (1408, 192, 832),   # the same, thirteen stages, many rows and few columns
+                                   (640, 576, 320), (384, 768, 832),    # 90 and 72 tiles
                                    (2048, 256, 64), (2048, 256, 256), (2048, 256, 320), (2048, 256, 832), (1024, 512, 3072),
-                                   (128, 4224, 320)])  # 132 tiles: the two groups of waves
+                                   (128, 4224, 320),   # 132 tiles, the next after 128: the two groups of waves
+                                   (128, 4096, 832), (128, 4224, 832)])
 def test_few_tiles(M, N, K):
-    if N % 128 and N % 192:
-        N = -(-N // 192) * 192
     tiles.test_every_tile_with_every_epilogue(M, N, K)
 
 

@@ -1,5 +1,5 @@
-"""Results copied to host memory in pieces (csrc/readback.hip): every bit arrives, whatever the number of 2 MiB chunks -
-one, two, more than all buffers hold at once, with and without a remainder - and from several threads at a time."""
+"""Results copied to host memory in pieces (csrc/readback.hip): every bit arrives, whatever the number of chunks -
+a few, more than all buffers hold at once, with and without a remainder - and from several threads at a time."""
 import threading
 
 import numpy as np
@@ -22,10 +22,10 @@ def roundtrip(cfg, seed):
         assert step == 3
 
 
-@pytest.mark.parametrize("d_model,depth,context", [(128, 1, 128),    # 1.1 MB: one chunk
-                                                   (256, 1, 128),    # 3.8 MB: two chunks, the second short
-                                                   (384, 3, 384),    # 23 MB: 11 chunks for 12 buffers
-                                                   (640, 3, 128)])   # 61 MB: every buffer used twice
+@pytest.mark.parametrize("d_model,depth,context", [(128, 1, 128),    # 1.1 MiB: halves of it down to 512 KiB
+                                                   (256, 1, 128),    # 3.6 MiB: one of 2 MiB, and halves
+                                                   (384, 3, 384),    # 22 MiB, twice that for the moments: 13 chunks, 24
+                                                   (640, 3, 128)])   # 58 MiB: 32 chunks, every buffer used twice and more
 def test_every_bit_of_the_state_arrives(d_model, depth, context):
     roundtrip(ModelConfig(d_model=d_model, depth=depth, context=context, batch=1), 7)
 

@@ -10,11 +10,16 @@ from test_gpu_width16_shapes import run
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("depth,context,batch", [(2, 4, 256), (2, 4, 257), (1, 5, 204), (1, 8, 2048), (1, 8, 2049), (1, 5, 3073), (2, 1, 16385)])
+@pytest.mark.parametrize("depth,context,batch", [(2, 4, 256),    # 16 blocks; eight chunks of 128 tokens, one an XCD
+                                                 (2, 4, 257),    # a sequence in a block and a chunk of its own
+                                                 (1, 5, 204),    # 17 blocks, fifteen tokens a wave; half a ninth chunk
+                                                 (1, 8, 2048),   # a block on every compute unit, 128 chunks
+                                                 (1, 8, 2049),   # one more with one sequence: 257 blocks, 129 chunks
+                                                 (1, 5, 3073), (2, 1, 16385)])  # the same with fifteen and sixteen tokens a wave
 def test_blocks(depth, context, batch):
     """Against the checker within the reference's own bounds; and the same sequences, the last one first, which moves all of them
-    to another wave: every tensor differs by the order of its sums alone, 1e-4 for at most 512 additions of 2^-24 each, three times
-    over."""
+    to another wave: every tensor differs by the order of its sums alone, 1e-4 for at most 257 additions of 2^-24 each (a chunk's
+    tokens, the chunks), six times over."""
     flat = reference_style_weights(depth)
     rng = np.random.default_rng(depth * 100 + context)
     x, y = (rng.integers(0, 256, (batch, context), dtype=np.uint8) for _ in range(2))
