@@ -1021,9 +1021,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
 
 // Up to how many 128-row blocks the 32-row ones with shared-out tiles are taken instead.  The longer the context, the
 // longer the chains that they cut, so the line rises with it.  Forward, microseconds, 128-row / 32-row:
-//   T 128: 120 blocks 4.7 / 4.6   144: 5.0 / 6.6     T 256: 128 blocks 6.6 / 5.3   144: 6.8 / 7.3
-//   T 384: 144 blocks 8.2 / 7.6   162: 8.6 / 8.7     T 512: 192 blocks 10.6 / 9.6   256: 11.0 / 11.0
-//   T 768: 252 blocks 14.4 / 12.6     T 1024: 288 blocks 18.1 / 16.2     T 1152: 324 blocks 20.0 / 18.6     T 1536: 384 blocks 26.1 / 24.2
+//   T 128: 128 blocks 4.6 / 4.6   144: 4.7 / 6.4     T 256: 128 blocks 6.2 / 5.2   144: 6.2 / 6.9
+//   T 384: 144 blocks 7.7 / 7.2   162: 7.8 / 8.1     T 512: 192 blocks 9.4 / 9.0   256: 9.6 / 9.9
+//   T 768: 252 blocks 12.7 / 11.5   288: 12.8 / 14.2     T 1024: 320 blocks 16.5 / 16.4   328: 16.8 / 16.9   352: 16.6 / 17.2
+//   T 1152: 324 blocks 18.4 / 17.1   351: 18.6 / 18.7   360: 18.1 / 18.5     T 1536: 384 blocks 23.3 / 21.9   432: 24.3 / 24.9
+//   T 2048: 384 blocks 29.4 / 27.1   448: 31.5 / 31.0     T 4096: 384 blocks 58.7 / 45.5   448: 60.5 / 53.7     T 8192: 448 blocks 121 / 102
+// So the cap, right at 1536, comes too soon from 4096 on.  A tile's largest probability is 1 in a wave's own sums, where
+// only a row's is in the longer chain: against 64 bits 32-row blocks are nearer by up to 1 % of the outputs' error (13,5,256 1.92e-3
+// against 1.94e-3), of bf16 roundings both.
 bool forward_splits(int B, int H, int T) {
     return size_t(B) * H * (T / 128) <= size_t(std::clamp(T / 4 + 64, 128, 384));
 }
@@ -1032,9 +1037,9 @@ bool forward_splits(int B, int H, int T) {
 // side by side:
 //   T 128: 128 blocks 10.5 / 10.9   144: 13.3 / 13.0     T 256: 128 blocks 11.9 / 13.3   144: 14.1 / 14.4   154: 15.2 / 14.7
 //   T 384: 144 blocks 16.1 / 16.2   162: 17.4 / 16.8     T 512: 128 blocks 14.9 / 18.2   160: 18.7 / 19.0   192: 20.6 / 19.9
-//   T 768: 144 blocks 20.8 / 23.6   192: 24.8 / 25.0     T 1024: 184 blocks 29.8 / 29.9     T 1280: 200 blocks 33.8 / 35.9
-//   T 1536: 216 blocks 41.2 / 41.1     T 2048: 192 blocks 44.5 / 51.4   208: 53.2 / 52.2     T 4096: 192 blocks 82 / 95   224: 98 / 95
-//   T 8192: 128 blocks 99 / 161   192: 148 / 176   256: 185 / 180
+//   T 768: 144 blocks 20.8 / 23.6   192: 24.8 / 25.0     T 1024: 184 blocks 29.8 / 29.9     T 1280: 200 blocks 32.2 / 34.0   210: 35.4 / 34.4
+//   T 1536: 204 blocks 38.2 / 39.6   216: 41.2 / 41.1     T 2048: 192 blocks 43.3 / 49.6   208: 50.6 / 49.7     T 4096: 192 blocks 80 / 92   224: 99 / 92
+//   T 8192: 128 blocks 99 / 161   192: 144 / 174   256: 179 / 175
 // and side by side / one after the other:
 //   T 128: 256 blocks 13.5 / 14.4     T 256: 256 blocks 15.4 / 18.5   512: 28.3 / 24.6     T 512: 384 blocks 27.6 / 30.0   576: 41.5 / 37.6
 //   T 1024: 512 blocks 48.9 / 50.8   768: 70.5 / 67.5     T 2048: 512 blocks 78.9 / 87.5   768: 112 / 108     T 4096: 512 blocks 141 / 163
@@ -1071,8 +1076,8 @@ extern "C" int tgk_attn_fwd(hipStream_t stream, int B, int H, int T, int hd, con
         require(lse && !(reinterpret_cast<uintptr_t>(lse) & 15), "attention: lse must be 16-byte aligned");
         const bool split = forward_splits(B, H, T);
         const CausalGrid grid = split ? causal_grid(B, H, T, 32) : causal_grid(B, H, T, 128, 64);
-        hipLaunchKernelGGL(split ? (T > 128 ? attn_fwd_split_kernel<true> : attn_fwd_split_kernel<false>) : attn_fwd_kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V,
-                           ld, O, ldo, lse, T, grid, scale * LOG2E);
+        const auto kernel = !split ? attn_fwd_kernel : T > 128 ? attn_fwd_split_kernel<true> : attn_fwd_split_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(grid.blocks()), dim3(256), 0, stream, Q, K, V, ld, O, ldo, lse, T, grid, scale * LOG2E);
         check_hip(hipGetLastError(), "attention forward launch: ");
     });
 }

@@ -1096,13 +1096,13 @@ __global__ __launch_bounds__(128 * (BM / WM) * (BN / WN)) void gemm_waves_kernel
 }
 
 // ---- tiles between 64 x 64 and 128 x 96, one a unit ---------------------------------------------------
-// 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48), and 128 x 64 (64 x 32).
-// 257 to 384 tiles of 64 x 64 put two on some units and leave others one; these are at most one a unit (launch_block).  A stage is TileProduct's,
-// with one barrier and every fragment read at once, and costs 0.27 us, two 64 x 64 in company 0.38: copies, reads and products one
-// after the other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 us from
-// the caches against 15.6, 19.3 and 17.5 from memory against 16.7), nor are two stages a barrier (17.9; 18.5); 96 x 32 or 96 x 16 a
-// wave are slower (22.8, 19.3).  The sums' order is
-// that of every tile.  Rows of 16-byte pieces: a lane finishes pieces l, l + 64 and l + 128 of its wave's 192.
+// 96 x 64 and 64 x 96 tiles, a quarter of the outputs a wave (48 x 32, 32 x 48), and 128 x 64 (64 x 32).  257 to 384 tiles of 64 x 64
+// put two on some units and leave others one; these are at most one a unit (launch_block).  A stage is TileProduct's, with one
+// barrier and every fragment read at once, and costs 0.27 us, two 64 x 64 in company 0.38: copies, reads and products one after the
+// other, fewer bytes of each.  Rings of three and five stages are no faster (1920 x 640, K = 3072 17.0 and 16.3 us from the caches
+// against 15.6, 19.3 and 17.5 from memory against 16.7), nor are two stages a barrier (17.9; 18.5); 96 x 32 or 96 x 16 a wave are
+// slower (22.8, 19.3).  The sums' order is that of every tile.  Rows of 16-byte pieces: a lane finishes pieces l, l + 64, ... of its
+// wave's, three of 192 or, with 128 x 64, four of 256.
 template <int BM, int BN, int S, bool BKC, class Epilogue>
 __global__ __launch_bounds__(256) void gemm_uneven_kernel(const bf16_t *__restrict__ A, int lda, const bf16_t *__restrict__ B, int ldb,
                                                           int k_chunks, TileGrid grid, Epilogue epilogue) {
@@ -2339,6 +2339,9 @@ void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_
 // 10.0).  Where 128 does not divide N it stands against three and more tiles of 64 x 64 a unit, whose start and end, GELU above all,
 // take less: it is 5 to 10 % slower up to K = 512 (640 x 4032, 256 with GELU 6.5, 7.0), as fast from 640 to 1024 (4224 x 576, 1024 -2 to
 // +5 %) and 10 to 20 % faster from 1536 on.
+// The costs of 64 x 64 are gemm_tile_kernel's.  Where launch_block puts smaller or uneven tiles in its place (up to 128 and 257 to 512
+// of them), a product costs up to a quarter less than they say, so near the lines to 64 x 128 and 128 x 96 a larger tile may be
+// taken than the fastest; those lines have not been measured again.
 enum Block { BLOCK_64x64, BLOCK_64x128, BLOCK_128x96, BLOCK_128x128, BLOCK_128x192 };
 Block choose_block(int M, int N, int K, bool k_contiguous) {
     static constexpr struct {
