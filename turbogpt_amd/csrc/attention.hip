@@ -1027,7 +1027,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(
 //   T 1152: 324 blocks 18.4 / 17.1   351: 18.6 / 18.7   360: 18.1 / 18.5     T 1536: 384 blocks 23.3 / 21.9   432: 24.3 / 24.9
 //   T 2048: 384 blocks 29.4 / 27.1   448: 31.5 / 31.0     T 4096: 384 blocks 58.7 / 45.5   448: 60.5 / 53.7     T 8192: 448 blocks 121 / 102
 // So the cap, right at 1536, comes too soon from 4096 on.  A tile's largest probability is 1 in a wave's own sums, where
-// only a row's is in the longer chain: against 64 bits 32-row blocks are nearer by up to 1 % of the outputs' error (13,5,256 1.92e-3
+// only a row's is in the longer chain: against 64 bits 32-row blocks are nearer by up to 0.8 % of the outputs' error (13,5,256 1.92e-3
 // against 1.94e-3), of bf16 roundings both.
 bool forward_splits(int B, int H, int T) {
     return size_t(B) * H * (T / 128) <= size_t(std::clamp(T / 4 + 64, 128, 384));
