@@ -76,17 +76,23 @@ TG_DEVICE uint64_t hash_u64(uint64_t x) { // utils.h:13-18
     x = (x ^ (x >> 27)) * 0x94d049bb133111ebULL;
     return x ^ (x >> 31);
 }
+// Over the 64 lanes by halves - lanes 32 apart, 16, 8, 4, 2, 1 - on the vector ALU alone: what is 8 or 4 apart is also that far
+// away within its row of sixteen turned round, as the values repeat there by then.
+template <class Join> TG_DEVICE float wave_join(float x, Join &&join) {
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = join(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = join(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+    x = join(x, __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), 0x128, 0xF, 0xF, true)))); // row_ror:8
+    x = join(x, __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), 0x124, 0xF, 0xF, true)))); // row_ror:4
+    x = join(x, __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), 0x4E, 0xF, 0xF, true))));  // quad_perm [2,3,0,1]
+    return join(x, __uint_as_float(uint32_t(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), 0xB1, 0xF, 0xF, true)))); // [1,0,3,2]
+}
 TG_DEVICE float wave_sum(float x) {
-#pragma unroll
-    for (int k = 32; k; k >>= 1)
-        x += __shfl_xor(x, k, 64);
-    return x;
+    return wave_join(x, [](float a, float b) { return a + b; });
 }
 TG_DEVICE float wave_max(float x) {
-#pragma unroll
-    for (int k = 32; k; k >>= 1)
-        x = fmaxf(x, __shfl_xor(x, k, 64));
-    return x;
+    return wave_join(x, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // One wave-wide global -> LDS copy of 16 bytes per lane (global_load_lds_dwordx4): lane l lands at

@@ -26,8 +26,8 @@ struct W16Batch {
 int w16_blocks(int batch, int context); // of a batch's forward and backward pass
 int w16_norm_count(int depth);
 int w16_norm_parts();
-// Samples the batches, forward, backward.  A context of 4 or 8.
-void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, const W16Batch *batches);
+// Samples the batches, forward, backward.  A context of 4 or 8.  flying: how many such calls run side by side, on streams of their own.
+void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, int flying, const W16Batch *batches);
 // AdamW on embedding, scales and head, Muon on the hidden matrices (cuda/optim.cuh:66-119): each step reads the weights at
 // `from`, which are those that the step before it wrote, and writes them to `to` (which may be the same).  norms:
 // norm_count sums of squares, in norm_parts parts each (1 or w16_norm_parts()).

@@ -4,11 +4,12 @@
 // cuda/ops.cuh:57-144, cuda/attention.cuh:4-106, cuda/optim.cuh:17-119.
 //
 // What bounds it is latency: a step is 1 GFLOP over some ten thousand tokens, and a sequence (at most eight positions)
-// never leaves a wave.  So a wave takes sixteen tokens - whole sequences - through all layers in registers, forward and
-// backward, with the weights staged in LDS as matrix operands.  Products run on
+// never leaves a team.  So a team of four waves takes sixteen tokens - whole sequences - through all layers in registers and LDS,
+// forward and backward, with the weights staged in LDS as matrix operands.  Products run on
 // v_mfma_f32_16x16x4_f32, which is bit for bit a chain of fmaf over its four k (measured on random and extreme values;
 // the bf16 forms add in an order of their own): every sum has one order, the k's own, whatever the kernel's shape, so
-// results do not depend on how the work is cut.  Lane 16 g + c works for token c:
+// results do not depend on how the work is cut.  This instruction takes 32 cycles in which its SIMD does no vector arithmetic,
+// of no wave (measured); of that a lone wave issues one instruction in five cycles, two waves two.  Lane 16 g + c works for token c:
 //   "feed" layout: register j holds feature 4 j + g - what step j of a product over features wants from that lane;
 //   "head" layout: register r holds feature 4 g + r - head g of the token, one head a lane, so attention reads other
 //   positions' keys and values with DPP row shifts.
@@ -29,7 +30,9 @@
 namespace {
 
 constexpr int W = 16, HEADS = 4, F = 48, V = 256, MAX_DEPTH = 8;
-constexpr int WAVES = 4;       // waves of a block: they share the staged weights
+constexpr int ROLES = 4;       // waves of a team, which has sixteen tokens; or it is a lone wave
+__host__ __device__ constexpr int block_waves(int roles) { return roles == 1 ? 8 : 16; } // they stage the weights, as many stay as are in teams
+constexpr int WAVES = 4;       // waves of a block of weight gradients, whose chunks are whole numbers of four teams' tokens
 constexpr int CHUNK_WAVES = 8; // waves' tokens in one partial sum of a weight gradient (128 tokens)
 
 struct Layer {
@@ -62,20 +65,19 @@ Layout make_layout(int depth) {
     return p;
 }
 
-// Rows kept between the launches, a tile of 64 x 8 bytes a wave and quantity in the lanes' own order.  For the backward
-// pass: block input, post-RoPE query, the winning key and value (head layout), post-attention residual, gate | up
-// (cuda/types.cuh:40-44, cuda/model.cuh:25-29).  For the weight gradients, side by side: normalised rows, attention output,
-// activation, and the gradients that are their other operands.  And words: GELU(top), GELU'(top), distance to the
-// winner, the two inverse norms.
-enum Tile {
-    T_X, T_Q, T_KEY, T_VALUE, T_MIDDLE, T_GU, T_OPERANDS = T_GU + 6,
-    T_N1 = T_OPERANDS, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, TILES
-};
-constexpr int OPERANDS = TILES - T_OPERANDS;
-enum Word { WORD_GATE, WORD_SLOPE, WORD_DISTANCE, WORD_INV1, WORD_INV2, WORDS };
+// Rows that a team leaves for the weight gradients, tiles of 64 x 8 bytes in the lanes' own order, side by side: normalised
+// rows, attention output, activation, and the gradients that are their other operands.
+enum Tile { T_N1, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, OPERANDS };
+// And what its own backward pass wants of a layer (cuda/types.cuh:40-44, cuda/model.cuh:25-29), a record of ROW_BYTES: tiles of
+// block input, post-RoPE query, the winning key and value (head layout) and post-attention residual; a word a lane of
+// GELU(top) and GELU'(top), a byte of the distance to the winner; a word a token of the two inverse norms.
+enum RowTile { R_X, R_Q, R_KEY, R_VALUE, R_MIDDLE, ROW_TILES };
+enum RowWord { R_GATE, R_SLOPE, ROW_WORDS };
+constexpr int ROW_DISTANCE = ROW_TILES * 512 + ROW_WORDS * 256, ROW_INVERSE = ROW_DISTANCE + 64, ROW_BYTES = ROW_INVERSE + 2 * W * 4;
+constexpr int ROW_FEATURES = ROW_BYTES, LONE_ROW_BYTES = ROW_FEATURES + 6 * 512; // a lone wave keeps gate and up there, too
 struct Workspace {
-    u32x2 *tiles;    // [depth][waves][TILES][64]
-    float *words;    // [depth][waves][WORDS][64]
+    u32x2 *tiles;        // [depth][waves][OPERANDS][64]
+    unsigned char *rows; // [depth][waves][LONE_ROW_BYTES], where they do not stay in LDS
     float *gz;       // [2 depth + 1][waves * 16][16]: g * z of every RMSNorm scale; the final norm's last
     u32x2 *hidden, *nf, *dh; // [waves][64]
     float *inverse;  // [waves][64] of the final norm
@@ -87,7 +89,7 @@ struct Workspace {
 // another batch's, whose memory lies `apart` bytes further on
 TG_DEVICE Workspace moved(Workspace s, int64_t apart) {
     const auto move = [&](auto *&p) { p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<char *>(p) + apart); };
-    move(s.tiles), move(s.words), move(s.gz), move(s.hidden), move(s.nf), move(s.dh), move(s.inverse), move(s.dlogits), move(s.partials);
+    move(s.tiles), move(s.rows), move(s.gz), move(s.hidden), move(s.nf), move(s.dh), move(s.inverse), move(s.dlogits), move(s.partials);
     return s;
 }
 int tokens_per_wave(int context) { return 16 / context * context; }
@@ -107,8 +109,8 @@ Workspace carve(int depth, int batch, int context, void *base) {
     r.waves = r.blocks * WAVES;
     r.chunks = (r.waves + CHUNK_WAVES - 1) / CHUNK_WAVES;
     const size_t n = size_t(r.waves) * 64;
-    r.tiles = static_cast<u32x2 *>(take(n * depth * TILES * sizeof(u32x2)));
-    r.words = static_cast<float *>(take(n * depth * WORDS * sizeof(float)));
+    r.tiles = static_cast<u32x2 *>(take(n * depth * OPERANDS * sizeof(u32x2)));
+    r.rows = static_cast<unsigned char *>(take(size_t(r.waves) * depth * LONE_ROW_BYTES));
     r.gz = static_cast<float *>(take(n * (2 * depth + 1) * 4 * sizeof(float)));
     r.hidden = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
     r.nf = static_cast<u32x2 *>(take(n * sizeof(u32x2)));
@@ -138,13 +140,43 @@ TG_DEVICE f32x4 rounded(const f32x4 &v) {
     return unpack4(pack4(v));
 }
 constexpr f32x4 ZERO = {0.f, 0.f, 0.f, 0.f};
+// These values are worked out here and not further on.
+template <class T> TG_DEVICE void ready(T &value) {
+    asm volatile("" : "+v"(value));
+}
+template <class T, class... More> TG_DEVICE void ready(T &value, More &...more) {
+    ready(value);
+    ready(more...);
+}
+// No vector arithmetic moves across; memory and scalar instructions may.
+TG_DEVICE void products_only() {
+    __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80);
+}
 // D[row][col] = fmaf chain over k = 0 .. 15 of A[row][k] B[k][col], on top of acc: lane 16 g + c gives A[c][4 j + g] and
-// B[4 j + g][c] in register j and gets D[4 g + r][c] in register r
-TG_DEVICE f32x4 multiply(const f32x4 &a, const f32x4 &b, f32x4 acc = ZERO) {
+// B[4 j + g][c] in register j and gets D[4 g + r][c] in register r.  The four instructions stand together: a wave's vector arithmetic
+// and this form of product take turns, 33 cycles a product in a chain, but 50 with the next one's operand made between them.
+TG_DEVICE f32x4 multiply(f32x4 a, f32x4 b, f32x4 acc = ZERO) {
+    ready(a, b);
+    products_only();
 #pragma unroll
     for (int j = 0; j < 4; ++j)
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+    products_only();
     return acc;
+}
+// N products with the same second operand
+template <int N> TG_DEVICE void multiply_all(f32x4 (&a)[N], f32x4 b, f32x4 (&product)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+        ready(a[n]), product[n] = ZERO;
+    ready(b);
+    products_only();
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            product[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][j], b[j], product[n], 0, 0, 0);
+    products_only();
 }
 TG_DEVICE float swap_add_16(float x) {
     const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -204,28 +236,41 @@ TG_DEVICE float divide(float x, float b, float r) {
     const float q = x * r;
     return fmaf(fmaf(-q, b, x), r, q);
 }
-// 1 / (1 + e^-x) taken 2^24 times too large, where the reciprocal stays in the normal range down to e^-x = 2^128; beyond that
-// 2^-126 stands for it, which the last product rounds to 0.
+// e^-x for a bf16 value x, bit for bit expf's over all of them: log2(e) in sixteen bits times x is exact, so that what the
+// rounding to a power of two leaves is, too, and one fused step brings the rest.  Beyond +-200 the result is 0 or infinite.
+TG_DEVICE float exp_of_minus(float x) {
+    const float y = __builtin_amdgcn_fmed3f(-x, -200.f, 200.f), t = y * 1.44268798828125f, n = __builtin_rintf(t);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(y, 7.052607713e-06f, t - n)), int(n));
+}
+// 1 / (1 + e^-x) of a bf16 value, taken 2^24 times too large, where the reciprocal stays in the normal range down to
+// e^-x = 2^128; beyond that 2^-126 stands for it, which the last product rounds to 0.  (Of NaN any value: it is multiplied by x.)
 TG_DEVICE float sigmoid(float x) {
-    return reciprocal(fminf(fmaf(expf(-x), 0x1p-24f, 0x1p-24f), 0x1p126f)) * 0x1p-24f;
+    return reciprocal(fminf(fmaf(exp_of_minus(x), 0x1p-24f, 0x1p-24f), 0x1p126f)) * 0x1p-24f;
 }
 
 struct Model {
     const bf16_t *hi;
     const uint16_t *lo;
     int depth, tokens, context, per_wave;
+    int teams; // of a block
 };
-// a lane's place: token `token` (if `live`) at `position` of its sequence
+// a lane's place: token `token` (if `live`) at `position` of its sequence, in the team `wave` of the batch, of which its wave
+// has the role `role`
 struct Lane {
-    int lane, c, g, wave, token, position;
+    int lane, c, g, wave, role, team, token, position;
     bool live;
 };
-TG_DEVICE Lane lane_of(const Model &m) {
+// Consecutive waves of a block sit on consecutive SIMDs: the teams' first roles, which have the longest way, on different ones.
+// A team beyond the batch's last repeats that one.
+template <int R = ROLES> TG_DEVICE Lane lane_of(const Model &m, int waves) {
     Lane p;
+    const int at = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     p.lane = threadIdx.x & 63;
     p.c = p.lane & 15;
     p.g = p.lane >> 4;
-    p.wave = blockIdx.x * WAVES + (threadIdx.x >> 6);
+    p.team = at / R;
+    p.role = (at + p.team) % R;
+    p.wave = min(int(blockIdx.x) * m.teams + p.team, waves - 1);
     p.token = p.wave * m.per_wave + p.c;
     p.live = p.c < m.per_wave && p.token < m.tokens;
     p.position = p.c % m.context;
@@ -236,12 +281,22 @@ TG_DEVICE Lane lane_of(const Model &m) {
 // 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
 // The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
 // Operands of dX = dY W (rows = inputs, k = outputs) are read from the same tiles with the transposing load, in feed
-// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Last
-// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own.
+// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Then
+// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own; behind the first
+// layer, which no wave passes before all have read theirs, its place is the teams' for the sums of the softmax.  Last, for
+// each team, what its waves hand one another and, where they fit, the rows that the backward pass wants.
 constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
 __host__ __device__ constexpr int staged_tiles(int depth) { return depth * (LAYER_TILES + 1) + HEAD_TILES; }
 __host__ __device__ constexpr size_t embedding_at(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
-__host__ __device__ constexpr size_t staged_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
+constexpr int EXCHANGE_BYTES = 16 * 1024 + 2 * ROLES * W * 4; // tiles, and a maximum and a picked logit of every role and token
+__host__ __device__ constexpr size_t teams_at(int depth, int teams) {
+    return embedding_at(depth) + (teams * 4096 > V * W * 2 ? teams * 4096 : V * W * 2);
+}
+__host__ __device__ constexpr size_t team_bytes(int depth, bool rows) { return EXCHANGE_BYTES + (rows ? depth * ROW_BYTES : 0); }
+__host__ __device__ constexpr size_t lds_bytes(int depth, int teams, bool rows) { return teams_at(depth, teams) + teams * team_bytes(depth, rows); }
+__host__ __device__ constexpr size_t lone_lds_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
+constexpr size_t LDS_BYTES = 160 * 1024;
+constexpr int STEP_TEAMS = 4; // of a unit, in batches in flight
 TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its own inverse
 // Byte offset, in a tile of items (g, c), of the item that lane 16 q + 4 j + m addresses for a transposing load: (m, 4 q + j)
 // or (m, 4 j + q).  Lane 16 q + i then gets element i % 4 of items (i / 4, 4 q + 0..3) or (i / 4, 4 * 0..3 + q).
@@ -252,14 +307,16 @@ TG_DEVICE int across_offset(int lane, bool natural) {
 TG_DEVICE u32x2 read_across(const unsigned char *at) {
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)at));
 }
-// Wave w stages tiles w, w + 4 and w + 8 of every layer, the thirteenth of layers w and w + 4, and four of the head's: all
-// loads go out before the first is waited for, and every address is a layer's away from the one before.
-struct Staging {
-    static constexpr int PER_LAYER = 3, TAIL = MAX_DEPTH * PER_LAYER, LAST = MAX_DEPTH / WAVES, HEADS = HEAD_TILES / WAVES, SCALES = 2;
+// Of n waves, wave w stages tiles w, w + n, ... of every layer and of the head: all loads go out before the first is waited for,
+// and every address is a layer's away from the one before.
+template <int R = ROLES> struct Staging {
+    static constexpr int WAVES = block_waves(R), PER_LAYER = (LAYER_TILES + WAVES - 1) / WAVES, HEADS = HEAD_TILES / WAVES;
+    static_assert(WAVES * 64 >= (2 * MAX_DEPTH + 1) * W && HEADS * WAVES == HEAD_TILES && V * W * 2 <= WAVES * 1024,
+                  "every scale has a thread, every tile a wave, every KiB of the embedding one");
     const Model &m;
     unsigned char *tiles;
-    u32x2 v[TAIL + LAST + HEADS];
-    float scale[SCALES];
+    u32x2 v[PER_LAYER][MAX_DEPTH], head[HEADS];
+    float scale;
     int lane, wave;
     TG_DEVICE Staging(const Model &m_, unsigned char *memory)
         : m(m_), tiles(memory), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
@@ -271,48 +328,34 @@ struct Staging {
         return k < 4 ? q.qkv + k * 256 : k < 10 ? q.gate + (k - 4) * 256 : q.down + (k - 10) * 16;
     }
     TG_DEVICE void request() {
-        const bf16_t *of_layer[PER_LAYER], *last = m.hi + tile_offset(12) + wave * LAYER_SIZE + row_offset(F);
 #pragma unroll
-        for (int i = 0; i < PER_LAYER; ++i) // rows of `down` are 48 long
-            of_layer[i] = m.hi + tile_offset(wave + i * WAVES) + (wave + i * WAVES < 10 ? row_offset(W) : row_offset(F));
+        for (int i = 0; i < PER_LAYER; ++i) {
+            const int k = wave + i * WAVES;
+            if (k >= LAYER_TILES)
+                break;
+            const bf16_t *from = m.hi + tile_offset(k) + (k < 10 ? row_offset(W) : row_offset(F)); // rows of `down` are 48 long
 #pragma unroll
-        for (int l = 0; l < MAX_DEPTH; ++l)
-            if (l < m.depth)
-#pragma unroll
-                for (int i = 0; i < PER_LAYER; ++i)
-                    v[l * PER_LAYER + i] = *reinterpret_cast<const u32x2 *>(of_layer[i] + l * LAYER_SIZE);
-#pragma unroll
-        for (int i = 0; i < LAST; ++i)
-            if (wave + i * WAVES < m.depth)
-                v[TAIL + i] = *reinterpret_cast<const u32x2 *>(last + i * WAVES * LAYER_SIZE);
-        const bf16_t *head = m.hi + V * W + m.depth * LAYER_SIZE + W + wave * 256 + row_offset(W);
+            for (int l = 0; l < MAX_DEPTH; ++l) // a layer beyond the last is the last again
+                v[i][l] = *reinterpret_cast<const u32x2 *>(from + min(l, m.depth - 1) * LAYER_SIZE);
+        }
 #pragma unroll
         for (int i = 0; i < HEADS; ++i)
-            v[TAIL + LAST + i] = *reinterpret_cast<const u32x2 *>(head + i * WAVES * 256);
-#pragma unroll
-        for (int i = 0; i < SCALES; ++i) {
-            const int at = threadIdx.x + i * 64 * WAVES, n = at >> 4; // attention and MLP norm of each layer, final
-            const Layer q = layer_layout(n >> 1);
-            const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
-            if (n <= 2 * m.depth)
-                scale[i] = master(m.hi, m.lo, offset + (at & 15));
-        }
+            head[i] = *reinterpret_cast<const u32x2 *>(m.hi + V * W + m.depth * LAYER_SIZE + W + row_offset(W) + (wave + i * WAVES) * 256);
+        const int n = threadIdx.x >> 4; // attention and MLP norm of each layer, final
+        const Layer q = layer_layout(n >> 1);
+        const int offset = n == 2 * m.depth ? V * W + m.depth * LAYER_SIZE : (n & 1) ? q.mlp_norm : q.attention_norm;
+        if (n <= 2 * m.depth)
+            scale = master(m.hi, m.lo, offset + (threadIdx.x & 15));
     }
-    // 8 KiB, 16 bytes a lane; `aligned` is false where the weights are not
+    // 8 KiB, 16 bytes a lane of the last eight waves; `aligned` is false where the weights are not
     TG_DEVICE void request_embedding(bool aligned = true) const {
-        if (!aligned) {
-            const u32x2 *from = reinterpret_cast<const u32x2 *>(m.hi);
-            u32x2 *to = reinterpret_cast<u32x2 *>(tiles + embedding_at(m.depth));
-#pragma unroll
-            for (int i = 0; i < V * W / 4 / (64 * WAVES); ++i)
-                to[threadIdx.x + i * 64 * WAVES] = from[threadIdx.x + i * 64 * WAVES];
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < V * W * 2 / 1024 / WAVES; ++i) {
-            const int piece = i * WAVES + wave;
-            async_copy16(lds_address(tiles) + uint32_t(embedding_at(m.depth)) + uint32_t(piece * 1024), m.hi, uint32_t(piece * 1024 + lane * 16));
-        }
+        unsigned char *to = tiles + embedding_at(m.depth);
+        const int piece = wave - (WAVES - V * W * 2 / 1024);
+        if (!aligned)
+            for (int i = threadIdx.x; i < V * W / 4; i += WAVES * 64)
+                reinterpret_cast<u32x2 *>(to)[i] = reinterpret_cast<const u32x2 *>(m.hi)[i];
+        else if (piece >= 0)
+            async_copy16(lds_address(to) + uint32_t(piece * 1024), m.hi, uint32_t(piece * 1024 + lane * 16));
     }
     TG_DEVICE static uint16_t element(const u32x2 &v, int e) { return uint16_t((e < 2 ? v.x : v.y) >> ((e & 1) * 16)); }
     // element e of a lane's four is k = 4 j + e: item (e, row), element j.  `to`: the lane's place in the tile
@@ -323,42 +366,37 @@ struct Staging {
     }
     TG_DEVICE void finish(bool backward) {
         const int row = lane >> 2, j = lane & 3;
-        unsigned char *natural = tiles + row * 8 + j * 2, *feed = tiles + feed_row(row) * 8 + j * 2, *of_layer[PER_LAYER];
-#pragma unroll
-        for (int i = 0; i < PER_LAYER; ++i)
-            of_layer[i] = (wave + i * WAVES > 2 ? feed : natural) + (wave + i * WAVES) * 512;
-        // the attention projection (wave 3's first) again: rows = inputs 4 j + e, k = output `row`: item (row % 4, input), element row / 4
+        unsigned char *natural = tiles + row * 8 + j * 2, *feed = tiles + feed_row(row) * 8 + j * 2;
+        // the attention projection again: rows = inputs 4 j + e, k = output `row`: item (row % 4, input), element row / 4
         unsigned char *turned = tiles + (m.depth * LAYER_TILES + HEAD_TILES) * 512 + ((row & 3) * 16 + 4 * j) * 8 + (row >> 2) * 2;
 #pragma unroll
-        for (int l = 0; l < MAX_DEPTH; ++l)
-            if (l < m.depth) {
+        for (int i = 0; i < PER_LAYER; ++i) {
+            const int k = wave + i * WAVES;
+            if (k >= LAYER_TILES)
+                break;
+            unsigned char *to = (k > 2 ? feed : natural) + k * 512;
 #pragma unroll
-                for (int i = 0; i < PER_LAYER; ++i)
-                    put(of_layer[i] + l * LAYER_TILES * 512, v[l * PER_LAYER + i]);
-                if (backward && wave == 3)
+            for (int l = 0; l < MAX_DEPTH; ++l) {
+                if (l >= m.depth)
+                    break;
+                put(to + l * LAYER_TILES * 512, v[i][l]);
+                if (backward && k == 3)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        *reinterpret_cast<uint16_t *>(turned + l * 512 + e * 8) = element(v[l * PER_LAYER], e);
+                        *reinterpret_cast<uint16_t *>(turned + l * 512 + e * 8) = element(v[i][l], e);
             }
-#pragma unroll
-        for (int i = 0; i < LAST; ++i)
-            if (wave + i * WAVES < m.depth)
-                put(feed + ((wave + i * WAVES) * LAYER_TILES + 12) * 512, v[TAIL + i]);
+        }
 #pragma unroll
         for (int i = 0; i < HEADS; ++i)
-            put(feed + (m.depth * LAYER_TILES + wave + i * WAVES) * 512, v[TAIL + LAST + i]);
-#pragma unroll
-        for (int i = 0; i < SCALES; ++i) {
-            const int at = threadIdx.x + i * 64 * WAVES;
-            if (at < (2 * m.depth + 1) * W)
-                scales()[at] = scale[i];
-        }
+            put(feed + (m.depth * LAYER_TILES + wave + i * WAVES) * 512, head[i]);
+        if (int(threadIdx.x) < (2 * m.depth + 1) * W)
+            scales()[threadIdx.x] = scale;
         wait_vmcnt<0>(); // the embedding
         __syncthreads();
     }
+    // whether this wave is in a team; the others have done their part
+    TG_DEVICE bool stays() const { return wave < m.teams * R; }
 };
-static_assert(Staging::SCALES * 64 * WAVES >= (2 * MAX_DEPTH + 1) * W && LAYER_TILES == Staging::PER_LAYER * WAVES + 1,
-              "every scale has a thread, every tile a wave");
 struct Staged {
     const unsigned char *tiles;
     const float *scales;
@@ -370,7 +408,8 @@ struct Staged {
           natural(across_offset(p.lane, true)) {}
     TG_DEVICE f32x4 operator()(int tile) const { return unpack4(*reinterpret_cast<const u32x2 *>(tiles + tile * 512 + lane * 8)); }
     // the transposed operand, of a tile in feed order or (q, k, v) in the matrix's own
-    TG_DEVICE f32x4 turned_feed(int tile) const { return unpack4(read_across(tiles + tile * 512 + feed)); }
+    TG_DEVICE u32x2 turned_feed_row(int tile) const { return read_across(tiles + tile * 512 + feed); }
+    TG_DEVICE f32x4 turned_feed(int tile) const { return unpack4(turned_feed_row(tile)); }
     TG_DEVICE f32x4 turned_natural(int tile) const { return unpack4(read_across(tiles + tile * 512 + natural)); }
     TG_DEVICE f32x4 scale(int norm) const {
         const float *s = scales + norm * W + g;
@@ -444,32 +483,141 @@ struct Group {
     }
 };
 
+// ---- teams -------------------------------------------------------------------------------------------
+// A team's waves each hold the lanes of all its tokens.  Role 0 has what is one chain - norms, projections of sixteen outputs,
+// attention, residuals - and roles 1 to 3 sixteen of the 48 features of the MLP each, forward and backward; the head's 256 logits
+// are shared by all four.  A sum over features or logits is still one wave's chain of fmaf in their order, so a
+// result does not depend on the roles.  What one wave's work another needs goes through LDS, a tile at a time.
+// A lone wave (R = 1) has all of it.
+struct Exchange {
+    unsigned char *at, *quarters;
+    int lane, c;
+    TG_DEVICE Exchange(const Model &m, unsigned char *memory, const Lane &p, bool rows)
+        : at(memory + teams_at(m.depth, m.teams) + p.team * team_bytes(m.depth, rows)), quarters(memory + embedding_at(m.depth) + p.team * 4096),
+          lane(p.lane), c(p.c) {}
+    // the input of the MLP or of the head; the place of the last tile
+    TG_DEVICE u32x2 &row() const { return reinterpret_cast<u32x2 *>(at + 15 * 1024)[lane]; }
+    // activation; or the gradients of gate and up, and behind them the gradient that they come from; or the logits' gradients.  In
+    // 32 bits, so that who waits for them need not take them apart.
+    TG_DEVICE f32x4 &tile(int k) const { return reinterpret_cast<f32x4 *>(at)[k * 64 + lane]; }
+    TG_DEVICE float &high(int role) const { return reinterpret_cast<float *>(at + 16 * 1024)[role * W + c]; }
+    TG_DEVICE float &picked(int role) const { return reinterpret_cast<float *>(at + 16 * 1024 + ROLES * W * 4)[role * W + c]; }
+    TG_DEVICE f32x4 &quarter(int role) const { return reinterpret_cast<f32x4 *>(quarters)[role * 64 + lane]; }
+};
+// What the block's waves have written to LDS is there for all of them.  Each role comes here as often as the others.
+TG_DEVICE void meet() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+// The rows of a layer that the backward pass wants: in the team's LDS, or in memory.
+template <bool LDS> struct Rows {
+    unsigned char *at;
+    int64_t apart; // from one layer to the next
+    int lane, c;
+    TG_DEVICE Rows(const Model &m, unsigned char *memory, const Workspace &s, const Lane &p) : lane(p.lane), c(p.c) {
+        if constexpr (LDS)
+            at = memory + teams_at(m.depth, m.teams) + p.team * team_bytes(m.depth, true) + EXCHANGE_BYTES, apart = ROW_BYTES;
+        else
+            at = s.rows + size_t(p.wave) * LONE_ROW_BYTES, apart = int64_t(s.waves) * LONE_ROW_BYTES;
+    }
+    TG_DEVICE u32x2 &tile(int l, int k) const { return reinterpret_cast<u32x2 *>(at + l * apart)[k * 64 + lane]; }
+    TG_DEVICE u32x2 &features(int l, int k) const { return reinterpret_cast<u32x2 *>(at + l * apart + ROW_FEATURES)[k * 64 + lane]; }
+    TG_DEVICE float &word(int l, int k) const { return reinterpret_cast<float *>(at + l * apart + ROW_TILES * 512)[k * 64 + lane]; }
+    TG_DEVICE uint8_t &distance(int l) const { return (at + l * apart + ROW_DISTANCE)[lane]; }
+    TG_DEVICE float &inverse(int l, int k) const { return reinterpret_cast<float *>(at + l * apart + ROW_INVERSE)[k * W + c]; }
+};
+// A layer's, as they are wanted
+template <int R> struct LayerRows {
+    u32x2 x, query, key, value, middle, features[R == 1 ? 6 : 1];
+    float gate, slope, inv1, inv2;
+    int distance;
+    template <class Rows> TG_DEVICE void request(const Rows &rows, int l) {
+        if constexpr (R == 1)
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                features[k] = rows.features(l, k);
+        x = rows.tile(l, R_X), query = rows.tile(l, R_Q), key = rows.tile(l, R_KEY), value = rows.tile(l, R_VALUE);
+        middle = rows.tile(l, R_MIDDLE), gate = rows.word(l, R_GATE), slope = rows.word(l, R_SLOPE);
+        inv1 = rows.inverse(l, 0), inv2 = rows.inverse(l, 1), distance = rows.distance(l);
+    }
+};
+// A row for the launch of the weight gradients, written through to memory: what the L2s hold of a launch's results is written back
+// behind its last block, and this one leaves 28 MB of such rows at depth 4, 10240 tokens (63.0 us a step, 59.8 so).
+TG_DEVICE void leave(u32x2 &to, const u32x2 &v) {
+    __hip_atomic_store(reinterpret_cast<uint64_t *>(&to), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+TG_DEVICE u32x2 *operands_of(const Workspace &s, const Lane &p, int l) {
+    return s.tiles + (size_t(l) * s.waves + p.wave) * OPERANDS * 64 + p.lane;
+}
+
 // ---- forward ---------------------------------------------------------------------------------------
-// What the head leaves for the backward pass; the logits' gradients in tiles of sixteen.
+// What role 0 keeps of the head for the backward pass.
 struct Head {
-    u32x2 dlogits[16], hidden;
+    u32x2 hidden;
     float inverse;
 };
 TG_DEVICE f32x4 embedding_row(const Model &m, const unsigned char *memory, const Lane &p, int token) {
     const bf16_t *row = reinterpret_cast<const bf16_t *>(memory + embedding_at(m.depth)) + token * W + p.g;
     return p.live ? f32x4{bf16_to_float(row[0]), bf16_to_float(row[4]), bf16_to_float(row[8]), bf16_to_float(row[12])} : ZERO;
 }
-// cuda/model.cuh:8-59.  dlogits = RN_bf16((p - onehot) / tokens).  GRADIENT: rows are kept in `s` and the head's in `head`.
-template <bool GRADIENT, int CONTEXT>
-TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight, const Workspace &s, f32x4 h, int target, float rc,
-                            float rs, float *__restrict__ token_losses, float *__restrict__ logits_out, Head &head) {
+// Sixteen features of the packed gate|up projection and of SwiGLU (cuda/model.cuh:22-29, cuda/ops.cuh:120-131: RN after SiLU and after
+// the product).  Roles 1 to 3 keep gate, up and the sigmoid of a layer in registers for the backward pass.
+struct Features {
+    u32x2 gate, up;
+    f32x4 sigmoid;
+    TG_DEVICE u32x2 activation() const { return pack4(rounded(unpack4(gate) * sigmoid) * unpack4(up)); }
+};
+TG_DEVICE f32x4 sigmoids(const u32x2 &gate) {
+    f32x4 v = unpack4(gate);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        v[r] = sigmoid(v[r]);
+    return v;
+}
+struct GateUp {
+    f32x4 of_both[2];
+    TG_DEVICE GateUp(const Staged &weight, int l, int t) : of_both{weight(l * LAYER_TILES + 4 + t), weight(l * LAYER_TILES + 7 + t)} {}
+    TG_DEVICE Features operator()(const f32x4 &row) {
+        f32x4 both[2];
+        multiply_all(of_both, row, both);
+        const u32x2 gate = pack4(both[0]);
+        return {gate, pack4(both[1]), sigmoids(gate)};
+    }
+};
+// Down projection and SwiGLU backward (cuda/model.cuh:72-80, cuda/ops.cuh:133-144) of sixteen features: what does not wait for the
+// gradient, and the gradients of gate and up
+struct FeaturesBackward {
+    f32x4 down, up, sig, silu, slope;
+    TG_DEVICE FeaturesBackward(const Staged &weight, int l, int t, const Features &f)
+        : down(weight.turned_feed(l * LAYER_TILES + 10 + t)), up(unpack4(f.up)), sig(f.sigmoid) {
+        const f32x4 gate = unpack4(f.gate);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            silu[r] = gate[r] * sig[r];
+            slope[r] = fmaf(gate[r], 1.f - sig[r], 1.f);
+        }
+        silu = rounded(silu);
+    }
+    TG_DEVICE void operator()(const f32x4 &dh, u32x2 &dgate, u32x2 &dup) const {
+        const f32x4 dy = rounded(multiply(down, dh)), da = rounded(dy * up);
+        dgate = pack4(da * sig * slope), dup = pack4(dy * silu);
+    }
+};
+// The layers, role 0 (cuda/model.cuh:8-31).  GRADIENT: rows are kept.  h: the embedding's rows, and then the last layer's.
+template <int R, bool GRADIENT, int CONTEXT, class Rows>
+TG_DEVICE void forward_chain(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Rows &rows, const Workspace &s,
+                             f32x4 &h, float rc, float rs) {
     const int context = CONTEXT ? CONTEXT : m.context;
     for (int l = 0; l < m.depth; ++l) {
         const int tile = l * LAYER_TILES;
-        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
-        float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
         // QKV projection, RoPE (cuda/model.cuh:14-19)
+        f32x4 of_qkv[3] = {weight(tile), weight(tile + 1), weight(tile + 2)};
         const float inv1 = inverse_rms(h, p);
         const u32x2 n1 = normalize(h, inv1, weight.scale(2 * l));
-        const f32x4 n1f = unpack4(n1);
-        const f32x4 query = rounded(rotate(rounded(multiply(weight(tile), n1f)), rc, rs));
-        const u32x2 key = pack4(rotate(rounded(multiply(weight(tile + 1), n1f)), rc, rs));
-        const u32x2 value = pack4(multiply(weight(tile + 2), n1f));
+        f32x4 qkv[3];
+        multiply_all(of_qkv, unpack4(n1), qkv);
+        const f32x4 query = rounded(rotate(rounded(qkv[0]), rc, rs));
+        const u32x2 key = pack4(rotate(rounded(qkv[1]), rc, rs));
+        const u32x2 value = pack4(qkv[2]);
         // arg-max attention with its GELU gate (cuda/attention.cuh:33-71); keys in order, the first one wins ties
         float top = -INFINITY;
         int distance = 0;
@@ -497,197 +645,273 @@ TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight,
         const f32x4 middle = rounded(rounded(multiply(weight(tile + 3), a)) + h);
         const float inv2 = inverse_rms(middle, p);
         const u32x2 n2 = normalize(middle, inv2, weight.scale(2 * l + 1));
-        if constexpr (GRADIENT) {
-            keep[T_X * 64] = pack4(h);
-            keep[T_N1 * 64] = n1;
-            keep[T_Q * 64] = pack4(query);
-            keep[T_KEY * 64] = best_key;
-            keep[T_VALUE * 64] = best_value;
-            keep[T_A * 64] = pack4(a);
-            keep[T_MIDDLE * 64] = pack4(middle);
-            keep[T_N2 * 64] = n2;
-            words[WORD_GATE * 64] = gate;
-            words[WORD_SLOPE * 64] = fmaf(top * 0.3989422804014327f, expf(-0.5f * top * top), 0.5f * e);
-            words[WORD_DISTANCE * 64] = __int_as_float(distance);
-            words[WORD_INV1 * 64] = inv1;
-            words[WORD_INV2 * 64] = inv2;
+        u32x2 *operand = operands_of(s, p, l);
+        const auto keep = [&] {
+            if constexpr (GRADIENT) {
+                rows.tile(l, R_X) = pack4(h);
+                rows.tile(l, R_Q) = pack4(query);
+                rows.tile(l, R_KEY) = best_key;
+                rows.tile(l, R_VALUE) = best_value;
+                rows.tile(l, R_MIDDLE) = pack4(middle);
+                rows.word(l, R_GATE) = gate;
+                rows.word(l, R_SLOPE) = fmaf(top * 0.3989422804014327f, expf(-0.5f * top * top), 0.5f * e);
+                rows.distance(l) = uint8_t(distance);
+                rows.inverse(l, 0) = inv1, rows.inverse(l, 1) = inv2;
+                leave(operand[T_N1 * 64], n1);
+                leave(operand[T_A * 64], pack4(a));
+                leave(operand[T_N2 * 64], n2);
+            }
+        };
+        f32x4 act[3], down[3];
+        if constexpr (R == 1) {
+            keep();
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                const Features f = GateUp(weight, l, t)(unpack4(n2));
+                const u32x2 act_row = f.activation();
+                act[t] = unpack4(act_row), down[t] = weight(tile + 10 + t);
+                if constexpr (GRADIENT) {
+                    rows.features(l, t) = f.gate, rows.features(l, 3 + t) = f.up;
+                    leave(operand[(T_ACT + t) * 64], act_row);
+                }
+            }
+        } else {
+            x.row() = n2;
+            meet(); // the MLP's features are worked on
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                down[t] = weight(tile + 10 + t);
+            keep();
+            ready(down[0], down[1], down[2]);
+            meet();
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                act[t] = x.tile(t);
         }
-        // packed gate|up projection, SwiGLU (RN after SiLU and after the product), down projection and residual
-        // (cuda/model.cuh:22-30, cuda/ops.cuh:120-131)
-        const f32x4 n2f = unpack4(n2);
+        // down projection and residual (cuda/model.cuh:30)
         f32x4 out = ZERO;
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const u32x2 gate_row = pack4(multiply(weight(tile + 4 + t), n2f)), up_row = pack4(multiply(weight(tile + 7 + t), n2f));
-            f32x4 act = unpack4(gate_row);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                act[r] = act[r] * sigmoid(act[r]);
-            const u32x2 act_row = pack4(rounded(act) * unpack4(up_row));
-            out = multiply(weight(tile + 10 + t), unpack4(act_row), out);
-            if constexpr (GRADIENT) {
-                keep[(T_GU + t) * 64] = gate_row;
-                keep[(T_GU + 3 + t) * 64] = up_row;
-                keep[(T_ACT + t) * 64] = act_row;
-            }
-        }
+        for (int t = 0; t < 3; ++t)
+            out = multiply(down[t], act[t], out);
         h = rounded(rounded(out) + middle);
     }
-    // final RMSNorm, head, softmax cross-entropy (cuda/model.cuh:32-58): register r of tile t is logit 16 t + 4 r + g
-    const float inv = inverse_rms(h, p);
-    const u32x2 nf = normalize(h, inv, weight.scale(2 * m.depth));
-    const f32x4 nff = unpack4(nf);
-    f32x4 logit[16];
+}
+template <bool GRADIENT>
+TG_DEVICE void forward_features(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Workspace &s,
+                                Features (&kept)[MAX_DEPTH]) {
+    const int t = p.role - 1;
+    u32x2 *operand = operands_of(s, p, 0) + (T_ACT + t) * 64;
+#pragma unroll
+    for (int l = 0; l < MAX_DEPTH; ++l) {
+        if (l >= m.depth)
+            break;
+        GateUp project(weight, l, t);
+        ready(project.of_both[0], project.of_both[1]);
+        meet();
+        kept[l] = project(unpack4(x.row()));
+        const u32x2 act_row = kept[l].activation();
+        x.tile(t) = unpack4(act_row);
+        meet();
+        if constexpr (GRADIENT)
+            leave(operand[size_t(l) * s.waves * (OPERANDS * 64)], act_row);
+    }
+}
+// cuda/model.cuh:8-59, all roles.  dlogits = RN_bf16((p - onehot) / tokens), left in memory and in LDS or, by a lone wave, in `head`.
+template <int R> struct Kept {
+    Features of_role[MAX_DEPTH];
+};
+template <> struct Kept<1> {
+    u32x2 dlogits[HEAD_TILES];
+};
+template <int R, bool GRADIENT, int CONTEXT, class Rows>
+TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Rows &rows, const Workspace &s,
+                            f32x4 h, int target, float rc, float rs, float *__restrict__ token_losses, float *__restrict__ logits_out,
+                            Head &head, Kept<R> &kept) {
+    constexpr int TILES = HEAD_TILES / R;
+    u32x2 nf;
+    if (R == 1 || p.role == 0) {
+        forward_chain<R, GRADIENT, CONTEXT>(m, p, weight, x, rows, s, h, rc, rs);
+        // final RMSNorm (cuda/model.cuh:32-34)
+        const float inv = inverse_rms(h, p);
+        nf = normalize(h, inv, weight.scale(2 * m.depth));
+        if constexpr (R > 1)
+            x.row() = nf;
+        if constexpr (GRADIENT) {
+            head.hidden = pack4(h), head.inverse = inv;
+            s.nf[size_t(p.wave) * 64 + p.lane] = nf;
+        }
+    } else if constexpr (R > 1)
+        forward_features<GRADIENT>(m, p, weight, x, s, kept.of_role);
+    // head, softmax cross-entropy (cuda/model.cuh:35-58): this role's tile i is the head's tile role + R i, whose register r is
+    // logit 16 (role + R i) + 4 r + g
+    f32x4 logit[TILES];
+    if constexpr (R > 1) {
+        f32x4 of_head[TILES];
+#pragma unroll
+        for (int i = 0; i < TILES; ++i)
+            of_head[i] = weight(weight.head + p.role + R * i), ready(of_head[i]);
+        meet();
+        multiply_all(of_head, unpack4(x.row()), logit);
+    } else
+#pragma unroll
+        for (int i = 0; i < TILES; ++i)
+            logit[i] = multiply(weight(weight.head + i), unpack4(nf));
     float high = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        logit[t] = rounded(multiply(weight(weight.head + t), nff));
-        high = fmaxf(fmaxf(high, fmaxf(logit[t][0], logit[t][1])), fmaxf(logit[t][2], logit[t][3]));
+    for (int i = 0; i < TILES; ++i) {
+        logit[i] = rounded(logit[i]);
+        high = fmaxf(fmaxf(high, fmaxf(logit[i][0], logit[i][1])), fmaxf(logit[i][2], logit[i][3]));
     }
     high = token_max(high);
+    if constexpr (R > 1) {
+        x.high(p.role) = high;
+        meet();
+        high = fmaxf(fmaxf(x.high(0), x.high(1)), fmaxf(x.high(2), x.high(3)));
+    }
     if (logits_out && p.live)
 #pragma unroll
-        for (int t = 0; t < 16; ++t)
+        for (int i = 0; i < TILES; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                logits_out[size_t(p.token) * V + t * 16 + 4 * r + p.g] = logit[t][r];
-    // the target's logit: tile target / 16, register target / 4 % 4 of the lane g = target % 4, by halves
-    float of_four[16];
+                logits_out[size_t(p.token) * V + (p.role + R * i) * 16 + 4 * r + p.g] = logit[i][r];
+    // the target's logit: register target / 4 % 4 of tile target / 16, of the lane g = target % 4
+    const bool holder = p.g == (target & 3) && p.role == (target >> 4) % R;
+    float picked = 0.f;
+    const int mine = holder ? (target >> 4) / R * 4 + ((target >> 2) & 3) : -1; // 4 i + r
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        const float even = target & 4 ? logit[t][1] : logit[t][0], odd = target & 4 ? logit[t][3] : logit[t][2];
-        of_four[t] = target & 8 ? odd : even;
-    }
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-    for (int bit = 0; bit < 4; ++bit)
-#pragma unroll
-        for (int t = 0; t < 8 >> bit; ++t)
-            of_four[t] = target & (16 << bit) ? of_four[2 * t + 1] : of_four[2 * t];
-    const bool holder = p.g == (target & 3);
-    float picked = holder ? of_four[0] : 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            logit[t][r] = expf(logit[t][r] - high);
+        for (int r = 0; r < 4; ++r) {
+            picked = 4 * i + r == mine ? logit[i][r] : picked;
+            logit[i][r] = expf(logit[i][r] - high);
+        }
+    picked = swap_add_16(swap_add_32(picked));
     // the sum's tree: every 64th logit in order, then halves of what is left (bits 5 .. 0 of the logit's number)
     f32x4 quarter[4];
+    if constexpr (R > 1) {
+        x.quarter(p.role) = ((logit[0] + logit[1]) + logit[2]) + logit[3];
+        x.picked(p.role) = picked;
+        meet();
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        quarter[q] = ((logit[q] + logit[q + 4]) + logit[q + 8]) + logit[q + 12];
+        for (int q = 0; q < 4; ++q)
+            quarter[q] = x.quarter(q);
+        picked = ((x.picked(0) + x.picked(1)) + x.picked(2)) + x.picked(3);
+    } else
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            quarter[q] = ((logit[q] + logit[q + 4]) + logit[q + 8]) + logit[q + 12];
     const f32x4 sixteenth = (quarter[0] + quarter[2]) + (quarter[1] + quarter[3]);
     const float sum = swap_add_16(swap_add_32((sixteenth[0] + sixteenth[2]) + (sixteenth[1] + sixteenth[3])));
-    picked = swap_add_16(swap_add_32(picked));
-    if (p.live && p.g == 0)
+    if (p.role == 0 && p.live && p.g == 0)
         token_losses[p.token] = high + logf(sum) - picked;
     if constexpr (GRADIENT) {
-        head.hidden = pack4(h), head.inverse = inv;
-        s.nf[size_t(p.wave) * 64 + p.lane] = nf;
         const float share = reciprocal(sum), tokens = float(m.tokens), per_token = 1.f / tokens;
-        const int mine = holder ? target >> 2 : -1; // 4 t + r
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
+        for (int i = 0; i < TILES; ++i) {
             f32x4 d;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                d[r] = divide(divide(logit[t][r], sum, share) - (4 * t + r == mine ? 1.f : 0.f), tokens, per_token);
-            const u32x2 packed = pack4(d);
-            head.dlogits[t].x = p.live ? packed.x : 0, head.dlogits[t].y = p.live ? packed.y : 0;
-            s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane] = head.dlogits[t];
+                d[r] = divide(divide(logit[i][r], sum, share) - (4 * i + r == mine ? 1.f : 0.f), tokens, per_token);
+            u32x2 packed = pack4(d);
+            packed.x = p.live ? packed.x : 0, packed.y = p.live ? packed.y : 0;
+            if constexpr (R > 1)
+                x.tile(p.role + R * i) = unpack4(packed);
+            else
+                kept.dlogits[i] = packed;
+            leave(s.dlogits[(size_t(p.wave) * 16 + p.role + R * i) * 64 + p.lane], packed);
         }
     }
 }
 
 // ---- backward --------------------------------------------------------------------------------------
-// cuda/model.cuh:61-99, without the weight gradients
-template <int CONTEXT>
-TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight, const Workspace &s, float rc, float rs,
-                             const Head &head) {
+// cuda/model.cuh:61-99, without the weight gradients.  Role 0:
+template <int R, int CONTEXT, class Rows>
+TG_DEVICE void backward_chain(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Rows &rows, const Workspace &s,
+                              float rc, float rs, const Head &head, const Kept<R> &kept) {
     const int context = CONTEXT ? CONTEXT : m.context;
     auto gz = [&](int norm) { return s.gz + ((size_t(norm) * s.waves + p.wave) * 16 + p.c) * W + p.g; };
 
-    // a layer's rows are requested while the layer above is worked on
-    struct Rows {
-        u32x2 x, query, key, value, middle, gate[3], up[3];
-        float gate_of_top, slope, inv1, inv2;
-        int distance;
-    };
-    auto request = [&](int l, Rows &r) {
-        const u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
-        const float *words = s.words + (size_t(l) * s.waves + p.wave) * WORDS * 64 + p.lane;
-#pragma unroll
-        for (int t = 0; t < 3; ++t)
-            r.gate[t] = keep[(T_GU + t) * 64], r.up[t] = keep[(T_GU + 3 + t) * 64];
-        r.middle = keep[T_MIDDLE * 64], r.query = keep[T_Q * 64], r.key = keep[T_KEY * 64], r.value = keep[T_VALUE * 64];
-        r.x = keep[T_X * 64];
-        r.gate_of_top = words[WORD_GATE * 64], r.slope = words[WORD_SLOPE * 64], r.inv1 = words[WORD_INV1 * 64];
-        r.inv2 = words[WORD_INV2 * 64], r.distance = __float_as_int(words[WORD_DISTANCE * 64]);
-    };
-
     // head input gradient and final RMSNorm backward (cuda/model.cuh:63-66)
-    Rows next;
-    request(m.depth - 1, next);
     f32x4 dn = ZERO;
+    LayerRows<R> next; // a lone wave's are requested while the layer above is worked on
+    if constexpr (R == 1) {
+        next.request(rows, m.depth - 1);
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
-        dn = multiply(weight.turned_feed(weight.head + t), unpack4(head.dlogits[t]), dn);
+        for (int t = 0; t < 16; ++t)
+            dn = multiply(weight.turned_feed(weight.head + t), unpack4(kept.dlogits[t]), dn);
+    } else {
+        u32x2 of_head[16];
+        f32x4 dlogits[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            of_head[t] = weight.turned_feed_row(weight.head + t), dlogits[t] = x.tile(t);
+        __builtin_amdgcn_sched_barrier(0); // every read goes out before the first product
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            dn = multiply(unpack4(of_head[t]), dlogits[t], dn);
+    }
     f32x4 dh = normalize_backward(unpack4(head.hidden), head.inverse, rounded(dn), weight.scale(2 * m.depth), gz(2 * m.depth), p);
     for (int l = m.depth - 1; l >= 0; --l) {
         const int tile = l * LAYER_TILES;
-        u32x2 *keep = s.tiles + (size_t(l) * s.waves + p.wave) * TILES * 64 + p.lane;
-        const Rows rows = next;
-        if (l)
-            request(l - 1, next);
-        // down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88, cuda/ops.cuh:133-144)
-        keep[T_DH_DOWN * 64] = pack4(dh);
-        f32x4 dgate[3], dup[3];
+        u32x2 *operand = operands_of(s, p, l);
+        LayerRows<R> of;
+        // down projection, SwiGLU, packed gate|up projection and RMSNorm backward (cuda/model.cuh:72-88)
+        if constexpr (R == 1) {
+            of = next;
+            if (l)
+                next.request(rows, l - 1);
+            leave(operand[T_DH_DOWN * 64], pack4(dh));
+            u32x2 gradient[6];
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const f32x4 gate = unpack4(rows.gate[t]), up = unpack4(rows.up[t]);
-            const f32x4 dy = rounded(multiply(weight.turned_feed(tile + 10 + t), dh)), da = rounded(dy * up);
-            f32x4 silu;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float g = gate[r], sig = sigmoid(g);
-                silu[r] = g * sig;
-                dgate[t][r] = da[r] * sig * fmaf(g, 1.f - sig, 1.f);
+            for (int t = 0; t < 3; ++t) {
+                FeaturesBackward(weight, l, t, {of.features[t], of.features[3 + t], sigmoids(of.features[t])})(dh, gradient[t], gradient[3 + t]);
+                leave(operand[(T_DGU + t) * 64], gradient[t]);
+                leave(operand[(T_DGU + 3 + t) * 64], gradient[3 + t]);
             }
-            const u32x2 dgate_row = pack4(dgate[t]), dup_row = pack4(dy * rounded(silu));
-            keep[(T_DGU + t) * 64] = dgate_row;
-            keep[(T_DGU + 3 + t) * 64] = dup_row;
-            dgate[t] = unpack4(dgate_row), dup[t] = unpack4(dup_row);
+            dn = ZERO;
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+                dn = multiply(weight.turned_feed(tile + 4 + t), unpack4(gradient[t]), dn);
+        } else {
+            x.tile(6) = dh;
+            meet();
+            leave(operand[T_DH_DOWN * 64], pack4(dh));
+            f32x4 gate_up[6];
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+                gate_up[t] = weight.turned_feed(tile + 4 + t);
+            of.request(rows, l);
+            ready(gate_up[0], gate_up[1], gate_up[2], gate_up[3], gate_up[4], gate_up[5]);
+            meet();
+            dn = ZERO;
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+                dn = multiply(gate_up[t], x.tile(t), dn);
         }
-        dn = ZERO;
-#pragma unroll
-        for (int t = 0; t < 3; ++t)
-            dn = multiply(weight.turned_feed(tile + 4 + t), dgate[t], dn);
-#pragma unroll
-        for (int t = 0; t < 3; ++t)
-            dn = multiply(weight.turned_feed(tile + 7 + t), dup[t], dn);
+        const f32x4 key = unpack4(of.key), value = unpack4(of.value);
+        const u32x2 query = of.query;
+        const float gate = of.gate;
         // residual gradients stay bf16 between operators (cuda/ops.cuh:74-76)
-        dh = rounded(dh + normalize_backward(unpack4(rows.middle), rows.inv2, rounded(dn), weight.scale(2 * l + 1), gz(2 * l + 1), p));
-        keep[T_DH_ATTENTION * 64] = pack4(dh);
+        dh = rounded(dh + normalize_backward(unpack4(of.middle), of.inv2, rounded(dn), weight.scale(2 * l + 1), gz(2 * l + 1), p));
+        leave(operand[T_DH_ATTENTION * 64], pack4(dh));
 
         // attention: output projection backward, the score gradient of the cached winner, query / key / value gradients
         // gathered over the sequence, inverse RoPE, QKV projection and RMSNorm backward (cuda/model.cuh:89-96,
         // cuda/attention.cuh:72-106)
-        const u32x2 query = rows.query;
-        const f32x4 key = unpack4(rows.key), value = unpack4(rows.value);
-        const float gate = rows.gate_of_top;
         const u32x2 dattn = pack4(multiply(weight(weight.turned_attention + l), dh));
         const f32x4 da = unpack4(dattn);
         float dt = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             dt = fmaf(da[c], value[c], dt);
-        dt *= rows.slope;
+        dt *= of.slope;
         f32x4 dk = ZERO, dv = ZERO;
         up_to<0, CONTEXT ? CONTEXT - 1 : 7>([&](auto step) { // queries of this token's sequence that chose it, in order
             constexpr int D = decltype(step)::value;
             if (D >= context)
                 return;
             // every lane takes part in the shifts, so none of them may sit behind a condition
-            const uint32_t theirs = later<D>(uint32_t(rows.distance));
+            const uint32_t theirs = later<D>(uint32_t(of.distance));
             const float their_dt = __uint_as_float(later<D>(__float_as_uint(dt))), their_gate = __uint_as_float(later<D>(__float_as_uint(gate)));
             const f32x4 qf = unpack4(u32x2{later<D>(query.x), later<D>(query.y)});
             const f32x4 df = unpack4(u32x2{later<D>(dattn.x), later<D>(dattn.y)});
@@ -703,71 +927,113 @@ TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight
         const f32x4 dq = turned(rounded(rotate_back(rounded(key * dt), rc, rs)));
         dk = turned(rounded(rotate_back(rounded(dk), rc, rs)));
         dv = turned(rounded(dv));
-        keep[T_DQKV * 64] = pack4(dq);
-        keep[(T_DQKV + 1) * 64] = pack4(dk);
-        keep[(T_DQKV + 2) * 64] = pack4(dv);
+        leave(operand[T_DQKV * 64], pack4(dq));
+        leave(operand[(T_DQKV + 1) * 64], pack4(dk));
+        leave(operand[(T_DQKV + 2) * 64], pack4(dv));
         dn = multiply(weight.turned_natural(tile + 2), dv,
                       multiply(weight.turned_natural(tile + 1), dk, multiply(weight.turned_natural(tile), dq)));
-        dh = rounded(dh + normalize_backward(unpack4(rows.x), rows.inv1, rounded(dn), weight.scale(2 * l), gz(2 * l), p));
+        dh = rounded(dh + normalize_backward(unpack4(of.x), of.inv1, rounded(dn), weight.scale(2 * l), gz(2 * l), p));
     }
     s.dh[size_t(p.wave) * 64 + p.lane] = pack4(dh);
+}
+TG_DEVICE void backward_features(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Workspace &s,
+                                 const Features (&kept)[MAX_DEPTH]) {
+    const int t = p.role - 1;
+#pragma unroll
+    for (int l = MAX_DEPTH - 1; l >= 0; --l) {
+        if (l >= m.depth)
+            continue;
+        FeaturesBackward backward(weight, l, t, kept[l]);
+        ready(backward.down, backward.up, backward.silu, backward.slope);
+        u32x2 dgate, dup;
+        meet();
+        backward(x.tile(6), dgate, dup);
+        x.tile(t) = unpack4(dgate);
+        x.tile(3 + t) = unpack4(dup);
+        meet();
+        u32x2 *operand = operands_of(s, p, l);
+        leave(operand[(T_DGU + t) * 64], dgate);
+        leave(operand[(T_DGU + 3 + t) * 64], dup);
+    }
+}
+template <int R, int CONTEXT, class Rows>
+TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight, const Exchange &x, const Rows &rows, const Workspace &s,
+                             float rc, float rs, const Head &head, const Kept<R> &kept) {
+    if constexpr (R > 1)
+        meet(); // the logits' gradients
+    if (R == 1 || p.role == 0)
+        backward_chain<R, CONTEXT>(m, p, weight, x, rows, s, rc, rs, head, kept);
+    else if constexpr (R > 1)
+        backward_features(m, p, weight, x, s, kept.of_role);
 }
 
 // ---- kernels -----------------------------------------------------------------------------------------
 template <bool GRADIENT>
-__global__ __launch_bounds__(64 * WAVES) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
-                                                               Workspace s, float *__restrict__ token_losses,
-                                                               float *__restrict__ logits_out) {
+__global__ __launch_bounds__(64 * block_waves(ROLES)) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
+                                                                             Workspace s, float *__restrict__ token_losses,
+                                                                             float *__restrict__ logits_out) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of(m);
+    const Lane p = lane_of(m, s.waves);
     const Staged weight(m, memory, p);
-    Staging staging(m, memory);
+    Staging<> staging(m, memory);
     const int token = p.live ? x[p.token] : 0, target = p.live ? y[p.token] : 0;
     staging.request();
     staging.request_embedding(!(reinterpret_cast<uintptr_t>(m.hi) & 15));
     staging.finish(false);
+    if (!staging.stays())
+        return;
     const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
     rotation(p.position, rc, rs);
     Head head;
-    forward_pass<GRADIENT, 0>(m, p, weight, s, h, target, rc, rs, token_losses, logits_out, head);
-    if constexpr (GRADIENT) {
-        const size_t here = size_t(p.wave) * 64 + p.lane;
-        s.hidden[here] = head.hidden, s.inverse[here] = head.inverse;
-    }
+    Kept<ROLES> kept;
+    forward_pass<ROLES, GRADIENT, 0>(m, p, weight, Exchange(m, memory, p, false), Rows<false>(m, memory, s, p), s, h, target, rc, rs, token_losses,
+                              logits_out, head, kept);
+    if constexpr (GRADIENT)
+        if (p.role == 0) {
+            const size_t here = size_t(p.wave) * 64 + p.lane;
+            s.hidden[here] = head.hidden, s.inverse[here] = head.inverse;
+        }
 }
-__global__ __launch_bounds__(64 * WAVES) void w16_backward_kernel(Model m, Workspace s) {
+__global__ __launch_bounds__(64 * block_waves(ROLES)) void w16_backward_kernel(Model m, Workspace s) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of(m);
+    const Lane p = lane_of(m, s.waves);
     const Staged weight(m, memory, p);
-    Staging staging(m, memory);
+    const Exchange exchange(m, memory, p, false);
+    Staging<> staging(m, memory);
     staging.request();
-    Head head;
     const size_t here = size_t(p.wave) * 64 + p.lane;
-    head.hidden = s.hidden[here], head.inverse = s.inverse[here];
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-        head.dlogits[t] = s.dlogits[(size_t(p.wave) * 16 + t) * 64 + p.lane];
+    const Head head = {s.hidden[here], s.inverse[here]};
     staging.finish(true);
+    if (!staging.stays())
+        return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        exchange.tile(p.role + 4 * i) = unpack4(s.dlogits[(size_t(p.wave) * 16 + p.role + 4 * i) * 64 + p.lane]);
     float rc, rs;
     rotation(p.position, rc, rs);
-    backward_pass<0>(m, p, weight, s, rc, rs, head);
+    const Rows<false> rows(m, memory, s, p);
+    Kept<ROLES> kept;
+    if (p.role)
+#pragma unroll
+        for (int l = 0; l < MAX_DEPTH; ++l)
+            if (l < m.depth)
+                kept.of_role[l] = GateUp(weight, l, p.role - 1)(unpack4(normalize(unpack4(rows.tile(l, R_MIDDLE)), rows.inverse(l, 1), weight.scale(2 * l + 1))));
+    backward_pass<ROLES, 0>(m, p, weight, exchange, rows, s, rc, rs, head, kept);
 }
-// A training step's both passes: a wave's backward pass reads only what its own forward pass kept, so the two are one launch
-// and the weights are staged once.  Depth 4, 2560 sequences of 4: 53.0 us as two launches that staged eight tiles at a time,
-// 38.8 so; depth 8, 16 of 8: 79.3 and 62.6.  Two waves a SIMD, which batches of more than 256 blocks need (10000 of 8 at depth 8
-// 498 us a step in two launches, 544 with 270 registers, 454 so).  Tokens and targets come straight out of the training
+// A training step's both passes: a team's backward pass reads only what its own forward pass kept, so the two are one launch
+// and the weights are staged once.  us a launch, all on lone waves and so: depth 4, 2560 sequences of 4 38.6 and 31.5; depth 8, four
+// batches of 16 of 8 64 and 41.  Of the 31.5 the weights take 2, a layer 2.5 forward and 2.6 back, the head 5.5.  Tokens and targets come straight out of the training
 // bytes, every sequence a window at a hashed place (cuda/dataset.cuh:13-27); the tokens are left for the embedding's gradient.
-template <int CONTEXT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void w16_step_kernel(
-    Model m, W16Data data, uint64_t inverse, Workspace first, Group group) {
+template <int CONTEXT, int R, bool ROWS>
+__global__ __launch_bounds__(64 * block_waves(R)) void w16_step_kernel(Model m, W16Data data, uint64_t inverse, Workspace first, Group group) {
     extern __shared__ __align__(16) unsigned char memory[];
     const W16Batch &batch = group.member[blockIdx.y];
     const Workspace s = group.workspace(first, blockIdx.y);
     m.hi = batch.weights.hi, m.lo = batch.weights.lo;
-    const Lane p = lane_of(m);
+    const Lane p = lane_of<R>(m, s.waves);
     const Staged weight(m, memory, p);
-    Staging staging(m, memory);
+    Staging<R> staging(m, memory);
     int token = 0, target = 0;
     if (p.live) {
         const int sequence = p.token / CONTEXT;
@@ -782,15 +1048,21 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     }
     staging.request();
     staging.request_embedding();
-    staging.finish(true);
-    if (p.live && p.g == 0)
-        batch.tokens[p.token] = uint8_t(token);
-    const f32x4 h = embedding_row(m, memory, p, token);
     float rc, rs;
     rotation(p.position, rc, rs);
+    ready(rc, rs);
+    staging.finish(true);
+    if (!staging.stays())
+        return;
+    if (p.live && p.g == 0 && p.role == 0)
+        batch.tokens[p.token] = uint8_t(token);
+    const f32x4 h = embedding_row(m, memory, p, token);
+    const Exchange exchange(m, memory, p, ROWS);
+    const Rows<ROWS> rows(m, memory, s, p);
     Head head;
-    forward_pass<true, CONTEXT>(m, p, weight, s, h, target, rc, rs, batch.token_losses, nullptr, head);
-    backward_pass<CONTEXT>(m, p, weight, s, rc, rs, head);
+    Kept<R> kept;
+    forward_pass<R, true, CONTEXT>(m, p, weight, exchange, rows, s, h, target, rc, rs, batch.token_losses, nullptr, head, kept);
+    backward_pass<R, CONTEXT>(m, p, weight, exchange, rows, s, rc, rs, head, kept);
 }
 
 // ---- weight gradients ------------------------------------------------------------------------------
@@ -798,9 +1070,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 // rows come to LDS as the waves kept them; the transposing load then gives lane 16 q + i feature 4 (i % 4) + i / 4 of tokens
 // 4 j + q, an operand of the fp32 instruction whose steps run over the tokens.  That moves data and computes nothing: an
 // infinity stays in its own feature.  A wave has three or four tiles of the gradient at a time, whose chains of dependent
-// instructions fill the matrix pipe, which bounds the kernel together with what the rows take on their way (half of them
-// are worked on while the others come): 93 tiles of 32 instructions a chunk at depth 4.  2560 sequences of 4 there: 15.3 us
-// with a wave for each tile that loaded its rows and turned them with the identity matrix, 13.1 so; 16 of 8 at depth 8 7.7 and 7.9.
+// instructions fill the matrix pipe, which bounds the kernel together with what the rows take on their way (a team's are
+// worked on while the next ones' come): 93 tiles of 32 instructions a chunk at depth 4, and 28 MB of rows.  2560 sequences of 4 there: 15.3 us
+// with a wave for each tile that loaded its rows and turned them with the identity matrix, 13.1 with every half of a chunk waited
+// for, 12.5 so; four batches of 16 of 8 at depth 8 11.1 and 10.2.
 // Half a chunk, as the last one or the only one may be, is all that is worked on: 16 sequences of 4 at depth 4 6.4 us with the
 // missing half as zeros, 4.6 so.
 constexpr int HEAD_ROWS = 17; // the head's tiles of a wave in LDS: dlogits, and the normalised rows
@@ -824,28 +1097,34 @@ struct ScaleTerms {
             for (int j = 0; j < 4; ++j)
                 v[w][j] = w < waves ? gz[(w * 4 + j) * 64] : 0.f;
     }
-};
-// TILES chains of products over the tokens of half a chunk's waves, and with SCALE one of a row of ones times the terms.
-// `rows` and `columns`: this lane's place in the first wave's tiles; a wave's are `stride` (columns: `column_stride`) bytes.
-template <int TILES, bool SCALE>
-TG_DEVICE void add_half(f32x4 (&sum)[4], const unsigned char *const (&rows)[TILES], const unsigned char *const (&columns)[TILES], int stride,
-                        int column_stride, const ScaleTerms &terms, int half) {
+    // a row of ones times the terms; lane c of the first sixteen has feature c
+    TG_DEVICE float sum() const {
+        f32x4 scale = ZERO;
 #pragma unroll
-    for (int k = 0; k < CHUNK_WAVES / 2; ++k) {
-        const int w = half * (CHUNK_WAVES / 2) + k;
-        f32x4 a[TILES], b[TILES];
+        for (int w = 0; w < CHUNK_WAVES; ++w)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                scale = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, v[w][j], scale, 0, 0, 0);
+        return scale[0];
+    }
+};
+// TILES chains of products over the tokens of one team.  `rows` and `columns`: this lane's place in the team's tiles.
+template <int TILES>
+TG_DEVICE void add_team(f32x4 (&sum)[4], const unsigned char *const (&rows)[TILES], const unsigned char *const (&columns)[TILES]) {
+    f32x4 a[TILES], b[TILES];
+#pragma unroll
+    for (int n = 0; n < TILES; ++n)
+        a[n] = unpack4(read_across(rows[n])), b[n] = unpack4(read_across(columns[n]));
+#pragma unroll
+    for (int n = 0; n < TILES; ++n)
+        ready(a[n], b[n]);
+    products_only();
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int n = 0; n < TILES; ++n)
-            a[n] = unpack4(read_across(rows[n] + w * stride)), b[n] = unpack4(read_across(columns[n] + w * column_stride));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int n = 0; n < TILES; ++n)
-                sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][j], b[n][j], sum[n], 0, 0, 0);
-            if constexpr (SCALE)
-                sum[TILES] = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], sum[TILES], 0, 0, 0);
-        }
-    }
+            sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][j], b[n][j], sum[n], 0, 0, 0);
+    products_only();
 }
 __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m, Workspace whole, Group group, int parameters) {
     extern __shared__ __align__(16) unsigned char memory[];
@@ -860,27 +1139,47 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
     const bool second_half = waves > CHUNK_WAVES / 2;
     float *out = s.partials + size_t(chunk) * parameters;
     const uint32_t lds = lds_address(memory);
-    // TILES tiles of every wave, `apart` bytes from one wave to the next in memory, one behind another in LDS; 16 bytes a lane.
-    // The last chunk's missing waves are zeros, of the second half only where it has any.
-    const auto copy = [&](auto tiles, const u32x2 *source, int apart, int to) {
-        constexpr int PIECES = decltype(tiles)::value * 32;
-        static_assert(CHUNK_WAVES * PIECES % (WAVES * 64) == 0, "every wave has as many copies");
+    // `tiles` tiles of every team, which lie one behind another in memory and do in LDS; 16 bytes a lane.  The last chunk's missing
+    // teams are zeros, of the second half only where it has any.
+    const auto copy = [&](auto tiles, const u32x2 *source, int to) {
+        constexpr int COPIES = decltype(tiles)::value;
+        static_assert(CHUNK_WAVES * 512 == 64 * WAVES * 16, "every wave has a copy for each of a team's tiles");
+        const unsigned char *from = reinterpret_cast<const unsigned char *>(uniform(source)) + wave * 1024;
+        const uint32_t at = lds + uint32_t(to + wave * 1024);
+        if (waves == CHUNK_WAVES) {
 #pragma unroll
-        for (int i = 0; i < CHUNK_WAVES * PIECES / (WAVES * 64); ++i) {
-            const int base = (i * WAVES + wave) * 64, piece = base + lane, w = piece / PIECES;
-            if (w < waves)
-                async_copy16(lds + uint32_t(to + base * 16), source, uint32_t(w * apart + (piece - w * PIECES) * 16));
-            else if (w < CHUNK_WAVES / 2 || second_half)
-                *reinterpret_cast<u32x4 *>(memory + to + piece * 16) = u32x4{0, 0, 0, 0};
+            for (int i = 0; i < COPIES; ++i)
+                async_copy16(at + uint32_t(i) * WAVES * 1024, from + i * WAVES * 1024, uint32_t(lane * 16));
+            return;
+        }
+        const int there = waves * COPIES * 512, wanted = (second_half ? CHUNK_WAVES : CHUNK_WAVES / 2) * COPIES * 512;
+        for (int i = 0; i < COPIES; ++i) {
+            const int piece = (i * WAVES + wave) * 1024 + lane * 16;
+            if (piece < there)
+                async_copy16(at + uint32_t(i) * WAVES * 1024, from + i * WAVES * 1024, uint32_t(lane * 16));
+            else if (piece < wanted)
+                *reinterpret_cast<u32x4 *>(memory + to + piece) = u32x4{0, 0, 0, 0};
         }
     };
-    const auto half_there = [&]() { // all but a wave's last eight copies; a chunk that is not full has fewer
-        if (waves == CHUNK_WAVES)
-            wait_vmcnt<8>();
-        else
-            wait_vmcnt<0>();
-        wait_lgkmcnt0();
-        __syncthreads();
+    // The teams' rows one after another, each as soon as it is there: team w's last tile is brought by a wave's copy
+    // ceil((w + 1) tiles / 8) - 1 of `tiles`.  A chunk that is not full has fewer copies: all of them are waited for.
+    // The wave's loads behind its copies, `younger` of them, may stay under way.
+    const auto each_team = [&](auto tiles, auto younger, auto &&add) {
+        constexpr int COPIES = decltype(tiles)::value, YOUNGER = decltype(younger)::value;
+        up_to<0, CHUNK_WAVES - 1>([&](auto team) {
+            constexpr int TEAM = decltype(team)::value;
+            if (TEAM >= CHUNK_WAVES / 2 && !second_half)
+                return;
+            if (waves == CHUNK_WAVES)
+                wait_vmcnt<COPIES - ((TEAM + 1) * COPIES + CHUNK_WAVES - 1) / CHUNK_WAVES + YOUNGER>();
+            else if (TEAM == 0) {
+                wait_vmcnt<0>();
+                wait_lgkmcnt0();
+            }
+            if (TEAM == 0 || waves == CHUNK_WAVES)
+                __syncthreads();
+            add(team);
+        });
     };
     const unsigned char *mine = memory + across_offset(lane, true);
     const auto tile = [&](int n) { return mine + n * 512; };
@@ -888,30 +1187,27 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
     ScaleTerms terms;
     if (unit < m.depth) {
         const Layer q = layer_layout(unit);
-        // waves 1 and 2 have a norm's scale besides gate and up
-        if (wave == 1 || wave == 2)
+        copy(std::integral_constant<int, OPERANDS>{}, s.tiles + (size_t(unit) * s.waves + first) * OPERANDS * 64, 0);
+        constexpr std::integral_constant<int, OPERANDS> tiles;
+        if (wave == 0)
+            each_team(tiles, std::integral_constant<int, 0>{}, [&](auto team) {
+                const unsigned char *at = tile(decltype(team)::value * OPERANDS), *n1 = at + T_N1 * 512, *dqkv = at + T_DQKV * 512;
+                add_team<4>(sum, {dqkv, dqkv + 512, dqkv + 1024, at + T_DH_ATTENTION * 512}, {n1, n1, n1, at + T_A * 512});
+            });
+        else if (wave == 3)
+            each_team(tiles, std::integral_constant<int, 0>{}, [&](auto team) {
+                const unsigned char *at = tile(decltype(team)::value * OPERANDS), *dh = at + T_DH_DOWN * 512, *act = at + T_ACT * 512;
+                add_team<3>(sum, {dh, dh, dh}, {act, act + 512, act + 1024});
+            });
+        else { // waves 1 and 2 have a norm's scale besides gate and up
             terms.request(s, 2 * unit + wave - 1, first, waves, lane);
-        copy(std::integral_constant<int, OPERANDS>{}, s.tiles + ((size_t(unit) * s.waves + first) * TILES + T_OPERANDS) * 64, TILES * 512, 0);
-        constexpr int N1 = T_N1 - T_OPERANDS, A = T_A - T_OPERANDS, N2 = T_N2 - T_OPERANDS, ACT = T_ACT - T_OPERANDS,
-                      DQKV = T_DQKV - T_OPERANDS, DH_ATTENTION = T_DH_ATTENTION - T_OPERANDS, DGU = T_DGU - T_OPERANDS,
-                      DH_DOWN = T_DH_DOWN - T_OPERANDS, STRIDE = OPERANDS * 512;
-        const auto layer = [&](int half) {
-            if (wave == 0)
-                add_half<4, false>(sum, {tile(DQKV), tile(DQKV + 1), tile(DQKV + 2), tile(DH_ATTENTION)}, {tile(N1), tile(N1), tile(N1), tile(A)},
-                                   STRIDE, STRIDE, terms, half);
-            else if (wave == 3)
-                add_half<3, false>(sum, {tile(DH_DOWN), tile(DH_DOWN), tile(DH_DOWN)}, {tile(ACT), tile(ACT + 1), tile(ACT + 2)}, STRIDE, STRIDE,
-                                   terms, half);
-            else
-                add_half<3, true>(sum, {tile(DGU + 3 * wave - 3), tile(DGU + 3 * wave - 2), tile(DGU + 3 * wave - 1)}, {tile(N2), tile(N2), tile(N2)},
-                                  STRIDE, STRIDE, terms, half);
-        };
-        half_there(); // brought by nine of a wave's seventeen copies
-        layer(0);
-        if (second_half) {
-            wait_vmcnt<0>();
-            __syncthreads();
-            layer(1);
+            each_team(tiles, std::integral_constant<int, CHUNK_WAVES * 4>{}, [&](auto team) {
+                const unsigned char *at = tile(decltype(team)::value * OPERANDS), *dgu = at + (T_DGU + 3 * wave - 3) * 512, *n2 = at + T_N2 * 512;
+                add_team<3>(sum, {dgu, dgu + 512, dgu + 1024}, {n2, n2, n2});
+            });
+            const float scale = terms.sum();
+            if (g == 0)
+                out[(wave == 1 ? q.attention_norm : q.mlp_norm) + c] = scale;
         }
         if (wave == 0) {
 #pragma unroll
@@ -922,54 +1218,41 @@ __global__ __launch_bounds__(64 * WAVES) void w16_weight_gradient_kernel(Model m
 #pragma unroll
         for (int t = 0; t < 3; ++t)
             store_tile(wave == 3 ? out + q.down + t * 16 : out + q.gate + ((wave - 1) * 3 + t) * 256, sum[t], wave == 3 ? F : W, lane);
-        if (wave < 3 && g == 0)
-            out[(wave == 1 ? q.attention_norm : q.mlp_norm) + c] = sum[3][0];
         return;
     }
     if (unit == m.depth) { // the head: a wave four tiles of logits
         constexpr int NF = CHUNK_WAVES * 16;
-        copy(std::integral_constant<int, 1>{}, s.nf + size_t(first) * 64, 512, NF * 512);
-        copy(std::integral_constant<int, 16>{}, s.dlogits + size_t(first) * 16 * 64, 16 * 512, 0);
-        const auto head = [&](int half) {
-            add_half<4, false>(sum, {tile(wave * 4), tile(wave * 4 + 1), tile(wave * 4 + 2), tile(wave * 4 + 3)},
-                               {tile(NF), tile(NF), tile(NF), tile(NF)}, 16 * 512, 512, terms, half);
+        copy(std::integral_constant<int, 1>{}, s.nf + size_t(first) * 64, NF * 512);
+        copy(std::integral_constant<int, 16>{}, s.dlogits + size_t(first) * 16 * 64, 0);
+        const auto add = [&](auto team) {
+            constexpr int TEAM = decltype(team)::value;
+            const unsigned char *of_wave = tile(TEAM * 16 + wave * 4), *nf = tile(NF + TEAM);
+            add_team<4>(sum, {of_wave, of_wave + 512, of_wave + 1024, of_wave + 1536}, {nf, nf, nf, nf});
         };
-        half_there(); // eight of the sixteen
-        head(0);
-        if (second_half) {
-            wait_vmcnt<0>();
-            __syncthreads();
-            head(1);
-        }
         const int at = V * W + m.depth * LAYER_SIZE + W;
+        if (wave == 0) {
+            terms.request(s, 2 * m.depth, first, waves, lane);
+            each_team(std::integral_constant<int, 16>{}, std::integral_constant<int, CHUNK_WAVES * 4>{}, add);
+            const float scale = terms.sum();
+            if (g == 0)
+                out[at - W + c] = scale;
+        } else
+            each_team(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{}, add);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
             store_tile(out + at + (wave * 4 + t) * 256, sum[t], W, lane);
-        if (wave == 0) {
-            terms.request(s, 2 * m.depth, first, waves, lane);
-            f32x4 scale = ZERO;
-#pragma unroll
-            for (int w = 0; w < CHUNK_WAVES; ++w)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    scale = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, terms.v[w][j], scale, 0, 0, 0);
-            if (g == 0)
-                out[at - W + c] = scale[0];
-        }
         return;
     }
     // The embedding's rows: the one-hot matrix of the tokens times the gradient.  0 times an infinity is NaN, in ids that have
     // no part in it, so where a row is not finite the rows are added one by one.
-    copy(std::integral_constant<int, 1>{}, s.dh + size_t(first) * 64, 512, 0);
+    copy(std::integral_constant<int, 1>{}, s.dh + size_t(first) * 64, 0);
     uint32_t ids[CHUNK_WAVES];
 #pragma unroll
     for (int w = 0; w < CHUNK_WAVES; ++w) {
         ids[w] = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int t = 4 * j + g, token = (first + w) * m.per_wave + t; // rows beyond the last token are zero: any id will do
-            ids[w] |= uint32_t(w < waves && t < m.per_wave && token < m.tokens ? x[token] : 0) << (8 * j);
-        }
+        for (int j = 0; j < 4; ++j) // rows beyond the last token are zero: any id will do, and every load goes out at once
+            ids[w] |= uint32_t(x[min((first + w) * m.per_wave + min(4 * j + g, m.per_wave - 1), m.tokens - 1)]) << (8 * j);
     }
     wait_vmcnt<0>();
     wait_lgkmcnt0();
@@ -1095,20 +1378,28 @@ struct Update {
     int count;
     W16Step step[W16_BATCHES];
 };
-// clip_factor of the norms, with the sums of a fold's quarters formed first
-TG_DEVICE float clip_factor(const Update &u, int n, float *waves) {
-    const W16Step &step = u.step[n];
-    if (u.norm_parts == 1 || !(step.adam.clip > 0.f))
-        return ::clip_factor(step.adam.clip, step.norms, u.norm_count, waves);
-    float sum = 0.f;
-    for (int i = threadIdx.x; i < u.norm_count; i += 256) {
-        const f32x4 part = *reinterpret_cast<const f32x4 *>(step.norms + i * FOLD_QUARTERS);
-        sum += (part[0] + part[1]) + (part[2] + part[3]);
+// clip_factor of the norms, with the sums of a fold's quarters formed first; those are asked for a step ahead.
+struct Clip {
+    const Update &u;
+    f32x4 next;
+    TG_DEVICE Clip(const Update &u_) : u(u_) { request(0); }
+    TG_DEVICE bool parts(int n) const { return u.norm_parts != 1 && u.step[n].adam.clip > 0.f; }
+    TG_DEVICE void request(int n) {
+        if (n < u.count && parts(n) && int(threadIdx.x) < u.norm_count)
+            next = reinterpret_cast<const f32x4 *>(u.step[n].norms)[threadIdx.x];
     }
-    return fminf(1.f, step.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
-}
+    TG_DEVICE float operator()(int n, float *waves) {
+        const W16Step &step = u.step[n];
+        if (!parts(n))
+            return ::clip_factor(step.adam.clip, step.norms, u.norm_count, waves);
+        const f32x4 part = next;
+        request(n + 1);
+        const float sum = int(threadIdx.x) < u.norm_count ? (part[0] + part[1]) + (part[2] + part[3]) : 0.f;
+        return fminf(1.f, step.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
+    }
+};
 TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
-    __shared__ float wide[2][16 * F];
+    __shared__ __align__(16) u32x2 wide[2][3][64]; // the iterate's tiles of sixteen columns, as the lanes hold them
     __shared__ float norm_waves[4];
     const Layer p = layer_layout(matrix / 5);
     const int type = matrix % 5;
@@ -1116,16 +1407,20 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
     const int rows = (type == 0 || type == 2 || type == 3) ? 48 : 16, cols = type == 4 ? 48 : 16;
     const int n = rows > cols ? rows : cols, size = rows * cols, tid = threadIdx.x;
     // element tid + 256 k of the matrix is this thread's until the iteration and again behind it; its place in the 16 x n form
-    auto place = [&](int i) { return rows > cols ? (i % cols) * rows + i / cols : i; };
     float next_g[3], m[3], w[3];
+    int place[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const int i = weight + tid + 256 * k;
+        const int i = weight + tid + 256 * k, line = (tid + 256 * k) / cols, at = tid + 256 * k - line * cols;
+        const int row = rows > cols ? at : line, col = rows > cols ? line : at;
+        place[k] = (((col >> 4) * 64 + (row >> 2) * 16 + (col & 15)) << 2) + (row & 3);
         const bool mine = tid + 256 * k < size;
         next_g[k] = mine ? u.step[0].gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f;
         w[k] = mine ? master(u.step[0].from.hi, u.step[0].from.lo, i) : 0.f;
     }
     const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
+    const int across = across_offset(lane, true);
+    Clip clip_of(u);
     for (int at = 0; at < u.count; ++at) {
         const W16Step &u_step = u.step[at];
         const MuonArgs &muon = u_step.muon;
@@ -1134,7 +1429,7 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
 #pragma unroll
             for (int k = 0; k < 3; ++k)
                 next_g[k] = tid + 256 * k < size ? u.step[at + 1].gradient[weight + tid + 256 * k] : 0.f;
-        const float clip = clip_factor(u, at, waves[at & 1]);
+        const float clip = clip_of(at, waves[at & 1]);
         float squares = 0.f, b[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k)
@@ -1148,49 +1443,46 @@ TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (tid + 256 * k < size)
-                wide[0][place(tid + 256 * k)] = round_bf16(b[k] / norm);
+                reinterpret_cast<bf16_t *>(wide[0])[place[k]] = float_to_bf16(b[k] / norm);
         __syncthreads();
         f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
         if (tile < tiles)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                x[r] = wide[0][(4 * gr + r) * n + 16 * tile + c];
+            x = unpack4(wide[0][tile][lane]);
         for (int step = 0; step < muon.ns_steps; ++step) {
-            const float *in = wide[step & 1];
-            float *out = wide[(step & 1) ^ 1];
             if (tile < tiles) {
-                f32x4 gram = ZERO; // A = X X^T, kept in bf16
+                const unsigned char *in = reinterpret_cast<const unsigned char *>(wide[step & 1]) + across;
+                f32x4 row[3], gram = ZERO; // A = X X^T, kept in bf16
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
-                    if (k < tiles) {
-                        f32x4 row;
+                    if (k < tiles)
+                        row[k] = unpack4(read_across(in + k * 512));
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            row[j] = in[c * n + 16 * k + 4 * j + gr];
-                        gram = multiply(row, row, gram);
-                    }
+                for (int k = 0; k < 3; ++k)
+                    if (k < tiles)
+                        gram = multiply(row[k], row[k], gram);
                 gram = rounded(gram);
                 const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
                 f32x4 work; // -4.775 A + 2.0315 A A
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
-                const f32x4 product = multiply(turned(rounded(work)), turned(x));
+                f32x4 product = multiply(turned(rounded(work)), turned(x));
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    x[r] = round_bf16(fmaf(3.4445f, x[r], product[r]));
-                    out[(4 * gr + r) * n + 16 * tile + c] = x[r];
-                }
+                for (int r = 0; r < 4; ++r)
+                    product[r] = fmaf(3.4445f, x[r], product[r]);
+                const u32x2 packed = pack4(product);
+                wide[(step & 1) ^ 1][tile][lane] = packed;
+                x = unpack4(packed);
             }
             __syncthreads();
         }
-        const float *result = wide[muon.ns_steps & 1];
+        const bf16_t *result = reinterpret_cast<const bf16_t *>(wide[muon.ns_steps & 1]);
         const float adjusted = muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-muon.lr, muon.weight_decay, 1.f);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (tid + 256 * k < size) {
                 const int i = weight + tid + 256 * k;
-                w[k] = fmaf(w[k], keep, -(adjusted * result[place(tid + 256 * k)]));
+                w[k] = fmaf(w[k], keep, -(adjusted * bf16_to_float(result[place[k]])));
                 const uint32_t bits = __float_as_uint(w[k]);
                 u_step.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
                 u_step.to.lo[i] = uint16_t(bits);
@@ -1224,12 +1516,13 @@ __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
     for (int k = 0; k < 4; ++k)
         w[k] = master(u.step[0].from.hi, u.step[0].from.lo, at + k);
     f32x4 next_g = *reinterpret_cast<const f32x4 *>(u.step[0].gradient + at);
+    Clip clip_of(u);
     for (int n = 0; n < u.count; ++n) {
         const W16Step &step = u.step[n];
         const f32x4 g = next_g;
         if (n + 1 < u.count)
             next_g = *reinterpret_cast<const f32x4 *>(u.step[n + 1].gradient + at);
-        const float scale = clip_factor(u, n, waves[n & 1]);
+        const float scale = clip_of(n, waves[n & 1]);
         if (!live)
             continue;
 #pragma unroll
@@ -1256,7 +1549,7 @@ void check_shape(int depth, int batch, int context) {
     require(int64_t(batch) * context <= (1 << 24), "w16: too many tokens");
 }
 Model make_model(int depth, int batch, int context, const uint16_t *hi, const uint16_t *lo) {
-    return Model{hi, lo, depth, batch * context, context, tokens_per_wave(context)};
+    return Model{hi, lo, depth, batch * context, context, tokens_per_wave(context), 0};
 }
 
 } // namespace
@@ -1273,7 +1566,7 @@ extern "C" size_t tgk_w16_workspace(int depth, int batch, int context) {
 
 namespace {
 // the kernels' LDS beyond 64 KiB is a per-device attribute
-template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&configured)[64], size_t bytes) {
+template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&configured)[64], size_t bytes = LDS_BYTES) {
     int device = 0;
     check_hip(hipGetDevice(&device));
     require(device >= 0 && device < 64, "w16: device index out of range");
@@ -1282,6 +1575,44 @@ template <class Kernel> void allow_lds(Kernel kernel, std::atomic<bool> (&config
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)),
               "w16 LDS size: ");
     configured[device].store(true, std::memory_order_release);
+}
+int compute_units() {
+    static std::atomic<int> cached[64];
+    int device = 0;
+    check_hip(hipGetDevice(&device));
+    require(device >= 0 && device < 64, "w16: device index out of range");
+    int units = cached[device].load(std::memory_order_relaxed);
+    if (!units) {
+        check_hip(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
+        cached[device].store(units > 0 ? units : 256, std::memory_order_relaxed);
+    }
+    return units;
+}
+// How a pass over `waves` teams in each of `count` batches is launched: the fewest teams a block that need no more than `places` blocks.
+struct Teams {
+    int teams, blocks, roles; // teams of a block
+    size_t lds;
+    bool rows; // stay in LDS
+};
+Teams teams_of(int waves, int count, int depth, int roles, bool rows, int places) {
+    const auto lds = [&](int teams) { return roles == 1 ? lone_lds_bytes(depth) : lds_bytes(depth, teams, rows); };
+    int teams = 1;
+    while ((teams + 1) * roles <= block_waves(roles) && (waves + teams - 1) / teams * count > places && lds(teams + 1) <= LDS_BYTES)
+        ++teams;
+    return {teams, (waves + teams - 1) / teams, roles, lds(teams), rows};
+}
+// Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that, also
+// for batches in flight (`flying` at a time on streams of their own), a lone wave does less in all: no handing over, two waves'
+// arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8 (context 4) 87 and 106, 1280
+// (context 8) 171 and 145; 640 with K = 4 on streams 73 and 59.  Of lone waves a block takes four where there are other batches (K = 4, 640
+// teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us), as many as leave every unit one block where there are none (1280 teams: 145, with four 149).
+Teams step_teams(int waves, int count, int depth, int flying) {
+    for (const bool rows : {true, false}) {
+        const Teams t = teams_of(waves, count, depth, ROLES, rows, compute_units());
+        if (t.blocks * count <= compute_units() && waves * count * flying <= STEP_TEAMS * compute_units())
+            return t;
+    }
+    return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : compute_units());
 }
 void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const Group &group, int count, bool losses) {
     const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
@@ -1302,12 +1633,14 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && y && workspace && token_losses, "w16_forward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
-        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
+        Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
         static std::atomic<bool> configured[2][64];
         const auto kernel = with_gradient ? w16_forward_kernel<true> : w16_forward_kernel<false>;
-        allow_lds(kernel, configured[with_gradient != 0], staged_bytes(MAX_DEPTH));
-        hipLaunchKernelGGL(kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, x, y, r, token_losses, logits);
+        allow_lds(kernel, configured[with_gradient != 0]);
+        const Teams t = teams_of(r.waves, 1, depth, ROLES, false, compute_units());
+        m.teams = t.teams;
+        hipLaunchKernelGGL(kernel, dim3(t.blocks), dim3(64 * block_waves(ROLES)), t.lds, stream, m, x, y, r, token_losses, logits);
         check_hip(hipGetLastError(), "w16_forward launch: ");
     });
 }
@@ -1318,11 +1651,13 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         check_shape(depth, batch, context);
         require(weight_hi && weight_lo && x && workspace && gradient, "w16_backward: missing operand");
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
-        const Model m = make_model(depth, batch, context, weight_hi, weight_lo);
+        Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
         static std::atomic<bool> configured[64];
-        allow_lds(w16_backward_kernel, configured, staged_bytes(MAX_DEPTH));
-        hipLaunchKernelGGL(w16_backward_kernel, dim3(r.blocks), dim3(64 * WAVES), staged_bytes(depth), stream, m, r);
+        allow_lds(w16_backward_kernel, configured);
+        const Teams t = teams_of(r.waves, 1, depth, ROLES, false, compute_units());
+        m.teams = t.teams;
+        hipLaunchKernelGGL(w16_backward_kernel, dim3(t.blocks), dim3(64 * block_waves(ROLES)), t.lds, stream, m, r);
         check_hip(hipGetLastError(), "w16_backward launch: ");
         Group group{};
         group.member[0].tokens = const_cast<uint8_t *>(x), group.member[0].workspace = workspace, group.member[0].gradient = gradient;
@@ -1339,23 +1674,27 @@ int w16_norm_count(int depth) {
 int w16_norm_parts() {
     return FOLD_QUARTERS;
 }
-void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, const W16Batch *batches) {
+void w16_gradients(hipStream_t stream, int depth, int batch, int context, const W16Data &data, int count, int flying, const W16Batch *batches) {
     require(context == 4 || context == 8, "w16: a training step has a context of 4 or 8");
     require(count >= 1 && count <= W16_BATCHES, "w16: too many batches for one launch");
-    const Model m = make_model(depth, batch, context, nullptr, nullptr);
+    Model m = make_model(depth, batch, context, nullptr, nullptr);
     const Workspace r = carve(depth, batch, context, batches[0].workspace);
     Group group{};
     std::copy(batches, batches + count, group.member);
-    static std::atomic<bool> configured[2][64];
-    const auto kernel = context == 4 ? w16_step_kernel<4> : w16_step_kernel<8>;
-    allow_lds(kernel, configured[context == 8], staged_bytes(MAX_DEPTH));
+    const Teams t = step_teams(r.waves, count, depth, flying);
+    m.teams = t.teams;
+    static std::atomic<bool> configured[6][64];
+    const auto kernel = context == 4 ? (t.roles == 1 ? w16_step_kernel<4, 1, false> : t.rows ? w16_step_kernel<4, ROLES, true> : w16_step_kernel<4, ROLES, false>)
+                                     : (t.roles == 1 ? w16_step_kernel<8, 1, false> : t.rows ? w16_step_kernel<8, ROLES, true> : w16_step_kernel<8, ROLES, false>);
+    allow_lds(kernel, configured[(context == 8) * 3 + (t.roles == 1 ? 2 : t.rows)]);
     const uint64_t places = uint64_t(data.size) - 8, inverse = places > 1 ? uint64_t((static_cast<unsigned __int128>(1) << 64) / places) : ~uint64_t(0);
-    hipLaunchKernelGGL(kernel, dim3(r.blocks, count), dim3(64 * WAVES), staged_bytes(depth), stream, m, data, inverse, r, group);
+    hipLaunchKernelGGL(kernel, dim3(t.blocks, count), dim3(64 * block_waves(t.roles)), t.lds, stream, m, data, inverse, r, group);
     check_hip(hipGetLastError(), "w16_step launch: ");
     launch_weight_gradients(stream, m, r, group, count, true);
 }
 void w16_updates(hipStream_t stream, int depth, float *momentum, float *variance, int norm_count, int norm_parts, int count,
                  const W16Step *steps) {
+    require(norm_parts == 1 || norm_count <= 256, "w16: a fold's norms have a thread each");
     require(count >= 1 && count <= W16_BATCHES, "w16: too many steps for one launch");
     Update u{momentum, variance, norm_count, norm_parts, depth, count, {}};
     std::copy(steps, steps + count, u.step);
