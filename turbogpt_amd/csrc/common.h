@@ -113,6 +113,13 @@ TG_DEVICE void async_copy16(uint32_t lds_base, const void *uniform_base, uint32_
                  : "s"(lds_base), "v"(lane_offset), "s"(uniform_base)
                  : "memory");
 }
+// A store that is written through to memory, where a plain one waits in its L2 until the launch has ended and is then written
+// back with everything else, behind the last block.  The line stays in the L2.  Worth it for whole lines of results that the launch's end
+// would wait for; a compute-bound launch's bus is better left alone.  The hardware wants two wait states between a 16-byte store and
+// the next write of its registers, and the compiler puts none behind assembly text.
+TG_DEVICE void store_through(void *global, const u32x4 &v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(global), "v"(v) : "memory");
+}
 // a pointer that is the same in every lane, in scalar registers
 template <class T> TG_DEVICE T *uniform(T *p) {
     const uint64_t bits = reinterpret_cast<uint64_t>(p);

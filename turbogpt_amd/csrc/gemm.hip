@@ -56,8 +56,14 @@ struct EpilogueBf16 {
     TG_DEVICE u32x4 load_aux(int m, int n) const {
         return *reinterpret_cast<const u32x4 *>(aux + size_t(m) * ld_aux + n);
     }
+    template <bool THROUGH> TG_DEVICE static void store(bf16_t *to, const u32x4 &v) {
+        if constexpr (THROUGH)
+            store_through(to, v);
+        else
+            *reinterpret_cast<u32x4 *>(to) = v;
+    }
     // y: the bf16-rounded accumulators of row m, columns n .. n+7
-    template <int MODE> TG_DEVICE void finish_as(int m, int n, u32x4 y, u32x4 a) const {
+    template <int MODE, bool THROUGH = false> TG_DEVICE void finish_as(int m, int n, u32x4 y, u32x4 a) const {
         if constexpr (MODE == EPI_RESIDUAL) {
             // RN(RN(acc) + residual): the bf16 add of cuda/mma.cuh:95-97
 #pragma unroll
@@ -75,9 +81,9 @@ struct EpilogueBf16 {
             for (int e = 0; e < 4; ++e)
                 g[e] = pack_bf16(gelu_f(bf16_lo(y[e])), gelu_f(bf16_hi(y[e])));
             if constexpr (MODE != EPI_GELU) {
-                *reinterpret_cast<u32x4 *>(out2 + size_t(m) * ld_out2 + n) = g;
+                store<THROUGH>(out2 + size_t(m) * ld_out2 + n, g);
                 if constexpr (MODE == EPI_GELU_CACHED)
-                    *reinterpret_cast<u32x4 *>(out + size_t(m) * ld_out + n) = y;
+                    store<THROUGH>(out + size_t(m) * ld_out + n, y);
                 return;
             }
             // Both outputs stream past the L2: the pre-activation is not read again before the backward pass, and the
@@ -88,7 +94,7 @@ struct EpilogueBf16 {
             __builtin_nontemporal_store(y, reinterpret_cast<u32x4 *>(out + size_t(m) * ld_out + n));
             return;
         }
-        *reinterpret_cast<u32x4 *>(out + size_t(m) * ld_out + n) = y;
+        store<THROUGH>(out + size_t(m) * ld_out + n, y);
     }
     TG_DEVICE void finish(int m, int n, u32x4 y, u32x4 a) const {
         if (mode == EPI_RESIDUAL)
@@ -107,16 +113,18 @@ struct EpilogueBf16 {
 // names how many younger operations may stay outstanding: with the mode decided by branches that number is unknown
 // and every 32 x 32 block of the epilogue ends up waiting for its own stores to be acknowledged; with straight-line
 // code the stores of a block stay in flight while the next is rounded and transposed.
-template <int MODE> struct EpilogueBf16As {
+// THROUGH: results are written through to memory.
+template <int MODE, bool THROUGH = false> struct EpilogueBf16As {
     static constexpr bool BF16 = true;
     // vector-memory instructions per 32 x 32 block of the staged epilogue: two 16-byte stores (four with the GELU
     // output), two 16-byte loads of the second input
     static constexpr int MEMORY_OPS_PER_BLOCK = MODE == EPI_PLAIN || MODE == EPI_GELU_ONLY ? 2 : 4;
     using Cached = EpilogueBf16As<MODE == EPI_GELU ? int(EPI_GELU_CACHED) : MODE>;
+    using Through = EpilogueBf16As<MODE == EPI_GELU ? int(EPI_GELU_CACHED) : MODE, true>;
     EpilogueBf16 any;
     TG_DEVICE bool wants_aux() const { return MODE == EPI_RESIDUAL || MODE == EPI_GELU_BWD; }
     TG_DEVICE u32x4 load_aux(int m, int n) const { return any.load_aux(m, n); }
-    TG_DEVICE void finish(int m, int n, u32x4 y, u32x4 a) const { any.finish_as<MODE>(m, n, y, a); }
+    TG_DEVICE void finish(int m, int n, u32x4 y, u32x4 a) const { any.finish_as<MODE, THROUGH>(m, n, y, a); }
 };
 
 // fp32 outputs (weight gradients, split-K slabs): tiles go through the same kind of wave-private LDS
@@ -2284,19 +2292,24 @@ void launch_gemm_tile_as(hipStream_t stream, const bf16_t *A, int lda, const bf1
 // GELU outputs that the eight L2s hold are left to them, where the next launch finds them (streamed past them the product
 // itself is 0.3 us faster, 16 training steps at d256 and text at d768 slower by 1 and 3 %); larger ones are streamed: the two of
 // 16384 x 4096, K = 1920 / 896 / 640 took 352 / 200 / 165 us through the caches, 285 / 160 / 128 past them.
+// Of at most 8 MiB each they are also written through to memory, so that the launch does not end with writing them back: 1920 x 640 and
+// 1920 x 1920, six products 76.0 -> 73.5 us; 16 steps of 2048 tokens at d256 5.79 -> 5.69 ms, of 1920 at d640 19.9 -> 19.6; 9216 x 2048 at
+// d512 was 0.6 % slower so.
 template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
 void launch_gemm_tile(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                       const Epilogue &e) {
     if (size_t(M) * N * 2 * sizeof(bf16_t) > size_t(8) * (4 << 20))
         launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, e);
+    else if (size_t(M) * N * sizeof(bf16_t) <= size_t(8) << 20)
+        launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Through{e.any});
     else
         launch_gemm_tile_as<BM, BN, S, BKC, GROUPS>(stream, A, lda, B, ldb, M, N, K, typename Epilogue::Cached{e.any});
 }
 template <int BM, int BN, bool BKC, class Epilogue>
 void launch_gemm_uneven(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K, const Epilogue &e) {
-    using Cached = typename Epilogue::Cached; // few outputs: the L2s hold them
+    using Through = typename Epilogue::Through; // few outputs
     constexpr int S = 4;
-    auto kernel = gemm_uneven_kernel<BM, BN, S, BKC, Cached>;
+    auto kernel = gemm_uneven_kernel<BM, BN, S, BKC, Through>;
     constexpr size_t lds = S * (BM + BN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
@@ -2307,13 +2320,13 @@ void launch_gemm_uneven(hipStream_t stream, const bf16_t *A, int lda, const bf16
     }
     const int rows = M / BM, cols = N / BN;
     hipLaunchKernelGGL(kernel, dim3(rows * cols), dim3(256), lds, stream, A, lda, B, ldb, K / 64,
-                       tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Cached{e.any});
+                       tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Through{e.any});
     check_hip(hipGetLastError(), "gemm launch: ");
 }
 template <int BM, int BN, int WM, int WN, int S, bool BKC, class Epilogue>
 void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K, const Epilogue &e) {
-    using Cached = typename Epilogue::Cached; // few outputs: the L2s hold them
-    auto kernel = gemm_waves_kernel<BM, BN, WM, WN, S, BKC, Cached>;
+    using Through = typename Epilogue::Through; // few outputs
+    auto kernel = gemm_waves_kernel<BM, BN, WM, WN, S, BKC, Through>;
     constexpr int waves = 2 * (BM / WM) * (BN / WN);
     constexpr size_t lds = waves * S * (WM + WN) * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
@@ -2325,7 +2338,7 @@ void launch_gemm_waves(hipStream_t stream, const bf16_t *A, int lda, const bf16_
     }
     const int rows = M / BM, cols = N / BN;
     hipLaunchKernelGGL(kernel, dim3(rows * cols), dim3(64 * waves), lds, stream, A, lda, B, ldb, K / 64,
-                       tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Cached{e.any});
+                       tile_grid(rows, cols, BM, BN, (rows * cols + 7) / 8), Through{e.any});
     check_hip(hipGetLastError(), "gemm launch: ");
 }
 // Which tile a product whose reduced dimension 64 divides is cut into.  The cost of a 64-k stage on the fullest compute
