@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const bf16_t *__rest
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
                     o[k] = v[j][k] * inv * gm[k] + bt[k];
-                *reinterpret_cast<u32x4 *>(y + size_t(row) * D + c * 8) = pack8(o);
+                store_through(y + size_t(row) * D + c * 8, pack8(o)); // the launch is short and ends with what its L2s hold
             }
         }
     }
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256 * TURNS) void layernorm_bwd_kernel(const bf16_t
                     for (int k = 0; k < 8; ++k)
                         o[k] = prior[k] + round_bf16(o[k]);
                 }
-                *reinterpret_cast<u32x4 *>(p) = pack8(o);
+                store_through(p, pack8(o)); // as in the forward pass
             }
         }
     }

@@ -141,7 +141,8 @@ struct EpilogueF32 {
         f32x4 *p = reinterpret_cast<f32x4 *>(out + split * split_stride + size_t(m) * ld_out + n);
         if (accumulate)
             value += *p;
-        *p = value;
+        // whole lines, written through to memory: 3840 tokens, two gradients of 384 x 1152 beside four products 70.3 -> 67.7 us
+        store_through(p, __builtin_bit_cast(u32x4, value));
     }
 };
 
