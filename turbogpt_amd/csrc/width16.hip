@@ -1368,138 +1368,176 @@ __global__ __launch_bounds__(256) void w16_fold_kernel(Workspace whole, Group gr
 // Blocks 0 .. 5 depth - 1: Muon, a hidden matrix each.  The rest: AdamW, 256 quads of embedding, scales and head each.
 // The Newton-Schulz iterate is a 16 x n matrix in 16 x 16 tiles, one a wave, lane 16 g + c holding rows 4 g .. of column c;
 // the products run on the fp32 matrix instruction (the same fmaf chains as a loop).  X X^T is symmetric to the last bit,
-// so its tile turned is the operand of the two products behind it, every wave computes it for itself, and a step
-// exchanges nothing but X through LDS: one barrier a step where there were four.
+// so its tile turned is the operand of the two products behind it, every wave computes it for itself, and a step of the
+// iteration exchanges nothing but X through LDS.
 // One launch makes as many steps, one after another, as there are gradients at hand: an element's (Muon: a matrix's) weights
-// and state stay in the registers between them.
+// and state stay in the registers between them.  What a matrix's iteration starts from hangs on gradients and momentum alone, so
+// up to four steps' iterations run side by side, each on a group of four waves, and only the weights' own chain is left in the steps'
+// order: every group follows it and writes its step's.
+constexpr int UPDATE_GROUPS = 4;
 struct Update {
     float *momentum, *variance;
     int norm_count, norm_parts, depth; // norms: norm_count sums of norm_parts partial sums each, 1 or FOLD_QUARTERS
-    int count;
+    int count, ns_steps;
     W16Step step[W16_BATCHES];
 };
-// clip_factor of the norms, with the sums of a fold's quarters formed first; those are asked for a step ahead.
-struct Clip {
-    const Update &u;
-    f32x4 next;
-    TG_DEVICE Clip(const Update &u_) : u(u_) { request(0); }
-    TG_DEVICE bool parts(int n) const { return u.norm_parts != 1 && u.step[n].adam.clip > 0.f; }
-    TG_DEVICE void request(int n) {
-        if (n < u.count && parts(n) && int(threadIdx.x) < u.norm_count)
-            next = reinterpret_cast<const f32x4 *>(u.step[n].norms)[threadIdx.x];
+// Clip factor of step n, by one wave: the sums of a fold's quarters first, then as clip_factor adds them (64 sums at most).
+TG_DEVICE float fold_clip(const Update &u, int n, const f32x4 &part) {
+    const float sum = int(threadIdx.x & 63) < u.norm_count ? (part[0] + part[1]) + (part[2] + part[3]) : 0.f;
+    return fminf(1.f, u.step[n].adam.clip / (sqrtf(wave_sum(0.f + sum)) + 1e-6f));
+}
+TG_DEVICE f32x4 fold_parts(const Update &u, int n) {
+    return int(threadIdx.x & 63) < u.norm_count ? reinterpret_cast<const f32x4 *>(u.step[n].norms)[threadIdx.x & 63] : ZERO;
+}
+// The clip factors of steps first .. first + groups - 1, for all threads; a group's waves have asked for its `part`.
+TG_DEVICE void clip_factors(const Update &u, int first, int groups, const f32x4 &part, float (&clips)[UPDATE_GROUPS], float *waves) {
+    const int group = threadIdx.x >> 8;
+    if (u.norm_parts == 1) { // more norms than a wave has lanes, in launches of one step
+        const float clip = clip_factor(u.step[first].adam.clip, u.step[first].norms, u.norm_count, waves);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            clips[0] = clip;
+    } else if ((threadIdx.x & 255) == 0 || u.step[first].adam.clip > 0.f) {
+        const float clip = u.step[first].adam.clip > 0.f ? fold_clip(u, min(first + group, u.count - 1), part) : 1.f;
+        if ((threadIdx.x & 255) == 0 && group < groups)
+            clips[group] = clip;
     }
-    TG_DEVICE float operator()(int n, float *waves) {
-        const W16Step &step = u.step[n];
-        if (!parts(n))
-            return ::clip_factor(step.adam.clip, step.norms, u.norm_count, waves);
-        const f32x4 part = next;
-        request(n + 1);
-        const float sum = int(threadIdx.x) < u.norm_count ? (part[0] + part[1]) + (part[2] + part[3]) : 0.f;
-        return fminf(1.f, step.adam.clip / (sqrtf(block_sum_256(sum, waves)) + 1e-6f));
+    __syncthreads();
+}
+template <int TILES> TG_DEVICE void iterate(u32x2 (&wide)[2][3][64], int steps, int across, int tile, int lane) {
+    f32x4 x = unpack4(wide[0][tile][lane]); // rows 4 g .. of column 16 tile + c
+    for (int step = 0; step < steps; ++step) {
+        const unsigned char *in = reinterpret_cast<const unsigned char *>(wide[step & 1]) + across;
+        f32x4 row[TILES], gram = ZERO; // A = X X^T, kept in bf16
+#pragma unroll
+        for (int k = 0; k < TILES; ++k)
+            row[k] = unpack4(read_across(in + k * 512));
+#pragma unroll
+        for (int k = 0; k < TILES; ++k)
+            gram = multiply(row[k], row[k], gram);
+        gram = rounded(gram);
+        const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
+        f32x4 work; // -4.775 A + 2.0315 A A
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
+        f32x4 product = multiply(turned(rounded(work)), turned(x));
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            product[r] = fmaf(3.4445f, x[r], product[r]);
+        const u32x2 packed = pack4(product);
+        wide[(step & 1) ^ 1][tile][lane] = packed;
+        x = unpack4(packed);
+        meet();
     }
-};
-TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&waves)[2][4]) {
-    __shared__ __align__(16) u32x2 wide[2][3][64]; // the iterate's tiles of sixteen columns, as the lanes hold them
-    __shared__ float norm_waves[4];
+}
+TG_DEVICE void muon_matrix(const Update &u, int matrix, float (&clips)[UPDATE_GROUPS], float *waves) {
+    __shared__ __align__(16) u32x2 wide[UPDATE_GROUPS][2][3][64]; // the iterate's tiles of sixteen columns, as the lanes hold them
+    __shared__ float norm_waves[UPDATE_GROUPS][4];
     const Layer p = layer_layout(matrix / 5);
     const int type = matrix % 5;
     const int weight = type == 0 ? p.qkv : type == 1 ? p.attention : type == 2 ? p.gate : type == 3 ? p.up : p.down;
     const int rows = (type == 0 || type == 2 || type == 3) ? 48 : 16, cols = type == 4 ? 48 : 16;
-    const int n = rows > cols ? rows : cols, size = rows * cols, tid = threadIdx.x;
+    const int tiles = max(rows, cols) / 16, size = rows * cols, tid = threadIdx.x & 255;
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), groups = blockDim.x >> 8;
+    const int lane = tid & 63, tile = __builtin_amdgcn_readfirstlane(tid >> 6), across = across_offset(lane, true);
     // element tid + 256 k of the matrix is this thread's until the iteration and again behind it; its place in the 16 x n form
-    float next_g[3], m[3], w[3];
+    float m[3], w[3], g[UPDATE_GROUPS][3];
     int place[3];
+    f32x4 part = ZERO;
+    const auto request = [&](int first) {
+        if (u.norm_parts != 1 && first < u.count)
+            part = fold_parts(u, min(first + group, u.count - 1));
+#pragma unroll
+        for (int n = 0; n < UPDATE_GROUPS; ++n)
+            if (n < groups && first + n < u.count)
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    g[n][k] = tid + 256 * k < size ? u.step[first + n].gradient[weight + tid + 256 * k] : 0.f;
+    };
+    request(0);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const int i = weight + tid + 256 * k, line = (tid + 256 * k) / cols, at = tid + 256 * k - line * cols;
         const int row = rows > cols ? at : line, col = rows > cols ? line : at;
         place[k] = (((col >> 4) * 64 + (row >> 2) * 16 + (col & 15)) << 2) + (row & 3);
         const bool mine = tid + 256 * k < size;
-        next_g[k] = mine ? u.step[0].gradient[i] : 0.f, m[k] = mine ? u.momentum[i] : 0.f;
+        m[k] = mine ? u.momentum[i] : 0.f;
         w[k] = mine ? master(u.step[0].from.hi, u.step[0].from.lo, i) : 0.f;
     }
-    const int lane = tid & 63, c = lane & 15, gr = lane >> 4, tile = tid >> 6, tiles = n / 16;
-    const int across = across_offset(lane, true);
-    Clip clip_of(u);
-    for (int at = 0; at < u.count; ++at) {
-        const W16Step &u_step = u.step[at];
-        const MuonArgs &muon = u_step.muon;
-        const float g[3] = {next_g[0], next_g[1], next_g[2]};
-        if (at + 1 < u.count)
+    for (int first = 0; first < u.count; first += groups) {
+        const int steps = min(groups, u.count - first);
+        clip_factors(u, first, steps, part, clips, waves);
+        float squares = 0.f, b[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                next_g[k] = tid + 256 * k < size ? u.step[at + 1].gradient[weight + tid + 256 * k] : 0.f;
-        const float clip = clip_of(at, waves[at & 1]);
-        float squares = 0.f, b[3];
+        for (int n = 0; n < UPDATE_GROUPS; ++n) {
+            if (n >= steps)
+                break;
+            const float rate = u.step[first + n].muon.momentum, clip = clips[n];
+            float sum = 0.f;
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (tid + 256 * k < size) {
-                const float gs = g[k] * clip;
-                m[k] = fmaf(1.f - muon.momentum, fmaf(g[k], clip, -m[k]), m[k]);
-                b[k] = round_bf16(fmaf(muon.momentum, m[k] - gs, gs));
-                squares = fmaf(b[k], b[k], squares);
+            for (int k = 0; k < 3; ++k) {
+                const float gs = g[n][k] * clip;
+                m[k] = fmaf(1.f - rate, fmaf(g[n][k], clip, -m[k]), m[k]);
+                const float mine = round_bf16(fmaf(rate, m[k] - gs, gs));
+                if (tid + 256 * k < size)
+                    sum = fmaf(mine, mine, sum);
+                b[k] = n == group ? mine : b[k];
             }
-        const float norm = fmaxf(round_bf16(sqrtf(block_sum_256(squares, norm_waves))), round_bf16(1e-7f));
+            squares = n == group ? sum : squares;
+        }
+        request(first + groups);
+        squares = wave_sum(squares);
+        if (lane == 0)
+            norm_waves[group][tile] = squares;
+        __syncthreads();
+        const float norm = fmaxf(round_bf16(sqrtf((norm_waves[group][0] + norm_waves[group][1]) + (norm_waves[group][2] + norm_waves[group][3]))),
+                                 round_bf16(1e-7f));
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (tid + 256 * k < size)
-                reinterpret_cast<bf16_t *>(wide[0])[place[k]] = float_to_bf16(b[k] / norm);
+                reinterpret_cast<bf16_t *>(wide[group][0])[place[k]] = float_to_bf16(b[k] / norm);
         __syncthreads();
-        f32x4 x = ZERO; // rows 4 gr .. of column 16 tile + c
-        if (tile < tiles)
-            x = unpack4(wide[0][tile][lane]);
-        for (int step = 0; step < muon.ns_steps; ++step) {
-            if (tile < tiles) {
-                const unsigned char *in = reinterpret_cast<const unsigned char *>(wide[step & 1]) + across;
-                f32x4 row[3], gram = ZERO; // A = X X^T, kept in bf16
+        if (tile >= tiles || group >= steps)
+            for (int step = 0; step < u.ns_steps; ++step)
+                meet();
+        else if (tiles == 3)
+            iterate<3>(wide[group], u.ns_steps, across, tile, lane);
+        else
+            iterate<1>(wide[group], u.ns_steps, across, tile, lane);
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    if (k < tiles)
-                        row[k] = unpack4(read_across(in + k * 512));
+        for (int n = 0; n < UPDATE_GROUPS; ++n) {
+            if (n >= steps)
+                break;
+            const W16Step &step = u.step[first + n];
+            const bf16_t *result = reinterpret_cast<const bf16_t *>(wide[n][u.ns_steps & 1]);
+            const float adjusted = step.muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-step.muon.lr, step.muon.weight_decay, 1.f);
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    if (k < tiles)
-                        gram = multiply(row[k], row[k], gram);
-                gram = rounded(gram);
-                const f32x4 gram_turned = turned(gram), square = multiply(gram_turned, gram_turned);
-                f32x4 work; // -4.775 A + 2.0315 A A
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    work[r] = fmaf(2.0315f, square[r], -4.775f * gram[r]);
-                f32x4 product = multiply(turned(rounded(work)), turned(x));
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    product[r] = fmaf(3.4445f, x[r], product[r]);
-                const u32x2 packed = pack4(product);
-                wide[(step & 1) ^ 1][tile][lane] = packed;
-                x = unpack4(packed);
-            }
-            __syncthreads();
+            for (int k = 0; k < 3; ++k)
+                if (tid + 256 * k < size) {
+                    const int i = weight + tid + 256 * k;
+                    w[k] = fmaf(w[k], keep, -(adjusted * bf16_to_float(result[place[k]])));
+                    if (n == group) {
+                        const uint32_t bits = __float_as_uint(w[k]);
+                        step.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
+                        step.to.lo[i] = uint16_t(bits);
+                    }
+                }
         }
-        const bf16_t *result = reinterpret_cast<const bf16_t *>(wide[muon.ns_steps & 1]);
-        const float adjusted = muon.lr * sqrtf(fmaxf(1.f, float(rows) / float(cols))), keep = fmaf(-muon.lr, muon.weight_decay, 1.f);
+        __syncthreads(); // the next steps' matrices go where these results are read, their clip factors where these are
+    }
+    if (group == 0)
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-            if (tid + 256 * k < size) {
-                const int i = weight + tid + 256 * k;
-                w[k] = fmaf(w[k], keep, -(adjusted * bf16_to_float(result[place[k]])));
-                const uint32_t bits = __float_as_uint(w[k]);
-                u_step.to.hi[i] = uint16_t(bits >> 16); // cuda/ops.cuh:10-14
-                u_step.to.lo[i] = uint16_t(bits);
-            }
-        __syncthreads(); // the next step's matrix goes where this one's result is read
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        if (tid + 256 * k < size)
-            u.momentum[weight + tid + 256 * k] = m[k];
+            if (tid + 256 * k < size)
+                u.momentum[weight + tid + 256 * k] = m[k];
 }
-__global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
-    __shared__ float waves[2][4];
+__global__ __launch_bounds__(256 * UPDATE_GROUPS) void w16_update_kernel(Update u) {
+    __shared__ float clips[UPDATE_GROUPS], waves[4];
     if (int(blockIdx.x) < 5 * u.depth)
-        return muon_matrix(u, blockIdx.x, waves);
+        return muon_matrix(u, blockIdx.x, clips, waves);
     // quads: the embedding's 1024, four for each scale, the head's 1024 (the only ones that decay)
-    const int quad = (blockIdx.x - 5 * u.depth) * 256 + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
+    const int quad = (blockIdx.x - 5 * u.depth) * blockDim.x + threadIdx.x, norm = (quad - V * W / 4) >> 2, norms = 2 * u.depth + 1;
     int at = quad * 4;
     bool decays = false, live = true;
     if (norm >= norms) {
@@ -1511,36 +1549,50 @@ __global__ __launch_bounds__(256) void w16_update_kernel(Update u) {
         const Layer q = layer_layout(norm >> 1);
         at = (norm == 2 * u.depth ? V * W + u.depth * LAYER_SIZE : (norm & 1) ? q.mlp_norm : q.attention_norm) + (quad & 3) * 4;
     }
+    const int groups = blockDim.x >> 8, group = threadIdx.x >> 8;
+    f32x4 g[UPDATE_GROUPS], part = ZERO;
+    const auto request = [&](int first) {
+        if (u.norm_parts != 1 && first < u.count)
+            part = fold_parts(u, min(first + group, u.count - 1));
+#pragma unroll
+        for (int n = 0; n < UPDATE_GROUPS; ++n)
+            if (n < groups && first + n < u.count)
+                g[n] = *reinterpret_cast<const f32x4 *>(u.step[first + n].gradient + at);
+    };
+    request(0);
     f32x4 m = *reinterpret_cast<const f32x4 *>(u.momentum + at), v = *reinterpret_cast<const f32x4 *>(u.variance + at), w;
 #pragma unroll
     for (int k = 0; k < 4; ++k)
         w[k] = master(u.step[0].from.hi, u.step[0].from.lo, at + k);
-    f32x4 next_g = *reinterpret_cast<const f32x4 *>(u.step[0].gradient + at);
-    Clip clip_of(u);
-    for (int n = 0; n < u.count; ++n) {
-        const W16Step &step = u.step[n];
-        const f32x4 g = next_g;
-        if (n + 1 < u.count)
-            next_g = *reinterpret_cast<const f32x4 *>(u.step[n + 1].gradient + at);
-        const float scale = clip_of(n, waves[n & 1]);
-        if (!live)
-            continue;
+    for (int first = 0; first < u.count; first += groups) {
+        const int steps = min(groups, u.count - first);
+        clip_factors(u, first, steps, part, clips, waves);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float mk = m[k], vk = v[k];
-            w[k] = adamw_element(step.adam, decays ? step.adam.weight_decay : 0.f, scale, w[k], mk, vk, g[k]);
-            m[k] = mk, v[k] = vk;
+        for (int n = 0; n < UPDATE_GROUPS; ++n) {
+            if (n >= steps)
+                break;
+            const W16Step &step = u.step[first + n];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float mk = m[k], vk = v[k];
+                w[k] = adamw_element(step.adam, decays ? step.adam.weight_decay : 0.f, clips[n], w[k], mk, vk, g[n][k]);
+                m[k] = mk, v[k] = vk;
+            }
+            const auto half = [&](int k, int shift) { return (__float_as_uint(w[k]) >> shift) & 0xffffu; };
+            if (live) {
+                *reinterpret_cast<u32x2 *>(step.to.hi + at) = u32x2{half(0, 16) | half(1, 16) << 16, half(2, 16) | half(3, 16) << 16};
+                *reinterpret_cast<u32x2 *>(step.to.lo + at) = u32x2{half(0, 0) | half(1, 0) << 16, half(2, 0) | half(3, 0) << 16};
+            }
         }
-        const auto half = [&](int k, int shift) { return (__float_as_uint(w[k]) >> shift) & 0xffffu; };
-        *reinterpret_cast<u32x2 *>(step.to.hi + at) = u32x2{half(0, 16) | half(1, 16) << 16, half(2, 16) | half(3, 16) << 16};
-        *reinterpret_cast<u32x2 *>(step.to.lo + at) = u32x2{half(0, 0) | half(1, 0) << 16, half(2, 0) | half(3, 0) << 16};
+        request(first + groups);
+        __syncthreads(); // the next clip factors go where these are read
     }
     if (!live)
         return;
     *reinterpret_cast<f32x4 *>(u.momentum + at) = m;
     *reinterpret_cast<f32x4 *>(u.variance + at) = v;
 }
-int adam_blocks(int depth) { return (2 * V * W / 4 + 4 * (2 * depth + 1) + 255) / 256; }
+int adam_blocks(int depth, int threads) { return (2 * V * W / 4 + 4 * (2 * depth + 1) + threads - 1) / threads; }
 
 void check_shape(int depth, int batch, int context) {
     require(depth >= 1 && depth <= MAX_DEPTH, "w16: depth must be 1..8");
@@ -1694,11 +1746,14 @@ void w16_gradients(hipStream_t stream, int depth, int batch, int context, const 
 }
 void w16_updates(hipStream_t stream, int depth, float *momentum, float *variance, int norm_count, int norm_parts, int count,
                  const W16Step *steps) {
-    require(norm_parts == 1 || norm_count <= 256, "w16: a fold's norms have a thread each");
+    require(norm_parts == 1 ? count == 1 : norm_count <= 64, "w16: a fold's norms have a lane each");
+    for (int i = 1; i < count; ++i)
+        require(steps[i].muon.ns_steps == steps[0].muon.ns_steps && (steps[i].adam.clip > 0.f) == (steps[0].adam.clip > 0.f), "w16: steps of one launch are alike");
     require(count >= 1 && count <= W16_BATCHES, "w16: too many steps for one launch");
-    Update u{momentum, variance, norm_count, norm_parts, depth, count, {}};
+    Update u{momentum, variance, norm_count, norm_parts, depth, count, steps[0].muon.ns_steps, {}};
     std::copy(steps, steps + count, u.step);
-    hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth + adam_blocks(depth)), dim3(256), 0, stream, u);
+    const int threads = 256 * std::min(count, UPDATE_GROUPS);
+    hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth + adam_blocks(depth, threads)), dim3(threads), 0, stream, u);
     check_hip(hipGetLastError(), "w16_update launch: ");
 }
 
@@ -1713,7 +1768,7 @@ extern "C" int tgk_w16_muon(hipStream_t stream, int depth, uint16_t *weight_hi, 
         AdamArgs adam{};
         adam.clip = clip;
         const W16Weights weights{weight_hi, weight_lo};
-        Update u{momentum, nullptr, norm_count, 1, depth, 1, {}};
+        Update u{momentum, nullptr, norm_count, 1, depth, 1, ns_steps, {}};
         u.step[0] = {weights, weights, gradient, norm_partials, adam, MuonArgs{lr, momentum_rate, weight_decay, ns_steps}};
         hipLaunchKernelGGL(w16_update_kernel, dim3(5 * depth), dim3(256), 0, stream, u); // the matrices' blocks alone
         check_hip(hipGetLastError(), "w16_muon launch: ");
