@@ -443,15 +443,15 @@ struct Engine {
     // Whether the batches of a call of `steps` steps share their launches.  On K streams a step costs the host 32 us of
     // launches and events at least, however small its batch, but steps of one call overlap with those of the next.  A shared launch
     // takes as long as one batch, 48 us at depth 4 and 77 at depth 8, and 8 us of optimizer a step: worth it from two and from 3.25
-    // steps a launch on, while a batch fills few units.  us a step on streams and shared (depth and context equal):
-    //   depth 8, 16 sequences: K = 2 46, 46; 4 37, 27; 16 35, 13; calls of one step at K = 4 38, 81; of five 36, 42
-    //   depth 4, 16 sequences: K = 2 35, 32; 8 34, 13; calls of two 32, 32   640 (40 blocks): K = 4 32, 23
-    //   80 blocks: depth 8, K = 4 46, 44; 8 47, 38; depth 4 35, 30; 36, 24   160 blocks: depth 8, K = 4 60, 69; 8 61, 61; depth 4 36, 41; 38, 38
-    //   depth 8, 10000 sequences, K = 4 379, 395
+    // steps a launch on, while a batch does not fill the units.  us a step on streams and shared (depth and context equal):
+    //   depth 8, 16 sequences: K = 2 46, 46; 4 37, 20; 16 35, 13; calls of one step at K = 4 38, 81; of five 36, 42
+    //   depth 4, 16 sequences: K = 2 35, 32; 8 34, 13; calls of two 32, 32
+    //   113 blocks: depth 8, K = 4 55, 45; depth 4 37, 29   138: depth 8 65, 64   160: depth 8 63, 64; K = 8 63, 58; depth 4, K = 4 40, 37; 8 41, 36
+    //   320 blocks: depth 8, K = 4 112, 114
     bool shares_launches(int steps) const {
         const Config &c = config.base;
         const int K = int(slots.size()), launches = (steps + K - 1) / K;
-        return K == 1 || (w16_blocks(c.batch, c.context) <= 96 && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
+        return K == 1 || (w16_blocks(c.batch, c.context) <= (c.depth == 4 ? 160 : 144) && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
     }
     // Training steps of the width-16 network from `at` on; returns how many.  Batch s reads the weights of version
     // max(floor, s - K + 1), whichever way it is launched.
