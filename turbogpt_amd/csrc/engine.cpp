@@ -114,6 +114,8 @@ struct Engine {
     TgModelConfig config{};
     TgParameterLayout layout{};
     hipStream_t stream = nullptr;
+    hipStream_t second = nullptr; // of large results
+    hipEvent_t branched = nullptr;
     std::vector<void *> allocations;
     size_t allocated_bytes = 0;
     int compute_units = 0;
@@ -216,7 +218,21 @@ struct Engine {
         check_hip(hipMemcpyAsync(device, host, n * sizeof(T), hipMemcpyHostToDevice, stream));
     }
     // results to the caller's memory, behind everything on the engine's stream; returns when they are there
-    void download(const std::vector<ReadbackPiece> &pieces) { readback->fetch(stream, pieces); }
+    void download(const std::vector<ReadbackPiece> &pieces) {
+        size_t bytes = 0;
+        for (const ReadbackPiece &piece : pieces)
+            bytes += piece.bytes;
+        const bool large = bytes >= Readback::LARGE;
+        if (large) {
+            if (!second)
+                check_hip(hipStreamCreate(&second)); // default priority
+            if (!branched)
+                check_hip(hipEventCreateWithFlags(&branched, hipEventDisableTiming));
+            check_hip(hipEventRecord(branched, stream));
+            check_hip(hipStreamWaitEvent(second, branched, 0));
+        }
+        readback->fetch(stream, pieces, large ? second : nullptr);
+    }
     ~Engine() { // cuda/engine_internal.h:28-37
         (void)hipSetDevice(config.base.device);
         for (Slot &slot : slots)
@@ -224,6 +240,8 @@ struct Engine {
                 (void)hipStreamSynchronize(slot.stream);
         if (stream)
             (void)hipStreamSynchronize(stream);
+        if (second)
+            (void)hipStreamSynchronize(second);
         for (void *allocation : allocations)
             (void)hipFree(allocation);
         for (Slot &slot : slots) {
@@ -239,6 +257,10 @@ struct Engine {
         }
         for (hipEvent_t pooled : event_pool)
             (void)hipEventDestroy(pooled);
+        if (branched)
+            (void)hipEventDestroy(branched);
+        if (second)
+            (void)hipStreamDestroy(second);
         if (stream)
             (void)hipStreamDestroy(stream);
     }

@@ -26,7 +26,9 @@ class Readback {
     // Copies the pieces out behind everything already on `stream`, one of the device's; returns when they are in host memory.
     // Calls on several threads run side by side, each with buffers of its own: what is on one engine's stream may take long, and
     // another engine's result does not wait for it.
-    void fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces);
+    // `second`: a stream of the caller's own behind the same work, where every second chunk goes; worth it from LARGE bytes on.
+    static constexpr size_t LARGE = size_t(48) << 20;
+    void fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces, hipStream_t second = nullptr);
 
   private:
     explicit Readback(int device_) : device(device_) {}

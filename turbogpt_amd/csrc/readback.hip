@@ -5,7 +5,8 @@
 // memory (joining the weight halves on the way, which a host loop did before), and several host threads, each with
 // two buffers of its own, copy finished chunks into the caller's pages while the next ones cross the bus.  What is left
 // behind the last chunk is one thread's copy of it (90 us for 2 MiB), so the last 2 MiB are cut in halves down to 512 KiB; not
-// smaller, as every chunk costs the bus 6 us for its event.  The first chunks go out behind what is on the stream, while that still
+// smaller, as every chunk costs its stream 6 us for its event: a large result goes by two streams in turn, so that the bus has one
+// chunk while the other's event is written (a small one's first chunk would only come later).  The first chunks go out behind what is on the stream, while that still
 // runs; the caller's thread alone waits for it, and the others start with the first chunk that is there (the next ones take 37 us
 // each to arrive, longer than a thread takes to start): a batch's 16 MB of gradient and logits at d256 812 us with
 // every thread at its own chunks from the start, 751 so.
@@ -120,7 +121,7 @@ struct Readback::Held {
     }
 };
 
-void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces) {
+void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &pieces, hipStream_t second) {
     struct Chunk {
         const ReadbackPiece *piece;
         size_t offset, bytes;
@@ -146,12 +147,18 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
     check_hip(hipSetDevice(device)); // its events are made here
     const Held held(*this, lanes * depth);
     const auto buffer = [&](size_t l, size_t round) -> const Buffer & { return held.buffers[l * depth + round % depth]; };
+    const auto drain = [&] {
+        (void)hipStreamSynchronize(stream);
+        if (second)
+            (void)hipStreamSynchronize(second);
+    };
     const auto start = [&](size_t l, size_t round) {
         const size_t c = l + round * lanes;
         if (c >= chunks.size())
             return;
-        enqueue(stream, *chunks[c].piece, chunks[c].offset, chunks[c].bytes, buffer(l, round).mapped);
-        check_hip(hipEventRecord(buffer(l, round).written, stream));
+        const hipStream_t on = second && (c & 1) ? second : stream;
+        enqueue(on, *chunks[c].piece, chunks[c].offset, chunks[c].bytes, buffer(l, round).mapped);
+        check_hip(hipEventRecord(buffer(l, round).written, on));
     };
     const auto wait = [&](size_t l, size_t round) { check_hip(hipEventSynchronize(buffer(l, round).written), "readback: "); };
     const auto lane = [&](size_t l) {
@@ -179,7 +186,7 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
                 start(l, round);
         wait(0, 0);
     } catch (...) {
-        (void)hipStreamSynchronize(stream); // nothing may still write to the staging buffers
+        drain(); // nothing may still write to the staging buffers
         throw;
     }
     try {
@@ -194,7 +201,7 @@ void Readback::fetch(hipStream_t stream, const std::vector<ReadbackPiece> &piece
         thread.join();
     for (const std::exception_ptr &failure : failures)
         if (failure) {
-            (void)hipStreamSynchronize(stream); // as above
+            drain(); // as above
             std::rethrow_exception(failure);
         }
 }
