@@ -21,7 +21,7 @@
 // lane ends up holding 4 consecutive n for one m.  Results leave through a wave-private LDS transposition so that stores cover
 // whole row pieces, with the residual / GELU / GELU' epilogues applied in that layout.
 //
-// Forward and input gradients: gemm256_kernel where 256-row tiles fill the compute units, gemm_tile_kernel or (128 x 192
+// Forward and input gradients: gemm256_kernel where it is estimated to be the fastest, gemm_tile_kernel or (128 x 192
 // tiles, k-contiguous operands) gemm64_kernel otherwise, gemm_kernel where 64 does not divide the reduced dimension.
 // Weight gradients: wgrad_list_kernel, wgrad_batch_kernel (several matrices in one launch), gemm64_kernel / gemm_kernel.
 #include "common.h"
@@ -255,6 +255,47 @@ TG_DEVICE void staged_store_bf16(const f32x4 (&acc)[FM][FN][2][2], const u32x4 (
             epilogue.finish(m + 16, n, *reinterpret_cast<const u32x4 *>(get + 1024), aux[1]);
             aux[0] = next[0];
             aux[1] = next[1];
+        }
+}
+// The same from accumulators pinned to the accumulation registers, all 256 of them with 256 x 256 tiles: each 16 x 16 tile is
+// read through assembly where it is rounded.  Plain reads would be hoisted, and the allocation of the whole kernel falls apart
+// (110 to 318 spilled registers; with 192 columns 224 accumulation registers instead of 192).
+template <int FM, int FN, class Epilogue>
+TG_DEVICE void staged_store_pinned(const f32x4 (&acc)[FM][FN][2][2], const u32x4 (&first)[2], unsigned char *mine, const Epilogue &epilogue, int m_base, int n_base, int lane) {
+    const int get_row = lane >> 2, get_chunk = lane & 3;
+    const int row = lane & 15;
+    unsigned char *put = mine + row * 64 + ((lane >> 4) & 1) * 8;
+    const int put_swizzle = (row >> 2) & 3, put_chunk = lane >> 5;
+    const bool wants_aux = epilogue.wants_aux();
+    u32x4 aux[2] = {first[0], first[1]};
+    const unsigned char *get = mine + get_row * 64 + ((get_chunk ^ ((get_row >> 2) & 3)) << 4);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            u32x4 next[2] = {aux[0], aux[1]};
+            if (wants_aux && i * FN + j + 1 < FM * FN)
+                load_aux_pair<FM, FN>(epilogue, i * FN + j + 1, m_base, n_base, lane, next);
+            const int m = m_base + i * 32 + get_row, n = n_base + j * 32 + get_chunk * 8;
+#pragma unroll
+            for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < 2; ++tn) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[e]) : "a"(acc[i][j][tm][tn][e]));
+                    u32x2 packed;
+                    packed.x = pack_bf16(v[0], v[1]);
+                    packed.y = pack_bf16(v[2], v[3]);
+                    *reinterpret_cast<u32x2 *>(put + tm * 1024 + (((2 * tn + put_chunk) ^ put_swizzle) << 4)) = packed;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            epilogue.finish(m, n, *reinterpret_cast<const u32x4 *>(get), aux[0]);
+            epilogue.finish(m + 16, n, *reinterpret_cast<const u32x4 *>(get + 1024), aux[1]);
+            aux[0] = next[0];
+            aux[1] = next[1];
+            __builtin_amdgcn_sched_barrier(0);
         }
 }
 template <int FM, int FN, class Epilogue>
@@ -1221,42 +1262,33 @@ TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64:
     const int row = row0 + (lane & 15), chunk = (ks * 4 + (lane >> 4)) ^ ((row >> 1) & 7);
     return uint32_t(row * 128 + chunk * 16);
 }
-// ---- 256-row tiles, one wave per SIMD: forward and input-gradient products with a long or plain epilogue -------------
+// ---- 256-row tiles, one wave per SIMD: forward and input-gradient products ---------------------------------------------
 // C = A B^T with both operands k-contiguous, a 256 x BN tile per block, four waves of 128 x BN/2 outputs each, one
-// block per compute unit.  What bounds these products is a compute unit's copy path: bytes per flop, whole
-// cache lines per request, and how many requests it keeps in flight.  Hence: 9.1 bytes per kFLOP at BN = 192 without
-// relying on another block's lines in L1; 64 k per stage (every request a whole 128-byte line); and rings of different
-// depth for the two operands - RA slots for A (activations, streamed from beyond the L2: a copy has two stages to
-// land) and two for B (the weights, mostly L2 hits: one stage).  With a lone wave per SIMD the fragments of the
-// next 32-k step are read into a second register set between the matrix instructions of the current one:
-//   first half of stage g : matrix instructions on (g, k 0..31), fragment reads of (g, k 32..63)
+// block per compute unit.  What bounds these products is a compute unit's copy path: bytes per flop (7.8 per kFLOP with 256
+// columns, 9.1 with 192, 11.7 with 128), whole cache lines per request, and how many requests it keeps in flight.  Hence 64 k per
+// stage (every request a whole 128-byte line), and two rings, whose copies go out over the two halves of a stage in turn: three
+// slots for A (activations, streamed from beyond the L2: a copy has a whole stage to land) and two for B (the weights, mostly
+// L2 hits: half a stage).  With a lone wave per SIMD the fragments of the next 32-k step are read into a second register set
+// between the matrix instructions of the current one:
+//   first half of stage g : matrix instructions on (g, k 0..31), fragment reads of (g, k 32..63), copies of A's stage g + 2
 //   wait (all but A's youngest stage), barrier: stage g + 1 is visible, nobody reads stage g's slots any more
-//   second half           : matrix instructions on (g, k 32..63), copies of B's stage g + 2 and A's stage g + RA,
-//                           fragment reads of (g + 1, k 0..31)
-// The loop is unrolled over the rings' common period P, so that every LDS address is a constant, and the reduced
-// dimension is a multiple of 64 P.  Two instantiations:
-//   BN = 192, RA = 3 (P = 6, 144 KB of rings + 8 KB for the epilogue): widths that 192 and 384 divide;
-//   BN = 128, RA = 4 (P = 4, 160 KB of rings: all of the LDS): widths that 128 and 256 divide (d_model 1024).  Three
-//   slots would do for A as far as latency goes - the fourth only makes the period a power of two.  The epilogue's
-//   buffers then lie in the first 8 KB of the A slot that the tile's last stage leaves, and the two copies per wave that
-//   refill those rows are held back until the wave's epilogue is over (each wave then copies the rows under its own
-//   buffer, so no barrier is needed; in their place copies 2 and 3 of the stage go out twice, which keeps the loop
-//   free of branches and every wait count fixed).
-template <int BN, int RA, class Epilogue>
+//   second half           : matrix instructions on (g, k 32..63), fragment reads of (g + 1, k 0..31), copies of B's stage g + 2
+// A's slots turn by an addition, B's are unrolled, so the reduced dimension is a multiple of 128.  With 256 columns the rings
+// are all of the LDS: the epilogue's buffers lie in the A slot that the tile's last stage leaves, each wave's in rows that
+// its own copies overwrite next, so it needs no barrier.  The accumulators stay in the accumulation registers throughout.
+// Measured at 16384 tokens: the products of d_model 1024 into or out of 1024 columns 71 to 73 us on average with 256 columns (84 to
+// 86 with 128 columns and a ring of four slots whose copies all went out in second halves); d_model 768's with 192 columns -4 %
+// from the same change of the copies (A and B together in second halves, a period of six unrolled stages).
+template <int BN, class Epilogue>
 __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restrict__ A, int lda,
                                                        const bf16_t *__restrict__ B, int ldb, int k_periods,
                                                        int tiles_n, int tiles_total, int xcd_cols,
                                                        Epilogue epilogue) {
     constexpr int BM = 256;
-    constexpr int P = RA % 2 ? 2 * RA : RA; // stages per period of the two rings (RA slots for A, two for B)
     constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, AF = 2 * FM, BF = 2 * FN, MFMAS = AF * BF;
-    constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, B_RING = RA * A_BYTES, BUFFERS = B_RING + 2 * B_BYTES;
-    // Where the rings fill the LDS, the epilogue's four transposition buffers (8 KB) lie in the first rows of the A slot
-    // that a tile's last stage leaves, and the two copies per wave that would refill those rows wait for the epilogue.
-    constexpr bool ALIAS = BUFFERS + 4 * 2048 > 160 * 1024;
-    static_assert(!ALIAS || (P == RA && BUFFERS <= 160 * 1024), "the aliased buffers assume the last stage's slot is the ring's last");
-    constexpr int LA = BM * 128 / 4096, LB = BN * 128 / 4096, LOADS = LA + LB; // copies per wave and stage
-    constexpr int READ_EVERY = MFMAS / (AF + BF), COPY_EVERY = MFMAS / LOADS;
+    constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, B_RING = 3 * A_BYTES;
+    constexpr int LA = BM * 128 / 4096, LB = BN * 128 / 4096; // copies per wave and stage
+    constexpr int READ_EVERY = MFMAS / (AF + BF);
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t smem_base = lds_address(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1279,10 +1311,12 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         n0 = tile_n * BN;
     };
 
-    // ---- producers: A three stages ahead of the consumer, B two --------------------------------------------------
-    const int copy_row = lane >> 3, copy_chunk = (lane & 7) ^ ((((wave & 1) * 4) + (lane >> 4)) & 7);
-    const uint32_t la = uint32_t(copy_row * lda + copy_chunk * 8) * 2, lb = uint32_t(copy_row * ldb + copy_chunk * 8) * 2;
-    const int64_t a_rows32 = int64_t(32) * lda * 2, b_rows32 = int64_t(32) * ldb * 2;
+    // ---- producers, both two stages ahead of the consumer ------------------------------------------------------------
+    // A wave's copies n and n + 1 (n even) are the 16 rows 16 w .. 16 w + 15 of the stage's 64-row group n / 2.
+    const int copy_row = lane >> 3, even_chunk = (lane & 7) ^ (lane >> 4), odd_chunk = even_chunk ^ 4;
+    const uint32_t la[2] = {uint32_t(copy_row * lda + even_chunk * 8) * 2, uint32_t((copy_row + 8) * lda + odd_chunk * 8) * 2};
+    const uint32_t lb[2] = {uint32_t(copy_row * ldb + even_chunk * 8) * 2, uint32_t((copy_row + 8) * ldb + odd_chunk * 8) * 2};
+    const int64_t a_rows64 = int64_t(64) * lda * 2, b_rows64 = int64_t(64) * ldb * 2;
     // wave-uniform: the stage either producer copies next (this wave's first row of it), the first stage of the tile
     // after the current one, and the bytes from one stage to the next (0 once the list is exhausted: the copies go
     // on, re-reading a stage into slots nobody consumes, and the loop stays straight-line code)
@@ -1291,8 +1325,8 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
     auto tile_origin = [&](int item, const char *&a, const char *&b) {
         int m0, n0;
         locate(item, m0, n0);
-        a = reinterpret_cast<const char *>(A + int64_t(m0 + wave * 8) * lda);
-        b = reinterpret_cast<const char *>(B + int64_t(n0 + wave * 8) * ldb);
+        a = reinterpret_cast<const char *>(A + int64_t(m0 + wave * 16) * lda);
+        b = reinterpret_cast<const char *>(B + int64_t(n0 + wave * 16) * ldb);
     };
     auto prepare_next = [&](int item) { // keeps the current origins when there is no further tile
         if (item < tiles_total)
@@ -1300,18 +1334,18 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         else
             next_step = 0;
     };
-    auto copy_a = [&](int n, int slot) __attribute__((always_inline)) {
-        async_copy16(smem_base + uint32_t(slot * A_BYTES + (n * 4 + wave) * 1024), pa_at + n * a_rows32, la);
+    auto copy_a = [&](int n, uint32_t slot) __attribute__((always_inline)) {
+        async_copy16(smem_base + slot + uint32_t((n >> 1) * 8192 + wave * 2048 + (n & 1) * 1024), pa_at + (n >> 1) * a_rows64, la[n & 1]);
     };
     auto copy_b = [&](int n, int slot) __attribute__((always_inline)) {
-        async_copy16(smem_base + uint32_t(B_RING + slot * B_BYTES + (n * 4 + wave) * 1024), pb_at + n * b_rows32, lb);
+        async_copy16(smem_base + uint32_t(B_RING + slot * B_BYTES + (n >> 1) * 8192 + wave * 2048 + (n & 1) * 1024),
+                     pb_at + (n >> 1) * b_rows64, lb[n & 1]);
     };
     if (int(blockIdx.x) >= tiles_total)
         return;
     tile_origin(blockIdx.x, pa_at, pb_at);
     a_next = pa_at, b_next = pb_at;
     prepare_next(blockIdx.x + stride);
-    // stages 0 and 1 of both, then A's further stages (so that A's youngest stages are the last ones issued, as in the loop)
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -1319,43 +1353,33 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
             copy_b(n, s);
 #pragma unroll
         for (int n = 0; n < LA; ++n)
-            copy_a(n, s);
+            copy_a(n, s * A_BYTES);
         pa_at += pa_step, pb_at += pb_step;
-    }
-#pragma unroll
-    for (int s = 2; s < RA; ++s) {
-#pragma unroll
-        for (int n = 0; n < LA; ++n)
-            copy_a(n, s);
-        pa_at += pa_step;
     }
 
     // ---- consumer ----------------------------------------------------------------------------------------------------
-    uint32_t fa_at[2], fa_far[2], fb_at[2]; // fragment 0 of either 32-k step; fragment i lies 2048 i bytes further on
+    uint32_t fa_at[2], fb_at[2]; // fragment 0 of either 32-k step; fragment i lies 2048 i bytes further on
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
         fa_at[ks] = kc64_frag16_offset(wm, ks, lane);
-        fa_far[ks] = fa_at[ks] + 2 * A_BYTES; // slot 2 lies beyond a ds_read's 16-bit offset
         fb_at[ks] = B_RING + kc64_frag16_offset(wn, ks, lane);
     }
-    auto read_fragment = [&](bf16x8 (&fa)[AF], bf16x8 (&fb)[BF], int slot_a, int slot_b, int ks, int f)
+    auto read_fragment = [&](bf16x8 (&fa)[AF], bf16x8 (&fb)[BF], uint32_t slot_a, int slot_b, int ks, int f)
                              __attribute__((always_inline)) {
         if (f < AF)
-            fa[f] = slot_a >= 2 ? *reinterpret_cast<const bf16x8 *>(smem + fa_far[ks] + (slot_a - 2) * A_BYTES + f * 2048)
-                                : *reinterpret_cast<const bf16x8 *>(smem + fa_at[ks] + slot_a * A_BYTES + f * 2048);
+            fa[f] = *reinterpret_cast<const bf16x8 *>(smem + (fa_at[ks] + slot_a) + f * 2048);
         else
             fb[f - AF] = *reinterpret_cast<const bf16x8 *>(smem + fb_at[ks] + slot_b * B_BYTES + (f - AF) * 2048);
     };
     f32x4 acc[FM][FN][2][2];
     bool last_period = k_periods == 1; // the consumer is in a tile's last period of stages
     bool behind_epilogue = false;
-    static_assert(LA + FM * FN * Epilogue::MEMORY_OPS_PER_BLOCK + (ALIAS ? 2 : 0) < 64, "the wait count has six bits");
-    // One 32-k step on `cur`; meanwhile the fragments of (next slots, next_ks) are read into `next`, and, in a
-    // stage's second half, the copies go out: B first, A behind it (so that a wait can leave A's youngest stage out).
-    auto half = [&](auto copy_tag, int next_a_slot, int next_b_slot, int next_ks, int copy_a_slot, int copy_b_slot,
-                    bool hold_back, const bf16x8 (&cur_a)[AF], const bf16x8 (&cur_b)[BF], bf16x8 (&next_a)[AF],
-                    bf16x8 (&next_b)[BF]) __attribute__((always_inline)) {
-        constexpr bool COPY = decltype(copy_tag)::value;
+    uint32_t slot = 0, next_slot = A_BYTES, free_slot = 2 * A_BYTES; // A's slots: this stage's, the next one's, the one before's
+    // One 32-k step on `cur`; meanwhile the fragments of (slots, ks) are read into `next` and one operand's copies go out.
+    auto half = [&](auto copy_tag, uint32_t slot_a, int slot_b, int ks, int copy_slot, const bf16x8 (&cur_a)[AF],
+                    const bf16x8 (&cur_b)[BF], bf16x8 (&next_a)[AF], bf16x8 (&next_b)[BF]) __attribute__((always_inline)) {
+        constexpr bool COPY_A = decltype(copy_tag)::value;
+        constexpr int COPIES = COPY_A ? LA : LB, COPY_EVERY = MFMAS / COPIES;
 #pragma unroll
         for (int j = 0; j < BF; ++j)
 #pragma unroll
@@ -1366,34 +1390,29 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
                              : "v"(cur_b[j]), "v"(cur_a[i]));
                 const int q = j * AF + i;
                 if (q % READ_EVERY == 0 && q / READ_EVERY < AF + BF)
-                    read_fragment(next_a, next_b, next_a_slot, next_b_slot, next_ks, q / READ_EVERY);
-                if (COPY && q % COPY_EVERY == 1 % COPY_EVERY && q / COPY_EVERY < LOADS) {
-                    const int n = q / COPY_EVERY;
-                    if (n < LB)
-                        copy_b(n, copy_b_slot);
-                    else if (ALIAS && n - LB < 2) // held back: the rows under the epilogue's buffers; copy 2 or 3 goes twice instead
-                        copy_a(hold_back ? n - LB + 2 : n - LB, copy_a_slot);
+                    read_fragment(next_a, next_b, slot_a, slot_b, ks, q / READ_EVERY);
+                if (q % COPY_EVERY == 1 && q / COPY_EVERY < COPIES) {
+                    if (COPY_A)
+                        copy_a(q / COPY_EVERY, free_slot);
                     else
-                        copy_a(n - LB, copy_a_slot);
+                        copy_b(q / COPY_EVERY, copy_slot);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
     };
-    // stage g = STAGE (mod P): A slot g % RA, B slot g % 2
+    constexpr int BEHIND = LA + FM * FN * Epilogue::MEMORY_OPS_PER_BLOCK;
     auto stage = [&](auto stage_tag, bf16x8 (&fa0)[AF], bf16x8 (&fb0)[BF], bf16x8 (&fa1)[AF], bf16x8 (&fb1)[BF])
                      __attribute__((always_inline)) {
-        constexpr int G = decltype(stage_tag)::value, SA = G % RA, SB = G % 2;
-        // In a tile's last period the producers cross into the next tile: A with the copies of stage P - RA (RA
-        // stages ahead), B with those of stage P - 2.  Selects, not branches.
-        if (G == P - RA && last_period)
-            pa_at = a_next, pa_step = next_step;
-        if (G == P - 2 && last_period)
-            pb_at = b_next, pb_step = next_step;
-        half(std::false_type{}, SA, SB, 1, 0, 0, false, fa0, fb0, fa1, fb1);
+        constexpr int G = decltype(stage_tag)::value; // B's slot
+        // In a tile's last period the producers cross into the next tile.  Selects, not branches.
+        if (G == 0 && last_period)
+            pa_at = a_next, pb_at = b_next, pa_step = pb_step = next_step;
+        half(std::true_type{}, slot, G, 1, 0, fa0, fb0, fa1, fb1);
+        pa_at += pa_step;
         // Everything but A's youngest stage has landed.  A wave's loads and stores retire in order through one counter;
-        // behind a tile's epilogue its loads and stores are the youngest operations, and their number is known.
+        // behind a tile's epilogue its loads and stores stand between B's youngest stage and A's, and their number is known.
         if (G == 0 && behind_epilogue)
-            wait_vmcnt<LA + FM * FN * Epilogue::MEMORY_OPS_PER_BLOCK + (ALIAS ? 2 : 0)>();
+            wait_vmcnt<(BEHIND < 63 ? BEHIND : 63)>();
         else
             wait_vmcnt<LA>();
         if (G == 0)
@@ -1401,9 +1420,10 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): and this wave's reads of this stage are done
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        // copies: B's stage g + 2 into B slot g % 2, A's stage g + 3 into A slot g % 3 (the slots this stage leaves)
-        half(std::true_type{}, (SA + 1) % RA, SB ^ 1, 0, SA, SB, ALIAS && G == P - 1 && last_period, fa1, fb1, fa0, fb0);
-        pa_at += pa_step, pb_at += pb_step;
+        half(std::false_type{}, next_slot, G ^ 1, 0, G, fa1, fb1, fa0, fb0);
+        pb_at += pb_step;
+        const uint32_t left = slot;
+        slot = next_slot, next_slot = free_slot, free_slot = left;
     };
     const bf16x8 zeros = {0, 0, 0, 0, 0, 0, 0, 0};
     auto clear = [&]() __attribute__((always_inline)) {
@@ -1418,23 +1438,16 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
                                  : "v"(zeros)); // zeroed in place, wait states included (see wgrad_list_kernel)
     };
     bf16x8 fa0[AF], fb0[BF], fa1[AF], fb1[BF];
-    wait_vmcnt<(RA - 1) * LA + LB>(); // stage 0
+    wait_vmcnt<LA + LB>(); // stage 0
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int f = 0; f < AF + BF; ++f)
         read_fragment(fa0, fb0, 0, 0, 0, f);
-    unsigned char *mine = smem + (ALIAS ? (RA - 1) * A_BYTES : BUFFERS) + wave * 2048;
     int item = blockIdx.x, periods_left = k_periods;
     clear();
     for (;;) {
         stage(std::integral_constant<int, 0>{}, fa0, fb0, fa1, fb1);
         stage(std::integral_constant<int, 1>{}, fa0, fb0, fa1, fb1);
-        stage(std::integral_constant<int, 2>{}, fa0, fb0, fa1, fb1);
-        stage(std::integral_constant<int, 3>{}, fa0, fb0, fa1, fb1);
-        if constexpr (P == 6) {
-            stage(std::integral_constant<int, 4>{}, fa0, fb0, fa1, fb1);
-            stage(std::integral_constant<int, 5>{}, fa0, fb0, fa1, fb1);
-        }
         if (--periods_left) {
             last_period = periods_left == 1;
             continue;
@@ -1445,20 +1458,10 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
         if (epilogue.wants_aux())
             load_aux_pair<FM, FN>(epilogue, 0, m0 + wm, n0 + wn, lane, aux);
-        staged_store_bf16<FM, FN>(acc, aux, mine, epilogue, m0 + wm, n0 + wn, lane);
-        behind_epilogue = true; // the stores stay in flight under the next tile's first stage
-        if (ALIAS) {
-            // the two copies held back in the last stage, as the rows that lie under this wave's own buffer (rows 16 w
-            // to 16 w + 15 of the stage: nobody else's buffer is touched, so no barrier); the producer has moved on
-            // by one stage since
-            __builtin_amdgcn_s_waitcnt(0xc07f); // this wave's reads of its buffer have returned
-#pragma unroll
-            for (int n = 0; n < 2; ++n) { // 1 KB piece 2 w + n of the stage: its rows' swizzle term goes by n, not by w
-                const int chunk = (lane & 7) ^ ((n * 4 + (lane >> 4)) & 7);
-                async_copy16(smem_base + uint32_t((RA - 1) * A_BYTES + (2 * wave + n) * 1024),
-                             pa_at - pa_step + int64_t(wave + n) * 8 * lda * 2, uint32_t(copy_row * lda + chunk * 8) * 2);
-            }
-        }
+        unsigned char *mine = smem + free_slot + wave * 2048; // rows that nobody but this wave will overwrite
+        staged_store_pinned<FM, FN>(acc, aux, mine, epilogue, m0 + wm, n0 + wn, lane);
+        __builtin_amdgcn_s_waitcnt(0xc07f); // this wave's reads of its buffer have returned
+        behind_epilogue = true;             // the stores stay in flight under the next tile's first stage
         item += stride;
         if (item >= tiles_total)
             break;
@@ -2104,8 +2107,8 @@ int compute_units() {
 enum Tile { TILE_NONE, TILE_128x128, TILE_128x192 };
 // 128x192, 3 stages (60 KiB of LDS, <= 186 VGPRs): two blocks are resident per CU, so one block's
 // MFMAs cover the other's epilogue, barrier and copy-issue gaps; at N = 768 / 2304 / 3072 and
-// M = 16384 it gives 512 / 1536 / 2048 tiles, whole multiples of the 512 resident blocks.  Measured
-// on MI355X it beats a 256x192 single-block-per-CU variant on every training shape.
+// M = 16384 it gives 512 / 1536 / 2048 tiles, whole multiples of the 512 resident blocks.  Where tiles of 256 rows
+// are the faster ones: columns_of_256.
 // 128x128, 4 stages: shapes that 192 does not divide.
 Tile choose_tile(int rows, int cols) {
     if (rows % 128 == 0 && cols % 192 == 0)
@@ -2209,32 +2212,44 @@ void launch_gemm64(hipStream_t stream, Tile tile, const bf16_t *A, int lda, cons
         launch_gemm64_tile<128, AKC, BKC>(stream, A, lda, B, ldb, M, N, K, splits, epilogue);
 }
 
-// The 256-row kernels take products with a plain or residual epilogue whose tiles fill the compute units a whole
-// number of times (or nearly): one block per unit, nothing to cover a tail or a long epilogue (the GELU epilogues
-// stay with gemm64_kernel, where the second block of a unit multiplies meanwhile).
-bool takes_256(int M, int N, int K, int bn, int k_period) {
-    if (M % 256 || N % bn || K % k_period)
-        return false;
-    const int tiles = (M / 256) * (N / bn), units = compute_units();
-    const int rounds = (tiles + units - 1) / units;
-    return tiles * 10 >= rounds * units * 9; // at least 90 % of the last round filled
+// Which products the 256-row kernel takes, and with which width: the least of estimated costs in columns times k.  Each of
+// a unit's rounds of tiles costs, per k, its width and a share that does not depend on it, and an epilogue by outputs; the
+// 128-row blocks, two to a unit, cost the same by pairs, where a lone block takes more than half a pair's time.  The constants are
+// a fit to 600 products of 2048 to 16384 rows at the widths of models of 256 to 1024 columns, plain, residual and with either
+// GELU: the choice is within 0.6 % of the best of the four (geometric mean, at worst 6 %), where taking 192 or else 128 columns for
+// tiles that fill 90 % of the last round was within 3.0 %.  Products of less than 768 of k (512 with a GELU) don't pay for a lone
+// block's cold start, nor do 128 columns of less than 768 unless they fill the units and 192 does not divide the width.
+// The forward GELU of widths that 192 divides stays with the 128 x 192 blocks: alone they are as fast (16384 x 3072 x 768 99.0 us,
+// with 256 columns 97.9), but inside a step the second block covers the writes of two results (eight steps at d_model 768 183.0 ms,
+// with 256 columns 187.1).
+int columns_of_256(int M, int N, int K, int mode) { // 0: the 128-row blocks
+    const bool gelu = mode != EPI_PLAIN && mode != EPI_RESIDUAL;
+    const int units = compute_units(), wide = N % 192 == 0 ? 192 : 128;
+    const int64_t blocks = int64_t(M / 128) * (N / wide), per_unit = (blocks + units - 1) / units;
+    if (M % 256 || K % 128 || per_unit < 2 || K < (gelu ? 512 : 768))
+        return 0;
+    if (gelu && mode != EPI_GELU_BWD && wide == 192)
+        return 0;
+    double best = (double(per_unit / 2) + per_unit % 2 * 0.83) *
+                  (double(K) * (wide + (gelu ? 100 : 86)) + wide * (gelu ? 810. : 410.));
+    int columns = 0;
+    for (int bn : {128, 192, 256}) {
+        if (N % bn)
+            continue;
+        const int64_t tiles = int64_t(M / 256) * (N / bn), rounds = (tiles + units - 1) / units;
+        if (bn == 128 && K < 768 && (wide == 192 || tiles * 10 < rounds * units * 9))
+            continue;
+        const double cost = double(rounds) * (double(K) * (bn + 52) + bn * (gelu ? 1050. : 480.));
+        if (cost < best)
+            best = cost, columns = bn;
+    }
+    return columns;
 }
-bool takes_256x192(int M, int N, int K, int mode) {
-    return (mode == EPI_PLAIN || mode == EPI_RESIDUAL) && takes_256(M, N, K, 192, 384);
-}
-// Where the 192-wide tile does not fit, with every epilogue: what the 128-wide tile competes with there is two
-// 128 x 128 blocks per unit, and its fewer operand bytes per flop outweigh the uncovered GELU epilogue (measured at
-// d_model 1024: +17 % and +19 % on the two GELU launches; at widths the 192-wide tiles take, gemm64_kernel's 128 x 192
-// blocks keep them)
-bool takes_256x128(int M, int N, int K) {
-    return !takes_256(M, N, K, 192, 384) && takes_256(M, N, K, 128, 256);
-}
-template <int BN = 192, int RA = 3, class Epilogue>
+template <int BN, class Epilogue>
 void launch_gemm256(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                     const Epilogue &epilogue) {
-    auto kernel = gemm256_kernel<BN, RA, Epilogue>;
-    constexpr size_t rings = RA * 256 * 128 + 2 * BN * 128, lds = rings + 4 * 2048 > 160 * 1024 ? rings : rings + 4 * 2048;
-    constexpr int P = RA % 2 ? 2 * RA : RA;
+    auto kernel = gemm256_kernel<BN, Epilogue>;
+    constexpr size_t lds = 3 * 256 * 128 + 2 * BN * 128;
     static std::atomic<bool> configured[MAX_DEVICES];
     const int device = current_device();
     if (!configured[device].load(std::memory_order_acquire)) {
@@ -2245,31 +2260,24 @@ void launch_gemm256(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *
     }
     const int tiles_m = M / 256, tiles_n = N / BN, tiles = tiles_m * tiles_n;
     const int units = compute_units(), blocks = tiles < units ? tiles : units;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, A, lda, B, ldb, K / (64 * P), tiles_n, tiles,
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, A, lda, B, ldb, K / 128, tiles_n, tiles,
                        xcd_columns(tiles_m, tiles_n, 256, BN, K, blocks), epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
+template <int BN>
 void launch_gemm256_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
                          const EpilogueBf16 &e) {
-    if (e.mode == EPI_RESIDUAL)
-        launch_gemm256(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
-    else
-        launch_gemm256(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_PLAIN>{e});
-}
-// 256 x 128 tiles, A ring of four slots (period of four stages: reduced dimensions that 256 divides)
-void launch_gemm256x128_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
-                             const EpilogueBf16 &e) {
     switch (e.mode) {
     case EPI_RESIDUAL:
-        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
+        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
     case EPI_GELU:
-        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
+        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
     case EPI_GELU_ONLY:
-        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
+        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
     case EPI_GELU_BWD:
-        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_BWD>{e});
+        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_BWD>{e});
     default:
-        return launch_gemm256<128, 4>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_PLAIN>{e});
+        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_PLAIN>{e});
     }
 }
 
@@ -2473,6 +2481,22 @@ void launch_block_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf16_
     }
 }
 
+// C = A B^T with both operands k-contiguous and an epilogue
+void launch_forward(hipStream_t stream, Tile tile, const bf16_t *A, int lda, const bf16_t *B, int ldb, int M, int N, int K,
+                    const EpilogueBf16 &e) {
+    const int columns = near(lda, ldb) ? columns_of_256(M, N, K, e.mode) : 0;
+    if (columns == 256)
+        launch_gemm256_bf16<256>(stream, A, lda, B, ldb, M, N, K, e);
+    else if (columns == 192)
+        launch_gemm256_bf16<192>(stream, A, lda, B, ldb, M, N, K, e);
+    else if (columns == 128)
+        launch_gemm256_bf16<128>(stream, A, lda, B, ldb, M, N, K, e);
+    else if (takes_64(tile, K) && near(lda, ldb))
+        launch_block_bf16<true>(stream, A, lda, B, ldb, M, N, K, e);
+    else
+        dispatch_gemm<true, true>(stream, tile, A, lda, B, ldb, M, N, K, 1, e);
+}
+
 template <int BM, int BN, int S, int GROUPS> void launch_wgrad_tiles(hipStream_t stream, const WgradTiles &w, int blocks) {
     auto kernel = wgrad_tiles_kernel<BM, BN, S, GROUPS>;
     constexpr size_t lds = GROUPS * S * (BM + BN) * 128;
@@ -2592,14 +2616,7 @@ void gemm_fwd(hipStream_t stream, int M, int N, int K, const bf16_t *X, int ldx,
         check_operand(e.aux, e.ld_aux, "residual");
     if (e.out2)
         check_operand(e.out2, e.ld_out2, "gelu_out");
-    if (takes_256x192(M, N, K, e.mode))
-        launch_gemm256_bf16(stream, X, ldx, W, ldw, M, N, K, e);
-    else if (takes_256x128(M, N, K))
-        launch_gemm256x128_bf16(stream, X, ldx, W, ldw, M, N, K, e);
-    else if (takes_64(tile, K) && near(ldx, ldw))
-        launch_block_bf16<true>(stream, X, ldx, W, ldw, M, N, K, e);
-    else
-        dispatch_gemm<true, true>(stream, tile, X, ldx, W, ldw, M, N, K, 1, e);
+    launch_forward(stream, tile, X, ldx, W, ldw, M, N, K, e);
 }
 } // namespace
 
@@ -2693,14 +2710,7 @@ extern "C" int tgk_gemm_dgrad_t(hipStream_t stream, int M, int N, int K, const u
             e.aux = gelu_pre, e.ld_aux = ldu, e.mode = EPI_GELU_BWD;
         }
         // C[m][i] = sum_o dY[m][o] Wt[i][o]: the forward product with (rows, reduced) = (K, N)
-        if (takes_256x192(M, K, N, e.mode))
-            launch_gemm256_bf16(stream, dY, lddy, Wt, ldwt, M, K, N, e);
-        else if (takes_256x128(M, K, N))
-            launch_gemm256x128_bf16(stream, dY, lddy, Wt, ldwt, M, K, N, e);
-        else if (takes_64(tile, N) && near(lddy, ldwt))
-            launch_block_bf16<true>(stream, dY, lddy, Wt, ldwt, M, K, N, e);
-        else
-            dispatch_gemm<true, true>(stream, tile, dY, lddy, Wt, ldwt, M, K, N, 1, e);
+        launch_forward(stream, tile, dY, lddy, Wt, ldwt, M, K, N, e);
     });
 }
 
