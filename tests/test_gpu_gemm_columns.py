@@ -1,6 +1,6 @@
 """Products on 256-row tiles (csrc/gemm.hip, gemm256_kernel) of each width, at the edges of its choice: a round that is partly
-filled, several rounds, odd numbers of 128-k periods, a reduced dimension that only the GELU epilogues take; with the checks and
-bounds of test_256x128_tiles_rows_sampled, bit for bit against the kernels for k-strided weights."""
+filled, several rounds, odd numbers of 128-k periods, a reduced dimension that only the GELU epilogues take, half a tile of rows at
+the end; with the checks and bounds of test_256x128_tiles_rows_sampled, bit for bit against the kernels for k-strided weights."""
 import pytest
 
 import test_gpu_gemm as gemm
@@ -14,6 +14,9 @@ pytestmark = gemm.pytestmark
                                           (12288, 768, 896, True),     # 192 tiles of 192 columns; backward: 336 of 128
                                           (10240, 640, 768, False),    # 200 tiles of 128 columns
                                           (16384, 1024, 640, True),    # only with a GELU
-                                          (16640, 1280, 1024, False)])  # 65 rows of tiles: 325 of 256 columns
+                                          (16640, 1280, 1024, False),  # 65 rows of tiles: 325 of 256 columns
+                                          # a last row of tiles of 128 rows
+                                          (8320, 896, 896, True), (12416, 768, 768, False), (10368, 1024, 1152, True),
+                                          (4224, 3072, 768, True)])
 def test_columns(orc, M, N, K, residual):
     gemm.test_256x128_tiles_rows_sampled(orc, M, N, K, residual)

@@ -1273,6 +1273,7 @@ TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64:
 //   first half of stage g : matrix instructions on (g, k 0..31), fragment reads of (g, k 32..63), copies of A's stage g + 2
 //   wait (all but A's youngest stage), barrier: stage g + 1 is visible, nobody reads stage g's slots any more
 //   second half           : matrix instructions on (g, k 32..63), fragment reads of (g + 1, k 0..31), copies of B's stage g + 2
+// The last row of tiles may be 128 rows high; the two waves without rows then skip the epilogue.
 // A's slots turn by an addition, B's are unrolled, so the reduced dimension is a multiple of 128.  With 256 columns the rings
 // are all of the LDS: the epilogue's buffers lie in the A slot that the tile's last stage leaves, each wave's in rows that
 // its own copies overwrite next, so it needs no barrier.  The accumulators stay in the accumulation registers throughout.
@@ -1281,7 +1282,7 @@ TG_DEVICE uint32_t kc64_frag16_offset(int row0, int ks, int lane) { // TileKC64:
 // from the same change of the copies (A and B together in second halves, a period of six unrolled stages).
 template <int BN, class Epilogue>
 __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restrict__ A, int lda,
-                                                       const bf16_t *__restrict__ B, int ldb, int k_periods,
+                                                       const bf16_t *__restrict__ B, int ldb, int M, int k_periods,
                                                        int tiles_n, int tiles_total, int xcd_cols,
                                                        Epilogue epilogue) {
     constexpr int BM = 256;
@@ -1303,7 +1304,8 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
             tile_m = (xcd / xcd_cols) * rows + index / cols;
             tile_n = (xcd % xcd_cols) * cols + index % cols;
         } else {
-            const int logical = (tiles_total & 7) == 0 ? (item & 7) * (tiles_total >> 3) + (item >> 3) : item;
+            // neighbours on one XCD, also where 8 does not divide the tiles: 8320 x 896 x 1792 27.1 us, in order of the items 38.9
+            const int logical = xcd_contiguous(item, tiles_total);
             tile_m = logical / tiles_n;
             tile_n = logical % tiles_n;
         }
@@ -1322,20 +1324,23 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
     // on, re-reading a stage into slots nobody consumes, and the loop stays straight-line code)
     const char *pa_at = nullptr, *pb_at = nullptr, *a_next = nullptr, *b_next = nullptr;
     int64_t pa_step = 128, pb_step = 128, next_step = 128;
-    auto tile_origin = [&](int item, const char *&a, const char *&b) {
+    // The last row of tiles may be 128 rows high: its copies of the other 128 read the first ones again.
+    int64_t pa_far = 0, far_next = 0; // from the tile's first row to its row 128, or 0
+    auto tile_origin = [&](int item, const char *&a, const char *&b, int64_t &far) {
         int m0, n0;
         locate(item, m0, n0);
+        far = m0 + 128 < M ? 2 * a_rows64 : 0;
         a = reinterpret_cast<const char *>(A + int64_t(m0 + wave * 16) * lda);
         b = reinterpret_cast<const char *>(B + int64_t(n0 + wave * 16) * ldb);
     };
     auto prepare_next = [&](int item) { // keeps the current origins when there is no further tile
         if (item < tiles_total)
-            tile_origin(item, a_next, b_next);
+            tile_origin(item, a_next, b_next, far_next);
         else
             next_step = 0;
     };
     auto copy_a = [&](int n, uint32_t slot) __attribute__((always_inline)) {
-        async_copy16(smem_base + slot + uint32_t((n >> 1) * 8192 + wave * 2048 + (n & 1) * 1024), pa_at + (n >> 1) * a_rows64, la[n & 1]);
+        async_copy16(smem_base + slot + uint32_t((n >> 1) * 8192 + wave * 2048 + (n & 1) * 1024), pa_at + (n < 4 ? 0 : pa_far) + ((n >> 1) & 1) * a_rows64, la[n & 1]);
     };
     auto copy_b = [&](int n, int slot) __attribute__((always_inline)) {
         async_copy16(smem_base + uint32_t(B_RING + slot * B_BYTES + (n >> 1) * 8192 + wave * 2048 + (n & 1) * 1024),
@@ -1343,8 +1348,8 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
     };
     if (int(blockIdx.x) >= tiles_total)
         return;
-    tile_origin(blockIdx.x, pa_at, pb_at);
-    a_next = pa_at, b_next = pb_at;
+    tile_origin(blockIdx.x, pa_at, pb_at, pa_far);
+    a_next = pa_at, b_next = pb_at, far_next = pa_far;
     prepare_next(blockIdx.x + stride);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -1406,7 +1411,7 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         constexpr int G = decltype(stage_tag)::value; // B's slot
         // In a tile's last period the producers cross into the next tile.  Selects, not branches.
         if (G == 0 && last_period)
-            pa_at = a_next, pb_at = b_next, pa_step = pb_step = next_step;
+            pa_at = a_next, pb_at = b_next, pa_far = far_next, pa_step = pb_step = next_step;
         half(std::true_type{}, slot, G, 1, 0, fa0, fb0, fa1, fb1);
         pa_at += pa_step;
         // Everything but A's youngest stage has landed.  A wave's loads and stores retire in order through one counter;
@@ -1455,13 +1460,15 @@ __global__ __launch_bounds__(256, 1) void gemm256_kernel(const bf16_t *__restric
         asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7"); // the compiler does not know that matrix instructions wrote the accumulators
         int m0, n0;
         locate(item, m0, n0);
-        u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
-        if (epilogue.wants_aux())
-            load_aux_pair<FM, FN>(epilogue, 0, m0 + wm, n0 + wn, lane, aux);
-        unsigned char *mine = smem + free_slot + wave * 2048; // rows that nobody but this wave will overwrite
-        staged_store_pinned<FM, FN>(acc, aux, mine, epilogue, m0 + wm, n0 + wn, lane);
-        __builtin_amdgcn_s_waitcnt(0xc07f); // this wave's reads of its buffer have returned
-        behind_epilogue = true;             // the stores stay in flight under the next tile's first stage
+        if (m0 + wm < M) {
+            u32x4 aux[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
+            if (epilogue.wants_aux())
+                load_aux_pair<FM, FN>(epilogue, 0, m0 + wm, n0 + wn, lane, aux);
+            unsigned char *mine = smem + free_slot + wave * 2048; // rows that nobody but this wave will overwrite
+            staged_store_pinned<FM, FN>(acc, aux, mine, epilogue, m0 + wm, n0 + wn, lane);
+            __builtin_amdgcn_s_waitcnt(0xc07f); // this wave's reads of its buffer have returned
+            behind_epilogue = true;             // the stores stay in flight under the next tile's first stage
+        }
         item += stride;
         if (item >= tiles_total)
             break;
@@ -2221,12 +2228,14 @@ void launch_gemm64(hipStream_t stream, Tile tile, const bf16_t *A, int lda, cons
 // block's cold start, nor do 128 columns of less than 768 unless they fill the units and 192 does not divide the width.
 // The forward GELU of widths that 192 divides stays with the 128 x 192 blocks: alone they are as fast (16384 x 3072 x 768 99.0 us,
 // with 256 columns 97.9), but inside a step the second block covers the writes of two results (eight steps at d_model 768 183.0 ms,
-// with 256 columns 187.1).
+// with 256 columns 187.1).  Rows that 128 divides and 256 does not: the half tiles count as whole ones, and over the same products of
+// 4224 to 16256 rows the choice takes 1.5 to 6.1 % less than 128-row blocks alone (10368 x 1024 x 4096 100.3 -> 79.2 us,
+// 16256 x 768 x 3072 75.6 -> 59.8), at 2176 rows 0.2 %.
 int columns_of_256(int M, int N, int K, int mode) { // 0: the 128-row blocks
     const bool gelu = mode != EPI_PLAIN && mode != EPI_RESIDUAL;
     const int units = compute_units(), wide = N % 192 == 0 ? 192 : 128;
     const int64_t blocks = int64_t(M / 128) * (N / wide), per_unit = (blocks + units - 1) / units;
-    if (M % 256 || K % 128 || per_unit < 2 || K < (gelu ? 512 : 768))
+    if (M % 128 || K % 128 || per_unit < 2 || K < (gelu ? 512 : 768))
         return 0;
     if (gelu && mode != EPI_GELU_BWD && wide == 192)
         return 0;
@@ -2236,7 +2245,7 @@ int columns_of_256(int M, int N, int K, int mode) { // 0: the 128-row blocks
     for (int bn : {128, 192, 256}) {
         if (N % bn)
             continue;
-        const int64_t tiles = int64_t(M / 256) * (N / bn), rounds = (tiles + units - 1) / units;
+        const int64_t tiles = int64_t((M + 255) / 256) * (N / bn), rounds = (tiles + units - 1) / units;
         if (bn == 128 && K < 768 && (wide == 192 || tiles * 10 < rounds * units * 9))
             continue;
         const double cost = double(rounds) * (double(K) * (bn + 52) + bn * (gelu ? 1050. : 480.));
@@ -2258,9 +2267,9 @@ void launch_gemm256(hipStream_t stream, const bf16_t *A, int lda, const bf16_t *
                   "gemm LDS size: ");
         configured[device].store(true, std::memory_order_release);
     }
-    const int tiles_m = M / 256, tiles_n = N / BN, tiles = tiles_m * tiles_n;
+    const int tiles_m = (M + 255) / 256, tiles_n = N / BN, tiles = tiles_m * tiles_n;
     const int units = compute_units(), blocks = tiles < units ? tiles : units;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, A, lda, B, ldb, K / 128, tiles_n, tiles,
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, A, lda, B, ldb, M, K / 128, tiles_n, tiles,
                        xcd_columns(tiles_m, tiles_n, 256, BN, K, blocks), epilogue);
     check_hip(hipGetLastError(), "gemm launch: ");
 }
