@@ -2280,14 +2280,19 @@ void launch_gemm256_bf16(hipStream_t stream, const bf16_t *A, int lda, const bf1
     case EPI_RESIDUAL:
         return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_RESIDUAL>{e});
     case EPI_GELU:
-        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
+        if constexpr (BN != 192)
+            return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU>{e});
+        break;
     case EPI_GELU_ONLY:
-        return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
+        if constexpr (BN != 192)
+            return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_ONLY>{e});
+        break;
     case EPI_GELU_BWD:
         return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_GELU_BWD>{e});
     default:
         return launch_gemm256<BN>(stream, A, lda, B, ldb, M, N, K, EpilogueBf16As<EPI_PLAIN>{e});
     }
+    throw std::logic_error("gemm: columns_of_256 leaves no forward GELU to 192 columns");
 }
 
 template <int BM, int BN, int S, bool BKC, int GROUPS = 1, class Epilogue>
