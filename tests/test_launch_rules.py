@@ -1,0 +1,42 @@
+"""Which kernel a call's shape is given, at the lines where it changes (csrc/*_launch.h), on the host alone and for the 256 compute
+units that the lines were measured on.  The results that either side of a line computes are the GPU tests' matter."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+UNITS = 256
+TEAM, LONE = 4, 1  # waves that share sixteen tokens
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    library = tmp_path_factory.mktemp("rules") / "librules.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", str(ROOT / "tests/launch_rules.cpp"), "-o", str(library)],
+                   check=True)
+    return C.CDLL(str(library))
+
+
+def teams(rules, waves, depth, passes=False, count=1, flying=1):
+    out = (C.c_int * 4)()
+    rules.w16_teams(int(passes), waves, count, depth, flying, UNITS, out)
+    return dict(zip(("teams", "blocks", "waves", "rows"), out))
+
+
+@pytest.mark.parametrize("depth", [1, 4, 8])
+@pytest.mark.parametrize("waves,roles", [(4, TEAM), (256, TEAM), (1024, TEAM), (1025, LONE), (3072, LONE), (8192, LONE)])
+def test_width16_passes_of_their_own(rules, depth, waves, roles):
+    """Beyond four teams a unit both passes go to lone waves, like a step's."""
+    for passes in (False, True):
+        chosen = teams(rules, waves, depth, passes)
+        assert chosen["waves"] == roles
+        assert chosen["teams"] * chosen["blocks"] >= waves > chosen["teams"] * (chosen["blocks"] - 1)
+        assert not (passes and chosen["rows"])  # the backward pass is another launch
+
+
+@pytest.mark.parametrize("waves,teams_of_a_block", [(1025, 5), (2048, 8), (2049, 5), (3072, 6), (4096, 8), (65536, 8)])
+def test_width16_lone_waves_are_shared_out_evenly(rules, waves, teams_of_a_block):
+    """One block a unit up to eight lone waves a unit, then two."""
+    assert teams(rules, waves, 8, passes=True)["teams"] == teams_of_a_block

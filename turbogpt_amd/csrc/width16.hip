@@ -19,6 +19,7 @@
 // (the place of weight_gradient's read-modify-write and of reduce_gradients, cuda/ops.cuh:83-109, cuda/trainer.cuh:9-47).
 #include "common.h"
 #include "width16.h"
+#include "width16_launch.h"
 #include "../../include/tgk_kernels.h"
 #include <algorithm>
 #include <atomic>
@@ -29,9 +30,8 @@
 
 namespace {
 
-constexpr int W = 16, HEADS = 4, F = 48, V = 256, MAX_DEPTH = 8;
-constexpr int ROLES = 4;       // waves of a team, which has sixteen tokens; or it is a lone wave
-__host__ __device__ constexpr int block_waves(int roles) { return roles == 1 ? 8 : 16; } // they stage the weights, as many stay as are in teams
+using namespace w16;
+constexpr int HEADS = 4, F = 48;
 constexpr int WAVES = 4;       // waves of a block of weight gradients, whose chunks are whole numbers of four teams' tokens
 constexpr int CHUNK_WAVES = 8; // waves' tokens in one partial sum of a weight gradient (128 tokens)
 
@@ -68,12 +68,6 @@ Layout make_layout(int depth) {
 // Rows that a team leaves for the weight gradients, tiles of 64 x 8 bytes in the lanes' own order, side by side: normalised
 // rows, attention output, activation, and the gradients that are their other operands.
 enum Tile { T_N1, T_A, T_N2, T_ACT, T_DQKV = T_ACT + 3, T_DH_ATTENTION = T_DQKV + 3, T_DGU, T_DH_DOWN = T_DGU + 6, OPERANDS };
-// And what its own backward pass wants of a layer (cuda/types.cuh:40-44, cuda/model.cuh:25-29), a record of ROW_BYTES: tiles of
-// block input, post-RoPE query, the winning key and value (head layout) and post-attention residual; a word a lane of
-// GELU(top) and GELU'(top), a byte of the distance to the winner; a word a token of the two inverse norms.
-enum RowTile { R_X, R_Q, R_KEY, R_VALUE, R_MIDDLE, ROW_TILES };
-enum RowWord { R_GATE, R_SLOPE, ROW_WORDS };
-constexpr int ROW_DISTANCE = ROW_TILES * 512 + ROW_WORDS * 256, ROW_INVERSE = ROW_DISTANCE + 64, ROW_BYTES = ROW_INVERSE + 2 * W * 4;
 constexpr int ROW_FEATURES = ROW_BYTES, LONE_ROW_BYTES = ROW_FEATURES + 6 * 512; // a lone wave keeps gate and up there, too
 struct Workspace {
     u32x2 *tiles;        // [depth][waves][OPERANDS][64]
@@ -277,26 +271,6 @@ template <int R = ROLES> TG_DEVICE Lane lane_of(const Model &m, int waves) {
     return p;
 }
 
-// The weights in LDS as first operands, a tile of 64 x 8 bytes each (lane 16 g + c: elements (row c, k = 4 j + g), j = 0..3):
-// 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
-// The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
-// Operands of dX = dY W (rows = inputs, k = outputs) are read from the same tiles with the transposing load, in feed
-// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Then
-// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own; behind the first
-// layer, which no wave passes before all have read theirs, its place is the teams' for the sums of the softmax.  Last, for
-// each team, what its waves hand one another and, where they fit, the rows that the backward pass wants.
-constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
-__host__ __device__ constexpr int staged_tiles(int depth) { return depth * (LAYER_TILES + 1) + HEAD_TILES; }
-__host__ __device__ constexpr size_t embedding_at(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
-constexpr int EXCHANGE_BYTES = 16 * 1024 + 2 * ROLES * W * 4; // tiles, and a maximum and a picked logit of every role and token
-__host__ __device__ constexpr size_t teams_at(int depth, int teams) {
-    return embedding_at(depth) + (teams * 4096 > V * W * 2 ? teams * 4096 : V * W * 2);
-}
-__host__ __device__ constexpr size_t team_bytes(int depth, bool rows) { return EXCHANGE_BYTES + (rows ? depth * ROW_BYTES : 0); }
-__host__ __device__ constexpr size_t lds_bytes(int depth, int teams, bool rows) { return teams_at(depth, teams) + teams * team_bytes(depth, rows); }
-__host__ __device__ constexpr size_t lone_lds_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
-constexpr size_t LDS_BYTES = 160 * 1024;
-constexpr int STEP_TEAMS = 4; // of a unit, in batches in flight
 TG_DEVICE int feed_row(int row) { return ((row & 3) << 2) | (row >> 2); } // its own inverse
 // Byte offset, in a tile of items (g, c), of the item that lane 16 q + 4 j + m addresses for a transposing load: (m, 4 q + j)
 // or (m, 4 j + q).  Lane 16 q + i then gets element i % 4 of items (i / 4, 4 q + 0..3) or (i / 4, 4 * 0..3 + q).
@@ -968,14 +942,16 @@ TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight
 }
 
 // ---- kernels -----------------------------------------------------------------------------------------
-template <bool GRADIENT>
-__global__ __launch_bounds__(64 * block_waves(ROLES)) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
-                                                                             Workspace s, float *__restrict__ token_losses,
-                                                                             float *__restrict__ logits_out) {
+// Four waves a SIMD: of lone waves two blocks share a unit (128 registers, 8 to 15 of them spilled; with 155 to 177 and one block
+// 131072 tokens at depth 8 173 us forward and 242 with gradient, so 160 and 230).
+template <bool GRADIENT, int R>
+__global__ __launch_bounds__(64 * block_waves(R), 4) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
+                                                                         Workspace s, float *__restrict__ token_losses,
+                                                                         float *__restrict__ logits_out) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of(m, s.waves);
+    const Lane p = lane_of<R>(m, s.waves);
     const Staged weight(m, memory, p);
-    Staging<> staging(m, memory);
+    Staging<R> staging(m, memory);
     const int token = p.live ? x[p.token] : 0, target = p.live ? y[p.token] : 0;
     staging.request();
     staging.request_embedding(!(reinterpret_cast<uintptr_t>(m.hi) & 15));
@@ -986,40 +962,46 @@ __global__ __launch_bounds__(64 * block_waves(ROLES)) void w16_forward_kernel(Mo
     float rc, rs;
     rotation(p.position, rc, rs);
     Head head;
-    Kept<ROLES> kept;
-    forward_pass<ROLES, GRADIENT, 0>(m, p, weight, Exchange(m, memory, p, false), Rows<false>(m, memory, s, p), s, h, target, rc, rs, token_losses,
-                              logits_out, head, kept);
+    Kept<R> kept;
+    forward_pass<R, GRADIENT, 0>(m, p, weight, Exchange(m, memory, p, false), Rows<false>(m, memory, s, p), s, h, target, rc, rs, token_losses,
+                                 logits_out, head, kept);
     if constexpr (GRADIENT)
         if (p.role == 0) {
             const size_t here = size_t(p.wave) * 64 + p.lane;
             s.hidden[here] = head.hidden, s.inverse[here] = head.inverse;
         }
 }
-__global__ __launch_bounds__(64 * block_waves(ROLES)) void w16_backward_kernel(Model m, Workspace s) {
+template <int R> __global__ __launch_bounds__(64 * block_waves(R)) void w16_backward_kernel(Model m, Workspace s) {
     extern __shared__ __align__(16) unsigned char memory[];
-    const Lane p = lane_of(m, s.waves);
+    const Lane p = lane_of<R>(m, s.waves);
     const Staged weight(m, memory, p);
     const Exchange exchange(m, memory, p, false);
-    Staging<> staging(m, memory);
+    Staging<R> staging(m, memory);
     staging.request();
     const size_t here = size_t(p.wave) * 64 + p.lane;
     const Head head = {s.hidden[here], s.inverse[here]};
     staging.finish(true);
     if (!staging.stays())
         return;
+    const Rows<false> rows(m, memory, s, p);
+    Kept<R> kept;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        exchange.tile(p.role + 4 * i) = unpack4(s.dlogits[(size_t(p.wave) * 16 + p.role + 4 * i) * 64 + p.lane]);
+    for (int i = 0; i < HEAD_TILES / R; ++i) {
+        const u32x2 row = s.dlogits[(size_t(p.wave) * 16 + p.role + R * i) * 64 + p.lane];
+        if constexpr (R > 1)
+            exchange.tile(p.role + R * i) = unpack4(row);
+        else
+            kept.dlogits[i] = row;
+    }
     float rc, rs;
     rotation(p.position, rc, rs);
-    const Rows<false> rows(m, memory, s, p);
-    Kept<ROLES> kept;
-    if (p.role)
+    if constexpr (R > 1)
+        if (p.role)
 #pragma unroll
-        for (int l = 0; l < MAX_DEPTH; ++l)
-            if (l < m.depth)
-                kept.of_role[l] = GateUp(weight, l, p.role - 1)(unpack4(normalize(unpack4(rows.tile(l, R_MIDDLE)), rows.inverse(l, 1), weight.scale(2 * l + 1))));
-    backward_pass<ROLES, 0>(m, p, weight, exchange, rows, s, rc, rs, head, kept);
+            for (int l = 0; l < MAX_DEPTH; ++l)
+                if (l < m.depth)
+                    kept.of_role[l] = GateUp(weight, l, p.role - 1)(unpack4(normalize(unpack4(rows.tile(l, R_MIDDLE)), rows.inverse(l, 1), weight.scale(2 * l + 1))));
+    backward_pass<R, 0>(m, p, weight, exchange, rows, s, rc, rs, head, kept);
 }
 // A training step's both passes: a team's backward pass reads only what its own forward pass kept, so the two are one launch
 // and the weights are staged once.  us a launch, all on lone waves and so: depth 4, 2560 sequences of 4 38.6 and 31.5; depth 8, four
@@ -1640,32 +1622,6 @@ int compute_units() {
     }
     return units;
 }
-// How a pass over `waves` teams in each of `count` batches is launched: the fewest teams a block that need no more than `places` blocks.
-struct Teams {
-    int teams, blocks, roles; // teams of a block
-    size_t lds;
-    bool rows; // stay in LDS
-};
-Teams teams_of(int waves, int count, int depth, int roles, bool rows, int places) {
-    const auto lds = [&](int teams) { return roles == 1 ? lone_lds_bytes(depth) : lds_bytes(depth, teams, rows); };
-    int teams = 1;
-    while ((teams + 1) * roles <= block_waves(roles) && (waves + teams - 1) / teams * count > places && lds(teams + 1) <= LDS_BYTES)
-        ++teams;
-    return {teams, (waves + teams - 1) / teams, roles, lds(teams), rows};
-}
-// Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that, also
-// for batches in flight (`flying` at a time on streams of their own), a lone wave does less in all: no handing over, two waves'
-// arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8 (context 4) 87 and 106, 1280
-// (context 8) 171 and 145; 640 with K = 4 on streams 73 and 59.  Of lone waves a block takes four where there are other batches (K = 4, 640
-// teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us), as many as leave every unit one block where there are none (1280 teams: 145, with four 149).
-Teams step_teams(int waves, int count, int depth, int flying) {
-    for (const bool rows : {true, false}) {
-        const Teams t = teams_of(waves, count, depth, ROLES, rows, compute_units());
-        if (t.blocks * count <= compute_units() && waves * count * flying <= STEP_TEAMS * compute_units())
-            return t;
-    }
-    return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : compute_units());
-}
 void launch_weight_gradients(hipStream_t stream, const Model &m, const Workspace &r, const Group &group, int count, bool losses) {
     const int parameters = make_layout(m.depth).count, blocks = fold_blocks(parameters);
     static std::atomic<bool> configured[64];
@@ -1687,12 +1643,14 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
         Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        static std::atomic<bool> configured[2][64];
-        const auto kernel = with_gradient ? w16_forward_kernel<true> : w16_forward_kernel<false>;
-        allow_lds(kernel, configured[with_gradient != 0]);
-        const Teams t = teams_of(r.waves, 1, depth, ROLES, false, compute_units());
+        const Teams t = pass_teams(r.waves, depth, compute_units());
         m.teams = t.teams;
-        hipLaunchKernelGGL(kernel, dim3(t.blocks), dim3(64 * block_waves(ROLES)), t.lds, stream, m, x, y, r, token_losses, logits);
+        static std::atomic<bool> configured[4][64];
+        const bool lone = t.roles == 1;
+        const auto kernel = with_gradient ? (lone ? w16_forward_kernel<true, 1> : w16_forward_kernel<true, ROLES>)
+                                          : (lone ? w16_forward_kernel<false, 1> : w16_forward_kernel<false, ROLES>);
+        allow_lds(kernel, configured[(with_gradient != 0) * 2 + lone]);
+        hipLaunchKernelGGL(kernel, dim3(t.blocks), dim3(64 * block_waves(t.roles)), t.lds, stream, m, x, y, r, token_losses, logits);
         check_hip(hipGetLastError(), "w16_forward launch: ");
     });
 }
@@ -1705,11 +1663,13 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
         Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        static std::atomic<bool> configured[64];
-        allow_lds(w16_backward_kernel, configured);
-        const Teams t = teams_of(r.waves, 1, depth, ROLES, false, compute_units());
+        const Teams t = pass_teams(r.waves, depth, compute_units());
         m.teams = t.teams;
-        hipLaunchKernelGGL(w16_backward_kernel, dim3(t.blocks), dim3(64 * block_waves(ROLES)), t.lds, stream, m, r);
+        static std::atomic<bool> configured[2][64];
+        const bool lone = t.roles == 1;
+        const auto kernel = lone ? w16_backward_kernel<1> : w16_backward_kernel<ROLES>;
+        allow_lds(kernel, configured[lone]);
+        hipLaunchKernelGGL(kernel, dim3(t.blocks), dim3(64 * block_waves(t.roles)), t.lds, stream, m, r);
         check_hip(hipGetLastError(), "w16_backward launch: ");
         Group group{};
         group.member[0].tokens = const_cast<uint8_t *>(x), group.member[0].workspace = workspace, group.member[0].gradient = gradient;
@@ -1733,7 +1693,7 @@ void w16_gradients(hipStream_t stream, int depth, int batch, int context, const 
     const Workspace r = carve(depth, batch, context, batches[0].workspace);
     Group group{};
     std::copy(batches, batches + count, group.member);
-    const Teams t = step_teams(r.waves, count, depth, flying);
+    const Teams t = step_teams(r.waves, count, depth, flying, compute_units());
     m.teams = t.teams;
     static std::atomic<bool> configured[6][64];
     const auto kernel = context == 4 ? (t.roles == 1 ? w16_step_kernel<4, 1, false> : t.rows ? w16_step_kernel<4, ROLES, true> : w16_step_kernel<4, ROLES, false>)

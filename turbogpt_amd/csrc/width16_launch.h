@@ -1,0 +1,79 @@
+// How the width-16 network's passes are cut into blocks (width16.hip), and what a block has in LDS.  Plain functions of the shape and
+// of the number of compute units.
+#pragma once
+#include <cstddef>
+#include <initializer_list>
+
+namespace w16 {
+
+constexpr int W = 16, V = 256, MAX_DEPTH = 8;
+constexpr int ROLES = 4; // waves of a team, which has sixteen tokens; or it is a lone wave
+constexpr int block_waves(int roles) { return roles == 1 ? 8 : 16; } // they stage the weights, as many stay as are in teams
+
+// What a team's own backward pass wants of a layer (cuda/types.cuh:40-44, cuda/model.cuh:25-29), a record of ROW_BYTES: tiles of
+// block input, post-RoPE query, the winning key and value (head layout) and post-attention residual; a word a lane of
+// GELU(top) and GELU'(top), a byte of the distance to the winner; a word a token of the two inverse norms.
+enum RowTile { R_X, R_Q, R_KEY, R_VALUE, R_MIDDLE, ROW_TILES };
+enum RowWord { R_GATE, R_SLOPE, ROW_WORDS };
+constexpr int ROW_DISTANCE = ROW_TILES * 512 + ROW_WORDS * 256, ROW_INVERSE = ROW_DISTANCE + 64, ROW_BYTES = ROW_INVERSE + 2 * W * 4;
+
+// The weights in LDS as first operands, a tile of 64 x 8 bytes each (lane 16 g + c: elements (row c, k = 4 j + g), j = 0..3):
+// 13 tiles a layer - q, k, v, attention, gate x 3, up x 3, down x 3 - and the head's 16; and every RMSNorm scale in fp32.
+// The order of a tile's rows makes the product's layout: row c of a feed tile is the matrix's row 4 (c % 4) + c / 4.
+// Operands of dX = dY W (rows = inputs, k = outputs) are read from the same tiles with the transposing load, in feed
+// layout; the attention projection's, which are wanted in head layout, are staged a second time, behind the head's.  Then
+// comes the embedding as it is, so that a token's row is no further trip to memory behind the token's own; behind the first
+// layer, which no wave passes before all have read theirs, its place is the teams' for the sums of the softmax.  Last, for
+// each team, what its waves hand one another and, where they fit, the rows that the backward pass wants.
+constexpr int LAYER_TILES = 13, HEAD_TILES = 16;
+constexpr int staged_tiles(int depth) { return depth * (LAYER_TILES + 1) + HEAD_TILES; }
+constexpr size_t embedding_at(int depth) { return size_t(staged_tiles(depth)) * 512 + size_t(2 * depth + 1) * W * 4; }
+constexpr int EXCHANGE_BYTES = 16 * 1024 + 2 * ROLES * W * 4; // tiles, and a maximum and a picked logit of every role and token
+constexpr size_t teams_at(int depth, int teams) {
+    return embedding_at(depth) + (teams * 4096 > V * W * 2 ? teams * 4096 : V * W * 2);
+}
+constexpr size_t team_bytes(int depth, bool rows) { return EXCHANGE_BYTES + (rows ? depth * ROW_BYTES : 0); }
+constexpr size_t lds_bytes(int depth, int teams, bool rows) { return teams_at(depth, teams) + teams * team_bytes(depth, rows); }
+constexpr size_t lone_lds_bytes(int depth) { return embedding_at(depth) + V * W * 2; }
+constexpr size_t LDS_BYTES = 160 * 1024;
+
+// How a pass over `waves` teams in each of `count` batches is launched: the fewest teams a block that need no more than `places` blocks.
+struct Teams {
+    int teams, blocks, roles; // teams of a block
+    size_t lds;
+    bool rows; // stay in LDS
+};
+inline Teams teams_of(int waves, int count, int depth, int roles, bool rows, int places) {
+    const auto lds = [&](int teams) { return roles == 1 ? lone_lds_bytes(depth) : lds_bytes(depth, teams, rows); };
+    int teams = 1;
+    while ((teams + 1) * roles <= block_waves(roles) && (waves + teams - 1) / teams * count > places && lds(teams + 1) <= LDS_BYTES)
+        ++teams;
+    return {teams, (waves + teams - 1) / teams, roles, lds(teams), rows};
+}
+// Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that, also
+// for batches in flight (`flying` at a time on streams of their own), a lone wave does less in all: no handing over, two waves'
+// arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8 (context 4) 87 and 106, 1280
+// (context 8) 171 and 145; 640 with K = 4 on streams 73 and 59.  Of lone waves a block takes four where there are other batches (K = 4, 640
+// teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us), as many as leave every unit one block where there are none (1280 teams: 145, with four 149).
+constexpr int STEP_TEAMS = 4; // of a unit
+inline Teams step_teams(int waves, int count, int depth, int flying, int units, bool rows_in_lds = true) {
+    for (const bool rows : {true, false}) {
+        if (rows && !rows_in_lds)
+            continue;
+        const Teams t = teams_of(waves, count, depth, ROLES, rows, units);
+        if (t.blocks * count <= units && waves * count * flying <= STEP_TEAMS * units)
+            return t;
+    }
+    return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : units);
+}
+// The forward and the backward pass as launches of their own: by the same rule, and both alike, as a lone wave leaves its
+// features' rows to the backward pass.  us forward, with gradient, and backward with the weight gradients at depth 8, context 8, teams;
+// lone waves: 16384 tokens 35, 39, 70; (older kernels) 39, 44, 75   20480 66, 71, 107; 47, 58, 87   131072 258, 276, 549; 160, 230, 443
+// Two blocks fit a unit.  Of more than eight lone waves a unit both have the same share: 49152 tokens, eight a block 88, 114, 184, six 82,
+// 107, 179.
+inline Teams pass_teams(int waves, int depth, int units) {
+    const Teams t = step_teams(waves, 1, depth, 1, units, false);
+    return t.roles == 1 && waves > 8 * units ? teams_of(waves, 1, depth, 1, false, 2 * units) : t;
+}
+
+} // namespace w16
