@@ -479,11 +479,11 @@ struct Engine {
     // max(floor, s - K + 1), whichever way it is launched.
     // `shared`: up to K batches go out as one launch of each kernel on the engine's stream, and their optimizer steps as one
     // more.  The versions that they read are there before the first of those, as batch s reads nothing newer than `at`.
-    // Otherwise one batch and its optimizer step, on one of at most three streams.  Its slot is free, and the version that it
-    // reads is there, behind step at - K: that ran on this stream, or is waited for, or shared a launch, whose last one left
-    // version shared_end.  Three, as the process has four hardware queues and other work has one of them: where two of four streams
-    // share a queue, a batch stands behind the wait of another.  Depth 8, 1280 sequences of 8, K = 4, in calls of one step, us a step: on
-    // four streams 54 in a process of its own and 71 where another engine has run before, on three 60 in both.
+    // Otherwise one batch and its optimizer step, on its slot's stream, as the wide model's below.  Its slot is free, and
+    // the version that it reads is there, behind step at - K: that ran on this stream, or shared a launch, whose last one left
+    // version shared_end.  A stream for every slot: the process has four hardware queues, and which streams share one hangs on what else the
+    // process does.  Depth 8, 768 sequences of 8, K = 4, us a step on three streams and on four: alone 48, 40; with another engine or torch
+    // at work before 72, 57; after an engine that is gone 48, 59.  K = 8, three, four and eight: 49, 41, 41; 73, 58, 52; 49, 60, 50.
     int train_width16(uint64_t at, int most, bool shared, int *trace) {
         const Config &c = config.base;
         const uint64_t K = slots.size(), ring = versions.size();
@@ -500,8 +500,7 @@ struct Engine {
             total_staleness += step - read;
             max_staleness = std::max(max_staleness, int(step - read));
         }
-        const uint64_t streams = std::min<uint64_t>(K, 3);
-        const hipStream_t on = shared ? stream : slots[at % streams].stream;
+        const hipStream_t on = shared ? stream : slots[at % K].stream;
         const auto wait_for = [&](uint64_t version) { check_hip(hipStreamWaitEvent(on, versions[version % ring].done, 0)); };
         if (shared && K > 1 && at != shared_end) // the steps before ran on their slots' streams
             wait_for(at);
@@ -510,8 +509,7 @@ struct Engine {
                 check_hip(hipEventRecord(versions[shared_end % ring].done, stream));
             shared_recorded = true;
             wait_for(shared_end);
-        } else if (!shared && streams < K)
-            wait_for(at + 1 - K);
+        }
         {
             Scope profile_scope(this, TG_CLASS_OTHER);
             w16_gradients(on, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, shared ? 1 : int(K), batches);
