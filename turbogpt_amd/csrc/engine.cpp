@@ -481,9 +481,7 @@ struct Engine {
     // more.  The versions that they read are there before the first of those, as batch s reads nothing newer than `at`.
     // Otherwise one batch and its optimizer step, on its slot's stream, as the wide model's below.  Its slot is free, and
     // the version that it reads is there, behind step at - K: that ran on this stream, or shared a launch, whose last one left
-    // version shared_end.  A stream for every slot: the process has four hardware queues, and which streams share one hangs on what else the
-    // process does.  Depth 8, 768 sequences of 8, K = 4, us a step on three streams and on four: alone 48, 40; with another engine or torch
-    // at work before 72, 57; after an engine that is gone 48, 59.  K = 8, three, four and eight: 49, 41, 41; 73, 58, 52; 49, 60, 50.
+    // version shared_end.
     int train_width16(uint64_t at, int most, bool shared, int *trace) {
         const Config &c = config.base;
         const uint64_t K = slots.size(), ring = versions.size();
@@ -590,17 +588,38 @@ void validate(const TgModelConfig &m) {
         throw std::runtime_error("ln_eps must be positive");
 }
 
-// Streams, events, staging memory and the buffers every model kind needs per slot and per weight version.
+// The engine's stream, which is slot 0's, and one for every further slot.  The runtime has a few hardware queues, makes them as
+// streams come and then gives each new stream the one that has the fewest, so streams made one behind another have
+// different ones, but only once every queue is there and has as many: two slots that share one run one behind the other.  So as
+// many streams are made first, and given back.  Depth 8, 768 sequences of 8, K = 4, us a step without and with them: alone 40, 40;
+// beside another engine, torch, or after an engine that is gone 57, 58, 58 and 40.
+void build_streams(Engine *e, int inflight) {
+    constexpr int HARDWARE_QUEUES = 4; // the runtime's default
+    struct Spare {
+        std::vector<hipStream_t> streams;
+        ~Spare() {
+            for (hipStream_t stream : streams)
+                (void)hipStreamDestroy(stream);
+        }
+    } spare;
+    hipStream_t made = nullptr;
+    while (inflight > 1 && spare.streams.size() < HARDWARE_QUEUES && hipStreamCreate(&made) == hipSuccess)
+        spare.streams.push_back(made);
+    (void)hipGetLastError(); // one that is not to be had is no later call's error
+    e->slots.resize(size_t(inflight));
+    for (Slot &slot : e->slots) {
+        check_hip(hipStreamCreate(&slot.stream)); // default priority
+        if (&slot == &e->slots[0])
+            e->stream = slot.stream;
+    }
+}
+
+// Events, staging memory and the buffers every model kind needs per slot and per weight version.
 void build_slots(Engine *e, int inflight, bool transposed_copies) {
     const size_t P = size_t(e->layout.count), M = size_t(e->tokens());
     e->readback = Readback::shared(e->config.base.device);
-    e->slots.resize(size_t(inflight));
     e->versions.resize(inflight > 1 ? size_t(inflight) + 1 : 1);
     for (Slot &slot : e->slots) {
-        if (&slot == &e->slots[0])
-            slot.stream = e->stream;
-        else
-            check_hip(hipStreamCreate(&slot.stream)); // default priority
         e->allocate(slot.input, M);
         e->allocate(slot.target, M);
         e->allocate(slot.token_losses, M);
@@ -826,7 +845,7 @@ TG_API Engine *tg_create(const Config *c) {
         e->config.ln_eps = 1e-6f;
         e->layout.count = tgk_w16_parameter_count(c->depth);
         e->compute_units = prop.multiProcessorCount;
-        check_hip(hipStreamCreate(&e->stream));
+        build_streams(e, c->inflight);
         const size_t P = size_t(e->layout.count);
         build_slots(e, c->inflight, false);
         e->allocate(e->momentum, P);
@@ -873,9 +892,8 @@ TG_API Engine *tg_create_ex(const TgModelConfig *model) {
         e->compute_units = prop.multiProcessorCount;
         if (e->layout.count > INT_MAX)
             throw std::runtime_error("Parameter count exceeds signed 32-bit indexing");
-        check_hip(hipStreamCreate(&e->stream));
-
         const Config &c = model->base;
+        build_streams(e, c.inflight);
         const size_t P = size_t(e->layout.count), M = size_t(e->tokens()), d = size_t(model->d_model);
         const size_t F = size_t(model->ffn), V = size_t(model->vocab);
         build_slots(e, c.inflight, true);
