@@ -40,3 +40,17 @@ def test_width16_passes_of_their_own(rules, depth, waves, roles):
 def test_width16_lone_waves_are_shared_out_evenly(rules, waves, teams_of_a_block):
     """One block a unit up to eight lone waves a unit, then two."""
     assert teams(rules, waves, 8, passes=True)["teams"] == teams_of_a_block
+
+
+@pytest.mark.parametrize("depth", [4, 8])
+@pytest.mark.parametrize("flying,last", [(2, 224), (3, 179), (4, 149)])
+def test_width16_batches_in_flight_fit_side_by_side(rules, depth, flying, last):
+    """A unit has room for one block of teams: on streams of their own, `flying` batches' blocks are no more than the units - an eighth more
+    with the rows in LDS - unless blocks of four teams, the largest, already are.  Beyond `last` blocks of four teams' tokens, lone waves."""
+    for blocks in range(1, last + 40):
+        chosen = teams(rules, 4 * blocks, depth, flying=flying)
+        assert chosen["waves"] == (TEAM if blocks <= last else LONE), blocks
+        if blocks <= last:
+            places = UNITS * 9 // 8 if chosen["rows"] else UNITS
+            assert chosen["blocks"] * flying <= places or (chosen["teams"] == 4 and not chosen["rows"]), (blocks, chosen)
+        assert chosen["teams"] * chosen["blocks"] >= 4 * blocks > chosen["teams"] * (chosen["blocks"] - 1)

@@ -22,6 +22,7 @@ constexpr int MaxLaunchSteps = 4096; // cuda/types.cuh:10
 constexpr int NormPartials = 1024;
 constexpr int ListUnit = 128;   // every width is a multiple of it (wgrad_list)
 constexpr int RowTile = 128;    // smallest number of rows the matrix products take
+constexpr int HardwareQueues = 4; // of the process, the runtime's default: as many streams run side by side
 constexpr int MaxInFlight = 16; // batches in flight, each with its own stream and saved activations
 // Rows of the loss history, a ring over the steps: two steps that share a row are at least MaxInFlight apart, so the later
 // one is behind the earlier one also where they are in different launches and on different streams.
@@ -475,6 +476,7 @@ struct Engine {
         const int K = int(slots.size()), launches = (steps + K - 1) / K;
         return K == 1 || (w16_blocks(c.batch, c.context) <= (c.depth == 4 ? 160 : 144) && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
     }
+    int flying() const { return std::min(int(slots.size()), HardwareQueues); } // batches on streams of their own that run side by side
     // Training steps of the width-16 network from `at` on; returns how many.  Batch s reads the weights of version
     // max(floor, s - K + 1), whichever way it is launched.
     // `shared`: up to K batches go out as one launch of each kernel on the engine's stream, and their optimizer steps as one
@@ -510,7 +512,7 @@ struct Engine {
         }
         {
             Scope profile_scope(this, TG_CLASS_OTHER);
-            w16_gradients(on, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, shared ? 1 : int(K), batches);
+            w16_gradients(on, c.depth, c.batch, c.context, {data, data_size, c.seed}, count, shared ? 1 : flying(), batches);
         }
         if (!shared && at != shared_end)
             wait_for(at);
@@ -594,7 +596,6 @@ void validate(const TgModelConfig &m) {
 // many streams are made first, and given back.  Depth 8, 768 sequences of 8, K = 4, us a step without and with them: alone 40, 40;
 // beside another engine, torch, or after an engine that is gone 57, 58, 58 and 40.
 void build_streams(Engine *e, int inflight) {
-    constexpr int HARDWARE_QUEUES = 4; // the runtime's default
     struct Spare {
         std::vector<hipStream_t> streams;
         ~Spare() {
@@ -603,7 +604,7 @@ void build_streams(Engine *e, int inflight) {
         }
     } spare;
     hipStream_t made = nullptr;
-    while (inflight > 1 && spare.streams.size() < HARDWARE_QUEUES && hipStreamCreate(&made) == hipSuccess)
+    while (inflight > 1 && spare.streams.size() < HardwareQueues && hipStreamCreate(&made) == hipSuccess)
         spare.streams.push_back(made);
     (void)hipGetLastError(); // one that is not to be had is no later call's error
     e->slots.resize(size_t(inflight));

@@ -50,18 +50,28 @@ inline Teams teams_of(int waves, int count, int depth, int roles, bool rows, int
         ++teams;
     return {teams, (waves + teams - 1) / teams, roles, lds(teams), rows};
 }
-// Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that, also
-// for batches in flight (`flying` at a time on streams of their own), a lone wave does less in all: no handing over, two waves'
-// arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8 (context 4) 87 and 106, 1280
-// (context 8) 171 and 145; 640 with K = 4 on streams 73 and 59.  Of lone waves a block takes four where there are other batches (K = 4, 640
-// teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us), as many as leave every unit one block where there are none (1280 teams: 145, with four 149).
+// Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that a lone wave
+// does less in all: no handing over, two waves' arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8
+// (context 4) 87 and 106, 1280 (context 8) 171 and 145.  Of lone waves a block takes as many as leave every unit one block (1280 teams: 145, with
+// four 149), four where there are other batches (K = 4, 640 teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us).
+// `flying` such launches run side by side, on streams of their own, and a unit has room for one block of teams: they are cut so that all of
+// them fit, their rows left out of LDS for more teams a block, and one's tail is another's start, so that teams are the better form for
+// longer.  Depth 8, 64 blocks of four teams (256 teams a batch), calls of one step, us a step with one, two (rows in LDS) and four teams a block
+// and on lone waves: two flying 54.8, 41.4, 44.6, 52; three 43.8, 31, 32.5, 38; four 45, 31, 31.5, 36.  96 blocks, one to four teams
+// without rows, lone waves: two 65.5, 50.8, 47.8, 48.9, 57; four 63, 43.5, 37.7, 32.0, 40.3.  Two a block with rows may be an eighth too many
+// (two flying, 72 blocks 42.7, three without 46.9).  Lone waves take over at some 220, 190 and 160 blocks, four teams a block against
+// them: two flying 200 66.9, 70.0; 240 83.6, 80.2; three 180 61.8, 65.0; 200 70.8, 69.0; four 144 49.0, 51.4; 180 60.8, 59.8.  At depth 4 the lines
+// lie further out, by differences of a tenth at most.
 constexpr int STEP_TEAMS = 4; // of a unit
 inline Teams step_teams(int waves, int count, int depth, int flying, int units, bool rows_in_lds = true) {
     for (const bool rows : {true, false}) {
         if (rows && !rows_in_lds)
             continue;
-        const Teams t = teams_of(waves, count, depth, ROLES, rows, units);
-        if (t.blocks * count <= units && waves * count * flying <= STEP_TEAMS * units)
+        if (flying > 1 ? waves * count * (flying + 2) > 14 * units : waves * count > STEP_TEAMS * units)
+            break;
+        const int places = flying > 1 ? (rows ? units * 9 / 8 : units) / flying : units;
+        const Teams t = teams_of(waves, count, depth, ROLES, rows, places);
+        if (t.blocks * count <= places || (flying > 1 && !rows))
             return t;
     }
     return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : units);
