@@ -7,4 +7,7 @@ void w16_teams(int passes, int waves, int count, int depth, int flying, int unit
     const w16::Teams t = passes ? w16::pass_teams(waves, depth, units) : w16::step_teams(waves, count, depth, flying, units);
     out[0] = t.teams, out[1] = t.blocks, out[2] = t.roles, out[3] = t.rows;
 }
+int w16_shares_launches(int depth, int K, int flying, int blocks, int steps, int units) {
+    return w16::shares_launches(depth, K, flying, blocks, steps, units);
+}
 }

@@ -44,8 +44,8 @@ def measure(others):
 
 @pytest.mark.parametrize("others", [0, 1, 2])
 def test_short_calls_overlap_beside_other_engines(others):
-    """Two, three and four batches in flight take some 66, 58 and 55 us a step, where two of them share a queue 98, 79 and 71 to 80;
-    one behind another some 83."""
+    """Two, three and four batches in flight take some 59, 49 and 54 us a step, where two of them share a queue 91, 69 and 71; one behind
+    another some 83."""
     result = subprocess.run([sys.executable, __file__, str(others)], cwd=ROOT, env={**os.environ, "PYTHONPATH": str(ROOT)},
                             capture_output=True, text=True, timeout=100)
     assert result.returncode == 0, result.stderr

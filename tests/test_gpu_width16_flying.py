@@ -32,3 +32,19 @@ def test_a_step_is_its_gradient_and_its_update(depth, context, inflight, blocks,
         apart.optimizer_test(gradient)
         np.testing.assert_allclose(engine.training_losses(1)[0], losses, rtol=1e-6)  # means in double of the same losses
         np.testing.assert_array_equal(engine.weights(), apart.weights())
+
+
+@pytest.mark.parametrize("depth,inflight,blocks", [(8, 2, 1), (8, 2, 128), (8, 3, 1), (8, 3, 40), (8, 4, 64), (4, 2, 128), (4, 8, 96)])
+def test_shared_launches_train_like_streams(depth, inflight, blocks):
+    """Calls of as many steps as there are batches in flight share their launches, calls of one do not: bit for bit the same weights."""
+    data = np.random.default_rng(blocks).integers(0, 256, 1 << 16, dtype=np.uint8)
+    with bridge.Native(bridge.Config(depth=depth, context=depth, batch=64 * blocks // depth, inflight=inflight)) as engine:
+        engine.set_data(data)
+        weights = []
+        for calls in ([inflight] * 3, [1] * (3 * inflight), [1, inflight, inflight - 1, inflight]):
+            engine.set_weights(reference_style_weights(depth, scale=.05))
+            for steps in calls:
+                engine.train(steps)
+            weights.append(engine.weights())
+        for others in weights[1:]:
+            np.testing.assert_array_equal(others, weights[0])

@@ -54,3 +54,17 @@ def test_width16_batches_in_flight_fit_side_by_side(rules, depth, flying, last):
             places = UNITS * 9 // 8 if chosen["rows"] else UNITS
             assert chosen["blocks"] * flying <= places or (chosen["teams"] == 4 and not chosen["rows"]), (blocks, chosen)
         assert chosen["teams"] * chosen["blocks"] >= 4 * blocks > chosen["teams"] * (chosen["blocks"] - 1)
+
+
+@pytest.mark.parametrize("depth,K,blocks,steps,shared", [
+    (8, 1, 1, 1, True), (4, 1, 4000, 64, True),                           # one batch: its launch is all there is
+    (8, 2, 1, 2, True), (8, 2, 128, 2, True), (8, 2, 160, 2, False),      # depth 8, two in flight
+    (8, 3, 1, 3, True), (8, 3, 40, 3, True), (8, 3, 1, 6, True), (8, 3, 96, 4, False),
+    (8, 4, 1, 1, False), (8, 4, 1, 3, True), (8, 4, 1, 5, True), (8, 4, 40, 4, True), (8, 4, 96, 4, False), (8, 4, 128, 4, False),
+    (8, 16, 16, 16, True), (8, 8, 200, 8, False),
+    (4, 2, 1, 1, False), (4, 2, 1, 3, True), (4, 2, 96, 2, True), (4, 4, 128, 4, True), (4, 4, 160, 2, False), (4, 8, 160, 2, False),
+    (4, 4, 200, 4, False), (4, 8, 200, 8, False),
+])
+def test_width16_shared_launches(rules, depth, K, blocks, steps, shared):
+    """The better one of the two as they were measured, where they differ by 5 % or more (csrc/width16_launch.h)."""
+    assert bool(rules.w16_shares_launches(depth, K, min(K, 4), blocks, steps, UNITS)) is shared

@@ -8,6 +8,7 @@
 #include "readback.h"
 #include "step.h"
 #include "width16.h"
+#include "width16_launch.h"
 #include "../../include/tg_model.h"
 #include "../../include/tgk_kernels.h"
 #include <algorithm>
@@ -463,18 +464,10 @@ struct Engine {
         forward(s, v, true, nullptr, c.batch, false, true);
         backward(s, v, history_row(at));
     }
-    // Whether the batches of a call of `steps` steps share their launches.  On K streams a step costs the host 32 us of
-    // launches and events at least, however small its batch, but steps of one call overlap with those of the next.  A shared launch
-    // takes as long as one batch, 48 us at depth 4 and 77 at depth 8, and 8 us of optimizer a step: worth it from two and from 3.25
-    // steps a launch on, while a batch does not fill the units.  us a step on streams and shared (depth and context equal):
-    //   depth 8, 16 sequences: K = 2 46, 46; 4 37, 20; 16 35, 13; calls of one step at K = 4 38, 81; of five 36, 42
-    //   depth 4, 16 sequences: K = 2 35, 32; 8 34, 13; calls of two 32, 32
-    //   113 blocks: depth 8, K = 4 55, 45; depth 4 37, 29   138: depth 8 65, 64   160: depth 8 63, 64; K = 8 63, 58; depth 4, K = 4 40, 37; 8 41, 36
-    //   320 blocks: depth 8, K = 4 112, 114
+    // Whether the batches of a call of `steps` steps share their launches.
     bool shares_launches(int steps) const {
         const Config &c = config.base;
-        const int K = int(slots.size()), launches = (steps + K - 1) / K;
-        return K == 1 || (w16_blocks(c.batch, c.context) <= (c.depth == 4 ? 160 : 144) && steps * 4 >= launches * (c.depth == 4 ? 8 : 13));
+        return w16::shares_launches(c.depth, int(slots.size()), flying(), w16_blocks(c.batch, c.context), steps, compute_units);
     }
     int flying() const { return std::min(int(slots.size()), HardwareQueues); } // batches on streams of their own that run side by side
     // Training steps of the width-16 network from `at` on; returns how many.  Batch s reads the weights of version
@@ -593,8 +586,8 @@ void validate(const TgModelConfig &m) {
 // The engine's stream, which is slot 0's, and one for every further slot.  The runtime has a few hardware queues, makes them as
 // streams come and then gives each new stream the one that has the fewest, so streams made one behind another have
 // different ones, but only once every queue is there and has as many: two slots that share one run one behind the other.  So as
-// many streams are made first, and given back.  Depth 8, 768 sequences of 8, K = 4, us a step without and with them: alone 40, 40;
-// beside another engine, torch, or after an engine that is gone 57, 58, 58 and 40.
+// many streams are made first, and given back.  Depth 8, 768 sequences of 8, K = 4, calls of one step, us a step without and with them:
+// alone 36, 36; beside another engine or two, after one that is gone, with torch at work 49 to 51, 33 to 36.  K = 2 beside two others 80, 48.
 void build_streams(Engine *e, int inflight) {
     struct Spare {
         std::vector<hipStream_t> streams;

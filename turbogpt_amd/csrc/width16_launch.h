@@ -1,6 +1,7 @@
 // How the width-16 network's passes are cut into blocks (width16.hip), and what a block has in LDS.  Plain functions of the shape and
 // of the number of compute units.
 #pragma once
+#include <algorithm>
 #include <cstddef>
 #include <initializer_list>
 
@@ -75,6 +76,31 @@ inline Teams step_teams(int waves, int count, int depth, int flying, int units, 
             return t;
     }
     return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : units);
+}
+// Whether the batches of a call of `steps` steps, K of them in flight, share their launches: by the lesser of two estimated times in
+// us, for batches of `blocks` blocks of four teams' tokens at depth 4 or 8.  A shared launch's batches and their optimizer steps go as one
+// (a launch's time, 4 us a batch, and the blocks of all of them in one, two or more rounds on the units), but the next launch stands
+// behind it.  On streams a step costs the host 34 us, hides behind as many others as there are hardware queues (`flying`), and with those fills
+// the units.  The constants are a fit to K = 2 to 16, calls of 1 to 32 steps and 1 to 512 blocks, 1372 points: the choice is within 0.3 % of
+// the better one (geometric mean; beyond 10 % at six).  us a step, streams and shared:
+//   depth 8, 1 block, calls of K: K = 2 35, 29; 3 34, 20; 4 34, 17; calls of one at K = 4 34, 54; of five 34, 25
+//   depth 8, K = 4, calls of four: 96 blocks 35, 39; 128 42, 45   K = 2, calls of two: 96 48, 44; 128 52, 48; 160 59, 71
+//   depth 4, 1 block, calls of K: K = 2 33, 20; 4 33, 12   K = 4, calls of four: 128 blocks 34, 27; 160 34, 34   calls of two: 40 34, 25; 160 33, 46
+// A batch that fills three quarters of the units by itself stays on streams (depth 4, K = 8, 200 blocks 41, 42; depth 8 65, 70).
+inline bool shares_launches(int depth, int K, int flying, int blocks, int steps, int units) {
+    if (K == 1)
+        return true;
+    if (blocks > units * 3 / 4)
+        return false;
+    const double share = double(blocks) / units; // of the units that one batch fills
+    const auto together = [&](int n) {
+        const double all = n * share;
+        const double time = depth == 4 ? (all <= 1 ? 34 + 26 * all : all <= 2 ? 66 + 17 * all : 54 + 33 * all)
+                                       : (all <= 1 ? 50 + 44 * all : all <= 2 ? 95 + 33 * all : 80 + 64 * all);
+        return time + 4 * n;
+    };
+    const double alone = depth == 4 ? std::max((26 + 84 * share) / flying, 46 * share) : std::max((62 + 90 * share) / flying, 82 * share);
+    return steps / K * together(K) + (steps % K ? together(steps % K) : 0.) < steps * std::max(34., alone);
 }
 // The forward and the backward pass as launches of their own: by the same rule, and both alike, as a lone wave leaves its
 // features' rows to the backward pass.  us forward, with gradient, and backward with the weight gradients at depth 8, context 8, teams;
