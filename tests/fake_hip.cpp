@@ -209,16 +209,21 @@ void *readback_open(int device) {
     return new std::shared_ptr<Readback>(Readback::shared(device));
 }
 void readback_close(void *handle) { delete static_cast<std::shared_ptr<Readback> *>(handle); }
-// plain copies of `count` pieces, or joins where lo[i] is given; 0, or -1 with the message in readback_error()
-int readback_fetch(void *handle, void *stream, int device, int count, void **host, const size_t *bytes, void **source, void **lo) {
+// plain copies of `count` pieces, or joins where lo[i] is given, with every second chunk on `second` unless that is null; 0, or -1 with
+// the message in readback_error()
+int readback_fetch_by_two(void *handle, void *stream, void *second, int device, int count, void **host, const size_t *bytes, void **source,
+                          void **lo) {
     current_device = device;
     return guarded([&] {
         std::vector<ReadbackPiece> pieces;
         for (int i = 0; i < count; ++i)
             pieces.push_back({host[i], bytes[i], lo[i] ? nullptr : source[i], static_cast<uint16_t *>(lo[i] ? source[i] : nullptr),
                               static_cast<uint16_t *>(lo[i])});
-        (*static_cast<std::shared_ptr<Readback> *>(handle))->fetch(static_cast<hipStream_t>(stream), pieces);
+        (*static_cast<std::shared_ptr<Readback> *>(handle))->fetch(static_cast<hipStream_t>(stream), pieces, static_cast<hipStream_t>(second));
     });
+}
+int readback_fetch(void *handle, void *stream, int device, int count, void **host, const size_t *bytes, void **source, void **lo) {
+    return readback_fetch_by_two(handle, stream, nullptr, device, count, host, bytes, source, lo);
 }
 const char *readback_error() { return tg_last_error.c_str(); }
 }
