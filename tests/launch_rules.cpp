@@ -1,7 +1,11 @@
 // The rules by which launches are chosen, for tests without a GPU: plain functions of a call's shape and the number of compute units.
+#include "../turbogpt_amd/csrc/gemm_launch.h"
 #include "../turbogpt_amd/csrc/width16_launch.h"
 
 extern "C" {
+int gemm_columns_of_256(int M, int N, int K, int mode, int units) {
+    return columns_of_256(M, N, K, mode, units);
+}
 // teams of a block, blocks, waves of a team, whether the rows stay in LDS; passes: of the separate forward and backward launches
 void w16_teams(int passes, int waves, int count, int depth, int flying, int units, int *out) {
     const w16::Teams t = passes ? w16::pass_teams(waves, depth, units) : w16::step_teams(waves, count, depth, flying, units);

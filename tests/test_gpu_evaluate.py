@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("d,ffn,context,batch", [(128, 256, 128, 1),     # 64 x 64 tiles
                                                  (256, 1024, 256, 8),    # 64 x 128 tiles
                                                  (640, 2560, 512, 8),    # 128 x 128 tiles
-                                                 (1024, 4096, 1024, 4),  # 256 x 128 tiles
+                                                 (1024, 4096, 1024, 4),  # 256 x 256 tiles
                                                  (384, 1536, 1024, 16)])  # 128 x 192 tiles
 def test_evaluation_matches_the_batch_with_gradient(d, ffn, context, batch):
     rng = np.random.default_rng(d + context)

@@ -380,10 +380,9 @@ def test_rejects_bad_shapes_without_launching():
 @pytest.mark.parametrize("M,N,K,residual", [(16384, 1024, 256, False), (16384, 1024, 512, True), (8192, 2048, 1024, False),
                                           (16384, 3072, 1024, True), (16384, 1024, 4096, False)])
 def test_256x128_tiles_rows_sampled(orc, M, N, K, residual):
-    """The widths of configs[4] (multiples of 128 and 256 that 192 does not divide) run on 256 x 128 tiles whose
-    epilogue buffers lie in a ring slot: forward with every epilogue and the input gradient on the transposed weight,
-    plain and times GELU', one to six tiles per block and one to sixteen periods per tile, against the checker on sampled rows and bit
-    for bit against the kernels for k-strided weights, which sum in the same order."""
+    """Products that tiles of 256 rows take, with the exception of the shortest: forward with every epilogue and the input gradient on
+    the transposed weight, plain and times GELU', one to four tiles a block and four to thirty-two 128-k periods a tile, against the
+    checker on sampled rows and bit for bit against the kernels for k-strided weights, which sum in the same order."""
     lib = library()
     rng = np.random.default_rng(M + N + K)
     x, xh = to_bf16_device(rng.standard_normal((M, K)))

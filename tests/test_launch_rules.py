@@ -68,3 +68,39 @@ def test_width16_batches_in_flight_fit_side_by_side(rules, depth, flying, last):
 def test_width16_shared_launches(rules, depth, K, blocks, steps, shared):
     """The better one of the two as they were measured, where they differ by 5 % or more (csrc/width16_launch.h)."""
     assert bool(rules.w16_shares_launches(depth, K, min(K, 4), blocks, steps, UNITS)) is shared
+
+
+PLAIN, GELU, GELU_BACKWARD, GELU_ONLY = 0, 2, 3, 5  # epilogues
+
+
+@pytest.mark.parametrize("M,N,K,forward,gelu,backward,gelu_backward", [
+    # test_gpu_gemm.py
+    (16384, 1024, 256, 0, 0, 0, 0), (16384, 1024, 512, 0, 256, 128, 128), (8192, 2048, 1024, 256, 256, 128, 128),
+    (16384, 3072, 1024, 256, 0, 256, 256), (16384, 1024, 4096, 256, 256, 256, 256),
+    # test_gpu_gemm_columns.py
+    (10240, 1024, 1152, 256, 256, 192, 192), (4096, 3584, 896, 256, 256, 0, 0), (12288, 768, 896, 192, 0, 0, 0),
+    (10240, 640, 768, 128, 128, 0, 0), (16384, 1024, 640, 0, 256, 128, 0), (16640, 1280, 1024, 128, 128, 128, 0),
+    (8320, 896, 896, 128, 128, 128, 128), (12416, 768, 768, 192, 0, 192, 0), (10368, 1024, 1152, 256, 256, 192, 192),
+    (4224, 3072, 768, 256, 0, 0, 0),
+])
+def test_columns_of_256_row_tiles(rules, M, N, K, forward, gelu, backward, gelu_backward):
+    """What the shapes of the kernel's tests are given; 0: 128-row blocks."""
+    def columns(N, K, mode):
+        return rules.gemm_columns_of_256(M, N, K, mode, UNITS)
+
+    assert (columns(N, K, PLAIN), columns(N, K, GELU)) == (forward, gelu)
+    assert columns(N, K, GELU_ONLY) == gelu
+    assert (columns(K, N, PLAIN), columns(K, N, GELU_BACKWARD)) == (backward, gelu_backward)
+
+
+def test_columns_of_256_row_tiles_in_several_rounds(rules):
+    """The shapes of test_gpu_gemm_columns_rounds.py: more tiles than units, and half a tile of rows at the end."""
+    import test_gpu_gemm_columns_rounds as shapes
+    for mode, listed in ((PLAIN, shapes.PLAIN), (GELU, shapes.GELU), (GELU_ONLY, shapes.GELU), (GELU_BACKWARD, shapes.GELU_BACKWARD)):
+        for M, N, K, columns in listed:
+            if mode == GELU_BACKWARD:
+                N, K = K, N
+            assert rules.gemm_columns_of_256(M, N, K, mode, UNITS) == columns
+            assert M % 256 == 128 and (M + 255) // 256 * (N // columns) > UNITS
+    assert rules.gemm_columns_of_256(10240, 640, 768, GELU_ONLY, UNITS) == 128
+    assert rules.gemm_columns_of_256(4096, 4096, 1024, GELU_ONLY, UNITS) == 256  # test_gpu_evaluate.py
