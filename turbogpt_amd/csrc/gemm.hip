@@ -127,7 +127,10 @@ template <int MODE, bool THROUGH = false> struct EpilogueBf16As {
 
 // fp32 outputs (weight gradients, split-K slabs): tiles go through the same kind of wave-private LDS
 // buffer untouched, and a lane finishes 4 consecutive n - 8 lanes cover a 128-byte row piece.
-struct EpilogueF32 {
+// THROUGH: whole lines, written through to memory, slabs that the next launch reads among them: every block has one tile, and the launch would
+// end with writing all of them back.  Through the caches and so, us: 3840 tokens, 384 x 1152 14.7, 13.6; 128 tokens, 3072 x 768 6.45, 5.41;
+// 8192, 2304 x 768 in 7 slabs (50 MB) 40.3, 38.2; 16384, 3072 x 3072 (38 MB) 306, 302; nothing from 128 x 256 to there was slower.
+template <bool THROUGH> struct EpilogueF32As {
     static constexpr bool BF16 = false;
     float *out;
     int ld_out;
@@ -139,10 +142,13 @@ struct EpilogueF32 {
         f32x4 *p = reinterpret_cast<f32x4 *>(out + split * split_stride + size_t(m) * ld_out + n);
         if (accumulate)
             value += *p;
-        // whole lines, written through to memory: 3840 tokens, two gradients of 384 x 1152 beside four products 70.3 -> 67.7 us
-        store_through(p, __builtin_bit_cast(u32x4, value));
+        if constexpr (THROUGH)
+            store_through(p, __builtin_bit_cast(u32x4, value));
+        else
+            *p = value;
     }
 };
+using EpilogueF32 = EpilogueF32As<true>;
 
 // bf16 outputs: each 32x32 accumulator tile is rounded and transposed through a wave-private LDS buffer
 // (32 rows of 64 bytes, 16-byte chunk c of row r at c ^ ((r >> 2) & 3)), so that a lane finishes 8
@@ -1536,7 +1542,7 @@ TG_DEVICE bool wgrad_item(const WgradBatch &w, int group, int block, WgradItem &
     item.nc = (item.split + 1) * w.k_chunks / splits - item.c0;
     return true;
 }
-template <int BM, int BN>
+template <int BM, int BN, bool THROUGH>
 __global__ __launch_bounds__(256, 2) void wgrad_batch_kernel(WgradBatch w) {
     using TA = TileKS64<BM>;
     using TB = TileKS64<BN>;
@@ -1621,10 +1627,10 @@ __global__ __launch_bounds__(256, 2) void wgrad_batch_kernel(WgradBatch w) {
         unsigned char *mine = smem + (c_slot ^ 1) * SLOT + wave * 4096;
         if (item.splits == 1) {
             const WgradTile t = wgrad_tile<BM, BN>(w, item.tile);
-            const EpilogueF32 whole{w.dw[t.job], w.lddw[t.job], 0, w.accumulate};
+            const EpilogueF32As<THROUGH> whole{w.dw[t.job], w.lddw[t.job], 0, w.accumulate};
             staged_store_f32<FM, FN>(acc, mine, whole, t.m0 + wm, t.n0 + wn, lane, 0);
         } else {
-            const EpilogueF32 piece{w.pieces + size_t(piece_slot(w, item.tile, item.split)) * (BM * BN), BN, 0, 0};
+            const EpilogueF32As<THROUGH> piece{w.pieces + size_t(piece_slot(w, item.tile, item.split)) * (BM * BN), BN, 0, 0};
             staged_store_f32<FM, FN>(acc, mine, piece, wm, wn, lane, 0);
         }
     }
@@ -2825,15 +2831,20 @@ extern "C" int tgk_gemm_wgrad_batch(hipStream_t stream, int M, int count, const 
                 "gemm_wgrad_batch: workspace too small (see tgk_gemm_wgrad_batch_workspace)");
         w.accumulate = accumulate;
         w.pieces = static_cast<float *>(workspace);
-        auto kernel = wgrad_batch_kernel<128, 192>;
+        // Of more tiles than blocks most are written while their block's next one is worked on, and nothing is left to wait for once
+        // that takes long enough.  us with results through the caches and past them: four gradients of d_model 1152 (ffn 4608, 648 tiles)
+        // 256 tokens 21.0, 19.6; 1024 49.2, 50.1; 4096 133, 137; 16384 503, 506; 1536 (6144, 1152 tiles) 256 31.5, 31.1; 1024 67.8, 69.3; 16384
+        // 1004, 1046.  Of 48 to 480 tiles 256 tokens take 1 to 11 % less past them, from 1024 on the two are 0.1 % apart (-4 to 4 %).
+        const bool cached = w.first_tile[count] > resident_blocks(TILE_128x192) && M >= 1024;
+        const auto kernel = cached ? wgrad_batch_kernel<128, 192, false> : wgrad_batch_kernel<128, 192, true>;
         constexpr size_t lds = 2 * (128 + 192) * 128;
-        static std::atomic<bool> configured[MAX_DEVICES];
+        static std::atomic<bool> configured[2][MAX_DEVICES];
         const int device = current_device();
-        if (!configured[device].load(std::memory_order_acquire)) {
+        if (!configured[cached][device].load(std::memory_order_acquire)) {
             check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
                       "gemm LDS size: ");
-            configured[device].store(true, std::memory_order_release);
+            configured[cached][device].store(true, std::memory_order_release);
         }
         hipLaunchKernelGGL(kernel, dim3(wgrad_batch_blocks(w)), dim3(256), lds, stream, w);
         check_hip(hipGetLastError(), "wgrad batch launch: ");
