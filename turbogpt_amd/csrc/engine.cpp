@@ -588,6 +588,7 @@ void validate(const TgModelConfig &m) {
 // different ones, but only once every queue is there and has as many: two slots that share one run one behind the other.  So as
 // many streams are made first, and given back.  Depth 8, 768 sequences of 8, K = 4, calls of one step, us a step without and with them:
 // alone 36, 36; beside another engine or two, after one that is gone, with torch at work 49 to 51, 33 to 36.  K = 2 beside two others 80, 48.
+// They make the engine's creation longer, K = 2 / 4 / 8 0.2, 0.4, 1.2 -> 1.5, 2.8, 4.2 ms, as much as 100 to 200 steps give back.
 void build_streams(Engine *e, int inflight) {
     struct Spare {
         std::vector<hipStream_t> streams;
