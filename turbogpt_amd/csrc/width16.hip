@@ -750,13 +750,28 @@ TG_DEVICE void forward_pass(const Model &m, const Lane &p, const Staged &weight,
                 logits_out[size_t(p.token) * V + (p.role + R * i) * 16 + 4 * r + p.g] = logit[i][r];
     // the target's logit: register target / 4 % 4 of tile target / 16, of the lane g = target % 4
     const bool holder = p.g == (target & 3) && p.role == (target >> 4) % R;
+    const int tile = (target >> 4) / R, mine = holder ? tile * 4 + ((target >> 2) & 3) : -1; // 4 i + r
     float picked = 0.f;
-    const int mine = holder ? (target >> 4) / R * 4 + ((target >> 2) & 3) : -1; // 4 i + r
+    if constexpr (R == 1) { // by halves: one after another the 64 choices made lone waves spill 8 to 15 registers
+        float of_four[TILES];
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) {
+            const float even = target & 4 ? logit[i][1] : logit[i][0], odd = target & 4 ? logit[i][3] : logit[i][2];
+            of_four[i] = target & 8 ? odd : even;
+        }
+#pragma unroll
+        for (int half = TILES / 2, bit = 1; half; half >>= 1, bit <<= 1)
+#pragma unroll
+            for (int i = 0; i < half; ++i)
+                of_four[i] = tile & bit ? of_four[2 * i + 1] : of_four[2 * i];
+        picked = holder ? of_four[0] : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < TILES; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            picked = 4 * i + r == mine ? logit[i][r] : picked;
+            if constexpr (R > 1)
+                picked = 4 * i + r == mine ? logit[i][r] : picked;
             logit[i][r] = expf(logit[i][r] - high);
         }
     picked = swap_add_16(swap_add_32(picked));
@@ -942,8 +957,9 @@ TG_DEVICE void backward_pass(const Model &m, const Lane &p, const Staged &weight
 }
 
 // ---- kernels -----------------------------------------------------------------------------------------
-// Four waves a SIMD: of lone waves two blocks share a unit (128 registers, 8 to 15 of them spilled; with 155 to 177 and one block
-// 131072 tokens at depth 8 173 us forward and 242 with gradient, so 160 and 230).
+// Four waves a SIMD: of lone waves two blocks share a unit (128 registers; with 155 to 177 and one block 131072 tokens at depth 8 173 us
+// forward and 242 with gradient, so 156 and 221; 160 and 230 while 8 to 15 registers were spilled, which cost 524288 tokens at depth 1 372 and
+// 444 us for 324 and 387).
 template <bool GRADIENT, int R>
 __global__ __launch_bounds__(64 * block_waves(R), 4) void w16_forward_kernel(Model m, const uint8_t *__restrict__ x, const uint8_t *__restrict__ y,
                                                                          Workspace s, float *__restrict__ token_losses,
