@@ -19,9 +19,9 @@ def rules(tmp_path_factory):
     return C.CDLL(str(library))
 
 
-def teams(rules, waves, depth, passes=False, count=1, flying=1):
+def teams(rules, waves, depth, passes=0, count=1, flying=1):
     out = (C.c_int * 4)()
-    rules.w16_teams(int(passes), waves, count, depth, flying, UNITS, out)
+    rules.w16_teams(passes, waves, count, depth, flying, UNITS, out)
     return dict(zip(("teams", "blocks", "waves", "rows"), out))
 
 
@@ -29,17 +29,22 @@ def teams(rules, waves, depth, passes=False, count=1, flying=1):
 @pytest.mark.parametrize("waves,roles", [(4, TEAM), (256, TEAM), (1024, TEAM), (1025, LONE), (3072, LONE), (8192, LONE)])
 def test_width16_passes_of_their_own(rules, depth, waves, roles):
     """Beyond four teams a unit both passes go to lone waves, like a step's."""
-    for passes in (False, True):
+    for passes in (0, 1, 2):
         chosen = teams(rules, waves, depth, passes)
         assert chosen["waves"] == roles
         assert chosen["teams"] * chosen["blocks"] >= waves > chosen["teams"] * (chosen["blocks"] - 1)
         assert not (passes and chosen["rows"])  # the backward pass is another launch
 
 
-@pytest.mark.parametrize("waves,teams_of_a_block", [(1025, 5), (2048, 8), (2049, 5), (3072, 6), (4096, 8), (65536, 8)])
-def test_width16_lone_waves_are_shared_out_evenly(rules, waves, teams_of_a_block):
-    """One block a unit up to eight lone waves a unit, then two."""
-    assert teams(rules, waves, 8, passes=True)["teams"] == teams_of_a_block
+@pytest.mark.parametrize("waves,evaluated,with_gradient", [(1025, 5, 5), (2048, 8, 8), (2049, 5, 5), (2560, 5, 5), (2561, 6, 4), (3072, 6, 4), (3073, 7, 7),
+                                                           (4096, 8, 8), (4097, 6, 6), (4608, 6, 6), (8192, 8, 8), (8193, 7, 7), (65536, 8, 8)])
+def test_width16_lone_waves_are_shared_out_evenly(rules, waves, evaluated, with_gradient):
+    """Every unit has as many blocks, of eight lone waves at most, and every block as many waves."""
+    for passes, share in ((1, evaluated), (2, with_gradient)):
+        chosen = teams(rules, waves, 8, passes=passes)
+        assert chosen["teams"] == share
+        per_unit = -(-chosen["blocks"] // UNITS)
+        assert (share - 1) * per_unit * UNITS < waves <= share * per_unit * UNITS
 
 
 @pytest.mark.parametrize("depth", [4, 8])

@@ -1659,7 +1659,7 @@ extern "C" int tgk_w16_forward(hipStream_t stream, int depth, int batch, int con
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_forward: workspace must be 256-byte aligned");
         Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        const Teams t = pass_teams(r.waves, depth, compute_units());
+        const Teams t = pass_teams(r.waves, depth, with_gradient != 0, compute_units());
         m.teams = t.teams;
         static std::atomic<bool> configured[4][64];
         const bool lone = t.roles == 1;
@@ -1679,7 +1679,7 @@ extern "C" int tgk_w16_backward(hipStream_t stream, int depth, int batch, int co
         require(!(reinterpret_cast<uintptr_t>(workspace) & 255), "w16_backward: workspace must be 256-byte aligned");
         Model m = make_model(depth, batch, context, weight_hi, weight_lo);
         const Workspace r = carve(depth, batch, context, workspace);
-        const Teams t = pass_teams(r.waves, depth, compute_units());
+        const Teams t = pass_teams(r.waves, depth, true, compute_units());
         m.teams = t.teams;
         static std::atomic<bool> configured[2][64];
         const bool lone = t.roles == 1;

@@ -104,12 +104,18 @@ inline bool shares_launches(int depth, int K, int flying, int blocks, int steps,
 }
 // The forward and the backward pass as launches of their own: by the same rule, and both alike, as a lone wave leaves its
 // features' rows to the backward pass.  us forward, with gradient, and backward with the weight gradients at depth 8, context 8, teams;
-// lone waves: 16384 tokens 35, 39, 70; (older kernels) 39, 44, 75   20480 66, 71, 107; 47, 58, 87   131072 258, 276, 549; 160, 230, 443
-// Two blocks fit a unit.  Of more than eight lone waves a unit both have the same share: 49152 tokens, eight a block 88, 114, 184, six 82,
-// 107, 179.
-inline Teams pass_teams(int waves, int depth, int units) {
+// lone waves: 16384 tokens 35, 39, 70; (older kernels) 39, 44, 75   20480 66, 71, 107; 46, 57, 87   131072 258, 276, 549; 156, 222, 442
+// Two blocks fit a unit, and the next one starts where one ends: of more than eight lone waves a unit every block has the same share, as
+// few blocks as that takes a unit, so that no unit has one more than another.  us forward, eight a block and so: depth 8, 73728 tokens (18 lone waves a
+// unit, six a block) 120, 102; depth 4, context 5, 131072 (34, seven) 131, 118; depth 1 65536 (17, six) 59, 50.  With gradient and backward blocks of
+// six are the slowest for their number (three waves a SIMD, two of them on one): at 10 to 12 a unit three blocks of four, 49152 tokens at depth 8
+// 102, 95 and 179, 172; depth 4 69, 65 and 105, 101; forward 81, 83.
+inline Teams pass_teams(int waves, int depth, bool gradient, int units) {
     const Teams t = step_teams(waves, 1, depth, 1, units, false);
-    return t.roles == 1 && waves > 8 * units ? teams_of(waves, 1, depth, 1, false, 2 * units) : t;
+    if (t.roles > 1)
+        return t;
+    const bool of_four = gradient && waves > 10 * units && waves <= 12 * units;
+    return teams_of(waves, 1, depth, 1, false, (of_four ? 3 : (waves + 8 * units - 1) / (8 * units)) * units);
 }
 
 } // namespace w16
