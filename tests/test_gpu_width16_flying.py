@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
     (8, 8, 2, 73), (8, 4, 3, 63), (4, 8, 4, 54),     # three, rows in memory; and in LDS
     (8, 8, 2, 97), (8, 8, 3, 179), (4, 4, 3, 73), (8, 8, 4, 49), (4, 4, 16, 149),  # four
     (8, 8, 2, 225), (8, 8, 3, 180), (4, 8, 4, 150),  # lone waves
+    (4, 4, 1, 640), (4, 8, 1, 641), (4, 4, 1, 1025), # one batch: blocks of five, four and six lone waves
 ])
 def test_a_step_is_its_gradient_and_its_update(depth, context, inflight, blocks, orc):
     """Bit for bit, as every sum has one order whatever the launch; the last block of four teams has one team's tokens.  No clipping: the

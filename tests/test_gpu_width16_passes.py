@@ -27,7 +27,8 @@ def forward(depth, context, batch, flat, x, y):
 
 @pytest.mark.parametrize("depth,context,batch", [(2, 8, 2048), (2, 8, 2049),  # the last on teams, the first on lone waves
                                                  (8, 4, 4097), (3, 5, 3073),  # lone waves with sixteen and fifteen tokens
-                                                 (1, 8, 8197)])               # sixteen lone waves a unit
+                                                 (1, 8, 5121),                # ten a unit: blocks of six, with gradient of four
+                                                 (1, 8, 8197)])               # sixteen and one: three blocks of six a unit
 def test_passes(depth, context, batch):
     flat = reference_style_weights(depth)
     rng = np.random.default_rng(batch)

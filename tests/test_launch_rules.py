@@ -40,7 +40,7 @@ def test_width16_passes_of_their_own(rules, depth, waves, roles):
                                                            (4096, 8, 8), (4097, 6, 6), (4608, 6, 6), (8192, 8, 8), (8193, 7, 7), (65536, 8, 8)])
 def test_width16_lone_waves_are_shared_out_evenly(rules, waves, evaluated, with_gradient):
     """Every unit has as many blocks, of eight lone waves at most, and every block as many waves."""
-    for passes, share in ((1, evaluated), (2, with_gradient)):
+    for passes, share in ((0, with_gradient), (1, evaluated), (2, with_gradient)):
         chosen = teams(rules, waves, 8, passes=passes)
         assert chosen["teams"] == share
         per_unit = -(-chosen["blocks"] // UNITS)

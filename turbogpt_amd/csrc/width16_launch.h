@@ -51,10 +51,19 @@ inline Teams teams_of(int waves, int count, int depth, int roles, bool rows, int
         ++teams;
     return {teams, (waves + teams - 1) / teams, roles, lds(teams), rows};
 }
+// Lone waves with the units to themselves.  Two blocks fit a unit, and the next one starts where one ends: every block has the same share, as
+// few blocks a unit as that takes, so that no unit has one more than another.  us forward, eight a block and so: depth 8, 73728 tokens (18 lone waves
+// a unit, six a block) 120, 102; depth 4, context 5, 131072 (34, seven) 131, 118; depth 1 65536 (17, six) 59, 50; a step at depth 8: 40960 267, 231;
+// 73728 424, 399.  With gradient and backward blocks of six are the slowest for their number (three waves a SIMD, two of them on one): at 10
+// to 12 a unit three blocks of four, 49152 tokens at depth 8 102, 93 and 179, 173, a step 286, 269; depth 4 69, 61 and 105, 101, 162, 149; forward 81, 83.
+inline Teams lone_teams(int waves, int depth, bool gradient, int units) {
+    const bool of_four = gradient && waves > 10 * units && waves <= 12 * units;
+    return teams_of(waves, 1, depth, 1, false, (of_four ? 3 : (waves + 8 * units - 1) / (8 * units)) * units);
+}
 // Teams of four waves while every one has a place on the units at once, with its rows in LDS where they fit.  Beyond that a lone wave
 // does less in all: no handing over, two waves' arithmetic side by side on a SIMD.  us a step, teams and lone waves: 640 teams at depth 8
-// (context 4) 87 and 106, 1280 (context 8) 171 and 145.  Of lone waves a block takes as many as leave every unit one block (1280 teams: 145, with
-// four 149), four where there are other batches (K = 4, 640 teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us).
+// (context 4) 87 and 106, 1280 (context 8) 171 and 145.  Where there are other batches a block takes four lone waves (K = 4, 640
+// teams: 3, 4, 5, 8 a block 62, 59, 68, 67 us).
 // `flying` such launches run side by side, on streams of their own, and a unit has room for one block of teams: they are cut so that all of
 // them fit, their rows left out of LDS for more teams a block, and one's tail is another's start, so that teams are the better form for
 // longer.  Depth 8, 64 blocks of four teams (256 teams a batch), calls of one step, us a step with one, two (rows in LDS) and four teams a block
@@ -75,7 +84,7 @@ inline Teams step_teams(int waves, int count, int depth, int flying, int units, 
         if (t.blocks * count <= places || (flying > 1 && !rows))
             return t;
     }
-    return teams_of(waves, count, depth, 1, false, count * flying > 1 ? (waves + 3) / 4 * count : units);
+    return count * flying > 1 ? teams_of(waves, count, depth, 1, false, (waves + 3) / 4 * count) : lone_teams(waves, depth, true, units);
 }
 // Whether the batches of a call of `steps` steps, K of them in flight, share their launches: by the lesser of two estimated times in
 // us, for batches of `blocks` blocks of four teams' tokens at depth 4 or 8.  A shared launch's batches and their optimizer steps go as one
@@ -105,17 +114,9 @@ inline bool shares_launches(int depth, int K, int flying, int blocks, int steps,
 // The forward and the backward pass as launches of their own: by the same rule, and both alike, as a lone wave leaves its
 // features' rows to the backward pass.  us forward, with gradient, and backward with the weight gradients at depth 8, context 8, teams;
 // lone waves: 16384 tokens 35, 39, 70; (older kernels) 39, 44, 75   20480 66, 71, 107; 46, 57, 87   131072 258, 276, 549; 156, 222, 442
-// Two blocks fit a unit, and the next one starts where one ends: of more than eight lone waves a unit every block has the same share, as
-// few blocks as that takes a unit, so that no unit has one more than another.  us forward, eight a block and so: depth 8, 73728 tokens (18 lone waves a
-// unit, six a block) 120, 102; depth 4, context 5, 131072 (34, seven) 131, 118; depth 1 65536 (17, six) 59, 50.  With gradient and backward blocks of
-// six are the slowest for their number (three waves a SIMD, two of them on one): at 10 to 12 a unit three blocks of four, 49152 tokens at depth 8
-// 102, 95 and 179, 172; depth 4 69, 65 and 105, 101; forward 81, 83.
 inline Teams pass_teams(int waves, int depth, bool gradient, int units) {
     const Teams t = step_teams(waves, 1, depth, 1, units, false);
-    if (t.roles > 1)
-        return t;
-    const bool of_four = gradient && waves > 10 * units && waves <= 12 * units;
-    return teams_of(waves, 1, depth, 1, false, (of_four ? 3 : (waves + 8 * units - 1) / (8 * units)) * units);
+    return t.roles > 1 ? t : lone_teams(waves, depth, gradient, units);
 }
 
 } // namespace w16
