@@ -11,7 +11,7 @@ pytestmark = gemm.pytestmark
 # forward N x K, its mirror image the input gradient K x N
 PLAIN = [(1408, 6016, 896, 128), (2176, 8832, 768, 192), (2688, 9472, 768, 256)]
 GELU = [(2688, 4736, 768, 128), (3456, 8704, 512, 256)]
-GELU_BACKWARD = [(1408, 768, 9856, 128), (2176, 1024, 8832, 192), (2688, 512, 9984, 256)]
+GELU_BACKWARD = [(1408, 768, 9856, 128), (2176, 1024, 8832, 192), (2944, 512, 9984, 256)]
 
 
 @pytest.mark.parametrize("residual", [False, True])

@@ -98,6 +98,13 @@ def test_columns_of_256_row_tiles(rules, M, N, K, forward, gelu, backward, gelu_
     assert (columns(K, N, PLAIN), columns(K, N, GELU_BACKWARD)) == (backward, gelu_backward)
 
 
+@pytest.mark.parametrize("M,N,K", [(3584, 1920, 1024), (10240, 768, 1024), (4224, 1536, 1280), (2176, 3072, 1024), (4352, 3456, 2816), (13312, 1152, 3840)])
+def test_gelu_backward_where_two_blocks_of_128_columns_fit_every_unit(rules, M, N, K):
+    """22 to 29 % slower on 256-row tiles of 192 columns, which fill half of a round or of the second one (M x N outputs)."""
+    assert rules.gemm_columns_of_256(M, N, K, GELU_BACKWARD, UNITS) == 0
+    assert rules.gemm_columns_of_256(4096, 2304, 2304, GELU_BACKWARD, UNITS) == 192  # 216 tiles: 10 % faster
+
+
 def test_columns_of_256_row_tiles_in_several_rounds(rules):
     """The shapes of test_gpu_gemm_columns_rounds.py: more tiles than units, and half a tile of rows at the end."""
     import test_gpu_gemm_columns_rounds as shapes
