@@ -382,7 +382,7 @@ def test_rejects_bad_shapes_without_launching():
 def test_256x128_tiles_rows_sampled(orc, M, N, K, residual):
     """Products that tiles of 256 rows take, with the exception of the shortest: forward with every epilogue and the input gradient on
     the transposed weight, plain and times GELU', one to four tiles a block and four to thirty-two 128-k periods a tile, against the
-    checker on sampled rows and bit for bit against the kernels for k-strided weights, which sum in the same order."""
+    oracle on sampled rows and bit for bit against the kernels for k-strided weights, which sum in the same order."""
     lib = library()
     rng = np.random.default_rng(M + N + K)
     x, xh = to_bf16_device(rng.standard_normal((M, K)))

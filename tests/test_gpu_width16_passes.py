@@ -1,6 +1,6 @@
 """tgk_w16_forward and tgk_w16_backward on teams and on lone waves, on either side of the line between them (1024 teams on 256
 compute units): a sequence's logits do not depend on which, nor on whether a gradient is wanted, bit for bit.  Values and gradients
-of both against the checker: test_gpu_width16_blocks."""
+of both against the oracle: test_gpu_width16_blocks."""
 import numpy as np
 import pytest
 import torch
